@@ -692,7 +692,8 @@ int tdh_batchnorm_update_moving(int channels, float momentum, const float *mean_
   TDH_CHECK_ARG(channels >= 0, "tdh_batchnorm_update_moving: negative size");
   if (channels == 0) return TDH_OK;
   TDH_CHECK_ARG(mean_cur && var_cur && mean && variance, "tdh_batchnorm_update_moving: null tensor");
-  return batchnorm_update_moving(channels, momentum, mean_cur, var_cur, mean, variance);
+  const BnMoving job{mean_cur, var_cur, mean, variance, momentum, channels};
+  return batchnorm_update_moving(&job, 1);
 }
 
 int tdh_dropout_fwd(int batch, int len, int train, float scale, const uint8_t *mask, const float *x,

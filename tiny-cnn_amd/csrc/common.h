@@ -262,8 +262,18 @@ int batchnorm_fwd(int channels, int spatial, int batch, float eps, int train, co
                   float *mean, float *variance, float *stddev, float *y);
 int batchnorm_bwd(int channels, int spatial, int batch, const float *y, const float *dy,
                   const float *stddev, float *dx);
-int batchnorm_update_moving(int channels, float momentum, const float *mean_cur,
-                            const float *var_cur, float *mean, float *var);
+// the running averages of up to BN_MOVING_MAX layers a launch
+struct BnMoving {
+  const float *mean_cur, *var_cur;
+  float *mean, *var;
+  float momentum;
+  int channels;
+};
+constexpr int BN_MOVING_MAX = 16;
+struct BnMovingJobs {
+  BnMoving job[BN_MOVING_MAX];
+};
+int batchnorm_update_moving(const BnMoving *jobs, int n);
 int dropout_fwd(size_t total, int train, float scale, const uint8_t *mask, const float *x, float *y);
 int dropout_bwd(size_t total, const uint8_t *mask, const float *dy, float *dx);
 size_t rowsum_workspace_bytes(int outer, int rows, int cols);

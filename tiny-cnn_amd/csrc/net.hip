@@ -804,11 +804,11 @@ int tdh_net_reset_optimizer(tdh_net *net) {
 // layer::update_weight ends in post_update (layer.h:681): a batch-norm layer moves its running
 // averages towards the moments of the batch (batch_normalization_layer.h:171-177)
 static int post_update(tdh_net *net) {
-  for (tdh_net::Layer &L : net->layers)
+  std::vector<BnMoving> jobs;
+  for (const tdh_net::Layer &L : net->layers)
     if (L.spec.kind == TDH_L_BATCHNORM)
-      TDH_TRY(batchnorm_update_moving(L.spec.bn_channels, L.spec.bn_momentum, L.bn_mean_cur, L.bn_var_cur,
-                                      L.bn_mean, L.bn_var));
-  return TDH_OK;
+      jobs.push_back(BnMoving{L.bn_mean_cur, L.bn_var_cur, L.bn_mean, L.bn_var, L.spec.bn_momentum, L.spec.bn_channels});
+  return batchnorm_update_moving(jobs.data(), static_cast<int>(jobs.size()));
 }
 
 int tdh_net_update_weights(tdh_net *net, tdh_opt *opt) {
