@@ -306,6 +306,7 @@ int tdh_shutdown(void) {
   Context &c = ctx();
   if (!c.ready) return TDH_OK;
   TDH_HIP(hipStreamSynchronize(c.stream));
+  host_copy_release();
   if (c.workspace) TDH_HIP(hipFree(c.workspace));
   for (hipStream_t s : c.side)
     if (s) TDH_HIP(hipStreamDestroy(s));
@@ -344,6 +345,7 @@ int tdh_memcpy_h2d(void *dst, const void *src, size_t bytes) {
   TDH_REQUIRE_INIT();
   if (bytes == 0) return TDH_OK;
   TDH_CHECK_ARG(dst && src, "tdh_memcpy_h2d: null pointer");
+  if (host_copy_up_applies(bytes)) return host_copy_up(dst, src, bytes);
   TDH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx().stream));
   TDH_HIP(hipStreamSynchronize(ctx().stream));  // the host buffer may be reused on return
   return TDH_OK;
@@ -353,6 +355,7 @@ int tdh_memcpy_d2h(void *dst, const void *src, size_t bytes) {
   TDH_REQUIRE_INIT();
   if (bytes == 0) return TDH_OK;
   TDH_CHECK_ARG(dst && src, "tdh_memcpy_d2h: null pointer");
+  if (host_copy_down_applies(bytes)) return host_copy_down(dst, src, bytes);
   TDH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx().stream));
   TDH_HIP(hipStreamSynchronize(ctx().stream));
   return TDH_OK;

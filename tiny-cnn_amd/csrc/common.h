@@ -161,6 +161,13 @@ int pool_out_length(int in_length, int window, int stride, int ceil_mode, int pa
 // elementwise.hip
 int launch_fill_zero(void *p, size_t bytes, const char *tag = "fill_zero");
 int launch_copy(void *dst, const void *src, size_t bytes);  // bytes % 4 == 0
+// hostcopy.hip: small copies between pageable host memory and the device. The upload returns when `src` has been read and is ordered on the library stream; the
+// download returns when `dst` has been written, behind the work queued before it.
+bool host_copy_up_applies(size_t bytes);
+bool host_copy_down_applies(size_t bytes);
+int host_copy_up(void *dst, const void *src, size_t bytes);
+int host_copy_down(void *dst, const void *src, size_t bytes);
+void host_copy_release();
 // p: two constructor parameters (never null); x may be null unless the kind's gradient reads it
 int launch_act_fwd(int kind, const float *p, int batch, int len, const float *x, float *y);
 int launch_act_bwd(int kind, const float *p, int batch, int len, const float *x, const float *y,

@@ -58,9 +58,11 @@ struct tdh_net {
     const void *scratch = nullptr;      // the library scratch buffer the captured kernels use
     tdh_opt hyper = {};                 // hyper-parameters only (powers zeroed)
   };
-  // a few captured steps are kept, so that alternating input buffers (double-buffered
-  // uploads) or batch sizes (the short last batch of an epoch) do not re-capture every step
-  static constexpr int kGraphSlots = 8;
+  // Captured steps are kept, so that rotating input buffers or batch sizes (the short last batch
+  // of an epoch) do not re-capture: a pass over host batches comes with three device slots, two
+  // batch sizes and, under Adam, two power buffers, 12 keys in all. (With 8 the short batch's
+  // three keys pushed each other out: CIFAR net, 500 samples in batches of 64, 1440 us a pass.)
+  static constexpr int kGraphSlots = 16;
   struct GraphSlot {
     hipGraphExec_t exec = nullptr;
     GraphKey key;
@@ -867,10 +869,24 @@ const int32_t *tdh_net_layer_argmax(const tdh_net *net, int layer) {
   return (layer >= 0 && layer < static_cast<int>(net->layers.size())) ? net->layers[layer].argmax : nullptr;
 }
 
+// The filters in the stride-1 kernels' layout: packed here when the weights came from outside
+// (creation, tdh_net_set_param, a pointer handed out), by the optimizer kernel after that.
+static int refresh_packs(tdh_net *net) {
+  if (!(net->flags & TDH_NET_GRAPH) || net->packs_valid) return TDH_OK;
+  for (tdh_net::Layer &L : net->layers) {
+    if (!L.wp_fwd) continue;
+    TDH_TRY(conv_pack_filters(&L.spec.conv, 0, L.w, L.tbl_dev, L.wp_fwd));
+    TDH_TRY(conv_pack_filters(&L.spec.conv, 1, L.w, L.tbl_dev, L.wp_dx));
+  }
+  net->packs_valid = true;
+  return TDH_OK;
+}
+
 int tdh_net_forward(tdh_net *net, int batch, const float *x) {
   TDH_REQUIRE_INIT();
   TDH_CHECK_ARG(net && x && batch > 0 && batch <= net->max_batch, "tdh_net_forward: bad argument");
-  return forward(net, batch, x);
+  TDH_TRY(refresh_packs(net));
+  return forward(net, batch, x, net->packs_valid);
 }
 
 // Queues one whole train step on the library stream. forked (only while the stream is being
@@ -1242,18 +1258,7 @@ static bool same_key(const tdh_net::GraphKey &a, const tdh_net::GraphKey &b) {
 // captured into one graph and replayed
 static int train_steps(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, int n_steps, const float *const *xs,
                        const float *const *ts, int do_update) {
-  const float *x = xs[0], *t = ts[0];
-  // The filters in the stride-1 kernels' layout: packed here when the weights came from
-  // outside (creation, tdh_net_set_param, a pointer handed out), by the optimizer kernel after
-  // that.
-  if ((net->flags & TDH_NET_GRAPH) && !net->packs_valid) {
-    for (tdh_net::Layer &L : net->layers) {
-      if (!L.wp_fwd) continue;
-      TDH_TRY(conv_pack_filters(&L.spec.conv, 0, L.w, L.tbl_dev, L.wp_fwd));
-      TDH_TRY(conv_pack_filters(&L.spec.conv, 1, L.w, L.tbl_dev, L.wp_dx));
-    }
-    net->packs_valid = true;
-  }
+  TDH_TRY(refresh_packs(net));
   // per-kernel timing needs the launches themselves, not a replay
   if (!(net->flags & TDH_NET_GRAPH) || profiling_active()) {
     // (the timing pass of a branching step keeps every layer's scratch piece until the optimizer
