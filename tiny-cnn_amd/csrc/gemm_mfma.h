@@ -31,6 +31,8 @@
 //                __device__ void store(int m, const Col&, float v) const; };
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace tdh {
@@ -184,11 +186,18 @@ struct EpiImageRowsAct {
   }
 };
 
+// An operand may differ from one column tile to the next: the kernel works with what bind_tile
+// returns for its first column, and reduces over the first tile_k of the K terms.
+template <class Op>
+__device__ __forceinline__ const Op &bind_tile(const Op &op, int) { return op; }
+template <class Op>
+__device__ __forceinline__ int tile_k(const Op &, int, int K) { return K; }
+
 // --------------------------------------------------------------------- kernel
 template <int BM, int BN, int WM, int WN, bool A_LANE_K, bool B_LANE_K, bool A_VEC, bool B_VEC,
           class AOp, class BOp, class Epi>
 __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(3, 8)))
-gemm_mfma_kernel(const AOp aop, const BOp bop, const Epi epi, const int M, const int N,
+gemm_mfma_kernel(const AOp a_op, const BOp b_op, const Epi epi, const int M, const int N,
                  const int K, const int k_per_split, float *__restrict__ partial) {
   constexpr int BK  = GEMM_BK;
   constexpr int NT  = 64 * WM * WN;  // threads per workgroup
@@ -231,7 +240,11 @@ gemm_mfma_kernel(const AOp aop, const BOp bop, const Epi epi, const int M, const
   const int m0   = by * BM;
   const int n0   = bx * BN;
   const int kbeg = bz * k_per_split;
-  const int kend = min(K, kbeg + k_per_split);
+  const int kend = min(tile_k(b_op, n0, K), kbeg + k_per_split);
+  const auto &aop = bind_tile(a_op, n0);
+  const auto &bop = bind_tile(b_op, n0);
+  using ATile = std::decay_t<decltype(aop)>;
+  using BTile = std::decay_t<decltype(bop)>;
 
   // ---- per-thread staging assignment
   // LANE_K : k_local = tid % 16 (fixed), rows (tid/16) + (NT/16)*i
@@ -239,8 +252,8 @@ gemm_mfma_kernel(const AOp aop, const BOp bop, const Epi epi, const int M, const
   //          tile width is a multiple of NT the row is the same for every i
   constexpr bool A_ONE_ROW = (NT % BM) == 0;
   constexpr bool B_ONE_ROW = (NT % BN) == 0;
-  typename AOp::Fix fa[(A_LANE_K || !A_ONE_ROW) ? CA : 1];
-  typename BOp::Fix fb[(B_LANE_K || !B_ONE_ROW) ? CB : 1];
+  typename ATile::Fix fa[(A_LANE_K || !A_ONE_ROW) ? CA : 1];
+  typename BTile::Fix fb[(B_LANE_K || !B_ONE_ROW) ? CB : 1];
   if constexpr (A_VEC && A_LANE_K) {
     // k group = tid % 4, rows (tid/4) + (NT/4)*i
 #pragma unroll
@@ -300,7 +313,7 @@ gemm_mfma_kernel(const AOp aop, const BOp bop, const Epi epi, const int M, const
     } else if (A_LANE_K) {
       const int k = kt + (tid & 15);
       if (k < kend) {
-        const typename AOp::KDec kd = aop.kdec(k);
+        const typename ATile::KDec kd = aop.kdec(k);
 #pragma unroll
         for (int i = 0; i < CA; ++i) ra[i] = aop.load(fa[i], kd);
       } else {
@@ -340,7 +353,7 @@ gemm_mfma_kernel(const AOp aop, const BOp bop, const Epi epi, const int M, const
     } else if (B_LANE_K) {
       const int k = kt + (tid & 15);
       if (k < kend) {
-        const typename BOp::KDec kd = bop.kdec(k);
+        const typename BTile::KDec kd = bop.kdec(k);
 #pragma unroll
         for (int i = 0; i < CB; ++i) rb[i] = bop.load(fb[i], kd);
       } else {
