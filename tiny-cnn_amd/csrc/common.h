@@ -35,6 +35,16 @@ struct Context {
   // leave_split_sum: the caller of a convolution asks it to leave a split reduction to the
   // kernel that reads the result next; split_sum_left: one was left (left_split_sum())
   bool leave_split_sum = false, split_sum_left = false;
+  // Products keep to the fp32 matrix instructions while this is set. The three-part products of
+  // split_bf16.h are no less precise, but they round differently, and there are two places where a
+  // train step turns roundings into something larger, so that a training run would take another
+  // course than it always has:
+  //  - its forward pass decides signs (relu) and maxima (max-pool), and with them where whole
+  //    gradients go: one choice in a million changes, and the input gradient of the VGG-style
+  //    stack by 1.6e-3 with it;
+  //  - the bias gradient of a convolution in front of a batch normalization is zero but for its
+  //    rounding, and an optimizer that divides by the gradient's size makes full steps of that.
+  bool keep_f32 = false;
   // two more streams (default priority) for work that branches off the main one inside a
   // captured train step; created on first use
   hipStream_t side[2]   = {nullptr, nullptr};
@@ -189,6 +199,8 @@ struct OptTensor {
   // layout: the update also writes the new value into those copies (wp_fwd[t][ci][co],
   // wp_dx[rs-1-t][co][ci]; unconnected pairs of the connection table as zero). NULL: none.
   float *wp_fwd, *wp_dx;
+  // the same in the three bf16 parts of the kernel of conv_x3_inst.hip (with wp_fwd only)
+  uint16_t *wx_fwd, *wx_dx;
   const uint8_t *tbl;
   uint32_t C, Kc, rs;
 };
@@ -313,7 +325,8 @@ int finish_split_sum();      // the reduction as a launch of its own, when nobod
 
 
 // conv.hip / fc.hip
-// prepacked: filters already packed by conv_pack_filters for this direction (and only then)
+// prepacked: filters already packed by conv_pack_filters for this direction, in the kind that
+// conv_packed_kind names
 // A 2x2 / stride-2 max-pool layer (and the pointwise activation behind it) computed by the
 // forward kernel of the layer in front of it
 struct PoolFuse {
@@ -323,7 +336,7 @@ struct PoolFuse {
   int act_kind;
 };
 int conv2d_fwd(const tdh_conv_desc *d, int batch, const float *x, const float *w, const float *b,
-               float *y, const uint8_t *tbl_resident = nullptr, const float *prepacked = nullptr,
+               float *y, const uint8_t *tbl_resident = nullptr, const void *prepacked = nullptr,
                float *act_out = nullptr, int act_kind = 0, const PoolFuse *pool = nullptr);
 // dX, dW and db of this (first) convolution leave conv2d_bwd as one launch when all three are
 // asked for together (pooled: the gradient is read through the max-pool behind the layer)
@@ -345,17 +358,20 @@ int conv_fwd_small_run(int batch, int C, int Kc, const float *x, const float *w,
 // and may be null); only where conv_bwd_reads_pooled says so
 int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w, const float *dy,
                float *dx, float *dw, float *db, int accumulate, ActGrad dx_act,
-               const uint8_t *tbl_resident = nullptr, const float *prepacked_dx = nullptr,
+               const uint8_t *tbl_resident = nullptr, const void *prepacked_dx = nullptr,
                const PoolGather *dy_pool = nullptr);
 // the backward kernels of this layer (the two of a first layer: few input channels, stride 1)
 // can read their output gradient through this 2x2 / stride-2 max-pool over the layer's output
 bool conv_bwd_reads_pooled(const tdh_conv_desc *d, const tdh_pool_desc *pool, int batch);
-// true when forward (flip = 0) / dX (flip = 1) of this layer reads packed filters
-bool conv_uses_packed(const tdh_conv_desc *d, int batch, int flip);
+// the packed filters that forward (flip = 0) / dX (flip = 1) of this layer reads: none, floats
+// (conv_s1_inst.hip) or three bf16 parts (conv_x3_inst.hip), and the bytes they take
+enum { CONV_PACK_NONE = 0, CONV_PACK_F32 = 1, CONV_PACK_X3 = 2 };
+int conv_packed_kind(const tdh_conv_desc *d, int batch, int flip);
+size_t conv_packed_bytes(const tdh_conv_desc *d, int kind, int flip);
 bool conv_fwd_applies_act(const tdh_conv_desc *d, int batch, bool prepacked);
-// packs w (masked by the device-resident connection table, if any) into wp[k_w*k_h*in_c*out_c]
-int conv_pack_filters(const tdh_conv_desc *d, int flip, const float *w, const uint8_t *tbl_resident,
-                      float *wp);
+// packs w (masked by the device-resident connection table, if any) into wp
+int conv_pack_filters(const tdh_conv_desc *d, int kind, int flip, const float *w, const uint8_t *tbl_resident,
+                      void *wp);
 int fc_fwd(int in, int out, int has_bias, int batch, const float *x, const float *w,
            const float *b, float *y, float *act_out = nullptr, int act_kind = 0);
 // The backward pass of a 2x2 / stride-2 max-pool layer in front of a fully-connected layer,
@@ -398,7 +414,7 @@ size_t conv_s1_workspace_bytes(int R, int S, int batch, int C, int Kc, int flip,
 int conv_s1_run(int R, int S, int batch, int C, int Kc, int flip, const float *in, const float *w,
                 const uint8_t *tbl_dev, const float *bias, float *out, int IH, int IW, int OH,
                 int OW, int ph, int pw, ActGrad ag, const char *tag,
-                const float *prepacked = nullptr, float *act_out = nullptr, int act_kind = 0,
+                const void *prepacked = nullptr, float *act_out = nullptr, int act_kind = 0,
                 const PoolFuse *pool = nullptr);
 // the forward kernel of this shape can also compute the 2x2 / stride-2 max-pool behind it (and
 // a relu behind that pool); `out` may then be null
@@ -408,7 +424,10 @@ bool conv_s1_fuses_pool(int R, int S, int batch, int KC, int MC, int IH, int IW,
 bool conv_s1_single_pass(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW,
                          int ph, int pw);
 int conv_s1_repack(int R, int S, int C, int Kc, int flip, const float *w, const uint8_t *tbl_dev,
-                   float *wp);
+                   void *wp, bool x3);
+// conv_packed_kind / conv_packed_bytes of a shape this file runs
+int conv_s1_packed_kind(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw);
+size_t conv_s1_packed_bytes(int kind, int RS, int KC, int MC);
 // conv_dw.hip: stride-1 weight gradient from LDS-staged tiles (3x3 and 5x5 windows)
 bool conv_dw_halo_applicable(int R, int S, int batch, int C, int Kc, int H, int W, int OH, int OW,
                              int ph, int pw);

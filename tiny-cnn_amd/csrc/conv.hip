@@ -1114,6 +1114,10 @@ static void launch_small_cin_dx_window(const ConvGeom &g, const DxsPlan &p, int 
 
 
 static bool fwd_small_applies(const ConvGeom &g, int batch) {
+  // (small windows over many channels are short reductions as well, but no first layers)
+  if (g.C >= 16 && g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 &&
+      conv_s1_packed_kind(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w) == CONV_PACK_X3)
+    return false;
   return conv_fwd_small_applicable(batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.R, g.S, g.sh, g.sw, g.dh,
                                    g.dw, g.pad_h, g.pad_w);
 }
@@ -1267,12 +1271,12 @@ bool conv_dw_gives_db(const tdh_conv_desc *d, int batch) {
 bool conv_fwd_applies_act(const tdh_conv_desc *d, int batch, bool prepacked) {
   // every forward kernel does: the packed stride-1 kernel, the first-layer kernel, the
   // stride-1 kernel that packs for itself and the GEMM (in its epilogue or its split reduction)
-  return prepacked ? conv_uses_packed(d, batch, 0) : true;
+  return prepacked ? conv_packed_kind(d, batch, 0) != CONV_PACK_NONE : true;
 }
 
 // the stride-1 kernel runs this forward pass (with filters packed by the caller, or by itself)
 static bool fwd_s1_applies(const tdh_conv_desc *d, const ConvGeom &g, int batch, bool prepacked) {
-  if (prepacked) return conv_uses_packed(d, batch, 0);
+  if (prepacked) return conv_packed_kind(d, batch, 0) != CONV_PACK_NONE;
   return !fwd_small_applies(g, batch) && g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 &&
          conv_s1_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
 }
@@ -1301,25 +1305,30 @@ bool conv_fwd_pool_applies_act(const tdh_conv_desc *d, int batch, bool prepacked
   return act_kind == TDH_ACT_RELU;
 }
 
-bool conv_uses_packed(const tdh_conv_desc *d, int batch, int flip) {
+int conv_packed_kind(const tdh_conv_desc *d, int batch, int flip) {
   const ConvGeom g = make_geom(d);
-  if (g.sh != 1 || g.sw != 1) return false;
+  if (g.sh != 1 || g.sw != 1) return CONV_PACK_NONE;
   if (!flip)
-    return g.dh == 1 && g.dw == 1 && !fwd_small_applies(g, batch) &&
-           conv_s1_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
+    return g.dh == 1 && g.dw == 1 && !fwd_small_applies(g, batch)
+             ? conv_s1_packed_kind(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w)
+             : CONV_PACK_NONE;
   DxsPlan dxs;
-  if (small_cin_dx_plan(g, dxs)) return false;
-  return conv_s1_applicable(g.R, g.S, batch, g.Kc, g.C, g.OH, g.OW, g.H, g.W, g.R - 1 - g.pad_h,
-                            g.S - 1 - g.pad_w);
+  if (small_cin_dx_plan(g, dxs)) return CONV_PACK_NONE;
+  return conv_s1_packed_kind(g.R, g.S, batch, g.Kc, g.C, g.OH, g.OW, g.H, g.W, g.R - 1 - g.pad_h,
+                             g.S - 1 - g.pad_w);
+}
+size_t conv_packed_bytes(const tdh_conv_desc *d, int kind, int flip) {
+  return conv_s1_packed_bytes(kind, d->k_h * d->k_w, flip ? d->out_c : d->in_c, flip ? d->in_c : d->out_c);
 }
 
-int conv_pack_filters(const tdh_conv_desc *d, int flip, const float *w, const uint8_t *tbl_resident,
-                      float *wp) {
-  return conv_s1_repack(d->k_h, d->k_w, d->in_c, d->out_c, flip, w, d->tbl ? tbl_resident : nullptr, wp);
+int conv_pack_filters(const tdh_conv_desc *d, int kind, int flip, const float *w, const uint8_t *tbl_resident,
+                      void *wp) {
+  return conv_s1_repack(d->k_h, d->k_w, d->in_c, d->out_c, flip, w, d->tbl ? tbl_resident : nullptr, wp,
+                        kind == CONV_PACK_X3);
 }
 
 int conv2d_fwd(const tdh_conv_desc *d, int batch, const float *x, const float *w, const float *b,
-               float *y, const uint8_t *tbl_resident, const float *prepacked, float *act_out,
+               float *y, const uint8_t *tbl_resident, const void *prepacked, float *act_out,
                int act_kind, const PoolFuse *pool) {
   const ConvGeom g = make_geom(d);
   if (pool) {
@@ -1424,7 +1433,7 @@ static int run_first_both(const ConvGeom &g, int batch, const float *x, const fl
 
 int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w, const float *dy,
                float *dx, float *dw, float *db, int accumulate, ActGrad dx_act,
-               const uint8_t *tbl_resident, const float *prepacked_dx, const PoolGather *dy_pool) {
+               const uint8_t *tbl_resident, const void *prepacked_dx, const PoolGather *dy_pool) {
   const ConvGeom g = make_geom(d);
   const int ohw = g.OH * g.OW, crs = g.C * g.R * g.S;
   if (dy_pool) {

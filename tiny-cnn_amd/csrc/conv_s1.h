@@ -22,8 +22,23 @@ constexpr int s1_niq(int R, int S, int TC, int TM, int TN) {
   return n > 16 ? 16 : n;
 }
 
+// The three-part bf16 kernel (conv_x3_inst.hip): 16 channels a chunk, words of eight channels that
+// a thread stages per chunk at most (32 registers each).
+constexpr int X3_KCH = 16;
+constexpr int x3_items(int TM, int TN) { return TM * TN >= 4 ? 1 : 2; }
+// rows of the packed filters: whole tiles of either width
+constexpr int x3_mc_pad(int MC) { return MC > 32 ? (MC + 63) / 64 * 64 : 32; }
+constexpr size_t x3_pack_bytes(int RS, int KC, int MC) {
+  return static_cast<size_t>((KC + 15) / 16) * RS * 6 * x3_mc_pad(MC) * 16;
+}
+
+// the sign of step u's products (chunk, tap): the packed filters carry it
+__host__ __device__ constexpr float x3_sign(int u) { return u & 1 ? -1.0f : 1.0f; }
+
 struct ConvS1Args {
-  const float *in, *wp, *bias;
+  const float *in;
+  const void *wp;              // filters: floats [tap][kc][m], or the parts of conv_x3_inst.hip
+  const float *bias;
   float *out;
   ActGrad ag;
   float *act_out;              // forward: act(out) of the pointwise activation layer that follows
@@ -43,12 +58,14 @@ struct ConvS1Args {
   // split over the reduction channels: workgroup z sums channels [z*kc_split, (z+1)*kc_split)
   // into part[z][...] (laid out like out); part == nullptr: one pass, written to out
   int kc_split;
+  int mc_pad;                  // rows of the packed filters (three-part kernel)
   float *part;
   size_t part_stride;
 };
 
 struct S1Plan {
   bool ok;
+  bool x3;                     // the three-part bf16 kernel
   int tc, tm, tn;
   ConvS1Args args;
   size_t lds_bytes;
@@ -61,5 +78,13 @@ int s1_launch_3x3_vec(const S1Plan &p);
 int s1_launch_3x3_scalar(const S1Plan &p);
 int s1_launch_5x5_vec(const S1Plan &p);
 int s1_launch_5x5_scalar(const S1Plan &p);
+int x3_launch_1_vec(const S1Plan &p);
+int x3_launch_1_scalar(const S1Plan &p);
+int x3_launch_3_vec(const S1Plan &p);
+int x3_launch_3_scalar(const S1Plan &p);
+int x3_launch_5_vec(const S1Plan &p);
+int x3_launch_5_scalar(const S1Plan &p);
+int x3_launch_7_vec(const S1Plan &p);
+int x3_launch_7_scalar(const S1Plan &p);
 
 }  // namespace tdh

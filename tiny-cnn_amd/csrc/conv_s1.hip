@@ -1,6 +1,9 @@
 // conv_s1.hip — host side of the stride-1 convolution (forward and dX) on the LDS-halo MFMA
 // kernel of conv_s1_inst.hip: tile choice, filter repacking, split-K reduction.
+#include <algorithm>
+
 #include "conv_s1.h"
+#include "split_bf16.h"
 
 namespace tdh {
 
@@ -54,6 +57,40 @@ repack_weights_kernel(const float *__restrict__ w, const uint8_t *__restrict__ t
     wp[(static_cast<size_t>(rs - 1 - t) * Kc + co) * C + ci] = v;
 }
 
+// The filters of the three-part kernel: unit ((g*rs + t)*3 + part)*2 + half)*mc_pad + m holds the
+// parts of channels 16g + 8*half .. +7 of row m (zero beyond the tensor), with the sign of step
+// g*rs + t. A thread writes the
+// three units of eight channels.
+__global__ void __launch_bounds__(256)
+x3_pack_kernel(const float *__restrict__ w, const uint8_t *__restrict__ tbl, uint4 *__restrict__ wp,
+               const int C, const int Kc, const int rs, const int flip, const int mc_pad) {
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  const int m = e % mc_pad, rest = e / mc_pad;
+  const int half = rest & 1, t = (rest >> 1) % rs, g = (rest >> 1) / rs;
+  const int KC = flip ? Kc : C, MC = flip ? C : Kc;
+  if (g * 16 >= KC) return;
+  float v[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int kc = 16 * g + 8 * half + k;
+    const int co = flip ? kc : m, ci = flip ? m : kc;
+    const bool in = kc < KC && m < MC && (!tbl || tbl[ci * Kc + co]);
+    v[k] = in ? x3_sign(g * rs + t) * w[(static_cast<size_t>(co) * C + ci) * rs + (flip ? rs - 1 - t : t)] : 0.0f;
+  }
+  uint32_t part[X3_PARTS][4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    uint32_t p3[X3_PARTS];
+    split_pair(v[2 * k], v[2 * k + 1], p3);
+#pragma unroll
+    for (int p = 0; p < X3_PARTS; ++p) part[p][k] = p3[p];
+  }
+#pragma unroll
+  for (int p = 0; p < X3_PARTS; ++p)
+    wp[((static_cast<size_t>(g * rs + t) * X3_PARTS + p) * 2 + half) * mc_pad + m] =
+      make_uint4(part[p][0], part[p][1], part[p][2], part[p][3]);
+}
+
 int pow2_ceil(int v) {
   int p = 1;
   while (p < v) p <<= 1;
@@ -66,8 +103,7 @@ int ilog2(int v) {
 }
 
 // Splits the reduction channels over grid.z when the tiles alone leave most of the chip idle.
-void choose_split(S1Plan &p, int rs, long blocks) {
-  const int kch     = s1_kch(rs, p.tm, p.tn);
+void choose_split(S1Plan &p, int kch, long blocks) {
   const int nchunks = ceil_div(p.args.KC, kch);
   int splits = 1;
   if (blocks < 384 && nchunks >= 4) {
@@ -90,23 +126,30 @@ void choose_split(S1Plan &p, int rs, long blocks) {
 // Candidates run from the largest workgroup tile to the smallest; the first one that yields
 // at least 256 workgroups wins, else the one with the most workgroups, and shapes that cannot
 // even fill a quarter of the chip are left to the split-K GEMM.
-S1Plan make_plan(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph,
-                 int pw) {
+S1Plan make_plan_of(bool x3, int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph,
+                    int pw) {
   S1Plan best;
   best.ok = false;
-  if (!((R == 3 && S == 3) || (R == 5 && S == 5))) return best;
+  best.x3 = x3;
+  if (R != S || !(R == 3 || R == 5 || (x3 && (R == 1 || R == 7)))) return best;
   if (MC < 16 || KC < 8 || OW < 4 || OH < 1 || pw > 4) return best;
   // offsets inside the input are 32-bit
   if (static_cast<long>(batch) * KC * IH * IW >= (1L << 31)) return best;
   static const int cand_wide[3][2]   = {{2, 2}, {2, 1}, {1, 1}};  // MC > 32
   static const int cand_narrow[3][2] = {{1, 4}, {1, 2}, {1, 1}};  // MC <= 32
+  // (three parts: tiles of at least two accumulator blocks a wave, or the filter operands that a
+  // wave reads for every tap are more than its products cover: 16x16 images, 32 -> 32 channels, 5x5,
+  // batch 128: 25 us with one block, 21 in fp32)
+  const int n_cand = !x3 ? 3 : MC > 32 ? 2 : 1;
   long best_blocks = 0;
-  for (int ci = 0; ci < 3; ++ci) {
+  for (int ci = 0; ci < n_cand; ++ci) {
     S1Plan p;
     p.ok = false;
+    p.x3 = x3;
+    const int *narrow = x3 ? cand_narrow[1] : cand_narrow[ci];
     p.tc = OW >= 48 ? 64 : OW >= 24 ? 32 : OW >= 12 ? 16 : 8;
-    p.tm = MC > 32 ? cand_wide[ci][0] : cand_narrow[ci][0];
-    p.tn = MC > 32 ? cand_wide[ci][1] : cand_narrow[ci][1];
+    p.tm = MC > 32 ? cand_wide[ci][0] : narrow[0];
+    p.tn = MC > 32 ? cand_wide[ci][1] : narrow[1];
     const int pix = 128 * p.tn;
     if (pix < p.tc) continue;
     int tr = pix / p.tc;
@@ -121,16 +164,33 @@ S1Plan make_plan(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH
     const int nq     = (3 + p.tc + S - 1 + 3) / 4;
     const int planeq = ti * (tr + R - 1) * nq;
     a.div_rows = FastDiv((tr + R - 1) * nq);
-    const int kch = s1_kch(R * S, p.tm, p.tn);
-    if (ceil_div(planeq, 256 / kch) > s1_niq(R, S, p.tc, p.tm, p.tn)) continue;
-    p.lds_bytes = sizeof(float) * kch * (4 * static_cast<size_t>(planeq) + R * S * 32 * p.tm);
-    if (p.lds_bytes > 150 * 1024) continue;
+    const int kch = x3 ? X3_KCH : s1_kch(R * S, p.tm, p.tn);
+    if (x3) {
+      if (2 * planeq > 256 * x3_items(p.tm, p.tn)) continue;
+      p.lds_bytes = 6 * 16 * 4 * static_cast<size_t>(planeq);
+      if (p.lds_bytes > 80 * 1024) continue;  // two workgroups a compute unit
+      if (static_cast<long>(ti) * KC * IH * IW >= (1L << 29)) continue;  // 32-bit byte offsets inside a tile
+      a.mc_pad = x3_mc_pad(MC);
+    } else {
+      if (ceil_div(planeq, 256 / kch) > s1_niq(R, S, p.tc, p.tm, p.tn)) continue;
+      p.lds_bytes = sizeof(float) * kch * (4 * static_cast<size_t>(planeq) + R * S * 32 * p.tm);
+      if (p.lds_bytes > 150 * 1024) continue;
+    }
     const long tiles  = static_cast<long>(a.tiles_x) * a.tiles_y * ceil_div(batch, ti);
     const long blocks = tiles * ceil_div(MC, 32 * p.tm);
     if (tiles > 2000000000L) continue;
     p.grid = dim3(static_cast<unsigned>(tiles), ceil_div(MC, 32 * p.tm), 1);
     p.ok   = true;
-    choose_split(p, R * S, blocks);
+    if (x3) {
+      // unsplit, and a workgroup for every compute unit at least; two where a single short chunk has
+      // nothing to cover its loads with (32x32 images, 16 -> 32 channels, 3x3, batch 64: 12.6 us with
+      // one a unit, 11.2 in fp32)
+      if (blocks < (KC * R * S < 256 ? 512 : 256)) continue;
+      p.splits = 1;
+      a.kc_split = KC; a.part = nullptr; a.part_stride = 0;
+      return p;
+    }
+    choose_split(p, kch, blocks);
     // short reductions have nothing to overlap their loads with inside a workgroup: ask for
     // more, smaller workgroups then
     if (blocks >= (KC * R * S < 256 ? 1024 : 256)) return p;
@@ -143,6 +203,14 @@ S1Plan make_plan(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH
   return best;
 }
 
+S1Plan make_plan(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw) {
+  if (!ctx().keep_f32) {
+    const S1Plan p = make_plan_of(true, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw);
+    if (p.ok) return p;
+  }
+  return make_plan_of(false, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw);
+}
+
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 }  // namespace
@@ -150,6 +218,14 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 bool conv_s1_applicable(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW,
                         int ph, int pw) {
   return make_plan(R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw).ok;
+}
+
+int conv_s1_packed_kind(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw) {
+  const S1Plan p = make_plan(R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw);
+  return !p.ok ? CONV_PACK_NONE : p.x3 ? CONV_PACK_X3 : CONV_PACK_F32;
+}
+size_t conv_s1_packed_bytes(int kind, int RS, int KC, int MC) {
+  return kind == CONV_PACK_X3 ? x3_pack_bytes(RS, KC, MC) : sizeof(float) * static_cast<size_t>(RS) * KC * MC;
 }
 
 bool conv_s1_single_pass(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW,
@@ -171,19 +247,30 @@ bool conv_s1_fuses_pool(int R, int S, int batch, int KC, int MC, int IH, int IW,
 size_t conv_s1_workspace_bytes(int R, int S, int batch, int C, int Kc, int flip, int IH, int IW,
                                int OH, int OW, int ph, int pw) {
   const int KC = flip ? Kc : C, MC = flip ? C : Kc;
-  const S1Plan p = make_plan(R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw);
-  if (!p.ok) return 0;
-  size_t total = ws_align(sizeof(float) * static_cast<size_t>(R) * S * C * Kc);  // repacked filter
-  if (p.splits > 1) total += ws_align(sizeof(float) * p.splits * p.args.part_stride);
-  return total;
+  size_t most = 0;
+  for (int x3 = 0; x3 < 2; ++x3) {  // (which of the two kernels runs is the caller's choice as well)
+    const S1Plan p = make_plan_of(x3 != 0, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw);
+    if (!p.ok) continue;
+    size_t total = ws_align(conv_s1_packed_bytes(p.x3 ? CONV_PACK_X3 : CONV_PACK_F32, R * S, KC, MC));
+    if (p.splits > 1) total += ws_align(sizeof(float) * p.splits * p.args.part_stride);
+    most = std::max(most, total);
+  }
+  return most;
 }
 
 // wp = the filter in the kernel's layout [tap][kc][m] (R*S*C*Kc floats); flip as in conv_s1_run
 int conv_s1_repack(int R, int S, int C, int Kc, int flip, const float *w, const uint8_t *tbl_dev,
-                   float *wp) {
-  ProfScope prof("conv_repack_weights", 8.0 * R * S * C * Kc, WORK_BYTE);
+                   void *wp, bool x3) {
+  ProfScope prof("conv_repack_weights", (x3 ? 10.0 : 8.0) * R * S * C * Kc, WORK_BYTE);
+  if (x3) {
+    const int KC = flip ? Kc : C, mc_pad = x3_mc_pad(flip ? C : Kc);
+    TDH_LAUNCH(x3_pack_kernel, dim3(ceil_div(ceil_div(KC, 16) * R * S * 2 * mc_pad, 256)), dim3(256), 0, ctx().stream,
+               w, tbl_dev, static_cast<uint4 *>(wp), C, Kc, R * S, flip, mc_pad);
+    TDH_LAUNCH_CHECK();
+    return TDH_OK;
+  }
   TDH_LAUNCH(repack_weights_kernel, dim3(ceil_div(R * S * C * Kc, 256)), dim3(256), 0,
-                     ctx().stream, w, tbl_dev, wp, C, Kc, R * S, flip);
+                     ctx().stream, w, tbl_dev, static_cast<float *>(wp), C, Kc, R * S, flip);
   TDH_LAUNCH_CHECK();
   return TDH_OK;
 }
@@ -193,7 +280,7 @@ int conv_s1_repack(int R, int S, int C, int Kc, int flip, const float *w, const 
 // result of conv_s1_repack for this filter, when the caller already has it (w is not read).
 int conv_s1_run(int R, int S, int batch, int C, int Kc, int flip, const float *in, const float *w,
                 const uint8_t *tbl_dev, const float *bias, float *out, int IH, int IW, int OH,
-                int OW, int ph, int pw, ActGrad ag, const char *tag, const float *prepacked,
+                int OW, int ph, int pw, ActGrad ag, const char *tag, const void *prepacked,
                 float *act_out, int act_kind, const PoolFuse *pool) {
   const int KC = flip ? Kc : C, MC = flip ? C : Kc;
   S1Plan p = make_plan(R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw);
@@ -207,11 +294,11 @@ int conv_s1_run(int R, int S, int batch, int C, int Kc, int flip, const float *i
   const void *wp = prepacked;
   if (!prepacked) {
     void *fresh = nullptr;
-    TDH_TRY(ws_take(sizeof(float) * static_cast<size_t>(R) * S * C * Kc, &fresh));
-    TDH_TRY(conv_s1_repack(R, S, C, Kc, flip, w, tbl_dev, static_cast<float *>(fresh)));
+    TDH_TRY(ws_take(conv_s1_packed_bytes(p.x3 ? CONV_PACK_X3 : CONV_PACK_F32, R * S, KC, MC), &fresh));
+    TDH_TRY(conv_s1_repack(R, S, C, Kc, flip, w, tbl_dev, fresh, p.x3));
     wp = fresh;
   }
-  p.args.in = in; p.args.wp = static_cast<const float *>(wp); p.args.bias = bias;
+  p.args.in = in; p.args.wp = wp; p.args.bias = bias;
   p.args.out = out; p.args.ag = ag;
   p.args.act_out = act_out; p.args.act_kind = act_kind;
   p.args.pool_out     = pool ? pool->out : nullptr;
@@ -224,8 +311,12 @@ int conv_s1_run(int R, int S, int batch, int C, int Kc, int flip, const float *i
   }
   {
     ProfScope prof(pool ? "conv_fwd_s1_pool" : tag, MC, batch * OH * OW, KC * R * S);
-    const bool vec = IW % 4 == 0 && MC % 4 == 0 && aligned16(in) && aligned16(wp);
-    if (vec) TDH_TRY(R == 3 ? s1_launch_3x3_vec(p) : s1_launch_5x5_vec(p));
+    const bool vec = IW % 4 == 0 && aligned16(in) && (p.x3 || (MC % 4 == 0 && aligned16(wp)));
+    if (p.x3 && vec)
+      TDH_TRY(R == 1 ? x3_launch_1_vec(p) : R == 3 ? x3_launch_3_vec(p) : R == 5 ? x3_launch_5_vec(p) : x3_launch_7_vec(p));
+    else if (p.x3)
+      TDH_TRY(R == 1 ? x3_launch_1_scalar(p) : R == 3 ? x3_launch_3_scalar(p) : R == 5 ? x3_launch_5_scalar(p) : x3_launch_7_scalar(p));
+    else if (vec) TDH_TRY(R == 3 ? s1_launch_3x3_vec(p) : s1_launch_5x5_vec(p));
     else TDH_TRY(R == 3 ? s1_launch_3x3_scalar(p) : s1_launch_5x5_scalar(p));
   }
   if (p.splits > 1) {

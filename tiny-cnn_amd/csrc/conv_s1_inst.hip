@@ -29,29 +29,18 @@
 //
 // This file holds the kernel and is compiled four times, -DTDH_S1_PART=0..3: 3x3 and 5x5 windows,
 // each with 16-byte and with scalar loads.
-#include "conv_s1.h"
+#include "conv_s1_epilogue.h"
 #include <type_traits>
 
 namespace tdh {
 
 namespace {
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // a word that does not exist is loaded from here (not const: the loads must stay in the global
 // address space, like those of the tensors)
 __device__ __align__(16) float s1_zero_word[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-
-// the value of lane l ^ 1 (a swap inside lane pairs, done by the DPP path of a move)
-__device__ __forceinline__ float s1_lane_xor1(const float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));
-}
-// the value of lane l ^ X, X = 8 or 16 (a swizzle inside groups of 32 lanes: and 0x1F, or 0, xor X)
-template <int X>
-__device__ __forceinline__ float s1_lane_xor(const float v) {
-  return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (X << 10) | 0x1F));
-}
 
 template <int R, int S, int TC, int TM, int TN, bool VEC>
 __global__ void __launch_bounds__(256, 2) conv_s1_kernel(const ConvS1Args a) {
@@ -174,7 +163,7 @@ __global__ void __launch_bounds__(256, 2) conv_s1_kernel(const ConvS1Args a) {
       }
     }
     const bool wch_ok = w_ok && kc0 + wkc < kc_hi;
-    const float *wb   = a.wp + static_cast<size_t>(kc0 + wkc) * a.MC + m0 + 4 * wm4;
+    const float *wb   = static_cast<const float *>(a.wp) + static_cast<size_t>(kc0 + wkc) * a.MC + m0 + 4 * wm4;
 #pragma unroll
     for (int i = 0; i < NWQ; ++i) {
       if (part >= 0 && ((S1_NIQ + i) * STEPS) / NLOAD != part) continue;
@@ -248,94 +237,7 @@ __global__ void __launch_bounds__(256, 2) conv_s1_kernel(const ConvS1Args a) {
     for (int p0 = PU; p0 < KCH / 2; p0 += PU) mfma_group(p0, 0, std::false_type());
   }
 
-  // ---- epilogue: reg r of lane l holds channel 8*(r/4) + 4*(l/32) + r%4, pixel l%32
-  const int ohw = a.OH * a.OW;
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int q   = (wn * TN + j) * 32 + (lane & 31);
-    const int ti  = q >> (a.log_tr + LOG_TC);
-    const int r   = (q >> LOG_TC) & (a.TR - 1);
-    const int c   = q & (TC - 1);
-    const int img = img0 + ti, oy = y0 + r, ox = x0 + c;
-    if (img >= a.batch || oy >= a.OH || ox >= a.OW) continue;
-    const size_t pbase = static_cast<size_t>(img) * a.MC * ohw + oy * a.OW + ox;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      // the 16 values of this lane: channels mb + 8*(rr/4) + rr%4, all at pixel pbase
-      const int mb = m0 + 32 * i + 4 * (lane >> 5);
-      float *dst = a.part ? a.part + blockIdx.z * a.part_stride : a.out;
-      float v[16];
-#pragma unroll
-      for (int rr = 0; rr < 16; ++rr) v[rr] = acc[i][j][rr];
-      if (!a.part) {
-        if (a.bias) {
-#pragma unroll
-          for (int rr = 0; rr < 16; ++rr) {
-            const int m = mb + 8 * (rr >> 2) + (rr & 3);
-            v[rr] += a.bias[min(m, a.MC - 1)];
-          }
-        }
-        if (a.ag.kind != TDH_ACT_NONE) {
-          // all loads of y first: one at a time they would each cost a trip to memory
-          float yv[16];
-#pragma unroll
-          for (int rr = 0; rr < 16; ++rr) {
-            const int m = mb + 8 * (rr >> 2) + (rr & 3);
-            yv[rr] = a.ag.y[pbase + static_cast<size_t>(min(m, a.MC - 1)) * ohw];
-          }
-#pragma unroll
-          for (int rr = 0; rr < 16; ++rr) v[rr] *= act_grad_factor(a.ag.kind, yv[rr]);
-        }
-      }
-      if (dst) {  // (null: the pool behind leaves this kernel too and nobody reads the convolution's own output)
-#pragma unroll
-        for (int rr = 0; rr < 16; ++rr) {
-          const int m = mb + 8 * (rr >> 2) + (rr & 3);
-          if (m < a.MC) dst[pbase + static_cast<size_t>(m) * ohw] = v[rr];
-        }
-      }
-      if (!a.part && a.act_out) {
-#pragma unroll
-        for (int rr = 0; rr < 16; ++rr) {
-          const int m = mb + 8 * (rr >> 2) + (rr & 3);
-          v[rr]       = act_apply(a.act_kind, v[rr]);
-          if (m < a.MC) a.act_out[pbase + static_cast<size_t>(m) * ohw] = v[rr];
-        }
-      }
-      if constexpr (TC <= 16) {
-        if (!a.part && a.pool_out) {
-          // A 32-pixel block is whole rows of TC pixels, the first one even: the window of the
-          // lane with an even row and column is its own value, lane^1's, lane^TC's and
-          // lane^(TC+1)'s, scanned in that order with strict '>' from lowest()
-          // (maxpool_op_internal.h:17-47). Every lane runs the exchange, the anchors store.
-          const bool anchor = !(lane & 1) && !(lane & TC);
-          const int pw2 = a.OW >> 1, pohw = (a.OH >> 1) * pw2;
-          const size_t pobase = static_cast<size_t>(img) * a.MC * pohw + (oy >> 1) * pw2 + (ox >> 1);
-          const int pix = oy * a.OW + ox;
-#pragma unroll
-          for (int rr = 0; rr < 16; ++rr) {
-            const int m = mb + 8 * (rr >> 2) + (rr & 3);
-            const float right = s1_lane_xor1(v[rr]);
-            const float w4[4] = {v[rr], right, s1_lane_xor<TC>(v[rr]), s1_lane_xor<TC>(right)};
-            float best = -3.402823466e+38f;
-            int sel    = -1;
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-              if (w4[k] > best) {
-                best = w4[k];
-                sel  = k;
-              }
-            if (anchor && m < a.MC) {
-              const size_t at = pobase + static_cast<size_t>(m) * pohw;
-              a.pool_out[at]    = best;
-              a.pool_argmax[at] = sel < 0 ? 0 : m * ohw + pix + (sel >> 1) * a.OW + (sel & 1);
-              if (a.pool_act_out) a.pool_act_out[at] = best > 0.0f ? best : 0.0f;
-            }
-          }
-        }
-      }
-    }
-  }
+  s1_epilogue<TC, TM, TN>(a, acc, wn, lane, img0, y0, x0, m0);
 }
 
 template <int R, int S, int TC, int TM, int TN, bool VEC>

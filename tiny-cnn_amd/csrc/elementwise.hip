@@ -7,6 +7,8 @@
 #include <vector>
 
 #include "common.h"
+#include "conv_s1.h"
+#include "split_bf16.h"
 
 namespace tdh {
 
@@ -429,6 +431,17 @@ int launch_opt(size_t n, const float *g, float *w, float *s0, float *s1, const O
   return TDH_OK;
 }
 
+// the parts of a filter value at (tap, reduction channel kc, row m of mc)
+__device__ __forceinline__ void opt_part_store(uint16_t *wx, const uint32_t rs, const uint32_t tap, const uint32_t kc,
+                                               const uint32_t m, const uint32_t mc, const float v) {
+  const uint32_t step = (kc >> 4) * rs + tap;
+  const size_t pad = x3_mc_pad(mc), unit = step * X3_PARTS;
+  uint32_t part[X3_PARTS];
+  split_pair(x3_sign(step) * v, 0.0f, part);
+#pragma unroll
+  for (int p = 0; p < X3_PARTS; ++p)
+    wx[(((unit + p) * 2 + ((kc >> 3) & 1)) * pad + m) * 8 + (kc & 7)] = static_cast<uint16_t>(part[p]);
+}
 // The packed copies of element e = (co*C + ci)*rs + t of a convolution's weight tensor
 __device__ __forceinline__ void opt_pack_store(const OptTensor &t, const uint32_t e, float v) {
   const uint32_t tap = e % t.rs, pair = e / t.rs;
@@ -436,6 +449,8 @@ __device__ __forceinline__ void opt_pack_store(const OptTensor &t, const uint32_
   if (t.tbl && !t.tbl[ci * t.Kc + co]) v = 0.0f;
   t.wp_fwd[(static_cast<size_t>(tap) * t.C + ci) * t.Kc + co] = v;
   t.wp_dx[(static_cast<size_t>(t.rs - 1 - tap) * t.Kc + co) * t.C + ci] = v;
+  if (t.wx_fwd) opt_part_store(t.wx_fwd, t.rs, tap, ci, co, t.Kc, v);
+  if (t.wx_dx) opt_part_store(t.wx_dx, t.rs, t.rs - 1 - tap, co, ci, t.C, v);
 }
 
 // Multi-tensor form: block b works on tensor j = the table entry whose block range holds b.

@@ -27,6 +27,7 @@ struct tdh_net {
     // filters in the LDS-halo kernels' layout for forward / dX, packed on a side stream at the
     // start of a captured step (stride-1 conv layers of a TDH_NET_GRAPH net)
     float *wp_fwd = nullptr, *wp_dx = nullptr;  // kept current by the optimizer kernel
+    float *wx_fwd = nullptr, *wx_dx = nullptr;  // likewise, in three bf16 parts (directions that read them)
     // batch-norm: running averages, this batch's moments, sqrt(variance + eps); dropout: mask
     float *bn_mean = nullptr, *bn_var = nullptr, *bn_mean_cur = nullptr, *bn_var_cur = nullptr,
           *bn_stddev = nullptr;
@@ -426,6 +427,29 @@ TailPlan plan_tail(tdh_net *net, int loss_kind, int batch) {
   return plan;
 }
 
+// the packed filters that this direction of a layer reads at this batch, or null: it has none, or
+// packs for itself
+const void *packed_filters(const tdh_net::Layer &L, int batch, int flip) {
+  if (!L.wp_fwd) return nullptr;
+  switch (conv_packed_kind(&L.spec.conv, batch, flip)) {
+    case CONV_PACK_F32: return flip ? L.wp_dx : L.wp_fwd;
+    case CONV_PACK_X3: return flip ? L.wx_dx : L.wx_fwd;
+    default: return nullptr;
+  }
+}
+
+// Products inside the scope keep to fp32 instructions (see Context::keep_f32).
+struct KeepF32 {
+  const bool was;
+  explicit KeepF32(bool on) : was(ctx().keep_f32) { ctx().keep_f32 = was || on; }
+  ~KeepF32() { ctx().keep_f32 = was; }
+};
+bool has_batchnorm(const tdh_net *net) {
+  for (const tdh_net::Layer &L : net->layers)
+    if (L.spec.kind == TDH_L_BATCHNORM) return true;
+  return false;
+}
+
 // packed: the layers' wp_fwd hold the current filters in the stride-1 kernels' layout
 // xent_t / xent_dz: the net ends in softmax and the step's loss is cross_entropy_multiclass: the
 // last layer's kernel also writes the loss gradient with respect to the softmax input
@@ -437,6 +461,7 @@ TailPlan plan_tail(tdh_net *net, int loss_kind, int batch) {
 // same kernel) is not written
 int forward(tdh_net *net, int batch, const float *x, bool packed = false, const float *xent_t = nullptr,
             float *xent_dz = nullptr, const TailPlan *tail = nullptr, bool training = false) {
+  const KeepF32 keep(training);
   const float *in = x;
   const int n     = static_cast<int>(net->layers.size());
   net->out_unwritten.assign(n, 0);
@@ -447,7 +472,7 @@ int forward(tdh_net *net, int batch, const float *x, bool packed = false, const 
       case TDH_L_CONV:
         TDH_TRY(ws_begin(conv2d_workspace_bytes(&s.conv, batch)));
       {
-        const float *wp = packed && L.wp_fwd && conv_uses_packed(&s.conv, batch, 0) ? L.wp_fwd : nullptr;
+        const void *wp = packed ? packed_filters(L, batch, 0) : nullptr;
         const bool fuse = (net->flags & TDH_NET_FUSE_ACT_GRAD) != 0;
         auto pointwise = [&](int k) {
           return k < n && net->layers[k].spec.kind == TDH_L_ACT && is_pointwise_act(net->layers[k].spec.act);
@@ -634,6 +659,11 @@ int tdh_net_create(const tdh_layer *layers, int n_layers, int max_batch, int fla
         L.spec.conv.h_stride == 1) {
       if ((rc = net_alloc(net, L.w_size, &L.wp_fwd, false))) break;
       if ((rc = net_alloc(net, L.w_size, &L.wp_dx, false))) break;
+      for (int flip = 0; flip < 2 && rc == TDH_OK; ++flip)
+        if (conv_packed_kind(&L.spec.conv, max_batch, flip) == CONV_PACK_X3)
+          rc = net_alloc(net, conv_packed_bytes(&L.spec.conv, CONV_PACK_X3, flip) / sizeof(float),
+                         flip ? &L.wx_dx : &L.wx_fwd, false);
+      if (rc != TDH_OK) break;
     }
     if (!L.tbl.empty()) {
       float *p = nullptr;
@@ -670,11 +700,14 @@ int tdh_net_create(const tdh_layer *layers, int n_layers, int max_batch, int fla
         if (!n) continue;
         OptTensor t;
         t.wp_fwd = t.wp_dx = nullptr;
+        t.wx_fwd = t.wx_dx = nullptr;
         t.tbl = nullptr;
         t.C = t.Kc = t.rs = 1;
         if (!which && L.wp_fwd) {
           t.wp_fwd = L.wp_fwd;
           t.wp_dx  = L.wp_dx;
+          t.wx_fwd = reinterpret_cast<uint16_t *>(L.wx_fwd);
+          t.wx_dx  = reinterpret_cast<uint16_t *>(L.wx_dx);
           t.tbl    = L.spec.conv.tbl ? L.tbl_dev : nullptr;
           t.C      = static_cast<uint32_t>(L.spec.conv.in_c);
           t.Kc     = static_cast<uint32_t>(L.spec.conv.out_c);
@@ -875,8 +908,11 @@ static int refresh_packs(tdh_net *net) {
   if (!(net->flags & TDH_NET_GRAPH) || net->packs_valid) return TDH_OK;
   for (tdh_net::Layer &L : net->layers) {
     if (!L.wp_fwd) continue;
-    TDH_TRY(conv_pack_filters(&L.spec.conv, 0, L.w, L.tbl_dev, L.wp_fwd));
-    TDH_TRY(conv_pack_filters(&L.spec.conv, 1, L.w, L.tbl_dev, L.wp_dx));
+    for (int flip = 0; flip < 2; ++flip) {
+      TDH_TRY(conv_pack_filters(&L.spec.conv, CONV_PACK_F32, flip, L.w, L.tbl_dev, flip ? L.wp_dx : L.wp_fwd));
+      if (float *wx = flip ? L.wx_dx : L.wx_fwd)
+        TDH_TRY(conv_pack_filters(&L.spec.conv, CONV_PACK_X3, flip, L.w, L.tbl_dev, wx));
+    }
   }
   net->packs_valid = true;
   return TDH_OK;
@@ -897,6 +933,7 @@ int tdh_net_forward(tdh_net *net, int batch, const float *x) {
 static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, const float *x,
                         const float *t, int do_update, const float *powers_in, float *powers_out,
                         bool forked = false) {
+  const KeepF32 keep_f32(has_batchnorm(net));
   if (tiny_step_applies(net, loss_kind)) {
     // a small net: one workgroup per sample runs forward, loss and the input gradients out of
     // LDS, a second launch computes every sample's weight and bias gradients, a third adds
@@ -1047,7 +1084,7 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
         TDH_TRY(ws_begin((forked || as_forked ? 3 : 1) * conv2d_workspace_bytes(&s.conv, batch)));
       {
         const PoolGather *gp = i == through_pool_for ? &through_pool : nullptr;
-        const float *wp = packed && L.wp_dx && conv_uses_packed(&s.conv, batch, 1) ? L.wp_dx : nullptr;
+        const void *wp = packed ? packed_filters(L, batch, 1) : nullptr;
         // the layer that reads this dX next (behind a folded activation) is a max-pool: its
         // backward kernel can add up a split reduction of dX
         const int reader = i - 1 - ((i >= 1 && net->layers[i - 1].grad_folded) ? 1 : 0);
