@@ -1,0 +1,68 @@
+"""The convolution kernels on three-part bf16 operands: against the oracle at the edges of their tiles,
+and against float64, from which they may be no further than a sum in fp32."""
+import numpy as np
+import pytest
+
+from conftest import assert_close
+
+pytestmark = pytest.mark.gpu
+
+
+def run(T, cfg, rng, spread=0.0):
+    iw, ih, ic, k, oc, same, bs = cfg
+    d = T.conv_desc(iw, ih, ic, k, k, oc, pad_same=same)
+    ow, oh = T.conv_out_shape(d)
+    x = rng.standard_normal((bs, ic * ih * iw)).astype(np.float32)
+    w = rng.uniform(-0.3, 0.3, oc * ic * k * k).astype(np.float32)
+    dy = rng.standard_normal((bs, oc * oh * ow)).astype(np.float32)
+    if spread:
+        x *= np.exp(spread * rng.standard_normal(x.shape)).astype(np.float32)
+    b = rng.standard_normal(oc).astype(np.float32)
+    xd, wd, dyd, bd = (T.to_device(a) for a in (x, w, dy, b))
+    y, dx, dw, db = T.DevBuf(dy.shape), T.DevBuf(x.shape), T.DevBuf(w.shape), T.DevBuf((oc,))
+    T.conv2d_fwd(d, bs, xd, wd, bd, y)
+    T.conv2d_bwd(d, bs, xd, wd, dyd, dx, dw, db)
+    return (x, w, b, dy), [a.numpy() for a in (y, dx, dw, db)]
+
+
+@pytest.mark.parametrize("cfg", [
+    # in_w, in_h, in_c, k, out_c, same, batch
+    (64, 12, 16, 3, 64, True, 86),      # one chunk of channels
+    (66, 17, 33, 3, 65, True, 26),      # channels past a chunk and a tile, a second column tile, scalar loads
+    (50, 11, 40, 3, 24, False, 37),     # no padding, fewer than 32 channels in dX
+    (17, 33, 48, 3, 96, True, 33),      # tiles of 16 columns, ragged rows
+    (30, 30, 64, 3, 40, False, 20),     # tiles of 32 columns
+    (8, 8, 32, 5, 64, True, 600),       # several images a tile
+    (16, 16, 32, 5, 20, True, 300),     # 5x5
+    (53, 50, 20, 5, 40, True, 7),       # 5x5, scalar loads: dW by filter-row groups, one of them half empty
+    (49, 50, 34, 5, 33, False, 6),
+    (40, 40, 50, 1, 70, True, 12),      # 1x1
+    (36, 30, 20, 7, 40, True, 12),      # 7x7
+    (128, 4, 64, 3, 64, True, 65),      # images of fewer rows than a slice warms up
+])
+def test_matches_oracle(T, O, cfg):
+    iw, ih, ic, k, oc, same, bs = cfg
+    (x, w, b, dy), got = run(T, cfg, np.random.default_rng(3))
+    do = O.conv_desc(iw, ih, ic, k, k, oc, pad_same=same)
+    want = [O.conv2d_fwd(do, x, w, b), *O.conv2d_bwd(do, x, w, dy)]
+    for g, r, name in zip(got, want, ("y", "dx", "dw", "db")):
+        assert_close(g.ravel(), r.ravel(), what=f"{cfg} {name}")
+
+
+@pytest.mark.parametrize("spread", [0.0, 3.0])
+def test_no_further_from_float64_than_fp32_sums(T, spread):
+    import torch
+    cfg = (64, 64, 32, 3, 64, True, 16)
+    iw, ih, ic, k, oc, _, bs = cfg
+    (x, w, b, dy), got = run(T, cfg, np.random.default_rng(4), spread)
+    xt = torch.from_numpy(x).double().reshape(bs, ic, ih, iw).requires_grad_()
+    wt = torch.from_numpy(w).double().reshape(oc, ic, k, k).requires_grad_()
+    y = torch.nn.functional.conv2d(xt, wt, torch.from_numpy(b).double(), padding=1)
+    y.backward(torch.from_numpy(dy).double().reshape(y.shape))
+    for g, r, name in zip(got, (y, xt.grad, wt.grad), ("y", "dx", "dw")):
+        r = r.detach().numpy().ravel()
+        e = g.ravel().astype(np.float64) - r
+        # (a sum of n products rounded after each: sqrt(n) half-ulps and more; the fp32 kernels
+        # measure 2.2e-7 to 3.0e-7 here)
+        assert np.linalg.norm(e) <= 2.0e-7 * np.linalg.norm(r), (name, np.linalg.norm(e) / np.linalg.norm(r))
+        assert abs(e.mean()) <= 2e-8 * np.sqrt(np.mean(r * r)), (name, e.mean())

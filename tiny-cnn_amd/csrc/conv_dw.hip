@@ -35,6 +35,7 @@
 // WORKGROUPS (grid z = channel block x filter row) and the kernel runs as a 1x5 window whose
 // input rows are shifted by the filter row. Such a window needs no halo rows, so on small
 // images a chunk holds TI whole images stacked as rows.
+#include "conv_dwx.h"
 #include "gemm_mfma.h"
 
 namespace tdh {
@@ -724,21 +725,81 @@ int launch_dw_vec(const DwHaloPlan &p) {
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// The three-part kernel of conv_dwx_inst.hip. It takes most of a compute unit's LDS, so the channel tiles x columns x filter-row groups x slices are chosen to come out just
+// under a whole number of rounds of the 256 units; a slice keeps at least four steps for its
+// prologue and partial tile. Two blocks of 32 channels on one side at least: with 32 x 32 half of
+// every tile would be empty.
+DwxPlan make_dwx_plan(int R, int S, int batch, int C, int Kc, int H, int W, int OH, int OW, int ph, int pw) {
+  DwxPlan p;
+  p.ok = false;
+  if (ctx().keep_f32 || R != S || (R != 3 && R != 5) || ph != pw || (pw != 0 && pw != R / 2)) return p;
+  if (C < 16 || Kc < 16 || (C <= 32 && Kc <= 32) || OW < 12) return p;
+  if (static_cast<long>(C) * H * W >= (1L << 29) || static_cast<long>(Kc) * OH * OW >= (1L << 29)) return p;
+  p.tc  = OW >= 48 ? 64 : OW >= 24 ? 32 : 16;
+  // Rows that fill less than four fifths of a narrow tile are better off with the fp32 kernel, whose
+  // steps cost less (24x24 images, 64 -> 64, batch 100: 60 us there, 63 here; 28x28, 48 -> 96, batch
+  // 50: 68 and 55). A 5x5 window goes through three groups of two filter rows, one of the six rows
+  // empty: ahead only where the fp32 kernel has to load float by float (45x45, 33 -> 70, batch 19: 241
+  // and 148; 64x64, 32 -> 64, batch 16: 72 and 73).
+  if (p.tc < 64 && 5 * OW < 4 * p.tc * ceil_div(OW, p.tc)) return p;
+  if (R == 5 && (p.tc < 64 || (W % 4 == 0 && OW % 4 == 0))) return p;
+  p.cob = Kc > 32 ? 2 : 1;
+  p.cib = C > 32 ? 2 : 1;
+  const int rw = R == 3 ? 3 : 2, rps = 64 / p.tc;
+  DwxArgs &a = p.args;
+  a.batch = batch; a.C = C; a.Kc = Kc; a.H = H; a.W = W; a.OH = OH; a.OW = OW; a.ph = ph; a.pw = pw;
+  a.R = R; a.RS = R * S;
+  a.pwa   = (pw + 3) & ~3;
+  p.shift = a.pwa - pw;
+  a.tiles_x   = ceil_div(OW, p.tc);
+  a.co_tiles  = ceil_div(Kc, 32 * p.cob);
+  a.ci_tiles  = ceil_div(C, 32 * p.cib);
+  a.fy_groups = ceil_div(R, rw);
+  a.chunks_per_image = ceil_div(OH, rps);
+  a.chunks_total     = batch * a.chunks_per_image;
+  const int base     = a.tiles_x * a.co_tiles * a.ci_tiles * a.fy_groups;
+  const int most     = a.chunks_total / 4;
+  if (static_cast<long>(base) * most < 192 || base > 4096) return p;
+  int slices = 1;
+  double best = 0.0;
+  for (int s = 1; s <= most && (s == 1 || base * s <= 512); ++s) {
+    const int rounds  = ceil_div(base * s, 256);
+    const double fill = base * s / (256.0 * rounds) - 0.02 * rounds;
+    if (fill > best) {
+      best   = fill;
+      slices = s;
+    }
+  }
+  a.chunks_per_slice = ceil_div(a.chunks_total, slices);
+  p.slices     = ceil_div(a.chunks_total, a.chunks_per_slice);
+  p.workgroups = base * p.slices;
+  const size_t stage = 2u * 3 * (static_cast<size_t>(rw - 1 + rps) * 32 * p.cib * 4 * dwx_words(p.tc, S) + 32u * p.cob * 72);
+  const int blocks   = p.cob * p.cib, shares = 4 / blocks;
+  const size_t sums  = static_cast<size_t>(shares - 1) * blocks * rw * S * 16 * 64 * sizeof(float);
+  p.lds_bytes = std::max(stage, sums);
+  p.ok = p.lds_bytes <= 160 * 1024;
+  return p;
+}
+int dwx_slices(const DwxPlan &p) { return p.slices * p.args.tiles_x; }
+
 }  // namespace
 
 bool conv_dw_halo_applicable(int R, int S, int batch, int C, int Kc, int H, int W, int OH, int OW,
                              int ph, int pw) {
-  return make_dw_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw).ok;
+  return make_dwx_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw).ok ||
+         make_dw_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw).ok;
 }
 
 size_t conv_dw_halo_workspace_bytes(int R, int S, int batch, int C, int Kc, int H, int W, int OH,
                                     int OW, int ph, int pw) {
+  const DwxPlan x3   = make_dwx_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
   const DwHaloPlan p = make_dw_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
-  if (!p.ok) return 0;
+  if (!p.ok && !x3.ok) return 0;
   // (tensors that are not 16-byte aligned take the general kernel's plan where the 8x8-image
   // kernel would run: room for whichever has more slices)
-  const DwHaloPlan q = p.img8 ? make_dw_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw, false) : p;
-  const size_t slices = std::max(p.grid.x, q.ok ? q.grid.x : 0u);
+  const DwHaloPlan q = p.ok && p.img8 ? make_dw_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw, false) : p;
+  size_t slices = std::max(p.ok ? p.grid.x : 0u, q.ok ? q.grid.x : 0u);
+  if (x3.ok) slices = std::max(slices, static_cast<size_t>(dwx_slices(x3)));
   return ws_align(sizeof(float) * slices * Kc * C * R * S) + ws_align(sizeof(float) * slices * Kc);
 }
 
@@ -747,19 +808,22 @@ int conv_dw_halo_run(int R, int S, int batch, int C, int Kc, const float *x, con
                      float *dw, int H, int W, int OH, int OW, int ph, int pw, int accumulate,
                      float *db) {
   const bool vec = W % 4 == 0 && OW % 4 == 0 && aligned16(x) && aligned16(dy);
+  DwxPlan x3   = make_dwx_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
   DwHaloPlan p = make_dw_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw, /*allow_img8=*/vec);
-  if (!p.ok) return set_error(TDH_ERR_INVALID, "conv_dw_halo_run: shape not supported");
-  const int crs = C * R * S;
-  void *part = nullptr;
-  TDH_TRY(ws_take(sizeof(float) * static_cast<size_t>(p.grid.x) * Kc * crs, &part));
-  p.args.x = x; p.args.dy = dy; p.args.partial = static_cast<float *>(part);
-  p.args.partial_db = nullptr;
-  if (db) {
-    void *part_db = nullptr;
-    TDH_TRY(ws_take(sizeof(float) * static_cast<size_t>(p.grid.x) * Kc, &part_db));
-    p.args.partial_db = static_cast<float *>(part_db);
-  }
+  if (!p.ok && !x3.ok) return set_error(TDH_ERR_INVALID, "conv_dw_halo_run: shape not supported");
+  const int crs = C * R * S, slices = x3.ok ? dwx_slices(x3) : static_cast<int>(p.grid.x);
+  void *part = nullptr, *part_db = nullptr;
+  TDH_TRY(ws_take(sizeof(float) * static_cast<size_t>(slices) * Kc * crs, &part));
+  if (db) TDH_TRY(ws_take(sizeof(float) * static_cast<size_t>(slices) * Kc, &part_db));
+  if (x3.ok) {
+    x3.args.x = x; x3.args.dy = dy;
+    x3.args.partial = static_cast<float *>(part); x3.args.partial_db = static_cast<float *>(part_db);
+    ProfScope prof(db ? "conv_dw_db_x3" : "conv_dw_x3", Kc, crs, batch * OH * OW);
+    TDH_TRY(R == 5 ? dwx_launch_5_scalar(x3) : vec ? dwx_launch_3_vec(x3) : dwx_launch_3_scalar(x3));
+  } else
   {
+    p.args.x = x; p.args.dy = dy; p.args.partial = static_cast<float *>(part);
+    p.args.partial_db = static_cast<float *>(part_db);
     ProfScope prof(db ? "conv_dw_db_halo" : "conv_dw_halo", Kc, crs, batch * OH * OW);
     if (p.img8) {
       p.i8.x = x; p.i8.dy = dy; p.i8.partial = p.args.partial; p.i8.partial_db = p.args.partial_db;
@@ -780,15 +844,14 @@ int conv_dw_halo_run(int R, int S, int batch, int C, int Kc, const float *x, con
       TDH_TRY(launch_dw_vec<false>(p));
     }
   }
-  const int slices = static_cast<int>(p.grid.x);
   EpiRowMajor epi{dw, crs, nullptr, ActGrad(), accumulate};
   EpiRowMajor epi_b{db, 1, nullptr, ActGrad(), accumulate};
   // the two reductions leave as one launch: collected by the train step, or here
   const bool collect_here = !ctx().defer_reduce;
   if (collect_here) flush_deferred_reduces(false);  // nothing may be left from a failed call
   ctx().defer_reduce = true;
-  defer_reduce(p.args.partial, slices, Kc, crs, epi);
-  if (db) defer_reduce(p.args.partial_db, slices, Kc, 1, epi_b);
+  defer_reduce(static_cast<const float *>(part), slices, Kc, crs, epi);
+  if (db) defer_reduce(static_cast<const float *>(part_db), slices, Kc, 1, epi_b);
   if (!collect_here) return TDH_OK;
   ctx().defer_reduce = false;
   return flush_deferred_reduces();
