@@ -1,4 +1,4 @@
-"""The convolution kernels on three-part bf16 operands: against the oracle at the edges of their tiles,
+"""The convolution and fully-connected kernels on three-part bf16 operands: against the oracle at the edges of their tiles,
 and against float64, from which they may be no further than a sum in fp32."""
 import numpy as np
 import pytest
@@ -47,6 +47,36 @@ def test_matches_oracle(T, O, cfg):
     want = [O.conv2d_fwd(do, x, w, b), *O.conv2d_bwd(do, x, w, dy)]
     for g, r, name in zip(got, want, ("y", "dx", "dw", "db")):
         assert_close(g.ravel(), r.ravel(), what=f"{cfg} {name}")
+
+
+@pytest.mark.parametrize("cfg", [
+    # in, out, batch
+    (4096, 1024, 64),      # tiles of 64 rows
+    (1028, 1012, 260),     # ragged on every side, a last step of four indices
+    (2048, 64, 512),       # tiles of 64 columns
+    (16384, 68, 132),      # a reduction of two steps and four indices
+])
+def test_fc_matches_oracle(T, O, W, cfg):
+    """dX as an operator, the forward product as a net's inference."""
+    ni, no, bs = cfg
+    rng = np.random.default_rng(6)
+    x = rng.standard_normal((bs, ni)).astype(np.float32)
+    w = rng.uniform(-0.2, 0.2, ni * no).astype(np.float32)
+    b = rng.standard_normal(no).astype(np.float32)
+    dy = rng.standard_normal((bs, no)).astype(np.float32)
+    xd, dx = T.to_device(x), T.DevBuf(x.shape)
+    T.fc_bwd(ni, no, True, bs, xd, T.to_device(w), T.to_device(dy), dx, None, None)
+    assert_close(dx.numpy(), O.fc_bwd(x, w, dy)[0], what=f"{cfg} dx")
+    want = O.fc_fwd(x, w, b)
+    for flags, act in ((0, False), (T.NET_FUSE_ACT_GRAD, True)):
+        spec = [("fc", ni, no)] + ([("act", "relu")] if act else [])
+        net = T.Net(W.build_layers(T, spec), bs, flags)
+        net.set_param(0, 0, w); net.set_param(0, 1, b)
+        net.forward(bs, xd)
+        assert_close(net.layer_out(0, bs), want, what=f"{cfg} y")
+        if act:
+            assert_close(net.layer_out(1, bs), np.maximum(want, 0), what=f"{cfg} relu")
+        net.close()
 
 
 @pytest.mark.parametrize("spread", [0.0, 3.0])

@@ -42,6 +42,9 @@ struct Context {
   //  - its forward pass decides signs (relu) and maxima (max-pool), and with them where whole
   //    gradients go: one choice in a million changes, and the input gradient of the VGG-style
   //    stack by 1.6e-3 with it;
+  //    (A fully-connected product called as an operator may be the forward half of such a step: every
+  //    bias gradient hangs on its last bits through the activation behind it, and Adam makes a full
+  //    step of one that is nearly zero.)
   //  - the bias gradient of a convolution in front of a batch normalization is zero but for its
   //    rounding, and an optimizer that divides by the gradient's size makes full steps of that.
   bool keep_f32 = false;
@@ -58,6 +61,12 @@ struct StreamSwap {
 };
 
 Context &ctx();
+// Products inside the scope keep to fp32 instructions (see Context::keep_f32).
+struct KeepF32 {
+  const bool was;
+  explicit KeepF32(bool on) : was(ctx().keep_f32) { ctx().keep_f32 = was || on; }
+  ~KeepF32() { ctx().keep_f32 = was; }
+};
 int set_error(int code, const char *fmt, ...);
 // Makes sure the scratch buffer holds `total` bytes and rewinds it. Growing frees and
 // reallocates (hipFree waits for queued kernels), which is refused while ws_locked.

@@ -193,6 +193,15 @@ __device__ __forceinline__ const Op &bind_tile(const Op &op, int) { return op; }
 template <class Op>
 __device__ __forceinline__ int tile_k(const Op &, int, int K) { return K; }
 
+// fc_x3.hip: products of plain matrices with three-part operands, A rows along k, B rows along k or
+// n; lda, ldb: floats from row to row
+bool fc_x3_applies(int M, int N, int K, const float *A, const float *B, int lda, int ldb);
+size_t fc_x3_workspace_bytes(int M, int N, int K);
+int fc_x3_run(bool b_along_k, const float *A, const float *B, int lda, int ldb, const EpiRowMajor &epi, int M, int N, int K,
+              const char *tag, const char *reduce_tag);
+int fc_x3_run_act(const float *A, const float *B, int lda, int ldb, const EpiRowMajorAct &epi, int M, int N, int K,
+                  const char *tag, const char *reduce_tag);
+
 // --------------------------------------------------------------------- kernel
 template <int BM, int BN, int WM, int WN, bool A_LANE_K, bool B_LANE_K, bool A_VEC, bool B_VEC,
           class AOp, class BOp, class Epi>
@@ -703,6 +712,22 @@ int launch_gemm_tile(const AOp &a, const BOp &b, const Epi &epi, int M, int N, i
   return TDH_OK;
 }
 
+// adds up the partial tiles of a split product (or records the sum, see defer_reduce)
+template <class Epi>
+int launch_splitk_reduce(const float *partial, int splits, int M, int N, const Epi &epi, const char *reduce_tag) {
+  // reads every partial tile once and writes the result once
+  if (defer_reduce(partial, splits, M, N, epi)) return TDH_OK;
+  ProfScope prof(reduce_tag, 4.0 * M * N * (splits + 1), WORK_BYTE);
+  if (N % 4 == 0 && static_cast<long>(M) * N >= REDUCE_WIDE_MIN && (reinterpret_cast<uintptr_t>(partial) & 15u) == 0)
+    TDH_LAUNCH((splitk_reduce_wide_kernel<Epi>), dim3(static_cast<unsigned>(ceil_div_sz(static_cast<size_t>(M) * N / 4, 256))),
+               dim3(256), 0, ctx().stream, partial, splits, M, N, epi);
+  else
+    TDH_LAUNCH((splitk_reduce_kernel<Epi>), dim3(ceil_div(M * N, REDUCE_OUTPUTS)), dim3(256), 0,
+               ctx().stream, partial, splits, M, N, epi);
+  TDH_LAUNCH_CHECK();
+  return TDH_OK;
+}
+
 // A_VEC / B_VEC: the operand provides load4k (LANE_K) or load4m (otherwise) and its layout
 // allows groups of four; used by the tiles wide enough for it (the rest stage scalars).
 template <bool A_LANE_K, bool B_LANE_K, bool A_VEC = false, bool B_VEC = false, class AOp,
@@ -738,20 +763,7 @@ int launch_gemm(const AOp &a, const BOp &b, const Epi &epi, int M, int N, int K,
   }
 #undef TDH_TILE
   TDH_TRY(rc);
-  if (p.splits > 1) {
-    // reads every partial tile once and writes the result once
-    if (defer_reduce(partial, p.splits, M, N, epi)) return TDH_OK;
-    ProfScope prof(reduce_tag, 4.0 * M * N * (p.splits + 1), WORK_BYTE);
-    if (N % 4 == 0 && static_cast<long>(M) * N >= REDUCE_WIDE_MIN &&
-        (reinterpret_cast<uintptr_t>(partial) & 15u) == 0)
-      TDH_LAUNCH((splitk_reduce_wide_kernel<Epi>), dim3(static_cast<unsigned>(ceil_div_sz(static_cast<size_t>(M) * N / 4, 256))),
-                 dim3(256), 0, ctx().stream, partial, p.splits, M, N, epi);
-    else
-      TDH_LAUNCH((splitk_reduce_kernel<Epi>), dim3(ceil_div(M * N, REDUCE_OUTPUTS)), dim3(256), 0,
-                 ctx().stream, partial, p.splits, M, N, epi);
-    TDH_LAUNCH_CHECK();
-  }
-  return TDH_OK;
+  return p.splits > 1 ? launch_splitk_reduce(partial, p.splits, M, N, epi, reduce_tag) : TDH_OK;
 }
 
 }  // namespace tdh

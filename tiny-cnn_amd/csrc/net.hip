@@ -438,12 +438,6 @@ const void *packed_filters(const tdh_net::Layer &L, int batch, int flip) {
   }
 }
 
-// Products inside the scope keep to fp32 instructions (see Context::keep_f32).
-struct KeepF32 {
-  const bool was;
-  explicit KeepF32(bool on) : was(ctx().keep_f32) { ctx().keep_f32 = was || on; }
-  ~KeepF32() { ctx().keep_f32 = was; }
-};
 bool has_batchnorm(const tdh_net *net) {
   for (const tdh_net::Layer &L : net->layers)
     if (L.spec.kind == TDH_L_BATCHNORM) return true;

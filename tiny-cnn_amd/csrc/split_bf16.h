@@ -47,11 +47,11 @@ __device__ __forceinline__ void split_pair(const float a, const float b, uint32_
   part[2]        = pack_bf16(ra - low_bf16(part[1]), rb - high_bf16(part[1]));
 }
 
-// acc[i][j] += sign * (a[i] * b[j]) over the 16 reduction indices of one step, smallest products
+// acc[i][j] += sign * (a[i] * b[j]) over the 16*KS reduction indices of KS steps, smallest products
 // first; sign is 1 or -1
-template <int TM, int TN>
-__device__ __forceinline__ void mfma_x3(floatx16_x3 (&acc)[TM][TN], const bf16x8 (&a)[TM][X3_PARTS],
-                                        const bf16x8 (&b)[TN][X3_PARTS], const float sign) {
+template <int TM, int TN, int KS>
+__device__ __forceinline__ void mfma_x3(floatx16_x3 (&acc)[TM][TN], const bf16x8 (&a)[KS][TM][X3_PARTS],
+                                        const bf16x8 (&b)[KS][TN][X3_PARTS], const float sign) {
   constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
@@ -61,8 +61,10 @@ __device__ __forceinline__ void mfma_x3(floatx16_x3 (&acc)[TM][TN], const bf16x8
 #pragma unroll
     for (int q = 0; q < 6; ++q)
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
-        sum[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][pa[q]], b[j][pb[q]], sum[j], 0, 0, 0);
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          sum[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s][i][pa[q]], b[s][j][pb[q]], sum[j], 0, 0, 0);
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
 #pragma unroll
@@ -70,6 +72,12 @@ __device__ __forceinline__ void mfma_x3(floatx16_x3 (&acc)[TM][TN], const bf16x8
       asm volatile("" : "+v"(acc[i][j]));  // (here and now: deferred, the sums pile up in memory)
     }
   }
+}
+template <int TM, int TN>
+__device__ __forceinline__ void mfma_x3(floatx16_x3 (&acc)[TM][TN], const bf16x8 (&a)[TM][X3_PARTS],
+                                        const bf16x8 (&b)[TN][X3_PARTS], const float sign) {
+  mfma_x3<TM, TN, 1>(acc, reinterpret_cast<const bf16x8(&)[1][TM][X3_PARTS]>(a),
+                     reinterpret_cast<const bf16x8(&)[1][TN][X3_PARTS]>(b), sign);
 }
 
 }  // namespace
