@@ -1381,7 +1381,13 @@ bool conv_bwd_one_launch(const tdh_conv_desc *d, int batch, bool pooled) {
   return one_launch_band(d, make_geom(d), batch, pooled) > 0;
 }
 
-// the slices of that launch: one per band and image
+bool conv_bwd_pairs(const tdh_conv_desc *d, int batch) {
+  const ConvGeom g = make_geom(d);
+  return !d->tbl && g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 &&
+         conv_bwd_pair_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
+}
+
+// the slices of the first convolution's launch: one per band and image
 static size_t first_both_workspace_bytes(const tdh_conv_desc *d, const ConvGeom &g, int batch) {
   size_t most = 0;
   for (int pooled = 0; pooled < 2; ++pooled) {
@@ -1466,6 +1472,9 @@ int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
                                 one_launch_band(d, g, batch, true)));
     return TDH_OK;
   }
+  if (dx && dw && conv_bwd_pairs(d, batch) && !((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy)) & 15))
+    return conv_bwd_pair_run(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.pad_h, g.pad_w, x, dy, w, prepacked_dx, dx, dx_act,
+                             dw, db, accumulate);
   if (dx && prepacked_dx) {
     TDH_TRY(conv_s1_run(g.R, g.S, batch, g.C, g.Kc, 1, dy, w, nullptr, nullptr, dx, g.OH, g.OW, g.H,
                         g.W, g.R - 1 - g.pad_h, g.S - 1 - g.pad_w, dx_act, "conv_dx_s1", prepacked_dx));

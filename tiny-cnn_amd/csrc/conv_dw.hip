@@ -35,6 +35,7 @@
 // WORKGROUPS (grid z = channel block x filter row) and the kernel runs as a 1x5 window whose
 // input rows are shifted by the filter row. Such a window needs no halo rows, so on small
 // images a chunk holds TI whole images stacked as rows.
+#include "conv_dw_img.h"
 #include "conv_dwx.h"
 #include "gemm_mfma.h"
 
@@ -372,222 +373,15 @@ __global__ void __launch_bounds__(64 * WCO * WK * WFY, 1) conv_dw_halo_kernel(co
 }
 
 
-// ---- 5x5 windows (padding 2, stride 1) on 8x8 images: every filter row in one workgroup
-//
-// The kernel above gives such a layer workgroups of (one filter row) x (two chunks of images):
-// 1280 wave-sized pieces of 160 MFMAs for 1024 SIMDs, so some SIMD runs two whatever the split,
-// five workgroups stage the same tiles, and a wave's slice leaves as 80 scattered 4-byte stores.
-// Here a workgroup owns 32 output channels x 32 input channels x one of FOUR GROUPS OF TAPS
-// (7 + 6 + 6 + 6 of the 25, each group lies in two filter rows) for a run of chunks of four
-// images; its four waves take one image each, so a wave's piece is 224 (or 192) MFMAs and a
-// 32 -> 64-channel layer at batch 128 is 256 workgroups of one chunk: every SIMD gets one wave.
-// An image is staged whole with its zero frame (12 x 12 per channel), so the X fragment of
-// output row oy and filter row fy is two 16-byte reads, eight floats, that serve all five taps
-// of the row; a dY fragment (one 16-byte read per output row) serves all taps of the group.
-// The pixel pairing is the one of the kernel above: k = 0 lanes take the left half of a row,
-// k = 1 lanes the right half. The four waves' sums meet in LDS (pairwise, image order), and the
-// whole workgroup stores the slice. The bias gradient comes from the workgroups of tap group 0
-// and input-channel block 0, out of the dY they stage anyway.
-//
-// 16x16 images (IS = 16) run the same way with ONE image a chunk: a wave takes four of its rows,
-// 64 pixels again, as eight groups of eight; with more than one chunk a workgroup the next
-// chunk's words travel while the current one is multiplied.
-constexpr int I8_NT  = 256;
-constexpr int I8_DYP = 4 * 64 + 4;    // floats per staged dY channel: 256 pixels (4 mod 64)
-// geometry of a chunk for images of IS x IS pixels
-template <int IS> struct I8Geom {
-  static constexpr int IPC   = IS == 8 ? 4 : 1;              // images a chunk
-  static constexpr int FP    = IS + 4;                       // framed row
-  static constexpr int XP    = IPC * FP * FP + 4;            // floats per staged X channel (4 mod 32 / 20 mod 32)
-  static constexpr int WAVEX = IS == 8 ? FP * FP : 4 * FP;   // a wave's first framed row: its image / its four rows
-  static constexpr int LDS_FLOATS = 32 * I8_DYP + 32 * XP;
-};
-
-struct DwImg8Args {
-  const float *x, *dy;
-  float *partial;      // [slices][Kc][C*25]
-  float *partial_db;   // [slices][Kc], or null
-  int batch, C, Kc;
-  int chunks_total, chunks_per_slice;   // chunks of four images
-  int co_blocks, ci_blocks;
-};
-
-// tap group G: taps T0 .. T0+N-1 of the 25 (tap = 5*fy + fx)
-template <int G> struct I8Taps {
-  static constexpr int T0 = G == 0 ? 0 : G == 1 ? 7 : G == 2 ? 13 : 19;
-  static constexpr int N  = G == 0 ? 7 : 6;
-  static constexpr int FY0 = T0 / 5, FY1 = (T0 + N - 1) / 5;
-};
-
-// the products of the wave's 64 pixels (eight groups of eight: an image's rows, or halves of four
-// rows) for tap group G: acc[t - T0] += dY x X shifted by tap t
-template <int G, int IS>
-__device__ __forceinline__ void img8_products(const float *ap, const float *bp, floatx16 (&acc)[7]) {
-  using TG = I8Taps<G>;
-  constexpr int FP = I8Geom<IS>::FP;
-#pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    const int oy = IS == 8 ? u : u >> 1, ox = IS == 8 ? 0 : 8 * (u & 1);
-    const floatx4 a4 = *reinterpret_cast<const floatx4 *>(ap + u * 8);
-    const float av[4] = {a4.x, a4.y, a4.z, a4.w};
-#pragma unroll
-    for (int fy = TG::FY0; fy <= TG::FY1; ++fy) {
-      const floatx4 b0 = *reinterpret_cast<const floatx4 *>(bp + (oy + fy) * FP + ox);
-      const floatx4 b1 = *reinterpret_cast<const floatx4 *>(bp + (oy + fy) * FP + ox + 4);
-      const float bv[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
-#pragma unroll
-      for (int fx = 0; fx < 5; ++fx) {
-        const int t = 5 * fy + fx - TG::T0;
-        if (t < 0 || t >= TG::N) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[j], bv[j + fx], acc[t], 0, 0, 0);
-      }
-    }
-  }
-}
-
+// 5x5 windows on 8x8 and 16x16 images (conv_dw_img.h)
 template <int IS>
-__global__ void __launch_bounds__(I8_NT, 1) conv_dw_img8_kernel(const DwImg8Args a) {
-  using GE = I8Geom<IS>;
-  constexpr int I8_XP = GE::XP, IPC = GE::IPC, FP = GE::FP, PIX = IS * IS;
+__global__ void __launch_bounds__(DWI_NT, 2) conv_dw_img_kernel(const DwImgArgs a) {
   extern __shared__ __align__(16) float smem[];
-  float *dy_l = smem;                 // [32][I8_DYP]
-  float *x_l  = smem + 32 * I8_DYP;   // [32][I8_XP], frames of zeros around the images
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // workgroups that read the same tiles (the four tap groups and the output-channel blocks of a
-  // slice) are neighbours after the renumbering, and so share an XCD's L2
-  int id = xcd_compact_id(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
-  const int grp = id & 3;
-  id >>= 2;
-  const int cob = id % a.co_blocks;
-  id /= a.co_blocks;
-  const int cib = id % a.ci_blocks, slice = id / a.ci_blocks;
-  const int co0 = cob * 32, ci0 = cib * 32;
-  const int kohw = a.Kc * PIX, chw = a.C * PIX;
-
-  floatx16 acc[7];
-#pragma unroll
-  for (int t = 0; t < 7; ++t)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[t][r] = 0.0f;
-  const bool sums_dy = a.partial_db != nullptr && grp == 0 && cib == 0;
-  float dbs = 0.0f;   // this thread's share of the bias gradient of channel tid / 8
-
-  // fragment bases: A lane = (output channel l%32, half l/32), B lane = (input channel l%32, half)
-  const float *ap = dy_l + (lane & 31) * I8_DYP + wave * 64 + 4 * (lane >> 5);
-  const float *bp = x_l + (lane & 31) * I8_XP + wave * GE::WAVEX + 4 * (lane >> 5);
-
-  const int c_begin = slice * a.chunks_per_slice;
-  const int c_end   = min(a.chunks_total, c_begin + a.chunks_per_slice);
-  // ---- staging: a thread moves eight 16-byte words of dY and eight of X per chunk, all loads
-  //      asked for before the first store (an image past the batch reads image 0 and is stored
-  //      as zeros). Word e: IS = 8: image e / 512 of the chunk's four, channel (e / 16) % 32,
-  //      word e % 16 of its 64 pixels; IS = 16: channel e / 64, word e % 64 of the image.
-  floatx4 rdy[8], rx[8];
-  auto fetch = [&](int chunk) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int e = tid + I8_NT * i;
-      const int im = IS == 8 ? e >> 9 : 0, c = IS == 8 ? (e >> 4) & 31 : e >> 6, q = IS == 8 ? e & 15 : e & 63;
-      const int img = chunk * IPC + im;
-      const size_t ig = img < a.batch ? img : 0;
-      rdy[i] = *reinterpret_cast<const floatx4 *>(a.dy + ig * kohw + static_cast<size_t>(co0 + c) * PIX + 4 * q);
-      rx[i]  = *reinterpret_cast<const floatx4 *>(a.x + ig * chw + static_cast<size_t>(ci0 + c) * PIX + 4 * q);
-    }
-  };
-  fetch(c_begin);
-  for (int chunk = c_begin; chunk < c_end; ++chunk) {
-    if (chunk == c_begin) {   // the frames of zeros, written while the first loads are on their way
-      for (int i = tid; i < 32 * I8_XP / 4; i += I8_NT) reinterpret_cast<floatx4 *>(x_l)[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-    }
-    __syncthreads();   // (the previous chunk's fragments have been read; the first time: the zeros are in place)
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int e = tid + I8_NT * i;
-      const int im = IS == 8 ? e >> 9 : 0, c = IS == 8 ? (e >> 4) & 31 : e >> 6, q = IS == 8 ? e & 15 : e & 63;
-      const bool on = chunk * IPC + im < a.batch;
-      const floatx4 z = floatx4{0.f, 0.f, 0.f, 0.f};
-      *reinterpret_cast<floatx4 *>(dy_l + c * I8_DYP + im * 64 + 4 * q) = on ? rdy[i] : z;
-      // X row, word of the row -> framed row + 2, columns 2 + 4 * word .. + 3 (8-byte aligned)
-      constexpr int WPR = IS / 4;   // words per image row
-      const floatx4 v = on ? rx[i] : z;
-      float *d = x_l + c * I8_XP + im * (FP * FP) + ((q / WPR) + 2) * FP + 2 + 4 * (q % WPR);
-      *reinterpret_cast<float2 *>(d)     = make_float2(v.x, v.y);
-      *reinterpret_cast<float2 *>(d + 2) = make_float2(v.z, v.w);
-    }
-    __syncthreads();
-    if (chunk + 1 < c_end) fetch(chunk + 1);   // (travels while this chunk is multiplied)
-    if (sums_dy) {   // channel tid/8, floats (tid%8)*32 .. +31 of its 256 pixels
-      const floatx4 *row = reinterpret_cast<const floatx4 *>(dy_l + (tid >> 3) * I8_DYP + (tid & 7) * 32);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const floatx4 v = row[k];
-        dbs += (v.x + v.y) + (v.z + v.w);
-      }
-    }
-    switch (grp) {
-      case 0: img8_products<0, IS>(ap, bp, acc); break;
-      case 1: img8_products<1, IS>(ap, bp, acc); break;
-      case 2: img8_products<2, IS>(ap, bp, acc); break;
-      default: img8_products<3, IS>(ap, bp, acc); break;
-    }
-  }
-
-  // ---- the four images' sums, pairwise in image order: (0 + 2) + (1 + 3). Waves 2 and 3 park
-  //      their sums, waves 0 and 1 add them to their own and park the two results transposed,
-  //      [output channel][input channel][tap] (rows of nine floats: no two lanes of a store share
-  //      a bank), and the whole workgroup adds those two and stores: a lane's neighbours then
-  //      write neighbouring taps and input channels, seven cache lines a store instead of 64.
-  float *red = smem;   // [2][7*16][64], then [2][32*32][9]
-  const int ntaps = grp == 0 ? 7 : 6, t0 = grp == 0 ? 0 : 1 + 6 * grp;
-  __syncthreads();
-  if (wave >= 2) {
-    float *dst = red + (wave - 2) * (7 * 16 * 64) + lane;
-#pragma unroll
-    for (int t = 0; t < 7; ++t)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) dst[(t * 16 + r) * 64] = acc[t][r];
-  }
-  __syncthreads();
-  if (wave < 2) {
-    const float *src = red + wave * (7 * 16 * 64) + lane;
-#pragma unroll
-    for (int t = 0; t < 7; ++t)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[t][r] += src[(t * 16 + r) * 64];
-  }
-  __syncthreads();
-  if (wave < 2) {
-    // reg r of lane l: output channel 8*(r/4) + 4*(l/32) + r%4, input channel l%32
-    float *dst = red + wave * (32 * 32 * 9) + (4 * (lane >> 5) * 32 + (lane & 31)) * 9;
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-#pragma unroll
-      for (int t = 0; t < 7; ++t) dst[(8 * (r >> 2) + (r & 3)) * (32 * 9) + t] = acc[t][r];
-  }
-  __syncthreads();
-  const int crs = a.C * 25;
-  float *out = a.partial + (static_cast<size_t>(slice) * a.Kc + co0) * crs + ci0 * 25 + t0;
-  for (int e = tid; e < 32 * 32 * 8; e += I8_NT) {
-    const int t = e & 7, pair = e >> 3;   // pair = output channel * 32 + input channel
-    if (t < ntaps)
-      out[static_cast<size_t>(pair >> 5) * crs + (pair & 31) * 25 + t] = red[pair * 9 + t] + red[32 * 32 * 9 + pair * 9 + t];
-  }
-  if (sums_dy) {
-    // the eight shares of a channel sit in neighbouring lanes: added with a fixed butterfly
-    dbs += __shfl_xor(dbs, 1, 64);
-    dbs += __shfl_xor(dbs, 2, 64);
-    dbs += __shfl_xor(dbs, 4, 64);
-    if ((tid & 7) == 0) a.partial_db[static_cast<size_t>(slice) * a.Kc + co0 + (tid >> 3)] = dbs;
-  }
+  dw_img_workgroup<IS>(a, smem, blockIdx.x, gridDim.x);
 }
 
 struct DwHaloPlan {
   bool ok;
-  bool img8;            // the image-sized kernel runs this shape
-  int img_size;         // ... on images of 8x8 or 16x16 pixels
-  DwImg8Args i8;
   int tc, wco, wk, wfy, nt;
   int rows_block;  // filter rows one workgroup covers
   DwHaloArgs args;
@@ -602,36 +396,12 @@ int pad_to_4_mod_32(int v) {
 }
 
 DwHaloPlan make_dw_plan(int R, int S, int batch, int C, int Kc, int H, int W, int OH, int OW, int ph,
-                        int pw, bool allow_img8 = true) {
+                        int pw) {
   DwHaloPlan p;
   p.ok = false;
   const bool five = R == 5 && S == 5;
   if (!(R == 3 && S == 3) && !five) return p;
   if (C < 16 || Kc < 16 || OW < 8 || OH < 2 || pw > 4) return p;
-  p.img8 = false;
-  // (16x16 images: from the batch on where the chunks give every compute unit a workgroup; the
-  // kernel below has fewer, longer workgroups, which is what a step that runs it beside its
-  // main chain wants)
-  const int is = H == 8 ? 8 : 16;
-  if (allow_img8 && five && H == is && W == is && OH == is && OW == is && ph == 2 && pw == 2 && C % 32 == 0 &&
-      Kc % 32 == 0 && batch >= (is == 8 ? 4 : 96) && static_cast<long>(batch) * std::max(C, Kc) * is * is < (1L << 30)) {
-    DwImg8Args &i = p.i8;
-    p.img_size = is;
-    i.batch = batch; i.C = C; i.Kc = Kc;
-    i.co_blocks = Kc / 32; i.ci_blocks = C / 32;
-    i.chunks_total = is == 8 ? ceil_div(batch, 4) : batch;
-    // one workgroup per compute unit where the batch allows it
-    const int base = 4 * i.co_blocks * i.ci_blocks;
-    int slices = std::max(1, 256 / base);
-    slices = std::min(slices, i.chunks_total);
-    i.chunks_per_slice = ceil_div(i.chunks_total, slices);
-    p.slices = ceil_div(i.chunks_total, i.chunks_per_slice);
-    p.grid   = dim3(static_cast<unsigned>(p.slices));   // (grid.x counts the slices, as below; the launch multiplies)
-    p.lds_bytes = sizeof(float) * (is == 8 ? I8Geom<8>::LDS_FLOATS : I8Geom<16>::LDS_FLOATS);
-    p.img8 = true;
-    p.ok   = true;
-    return p;
-  }
   p.tc = OW >= 48 ? 64 : OW >= 24 ? 32 : OW >= 12 ? 16 : 8;
   p.wfy = 1;
   // more than 32 output channels: two channel blocks share a workgroup's staged X patch (half
@@ -784,6 +554,31 @@ int dwx_slices(const DwxPlan &p) { return p.slices * p.args.tiles_x; }
 
 }  // namespace
 
+// One workgroup per compute unit and tap group where the batch allows it. 16x16 images: from the
+// batch on where the chunks give every compute unit a workgroup; the kernel above has fewer,
+// longer workgroups, which is what a step that runs it beside its main chain wants.
+DwImgPlan make_dw_img_plan(int R, int S, int batch, int C, int Kc, int H, int W, int OH, int OW, int ph, int pw) {
+  DwImgPlan p;
+  p.ok = false;
+  const int is = H;
+  if (R != 5 || S != 5 || (is != 8 && is != 16) || W != is || OH != is || OW != is || ph != 2 || pw != 2 ||
+      C % 32 != 0 || Kc % 32 != 0 || batch < 4 || static_cast<long>(batch) * std::max(C, Kc) * is * is >= (1L << 30))
+    return p;
+  DwImgArgs &a = p.args;
+  p.size = is;
+  a.batch = batch; a.C = C; a.Kc = Kc;
+  a.co_blocks = Kc / 32; a.ci_blocks = C / 32;
+  a.chunks_total = is == 8 ? ceil_div(batch, 2) : 2 * batch;
+  const int base   = 4 * a.co_blocks * a.ci_blocks;
+  const int slices = std::min(std::max(1, 256 / base), a.chunks_total);
+  a.chunks_per_slice = ceil_div(a.chunks_total, slices);
+  p.slices     = ceil_div(a.chunks_total, a.chunks_per_slice);
+  p.workgroups = base * p.slices;
+  p.lds_bytes  = sizeof(float) * (is == 8 ? DwImgGeom<8>::LDS_FLOATS : DwImgGeom<16>::LDS_FLOATS);
+  p.ok = true;
+  return p;
+}
+
 bool conv_dw_halo_applicable(int R, int S, int batch, int C, int Kc, int H, int W, int OH, int OW,
                              int ph, int pw) {
   return make_dwx_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw).ok ||
@@ -794,56 +589,18 @@ size_t conv_dw_halo_workspace_bytes(int R, int S, int batch, int C, int Kc, int 
                                     int OW, int ph, int pw) {
   const DwxPlan x3   = make_dwx_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
   const DwHaloPlan p = make_dw_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
-  if (!p.ok && !x3.ok) return 0;
-  // (tensors that are not 16-byte aligned take the general kernel's plan where the 8x8-image
-  // kernel would run: room for whichever has more slices)
-  const DwHaloPlan q = p.ok && p.img8 ? make_dw_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw, false) : p;
-  size_t slices = std::max(p.ok ? p.grid.x : 0u, q.ok ? q.grid.x : 0u);
+  const DwImgPlan im = make_dw_img_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
+  // (which of them runs also depends on the tensors' alignment: room for whichever has more slices)
+  size_t slices = 0;
+  if (p.ok) slices = p.grid.x;
   if (x3.ok) slices = std::max(slices, static_cast<size_t>(dwx_slices(x3)));
-  return ws_align(sizeof(float) * slices * Kc * C * R * S) + ws_align(sizeof(float) * slices * Kc);
+  if (im.ok) slices = std::max(slices, static_cast<size_t>(im.slices));
+  return slices == 0 ? 0 : ws_align(sizeof(float) * slices * Kc * C * R * S) + ws_align(sizeof(float) * slices * Kc);
 }
 
-// dw (+)= sum over the batch; the caller has checked applicability and reserved the workspace
-int conv_dw_halo_run(int R, int S, int batch, int C, int Kc, const float *x, const float *dy,
-                     float *dw, int H, int W, int OH, int OW, int ph, int pw, int accumulate,
-                     float *db) {
-  const bool vec = W % 4 == 0 && OW % 4 == 0 && aligned16(x) && aligned16(dy);
-  DwxPlan x3   = make_dwx_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
-  DwHaloPlan p = make_dw_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw, /*allow_img8=*/vec);
-  if (!p.ok && !x3.ok) return set_error(TDH_ERR_INVALID, "conv_dw_halo_run: shape not supported");
-  const int crs = C * R * S, slices = x3.ok ? dwx_slices(x3) : static_cast<int>(p.grid.x);
-  void *part = nullptr, *part_db = nullptr;
-  TDH_TRY(ws_take(sizeof(float) * static_cast<size_t>(slices) * Kc * crs, &part));
-  if (db) TDH_TRY(ws_take(sizeof(float) * static_cast<size_t>(slices) * Kc, &part_db));
-  if (x3.ok) {
-    x3.args.x = x; x3.args.dy = dy;
-    x3.args.partial = static_cast<float *>(part); x3.args.partial_db = static_cast<float *>(part_db);
-    ProfScope prof(db ? "conv_dw_db_x3" : "conv_dw_x3", Kc, crs, batch * OH * OW);
-    TDH_TRY(R == 5 ? dwx_launch_5_scalar(x3) : vec ? dwx_launch_3_vec(x3) : dwx_launch_3_scalar(x3));
-  } else
-  {
-    p.args.x = x; p.args.dy = dy; p.args.partial = static_cast<float *>(part);
-    p.args.partial_db = static_cast<float *>(part_db);
-    ProfScope prof(db ? "conv_dw_db_halo" : "conv_dw_halo", Kc, crs, batch * OH * OW);
-    if (p.img8) {
-      p.i8.x = x; p.i8.dy = dy; p.i8.partial = p.args.partial; p.i8.partial_db = p.args.partial_db;
-      static bool raised[2] = {false, false};
-      const int which = p.img_size == 8 ? 0 : 1;
-      void (*kernel)(const DwImg8Args) = which ? conv_dw_img8_kernel<16> : conv_dw_img8_kernel<8>;
-      if (!raised[which]) {
-        TDH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(p.lds_bytes)));
-        raised[which] = true;
-      }
-      TDH_LAUNCH(kernel, dim3(p.slices * p.i8.ci_blocks * p.i8.co_blocks * 4), dim3(I8_NT), p.lds_bytes,
-                 ctx().stream, p.i8);
-      TDH_LAUNCH_CHECK();
-    } else if (vec) {
-      TDH_TRY(launch_dw_vec<true>(p));
-    } else {
-      TDH_TRY(launch_dw_vec<false>(p));
-    }
-  }
+// dw (+)= the slices of part, db (+)= those of part_db: left to the train step, or launched here
+int conv_dw_sum_slices(const void *part, const void *part_db, int slices, int Kc, int crs, float *dw, float *db,
+                       int accumulate) {
   EpiRowMajor epi{dw, crs, nullptr, ActGrad(), accumulate};
   EpiRowMajor epi_b{db, 1, nullptr, ActGrad(), accumulate};
   // the two reductions leave as one launch: collected by the train step, or here
@@ -855,6 +612,49 @@ int conv_dw_halo_run(int R, int S, int batch, int C, int Kc, const float *x, con
   if (!collect_here) return TDH_OK;
   ctx().defer_reduce = false;
   return flush_deferred_reduces();
+}
+
+// dw (+)= sum over the batch; the caller has checked applicability and reserved the workspace
+int conv_dw_halo_run(int R, int S, int batch, int C, int Kc, const float *x, const float *dy,
+                     float *dw, int H, int W, int OH, int OW, int ph, int pw, int accumulate,
+                     float *db) {
+  const bool vec = W % 4 == 0 && OW % 4 == 0 && aligned16(x) && aligned16(dy);
+  DwxPlan x3   = make_dwx_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
+  DwImgPlan im = make_dw_img_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
+  DwHaloPlan p = make_dw_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
+  im.ok = im.ok && vec && (im.size == 8 || batch >= 96);
+  if (!p.ok && !x3.ok && !im.ok) return set_error(TDH_ERR_INVALID, "conv_dw_halo_run: shape not supported");
+  const int crs = C * R * S, slices = x3.ok ? dwx_slices(x3) : im.ok ? im.slices : static_cast<int>(p.grid.x);
+  void *part = nullptr, *part_db = nullptr;
+  TDH_TRY(ws_take(sizeof(float) * static_cast<size_t>(slices) * Kc * crs, &part));
+  if (db) TDH_TRY(ws_take(sizeof(float) * static_cast<size_t>(slices) * Kc, &part_db));
+  if (x3.ok) {
+    x3.args.x = x; x3.args.dy = dy;
+    x3.args.partial = static_cast<float *>(part); x3.args.partial_db = static_cast<float *>(part_db);
+    ProfScope prof(db ? "conv_dw_db_x3" : "conv_dw_x3", Kc, crs, batch * OH * OW);
+    TDH_TRY(R == 5 ? dwx_launch_5_scalar(x3) : vec ? dwx_launch_3_vec(x3) : dwx_launch_3_scalar(x3));
+  } else {
+    ProfScope prof(db ? "conv_dw_db_halo" : "conv_dw_halo", Kc, crs, batch * OH * OW);
+    if (im.ok) {
+      im.args.x = x; im.args.dy = dy;
+      im.args.partial = static_cast<float *>(part); im.args.partial_db = static_cast<float *>(part_db);
+      static bool raised[2] = {false, false};
+      const int which = im.size == 8 ? 0 : 1;
+      void (*kernel)(const DwImgArgs) = which ? conv_dw_img_kernel<16> : conv_dw_img_kernel<8>;
+      if (!raised[which]) {
+        TDH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(im.lds_bytes)));
+        raised[which] = true;
+      }
+      TDH_LAUNCH(kernel, dim3(im.workgroups), dim3(DWI_NT), im.lds_bytes, ctx().stream, im.args);
+      TDH_LAUNCH_CHECK();
+    } else {
+      p.args.x = x; p.args.dy = dy; p.args.partial = static_cast<float *>(part);
+      p.args.partial_db = static_cast<float *>(part_db);
+      TDH_TRY(vec ? launch_dw_vec<true>(p) : launch_dw_vec<false>(p));
+    }
+  }
+  return conv_dw_sum_slices(part, part_db, slices, Kc, crs, dw, db, accumulate);
 }
 
 }  // namespace tdh

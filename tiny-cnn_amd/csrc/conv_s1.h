@@ -73,6 +73,11 @@ struct S1Plan {
   int splits;
 };
 
+// the plan of a dX that shares its launch with the weight gradient (conv_bwd_pair.hip); ok = false also
+// where the three-part kernel runs dX
+S1Plan make_s1_pair_plan(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw);
+int finish_s1_split(const S1Plan &p, const float *bias, ActGrad ag, float *out, float *act_out, int act_kind);
+
 // one launcher per translation unit of kernel instances
 int s1_launch_3x3_vec(const S1Plan &p);
 int s1_launch_3x3_scalar(const S1Plan &p);

@@ -126,8 +126,9 @@ void choose_split(S1Plan &p, int kch, long blocks) {
 // Candidates run from the largest workgroup tile to the smallest; the first one that yields
 // at least 256 workgroups wins, else the one with the most workgroups, and shapes that cannot
 // even fill a quarter of the chip are left to the split-K GEMM.
+// small_tiles: only workgroups of 32 channels x 128 pixels (conv_bwd_pair.hip), however few.
 S1Plan make_plan_of(bool x3, int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph,
-                    int pw) {
+                    int pw, bool small_tiles = false) {
   S1Plan best;
   best.ok = false;
   best.x3 = x3;
@@ -142,7 +143,7 @@ S1Plan make_plan_of(bool x3, int R, int S, int batch, int KC, int MC, int IH, in
   // batch 128: 25 us with one block, 21 in fp32)
   const int n_cand = !x3 ? 3 : MC > 32 ? 2 : 1;
   long best_blocks = 0;
-  for (int ci = 0; ci < n_cand; ++ci) {
+  for (int ci = small_tiles ? 2 : 0; ci < n_cand; ++ci) {
     S1Plan p;
     p.ok = false;
     p.x3 = x3;
@@ -193,7 +194,7 @@ S1Plan make_plan_of(bool x3, int R, int S, int batch, int KC, int MC, int IH, in
     choose_split(p, kch, blocks);
     // short reductions have nothing to overlap their loads with inside a workgroup: ask for
     // more, smaller workgroups then
-    if (blocks >= (KC * R * S < 256 ? 1024 : 256)) return p;
+    if (small_tiles || blocks >= (KC * R * S < 256 ? 1024 : 256)) return p;
     if (blocks > best_blocks) {
       best_blocks = blocks;
       best        = p;
@@ -214,6 +215,14 @@ S1Plan make_plan(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 }  // namespace
+
+S1Plan make_s1_pair_plan(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw) {
+  S1Plan p;
+  p.ok = false;
+  if (ctx().keep_f32 || !make_plan_of(true, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw).ok)
+    p = make_plan_of(false, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw, true);
+  return p;
+}
 
 bool conv_s1_applicable(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW,
                         int ph, int pw) {
@@ -248,8 +257,8 @@ size_t conv_s1_workspace_bytes(int R, int S, int batch, int C, int Kc, int flip,
                                int OH, int OW, int ph, int pw) {
   const int KC = flip ? Kc : C, MC = flip ? C : Kc;
   size_t most = 0;
-  for (int x3 = 0; x3 < 2; ++x3) {  // (which of the two kernels runs is the caller's choice as well)
-    const S1Plan p = make_plan_of(x3 != 0, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw);
+  for (int k = 0; k < 3; ++k) {  // (which of the kernels runs is the caller's choice as well)
+    const S1Plan p = make_plan_of(k == 1, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw, k == 2);
     if (!p.ok) continue;
     size_t total = ws_align(conv_s1_packed_bytes(p.x3 ? CONV_PACK_X3 : CONV_PACK_F32, R * S, KC, MC));
     if (p.splits > 1) total += ws_align(sizeof(float) * p.splits * p.args.part_stride);
@@ -319,19 +328,21 @@ int conv_s1_run(int R, int S, int batch, int C, int Kc, int flip, const float *i
     else if (vec) TDH_TRY(R == 3 ? s1_launch_3x3_vec(p) : s1_launch_5x5_vec(p));
     else TDH_TRY(R == 3 ? s1_launch_3x3_scalar(p) : s1_launch_5x5_scalar(p));
   }
-  if (p.splits > 1) {
-    SplitSum sum;
-    sum.part = p.args.part; sum.splits = p.splits; sum.stride = p.args.part_stride;
-    sum.bias = bias; sum.MC = MC; sum.div_plane = FastDiv(OH * OW); sum.ag = ag; sum.out = out;
-    if (ctx().leave_split_sum && !act_out) {
-      // the kernel that reads `out` next adds the partials up (and writes `out`)
-      left_split_sum()     = sum;
-      ctx().split_sum_left = true;
-      return TDH_OK;
-    }
-    TDH_TRY(launch_split_reduce(sum, OH * OW, act_out, act_kind));
+  return p.splits > 1 ? finish_s1_split(p, bias, ag, out, act_out, act_kind) : TDH_OK;
+}
+
+// out from the partial sums of a split: left to the kernel that reads `out` next, if the caller has
+// asked for that (it adds the partials up and writes `out`), or launched here
+int finish_s1_split(const S1Plan &p, const float *bias, ActGrad ag, float *out, float *act_out, int act_kind) {
+  SplitSum sum;
+  sum.part = p.args.part; sum.splits = p.splits; sum.stride = p.args.part_stride;
+  sum.bias = bias; sum.MC = p.args.MC; sum.div_plane = FastDiv(p.args.OH * p.args.OW); sum.ag = ag; sum.out = out;
+  if (ctx().leave_split_sum && !act_out) {
+    left_split_sum()     = sum;
+    ctx().split_sum_left = true;
+    return TDH_OK;
   }
-  return TDH_OK;
+  return launch_split_reduce(sum, p.args.OH * p.args.OW, act_out, act_kind);
 }
 
 SplitSum &left_split_sum() {

@@ -23,7 +23,7 @@ __device__ __forceinline__ float s1_lane_xor(const float v) {
 template <int TC, int TM, int TN>
 __device__ __forceinline__ void s1_epilogue(const ConvS1Args &a, const floatx16 (&acc)[TM][TN], const int wn,
                                             const int lane, const int img0, const int y0, const int x0,
-                                            const int m0) {
+                                            const int m0, const int bz) {
   constexpr int LOG_TC = TC == 64 ? 6 : TC == 32 ? 5 : TC == 16 ? 4 : 3;
   // reg r of lane l holds channel 8*(r/4) + 4*(l/32) + r%4, pixel l%32
   const int ohw = a.OH * a.OW;
@@ -40,7 +40,7 @@ __device__ __forceinline__ void s1_epilogue(const ConvS1Args &a, const floatx16 
     for (int i = 0; i < TM; ++i) {
       // the 16 values of this lane: channels mb + 8*(rr/4) + rr%4, all at pixel pbase
       const int mb = m0 + 32 * i + 4 * (lane >> 5);
-      float *dst = a.part ? a.part + blockIdx.z * a.part_stride : a.out;
+      float *dst = a.part ? a.part + bz * a.part_stride : a.out;
       float v[16];
 #pragma unroll
       for (int rr = 0; rr < 16; ++rr) v[rr] = acc[i][j][rr];

@@ -1,4 +1,4 @@
-// conv_x3_inst.hip — the stride-1 convolution (forward and dX) of conv_s1_inst.hip on the bf16
+// conv_x3_inst.hip — the stride-1 convolution (forward and dX) of conv_s1_body.h on the bf16
 // matrix cores with three-part operands (split_bf16.h): the same tiles and epilogue, another
 // inner loop. Bound: bf16 MFMA issue; 6 instructions of 32768 FLOP stand for one fp32 product.
 //
@@ -201,7 +201,7 @@ __global__ void __launch_bounds__(256, 2) conv_x3_kernel(const ConvS1Args a) {
         for (int p = 0; p < X3_PARTS; ++p) wf[0][i][p] = wf[1][i][p];
     }
   }
-  s1_epilogue<TC, TM, TN>(a, acc, wn, lane, img0, y0, x0, m0);
+  s1_epilogue<TC, TM, TN>(a, acc, wn, lane, img0, y0, x0, m0, blockIdx.z);
 }
 
 template <int R, int S, int TC, int TM, int TN, bool VEC>

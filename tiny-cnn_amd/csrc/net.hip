@@ -1060,7 +1060,9 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
     // a small fully-connected layer computes its three gradients in one launch on the main
     // chain: its weight and bias products are too small to be worth a branch
     const bool fc_one_launch = s.kind == TDH_L_FC && fc_bwd_fuses(s.fc_in, s.fc_out, batch);
-    const bool fork = forked && layer_forks(L) && !fc_one_launch;
+    // so does a convolution whose gradients share a launch
+    const bool conv_pair = s.kind == TDH_L_CONV && dx && i != through_pool_for && conv_bwd_pairs(&s.conv, batch);
+    const bool fork = forked && layer_forks(L) && !fc_one_launch && !conv_pair;
     if (fork) {
       // this layer's output gradient is complete here: let the side streams start from it
       TDH_HIP(hipEventRecord(net->events[i], c.stream));
@@ -1078,17 +1080,20 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
         TDH_TRY(ws_begin((forked || as_forked ? 3 : 1) * conv2d_workspace_bytes(&s.conv, batch)));
       {
         const PoolGather *gp = i == through_pool_for ? &through_pool : nullptr;
-        const void *wp = packed ? packed_filters(L, batch, 1) : nullptr;
+        const void *wp = !packed ? nullptr : conv_pair ? L.wp_dx : packed_filters(L, batch, 1);
         // the layer that reads this dX next (behind a folded activation) is a max-pool: its
         // backward kernel can add up a split reduction of dX
         const int reader = i - 1 - ((i >= 1 && net->layers[i - 1].grad_folded) ? 1 : 0);
         const bool pool_reads = (net->flags & TDH_NET_FUSE_ACT_GRAD) && reader >= 0 &&
                                 net->layers[reader].spec.kind == TDH_L_MAXPOOL;
         if (forked) {
-          if (!fork) {
+          if (conv_pair) {
             LeaveSplitSum leave(c, pool_reads);
+            c.defer_reduce = true;
             TDH_TRY(conv2d_bwd(&s.conv, batch, in, L.w, L.dout, dx, L.dw, L.b_size ? L.db : nullptr, 1, fold,
                                L.tbl_dev, wp, gp));
+            c.defer_reduce = false;
+            last_dw_on_main = true;
             break;
           }
           const bool db_with_dw = L.b_size && conv_dw_gives_db(&s.conv, batch);
@@ -1134,6 +1139,14 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
           }
         } else if (as_forked) {
           // the launches of the captured, branching step, one after the other
+          if (conv_pair) {
+            LeaveSplitSum leave(c, pool_reads);
+            c.defer_reduce = true;
+            TDH_TRY(conv2d_bwd(&s.conv, batch, in, L.w, L.dout, dx, L.dw, L.b_size ? L.db : nullptr, 1, fold,
+                               L.tbl_dev, wp, gp));
+            c.defer_reduce = false;
+            break;
+          }
           if (i == 0 && dx && !wp && conv_bwd_one_launch(&s.conv, batch, gp != nullptr)) {
             c.defer_reduce = true;
             TDH_TRY(conv2d_bwd(&s.conv, batch, in, L.w, L.dout, dx, L.dw, L.b_size ? L.db : nullptr, 1, fold,
@@ -1234,7 +1247,7 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
   OptPending pending;
   pending.n = 0;
   bool to_optimizer = false;
-  if ((side_used[0] || as_forked) && do_update && peek_deferred_reduces(&pending)) {
+  if ((side_used[0] || as_forked || last_dw_on_main) && do_update && peek_deferred_reduces(&pending)) {
     to_optimizer = true;
     for (int k = 0; k < pending.n; ++k) {
       bool small_blocks = false;
