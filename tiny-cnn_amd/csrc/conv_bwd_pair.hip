@@ -10,7 +10,7 @@
 #include <algorithm>
 
 #include "conv_dw_img.h"
-#include "conv_s1_body.h"
+#include "conv_x3_body.h"
 
 namespace tdh {
 
@@ -29,7 +29,7 @@ conv_bwd_pair_kernel(const ConvS1Args dx, const DwImgArgs dw, const int dx_block
   uint32_t rest, tile, m, split;
   div_tiles.divmod(id, rest, tile);
   div_m.divmod(rest, split, m);
-  conv_s1_workgroup<5, 5, IS, 1, 1, true>(dx, smem, tile, m, split);
+  conv_x3_workgroup<5, 5, IS, 1, 1, true, true>(dx, smem, tile, m, split);
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -54,8 +54,8 @@ int conv_bwd_pair_run(int R, int S, int batch, int C, int Kc, int H, int W, int 
   const void *wp = prepacked;
   if (!prepacked) {
     void *fresh = nullptr;
-    TDH_TRY(ws_take(conv_s1_packed_bytes(CONV_PACK_F32, R * S, Kc, C), &fresh));
-    TDH_TRY(conv_s1_repack(R, S, C, Kc, 1, w, nullptr, fresh, false));
+    TDH_TRY(ws_take(conv_s1_packed_bytes(CONV_PACK_X3, R * S, Kc, C), &fresh));
+    TDH_TRY(conv_s1_repack(R, S, C, Kc, 1, w, nullptr, fresh, true));
     wp = fresh;
   }
   ConvS1Args &a = p.args;

@@ -25,7 +25,7 @@ constexpr int s1_niq(int R, int S, int TC, int TM, int TN) {
 // The three-part bf16 kernel (conv_x3_inst.hip): 16 channels a chunk, words of eight channels that
 // a thread stages per chunk at most (32 registers each).
 constexpr int X3_KCH = 16;
-constexpr int x3_items(int TM, int TN) { return TM * TN >= 4 ? 1 : 2; }
+constexpr int x3_items(int TM, int TN) { return TM * TN >= 4 || TM * TN == 1 ? 1 : 2; }
 // rows of the packed filters: whole tiles of either width
 constexpr int x3_mc_pad(int MC) { return MC > 32 ? (MC + 63) / 64 * 64 : 32; }
 constexpr size_t x3_pack_bytes(int RS, int KC, int MC) {

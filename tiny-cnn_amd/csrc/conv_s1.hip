@@ -141,13 +141,14 @@ S1Plan make_plan_of(bool x3, int R, int S, int batch, int KC, int MC, int IH, in
   // (three parts: tiles of at least two accumulator blocks a wave, or the filter operands that a
   // wave reads for every tap are more than its products cover: 16x16 images, 32 -> 32 channels, 5x5,
   // batch 128: 25 us with one block, 21 in fp32)
-  const int n_cand = !x3 ? 3 : MC > 32 ? 2 : 1;
+  const int x3t = small_tiles;
+  const int n_cand = !x3 ? 3 : MC > 32 ? (x3t ? 3 : 2) : (x3t ? 2 : 1);
   long best_blocks = 0;
-  for (int ci = small_tiles ? 2 : 0; ci < n_cand; ++ci) {
+  for (int ci = small_tiles ? n_cand - 1 : 0; ci < n_cand; ++ci) {
     S1Plan p;
     p.ok = false;
     p.x3 = x3;
-    const int *narrow = x3 ? cand_narrow[1] : cand_narrow[ci];
+    const int *narrow = cand_narrow[x3 ? ci + 1 : ci];
     p.tc = OW >= 48 ? 64 : OW >= 24 ? 32 : OW >= 12 ? 16 : 8;
     p.tm = MC > 32 ? cand_wide[ci][0] : narrow[0];
     p.tn = MC > 32 ? cand_wide[ci][1] : narrow[1];
@@ -172,6 +173,10 @@ S1Plan make_plan_of(bool x3, int R, int S, int batch, int KC, int MC, int IH, in
       if (p.lds_bytes > 80 * 1024) continue;  // two workgroups a compute unit
       if (static_cast<long>(ti) * KC * IH * IW >= (1L << 29)) continue;  // 32-bit byte offsets inside a tile
       a.mc_pad = x3_mc_pad(MC);
+      if (p.tm * p.tn == 1) {  // (the waves' sums)
+        if (R == 1) continue;
+        p.lds_bytes = std::max<size_t>(p.lds_bytes, 64 * 1024);
+      }
     } else {
       if (ceil_div(planeq, 256 / kch) > s1_niq(R, S, p.tc, p.tm, p.tn)) continue;
       p.lds_bytes = sizeof(float) * kch * (4 * static_cast<size_t>(planeq) + R * S * 32 * p.tm);
@@ -186,6 +191,10 @@ S1Plan make_plan_of(bool x3, int R, int S, int batch, int KC, int MC, int IH, in
       // unsplit, and a workgroup for every compute unit at least; two where a single short chunk has
       // nothing to cover its loads with (32x32 images, 16 -> 32 channels, 3x3, batch 64: 12.6 us with
       // one a unit, 11.2 in fp32)
+      if (p.tm * p.tn == 1) {
+        choose_split(p, kch, blocks);
+        return p;
+      }
       if (blocks < (KC * R * S < 256 ? 512 : 256)) continue;
       p.splits = 1;
       a.kc_split = KC; a.part = nullptr; a.part_stride = 0;
@@ -219,8 +228,8 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 S1Plan make_s1_pair_plan(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw) {
   S1Plan p;
   p.ok = false;
-  if (ctx().keep_f32 || !make_plan_of(true, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw).ok)
-    p = make_plan_of(false, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw, true);
+  if (!ctx().keep_f32 && !make_plan_of(true, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw).ok)
+    p = make_plan_of(true, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw, true);
   return p;
 }
 
@@ -258,7 +267,7 @@ size_t conv_s1_workspace_bytes(int R, int S, int batch, int C, int Kc, int flip,
   const int KC = flip ? Kc : C, MC = flip ? C : Kc;
   size_t most = 0;
   for (int k = 0; k < 3; ++k) {  // (which of the kernels runs is the caller's choice as well)
-    const S1Plan p = make_plan_of(k == 1, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw, k == 2);
+    const S1Plan p = make_plan_of(k != 0, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw, k == 2);
     if (!p.ok) continue;
     size_t total = ws_align(conv_s1_packed_bytes(p.x3 ? CONV_PACK_X3 : CONV_PACK_F32, R * S, KC, MC));
     if (p.splits > 1) total += ws_align(sizeof(float) * p.splits * p.args.part_stride);

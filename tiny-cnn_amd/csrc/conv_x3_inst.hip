@@ -1,212 +1,20 @@
-// conv_x3_inst.hip — the stride-1 convolution (forward and dX) of conv_s1_body.h on the bf16
-// matrix cores with three-part operands (split_bf16.h): the same tiles and epilogue, another
-// inner loop. Bound: bf16 MFMA issue; 6 instructions of 32768 FLOP stand for one fp32 product.
-//
-// Per chunk of 16 reduction channels a workgroup loads the input patch with its halo as 16-byte
-// words of four pixels, eight channels of a word to a thread, splits them once and leaves them in
-// LDS as [part][8-channel half][pixel][8 channels]: the operand of one lane of a
-// 32x32x16 product is then one aligned 16-byte read at a pixel, every filter tap is a constant
-// number of pixels away, and a split is shared by all taps and all output channels. The filters
-// come split from memory ([chunk][tap][part][half][m][8 channels], x3_pack_kernel): a wave reads its
-// own operands of the next tap from there while it multiplies the current one (the four waves of
-// a workgroup read the same lines, so all but the first find them in L1), which leaves the LDS
-// to the patch: 41 KB for 64 channels x 4 rows of 64 pixels, two workgroups a compute unit.
-#include "conv_s1_epilogue.h"
-#include "split_bf16.h"
-#include <type_traits>
+// conv_x3_inst.hip — the three-part stride-1 convolution kernel of conv_x3_body.h, compiled eight
+// times, -DTDH_X3_PART=0..7: windows of 1, 3, 5 and 7, with 16-byte and scalar loads.
+#include "conv_x3_body.h"
 
 namespace tdh {
 
 namespace {
 
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
-
-constexpr unsigned X3_NOWHERE = 0x80000000u;  // past the end of every tile's images
-
-template <int R, int S, int TC, int TM, int TN, bool VEC>
+template <int R, int S, int TC, int TM, int TN, bool VEC, bool BY_TAPS>
 __global__ void __launch_bounds__(256, 2) conv_x3_kernel(const ConvS1Args a) {
-  constexpr int RS     = R * S;
-  constexpr int NI     = x3_items(TM, TN);
-  constexpr int NQ     = (3 + TC + S - 1 + 3) / 4;  // words per staged row
-  constexpr int PITCH  = 4 * NQ;
-  constexpr int BM     = 32 * TM;
-  constexpr int LOG_TC = TC == 64 ? 6 : TC == 32 ? 5 : TC == 16 ? 4 : 3;
-
-  extern __shared__ __align__(16) uintx4 patch[];  // [part][half][pixel]
-  const int TRH    = a.TR + R - 1;
-  const int planeq = a.TI * TRH * NQ;  // words of one channel of the staged patch
-  const int npix   = 4 * planeq;
-
-  const int tid = threadIdx.x, lane = tid & 63, wn = tid >> 6;
-  int bt        = blockIdx.x;
-  const int tx  = bt % a.tiles_x;
-  bt /= a.tiles_x;
-  const int ty    = bt % a.tiles_y;
-  const int tb    = bt / a.tiles_y;
-  const int img0  = tb << a.log_ti;
-  const int y0    = ty << a.log_tr;
-  const int x0    = tx * TC;
-  const int m0    = blockIdx.y * BM;
-  const int ihw   = a.IH * a.IW;
-  const int kc_lo = blockIdx.z * a.kc_split;
-  const int kc_hi = min(a.KC, kc_lo + a.kc_split);
-
-  // ---- staging plan: item tid + 256*i -> channel half, word of the patch. Loads go through a
-  // buffer descriptor that starts at the tile's first image and ends at the last one: words that
-  // do not exist get an offset past its end and come back as zeros.
-  const float *in0   = a.in + static_cast<size_t>(img0) * a.KC * ihw;
-  const int n_img    = min(a.TI, a.batch - img0);
-  const unsigned in_bytes = 4u * n_img * a.KC * ihw;
-  unsigned goff[NI];
-  int ihalf[NI], ipix[NI];
-  unsigned gkeep = 0;  // scalar loads: 4 bits per item, float k lies inside the row
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int e = tid + 256 * i;
-    goff[i]     = X3_NOWHERE;
-    ipix[i]     = -1;
-    ihalf[i]    = 0;
-    if (e < 2 * planeq) {
-      const int half = e >= planeq, pe = e - half * planeq;
-      uint32_t ti, rem;
-      a.div_rows.divmod(pe, ti, rem);
-      const int r = rem / NQ, q = rem - r * NQ;
-      const int iy = y0 - a.ph + r, ix = x0 - a.pwa + 4 * q;
-      unsigned keep = 0;
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (static_cast<unsigned>(ix + k) < static_cast<unsigned>(a.IW)) keep |= 1u << k;
-      ihalf[i] = half;
-      ipix[i]  = half * npix + 4 * pe;
-      if (static_cast<int>(ti) < n_img && static_cast<unsigned>(iy) < static_cast<unsigned>(a.IH) &&
-          (VEC ? keep == 15u : keep != 0u)) {
-        goff[i] = 4u * ((ti * a.KC + 8 * half) * ihw + iy * a.IW + ix);
-        gkeep |= keep << (4 * i);
-      }
-    }
-  }
-
-  // ---- operand positions: pixel of lane l of block j, and this lane's filter operands
-  int bpix[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int q  = (wn * TN + j) * 32 + (lane & 31);
-    const int ti = q >> (a.log_tr + LOG_TC);
-    const int r  = (q >> LOG_TC) & (a.TR - 1);
-    const int c  = q & (TC - 1);
-    bpix[j]      = (ti * TRH + r) * PITCH + c + (a.pwa - a.pw) + (lane >> 5) * npix;
-  }
-  const char *wall     = static_cast<const char *>(a.wp);
-  const uint32_t wlane = 16u * ((lane >> 5) * a.mc_pad + m0 + (lane & 31));
-  const int wpart      = 2 * 16 * a.mc_pad;  // bytes from one part to the next
-
-  floatx16 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-  floatx4 rin[NI][8];
-  // the eight channels of every item of the chunk starting at kc0
-  auto fetch = [&](int kc0) {
-    const auto desc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(in0), 0, in_bytes, 0x00027000);
-    const int left  = kc_hi - kc0;
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        const int at       = 4 * (kc0 + c) * ihw;
-        const unsigned off = left >= 16 || 8 * ihalf[i] + c < left ? goff[i] : X3_NOWHERE;
-        if (VEC) {
-          rin[i][c] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(desc, off, at, 0));
-        } else {
-          const unsigned keep = gkeep >> (4 * i);
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-            rin[i][c][k] = __builtin_bit_cast(
-                float, __builtin_amdgcn_raw_buffer_load_b32(desc, keep >> k & 1u ? off + 4 * k : X3_NOWHERE, at, 0));
-        }
-      }
-  };
-  auto stage = [&]() {
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      if (ipix[i] < 0) continue;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        uintx4 part[X3_PARTS];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          uint32_t p3[X3_PARTS];
-          split_pair(rin[i][2 * c][k], rin[i][2 * c + 1][k], p3);
-#pragma unroll
-          for (int p = 0; p < X3_PARTS; ++p) part[p][c] = p3[p];
-        }
-#pragma unroll
-        for (int p = 0; p < X3_PARTS; ++p) patch[p * 2 * npix + ipix[i] + k] = part[p];
-      }
-    }
-  };
-
-  // operands of tap u, counted over the chunks
-  bf16x8 wf[2][TM][X3_PARTS], xf[TN][X3_PARTS];
-  auto read_filters = [&](int u, int to) {
-    const char *w = wall + static_cast<size_t>(u) * X3_PARTS * wpart;
-#pragma unroll
-    for (int p = 0; p < X3_PARTS; ++p)
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-        wf[to][i][p] = *reinterpret_cast<const bf16x8 *>(w + static_cast<size_t>(p) * wpart + (wlane + 512u * i));
-  };
-  auto read_patch = [&](int t) {
-#pragma unroll
-    for (int p = 0; p < X3_PARTS; ++p)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        xf[j][p] = __builtin_bit_cast(bf16x8, patch[p * 2 * npix + bpix[j] + (t / S) * PITCH + t % S]);
-  };
-
-  // Loads are waited for in the order of their issue, so the filters of the tap after next would
-  // wait for the patch of the next chunk, which comes from much further away, wherever that is
-  // issued in between: it is issued once per chunk, behind the filters of tap 1, and has the
-  // products of two taps to arrive. us for 64 -> 64 channels of 128x128 / 128 -> 128 of 64x64 /
-  // 32 -> 64 of 64x64, batch 64: fp32 kernel 600 / 589 / 92, here 431 / 381 / 63 (179 / 203 / 153
-  // TFLOP/s); the patch loads spread over the taps cost 6 % more, a second set of patch operands or
-  // the reads pinned in front of the products 7-11 %. Without the loads, the LDS traffic and the
-  // additions behind the products of all but the first chunk it is 327 / 290 / 50: what the matrix
-  // cores and the power limit leave.
-  fetch(kc_lo);
-  read_filters(kc_lo / 16 * RS, 0);
-  for (int kc0 = kc_lo; kc0 < kc_hi; kc0 += 16) {
-    const bool more = kc0 + 16 < kc_hi;
-    if (kc0 > kc_lo) __syncthreads();  // everyone is done reading the previous chunk
-    stage();
-    __syncthreads();
-#pragma unroll
-    for (int t = 0; t < RS; ++t) {
-      const int cur = t & 1;
-      if (t + 1 < RS || more) read_filters(kc0 / 16 * RS + t + 1, cur ^ 1);
-      read_patch(t);
-      if (t == 0 && more) fetch(kc0 + 16);
-      mfma_x3<TM, TN>(acc, wf[cur], xf, x3_sign(kc0 / 16 * RS + t));
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (RS & 1) {  // the next chunk's first tap is read from buffer 0
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int p = 0; p < X3_PARTS; ++p) wf[0][i][p] = wf[1][i][p];
-    }
-  }
-  s1_epilogue<TC, TM, TN>(a, acc, wn, lane, img0, y0, x0, m0, blockIdx.z);
+  extern __shared__ __align__(16) uint32_t x3_lds[];
+  conv_x3_workgroup<R, S, TC, TM, TN, VEC, BY_TAPS>(a, x3_lds, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
-template <int R, int S, int TC, int TM, int TN, bool VEC>
+template <int R, int S, int TC, int TM, int TN, bool VEC, bool BY_TAPS = false>
 int launch_x3_inst(const S1Plan &p) {
-  auto kernel = conv_x3_kernel<R, S, TC, TM, TN, VEC>;
+  auto kernel = conv_x3_kernel<R, S, TC, TM, TN, VEC, BY_TAPS>;
   if (p.lds_bytes > 64 * 1024) {
     static size_t raised = 0;
     if (p.lds_bytes > raised) {
@@ -226,7 +34,9 @@ int launch_x3_tc(const S1Plan &p) {
     case 22: return launch_x3_inst<R, S, TC, 2, 2, VEC>(p);
     case 21: return launch_x3_inst<R, S, TC, 2, 1, VEC>(p);
     case 12: return launch_x3_inst<R, S, TC, 1, 2, VEC>(p);
-    default: return launch_x3_inst<R, S, TC, 1, 1, VEC>(p);
+    default:  // by filter taps; a 1x1 window has only one
+      if constexpr (R > 1) return launch_x3_inst<R, S, TC, 1, 1, VEC, true>(p);
+      else return set_error(TDH_ERR_INVALID, "three-part convolution: no such tile");
   }
 }
 
@@ -242,7 +52,6 @@ int launch_x3_rs(const S1Plan &p) {
 
 }  // namespace
 
-// compiled eight times, -DTDH_X3_PART=0..7: windows of 1, 3, 5 and 7, with 16-byte and scalar loads
 #define X3_JOIN_(a, b, c, d) a##b##c##d
 #define X3_JOIN(a, b, c, d) X3_JOIN_(a, b, c, d)
 #if TDH_X3_PART < 2

@@ -654,7 +654,8 @@ int tdh_net_create(const tdh_layer *layers, int n_layers, int max_batch, int fla
       if ((rc = net_alloc(net, L.w_size, &L.wp_fwd, false))) break;
       if ((rc = net_alloc(net, L.w_size, &L.wp_dx, false))) break;
       for (int flip = 0; flip < 2 && rc == TDH_OK; ++flip)
-        if (conv_packed_kind(&L.spec.conv, max_batch, flip) == CONV_PACK_X3)
+        if (conv_packed_kind(&L.spec.conv, max_batch, flip) == CONV_PACK_X3 ||
+            (flip && conv_bwd_pairs(&L.spec.conv, max_batch)))
           rc = net_alloc(net, conv_packed_bytes(&L.spec.conv, CONV_PACK_X3, flip) / sizeof(float),
                          flip ? &L.wx_dx : &L.wx_fwd, false);
       if (rc != TDH_OK) break;
@@ -1080,7 +1081,7 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
         TDH_TRY(ws_begin((forked || as_forked ? 3 : 1) * conv2d_workspace_bytes(&s.conv, batch)));
       {
         const PoolGather *gp = i == through_pool_for ? &through_pool : nullptr;
-        const void *wp = !packed ? nullptr : conv_pair ? L.wp_dx : packed_filters(L, batch, 1);
+        const void *wp = !packed ? nullptr : conv_pair ? L.wx_dx : packed_filters(L, batch, 1);
         // the layer that reads this dX next (behind a folded activation) is a max-pool: its
         // backward kernel can add up a split reduction of dX
         const int reader = i - 1 - ((i >= 1 && net->layers[i - 1].grad_folded) ? 1 : 0);
