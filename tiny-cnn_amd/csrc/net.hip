@@ -180,9 +180,27 @@ bool net_skips_input_grad(const tdh_net *net) {
   return kind == TDH_L_CONV || kind == TDH_L_FC;
 }
 
+bool has_batchnorm(const tdh_net *net) {
+  for (const tdh_net::Layer &L : net->layers)
+    if (L.spec.kind == TDH_L_BATCHNORM) return true;
+  return false;
+}
+
+// whether the step has a gradient to put on a branch: one that is not part of a launch on the
+// main chain
+bool layer_branches(const tdh_net *net, int i, int batch) {
+  const tdh_net::Layer &L = net->layers[i];
+  if (L.spec.kind == TDH_L_FC) return !fc_bwd_fuses(L.spec.fc_in, L.spec.fc_out, batch);
+  if (L.spec.kind != TDH_L_CONV) return false;
+  return i > 0 ? !conv_bwd_pairs(&L.spec.conv, batch) : L.b_size && !conv_dw_gives_db(&L.spec.conv, batch);
+}
 bool net_forks(const tdh_net *net, int batch) {
   const double flop = net_forward_flop(net, batch);
-  return flop >= 1e8 && flop <= 3e10 && !(flop >= 2.2e9 && flop < 1e10);
+  if (!(flop >= 1e8 && flop <= 3e10 && !(flop >= 2.2e9 && flop < 1e10))) return false;
+  const KeepF32 keep_f32(has_batchnorm(net));  // (the choices of the step itself)
+  for (int i = 0; i < static_cast<int>(net->layers.size()); ++i)
+    if (layer_branches(net, i, batch)) return true;
+  return false;
 }
 // A step too small to branch (LeNet-5 at batch 16) is a chain of launches of a few
 // microseconds each, and what counts is how many there are; a larger step that does not
@@ -193,6 +211,18 @@ bool net_forks(const tdh_net *net, int batch) {
 bool net_defers_serially(const tdh_net *net, int batch) {
   return (net->flags & TDH_NET_GRAPH) && (net->flags & TDH_NET_FUSE_ACT_GRAD) &&
          !net_forks(net, batch);
+}
+
+bool tiny_step_applies(const tdh_net *net, int loss_kind);
+// A step without branches whose kernels take longer than their launches take the host: it is not
+// captured. Between two replays the device idles for some 6 us, between two launches that were
+// queued in time for 1 (the CIFAR-10-shape net, us a step replayed / launched: batch 16 115 / 114, 32 128 /
+// 123, 64 134 / 129, 128 164 / 158, 512 516 / 507), and a step on tensors that it has not seen, or
+// of another batch, starts without a capture. A layer comes to about two launches of 4 us; from
+// 5e7 FLOP a layer on its kernels take more.
+bool step_outlasts_launches(const tdh_net *net, int loss_kind, int batch) {
+  return !tiny_step_applies(net, loss_kind) && !net_forks(net, batch) &&
+         net_forward_flop(net, batch) >= 5e7 * static_cast<double>(net->layers.size());
 }
 
 // The plan of the one-workgroup-per-sample step (tiny_net.hip) for a net that qualifies: at most
@@ -436,12 +466,6 @@ const void *packed_filters(const tdh_net::Layer &L, int batch, int flip) {
     case CONV_PACK_X3: return flip ? L.wx_dx : L.wx_fwd;
     default: return nullptr;
   }
-}
-
-bool has_batchnorm(const tdh_net *net) {
-  for (const tdh_net::Layer &L : net->layers)
-    if (L.spec.kind == TDH_L_BATCHNORM) return true;
-  return false;
 }
 
 // packed: the layers' wp_fwd hold the current filters in the stride-1 kernels' layout
@@ -1305,7 +1329,7 @@ static int train_steps(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, int
                        const float *const *ts, int do_update) {
   TDH_TRY(refresh_packs(net));
   // per-kernel timing needs the launches themselves, not a replay
-  if (!(net->flags & TDH_NET_GRAPH) || profiling_active()) {
+  if (!(net->flags & TDH_NET_GRAPH) || profiling_active() || (n_steps == 1 && step_outlasts_launches(net, loss_kind, batch))) {
     // (the timing pass of a branching step keeps every layer's scratch piece until the optimizer
     // has read the split sums: the buffer must not grow, and so move, on the way)
     for (int s = 0; s < n_steps; ++s) {
