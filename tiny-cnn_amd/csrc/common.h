@@ -350,7 +350,7 @@ int conv2d_fwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
 // dX, dW and db of this (first) convolution leave conv2d_bwd as one launch when all three are
 // asked for together (pooled: the gradient is read through the max-pool behind the layer)
 bool conv_bwd_one_launch(const tdh_conv_desc *d, int batch, bool pooled);
-// ... of this later convolution; dX reads filters packed as CONV_PACK_F32
+// ... of this later convolution; dX reads filters packed as CONV_PACK_X3
 bool conv_bwd_pairs(const tdh_conv_desc *d, int batch);
 // the forward kernel of this convolution can also compute the max-pool layer `pool` behind it
 bool conv_fwd_fuses_pool(const tdh_conv_desc *d, const tdh_pool_desc *pool, int batch, bool prepacked);

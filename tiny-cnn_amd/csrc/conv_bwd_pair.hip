@@ -1,12 +1,18 @@
 // conv_bwd_pair.hip — dX and dW (and db) of a 5x5 convolution on small images as ONE launch: the
-// workgroups of conv_s1_body.h (dX, 32 channels x 128 pixels each) and, behind them, those of
+// workgroups of conv_x3_body.h (dX, 32 channels x 128 pixels each) and, behind them, those of
 // conv_dw_img.h (dW). Both read dY and neither reads what the other writes.
 //
 // Each of the two alone is about one workgroup, four waves, per compute unit, and half of its time a
 // wave waits: for its first loads, for the other waves between two chunks, for the sums at the end.
-// Together two workgroups sit on a compute unit (76 KB of LDS each, 256 registers a wave) and one
+// Together two workgroups sit on a compute unit (72 KB of LDS each, 256 registers a wave) and one
 // multiplies while the other waits. On two streams the kernels overlap as well, but a fork and a
 // join cost a replayed step 5 us each.
+//
+// dX shares its filter taps out to the waves, because a wave that keeps to 32 pixels of its own
+// reads more filter operands than its products cover (alone, 16x16 images, 32 -> 32 channels, batch
+// 128: 25 us; in fp32 21). us, two launches / this one with dX in fp32 / as it is, batch 128:
+// 16x16, 32 -> 32 channels 42.7 / 36.5 / 31.3; 8x8, 32 -> 64 28.2 / 23.3 / 19.8. Bound: MFMA issue,
+// the weight gradient's in fp32.
 #include <algorithm>
 
 #include "conv_dw_img.h"
@@ -20,16 +26,15 @@ template <int IS>
 __global__ void __launch_bounds__(256, 2)
 conv_bwd_pair_kernel(const ConvS1Args dx, const DwImgArgs dw, const int dx_blocks, const FastDiv div_tiles,
                      const FastDiv div_m) {
-  extern __shared__ __align__(16) float smem[];
   const int id = blockIdx.x;
   if (id >= dx_blocks) {
-    dw_img_workgroup<IS>(dw, smem, id - dx_blocks, gridDim.x - dx_blocks);
+    dw_img_workgroup<IS>(dw, id - dx_blocks, gridDim.x - dx_blocks);
     return;
   }
   uint32_t rest, tile, m, split;
   div_tiles.divmod(id, rest, tile);
   div_m.divmod(rest, split, m);
-  conv_x3_workgroup<5, 5, IS, 1, 1, true, true>(dx, smem, tile, m, split);
+  conv_x3_workgroup<5, 5, IS, 1, 1, true, true>(dx, tile, m, split);
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }

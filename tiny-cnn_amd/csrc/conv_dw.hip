@@ -376,8 +376,7 @@ __global__ void __launch_bounds__(64 * WCO * WK * WFY, 1) conv_dw_halo_kernel(co
 // 5x5 windows on 8x8 and 16x16 images (conv_dw_img.h)
 template <int IS>
 __global__ void __launch_bounds__(DWI_NT, 2) conv_dw_img_kernel(const DwImgArgs a) {
-  extern __shared__ __align__(16) float smem[];
-  dw_img_workgroup<IS>(a, smem, blockIdx.x, gridDim.x);
+  dw_img_workgroup<IS>(a, blockIdx.x, gridDim.x);
 }
 
 struct DwHaloPlan {

@@ -98,10 +98,11 @@ __device__ __forceinline__ void dw_img_products(const float *ap, const float *bp
 }
 
 template <int IS, int G>
-__device__ __forceinline__ void dw_img_taps(const DwImgArgs &a, float *smem, const int cob, const int cib, const int slice) {
+__device__ __forceinline__ void dw_img_taps(const DwImgArgs &a, const int cob, const int cib, const int slice) {
   using GE = DwImgGeom<IS>;
   using TG = DwImgTaps<G>;
   constexpr int XP = GE::XP, FP = GE::FP, PIX = IS * IS, WPR = GE::WPR, XW = GE::XW;
+  extern __shared__ __align__(16) float smem[];
   float *dy_l = smem;                  // [32][DWI_DYP]
   float *x_l  = smem + 32 * DWI_DYP;   // [32][XP], frames of zeros around the images
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -245,9 +246,9 @@ __device__ __forceinline__ void dw_img_taps(const DwImgArgs &a, float *smem, con
   }
 }
 
-// workgroup `block` of `blocks`; smem: DwImgGeom<IS>::LDS_FLOATS
+// workgroup `block` of `blocks`, launched with DwImgGeom<IS>::LDS_FLOATS of LDS
 template <int IS>
-__device__ __forceinline__ void dw_img_workgroup(const DwImgArgs &a, float *smem, const int block, const int blocks) {
+__device__ __forceinline__ void dw_img_workgroup(const DwImgArgs &a, const int block, const int blocks) {
   // workgroups that read the same tiles (the four tap groups and the output-channel blocks of a
   // slice) are neighbours after the renumbering, and so share an XCD's L2
   int id = xcd_compact_id(block, blocks);
@@ -258,10 +259,10 @@ __device__ __forceinline__ void dw_img_workgroup(const DwImgArgs &a, float *smem
   const int cib = id % a.ci_blocks, slice = id / a.ci_blocks;
   // (one copy of the loop per group: a switch inside it would move every accumulator between the copies)
   switch (grp) {
-    case 0: dw_img_taps<IS, 0>(a, smem, cob, cib, slice); break;
-    case 1: dw_img_taps<IS, 1>(a, smem, cob, cib, slice); break;
-    case 2: dw_img_taps<IS, 2>(a, smem, cob, cib, slice); break;
-    default: dw_img_taps<IS, 3>(a, smem, cob, cib, slice); break;
+    case 0: dw_img_taps<IS, 0>(a, cob, cib, slice); break;
+    case 1: dw_img_taps<IS, 1>(a, cob, cib, slice); break;
+    case 2: dw_img_taps<IS, 2>(a, cob, cib, slice); break;
+    default: dw_img_taps<IS, 3>(a, cob, cib, slice); break;
   }
 }
 

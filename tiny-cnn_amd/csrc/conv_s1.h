@@ -22,8 +22,8 @@ constexpr int s1_niq(int R, int S, int TC, int TM, int TN) {
   return n > 16 ? 16 : n;
 }
 
-// The three-part bf16 kernel (conv_x3_inst.hip): 16 channels a chunk, words of eight channels that
-// a thread stages per chunk at most (32 registers each).
+// The three-part bf16 kernel (conv_x3_body.h): 16 channels a chunk, words of eight channels that
+// a thread stages per chunk at most (32 registers each; 1 x 1: the tile shared by filter taps).
 constexpr int X3_KCH = 16;
 constexpr int x3_items(int TM, int TN) { return TM * TN >= 4 || TM * TN == 1 ? 1 : 2; }
 // rows of the packed filters: whole tiles of either width
@@ -73,8 +73,7 @@ struct S1Plan {
   int splits;
 };
 
-// the plan of a dX that shares its launch with the weight gradient (conv_bwd_pair.hip); ok = false also
-// where the three-part kernel runs dX
+// the plan of a dX that shares its launch with the weight gradient (conv_bwd_pair.hip)
 S1Plan make_s1_pair_plan(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw);
 int finish_s1_split(const S1Plan &p, const float *bias, ActGrad ag, float *out, float *act_out, int act_kind);
 

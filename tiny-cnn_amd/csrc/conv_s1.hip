@@ -126,9 +126,10 @@ void choose_split(S1Plan &p, int kch, long blocks) {
 // Candidates run from the largest workgroup tile to the smallest; the first one that yields
 // at least 256 workgroups wins, else the one with the most workgroups, and shapes that cannot
 // even fill a quarter of the chip are left to the split-K GEMM.
-// small_tiles: only workgroups of 32 channels x 128 pixels (conv_bwd_pair.hip), however few.
+// by_taps: the three-part kernel's workgroup of 32 channels x 128 pixels that the waves share by
+// filter taps (conv_bwd_pair.hip), however few of them, and split over the reduction channels.
 S1Plan make_plan_of(bool x3, int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph,
-                    int pw, bool small_tiles = false) {
+                    int pw, bool by_taps = false) {
   S1Plan best;
   best.ok = false;
   best.x3 = x3;
@@ -141,14 +142,13 @@ S1Plan make_plan_of(bool x3, int R, int S, int batch, int KC, int MC, int IH, in
   // (three parts: tiles of at least two accumulator blocks a wave, or the filter operands that a
   // wave reads for every tap are more than its products cover: 16x16 images, 32 -> 32 channels, 5x5,
   // batch 128: 25 us with one block, 21 in fp32)
-  const int x3t = small_tiles;
-  const int n_cand = !x3 ? 3 : MC > 32 ? (x3t ? 3 : 2) : (x3t ? 2 : 1);
+  const int n_cand = !x3 || by_taps ? 3 : MC > 32 ? 2 : 1;
   long best_blocks = 0;
-  for (int ci = small_tiles ? n_cand - 1 : 0; ci < n_cand; ++ci) {
+  for (int ci = by_taps ? 2 : 0; ci < n_cand; ++ci) {
     S1Plan p;
     p.ok = false;
     p.x3 = x3;
-    const int *narrow = cand_narrow[x3 ? ci + 1 : ci];
+    const int *narrow = cand_narrow[x3 && !by_taps ? 1 : ci];
     p.tc = OW >= 48 ? 64 : OW >= 24 ? 32 : OW >= 12 ? 16 : 8;
     p.tm = MC > 32 ? cand_wide[ci][0] : narrow[0];
     p.tn = MC > 32 ? cand_wide[ci][1] : narrow[1];
@@ -173,10 +173,7 @@ S1Plan make_plan_of(bool x3, int R, int S, int batch, int KC, int MC, int IH, in
       if (p.lds_bytes > 80 * 1024) continue;  // two workgroups a compute unit
       if (static_cast<long>(ti) * KC * IH * IW >= (1L << 29)) continue;  // 32-bit byte offsets inside a tile
       a.mc_pad = x3_mc_pad(MC);
-      if (p.tm * p.tn == 1) {  // (the waves' sums)
-        if (R == 1) continue;
-        p.lds_bytes = std::max<size_t>(p.lds_bytes, 64 * 1024);
-      }
+      if (by_taps) p.lds_bytes = std::max<size_t>(p.lds_bytes, 64 * 1024);  // (the waves' sums)
     } else {
       if (ceil_div(planeq, 256 / kch) > s1_niq(R, S, p.tc, p.tm, p.tn)) continue;
       p.lds_bytes = sizeof(float) * kch * (4 * static_cast<size_t>(planeq) + R * S * 32 * p.tm);
@@ -191,7 +188,7 @@ S1Plan make_plan_of(bool x3, int R, int S, int batch, int KC, int MC, int IH, in
       // unsplit, and a workgroup for every compute unit at least; two where a single short chunk has
       // nothing to cover its loads with (32x32 images, 16 -> 32 channels, 3x3, batch 64: 12.6 us with
       // one a unit, 11.2 in fp32)
-      if (p.tm * p.tn == 1) {
+      if (by_taps) {
         choose_split(p, kch, blocks);
         return p;
       }
@@ -203,7 +200,7 @@ S1Plan make_plan_of(bool x3, int R, int S, int batch, int KC, int MC, int IH, in
     choose_split(p, kch, blocks);
     // short reductions have nothing to overlap their loads with inside a workgroup: ask for
     // more, smaller workgroups then
-    if (small_tiles || blocks >= (KC * R * S < 256 ? 1024 : 256)) return p;
+    if (blocks >= (KC * R * S < 256 ? 1024 : 256)) return p;
     if (blocks > best_blocks) {
       best_blocks = blocks;
       best        = p;
@@ -228,8 +225,7 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 S1Plan make_s1_pair_plan(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw) {
   S1Plan p;
   p.ok = false;
-  if (!ctx().keep_f32 && !make_plan_of(true, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw).ok)
-    p = make_plan_of(true, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw, true);
+  if (!ctx().keep_f32) p = make_plan_of(true, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw, true);
   return p;
 }
 
@@ -267,7 +263,7 @@ size_t conv_s1_workspace_bytes(int R, int S, int batch, int C, int Kc, int flip,
   const int KC = flip ? Kc : C, MC = flip ? C : Kc;
   size_t most = 0;
   for (int k = 0; k < 3; ++k) {  // (which of the kernels runs is the caller's choice as well)
-    const S1Plan p = make_plan_of(k != 0, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw, k == 2);
+    const S1Plan p = make_plan_of(k != 0, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw, /*by_taps=*/k == 2);
     if (!p.ok) continue;
     size_t total = ws_align(conv_s1_packed_bytes(p.x3 ? CONV_PACK_X3 : CONV_PACK_F32, R * S, KC, MC));
     if (p.splits > 1) total += ws_align(sizeof(float) * p.splits * p.args.part_stride);

@@ -1,4 +1,4 @@
-// conv_x3_body.h — the stride-1 convolution (forward and dX) of conv_s1_body.h on the bf16
+// conv_x3_body.h — the stride-1 convolution (forward and dX) of conv_s1_inst.hip on the bf16
 // matrix cores with three-part operands (split_bf16.h): the same tiles and epilogue, another
 // inner loop. Bound: bf16 MFMA issue; 6 instructions of 32768 FLOP stand for one fp32 product.
 //
@@ -11,6 +11,7 @@
 // own operands of the next tap from there while it multiplies the current one (the four waves of
 // a workgroup read the same lines, so all but the first find them in L1), which leaves the LDS
 // to the patch: 41 KB for 64 channels x 4 rows of 64 pixels, two workgroups a compute unit.
+// What a workgroup does; the kernels around it are in conv_x3_inst.hip and conv_bwd_pair.hip.
 #pragma once
 #include "conv_s1_epilogue.h"
 #include "split_bf16.h"
@@ -24,11 +25,10 @@ typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 
 constexpr unsigned X3_NOWHERE = 0x80000000u;  // past the end of every tile's images
 
-// the workgroup at (bx, by, bz) of the grid; lds: the launch's LDS. BY_TAPS: the four waves share the
+// the workgroup at (bx, by, bz) of the grid. BY_TAPS: the four waves share the
 // workgroup's 32 channels x 128 pixels (TM = TN = 1) by filter taps instead of by pixels
 template <int R, int S, int TC, int TM, int TN, bool VEC, bool BY_TAPS>
-__device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, void *lds, const int bx, const int by,
-                                                  const int bz) {
+__device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, const int bx, const int by, const int bz) {
   static_assert(!BY_TAPS || (TM == 1 && TN == 1), "a tile of 32 channels x 128 pixels");
   constexpr int RS     = R * S;
   constexpr int NI     = BY_TAPS ? 1 : x3_items(TM, TN);
@@ -38,7 +38,7 @@ __device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, void *lds
   constexpr int BM     = 32 * TM;
   constexpr int LOG_TC = TC == 64 ? 6 : TC == 32 ? 5 : TC == 16 ? 4 : 3;
 
-  uintx4 *patch = static_cast<uintx4 *>(lds);       // [part][half][pixel]
+  extern __shared__ __align__(16) uintx4 patch[];   // [part][half][pixel]
   const int TRH    = a.TR + R - 1;
   const int planeq = a.TI * TRH * NQ;  // words of one channel of the staged patch
   const int npix   = 4 * planeq;
@@ -156,22 +156,17 @@ __device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, void *lds
     }
   };
 
-  // filter operands of tap u, counted over the chunks
-  auto read_filters = [&](int u, bf16x8 (&wf)[TM][X3_PARTS]) {
-    const char *w = wall + static_cast<size_t>(u) * X3_PARTS * wpart;
-#pragma unroll
-    for (int p = 0; p < X3_PARTS; ++p)
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-        wf[i][p] = *reinterpret_cast<const bf16x8 *>(w + static_cast<size_t>(p) * wpart + (wlane + 512u * i));
-  };
-
   if constexpr (BY_TAPS) {
     // Wave w multiplies the taps u = w, w + 4, .. (counted over the chunks, so the odd one moves
     // round the waves) with all four pixel blocks: the filters are read once per workgroup, not once
     // per wave, and each reading serves 24 products. The patch operands of two blocks are read
     // while the other two are multiplied.
     bf16x8 wf[1][X3_PARTS], wnext[1][X3_PARTS], xf[2][2][X3_PARTS];
+    auto read_filters = [&](int u) {
+      const char *w = wall + static_cast<size_t>(u) * X3_PARTS * wpart;
+#pragma unroll
+      for (int p = 0; p < X3_PARTS; ++p) wnext[0][p] = *reinterpret_cast<const bf16x8 *>(w + static_cast<size_t>(p) * wpart + wlane);
+    };
     const int wave = __builtin_amdgcn_readfirstlane(wn);
     auto read_pair = [&](int pair, int off) {
 #pragma unroll
@@ -185,7 +180,7 @@ __device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, void *lds
     int u = kc_lo / 16 * RS;
     u += (wave - u) & 3;
     fetch(kc_lo);
-    if (u < u_end) read_filters(u, wnext);
+    if (u < u_end) read_filters(u);
     for (int kc0 = kc_lo; kc0 < kc_hi; kc0 += 16) {
       if (kc0 > kc_lo) __syncthreads();  // everyone is done reading the previous chunk
       stage();
@@ -197,7 +192,7 @@ __device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, void *lds
       for (; u < u0 + RS; u += 4) {
 #pragma unroll
         for (int p = 0; p < X3_PARTS; ++p) wf[0][p] = wnext[0][p];
-        if (u + 4 < u_end) read_filters(u + 4, wnext);
+        if (u + 4 < u_end) read_filters(u + 4);
         read_pair(1, tap_at(u - u0));
         if (more) fetch(kc0 + 16);   // (once per chunk, behind the first tap's loads)
         more = false;
@@ -209,7 +204,7 @@ __device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, void *lds
     }
     // the waves' sums of a pixel block are added in wave order by the wave that stores the block
     __syncthreads();
-    floatx4 *red = static_cast<floatx4 *>(lds);   // [wave][block][r/4][lane]
+    floatx4 *red = reinterpret_cast<floatx4 *>(patch);   // [wave][block][r/4][lane]
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -229,7 +224,16 @@ __device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, void *lds
     s1_epilogue<TC, 1, 1>(a, sum, wn, lane, img0, y0, x0, m0, bz);
     return;
   } else {
+  // operands of tap u, counted over the chunks
   bf16x8 wf[2][TM][X3_PARTS], xf[TN][X3_PARTS];
+  auto read_filters = [&](int u, int to) {
+    const char *w = wall + static_cast<size_t>(u) * X3_PARTS * wpart;
+#pragma unroll
+    for (int p = 0; p < X3_PARTS; ++p)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+        wf[to][i][p] = *reinterpret_cast<const bf16x8 *>(w + static_cast<size_t>(p) * wpart + (wlane + 512u * i));
+  };
   auto read_patch = [&](int t) {
 #pragma unroll
     for (int p = 0; p < X3_PARTS; ++p)
@@ -248,7 +252,7 @@ __device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, void *lds
   // additions behind the products of all but the first chunk it is 327 / 290 / 50: what the matrix
   // cores and the power limit leave.
   fetch(kc_lo);
-  read_filters(kc_lo / 16 * RS, wf[0]);
+  read_filters(kc_lo / 16 * RS, 0);
   for (int kc0 = kc_lo; kc0 < kc_hi; kc0 += 16) {
     const bool more = kc0 + 16 < kc_hi;
     if (kc0 > kc_lo) __syncthreads();  // everyone is done reading the previous chunk
@@ -257,7 +261,7 @@ __device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, void *lds
 #pragma unroll
     for (int t = 0; t < RS; ++t) {
       const int cur = t & 1;
-      if (t + 1 < RS || more) read_filters(kc0 / 16 * RS + t + 1, wf[cur ^ 1]);
+      if (t + 1 < RS || more) read_filters(kc0 / 16 * RS + t + 1, cur ^ 1);
       read_patch(t);
       if (t == 0 && more) fetch(kc0 + 16);
       mfma_x3<TM, TN>(acc, wf[cur], xf, x3_sign(kc0 / 16 * RS + t));

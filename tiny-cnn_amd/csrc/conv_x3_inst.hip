@@ -6,15 +6,14 @@ namespace tdh {
 
 namespace {
 
-template <int R, int S, int TC, int TM, int TN, bool VEC, bool BY_TAPS>
+template <int R, int S, int TC, int TM, int TN, bool VEC>
 __global__ void __launch_bounds__(256, 2) conv_x3_kernel(const ConvS1Args a) {
-  extern __shared__ __align__(16) uint32_t x3_lds[];
-  conv_x3_workgroup<R, S, TC, TM, TN, VEC, BY_TAPS>(a, x3_lds, blockIdx.x, blockIdx.y, blockIdx.z);
+  conv_x3_workgroup<R, S, TC, TM, TN, VEC, false>(a, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
-template <int R, int S, int TC, int TM, int TN, bool VEC, bool BY_TAPS = false>
+template <int R, int S, int TC, int TM, int TN, bool VEC>
 int launch_x3_inst(const S1Plan &p) {
-  auto kernel = conv_x3_kernel<R, S, TC, TM, TN, VEC, BY_TAPS>;
+  auto kernel = conv_x3_kernel<R, S, TC, TM, TN, VEC>;
   if (p.lds_bytes > 64 * 1024) {
     static size_t raised = 0;
     if (p.lds_bytes > raised) {
@@ -33,10 +32,7 @@ int launch_x3_tc(const S1Plan &p) {
   switch (p.tm * 10 + p.tn) {
     case 22: return launch_x3_inst<R, S, TC, 2, 2, VEC>(p);
     case 21: return launch_x3_inst<R, S, TC, 2, 1, VEC>(p);
-    case 12: return launch_x3_inst<R, S, TC, 1, 2, VEC>(p);
-    default:  // by filter taps; a 1x1 window has only one
-      if constexpr (R > 1) return launch_x3_inst<R, S, TC, 1, 1, VEC, true>(p);
-      else return set_error(TDH_ERR_INVALID, "three-part convolution: no such tile");
+    default: return launch_x3_inst<R, S, TC, 1, 2, VEC>(p);
   }
 }
 

@@ -10,6 +10,7 @@
 // runtime maps the caller's pages and copies without staging: the limits lie there.)
 #include <atomic>
 #include <cstring>
+#include <mutex>
 
 #include "common.h"
 
@@ -28,6 +29,7 @@ struct Ring {
   int next = 0;
 };
 Ring g_ring;
+std::mutex g_ring_mutex;  // (callers on several threads: a download keeps its piece until its data has left it)
 
 // dst and src share the alignment of `word` bytes (16, 4 or 1)
 template <typename W>
@@ -104,6 +106,7 @@ bool host_copy_up_applies(size_t bytes) { return bytes <= HC_PIECE; }
 bool host_copy_down_applies(size_t bytes) { return bytes <= HC_MAX_DOWN; }
 
 int host_copy_up(void *dst, const void *src, size_t bytes) {
+  std::lock_guard<std::mutex> lock(g_ring_mutex);
   int i = 0;
   TDH_TRY(take_piece(&i));
   std::memcpy(g_ring.data + i * HC_PIECE, src, bytes);
@@ -111,6 +114,7 @@ int host_copy_up(void *dst, const void *src, size_t bytes) {
 }
 
 int host_copy_down(void *dst, const void *src, size_t bytes) {
+  std::lock_guard<std::mutex> lock(g_ring_mutex);
   int i = 0;
   TDH_TRY(take_piece(&i));
   TDH_TRY(launch_piece(g_ring.data + i * HC_PIECE, src, bytes, i));
@@ -120,6 +124,7 @@ int host_copy_down(void *dst, const void *src, size_t bytes) {
 }
 
 void host_copy_release() {
+  std::lock_guard<std::mutex> lock(g_ring_mutex);
   if (g_ring.data) (void)hipHostFree(g_ring.data);
   if (g_ring.turn) (void)hipHostFree(g_ring.turn);
   g_ring = Ring();

@@ -675,14 +675,19 @@ int tdh_net_create(const tdh_layer *layers, int n_layers, int max_batch, int fla
     }
     if ((flags & TDH_NET_GRAPH) && L.spec.kind == TDH_L_CONV && L.spec.conv.w_stride == 1 &&
         L.spec.conv.h_stride == 1) {
-      if ((rc = net_alloc(net, L.w_size, &L.wp_fwd, false))) break;
-      if ((rc = net_alloc(net, L.w_size, &L.wp_dx, false))) break;
-      for (int flip = 0; flip < 2 && rc == TDH_OK; ++flip)
+      // (one buffer: an allocation takes the host some 100 us)
+      auto padded = [](size_t floats) { return ceil_div_sz(floats, 64) * 64; };
+      size_t at[2] = {0, 0}, total = 2 * padded(L.w_size);
+      for (int flip = 0; flip < 2; ++flip)
         if (conv_packed_kind(&L.spec.conv, max_batch, flip) == CONV_PACK_X3 ||
-            (flip && conv_bwd_pairs(&L.spec.conv, max_batch)))
-          rc = net_alloc(net, conv_packed_bytes(&L.spec.conv, CONV_PACK_X3, flip) / sizeof(float),
-                         flip ? &L.wx_dx : &L.wx_fwd, false);
-      if (rc != TDH_OK) break;
+            (flip && conv_bwd_pairs(&L.spec.conv, max_batch))) {
+          at[flip] = total;
+          total += padded(conv_packed_bytes(&L.spec.conv, CONV_PACK_X3, flip) / sizeof(float));
+        }
+      if ((rc = net_alloc(net, total, &L.wp_fwd, false))) break;
+      L.wp_dx = L.wp_fwd + padded(L.w_size);
+      if (at[0]) L.wx_fwd = L.wp_fwd + at[0];
+      if (at[1]) L.wx_dx = L.wp_fwd + at[1];
     }
     if (!L.tbl.empty()) {
       float *p = nullptr;
