@@ -61,7 +61,8 @@ struct StreamSwap {
 };
 
 Context &ctx();
-// Products inside the scope keep to fp32 instructions (see Context::keep_f32).
+// Products inside the scope keep to fp32 instructions and to one order of their sums whatever the
+// batch's size (see Context::keep_f32).
 struct KeepF32 {
   const bool was;
   explicit KeepF32(bool on) : was(ctx().keep_f32) { ctx().keep_f32 = was || on; }
@@ -359,6 +360,11 @@ bool conv_fwd_pool_applies_act(const tdh_conv_desc *d, int batch, bool prepacked
 // the forward kernel of this layer can leave `y` out (null) when it writes the activation layer
 // or the pool behind the convolution itself
 bool conv_fwd_out_optional(const tdh_conv_desc *d, int batch, bool prepacked);
+// conv_fwd_direct.hip: forward pass of a layer that is a few small tiles, with the layers behind it
+bool conv_fwd_direct_applicable(int batch, int C, int Kc, int H, int W, int OH, int OW, int R, int S);
+int conv_fwd_direct_run(int batch, int C, int Kc, const float *x, const float *w, const float *bias, float *out, int H, int W,
+                        int OH, int OW, int R, int S, int sh, int sw, int dh, int dw, int ph, int pw, float *act_out,
+                        int act_kind, const PoolFuse *pool);
 // conv_fwd_small.hip
 bool conv_fwd_small_applicable(int batch, int C, int Kc, int H, int W, int OH, int OW, int R, int S,
                                int sh, int sw, int dh, int dw, int ph, int pw);
@@ -383,6 +389,11 @@ bool conv_fwd_applies_act(const tdh_conv_desc *d, int batch, bool prepacked);
 // packs w (masked by the device-resident connection table, if any) into wp
 int conv_pack_filters(const tdh_conv_desc *d, int kind, int flip, const float *w, const uint8_t *tbl_resident,
                       void *wp);
+// fc_fwd_direct.hip: a few samples, with the activation or (applies_softmax) the softmax behind the layer
+bool fc_fwd_direct_applicable(int in, int out, int batch);
+bool fc_fwd_direct_applies_softmax(int in, int out, int batch);
+int fc_fwd_direct_run(int in, int out, int batch, const float *x, const float *w, const float *bias, float *y,
+                      float *act_out, int act_kind);
 int fc_fwd(int in, int out, int has_bias, int batch, const float *x, const float *w,
            const float *b, float *y, float *act_out = nullptr, int act_kind = 0);
 // The backward pass of a 2x2 / stride-2 max-pool layer in front of a fully-connected layer,

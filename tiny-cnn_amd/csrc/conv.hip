@@ -1113,6 +1113,10 @@ static void launch_small_cin_dx_window(const ConvGeom &g, const DxsPlan &p, int 
 }
 
 
+static bool fwd_direct_applies(const ConvGeom &g, int batch) {
+  return conv_fwd_direct_applicable(batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.R, g.S);
+}
+
 static bool fwd_small_applies(const ConvGeom &g, int batch) {
   // (small windows over many channels are short reductions as well, but no first layers)
   if (g.C >= 16 && g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 &&
@@ -1277,7 +1281,7 @@ bool conv_fwd_applies_act(const tdh_conv_desc *d, int batch, bool prepacked) {
 // the stride-1 kernel runs this forward pass (with filters packed by the caller, or by itself)
 static bool fwd_s1_applies(const tdh_conv_desc *d, const ConvGeom &g, int batch, bool prepacked) {
   if (prepacked) return conv_packed_kind(d, batch, 0) != CONV_PACK_NONE;
-  return !fwd_small_applies(g, batch) && g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 &&
+  return !fwd_direct_applies(g, batch) && !fwd_small_applies(g, batch) && g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 &&
          conv_s1_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
 }
 
@@ -1286,22 +1290,22 @@ bool conv_fwd_fuses_pool(const tdh_conv_desc *d, const tdh_pool_desc *pool, int 
   if (!(pool->pool_w == 2 && pool->pool_h == 2 && pool->stride_w == 2 && pool->stride_h == 2 &&
         pool->in_w == g.OW && pool->in_h == g.OH && pool->in_c == g.Kc && g.OW % 2 == 0 && g.OH % 2 == 0))
     return false;
-  if (!prepacked && fwd_small_applies(g, batch)) return true;
+  if (!prepacked && (fwd_direct_applies(g, batch) || fwd_small_applies(g, batch))) return true;
   return fwd_s1_applies(d, g, batch, prepacked) &&
          conv_s1_fuses_pool(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
 }
 
 bool conv_fwd_out_optional(const tdh_conv_desc *d, int batch, bool prepacked) {
   const ConvGeom g = make_geom(d);
-  if (!prepacked && fwd_small_applies(g, batch)) return true;
+  if (!prepacked && (fwd_direct_applies(g, batch) || fwd_small_applies(g, batch))) return true;
   return fwd_s1_applies(d, g, batch, prepacked) &&
          conv_s1_single_pass(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
 }
 
 bool conv_fwd_pool_applies_act(const tdh_conv_desc *d, int batch, bool prepacked, int act_kind) {
   const ConvGeom g = make_geom(d);
-  // the first-layer kernel applies any pointwise kind, the stride-1 kernel relu
-  if (!prepacked && fwd_small_applies(g, batch)) return true;
+  // the direct and the first-layer kernel apply any pointwise kind, the stride-1 kernel relu
+  if (!prepacked && (fwd_direct_applies(g, batch) || fwd_small_applies(g, batch))) return true;
   return act_kind == TDH_ACT_RELU;
 }
 
@@ -1309,7 +1313,7 @@ int conv_packed_kind(const tdh_conv_desc *d, int batch, int flip) {
   const ConvGeom g = make_geom(d);
   if (g.sh != 1 || g.sw != 1) return CONV_PACK_NONE;
   if (!flip)
-    return g.dh == 1 && g.dw == 1 && !fwd_small_applies(g, batch)
+    return g.dh == 1 && g.dw == 1 && !fwd_direct_applies(g, batch) && !fwd_small_applies(g, batch)
              ? conv_s1_packed_kind(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w)
              : CONV_PACK_NONE;
   DxsPlan dxs;
@@ -1350,6 +1354,9 @@ int conv2d_fwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
   const uint8_t *tbl_dev;
   const float *w_eff;
   TDH_TRY(prepare_table(d, g, w, tbl_resident, &tbl_dev, &w_eff));
+  if (fwd_direct_applies(g, batch))
+    return conv_fwd_direct_run(batch, g.C, g.Kc, x, w_eff, d->has_bias ? b : nullptr, y, g.H, g.W, g.OH, g.OW, g.R, g.S,
+                               g.sh, g.sw, g.dh, g.dw, g.pad_h, g.pad_w, act_out, act_kind, pool);
   if (fwd_small_applies(g, batch))
     return conv_fwd_small_run(batch, g.C, g.Kc, x, w_eff, d->has_bias ? b : nullptr, y, g.H, g.W, g.OH, g.OW,
                               g.R, g.S, g.sh, g.sw, g.dh, g.dw, g.pad_h, g.pad_w, act_out, act_kind, pool);

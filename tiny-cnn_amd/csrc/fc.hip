@@ -950,6 +950,8 @@ size_t fc_workspace_bytes(int in, int out, int batch) {
 
 int fc_fwd(int in, int out, int has_bias, int batch, const float *x, const float *w,
            const float *b, float *y, float *act_out, int act_kind) {
+  if (fc_fwd_direct_applicable(in, out, batch))
+    return fc_fwd_direct_run(in, out, batch, x, w, has_bias ? b : nullptr, y, act_out, act_kind);
   StridedOperand A{x, in, 1, batch};   // X[s][k], k contiguous
   StridedOperand B{w, 1, out, out};    // W[k][n], n contiguous
   if (act_out) {  // the pointwise activation layer that follows leaves the same kernel

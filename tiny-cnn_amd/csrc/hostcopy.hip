@@ -44,7 +44,7 @@ __device__ __forceinline__ void copy_words(void *dst, const void *src, const uin
 }
 
 __global__ void __launch_bounds__(HC_THREADS)
-host_copy_kernel(void *dst, const void *src, const uint32_t bytes, uint32_t *turn, const uint32_t value) {
+host_copy_kernel(void *dst, const void *src, const uint32_t bytes, const bool down, uint32_t *turn, const uint32_t value) {
   const uintptr_t at = reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src);
   if (at % 16 == 0)
     copy_words<uint4>(dst, src, bytes);
@@ -52,9 +52,11 @@ host_copy_kernel(void *dst, const void *src, const uint32_t bytes, uint32_t *tur
     copy_words<uint32_t>(dst, src, bytes);
   else
     copy_words<char>(dst, src, bytes);
-  __threadfence_system();
+  // Of an upload the host waits only for the piece to have been read, which the barrier says; what a
+  // download has written must be there before the word.
+  if (down) __threadfence_system();
   __syncthreads();
-  if (threadIdx.x == 0) __hip_atomic_store(turn, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (threadIdx.x == 0) __hip_atomic_store(turn, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 int ring_ready() {
@@ -92,9 +94,9 @@ int take_piece(int *piece) {
   return wait_piece(*piece);
 }
 
-int launch_piece(void *dst, const void *src, size_t bytes, int i) {
+int launch_piece(void *dst, const void *src, size_t bytes, bool down, int i) {
   const uint32_t value = ++g_ring.issued[i];
-  TDH_LAUNCH(host_copy_kernel, dim3(1), dim3(HC_THREADS), 0, ctx().stream, dst, src, static_cast<uint32_t>(bytes),
+  TDH_LAUNCH(host_copy_kernel, dim3(1), dim3(HC_THREADS), 0, ctx().stream, dst, src, static_cast<uint32_t>(bytes), down,
              g_ring.turn + i, value);
   TDH_LAUNCH_CHECK();
   return TDH_OK;
@@ -110,14 +112,14 @@ int host_copy_up(void *dst, const void *src, size_t bytes) {
   int i = 0;
   TDH_TRY(take_piece(&i));
   std::memcpy(g_ring.data + i * HC_PIECE, src, bytes);
-  return launch_piece(dst, g_ring.data + i * HC_PIECE, bytes, i);
+  return launch_piece(dst, g_ring.data + i * HC_PIECE, bytes, /*down=*/false, i);
 }
 
 int host_copy_down(void *dst, const void *src, size_t bytes) {
   std::lock_guard<std::mutex> lock(g_ring_mutex);
   int i = 0;
   TDH_TRY(take_piece(&i));
-  TDH_TRY(launch_piece(g_ring.data + i * HC_PIECE, src, bytes, i));
+  TDH_TRY(launch_piece(g_ring.data + i * HC_PIECE, src, bytes, /*down=*/true, i));
   TDH_TRY(wait_piece(i));
   std::memcpy(dst, g_ring.data + i * HC_PIECE, bytes);
   return TDH_OK;

@@ -554,7 +554,9 @@ int forward(tdh_net *net, int batch, const float *x, bool packed = false, const 
           if (softmax_behind) ++i;
         } else
         if ((net->flags & TDH_NET_FUSE_ACT_GRAD) && i + 1 < n && net->layers[i + 1].spec.kind == TDH_L_ACT &&
-            is_pointwise_act(net->layers[i + 1].spec.act)) {
+            (is_pointwise_act(net->layers[i + 1].spec.act) ||
+             (!xent_t && net->layers[i + 1].spec.act == TDH_ACT_SOFTMAX &&
+              fc_fwd_direct_applies_softmax(s.fc_in, s.fc_out, batch)))) {
           // the activation layer behind the product leaves the same kernel
           TDH_TRY(fc_fwd(s.fc_in, s.fc_out, s.fc_bias, batch, in, L.w, L.b, L.out, net->layers[i + 1].out,
                          net->layers[i + 1].spec.act));
