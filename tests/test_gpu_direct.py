@@ -60,3 +60,34 @@ def test_inference_matches_oracle(T, O, W, spec, flags, batch):
     for i in range(len(spec)):
         assert_close(net.layer_out(i, batch).ravel(), ref.layer_out(i, batch).ravel(), what=f"layer {i}")
     net.close()
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("cfg", [
+    # in_w, in_h, in_c, k, out_c, same, stride, batch
+    (5, 5, 1, 5, 1, False, 1, 1),         # one output pixel
+    (9, 7, 3, 3, 16, True, 1, 1),         # db in a tile of its own columns' end: 27 + 1
+    (9, 8, 5, 3, 17, True, 1, 2),         # 45 + 1 columns, rows that are no multiple of four
+    (8, 8, 16, 1, 20, False, 1, 3),       # 16 columns: db alone in the second tile
+    (12, 12, 32, 5, 33, True, 1, 2),      # 825 indices of dX: sixteen waves
+    (16, 16, 8, 3, 24, True, 1, 8),       # 2048 pixels
+    (11, 10, 20, 3, 12, False, 2, 3),     # strided, rows that no window reaches
+    (13, 12, 6, 4, 10, True, 3, 2),       # stride 3, window of 4
+    (12, 9, 4, 1, 9, False, 2, 2),        # stride larger than the window
+])
+def test_conv_gradients_match_oracle(T, O, cfg, accumulate):
+    iw, ih, ic, k, oc, same, st, bs = cfg
+    rng = np.random.default_rng(12)
+    kw = dict(pad_same=same, w_stride=st, h_stride=st)
+    d = T.conv_desc(iw, ih, ic, k, k, oc, **kw)
+    ow, oh = T.conv_out_shape(d)
+    x = rng.standard_normal((bs, ic * ih * iw)).astype(np.float32)
+    w = rng.uniform(-0.3, 0.3, oc * ic * k * k).astype(np.float32)
+    dy = rng.standard_normal((bs, oc * oh * ow)).astype(np.float32)
+    start = [rng.standard_normal(n).astype(np.float32) if accumulate else np.full(n, 7, np.float32) for n in (w.size, oc)]
+    dx, dw, db = T.DevBuf(x.shape), T.to_device(start[0]), T.to_device(start[1])
+    T.conv2d_bwd(d, bs, T.to_device(x), T.to_device(w), T.to_device(dy), dx, dw, db, accumulate=accumulate)
+    want = O.conv2d_bwd(O.conv_desc(iw, ih, ic, k, k, oc, **kw), x, w, dy)
+    base = [np.zeros(1), *(start if accumulate else (np.zeros(1), np.zeros(1)))]
+    for g, r, b, name in zip((dx, dw, db), want, base, ("dx", "dw", "db")):
+        assert_close(g.numpy().ravel(), r.ravel() + b, what=f"{cfg} {name}")

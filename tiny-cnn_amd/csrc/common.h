@@ -351,7 +351,7 @@ int conv2d_fwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
 // dX, dW and db of this (first) convolution leave conv2d_bwd as one launch when all three are
 // asked for together (pooled: the gradient is read through the max-pool behind the layer)
 bool conv_bwd_one_launch(const tdh_conv_desc *d, int batch, bool pooled);
-// ... of this later convolution; dX reads filters packed as CONV_PACK_X3
+// ... of this later convolution; dX reads filters packed as CONV_PACK_X3, if any
 bool conv_bwd_pairs(const tdh_conv_desc *d, int batch);
 // the forward kernel of this convolution can also compute the max-pool layer `pool` behind it
 bool conv_fwd_fuses_pool(const tdh_conv_desc *d, const tdh_pool_desc *pool, int batch, bool prepacked);
@@ -458,6 +458,11 @@ size_t conv_dw_halo_workspace_bytes(int R, int S, int batch, int C, int Kc, int 
 int conv_dw_halo_run(int R, int S, int batch, int C, int Kc, const float *x, const float *dy,
                      float *dw, int H, int W, int OH, int OW, int ph, int pw, int accumulate,
                      float *db = nullptr);
+// conv_bwd_direct.hip: any of dX, dW and db of a layer that is a few small tiles, as one launch
+bool conv_bwd_direct_applicable(int batch, int C, int Kc, int H, int W, int OH, int OW, int R, int S);
+int conv_bwd_direct_run(int batch, int C, int Kc, const float *x, const float *w, const float *dy, float *dx, float *dw,
+                        float *db, int H, int W, int OH, int OW, int R, int S, int sh, int sw, int ph, int pw,
+                        int accumulate, ActGrad dx_act);
 // conv_bwd_pair.hip: dX, dW and db of a 5x5 convolution on small images as one launch
 bool conv_bwd_pair_applicable(int R, int S, int batch, int C, int Kc, int H, int W, int OH, int OW, int ph, int pw);
 int conv_bwd_pair_run(int R, int S, int batch, int C, int Kc, int H, int W, int ph, int pw, const float *x,

@@ -1247,6 +1247,14 @@ bool defer_reduce(const float *partial, int splits, int M, int N, const EpiRowMa
   return true;
 }
 
+static bool bwd_direct_applies(const tdh_conv_desc *d, const ConvGeom &g, int batch) {
+  if (d->tbl || g.dh != 1 || g.dw != 1 || !conv_bwd_direct_applicable(batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.R, g.S))
+    return false;
+  // (where the pair of MFMA-tiled kernels is one launch as well, it wins from 1024 pixels on)
+  return static_cast<long>(batch) * g.OH * g.OW <= 1024 || g.sh != 1 || g.sw != 1 ||
+         !conv_bwd_pair_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
+}
+
 static bool dw_small_applies(const tdh_conv_desc *d, const ConvGeom &g, int batch) {
   return !d->tbl && conv_dw_small_applicable(batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.R, g.S, g.sh, g.sw,
                                              g.dh, g.dw, g.pad_h, g.pad_w);
@@ -1267,7 +1275,7 @@ bool conv_bwd_reads_pooled(const tdh_conv_desc *d, const tdh_pool_desc *pool, in
 
 bool conv_dw_gives_db(const tdh_conv_desc *d, int batch) {
   const ConvGeom g = make_geom(d);
-  if (dw_small_applies(d, g, batch)) return true;
+  if (dw_small_applies(d, g, batch) || bwd_direct_applies(d, g, batch)) return true;
   return !d->tbl && g.sh == 1 && g.sw == 1 &&
          conv_dw_halo_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
 }
@@ -1390,8 +1398,9 @@ bool conv_bwd_one_launch(const tdh_conv_desc *d, int batch, bool pooled) {
 
 bool conv_bwd_pairs(const tdh_conv_desc *d, int batch) {
   const ConvGeom g = make_geom(d);
-  return !d->tbl && g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 &&
-         conv_bwd_pair_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
+  return bwd_direct_applies(d, g, batch) ||
+         (!d->tbl && g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 &&
+          conv_bwd_pair_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w));
 }
 
 // the slices of the first convolution's launch: one per band and image
@@ -1479,6 +1488,9 @@ int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
                                 one_launch_band(d, g, batch, true)));
     return TDH_OK;
   }
+  if (bwd_direct_applies(d, g, batch))
+    return conv_bwd_direct_run(batch, g.C, g.Kc, x, w, dy, dx, dw, db, g.H, g.W, g.OH, g.OW, g.R, g.S, g.sh, g.sw,
+                               g.pad_h, g.pad_w, accumulate, dx_act);
   if (dx && dw && conv_bwd_pairs(d, batch) && !((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy)) & 15))
     return conv_bwd_pair_run(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.pad_h, g.pad_w, x, dy, w, prepacked_dx, dx, dx_act,
                              dw, db, accumulate);
