@@ -74,6 +74,11 @@ def test_inference_matches_oracle(T, O, W, spec, flags, batch):
     (11, 10, 20, 3, 12, False, 2, 3),     # strided, rows that no window reaches
     (13, 12, 6, 4, 10, True, 3, 2),       # stride 3, window of 4
     (12, 9, 4, 1, 9, False, 2, 2),        # stride larger than the window
+    # too many pixels for that launch: the bias gradient is a column of the weight gradient's product
+    (27, 25, 5, 3, 9, False, 2, 17),      # 2856 pixels, 46 columns
+    (31, 29, 1, 1, 5, True, 1, 3),        # one weight and the bias
+    (25, 26, 7, 3, 40, True, 1, 4),       # 64 columns with the bias gradient's
+    (25, 26, 32, 1, 6, True, 1, 4),       # 32 columns without it: it stays a launch of its own
 ])
 def test_conv_gradients_match_oracle(T, O, cfg, accumulate):
     iw, ih, ic, k, oc, same, st, bs = cfg

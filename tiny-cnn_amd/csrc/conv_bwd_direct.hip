@@ -215,13 +215,14 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 // The lines of conv_fwd_direct.hip, and 2048 output pixels at most: dW gathers its columns pixel by
 // pixel, 16 waves to a compute unit, and from there on that takes as long as the launches it saves
 // (us before / here: 16x16 images, 32 -> 32, 5x5, 8 images 19.5 / 18.0; 32x32, 3 -> 32, 4 images 22.5 /
-// 27.9). Not where a result must not depend on the kernel: the order of the sums is its own.
+// 27.9). dX has no use for that many waves: with them 512 tiles of it at most (42x11, stride 2, 60 -> 13,
+// 14 images, 1620 tiles: 27.7 / 28.0). Not where a result must not depend on the kernel: the order of the sums is its own.
 bool conv_bwd_direct_applicable(int batch, int C, int Kc, int H, int W, int OH, int OW, int R, int S) {
   const long in_pixels = static_cast<long>(batch) * H * W, pixels = static_cast<long>(batch) * OH * OW;
   const long k = static_cast<long>(Kc) * R * S, cols = static_cast<long>(C) * R * S + 1;
   const long dx_tiles = ceil_div(C, 16) * ((in_pixels + 15) / 16), dw_tiles = ceil_div(Kc, 16) * ((cols + 15) / 16);
   return !ctx().keep_f32 && R <= 31 && S <= 31 && in_pixels <= 32768 &&
-         k <= BD_K_MAX && dx_tiles <= 2048 && dx_tiles * k <= 600000 && pixels <= 2048 && dw_tiles <= 2048 &&
+         k <= BD_K_MAX && dx_tiles <= (pixels > 512 ? 512 : 2048) && dx_tiles * k <= 600000 && pixels <= 2048 && dw_tiles <= 2048 &&
          dw_tiles * pixels <= 600000 && static_cast<long>(batch) * C * H * W < (1L << 30) && pixels * Kc < (1L << 30);
 }
 
