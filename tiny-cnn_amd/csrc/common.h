@@ -335,8 +335,15 @@ int finish_split_sum();      // the reduction as a launch of its own, when nobod
 
 
 // conv.hip / fc.hip
-// prepacked: filters already packed by conv_pack_filters for this direction, in the kind that
-// conv_packed_kind names
+// The layouts of packed filters: none, floats (conv_s1_inst.hip) or three bf16 parts (conv_x3_inst.hip)
+enum { CONV_PACK_NONE = 0, CONV_PACK_F32 = 1, CONV_PACK_X3 = 2 };
+// Filters packed by conv_pack_filters for one direction of a layer, with the layout they are in: a
+// kernel that reads another one packs for itself.
+struct PackedFilters {
+  const void *data = nullptr;
+  int kind         = CONV_PACK_NONE;
+  explicit operator bool() const { return data != nullptr; }
+};
 // A 2x2 / stride-2 max-pool layer (and the pointwise activation behind it) computed by the
 // forward kernel of the layer in front of it
 struct PoolFuse {
@@ -346,13 +353,14 @@ struct PoolFuse {
   int act_kind;
 };
 int conv2d_fwd(const tdh_conv_desc *d, int batch, const float *x, const float *w, const float *b,
-               float *y, const uint8_t *tbl_resident = nullptr, const void *prepacked = nullptr,
+               float *y, const uint8_t *tbl_resident = nullptr, PackedFilters prepacked = PackedFilters(),
                float *act_out = nullptr, int act_kind = 0, const PoolFuse *pool = nullptr);
 // dX, dW and db of this (first) convolution leave conv2d_bwd as one launch when all three are
 // asked for together (pooled: the gradient is read through the max-pool behind the layer)
 bool conv_bwd_one_launch(const tdh_conv_desc *d, int batch, bool pooled);
-// ... of this later convolution; dX reads filters packed as CONV_PACK_X3, if any
-bool conv_bwd_pairs(const tdh_conv_desc *d, int batch);
+// ... of this later convolution with these tensors (null: as aligned as the library's own); dX reads
+// filters packed as CONV_PACK_X3, if any
+bool conv_bwd_pairs(const tdh_conv_desc *d, int batch, const float *x = nullptr, const float *dy = nullptr);
 // the forward kernel of this convolution can also compute the max-pool layer `pool` behind it
 bool conv_fwd_fuses_pool(const tdh_conv_desc *d, const tdh_pool_desc *pool, int batch, bool prepacked);
 // ... and the pointwise activation of this kind behind that pool
@@ -375,14 +383,13 @@ int conv_fwd_small_run(int batch, int C, int Kc, const float *x, const float *w,
 // and may be null); only where conv_bwd_reads_pooled says so
 int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w, const float *dy,
                float *dx, float *dw, float *db, int accumulate, ActGrad dx_act,
-               const uint8_t *tbl_resident = nullptr, const void *prepacked_dx = nullptr,
+               const uint8_t *tbl_resident = nullptr, PackedFilters prepacked_dx = PackedFilters(),
                const PoolGather *dy_pool = nullptr);
 // the backward kernels of this layer (the two of a first layer: few input channels, stride 1)
 // can read their output gradient through this 2x2 / stride-2 max-pool over the layer's output
 bool conv_bwd_reads_pooled(const tdh_conv_desc *d, const tdh_pool_desc *pool, int batch);
-// the packed filters that forward (flip = 0) / dX (flip = 1) of this layer reads: none, floats
-// (conv_s1_inst.hip) or three bf16 parts (conv_x3_inst.hip), and the bytes they take
-enum { CONV_PACK_NONE = 0, CONV_PACK_F32 = 1, CONV_PACK_X3 = 2 };
+// the kind of packed filters that forward (flip = 0) / dX (flip = 1) of this layer reads, and the bytes
+// they take
 int conv_packed_kind(const tdh_conv_desc *d, int batch, int flip);
 size_t conv_packed_bytes(const tdh_conv_desc *d, int kind, int flip);
 bool conv_fwd_applies_act(const tdh_conv_desc *d, int batch, bool prepacked);
@@ -436,7 +443,7 @@ size_t conv_s1_workspace_bytes(int R, int S, int batch, int C, int Kc, int flip,
 int conv_s1_run(int R, int S, int batch, int C, int Kc, int flip, const float *in, const float *w,
                 const uint8_t *tbl_dev, const float *bias, float *out, int IH, int IW, int OH,
                 int OW, int ph, int pw, ActGrad ag, const char *tag,
-                const void *prepacked = nullptr, float *act_out = nullptr, int act_kind = 0,
+                PackedFilters prepacked = PackedFilters(), float *act_out = nullptr, int act_kind = 0,
                 const PoolFuse *pool = nullptr);
 // the forward kernel of this shape can also compute the 2x2 / stride-2 max-pool behind it (and
 // a relu behind that pool); `out` may then be null
@@ -466,7 +473,7 @@ int conv_bwd_direct_run(int batch, int C, int Kc, const float *x, const float *w
 // conv_bwd_pair.hip: dX, dW and db of a 5x5 convolution on small images as one launch
 bool conv_bwd_pair_applicable(int R, int S, int batch, int C, int Kc, int H, int W, int OH, int OW, int ph, int pw);
 int conv_bwd_pair_run(int R, int S, int batch, int C, int Kc, int H, int W, int ph, int pw, const float *x,
-                      const float *dy, const float *w, const void *prepacked, float *dx, ActGrad dx_act, float *dw,
+                      const float *dy, const float *w, PackedFilters prepacked, float *dx, ActGrad dx_act, float *dw,
                       float *db, int accumulate);
 // workspace bytes the op may ask for (so a net can reserve it before graph capture)
 size_t conv2d_workspace_bytes(const tdh_conv_desc *d, int batch);

@@ -1357,20 +1357,22 @@ int conv_pack_filters(const tdh_conv_desc *d, int kind, int flip, const float *w
 }
 
 int conv2d_fwd(const tdh_conv_desc *d, int batch, const float *x, const float *w, const float *b,
-               float *y, const uint8_t *tbl_resident, const void *prepacked, float *act_out,
+               float *y, const uint8_t *tbl_resident, PackedFilters prepacked, float *act_out,
                int act_kind, const PoolFuse *pool) {
   const ConvGeom g = make_geom(d);
   if (pool) {
     tdh_pool_desc behind{};
     behind.in_w = g.OW; behind.in_h = g.OH; behind.in_c = g.Kc;
     behind.pool_w = behind.pool_h = behind.stride_w = behind.stride_h = 2;
-    if (!conv_fwd_fuses_pool(d, &behind, batch, prepacked != nullptr) ||
-        (pool->act_out && !conv_fwd_pool_applies_act(d, batch, prepacked != nullptr, pool->act_kind)))
+    if (!conv_fwd_fuses_pool(d, &behind, batch, static_cast<bool>(prepacked)) ||
+        (pool->act_out && !conv_fwd_pool_applies_act(d, batch, static_cast<bool>(prepacked), pool->act_kind)))
       return set_error(TDH_ERR_INVALID, "conv2d_fwd: this kernel does not compute the pool layer behind it");
   }
   // (y null: only a kernel that also writes the activation or the pool behind the layer can leave it out)
-  if (!y && !pool && !(act_out && conv_fwd_out_optional(d, batch, prepacked != nullptr)))
+  if (!y && !pool && !(act_out && conv_fwd_out_optional(d, batch, static_cast<bool>(prepacked))))
     return set_error(TDH_ERR_INVALID, "conv2d_fwd: no output tensor");
+  if (prepacked && prepacked.kind != conv_packed_kind(d, batch, 0))
+    return set_error(TDH_ERR_INVALID, "conv2d_fwd: filters packed for another kernel");
   if (prepacked)
     return conv_s1_run(g.R, g.S, batch, g.C, g.Kc, 0, x, w, nullptr, d->has_bias ? b : nullptr, y, g.H,
                        g.W, g.OH, g.OW, g.pad_h, g.pad_w, ActGrad(), "conv_fwd_s1", prepacked, act_out,
@@ -1389,7 +1391,7 @@ int conv2d_fwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
       conv_s1_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w))
     return conv_s1_run(g.R, g.S, batch, g.C, g.Kc, 0, x, w_eff, nullptr,
                        d->has_bias ? b : nullptr, y, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w,
-                       ActGrad(), "conv_fwd_s1", nullptr, act_out, act_kind, pool);
+                       ActGrad(), "conv_fwd_s1", PackedFilters(), act_out, act_kind, pool);
   StridedOperand A{w_eff, crs, 1, g.Kc};
   FwdInputOperand B{x, g, batch * ohw};
   if (act_out) {  // the pointwise activation layer that follows leaves the same kernel
@@ -1413,10 +1415,10 @@ bool conv_bwd_one_launch(const tdh_conv_desc *d, int batch, bool pooled) {
   return one_launch_band(d, make_geom(d), batch, pooled) > 0;
 }
 
-bool conv_bwd_pairs(const tdh_conv_desc *d, int batch) {
+bool conv_bwd_pairs(const tdh_conv_desc *d, int batch, const float *x, const float *dy) {
   const ConvGeom g = make_geom(d);
   return bwd_direct_applies(d, g, batch) ||
-         (!d->tbl && g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 &&
+         (!((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy)) & 15) && !d->tbl && g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 &&
           conv_bwd_pair_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w));
 }
 
@@ -1472,7 +1474,7 @@ static int run_first_both(const ConvGeom &g, int batch, const float *x, const fl
 
 int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w, const float *dy,
                float *dx, float *dw, float *db, int accumulate, ActGrad dx_act,
-               const uint8_t *tbl_resident, const void *prepacked_dx, const PoolGather *dy_pool) {
+               const uint8_t *tbl_resident, PackedFilters prepacked_dx, const PoolGather *dy_pool) {
   const ConvGeom g = make_geom(d);
   const int ohw = g.OH * g.OW, crs = g.C * g.R * g.S;
   if (dy_pool) {
@@ -1508,9 +1510,11 @@ int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
   if (bwd_direct_applies(d, g, batch))
     return conv_bwd_direct_run(batch, g.C, g.Kc, x, w, dy, dx, dw, db, g.H, g.W, g.OH, g.OW, g.R, g.S, g.sh, g.sw,
                                g.pad_h, g.pad_w, accumulate, dx_act);
-  if (dx && dw && conv_bwd_pairs(d, batch) && !((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy)) & 15))
+  if (dx && dw && conv_bwd_pairs(d, batch, x, dy))
     return conv_bwd_pair_run(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.pad_h, g.pad_w, x, dy, w, prepacked_dx, dx, dx_act,
                              dw, db, accumulate);
+  // (packed for another kernel than the one that runs now: it packs for itself)
+  if (prepacked_dx.kind != conv_packed_kind(d, batch, 1)) prepacked_dx = PackedFilters();
   if (dx && prepacked_dx) {
     TDH_TRY(conv_s1_run(g.R, g.S, batch, g.C, g.Kc, 1, dy, w, nullptr, nullptr, dx, g.OH, g.OW, g.H,
                         g.W, g.R - 1 - g.pad_h, g.S - 1 - g.pad_w, dx_act, "conv_dx_s1", prepacked_dx));

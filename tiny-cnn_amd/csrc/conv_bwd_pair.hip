@@ -47,17 +47,17 @@ bool conv_bwd_pair_applicable(int R, int S, int batch, int C, int Kc, int H, int
 }
 
 // The caller has checked conv_bwd_pair_applicable and reserved the workspace of both gradients.
-// prepacked: the result of conv_s1_repack (flip = 1) for this filter, or null.
+// prepacked: this filter packed for dX (read where it is in three parts), or none.
 int conv_bwd_pair_run(int R, int S, int batch, int C, int Kc, int H, int W, int ph, int pw, const float *x, const float *dy,
-                      const float *w, const void *prepacked, float *dx, ActGrad dx_act, float *dw, float *db,
+                      const float *w, PackedFilters prepacked, float *dx, ActGrad dx_act, float *dw, float *db,
                       int accumulate) {
   S1Plan p     = make_s1_pair_plan(R, S, batch, Kc, C, H, W, H, W, R - 1 - ph, S - 1 - pw);
   DwImgPlan im = make_dw_img_plan(R, S, batch, C, Kc, H, W, H, W, ph, pw);
   if (!p.ok || !im.ok || !aligned16(x) || !aligned16(dy))
     return set_error(TDH_ERR_INVALID, "conv_bwd_pair_run: shape not supported");
   const int crs  = C * R * S;
-  const void *wp = prepacked;
-  if (!prepacked) {
+  const void *wp = prepacked.data;
+  if (!wp || prepacked.kind != CONV_PACK_X3) {
     void *fresh = nullptr;
     TDH_TRY(ws_take(conv_s1_packed_bytes(CONV_PACK_X3, R * S, Kc, C), &fresh));
     TDH_TRY(conv_s1_repack(R, S, C, Kc, 1, w, nullptr, fresh, true));

@@ -291,10 +291,11 @@ int conv_s1_repack(int R, int S, int C, int Kc, int flip, const float *w, const 
 
 // Runs out = conv(in, repack(w)) (+ bias) (* act'(y)); the caller has checked applicability
 // and reserved conv_s1_workspace_bytes of scratch. flip = 0: forward, 1: dX. prepacked: the
-// result of conv_s1_repack for this filter, when the caller already has it (w is not read).
+// result of conv_s1_repack for this filter, when the caller already has it in the layout of the
+// kernel that runs (w is not read then).
 int conv_s1_run(int R, int S, int batch, int C, int Kc, int flip, const float *in, const float *w,
                 const uint8_t *tbl_dev, const float *bias, float *out, int IH, int IW, int OH,
-                int OW, int ph, int pw, ActGrad ag, const char *tag, const void *prepacked,
+                int OW, int ph, int pw, ActGrad ag, const char *tag, PackedFilters prepacked,
                 float *act_out, int act_kind, const PoolFuse *pool) {
   const int KC = flip ? Kc : C, MC = flip ? C : Kc;
   S1Plan p = make_plan(R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw);
@@ -305,8 +306,8 @@ int conv_s1_run(int R, int S, int batch, int C, int Kc, int flip, const float *i
     return set_error(TDH_ERR_INVALID, "conv_s1_run: this shape does not compute the pool layer behind it");
   if (!out && !pool && !(act_out && p.splits == 1))
     return set_error(TDH_ERR_INVALID, "conv_s1_run: no output tensor");
-  const void *wp = prepacked;
-  if (!prepacked) {
+  const void *wp = prepacked.data;
+  if (!wp || prepacked.kind != (p.x3 ? CONV_PACK_X3 : CONV_PACK_F32)) {
     void *fresh = nullptr;
     TDH_TRY(ws_take(conv_s1_packed_bytes(p.x3 ? CONV_PACK_X3 : CONV_PACK_F32, R * S, KC, MC), &fresh));
     TDH_TRY(conv_s1_repack(R, S, C, Kc, flip, w, tbl_dev, fresh, p.x3));

@@ -457,15 +457,16 @@ TailPlan plan_tail(tdh_net *net, int loss_kind, int batch) {
   return plan;
 }
 
-// the packed filters that this direction of a layer reads at this batch, or null: it has none, or
-// packs for itself
-const void *packed_filters(const tdh_net::Layer &L, int batch, int flip) {
-  if (!L.wp_fwd) return nullptr;
-  switch (conv_packed_kind(&L.spec.conv, batch, flip)) {
-    case CONV_PACK_F32: return flip ? L.wp_dx : L.wp_fwd;
-    case CONV_PACK_X3: return flip ? L.wx_dx : L.wx_fwd;
-    default: return nullptr;
-  }
+// the layer's filters packed for this direction in this layout, or none: it has no such copy
+PackedFilters packed_as(const tdh_net::Layer &L, int kind, int flip) {
+  const void *p = nullptr;
+  if (kind == CONV_PACK_F32) p = flip ? L.wp_dx : L.wp_fwd;
+  if (kind == CONV_PACK_X3) p = flip ? L.wx_dx : L.wx_fwd;
+  return p ? PackedFilters{p, kind} : PackedFilters();
+}
+// ... in the layout that the direction reads at this batch (none: it packs for itself, or reads w)
+PackedFilters packed_filters(const tdh_net::Layer &L, int batch, int flip) {
+  return L.wp_fwd ? packed_as(L, conv_packed_kind(&L.spec.conv, batch, flip), flip) : PackedFilters();
 }
 
 // packed: the layers' wp_fwd hold the current filters in the stride-1 kernels' layout
@@ -490,7 +491,8 @@ int forward(tdh_net *net, int batch, const float *x, bool packed = false, const 
       case TDH_L_CONV:
         TDH_TRY(ws_begin(conv2d_workspace_bytes(&s.conv, batch)));
       {
-        const void *wp = packed ? packed_filters(L, batch, 0) : nullptr;
+        const PackedFilters wp = packed ? packed_filters(L, batch, 0) : PackedFilters();
+        const bool has_wp = static_cast<bool>(wp);
         const bool fuse = (net->flags & TDH_NET_FUSE_ACT_GRAD) != 0;
         auto pointwise = [&](int k) {
           return k < n && net->layers[k].spec.kind == TDH_L_ACT && is_pointwise_act(net->layers[k].spec.act);
@@ -500,7 +502,7 @@ int forward(tdh_net *net, int batch, const float *x, bool packed = false, const 
         int last = i;
         float *act_out = nullptr;
         int act_kind   = TDH_ACT_NONE;
-        if (fuse && pointwise(i + 1) && conv_fwd_applies_act(&s.conv, batch, wp != nullptr)) {
+        if (fuse && pointwise(i + 1) && conv_fwd_applies_act(&s.conv, batch, has_wp)) {
           last     = i + 1;
           act_out  = net->layers[last].out;
           act_kind = net->layers[last].spec.act;
@@ -508,12 +510,12 @@ int forward(tdh_net *net, int batch, const float *x, bool packed = false, const 
         PoolFuse pf{nullptr, nullptr, nullptr, TDH_ACT_NONE};
         if (fuse && !(pointwise(i + 1) && last == i) && last + 1 < n &&
             net->layers[last + 1].spec.kind == TDH_L_MAXPOOL &&
-            conv_fwd_fuses_pool(&s.conv, &net->layers[last + 1].spec.pool, batch, wp != nullptr)) {
+            conv_fwd_fuses_pool(&s.conv, &net->layers[last + 1].spec.pool, batch, has_wp)) {
           ++last;
           pf.out    = net->layers[last].out;
           pf.argmax = net->layers[last].argmax;
           if (pointwise(last + 1) &&
-              conv_fwd_pool_applies_act(&s.conv, batch, wp != nullptr, net->layers[last + 1].spec.act)) {
+              conv_fwd_pool_applies_act(&s.conv, batch, has_wp, net->layers[last + 1].spec.act)) {
             ++last;
             pf.act_out  = net->layers[last].out;
             pf.act_kind = net->layers[last].spec.act;
@@ -526,7 +528,7 @@ int forward(tdh_net *net, int batch, const float *x, bool packed = false, const 
           // (the backward pass reads the outputs of the layers that left the kernel, never the
           // convolution's own: the gradients of the pointwise activations are functions of y)
           const bool own_out = !(training && ((pf.out && !act_out) ||
-                                              (act_out && conv_fwd_out_optional(&s.conv, batch, wp != nullptr))));
+                                              (act_out && conv_fwd_out_optional(&s.conv, batch, has_wp))));
           if (!own_out) net->out_unwritten[i] = 1;
           TDH_TRY(conv2d_fwd(&s.conv, batch, in, L.w, L.b, own_out ? L.out : nullptr, L.tbl_dev, wp, act_out, act_kind,
                              pf.out ? &pf : nullptr));
@@ -1093,7 +1095,7 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
     // chain: its weight and bias products are too small to be worth a branch
     const bool fc_one_launch = s.kind == TDH_L_FC && fc_bwd_fuses(s.fc_in, s.fc_out, batch);
     // so does a convolution whose gradients share a launch
-    const bool conv_pair = s.kind == TDH_L_CONV && dx && i != through_pool_for && conv_bwd_pairs(&s.conv, batch);
+    const bool conv_pair = s.kind == TDH_L_CONV && dx && i != through_pool_for && conv_bwd_pairs(&s.conv, batch, in, L.dout);
     const bool fork = forked && layer_forks(L) && !fc_one_launch && !conv_pair;
     if (fork) {
       // this layer's output gradient is complete here: let the side streams start from it
@@ -1112,7 +1114,8 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
         TDH_TRY(ws_begin((forked || as_forked ? 3 : 1) * conv2d_workspace_bytes(&s.conv, batch)));
       {
         const PoolGather *gp = i == through_pool_for ? &through_pool : nullptr;
-        const void *wp = !packed ? nullptr : conv_pair ? L.wx_dx : packed_filters(L, batch, 1);
+        const PackedFilters wp = !packed ? PackedFilters()
+                                 : conv_pair ? packed_as(L, CONV_PACK_X3, 1) : packed_filters(L, batch, 1);
         // the layer that reads this dX next (behind a folded activation) is a max-pool: its
         // backward kernel can add up a split reduction of dX
         const int reader = i - 1 - ((i >= 1 && net->layers[i - 1].grad_folded) ? 1 : 0);
@@ -1134,7 +1137,7 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
             // like the two launches below)
             c.defer_reduce = true;
             TDH_TRY(conv2d_bwd(&s.conv, batch, in, L.w, L.dout, dx, L.dw, L.b_size ? L.db : nullptr, 1, fold,
-                               L.tbl_dev, nullptr, gp));
+                               L.tbl_dev, PackedFilters(), gp));
             c.defer_reduce = false;
             last_dw_on_main = true;
             break;
@@ -1151,7 +1154,7 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
             // wait across streams is 5 us of a replayed step whether or not it has to wait.)
             c.defer_reduce = true;
             TDH_TRY(conv2d_bwd(&s.conv, batch, in, L.w, L.dout, nullptr, L.dw, db_with_dw ? L.db : nullptr, 1,
-                               ActGrad(), L.tbl_dev, nullptr, gp));
+                               ActGrad(), L.tbl_dev, PackedFilters(), gp));
             c.defer_reduce = false;
             last_dw_on_main = true;
             break;
@@ -1160,13 +1163,13 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
             StreamSwap on_side(c.side[0]);
             c.defer_reduce = true;
             TDH_TRY(conv2d_bwd(&s.conv, batch, in, L.w, L.dout, nullptr, L.dw, db_with_dw ? L.db : nullptr, 1,
-                               ActGrad(), L.tbl_dev, nullptr, gp));
+                               ActGrad(), L.tbl_dev, PackedFilters(), gp));
             c.defer_reduce = false;
           }
           if (L.b_size && !db_with_dw) {
             StreamSwap on_side(c.side[1]);
             c.defer_rowsum = true;
-            TDH_TRY(conv2d_bwd(&s.conv, batch, in, L.w, L.dout, nullptr, nullptr, L.db, 1, ActGrad(), L.tbl_dev, nullptr, gp));
+            TDH_TRY(conv2d_bwd(&s.conv, batch, in, L.w, L.dout, nullptr, nullptr, L.db, 1, ActGrad(), L.tbl_dev, PackedFilters(), gp));
             c.defer_rowsum = false;
           }
         } else if (as_forked) {
@@ -1182,7 +1185,7 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
           if (i == 0 && dx && !wp && conv_bwd_one_launch(&s.conv, batch, gp != nullptr)) {
             c.defer_reduce = true;
             TDH_TRY(conv2d_bwd(&s.conv, batch, in, L.w, L.dout, dx, L.dw, L.b_size ? L.db : nullptr, 1, fold,
-                               L.tbl_dev, nullptr, gp));
+                               L.tbl_dev, PackedFilters(), gp));
             c.defer_reduce = false;
             break;
           }
@@ -1193,11 +1196,11 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
           const bool db_with_dw = L.b_size && conv_dw_gives_db(&s.conv, batch);
           c.defer_reduce = true;
           TDH_TRY(conv2d_bwd(&s.conv, batch, in, L.w, L.dout, nullptr, L.dw, db_with_dw ? L.db : nullptr, 1,
-                             ActGrad(), L.tbl_dev, nullptr, gp));
+                             ActGrad(), L.tbl_dev, PackedFilters(), gp));
           c.defer_reduce = false;
           if (L.b_size && !db_with_dw) {
             c.defer_rowsum = small_defers;
-            TDH_TRY(conv2d_bwd(&s.conv, batch, in, L.w, L.dout, nullptr, nullptr, L.db, 1, ActGrad(), L.tbl_dev, nullptr, gp));
+            TDH_TRY(conv2d_bwd(&s.conv, batch, in, L.w, L.dout, nullptr, nullptr, L.db, 1, ActGrad(), L.tbl_dev, PackedFilters(), gp));
             c.defer_rowsum = false;
           }
         } else {
