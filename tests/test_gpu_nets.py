@@ -1136,3 +1136,62 @@ def test_decisions_that_hang_on_summation_order_are_legitimate_and_the_gradients
             assert_close(net.layer_grad(i, which), ref.layer_dw(i) if which == 0 else ref.layer_db(i),
                          what=f"flags {flags}: gradient {i}.{which} vs oracle")
     net.close()
+
+
+STRIDE1_NET = [("conv", 16, 16, 16, 3, 40, True), ("act", "relu"), ("conv", 16, 16, 40, 5, 32, True), ("act", "tanh"),
+               ("maxpool", 16, 16, 32, 2), ("conv", 8, 8, 32, 5, 64, True), ("act", "relu"), ("fc", 64 * 64, 10)]
+
+
+def _stride1_net(T, O, W, batch, flags, rng):
+    net = T.Net(W.build_layers(T, STRIDE1_NET), batch, flags)
+    ref = O.OracleNet(W.build_layers(O, STRIDE1_NET), batch)
+    for i, l in enumerate(STRIDE1_NET):
+        for which, n in zip((0, 1), W.layer_fans(l)[:2]):
+            if n:
+                a = rng.uniform(-0.05, 0.05, n).astype(np.float32)
+                net.set_param(i, which, a)
+                (ref.weight(i) if which == 0 else ref.bias(i))[:] = a
+    return net, ref
+
+
+@pytest.mark.gpu
+def test_passes_pack_the_filters_that_they_read_and_no_others(T, O, W):
+    """One image reads no packed filters; a large batch packs at the first pass after the weights changed, in one
+    launch; and what train steps keep is not packed again, at this batch size or another."""
+    rng = np.random.default_rng(22)
+    net, ref = _stride1_net(T, O, W, 600, 3, rng)
+    x = rng.standard_normal((600, net.in_size())).astype(np.float32)
+    t = rng.uniform(-0.8, 0.8, (600, 10)).astype(np.float32)
+    xd, td = T.to_device(x), T.to_device(t)
+    opt, ropt = T.opt_desc("sgd", alpha=1e-5), O.opt_desc("sgd", alpha=1e-5)
+
+    def forward(batch):
+        T.profile_begin()
+        net.forward(batch, xd)
+        launches = sum(e["launches"] for e in T.profile_end() if e["tag"] == "conv_repack_weights")
+        ref.forward(x[:batch])
+        assert_close(net.layer_out(7, batch).ravel(), ref.layer_out(7, batch).ravel(), what=f"{batch} samples")
+        return launches
+
+    def step(batch):
+        T.profile_begin()
+        net.train_step(opt, "mse", batch, xd, td)
+        launches = sum(e["launches"] for e in T.profile_end() if e["tag"] == "conv_repack_weights")
+        ref.train_step(ropt, "mse", x[:batch], t[:batch])
+        assert_close(net.layer_out(7, batch).ravel(), ref.layer_out(7, batch).ravel(), what=f"step of {batch}")
+        return launches
+
+    assert forward(1) == 0
+    assert forward(600) == 1
+    assert forward(600) == 0 and forward(1) == 0
+    for batch in (600, 80, 5):
+        step(batch)             # (may pack what no step has read yet)
+        assert step(batch) == 0
+    assert step(600) == 0
+    assert forward(1) == 0
+    assert forward(600) == 1    # three-part filters, which no train step reads forward
+    a = rng.uniform(-0.05, 0.05, net.param_size(0, 0)).astype(np.float32)
+    net.set_param(0, 0, a)
+    ref.weight(0)[:] = a
+    assert step(600) == 1 and step(600) == 0
+    net.close()

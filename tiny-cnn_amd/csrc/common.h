@@ -206,11 +206,10 @@ struct OptTensor {
   uint32_t n, first_block;
   uint32_t block_elems;  // elements a workgroup updates: OPT_MULTI_ELEMS_PER_BLOCK or OPT_SUM_ELEMS_PER_BLOCK
   // A convolution's OIHW weight tensor whose filters the stride-1 kernels read in their own
-  // layout: the update also writes the new value into those copies (wp_fwd[t][ci][co],
-  // wp_dx[rs-1-t][co][ci]; unconnected pairs of the connection table as zero). NULL: none.
-  float *wp_fwd, *wp_dx;
-  // the same in the three bf16 parts of the kernel of conv_x3_inst.hip (with wp_fwd only)
-  uint16_t *wx_fwd, *wx_dx;
+  // layouts: the update also writes the new value into these copies (unconnected pairs of the
+  // connection table as zero): floats forward [t][ci][co] and for dX [rs-1-t][co][ci], then both
+  // directions in the three bf16 parts of conv_x3_inst.hip. NULL: nobody reads that one.
+  void *packed[4];
   const uint8_t *tbl;
   uint32_t C, Kc, rs;
 };
@@ -393,9 +392,20 @@ bool conv_bwd_reads_pooled(const tdh_conv_desc *d, const tdh_pool_desc *pool, in
 int conv_packed_kind(const tdh_conv_desc *d, int batch, int flip);
 size_t conv_packed_bytes(const tdh_conv_desc *d, int kind, int flip);
 bool conv_fwd_applies_act(const tdh_conv_desc *d, int batch, bool prepacked);
-// packs w (masked by the device-resident connection table, if any) into wp
-int conv_pack_filters(const tdh_conv_desc *d, int kind, int flip, const float *w, const uint8_t *tbl_resident,
-                      void *wp);
+// One packed copy to be made: w (masked by the device-resident connection table, if any) into wp. Any
+// number of them leave in one launch per CONV_PACK_JOBS.
+struct PackJob {
+  const float *w;
+  const uint8_t *tbl;   // device, or null
+  void *wp;
+  int C, Kc, R, S;
+  int kind, flip;
+};
+constexpr int CONV_PACK_JOBS = 16;
+int conv_pack_filters(const PackJob *jobs, int n);
+// (conv.hip) the kind that the backward pass of this layer reads when dX is computed together with dW
+// (x, dy: as in conv_bwd_pairs)
+int conv_bwd_packed_kind(const tdh_conv_desc *d, int batch, const float *x = nullptr, const float *dy = nullptr);
 // fc_fwd_direct.hip: a few samples, with the activation or (applies_softmax) the softmax behind the layer
 bool fc_fwd_direct_applicable(int in, int out, int batch);
 bool fc_fwd_direct_applies_softmax(int in, int out, int batch);
@@ -452,8 +462,6 @@ bool conv_s1_fuses_pool(int R, int S, int batch, int KC, int MC, int IH, int IW,
 // one pass over the reduction channels: the kernel's epilogue is the only writer of `out`
 bool conv_s1_single_pass(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW,
                          int ph, int pw);
-int conv_s1_repack(int R, int S, int C, int Kc, int flip, const float *w, const uint8_t *tbl_dev,
-                   void *wp, bool x3);
 // conv_packed_kind / conv_packed_bytes of a shape this file runs
 int conv_s1_packed_kind(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw);
 size_t conv_s1_packed_bytes(int kind, int RS, int KC, int MC);

@@ -1350,12 +1350,6 @@ size_t conv_packed_bytes(const tdh_conv_desc *d, int kind, int flip) {
   return conv_s1_packed_bytes(kind, d->k_h * d->k_w, flip ? d->out_c : d->in_c, flip ? d->in_c : d->out_c);
 }
 
-int conv_pack_filters(const tdh_conv_desc *d, int kind, int flip, const float *w, const uint8_t *tbl_resident,
-                      void *wp) {
-  return conv_s1_repack(d->k_h, d->k_w, d->in_c, d->out_c, flip, w, d->tbl ? tbl_resident : nullptr, wp,
-                        kind == CONV_PACK_X3);
-}
-
 int conv2d_fwd(const tdh_conv_desc *d, int batch, const float *x, const float *w, const float *b,
                float *y, const uint8_t *tbl_resident, PackedFilters prepacked, float *act_out,
                int act_kind, const PoolFuse *pool) {
@@ -1420,6 +1414,11 @@ bool conv_bwd_pairs(const tdh_conv_desc *d, int batch, const float *x, const flo
   return bwd_direct_applies(d, g, batch) ||
          (!((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy)) & 15) && !d->tbl && g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 &&
           conv_bwd_pair_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w));
+}
+
+int conv_bwd_packed_kind(const tdh_conv_desc *d, int batch, const float *x, const float *dy) {
+  if (bwd_direct_applies(d, make_geom(d), batch)) return CONV_PACK_NONE;   // (reads w)
+  return conv_bwd_pairs(d, batch, x, dy) ? CONV_PACK_X3 : conv_packed_kind(d, batch, 1);
 }
 
 // the slices of the first convolution's launch: one per band and image

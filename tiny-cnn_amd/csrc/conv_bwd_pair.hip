@@ -60,7 +60,8 @@ int conv_bwd_pair_run(int R, int S, int batch, int C, int Kc, int H, int W, int 
   if (!wp || prepacked.kind != CONV_PACK_X3) {
     void *fresh = nullptr;
     TDH_TRY(ws_take(conv_s1_packed_bytes(CONV_PACK_X3, R * S, Kc, C), &fresh));
-    TDH_TRY(conv_s1_repack(R, S, C, Kc, 1, w, nullptr, fresh, true));
+    const PackJob job{w, nullptr, fresh, C, Kc, R, S, CONV_PACK_X3, 1};
+    TDH_TRY(conv_pack_filters(&job, 1));
     wp = fresh;
   }
   ConvS1Args &a = p.args;

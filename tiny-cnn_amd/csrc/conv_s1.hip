@@ -1,6 +1,7 @@
 // conv_s1.hip — host side of the stride-1 convolution (forward and dX) on the LDS-halo MFMA
 // kernel of conv_s1_inst.hip: tile choice, filter repacking, split-K reduction.
 #include <algorithm>
+#include <climits>
 
 #include "conv_s1.h"
 #include "split_bf16.h"
@@ -38,44 +39,52 @@ int launch_split_reduce(const SplitSum &sum, int plane, float *act_out, int act_
   return TDH_OK;
 }
 
+// The filters of several layers in one launch: job k owns the workgroups [first_block[k],
+// first_block[k+1]). A launch of its own in every pass whose caller may have written the weights: bound by
+// latency, so nothing is divided and a thread's loads are asked for together. us for 5x5, 32 -> 32 and
+// 32 -> 64 channels, both directions' copies: one thread per weight with scattered stores 5.9.
+struct PackJobs {
+  PackJob job[CONV_PACK_JOBS];
+  FastDiv div_rs[CONV_PACK_JOBS], div_m[CONV_PACK_JOBS], div_kc[CONV_PACK_JOBS];
+  int first_block[CONV_PACK_JOBS];   // (past the last job: INT_MAX)
+};
+
 // wp[t][kc][m]: forward (flip = 0): kc = ci, m = co, t as is; dX (flip = 1): kc = co, m = ci,
-// tap reversed. An optional connection table zeroes unconnected (ci, co) pairs.
-__global__ void __launch_bounds__(256)
-repack_weights_kernel(const float *__restrict__ w, const uint8_t *__restrict__ tbl,
-                      float *__restrict__ wp, const int C, const int Kc, const int rs,
-                      const int flip) {
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  if (e >= C * Kc * rs) return;
-  // e indexes the OIHW source: ((co*C + ci)*rs + t)
-  const int t = e % rs, pair = e / rs;
-  const int co = pair / C, ci = pair - co * C;
-  float v = w[e];
-  if (tbl && !tbl[ci * Kc + co]) v = 0.0f;
-  if (!flip)
-    wp[(static_cast<size_t>(t) * C + ci) * Kc + co] = v;
-  else
-    wp[(static_cast<size_t>(rs - 1 - t) * Kc + co) * C + ci] = v;
+// tap reversed. An optional connection table zeroes unconnected (ci, co) pairs. e: element of wp.
+__device__ __forceinline__ void pack_f32(const PackJob &j, const FastDiv &div_m, const FastDiv &div_kc, const int e) {
+  const int rs = j.R * j.S;
+  if (e >= j.C * j.Kc * rs) return;
+  uint32_t rest, m, t, kc;
+  div_m.divmod(e, rest, m);
+  div_kc.divmod(rest, t, kc);
+  const int co = j.flip ? kc : m, ci = j.flip ? m : kc;
+  const float v = j.w[(static_cast<size_t>(co) * j.C + ci) * rs + (j.flip ? rs - 1 - t : t)];
+  static_cast<float *>(j.wp)[e] = j.tbl && !j.tbl[ci * j.Kc + co] ? 0.0f : v;
 }
 
 // The filters of the three-part kernel: unit ((g*rs + t)*3 + part)*2 + half)*mc_pad + m holds the
 // parts of channels 16g + 8*half .. +7 of row m (zero beyond the tensor), with the sign of step
 // g*rs + t. A thread writes the
 // three units of eight channels.
-__global__ void __launch_bounds__(256)
-x3_pack_kernel(const float *__restrict__ w, const uint8_t *__restrict__ tbl, uint4 *__restrict__ wp,
-               const int C, const int Kc, const int rs, const int flip, const int mc_pad) {
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  const int m = e % mc_pad, rest = e / mc_pad;
-  const int half = rest & 1, t = (rest >> 1) % rs, g = (rest >> 1) / rs;
-  const int KC = flip ? Kc : C, MC = flip ? C : Kc;
-  if (g * 16 >= KC) return;
+__device__ __forceinline__ void pack_x3(const PackJob &j, const FastDiv &div_m, const FastDiv &div_rs, const int e) {
+  const int rs = j.R * j.S, KC = j.flip ? j.Kc : j.C, MC = j.flip ? j.C : j.Kc, mc_pad = div_m.d;
+  uint32_t rest, m, g, t;
+  div_m.divmod(e, rest, m);
+  const int half = rest & 1;
+  div_rs.divmod(rest >> 1, g, t);
+  if (static_cast<int>(g) * 16 >= KC) return;
+  const int step = (j.flip ? j.C : 1) * rs, kc0 = 16 * g + 8 * half;   // floats from one channel to the next
+  const float *src = j.w + static_cast<size_t>(j.flip ? min(static_cast<int>(m), MC - 1) : min(static_cast<int>(m), MC - 1) * j.C) * rs +
+                     (j.flip ? rs - 1 - t : t);
   float v[8];
 #pragma unroll
+  for (int k = 0; k < 8; ++k) v[k] = src[static_cast<size_t>(min(kc0 + k, KC - 1)) * step];
+  const float sign = x3_sign(g * rs + t);
+#pragma unroll
   for (int k = 0; k < 8; ++k) {
-    const int kc = 16 * g + 8 * half + k;
-    const int co = flip ? kc : m, ci = flip ? m : kc;
-    const bool in = kc < KC && m < MC && (!tbl || tbl[ci * Kc + co]);
-    v[k] = in ? x3_sign(g * rs + t) * w[(static_cast<size_t>(co) * C + ci) * rs + (flip ? rs - 1 - t : t)] : 0.0f;
+    const int kc = kc0 + k, co = j.flip ? kc : m, ci = j.flip ? m : kc;
+    const bool in = kc < KC && static_cast<int>(m) < MC && (!j.tbl || j.tbl[ci * j.Kc + co]);
+    v[k] = in ? sign * v[k] : 0.0f;
   }
   uint32_t part[X3_PARTS][4];
 #pragma unroll
@@ -85,10 +94,23 @@ x3_pack_kernel(const float *__restrict__ w, const uint8_t *__restrict__ tbl, uin
 #pragma unroll
     for (int p = 0; p < X3_PARTS; ++p) part[p][k] = p3[p];
   }
+  uint4 *wp = static_cast<uint4 *>(j.wp);
 #pragma unroll
   for (int p = 0; p < X3_PARTS; ++p)
     wp[((static_cast<size_t>(g * rs + t) * X3_PARTS + p) * 2 + half) * mc_pad + m] =
       make_uint4(part[p][0], part[p][1], part[p][2], part[p][3]);
+}
+
+__global__ void __launch_bounds__(256) pack_filters_kernel(const PackJobs jobs) {
+  int k = 0;
+#pragma unroll
+  for (int i = 1; i < CONV_PACK_JOBS; ++i) k += jobs.first_block[i] <= static_cast<int>(blockIdx.x) ? 1 : 0;
+  const PackJob &j = jobs.job[k];
+  const int e      = (static_cast<int>(blockIdx.x) - jobs.first_block[k]) * 256 + threadIdx.x;
+  if (j.kind == CONV_PACK_X3)
+    pack_x3(j, jobs.div_m[k], jobs.div_rs[k], e);
+  else
+    pack_f32(j, jobs.div_m[k], jobs.div_kc[k], e);
 }
 
 int pow2_ceil(int v) {
@@ -272,26 +294,34 @@ size_t conv_s1_workspace_bytes(int R, int S, int batch, int C, int Kc, int flip,
   return most;
 }
 
-// wp = the filter in the kernel's layout [tap][kc][m] (R*S*C*Kc floats); flip as in conv_s1_run
-int conv_s1_repack(int R, int S, int C, int Kc, int flip, const float *w, const uint8_t *tbl_dev,
-                   void *wp, bool x3) {
-  ProfScope prof("conv_repack_weights", (x3 ? 10.0 : 8.0) * R * S * C * Kc, WORK_BYTE);
-  if (x3) {
-    const int KC = flip ? Kc : C, mc_pad = x3_mc_pad(flip ? C : Kc);
-    TDH_LAUNCH(x3_pack_kernel, dim3(ceil_div(ceil_div(KC, 16) * R * S * 2 * mc_pad, 256)), dim3(256), 0, ctx().stream,
-               w, tbl_dev, static_cast<uint4 *>(wp), C, Kc, R * S, flip, mc_pad);
+int conv_pack_filters(const PackJob *jobs, int n) {
+  for (int at = 0; at < n; at += CONV_PACK_JOBS) {
+    PackJobs p;
+    const int here = std::min(CONV_PACK_JOBS, n - at);
+    int blocks     = 0;
+    double bytes   = 0.0;
+    for (int k = 0; k < CONV_PACK_JOBS; ++k) {
+      p.first_block[k] = k < here ? blocks : INT_MAX;
+      if (k >= here) continue;
+      const PackJob &j = p.job[k] = jobs[at + k];
+      const bool x3    = j.kind == CONV_PACK_X3;
+      const int rs = j.R * j.S, KC = j.flip ? j.Kc : j.C, MC = j.flip ? j.C : j.Kc;
+      p.div_rs[k] = FastDiv(rs);
+      p.div_m[k]  = FastDiv(x3 ? x3_mc_pad(MC) : MC);
+      p.div_kc[k] = FastDiv(KC);
+      blocks += ceil_div(x3 ? ceil_div(KC, 16) * rs * 2 * x3_mc_pad(MC) : rs * KC * MC, 256);
+      bytes += (x3 ? 10.0 : 8.0) * rs * KC * MC;
+    }
+    ProfScope prof("conv_repack_weights", bytes, WORK_BYTE);
+    TDH_LAUNCH(pack_filters_kernel, dim3(blocks), dim3(256), 0, ctx().stream, p);
     TDH_LAUNCH_CHECK();
-    return TDH_OK;
   }
-  TDH_LAUNCH(repack_weights_kernel, dim3(ceil_div(R * S * C * Kc, 256)), dim3(256), 0,
-                     ctx().stream, w, tbl_dev, static_cast<float *>(wp), C, Kc, R * S, flip);
-  TDH_LAUNCH_CHECK();
   return TDH_OK;
 }
 
 // Runs out = conv(in, repack(w)) (+ bias) (* act'(y)); the caller has checked applicability
 // and reserved conv_s1_workspace_bytes of scratch. flip = 0: forward, 1: dX. prepacked: the
-// result of conv_s1_repack for this filter, when the caller already has it in the layout of the
+// result of conv_pack_filters for this filter, when the caller already has it in the layout of the
 // kernel that runs (w is not read then).
 int conv_s1_run(int R, int S, int batch, int C, int Kc, int flip, const float *in, const float *w,
                 const uint8_t *tbl_dev, const float *bias, float *out, int IH, int IW, int OH,
@@ -310,7 +340,8 @@ int conv_s1_run(int R, int S, int batch, int C, int Kc, int flip, const float *i
   if (!wp || prepacked.kind != (p.x3 ? CONV_PACK_X3 : CONV_PACK_F32)) {
     void *fresh = nullptr;
     TDH_TRY(ws_take(conv_s1_packed_bytes(p.x3 ? CONV_PACK_X3 : CONV_PACK_F32, R * S, KC, MC), &fresh));
-    TDH_TRY(conv_s1_repack(R, S, C, Kc, flip, w, tbl_dev, fresh, p.x3));
+    const PackJob job{w, tbl_dev, fresh, C, Kc, R, S, p.x3 ? CONV_PACK_X3 : CONV_PACK_F32, flip};
+    TDH_TRY(conv_pack_filters(&job, 1));
     wp = fresh;
   }
   p.args.in = in; p.args.wp = wp; p.args.bias = bias;

@@ -447,10 +447,10 @@ __device__ __forceinline__ void opt_pack_store(const OptTensor &t, const uint32_
   const uint32_t tap = e % t.rs, pair = e / t.rs;
   const uint32_t co = pair / t.C, ci = pair - co * t.C;
   if (t.tbl && !t.tbl[ci * t.Kc + co]) v = 0.0f;
-  t.wp_fwd[(static_cast<size_t>(tap) * t.C + ci) * t.Kc + co] = v;
-  t.wp_dx[(static_cast<size_t>(t.rs - 1 - tap) * t.Kc + co) * t.C + ci] = v;
-  if (t.wx_fwd) opt_part_store(t.wx_fwd, t.rs, tap, ci, co, t.Kc, v);
-  if (t.wx_dx) opt_part_store(t.wx_dx, t.rs, t.rs - 1 - tap, co, ci, t.C, v);
+  if (t.packed[0]) static_cast<float *>(t.packed[0])[(static_cast<size_t>(tap) * t.C + ci) * t.Kc + co] = v;
+  if (t.packed[1]) static_cast<float *>(t.packed[1])[(static_cast<size_t>(t.rs - 1 - tap) * t.Kc + co) * t.C + ci] = v;
+  if (t.packed[2]) opt_part_store(static_cast<uint16_t *>(t.packed[2]), t.rs, tap, ci, co, t.Kc, v);
+  if (t.packed[3]) opt_part_store(static_cast<uint16_t *>(t.packed[3]), t.rs, t.rs - 1 - tap, co, ci, t.C, v);
 }
 
 // Multi-tensor form: block b works on tensor j = the table entry whose block range holds b.
@@ -551,6 +551,7 @@ opt_multi_kernel(const OptTensor *__restrict__ table, const int n_tensors, OptSc
     for (uint32_t c = 0; c < VEC; ++c) pending_sum[grp][VEC * o + c] = s4[c];
     __syncthreads();
   }
+  const bool packs = t.packed[0] || t.packed[1] || t.packed[2] || t.packed[3];
   auto grad = [&](const uint32_t i, const float g) {
     if (pj < 0) return g;
     float tt = pending_sum[0][i - beg];
@@ -570,7 +571,7 @@ opt_multi_kernel(const OptTensor *__restrict__ table, const int n_tensors, OptSc
     opt_one<KIND>(vg.z, vw.z, v0.z, v1.z, p);
     opt_one<KIND>(vg.w, vw.w, v0.w, v1.w, p);
     *reinterpret_cast<float4 *>(t.w + i) = vw;
-    if (t.wp_fwd) {
+    if (packs) {
       opt_pack_store(t, i, vw.x);
       opt_pack_store(t, i + 1, vw.y);
       opt_pack_store(t, i + 2, vw.z);
@@ -586,7 +587,7 @@ opt_multi_kernel(const OptTensor *__restrict__ table, const int n_tensors, OptSc
     if (NSTATE >= 2) b = t.s1[i];
     opt_one<KIND>(grad(i, t.g[i]), ww, a, b, p);
     t.w[i] = ww;
-    if (t.wp_fwd) opt_pack_store(t, i, ww);
+    if (packs) opt_pack_store(t, i, ww);
     if (NSTATE >= 1) t.s0[i] = a;
     if (NSTATE >= 2) t.s1[i] = b;
     if (zero_grad) t.g[i] = 0.0f;

@@ -24,10 +24,15 @@ struct tdh_net {
     // set where the optimizer table is built: the tensor's entry there has the small blocks
     // (OPT_SUM_ELEMS_PER_BLOCK) that let the optimizer kernel add up K-split partial slices
     bool w_sums_in_opt = false, b_sums_in_opt = false;
-    // filters in the LDS-halo kernels' layout for forward / dX, packed on a side stream at the
-    // start of a captured step (stride-1 conv layers of a TDH_NET_GRAPH net)
-    float *wp_fwd = nullptr, *wp_dx = nullptr;  // kept current by the optimizer kernel
-    float *wx_fwd = nullptr, *wx_dx = nullptr;  // likewise, in three bf16 parts (directions that read them)
+    // Copies of the filters in the layouts that the stride-1 kernels read (stride-1 conv layers of a
+    // TDH_NET_GRAPH net; null: no kernel of this layer reads that one). current: it holds the
+    // weights as they are; kept: the optimizer kernel writes the new weights into it as well,
+    // which it does for the copies that train steps read.
+    enum Copy { FWD_F32, DX_F32, FWD_X3, DX_X3, COPIES };
+    static int copy_of(int kind, int flip) { return (kind == tdh::CONV_PACK_X3 ? 2 : 0) + flip; }
+    float *copy[COPIES] = {};
+    bool current[COPIES] = {}, kept[COPIES] = {};
+    int opt_entry = -1;   // of w in the optimizer's table
     // batch-norm: running averages, this batch's moments, sqrt(variance + eps); dropout: mask
     float *bn_mean = nullptr, *bn_var = nullptr, *bn_mean_cur = nullptr, *bn_var_cur = nullptr,
           *bn_stddev = nullptr;
@@ -40,7 +45,11 @@ struct tdh_net {
   float *dx_in   = nullptr;  // gradient w.r.t. the network input
   tdh::OptTensor *opt_table = nullptr;  // device table of trainable tensors, update order
   std::vector<tdh::OptTensor> opt_table_host;  // (its host copy)
-  bool packs_valid = false;  // wp_fwd / wp_dx of every layer match its weights
+  struct Reads {   // the copies that passes of this kind read, of the last batch size asked for (copies_read)
+    int batch = 0;
+    bool aligned = false;
+    std::vector<uint8_t> copies;
+  } reads[2];      // inference, train steps
   int opt_tensors = 0, opt_blocks = 0;
   double opt_params = 0.0;
   // graph replay (TDH_NET_GRAPH): one captured train step, re-captured when its key changes
@@ -457,19 +466,88 @@ TailPlan plan_tail(tdh_net *net, int loss_kind, int batch) {
   return plan;
 }
 
-// the layer's filters packed for this direction in this layout, or none: it has no such copy
+// the layer's filters packed for this direction in this layout, or none: it has no such copy, or not
+// of the weights as they are
 PackedFilters packed_as(const tdh_net::Layer &L, int kind, int flip) {
-  const void *p = nullptr;
-  if (kind == CONV_PACK_F32) p = flip ? L.wp_dx : L.wp_fwd;
-  if (kind == CONV_PACK_X3) p = flip ? L.wx_dx : L.wx_fwd;
-  return p ? PackedFilters{p, kind} : PackedFilters();
+  const int c = tdh_net::Layer::copy_of(kind, flip);
+  return kind != CONV_PACK_NONE && L.copy[c] && L.current[c] ? PackedFilters{L.copy[c], kind} : PackedFilters();
 }
 // ... in the layout that the direction reads at this batch (none: it packs for itself, or reads w)
 PackedFilters packed_filters(const tdh_net::Layer &L, int batch, int flip) {
-  return L.wp_fwd ? packed_as(L, conv_packed_kind(&L.spec.conv, batch, flip), flip) : PackedFilters();
+  return L.copy[0] ? packed_as(L, conv_packed_kind(&L.spec.conv, batch, flip), flip) : PackedFilters();
 }
 
-// packed: the layers' wp_fwd hold the current filters in the stride-1 kernels' layout
+// The copies of each layer's filters (bits by Copy) that a pass over this batch reads: forward, or
+// (training) the forward and backward pass of a train step on input x.
+const std::vector<uint8_t> &copies_read(tdh_net *net, int batch, const float *x, bool training) {
+  tdh_net::Reads &known = net->reads[training];
+  const bool aligned    = reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  if (known.batch == batch && known.aligned == aligned) return known.copies;
+  known.batch   = batch;
+  known.aligned = aligned;
+  known.copies.assign(net->layers.size(), 0);
+  for (size_t i = 0; i < net->layers.size(); ++i) {
+    const tdh_net::Layer &L = net->layers[i];
+    if (L.spec.kind != TDH_L_CONV || !L.copy[0]) continue;
+    auto add = [&](int kind, int flip) {
+      const int c = tdh_net::Layer::copy_of(kind, flip);
+      if (kind != CONV_PACK_NONE && L.copy[c]) known.copies[i] |= 1u << c;
+    };
+    {
+      const KeepF32 keep(training);
+      add(conv_packed_kind(&L.spec.conv, batch, 0), 0);
+    }
+    if (training && !(i == 0 && net_skips_input_grad(net))) {
+      const KeepF32 keep(has_batchnorm(net));
+      add(conv_bwd_packed_kind(&L.spec.conv, batch, i == 0 ? x : nullptr, nullptr), 1);
+    }
+  }
+  return known.copies;
+}
+
+// Packs the copies that the pass reads and that do not hold the weights as they are, in one launch.
+int pack_copies(tdh_net *net, int batch, const float *x, bool training) {
+  const std::vector<uint8_t> &reads = copies_read(net, batch, x, training);
+  std::vector<PackJob> jobs;
+  for (size_t i = 0; i < net->layers.size(); ++i) {
+    tdh_net::Layer &L = net->layers[i];
+    for (int c = 0; c < tdh_net::Layer::COPIES; ++c) {
+      if (!(reads[i] >> c & 1) || L.current[c]) continue;
+      const tdh_conv_desc &d = L.spec.conv;
+      jobs.push_back(PackJob{L.w, d.tbl ? L.tbl_dev : nullptr, L.copy[c], d.in_c, d.out_c, d.k_h, d.k_w,
+                             c >= 2 ? CONV_PACK_X3 : CONV_PACK_F32, c & 1});
+      L.current[c] = true;
+    }
+  }
+  return conv_pack_filters(jobs.data(), static_cast<int>(jobs.size()));
+}
+
+void forget_copies(tdh_net::Layer &L) { std::fill(L.current, L.current + tdh_net::Layer::COPIES, false); }
+
+// Has the optimizer kernel keep the copies that a train step reads current from here on. (Not inside a
+// capture: it writes the table that the captured kernels read.)
+int keep_copies(tdh_net *net, int batch, const float *x) {
+  const std::vector<uint8_t> &reads = copies_read(net, batch, x, /*training=*/true);
+  for (size_t i = 0; i < net->layers.size(); ++i) {
+    tdh_net::Layer &L = net->layers[i];
+    bool changed      = false;
+    for (int c = 0; c < tdh_net::Layer::COPIES; ++c) {
+      if (!(reads[i] >> c & 1) || L.kept[c]) continue;
+      net->opt_table_host[L.opt_entry].packed[c] = L.copy[c];
+      L.kept[c] = changed = true;
+    }
+    if (changed)
+      TDH_TRY(tdh_memcpy_h2d(net->opt_table + L.opt_entry, &net->opt_table_host[L.opt_entry], sizeof(OptTensor)));
+  }
+  return TDH_OK;
+}
+
+// The weights have been updated, and with them the copies that the optimizer kernel keeps.
+void after_update(tdh_net *net) {
+  for (tdh_net::Layer &L : net->layers)
+    for (int c = 0; c < tdh_net::Layer::COPIES; ++c) L.current[c] = L.current[c] && L.kept[c];
+}
+
 // xent_t / xent_dz: the net ends in softmax and the step's loss is cross_entropy_multiclass: the
 // last layer's kernel also writes the loss gradient with respect to the softmax input
 // tail: its layer runs as fc_softmax_xent, which also writes the loss gradient (to xent_dz, from
@@ -478,8 +556,8 @@ PackedFilters packed_filters(const tdh_net::Layer &L, int batch, int flip) {
 // training: the pass is the first half of a train step: an output that only the kernel which
 // computes it would read (a first convolution's, with the max-pool directly behind it in the
 // same kernel) is not written
-int forward(tdh_net *net, int batch, const float *x, bool packed = false, const float *xent_t = nullptr,
-            float *xent_dz = nullptr, const TailPlan *tail = nullptr, bool training = false) {
+int forward(tdh_net *net, int batch, const float *x, const float *xent_t = nullptr, float *xent_dz = nullptr,
+            const TailPlan *tail = nullptr, bool training = false) {
   const KeepF32 keep(training);
   const float *in = x;
   const int n     = static_cast<int>(net->layers.size());
@@ -491,7 +569,7 @@ int forward(tdh_net *net, int batch, const float *x, bool packed = false, const 
       case TDH_L_CONV:
         TDH_TRY(ws_begin(conv2d_workspace_bytes(&s.conv, batch)));
       {
-        const PackedFilters wp = packed ? packed_filters(L, batch, 0) : PackedFilters();
+        const PackedFilters wp = packed_filters(L, batch, 0);
         const bool has_wp = static_cast<bool>(wp);
         const bool fuse = (net->flags & TDH_NET_FUSE_ACT_GRAD) != 0;
         auto pointwise = [&](int k) {
@@ -688,10 +766,10 @@ int tdh_net_create(const tdh_layer *layers, int n_layers, int max_batch, int fla
           at[flip] = total;
           total += padded(conv_packed_bytes(&L.spec.conv, CONV_PACK_X3, flip) / sizeof(float));
         }
-      if ((rc = net_alloc(net, total, &L.wp_fwd, false))) break;
-      L.wp_dx = L.wp_fwd + padded(L.w_size);
-      if (at[0]) L.wx_fwd = L.wp_fwd + at[0];
-      if (at[1]) L.wx_dx = L.wp_fwd + at[1];
+      if ((rc = net_alloc(net, total, &L.copy[0], false))) break;
+      L.copy[tdh_net::Layer::DX_F32] = L.copy[0] + padded(L.w_size);
+      if (at[0]) L.copy[tdh_net::Layer::FWD_X3] = L.copy[0] + at[0];
+      if (at[1]) L.copy[tdh_net::Layer::DX_X3] = L.copy[0] + at[1];
     }
     if (!L.tbl.empty()) {
       float *p = nullptr;
@@ -727,15 +805,11 @@ int tdh_net_create(const tdh_layer *layers, int n_layers, int max_batch, int fla
         const size_t n = which ? L.b_size : L.w_size;
         if (!n) continue;
         OptTensor t;
-        t.wp_fwd = t.wp_dx = nullptr;
-        t.wx_fwd = t.wx_dx = nullptr;
+        std::fill(t.packed, t.packed + 4, nullptr);   // (keep_copies)
         t.tbl = nullptr;
         t.C = t.Kc = t.rs = 1;
-        if (!which && L.wp_fwd) {
-          t.wp_fwd = L.wp_fwd;
-          t.wp_dx  = L.wp_dx;
-          t.wx_fwd = reinterpret_cast<uint16_t *>(L.wx_fwd);
-          t.wx_dx  = reinterpret_cast<uint16_t *>(L.wx_dx);
+        if (!which && L.copy[0]) {
+          L.opt_entry = static_cast<int>(table.size());
           t.tbl    = L.spec.conv.tbl ? L.tbl_dev : nullptr;
           t.C      = static_cast<uint32_t>(L.spec.conv.in_c);
           t.Kc     = static_cast<uint32_t>(L.spec.conv.out_c);
@@ -843,14 +917,18 @@ static float *net_param_ptr(tdh_net *net, int layer, int which) {
   return which == 0 ? L.w : (which == 1 ? L.b : nullptr);
 }
 float *tdh_net_param(tdh_net *net, int layer, int which) {
-  if (net) net->packs_valid = false;  // the caller may write through the pointer
-  return net ? net_param_ptr(net, layer, which) : nullptr;
+  if (!net) return nullptr;
+  float *p = net_param_ptr(net, layer, which);
+  if (p && which == 0) forget_copies(net->layers[layer]);  // the caller may write through the pointer
+  return p;
 }
 int tdh_net_set_param(tdh_net *net, int layer, int which, const float *host_src) {
   TDH_REQUIRE_INIT();
-  float *dst = tdh_net_param(net, layer, which);  // marks the packed filters stale
+  TDH_CHECK_ARG(net != nullptr, "tdh_net_set_param: null net");
+  float *dst = net_param_ptr(net, layer, which);
   const size_t n = tdh_net_param_size(net, layer, which);
   TDH_CHECK_ARG(n == 0 || (dst && host_src), "tdh_net_set_param: no such parameter");
+  if (n && which == 0) forget_copies(net->layers[layer]);
   return tdh_memcpy_h2d(dst, host_src, n * sizeof(float));
 }
 int tdh_net_reset_optimizer(tdh_net *net) {
@@ -878,8 +956,9 @@ int tdh_net_update_weights(tdh_net *net, tdh_opt *opt) {
   TDH_REQUIRE_INIT();
   TDH_CHECK_ARG(net && opt, "tdh_net_update_weights: null argument");
   // the optimizer kernel keeps the packed filter copies of a graph net current, as in a step
-  TDH_TRY(launch_opt_update_multi(opt, net->opt_table, net->opt_tensors, net->opt_blocks,
-                                  net->opt_params, 1.0f, 1, nullptr, nullptr, nullptr, net->opt_table_host.data()));
+  TDH_TRY(launch_opt_update_multi(opt, net->opt_table, net->opt_tensors, net->opt_blocks, net->opt_params, 1.0f, 1,
+                                  nullptr, nullptr, nullptr, net->opt_table_host.data()));
+  after_update(net);
   return post_update(net);
 }
 int tdh_net_set_phase(tdh_net *net, int train) {
@@ -930,27 +1009,11 @@ const int32_t *tdh_net_layer_argmax(const tdh_net *net, int layer) {
   return (layer >= 0 && layer < static_cast<int>(net->layers.size())) ? net->layers[layer].argmax : nullptr;
 }
 
-// The filters in the stride-1 kernels' layout: packed here when the weights came from outside
-// (creation, tdh_net_set_param, a pointer handed out), by the optimizer kernel after that.
-static int refresh_packs(tdh_net *net) {
-  if (!(net->flags & TDH_NET_GRAPH) || net->packs_valid) return TDH_OK;
-  for (tdh_net::Layer &L : net->layers) {
-    if (!L.wp_fwd) continue;
-    for (int flip = 0; flip < 2; ++flip) {
-      TDH_TRY(conv_pack_filters(&L.spec.conv, CONV_PACK_F32, flip, L.w, L.tbl_dev, flip ? L.wp_dx : L.wp_fwd));
-      if (float *wx = flip ? L.wx_dx : L.wx_fwd)
-        TDH_TRY(conv_pack_filters(&L.spec.conv, CONV_PACK_X3, flip, L.w, L.tbl_dev, wx));
-    }
-  }
-  net->packs_valid = true;
-  return TDH_OK;
-}
-
 int tdh_net_forward(tdh_net *net, int batch, const float *x) {
   TDH_REQUIRE_INIT();
   TDH_CHECK_ARG(net && x && batch > 0 && batch <= net->max_batch, "tdh_net_forward: bad argument");
-  TDH_TRY(refresh_packs(net));
-  return forward(net, batch, x, net->packs_valid);
+  TDH_TRY(pack_copies(net, batch, x, /*training=*/false));
+  return forward(net, batch, x);
 }
 
 // Queues one whole train step on the library stream. forked (only while the stream is being
@@ -992,8 +1055,10 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
     TDH_TRY(launch_opt_update_multi(opt, net->opt_table, net->opt_tensors, net->opt_blocks, net->opt_params, 1.0f,
                                     1, powers_in, powers_out, to_optimizer ? &pending : nullptr,
                                     net->opt_table_host.data()));
+    after_update(net);
     return post_update(net);
   }
+  TDH_TRY(pack_copies(net, batch, x, /*training=*/true));
   Context &c = ctx();
   struct KeepScratch {  // hands out disjoint scratch pieces for the whole backward pass
     Context &c;
@@ -1025,8 +1090,6 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
   const bool as_forked = !forked && ((profiling_active() && (net->flags & TDH_NET_GRAPH) && net_forks(net, batch)) ||
                                      small_defers);
   const int n   = static_cast<int>(net->layers.size());
-  // the optimizer kernel keeps the packed filters of the stride-1 kernels current
-  const bool packed = net->packs_valid;
   tdh_net::Layer &last = net->layers[n - 1];
   int first_bwd        = n - 1;
   int tail_done        = -1;     // this layer already has the gradient of its input
@@ -1041,13 +1104,13 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
   tail_done           = plan.layer;
   if (loss_kind == TDH_LOSS_CE_MULTICLASS && last.spec.kind == TDH_L_ACT &&
       last.spec.act == TDH_ACT_SOFTMAX && n >= 2) {
-    TDH_TRY(forward(net, batch, x, packed, t, net->layers[n - 2].dout, tail_done >= 0 ? &plan : nullptr, true));
+    TDH_TRY(forward(net, batch, x, t, net->layers[n - 2].dout, tail_done >= 0 ? &plan : nullptr, true));
     first_bwd = n - 2;
   } else if (tail_done >= 0) {
     // mse on a closing fully-connected layer: its kernel writes the loss gradient too
-    TDH_TRY(forward(net, batch, x, packed, t, last.dout, &plan, true));
+    TDH_TRY(forward(net, batch, x, t, last.dout, &plan, true));
   } else {
-    TDH_TRY(forward(net, batch, x, packed, nullptr, nullptr, nullptr, true));
+    TDH_TRY(forward(net, batch, x, nullptr, nullptr, nullptr, true));
     TDH_TRY(launch_loss_grad(loss_kind, batch, static_cast<int>(last.out_size), last.out, t,
                              last.dout));
   }
@@ -1114,8 +1177,7 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
         TDH_TRY(ws_begin((forked || as_forked ? 3 : 1) * conv2d_workspace_bytes(&s.conv, batch)));
       {
         const PoolGather *gp = i == through_pool_for ? &through_pool : nullptr;
-        const PackedFilters wp = !packed ? PackedFilters()
-                                 : conv_pair ? packed_as(L, CONV_PACK_X3, 1) : packed_filters(L, batch, 1);
+        const PackedFilters wp = conv_pair ? packed_as(L, CONV_PACK_X3, 1) : packed_filters(L, batch, 1);
         // the layer that reads this dX next (behind a folded activation) is a max-pool: its
         // backward kernel can add up a split reduction of dX
         const int reader = i - 1 - ((i >= 1 && net->layers[i - 1].grad_folded) ? 1 : 0);
@@ -1321,6 +1383,7 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
   TDH_TRY(launch_opt_update_multi(opt, net->opt_table, net->opt_tensors, net->opt_blocks,
                                   net->opt_params, 1.0f, 1, powers_in, powers_out,
                                   to_optimizer ? &pending : nullptr, net->opt_table_host.data()));
+  after_update(net);
   return post_update(net);
 }
 
@@ -1337,7 +1400,9 @@ static bool same_key(const tdh_net::GraphKey &a, const tdh_net::GraphKey &b) {
 // captured into one graph and replayed
 static int train_steps(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, int n_steps, const float *const *xs,
                        const float *const *ts, int do_update) {
-  TDH_TRY(refresh_packs(net));
+  const bool tiny = tiny_step_applies(net, loss_kind);   // (reads the weights themselves)
+  if (!tiny)
+    for (int s = 0; s < n_steps; ++s) TDH_TRY(keep_copies(net, batch, xs[s]));
   // per-kernel timing needs the launches themselves, not a replay
   if (!(net->flags & TDH_NET_GRAPH) || profiling_active() || (n_steps == 1 && step_outlasts_launches(net, loss_kind, batch))) {
     // (the timing pass of a branching step keeps every layer's scratch piece until the optimizer
@@ -1354,6 +1419,8 @@ static int train_steps(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, int
   key.n_steps = n_steps;
   for (int s = 0; s < n_steps; ++s) { key.x[s] = xs[s]; key.t[s] = ts[s]; }
   key.test_phase = net->test_phase;
+  if (!tiny)
+    for (int s = 0; s < n_steps; ++s) TDH_TRY(pack_copies(net, batch, xs[s], /*training=*/true));
   // (only steps that advance the powers take turns between the two buffers)
   const bool powers_move = opt && do_update && (opt->kind == TDH_OPT_ADAM || opt->kind == TDH_OPT_ADAMAX);
   key.powers_at = powers_move ? net->powers_at : 0;
@@ -1399,6 +1466,8 @@ static int train_steps(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, int
       e = hipStreamEndCapture(c.stream, &graph);
     }
     c.ws_locked = false;
+    if (rc != TDH_OK || e != hipSuccess || !graph)   // (nothing of what was queued has run)
+      for (tdh_net::Layer &L : net->layers) forget_copies(L);
     if (rc != TDH_OK) {
       if (graph) (void)hipGraphDestroy(graph);
       return rc;
@@ -1428,6 +1497,7 @@ static int train_steps(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, int
   TDH_HIP(hipGraphLaunch(slot->exec, ctx().stream));
   net->dx_unwritten  = slot->dx_unwritten;
   net->out_unwritten = slot->out_unwritten;
+  if (do_update) after_update(net);   // (as the capture left it)
   if (opt && do_update) {
     // advance the host object exactly as the eager path does
     for (int j = 0; j < net->opt_tensors * n_steps; ++j) {
