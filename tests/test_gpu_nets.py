@@ -1195,3 +1195,41 @@ def test_passes_pack_the_filters_that_they_read_and_no_others(T, O, W):
     ref.weight(0)[:] = a
     assert step(600) == 1 and step(600) == 0
     net.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("flags", [0, 2, 3])
+@pytest.mark.parametrize("batch", [5, 80, 600])
+def test_weights_written_by_their_address_are_the_ones_used(T, O, W, flags, batch):
+    """tdh_net_param's pointer is asked for once and written through between the calls, inference as well as steps of
+    one and of three mini-batches: each call reads the weights as they are, not a packed copy from before."""
+    rng = np.random.default_rng(21)
+    net, ref = _stride1_net(T, O, W, batch, flags, rng)
+    convs = [i for i, l in enumerate(STRIDE1_NET) if l[0] == "conv"]
+    at = {i: T.DevBuf.view(T.lib().tdh_net_param(net.h, i, 0), (net.param_size(i, 0),)) for i in convs}
+    x = rng.standard_normal((batch, net.in_size())).astype(np.float32)
+    t = rng.uniform(-0.8, 0.8, (batch, 10)).astype(np.float32)
+    xd, td = T.to_device(x), T.to_device(t)
+    opt, ropt = T.opt_desc("sgd", alpha=1e-5), O.opt_desc("sgd", alpha=1e-5)
+    for turn in range(3):
+        for i in convs:
+            a = rng.uniform(-0.05, 0.05, net.param_size(i, 0)).astype(np.float32)
+            at[i].upload(a)
+            ref.weight(i)[:] = a
+        net.forward(batch, xd)
+        ref.forward(x)
+        assert_close(net.layer_out(7, batch).ravel(), ref.layer_out(7, batch).ravel(), what=f"turn {turn} forward")
+        for i in convs:
+            a = rng.uniform(-0.05, 0.05, net.param_size(i, 0)).astype(np.float32)
+            at[i].upload(a)
+            ref.weight(i)[:] = a
+        if turn == 1:
+            net.train_steps(opt, "mse", batch, [xd] * 3, [td] * 3)
+        else:
+            net.train_step(opt, "mse", batch, xd, td)
+        for _ in range(3 if turn == 1 else 1):
+            ref.train_step(ropt, "mse", x, t)
+        assert_close(net.layer_out(7, batch).ravel(), ref.layer_out(7, batch).ravel(), what=f"turn {turn} step")
+        for i in convs:
+            assert_close(net.get_param(i, 0), ref.weight(i), what=f"turn {turn} weights {i}")
+    net.close()

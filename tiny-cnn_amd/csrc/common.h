@@ -245,11 +245,13 @@ struct OptIndex {
   int8_t pend_of[OPT_INDEX_MAX];        // index into OptPending::sum, or -1
   int n;
 };
-// host_table: the host copy of dev_table (for the index above), or NULL
+// host_table: the host copy of dev_table (for the index above), or NULL; keep_packed: write the
+// packed copies as well
 int launch_opt_update_multi(tdh_opt *o, const OptTensor *dev_table, int n_tensors,
                             int total_blocks, double total_params, float grad_scale,
                             int zero_grad, const float *powers_in, float *powers_out,
-                            const OptPending *pending = nullptr, const OptTensor *host_table = nullptr);
+                            const OptPending *pending = nullptr, const OptTensor *host_table = nullptr,
+                            bool keep_packed = true);
 // conv.hip: the recorded split reductions in the optimizer's form (false: they do not all fit its
 // form or number). They stay recorded: flush_deferred_reduces launches or forgets them.
 bool peek_deferred_reduces(OptPending *out);

@@ -458,7 +458,7 @@ template <int KIND, int NSTATE>
 __global__ void __launch_bounds__(EW_THREADS)
 opt_multi_kernel(const OptTensor *__restrict__ table, const int n_tensors, OptScalars p,
                  float b1_t, float b2_t, const float *powers_in, float *powers_out, const int advance,
-                 const int zero_grad, const OptPending pend, const OptIndex idx) {
+                 const int zero_grad, const OptPending pend, const OptIndex idx, const bool keep_packed) {
   if (powers_in) {
     b1_t = powers_in[0];
     b2_t = powers_in[1];
@@ -551,7 +551,7 @@ opt_multi_kernel(const OptTensor *__restrict__ table, const int n_tensors, OptSc
     for (uint32_t c = 0; c < VEC; ++c) pending_sum[grp][VEC * o + c] = s4[c];
     __syncthreads();
   }
-  const bool packs = t.packed[0] || t.packed[1] || t.packed[2] || t.packed[3];
+  const bool packs = keep_packed && (t.packed[0] || t.packed[1] || t.packed[2] || t.packed[3]);
   auto grad = [&](const uint32_t i, const float g) {
     if (pj < 0) return g;
     float tt = pending_sum[0][i - beg];
@@ -865,7 +865,7 @@ size_t rowsum_workspace_bytes(int outer, int rows, int cols) {
 int launch_opt_update_multi(tdh_opt *o, const OptTensor *dev_table, int n_tensors,
                             int total_blocks, double total_params, float grad_scale,
                             int zero_grad, const float *powers_in, float *powers_out,
-                            const OptPending *pending, const OptTensor *host_table) {
+                            const OptPending *pending, const OptTensor *host_table, bool keep_packed) {
   if (n_tensors <= 0) return TDH_OK;
   OptPending pend;
   pend.n = 0;
@@ -906,7 +906,7 @@ int launch_opt_update_multi(tdh_opt *o, const OptTensor *dev_table, int n_tensor
 #define TDH_LAUNCH_MULTI(KIND, NS)                                                            \
   TDH_LAUNCH((opt_multi_kernel<KIND, NS>), dim3(total_blocks), dim3(EW_THREADS), 0,   \
                      ctx().stream, dev_table, n_tensors, p, o->b1_t, o->b2_t,                  \
-                     powers_in, powers_out, advance, zero_grad, pend, idx)
+                     powers_in, powers_out, advance, zero_grad, pend, idx, keep_packed)
   switch (o->kind) {
     case TDH_OPT_SGD: TDH_LAUNCH_MULTI(TDH_OPT_SGD, 0); break;
     case TDH_OPT_MOMENTUM: TDH_LAUNCH_MULTI(TDH_OPT_MOMENTUM, 1); break;

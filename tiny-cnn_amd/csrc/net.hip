@@ -45,6 +45,9 @@ struct tdh_net {
   float *dx_in   = nullptr;  // gradient w.r.t. the network input
   tdh::OptTensor *opt_table = nullptr;  // device table of trainable tensors, update order
   std::vector<tdh::OptTensor> opt_table_host;  // (its host copy)
+  // the address of a convolution's weights has been handed out (tdh_net_param): they may be written
+  // at any time, so every call packs the copies that it reads
+  bool weights_out = false;
   struct Reads {   // the copies that passes of this kind read, of the last batch size asked for (copies_read)
     int batch = 0;
     bool aligned = false;
@@ -63,6 +66,7 @@ struct tdh_net {
   struct GraphKey {
     int batch = 0, loss = 0, do_update = 0, test_phase = 0;
     int powers_at = 0;                  // which buffer of the powers the (first) captured optimizer launch reads
+    bool packs = false;                 // the graph packs the filters that its first step reads
     int n_steps = 1;
     const float *x[kMaxSteps] = {}, *t[kMaxSteps] = {};
     const void *scratch = nullptr;      // the library scratch buffer the captured kernels use
@@ -542,10 +546,10 @@ int keep_copies(tdh_net *net, int batch, const float *x) {
   return TDH_OK;
 }
 
-// The weights have been updated, and with them the copies that the optimizer kernel keeps.
-void after_update(tdh_net *net) {
+// The weights have been updated; kept: by a launch that wrote the copies it keeps as well.
+void after_update(tdh_net *net, bool kept) {
   for (tdh_net::Layer &L : net->layers)
-    for (int c = 0; c < tdh_net::Layer::COPIES; ++c) L.current[c] = L.current[c] && L.kept[c];
+    for (int c = 0; c < tdh_net::Layer::COPIES; ++c) L.current[c] = L.current[c] && L.kept[c] && kept;
 }
 
 // xent_t / xent_dz: the net ends in softmax and the step's loss is cross_entropy_multiclass: the
@@ -919,7 +923,7 @@ static float *net_param_ptr(tdh_net *net, int layer, int which) {
 float *tdh_net_param(tdh_net *net, int layer, int which) {
   if (!net) return nullptr;
   float *p = net_param_ptr(net, layer, which);
-  if (p && which == 0) forget_copies(net->layers[layer]);  // the caller may write through the pointer
+  if (p && which == 0 && net->layers[layer].copy[0]) net->weights_out = true;
   return p;
 }
 int tdh_net_set_param(tdh_net *net, int layer, int which, const float *host_src) {
@@ -957,8 +961,8 @@ int tdh_net_update_weights(tdh_net *net, tdh_opt *opt) {
   TDH_CHECK_ARG(net && opt, "tdh_net_update_weights: null argument");
   // the optimizer kernel keeps the packed filter copies of a graph net current, as in a step
   TDH_TRY(launch_opt_update_multi(opt, net->opt_table, net->opt_tensors, net->opt_blocks, net->opt_params, 1.0f, 1,
-                                  nullptr, nullptr, nullptr, net->opt_table_host.data()));
-  after_update(net);
+                                  nullptr, nullptr, nullptr, net->opt_table_host.data(), !net->weights_out));
+  after_update(net, !net->weights_out);
   return post_update(net);
 }
 int tdh_net_set_phase(tdh_net *net, int train) {
@@ -1009,9 +1013,17 @@ const int32_t *tdh_net_layer_argmax(const tdh_net *net, int layer) {
   return (layer >= 0 && layer < static_cast<int>(net->layers.size())) ? net->layers[layer].argmax : nullptr;
 }
 
+// At the start of a call: where the caller may have written weights by their address, no copy is
+// taken to hold them.
+static void distrust_copies(tdh_net *net) {
+  if (!net->weights_out) return;
+  for (tdh_net::Layer &L : net->layers) forget_copies(L);
+}
+
 int tdh_net_forward(tdh_net *net, int batch, const float *x) {
   TDH_REQUIRE_INIT();
   TDH_CHECK_ARG(net && x && batch > 0 && batch <= net->max_batch, "tdh_net_forward: bad argument");
+  distrust_copies(net);
   TDH_TRY(pack_copies(net, batch, x, /*training=*/false));
   return forward(net, batch, x);
 }
@@ -1021,9 +1033,10 @@ int tdh_net_forward(tdh_net *net, int batch, const float *x) {
 // stream, because nothing before the optimizer waits for them; the main stream carries only
 // the chain forward -> loss -> dX ... -> dX, and the two join in front of the optimizer. The
 // kernels and their arguments are the same either way, so are the results.
+// keep: the update writes the packed filters that the next step reads as well.
 static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, const float *x,
                         const float *t, int do_update, const float *powers_in, float *powers_out,
-                        bool forked = false) {
+                        bool keep_packs, bool forked = false) {
   const KeepF32 keep_f32(has_batchnorm(net));
   if (tiny_step_applies(net, loss_kind)) {
     // a small net: one workgroup per sample runs forward, loss and the input gradients out of
@@ -1054,8 +1067,8 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
     if (!do_update) return TDH_OK;
     TDH_TRY(launch_opt_update_multi(opt, net->opt_table, net->opt_tensors, net->opt_blocks, net->opt_params, 1.0f,
                                     1, powers_in, powers_out, to_optimizer ? &pending : nullptr,
-                                    net->opt_table_host.data()));
-    after_update(net);
+                                    net->opt_table_host.data(), keep_packs));
+    after_update(net, keep_packs);
     return post_update(net);
   }
   TDH_TRY(pack_copies(net, batch, x, /*training=*/true));
@@ -1382,8 +1395,8 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
   // cleared (layer.h:680)
   TDH_TRY(launch_opt_update_multi(opt, net->opt_table, net->opt_tensors, net->opt_blocks,
                                   net->opt_params, 1.0f, 1, powers_in, powers_out,
-                                  to_optimizer ? &pending : nullptr, net->opt_table_host.data()));
-  after_update(net);
+                                  to_optimizer ? &pending : nullptr, net->opt_table_host.data(), keep_packs));
+  after_update(net, keep_packs);
   return post_update(net);
 }
 
@@ -1391,7 +1404,7 @@ static bool same_key(const tdh_net::GraphKey &a, const tdh_net::GraphKey &b) {
   // field by field: a caller's tdh_opt may carry padding or unused fields it never wrote
   const tdh_opt &p = a.hyper, &q = b.hyper;
   return a.batch == b.batch && a.loss == b.loss && a.do_update == b.do_update && a.test_phase == b.test_phase &&
-         a.powers_at == b.powers_at && a.n_steps == b.n_steps &&
+         a.powers_at == b.powers_at && a.n_steps == b.n_steps && a.packs == b.packs &&
          std::equal(a.x, a.x + a.n_steps, b.x) && std::equal(a.t, a.t + a.n_steps, b.t) && a.scratch == b.scratch && p.kind == q.kind && p.alpha == q.alpha &&
          p.lambda == q.lambda && p.mu == q.mu && p.b1 == q.b1 && p.b2 == q.b2 && p.eps == q.eps;
 }
@@ -1401,15 +1414,19 @@ static bool same_key(const tdh_net::GraphKey &a, const tdh_net::GraphKey &b) {
 static int train_steps(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, int n_steps, const float *const *xs,
                        const float *const *ts, int do_update) {
   const bool tiny = tiny_step_applies(net, loss_kind);   // (reads the weights themselves)
+  distrust_copies(net);
   if (!tiny)
     for (int s = 0; s < n_steps; ++s) TDH_TRY(keep_copies(net, batch, xs[s]));
+  // whoever writes weights by their address does so between two calls: what the last step of a call
+  // would keep is packed again by the next call
+  auto keeps = [&](int s) { return !net->weights_out || s + 1 < n_steps; };
   // per-kernel timing needs the launches themselves, not a replay
   if (!(net->flags & TDH_NET_GRAPH) || profiling_active() || (n_steps == 1 && step_outlasts_launches(net, loss_kind, batch))) {
     // (the timing pass of a branching step keeps every layer's scratch piece until the optimizer
     // has read the split sums: the buffer must not grow, and so move, on the way)
     for (int s = 0; s < n_steps; ++s) {
       if (net->flags & TDH_NET_GRAPH) TDH_TRY(ws_begin(net->scratch));
-      TDH_TRY(enqueue_step(net, opt, loss_kind, batch, xs[s], ts[s], do_update, nullptr, nullptr));
+      TDH_TRY(enqueue_step(net, opt, loss_kind, batch, xs[s], ts[s], do_update, nullptr, nullptr, keeps(s)));
     }
     return TDH_OK;
   }
@@ -1419,7 +1436,8 @@ static int train_steps(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, int
   key.n_steps = n_steps;
   for (int s = 0; s < n_steps; ++s) { key.x[s] = xs[s]; key.t[s] = ts[s]; }
   key.test_phase = net->test_phase;
-  if (!tiny)
+  key.packs      = net->weights_out && !tiny;
+  if (!key.packs && !tiny)
     for (int s = 0; s < n_steps; ++s) TDH_TRY(pack_copies(net, batch, xs[s], /*training=*/true));
   // (only steps that advance the powers take turns between the two buffers)
   const bool powers_move = opt && do_update && (opt->kind == TDH_OPT_ADAM || opt->kind == TDH_OPT_ADAMAX);
@@ -1460,7 +1478,7 @@ static int train_steps(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, int
         // (steps that advance the powers take turns between the two buffers inside the graph as well)
         const int at = powers_move ? (key.powers_at + s) & 1 : key.powers_at;
         rc = enqueue_step(net, opt ? &capture_opt : nullptr, loss_kind, batch, xs[s], ts[s], do_update,
-                          net->dev_powers + 4 * at, net->dev_powers + 4 * (1 - at),
+                          net->dev_powers + 4 * at, net->dev_powers + 4 * (1 - at), keeps(s),
                           /*forked=*/net_forks(net, batch));
       }
       e = hipStreamEndCapture(c.stream, &graph);
@@ -1497,7 +1515,7 @@ static int train_steps(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, int
   TDH_HIP(hipGraphLaunch(slot->exec, ctx().stream));
   net->dx_unwritten  = slot->dx_unwritten;
   net->out_unwritten = slot->out_unwritten;
-  if (do_update) after_update(net);   // (as the capture left it)
+  if (do_update) after_update(net, !net->weights_out);   // (as the capture left it)
   if (opt && do_update) {
     // advance the host object exactly as the eager path does
     for (int j = 0; j < net->opt_tensors * n_steps; ++j) {
