@@ -169,7 +169,8 @@ int tdh_conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const floa
  * hipMalloc). It has no counterpart in the reference. It is refused (TDH_ERR_INVALID) while a
  * network step of this library is being captured or holds the scratch buffer, and
  * (TDH_ERR_UNSUPPORTED) for a descriptor with a connection table. Same
- * arguments, kernels and results as tdh_conv2d_bwd, but the kernels' scratch (split partial
+ * arguments, kernels and results as tdh_conv2d_bwd (a shape whose three-part kernels would not fit
+ * runs the fp32 ones instead), but the kernels' scratch (split partial
  * sums, repacked filters) lies in a static 64 MiB device array that the library holds on every
  * device it is initialised on, and the call allocates and frees nothing. A shape whose scratch
  * need exceeds the array is refused with TDH_ERR_INVALID (the message states both sizes); use

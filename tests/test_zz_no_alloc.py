@@ -115,3 +115,27 @@ def test_static_scratch_refuses_what_does_not_fit(T):
     dx2, dw2, db2 = T.DevBuf((2, 256)), T.DevBuf((144,)), T.DevBuf((4,))
     T.conv2d_bwd_static(d2, 2, T.to_device(one), T.to_device(np.zeros(144, np.float32)), T.to_device(one), dx2, dw2, db2)
     assert np.array_equal(db2.numpy(), np.full(4, 128.0, np.float32))
+
+
+@pytest.mark.parametrize("cfg", [
+    # in_w, in_h, in_c, k, out_c, same, stride, batch: what the operator may take beside the fp32 kernels
+    # that it once had (another product for dX, wider packed filters, more slices of dW) is over 64 MiB
+    (13, 60, 32, 7, 128, True, 2, 40),     # dX by phases of the stride
+    (24, 90, 128, 7, 128, True, 1, 1),     # three-part filters
+    (70, 9, 192, 5, 192, False, 1, 376),   # three-part dW: too many slices, it runs in fp32
+])
+def test_static_scratch_serves_what_its_fp32_kernels_fit(T, cfg):
+    """Compared with the allocating entry point, whose kernels round differently: 800 to 5000 products a sum."""
+    iw, ih, ic, k, oc, same, st, bs = cfg
+    rng = np.random.default_rng(9)
+    d = T.conv_desc(iw, ih, ic, k, k, oc, pad_same=same, w_stride=st, h_stride=st)
+    ow, oh = T.conv_out_shape(d)
+    x = T.to_device(rng.standard_normal((bs, ic * ih * iw)).astype(np.float32))
+    w = T.to_device(rng.uniform(-0.1, 0.1, oc * ic * k * k).astype(np.float32))
+    dy = T.to_device(rng.standard_normal((bs, oc * oh * ow)).astype(np.float32))
+    got = [T.DevBuf((bs, ic * ih * iw)), T.DevBuf((oc * ic * k * k,)), T.DevBuf((oc,))]
+    want = [T.DevBuf(b.shape) for b in got]
+    T.conv2d_bwd_static(d, bs, x, w, dy, *got)
+    T.conv2d_bwd(d, bs, x, w, dy, *want)
+    for g, r, name in zip(got, want, ("dx", "dw", "db")):
+        assert_close(g.numpy().ravel(), r.numpy().ravel(), what=f"{cfg} {name}")

@@ -549,12 +549,20 @@ int tdh_conv2d_bwd_static(const tdh_conv_desc *d, int batch, const float *x, con
                      "(the table is staged through a host copy); use tdh_conv2d_bwd");
   Context &c = ctx();
   TDH_CHECK_ARG(!c.ws_keep && !c.ws_locked, "tdh_conv2d_bwd_static: called inside a network step");
-  const size_t need = conv2d_workspace_bytes(d, batch);
-  if (need > kStaticScratchBytes)
+  const size_t declared = conv2d_declared_bytes(d, batch);
+  if (declared > kStaticScratchBytes)
     return set_error(TDH_ERR_INVALID,
                      "tdh_conv2d_bwd_static: this shape needs %zu bytes of scratch, the static buffer "
                      "holds %zu; use tdh_conv2d_bwd",
-                     need, kStaticScratchBytes);
+                     declared, kStaticScratchBytes);
+  // What this call takes. The three-part kernels of some shapes take more than the fp32 ones (more
+  // slices, wider packed filters): those shapes run in fp32 here.
+  auto needed = [&] {
+    return conv2d_bwd_workspace_bytes(d, batch, x, dy, dx != nullptr, dw != nullptr, d->has_bias && db, accumulate);
+  };
+  size_t need = needed();
+  const KeepF32 keep(need > kStaticScratchBytes);
+  if (need > kStaticScratchBytes) need = needed();
   char *ptr = c.device >= 0 && c.device < kMaxDevices ? g_static_scratch[c.device] : nullptr;
   if (!ptr) return set_error(TDH_ERR_NOT_INIT, "tdh_conv2d_bwd_static: no static scratch on device %d", c.device);
   // Nothing in the array has to start at zero: every partial-sum slice, packed filter and

@@ -452,6 +452,9 @@ bool conv_s1_applicable(int R, int S, int batch, int KC, int MC, int IH, int IW,
                         int ph, int pw);
 size_t conv_s1_workspace_bytes(int R, int S, int batch, int C, int Kc, int flip, int IH, int IW,
                                int OH, int OW, int ph, int pw);
+// ... of the kernel that conv_s1_run takes
+size_t conv_s1_run_workspace_bytes(int R, int S, int batch, int C, int Kc, int flip, int IH, int IW,
+                                   int OH, int OW, int ph, int pw);
 int conv_s1_run(int R, int S, int batch, int C, int Kc, int flip, const float *in, const float *w,
                 const uint8_t *tbl_dev, const float *bias, float *out, int IH, int IW, int OH,
                 int OW, int ph, int pw, ActGrad ag, const char *tag,
@@ -472,6 +475,9 @@ bool conv_dw_halo_applicable(int R, int S, int batch, int C, int Kc, int H, int 
                              int ph, int pw);
 size_t conv_dw_halo_workspace_bytes(int R, int S, int batch, int C, int Kc, int H, int W, int OH,
                                     int OW, int ph, int pw);
+// ... of the kernel that conv_dw_halo_run takes for these tensors
+size_t conv_dw_halo_run_workspace_bytes(int R, int S, int batch, int C, int Kc, const float *x, const float *dy,
+                                        int H, int W, int OH, int OW, int ph, int pw);
 int conv_dw_halo_run(int R, int S, int batch, int C, int Kc, const float *x, const float *dy,
                      float *dw, int H, int W, int OH, int OW, int ph, int pw, int accumulate,
                      float *db = nullptr);
@@ -485,8 +491,13 @@ bool conv_bwd_pair_applicable(int R, int S, int batch, int C, int Kc, int H, int
 int conv_bwd_pair_run(int R, int S, int batch, int C, int Kc, int H, int W, int ph, int pw, const float *x,
                       const float *dy, const float *w, PackedFilters prepacked, float *dx, ActGrad dx_act, float *dw,
                       float *db, int accumulate);
-// workspace bytes the op may ask for (so a net can reserve it before graph capture)
+size_t conv_bwd_pair_workspace_bytes(int R, int S, int batch, int C, int Kc, int H, int W, int ph, int pw);
+// workspace bytes the op may ask for, whichever of its kernels runs (so a net can reserve it before
+// graph capture), and what one call of conv2d_bwd without packed filters takes
 size_t conv2d_workspace_bytes(const tdh_conv_desc *d, int batch);
+size_t conv2d_declared_bytes(const tdh_conv_desc *d, int batch);
+size_t conv2d_bwd_workspace_bytes(const tdh_conv_desc *d, int batch, const float *x, const float *dy, bool dx, bool dw,
+                                  bool db, int accumulate);
 size_t fc_workspace_bytes(int in, int out, int batch);
 bool fc_bwd_fuses(int in, int out, int batch);
 // The last fully-connected layer in front of softmax + cross_entropy_multiclass in one launch:

@@ -1145,6 +1145,42 @@ static bool fwd_small_applies(const ConvGeom &g, int batch) {
 }  // namespace
 
 static size_t first_both_workspace_bytes(const tdh_conv_desc *d, const ConvGeom &g, int batch);
+static bool bwd_direct_applies(const tdh_conv_desc *d, const ConvGeom &g, int batch);
+static bool dw_small_applies(const tdh_conv_desc *d, const ConvGeom &g, int batch);
+
+// The bias gradient as one more column of the GEMM of dW: no pass over dY and no launches of its own
+// (5x5, stride 2, 21 -> 45 channels of 45x37, batch 19, dX, dW and db: 62.8 us / 58.0). Not where it
+// would start a new column of tiles; and not in a train step (which adds to its gradients), where
+// a bias gradient may be a branch of its own and has the same bits either way.
+static bool dw_takes_db(const tdh_conv_desc *d, int crs, bool db, int accumulate) {
+  return db && !d->tbl && crs % 32 != 0 && !accumulate;
+}
+
+// The scratch that the operator declares: room for the fp32 kernels of both directions side by side.
+// tdh_conv2d_bwd_static serves the shapes whose declared size fits its buffer.
+size_t conv2d_declared_bytes(const tdh_conv_desc *d, int batch) {
+  const KeepF32 fp32(true);
+  const ConvGeom g = make_geom(d);
+  const int ohw = g.OH * g.OW, crs = g.C * g.R * g.S;
+  size_t total = 0;
+  total += gemm_workspace_bytes(g.Kc, batch * ohw, crs, true);        // forward
+  total += gemm_workspace_bytes(g.Kc, crs, batch * ohw, true);        // dW
+  total += gemm_workspace_bytes(g.C, batch * g.H * g.W, g.Kc * g.R * g.S, true);  // dX
+  total += rowsum_workspace_bytes(batch, g.Kc, ohw);                  // db
+  if (d->tbl) total += ws_align(static_cast<size_t>(g.C) * g.Kc) + 2 * ws_align(sizeof(float) * g.Kc * crs);
+  total += conv_dw_small_workspace_bytes(batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.R, g.S, g.sh, g.sw,
+                                         g.dh, g.dw, g.pad_h, g.pad_w);
+  total += first_both_workspace_bytes(d, g, batch);
+  if (g.sh == 1 && g.sw == 1) {  // the LDS-halo kernels: repacked filters and split partial sums
+    // (of the weight gradient's kernels the one that takes tensors of any alignment)
+    const float *odd = reinterpret_cast<const float *>(sizeof(float));
+    total += conv_dw_halo_run_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, odd, odd, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
+    total += conv_s1_run_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, 0, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
+    total += conv_s1_run_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, 1, g.OH, g.OW, g.H, g.W,
+                                         g.R - 1 - g.pad_h, g.S - 1 - g.pad_w);
+  }
+  return total;
+}
 
 size_t conv2d_workspace_bytes(const tdh_conv_desc *d, int batch) {
   const ConvGeom g = make_geom(d);
@@ -1170,6 +1206,46 @@ size_t conv2d_workspace_bytes(const tdh_conv_desc *d, int batch) {
                                      g.R - 1 - g.pad_h, g.S - 1 - g.pad_w);
   }
 
+  return total;
+}
+
+// The branches of conv2d_bwd, in its order.
+size_t conv2d_bwd_workspace_bytes(const tdh_conv_desc *d, int batch, const float *x, const float *dy, bool dx, bool dw,
+                                  bool db, int accumulate) {
+  const ConvGeom g = make_geom(d);
+  const int ohw = g.OH * g.OW, crs = g.C * g.R * g.S;
+  const bool dy_aligned = !(reinterpret_cast<uintptr_t>(dy) & 15);
+  if (bwd_direct_applies(d, g, batch)) return 0;
+  if (dx && dw && conv_bwd_pairs(d, batch, x, dy))
+    return conv_bwd_pair_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.pad_h, g.pad_w);
+  if (dx && dw && dy_aligned && conv_bwd_one_launch(d, batch, false)) return first_both_workspace_bytes(d, g, batch);
+  size_t total = 0;
+  if (d->tbl) total += ws_align(static_cast<size_t>(g.C) * g.Kc) + 2 * ws_align(sizeof(float) * g.Kc * crs);
+  DxsPlan dxs;
+  DxPhases ph;
+  int columns = 0, longest = 0;
+  if (dx && !small_cin_dx_plan(g, dxs)) {
+    if (g.sh == 1 && g.sw == 1 &&
+        conv_s1_applicable(g.R, g.S, batch, g.Kc, g.C, g.OH, g.OW, g.H, g.W, g.R - 1 - g.pad_h, g.S - 1 - g.pad_w))
+      total += conv_s1_run_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, 1, g.OH, g.OW, g.H, g.W, g.R - 1 - g.pad_h,
+                                           g.S - 1 - g.pad_w);
+    else if (dx_phases(g, batch, ph, &columns, &longest))
+      total += gemm_workspace_bytes(g.C, columns, longest, true);
+    else
+      total += gemm_workspace_bytes(g.C, batch * g.H * g.W, g.Kc * g.R * g.S, true);
+  }
+  if (dw && dw_small_applies(d, g, batch) && dy_aligned)
+    return total + conv_dw_small_workspace_bytes(batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.R, g.S, g.sh, g.sw, g.dh, g.dw,
+                                                 g.pad_h, g.pad_w) +
+           first_both_workspace_bytes(d, g, batch);  // (its slices may be those of the launch that also computes dX)
+  if (dw) {
+    if (g.sh == 1 && g.sw == 1 &&
+        conv_dw_halo_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w))
+      total += conv_dw_halo_run_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, x, dy, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
+    else
+      total += gemm_workspace_bytes(g.Kc, crs + (dw_takes_db(d, crs, db, accumulate) ? 1 : 0), batch * ohw, true);
+  }
+  if (db) total += rowsum_workspace_bytes(batch, g.Kc, ohw);
   return total;
 }
 
@@ -1560,11 +1636,7 @@ int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
   }
   if (dw) {
     DwDyOperand A{dy, g.Kc, ohw, g.div_ohw};
-    // The bias gradient as one more column of the product: no pass over dY and no launches of its own
-    // (5x5, stride 2, 21 -> 45 channels of 45x37, batch 19, dX, dW and db: 62.8 us / 58.0). Not where it
-    // would start a new column of tiles; and not in a train step (which adds to its gradients), where
-    // a bias gradient may be a branch of its own and has the same bits either way.
-    const bool with_db = db && !d->tbl && crs % 32 != 0 && !accumulate;
+    const bool with_db = dw_takes_db(d, crs, db != nullptr, accumulate);
     DwInputOperand B{x, g, crs, with_db ? 1.0f : 0.0f};
     const bool halo = g.sh == 1 && g.sw == 1 &&
                       conv_dw_halo_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW,

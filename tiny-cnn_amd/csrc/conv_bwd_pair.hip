@@ -46,6 +46,16 @@ bool conv_bwd_pair_applicable(int R, int S, int batch, int C, int Kc, int H, int
          make_s1_pair_plan(R, S, batch, Kc, C, OH, OW, H, W, R - 1 - ph, S - 1 - pw).ok;
 }
 
+static size_t slices_bytes(const DwImgPlan &im, int Kc, int crs) {
+  return ws_align(sizeof(float) * static_cast<size_t>(im.slices) * Kc * crs) +
+         ws_align(sizeof(float) * static_cast<size_t>(im.slices) * Kc);
+}
+
+size_t conv_bwd_pair_workspace_bytes(int R, int S, int batch, int C, int Kc, int H, int W, int ph, int pw) {
+  return plan_workspace_bytes(make_s1_pair_plan(R, S, batch, Kc, C, H, W, H, W, R - 1 - ph, S - 1 - pw), R * S) +
+         slices_bytes(make_dw_img_plan(R, S, batch, C, Kc, H, W, H, W, ph, pw), Kc, C * R * S);
+}
+
 // The caller has checked conv_bwd_pair_applicable and reserved the workspace of both gradients.
 // prepacked: this filter packed for dX (read where it is in three parts), or none.
 int conv_bwd_pair_run(int R, int S, int batch, int C, int Kc, int H, int W, int ph, int pw, const float *x, const float *dy,

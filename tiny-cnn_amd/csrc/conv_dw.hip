@@ -597,6 +597,32 @@ size_t conv_dw_halo_workspace_bytes(int R, int S, int batch, int C, int Kc, int 
   return slices == 0 ? 0 : ws_align(sizeof(float) * slices * Kc * C * R * S) + ws_align(sizeof(float) * slices * Kc);
 }
 
+// the kernel that runs for these tensors: x3 if ok, else im if ok, else p (slices 0: none does)
+struct HaloChoice {
+  bool vec;
+  DwxPlan x3;
+  DwImgPlan im;
+  DwHaloPlan p;
+  int slices;
+};
+static HaloChoice choose_halo(int R, int S, int batch, int C, int Kc, const float *x, const float *dy, int H, int W,
+                              int OH, int OW, int ph, int pw) {
+  HaloChoice h;
+  h.vec = W % 4 == 0 && OW % 4 == 0 && aligned16(x) && aligned16(dy);
+  h.x3  = make_dwx_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
+  h.im  = make_dw_img_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
+  h.p   = make_dw_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
+  h.im.ok  = h.im.ok && h.vec && (h.im.size == 8 || batch >= 96);
+  h.slices = h.x3.ok ? dwx_slices(h.x3) : h.im.ok ? h.im.slices : h.p.ok ? static_cast<int>(h.p.grid.x) : 0;
+  return h;
+}
+
+size_t conv_dw_halo_run_workspace_bytes(int R, int S, int batch, int C, int Kc, const float *x, const float *dy,
+                                        int H, int W, int OH, int OW, int ph, int pw) {
+  const size_t slices = choose_halo(R, S, batch, C, Kc, x, dy, H, W, OH, OW, ph, pw).slices;
+  return ws_align(sizeof(float) * slices * Kc * C * R * S) + ws_align(sizeof(float) * slices * Kc);
+}
+
 // dw (+)= the slices of part, db (+)= those of part_db: left to the train step, or launched here
 int conv_dw_sum_slices(const void *part, const void *part_db, int slices, int Kc, int crs, float *dw, float *db,
                        int accumulate) {
@@ -617,13 +643,13 @@ int conv_dw_sum_slices(const void *part, const void *part_db, int slices, int Kc
 int conv_dw_halo_run(int R, int S, int batch, int C, int Kc, const float *x, const float *dy,
                      float *dw, int H, int W, int OH, int OW, int ph, int pw, int accumulate,
                      float *db) {
-  const bool vec = W % 4 == 0 && OW % 4 == 0 && aligned16(x) && aligned16(dy);
-  DwxPlan x3   = make_dwx_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
-  DwImgPlan im = make_dw_img_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
-  DwHaloPlan p = make_dw_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);
-  im.ok = im.ok && vec && (im.size == 8 || batch >= 96);
-  if (!p.ok && !x3.ok && !im.ok) return set_error(TDH_ERR_INVALID, "conv_dw_halo_run: shape not supported");
-  const int crs = C * R * S, slices = x3.ok ? dwx_slices(x3) : im.ok ? im.slices : static_cast<int>(p.grid.x);
+  HaloChoice h = choose_halo(R, S, batch, C, Kc, x, dy, H, W, OH, OW, ph, pw);
+  DwxPlan &x3   = h.x3;
+  DwImgPlan &im = h.im;
+  DwHaloPlan &p = h.p;
+  const bool vec = h.vec;
+  if (!h.slices) return set_error(TDH_ERR_INVALID, "conv_dw_halo_run: shape not supported");
+  const int crs = C * R * S, slices = h.slices;
   void *part = nullptr, *part_db = nullptr;
   TDH_TRY(ws_take(sizeof(float) * static_cast<size_t>(slices) * Kc * crs, &part));
   if (db) TDH_TRY(ws_take(sizeof(float) * static_cast<size_t>(slices) * Kc, &part_db));

@@ -75,6 +75,7 @@ struct S1Plan {
 
 // the plan of a dX that shares its launch with the weight gradient (conv_bwd_pair.hip)
 S1Plan make_s1_pair_plan(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw);
+size_t plan_workspace_bytes(const S1Plan &p, int RS);
 int finish_s1_split(const S1Plan &p, const float *bias, ActGrad ag, float *out, float *act_out, int act_kind);
 
 // one launcher per translation unit of kernel instances

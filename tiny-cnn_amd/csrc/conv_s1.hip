@@ -280,18 +280,28 @@ bool conv_s1_fuses_pool(int R, int S, int batch, int KC, int MC, int IH, int IW,
          static_cast<long>(MC) * OH * OW < (1L << 31);
 }
 
+// packed filters and the partial sums of a split
+size_t plan_workspace_bytes(const S1Plan &p, int RS) {
+  const size_t packed = ws_align(conv_s1_packed_bytes(p.x3 ? CONV_PACK_X3 : CONV_PACK_F32, RS, p.args.KC, p.args.MC));
+  return packed + (p.splits > 1 ? ws_align(sizeof(float) * p.splits * p.args.part_stride) : 0);
+}
+
 size_t conv_s1_workspace_bytes(int R, int S, int batch, int C, int Kc, int flip, int IH, int IW,
                                int OH, int OW, int ph, int pw) {
   const int KC = flip ? Kc : C, MC = flip ? C : Kc;
   size_t most = 0;
   for (int k = 0; k < 3; ++k) {  // (which of the kernels runs is the caller's choice as well)
     const S1Plan p = make_plan_of(k != 0, R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw, /*by_taps=*/k == 2);
-    if (!p.ok) continue;
-    size_t total = ws_align(conv_s1_packed_bytes(p.x3 ? CONV_PACK_X3 : CONV_PACK_F32, R * S, KC, MC));
-    if (p.splits > 1) total += ws_align(sizeof(float) * p.splits * p.args.part_stride);
-    most = std::max(most, total);
+    if (p.ok) most = std::max(most, plan_workspace_bytes(p, R * S));
   }
   return most;
+}
+
+size_t conv_s1_run_workspace_bytes(int R, int S, int batch, int C, int Kc, int flip, int IH, int IW,
+                                   int OH, int OW, int ph, int pw) {
+  const int KC = flip ? Kc : C, MC = flip ? C : Kc;
+  const S1Plan p = make_plan(R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw);
+  return p.ok ? plan_workspace_bytes(p, R * S) : 0;
 }
 
 int conv_pack_filters(const PackJob *jobs, int n) {
