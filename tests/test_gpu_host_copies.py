@@ -26,3 +26,16 @@ def test_a_source_may_be_overwritten_at_once_and_the_ring_comes_round(T):
         b.upload(a)
     for i, b in enumerate(bufs):
         assert (b.numpy() == i).all()
+
+
+@pytest.mark.parametrize("n", [1 << 13, 1 << 14])
+def test_a_copy_past_the_end_of_its_allocation_is_an_error(T, n):
+    buf = T.DevBuf((n,), np.uint8).upload(np.arange(n, dtype=np.uint8))
+    a = np.zeros(n, np.uint8)
+    for first in (1, n // 2, n - 1):
+        view = T.DevBuf.view(buf.ptr.value + first, (n,), np.uint8)
+        with pytest.raises(T.TdhError, match="past the end of its allocation"):
+            view.upload(a)
+        with pytest.raises(T.TdhError, match="past the end of its allocation"):
+            view.numpy()
+    assert np.array_equal(buf.numpy(), np.arange(n, dtype=np.uint8))

@@ -345,7 +345,9 @@ int tdh_memcpy_h2d(void *dst, const void *src, size_t bytes) {
   TDH_REQUIRE_INIT();
   if (bytes == 0) return TDH_OK;
   TDH_CHECK_ARG(dst && src, "tdh_memcpy_h2d: null pointer");
-  if (host_copy_up_applies(bytes)) return host_copy_up(dst, src, bytes);
+  bool small = false;
+  TDH_TRY(host_copy_up_applies(dst, bytes, &small));
+  if (small) return host_copy_up(dst, src, bytes);
   TDH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx().stream));
   TDH_HIP(hipStreamSynchronize(ctx().stream));  // the host buffer may be reused on return
   return TDH_OK;
@@ -355,7 +357,9 @@ int tdh_memcpy_d2h(void *dst, const void *src, size_t bytes) {
   TDH_REQUIRE_INIT();
   if (bytes == 0) return TDH_OK;
   TDH_CHECK_ARG(dst && src, "tdh_memcpy_d2h: null pointer");
-  if (host_copy_down_applies(bytes)) return host_copy_down(dst, src, bytes);
+  bool small = false;
+  TDH_TRY(host_copy_down_applies(src, bytes, &small));
+  if (small) return host_copy_down(dst, src, bytes);
   TDH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx().stream));
   TDH_HIP(hipStreamSynchronize(ctx().stream));
   return TDH_OK;

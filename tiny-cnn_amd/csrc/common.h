@@ -183,8 +183,10 @@ int launch_fill_zero(void *p, size_t bytes, const char *tag = "fill_zero");
 int launch_copy(void *dst, const void *src, size_t bytes);  // bytes % 4 == 0
 // hostcopy.hip: small copies between pageable host memory and the device. The upload returns when `src` has been read and is ordered on the library stream; the
 // download returns when `dst` has been written, behind the work queued before it.
-bool host_copy_up_applies(size_t bytes);
-bool host_copy_down_applies(size_t bytes);
+// applies: the copy is small and its device side is memory of this device (an error: it reaches past
+// that memory's end).
+int host_copy_up_applies(const void *device, size_t bytes, bool *applies);
+int host_copy_down_applies(const void *device, size_t bytes, bool *applies);
 int host_copy_up(void *dst, const void *src, size_t bytes);
 int host_copy_down(void *dst, const void *src, size_t bytes);
 void host_copy_release();

@@ -104,8 +104,38 @@ int launch_piece(void *dst, const void *src, size_t bytes, bool down, int i) {
 
 }  // namespace
 
-bool host_copy_up_applies(size_t bytes) { return bytes <= HC_PIECE; }
-bool host_copy_down_applies(size_t bytes) { return bytes <= HC_MAX_DOWN; }
+// What the runtime's copy would look at, and a kernel that is handed an address does not: whether it is
+// memory of this device, and whether the whole copy lies in that allocation. An address that is
+// nothing of the kind is left to the runtime's copy.
+static int kernel_may_copy(const void *device, size_t bytes, bool *may) {
+  *may = false;
+  hipPointerAttribute_t attr;
+  if (hipPointerGetAttributes(&attr, device) != hipSuccess) {
+    (void)hipGetLastError();
+    return TDH_OK;
+  }
+  if (attr.type != hipMemoryTypeDevice || attr.device != ctx().device) return TDH_OK;
+  hipDeviceptr_t base = nullptr;
+  size_t size         = 0;
+  if (hipMemGetAddressRange(&base, &size, const_cast<void *>(device)) != hipSuccess) {
+    (void)hipGetLastError();
+    return TDH_OK;
+  }
+  const size_t at = static_cast<size_t>(static_cast<const char *>(device) - static_cast<const char *>(base));
+  if (at > size || bytes > size - at)
+    return set_error(TDH_ERR_INVALID, "a copy of %zu bytes reaches past the end of its allocation (%zu bytes at %zu)", bytes,
+                     size, at);
+  *may = true;
+  return TDH_OK;
+}
+int host_copy_up_applies(const void *device, size_t bytes, bool *applies) {
+  *applies = false;
+  return bytes <= HC_PIECE ? kernel_may_copy(device, bytes, applies) : TDH_OK;
+}
+int host_copy_down_applies(const void *device, size_t bytes, bool *applies) {
+  *applies = false;
+  return bytes <= HC_MAX_DOWN ? kernel_may_copy(device, bytes, applies) : TDH_OK;
+}
 
 int host_copy_up(void *dst, const void *src, size_t bytes) {
   std::lock_guard<std::mutex> lock(g_ring_mutex);
