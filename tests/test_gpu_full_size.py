@@ -358,3 +358,36 @@ def test_config5_vgg_batch64_step_matches_reference_fit(T, W):
             assert rms(eg) <= max(5 * rms(eo), 5e-4), f"{key} parameter {i}.{which}: rms error {rms(eg):.2e}"
             assert np.quantile(eg, 0.99) <= 3e-3 and eg.max() <= 2e-2, f"{key} parameter {i}.{which}"
     net.close()
+
+
+@pytest.mark.parametrize("n, train", [(2 ** 31 - 4, True), (2 ** 31 - 1, False)])
+def test_batchnorm_of_one_channel_just_below_the_largest_tensor(T, n, train):
+    """Positions in a channel count to 2^31 - 1: in 16-byte and in 4-byte steps, to the last element."""
+    block = np.random.default_rng(13).standard_normal(1 << 24).astype(np.float32)
+    x = T.DevBuf((n,))
+    T.DevBuf.view(x.ptr.value, block.shape).upload(block)
+    done = block.size
+    while done < n:
+        m = min(done, n - done)
+        T.copy_d2d(x, x, 4 * m, dst_offset=4 * done)
+        done += m
+    mean, var, std, y = T.to_device(np.full(1, 0.5, np.float32)), T.to_device(np.full(1, 2, np.float32)), T.DevBuf((1,)), T.DevBuf((n,))
+    T.batchnorm_fwd(1, n, 1, x, mean, var, std, y, train=train)
+    m, v = mean.numpy()[0], var.numpy()[0]
+    if train:
+        # One workgroup adds the whole channel, a thread 8 million values one after the other. A thread's
+        # squares come to 2^23, and a float of 2^22 and more counts in halves: an addition rounds by up
+        # to a quarter of a value that is one on average. The values themselves add up to thousands.
+        assert abs(m - block.mean(dtype=np.float64)) < 1e-2 and abs(v - block.var(dtype=np.float64)) < 0.25
+    for first, count in ((0, 5000), (n // 2, 5000), (n - 9000000, 9000000)):
+        at = np.arange(first, first + count) % block.size
+        got = T.DevBuf.view(y.ptr.value + 4 * first, (count,)).numpy()
+        assert_close(got, (block[at].astype(np.float64) - m) / np.sqrt(v + 1e-5), tol=1e-6, what=f"elements from {first}")
+    # backward with dy = y: dx = (dy - mean(dy) - mean(dy*y) y) / std, every element by the same two numbers
+    dx = x
+    T.batchnorm_bwd(1, n, 1, y, y, std, dx)
+    s = std.numpy()[0]
+    head, tail = (T.DevBuf.view(b.ptr.value + 4 * first, (100000,)).numpy().astype(np.float64) for b, first in ((dx, 0), (dx, n - 100000)))
+    yh, yt = (T.DevBuf.view(y.ptr.value + 4 * first, (100000,)).numpy().astype(np.float64) for first in (0, n - 100000))
+    a, b = np.polyfit(yh, head * s, 1)
+    assert np.abs(tail * s - (a * yt + b)).max() < 1e-5

@@ -59,7 +59,8 @@ __device__ __forceinline__ void store_run(float *p, const float (&v)[V]) {
 
 // A workgroup's piece of its channel: elements [beg, end) of the channel's batch*spatial values
 // in steps of V adjacent ones (V = 4 where spatial is a multiple of 4 and the tensors are
-// 16-byte aligned: a step then never leaves its run).
+// 16-byte aligned: a step then never leaves its run). A channel may have just under 2^31 of them, so
+// positions are unsigned: the step behind the last one passes 2^31.
 struct BnGeom {
   int channels, spatial, batch, total;  // total: batch * spatial
   int chunk, groups;                    // pieces of the elementwise passes
@@ -68,8 +69,10 @@ struct BnGeom {
 };
 template <typename F>
 __device__ __forceinline__ void for_piece(const BnGeom &g, const int v, const F &visit) {
-  const int ch = blockIdx.x, beg = blockIdx.y * g.chunk, end = min(g.total, beg + g.chunk);
-  for (int e = beg + v * threadIdx.x; e < end; e += v * NT) {
+  const int ch       = blockIdx.x;
+  const uint32_t beg = blockIdx.y * static_cast<uint32_t>(g.chunk);
+  const uint32_t end = min(static_cast<uint32_t>(g.total), beg + g.chunk);
+  for (uint32_t e = beg + v * threadIdx.x; e < end; e += v * NT) {
     uint32_t img, i;
     g.div_spatial.divmod(e, img, i);
     visit((static_cast<size_t>(img) * g.channels + ch) * g.spatial + i);
@@ -107,8 +110,9 @@ bn_partial_kernel(const float *__restrict__ a, const float *__restrict__ b, cons
   };
   for (int o = blockIdx.y; o < g.batch; o += g.sum_groups) {
     const size_t base = (static_cast<size_t>(o) * g.channels + ch) * g.spatial;
-    int i = threadIdx.x;
-    for (; i + 3 * NT < g.spatial; i += 4 * NT) {
+    const uint32_t spatial = g.spatial;
+    uint32_t i             = threadIdx.x;
+    for (; i + 3 * NT < spatial; i += 4 * NT) {
       float va[4], vb[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
@@ -118,7 +122,7 @@ bn_partial_kernel(const float *__restrict__ a, const float *__restrict__ b, cons
 #pragma unroll
       for (int k = 0; k < 4; ++k) add(va[k], vb[k]);
     }
-    for (; i < g.spatial; i += NT) add(a[base + i], MODE == 2 ? b[base + i] : 0.0f);
+    for (; i < spatial; i += NT) add(a[base + i], MODE == 2 ? b[base + i] : 0.0f);
   }
   s0 = block_sum(s0, smem4);
   if (MODE == 2) s1 = block_sum(s1, smem4);
@@ -209,8 +213,9 @@ int bn_groups(int batch) { return batch < 64 ? batch : 64; }
 BnGeom bn_geom(int channels, int spatial, int batch) {
   BnGeom g;
   g.channels = channels; g.spatial = spatial; g.batch = batch; g.total = batch * spatial;
-  g.chunk       = ceil_div(ceil_div(g.total, std::min(256, std::max(1, 2048 / channels))), 4 * NT) * 4 * NT;
-  g.groups      = ceil_div(g.total, g.chunk);
+  const auto up = [](long a, long b) { return (a + b - 1) / b; };
+  g.chunk       = static_cast<int>(up(up(g.total, std::min(256, std::max(1, 2048 / channels))), 4 * NT) * 4 * NT);
+  g.groups      = static_cast<int>(up(g.total, g.chunk));
   g.sum_groups  = bn_groups(batch);
   g.div_spatial = FastDiv(spatial);
   return g;
