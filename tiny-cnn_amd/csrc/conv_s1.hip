@@ -43,20 +43,23 @@ int launch_split_reduce(const SplitSum &sum, int plane, float *act_out, int act_
 // first_block[k+1]). A launch of its own in every pass whose caller may have written the weights: bound by
 // latency, so nothing is divided and a thread's loads are asked for together. us for 5x5, 32 -> 32 and
 // 32 -> 64 channels, both directions' copies: one thread per weight with scattered stores 5.9.
+// (A single job goes as a kernel of its own, with a tenth of the arguments and no search.)
+struct PackPlan : PackJob {
+  FastDiv div_rs, div_m, div_kc;
+};
 struct PackJobs {
-  PackJob job[CONV_PACK_JOBS];
-  FastDiv div_rs[CONV_PACK_JOBS], div_m[CONV_PACK_JOBS], div_kc[CONV_PACK_JOBS];
+  PackPlan job[CONV_PACK_JOBS];
   int first_block[CONV_PACK_JOBS];   // (past the last job: INT_MAX)
 };
 
 // wp[t][kc][m]: forward (flip = 0): kc = ci, m = co, t as is; dX (flip = 1): kc = co, m = ci,
 // tap reversed. An optional connection table zeroes unconnected (ci, co) pairs. e: element of wp.
-__device__ __forceinline__ void pack_f32(const PackJob &j, const FastDiv &div_m, const FastDiv &div_kc, const int e) {
+__device__ __forceinline__ void pack_f32(const PackPlan &j, const int e) {
   const int rs = j.R * j.S;
   if (e >= j.C * j.Kc * rs) return;
   uint32_t rest, m, t, kc;
-  div_m.divmod(e, rest, m);
-  div_kc.divmod(rest, t, kc);
+  j.div_m.divmod(e, rest, m);
+  j.div_kc.divmod(rest, t, kc);
   const int co = j.flip ? kc : m, ci = j.flip ? m : kc;
   const float v = j.w[(static_cast<size_t>(co) * j.C + ci) * rs + (j.flip ? rs - 1 - t : t)];
   static_cast<float *>(j.wp)[e] = j.tbl && !j.tbl[ci * j.Kc + co] ? 0.0f : v;
@@ -66,12 +69,12 @@ __device__ __forceinline__ void pack_f32(const PackJob &j, const FastDiv &div_m,
 // parts of channels 16g + 8*half .. +7 of row m (zero beyond the tensor), with the sign of step
 // g*rs + t. A thread writes the
 // three units of eight channels.
-__device__ __forceinline__ void pack_x3(const PackJob &j, const FastDiv &div_m, const FastDiv &div_rs, const int e) {
-  const int rs = j.R * j.S, KC = j.flip ? j.Kc : j.C, MC = j.flip ? j.C : j.Kc, mc_pad = div_m.d;
+__device__ __forceinline__ void pack_x3(const PackPlan &j, const int e) {
+  const int rs = j.R * j.S, KC = j.flip ? j.Kc : j.C, MC = j.flip ? j.C : j.Kc, mc_pad = j.div_m.d;
   uint32_t rest, m, g, t;
-  div_m.divmod(e, rest, m);
+  j.div_m.divmod(e, rest, m);
   const int half = rest & 1;
-  div_rs.divmod(rest >> 1, g, t);
+  j.div_rs.divmod(rest >> 1, g, t);
   if (static_cast<int>(g) * 16 >= KC) return;
   const int step = (j.flip ? j.C : 1) * rs, kc0 = 16 * g + 8 * half;   // floats from one channel to the next
   const float *src = j.w + static_cast<size_t>(j.flip ? min(static_cast<int>(m), MC - 1) : min(static_cast<int>(m), MC - 1) * j.C) * rs +
@@ -101,17 +104,19 @@ __device__ __forceinline__ void pack_x3(const PackJob &j, const FastDiv &div_m, 
       make_uint4(part[p][0], part[p][1], part[p][2], part[p][3]);
 }
 
+__device__ __forceinline__ void pack_one(const PackPlan &j, const int e) {
+  if (j.kind == CONV_PACK_X3)
+    pack_x3(j, e);
+  else
+    pack_f32(j, e);
+}
 __global__ void __launch_bounds__(256) pack_filters_kernel(const PackJobs jobs) {
   int k = 0;
 #pragma unroll
   for (int i = 1; i < CONV_PACK_JOBS; ++i) k += jobs.first_block[i] <= static_cast<int>(blockIdx.x) ? 1 : 0;
-  const PackJob &j = jobs.job[k];
-  const int e      = (static_cast<int>(blockIdx.x) - jobs.first_block[k]) * 256 + threadIdx.x;
-  if (j.kind == CONV_PACK_X3)
-    pack_x3(j, jobs.div_m[k], jobs.div_rs[k], e);
-  else
-    pack_f32(j, jobs.div_m[k], jobs.div_kc[k], e);
+  pack_one(jobs.job[k], (static_cast<int>(blockIdx.x) - jobs.first_block[k]) * 256 + threadIdx.x);
 }
+__global__ void __launch_bounds__(256) pack_filter_kernel(const PackPlan j) { pack_one(j, blockIdx.x * 256 + threadIdx.x); }
 
 int pow2_ceil(int v) {
   int p = 1;
@@ -313,17 +318,21 @@ int conv_pack_filters(const PackJob *jobs, int n) {
     for (int k = 0; k < CONV_PACK_JOBS; ++k) {
       p.first_block[k] = k < here ? blocks : INT_MAX;
       if (k >= here) continue;
-      const PackJob &j = p.job[k] = jobs[at + k];
-      const bool x3    = j.kind == CONV_PACK_X3;
+      PackPlan &j = p.job[k];
+      static_cast<PackJob &>(j) = jobs[at + k];
+      const bool x3 = j.kind == CONV_PACK_X3;
       const int rs = j.R * j.S, KC = j.flip ? j.Kc : j.C, MC = j.flip ? j.C : j.Kc;
-      p.div_rs[k] = FastDiv(rs);
-      p.div_m[k]  = FastDiv(x3 ? x3_mc_pad(MC) : MC);
-      p.div_kc[k] = FastDiv(KC);
+      j.div_rs = FastDiv(rs);
+      j.div_m  = FastDiv(x3 ? x3_mc_pad(MC) : MC);
+      j.div_kc = FastDiv(KC);
       blocks += ceil_div(x3 ? ceil_div(KC, 16) * rs * 2 * x3_mc_pad(MC) : rs * KC * MC, 256);
       bytes += (x3 ? 10.0 : 8.0) * rs * KC * MC;
     }
     ProfScope prof("conv_repack_weights", bytes, WORK_BYTE);
-    TDH_LAUNCH(pack_filters_kernel, dim3(blocks), dim3(256), 0, ctx().stream, p);
+    if (here == 1)
+      TDH_LAUNCH(pack_filter_kernel, dim3(blocks), dim3(256), 0, ctx().stream, p.job[0]);
+    else
+      TDH_LAUNCH(pack_filters_kernel, dim3(blocks), dim3(256), 0, ctx().stream, p);
     TDH_LAUNCH_CHECK();
   }
   return TDH_OK;
