@@ -8,7 +8,7 @@ from conftest import assert_close
 pytestmark = pytest.mark.gpu
 
 
-def run(T, cfg, rng, spread=0.0):
+def run(T, cfg, rng, spread=0.0, scale=(0, 0, 0)):
     iw, ih, ic, k, oc, same, bs = cfg
     d = T.conv_desc(iw, ih, ic, k, k, oc, pad_same=same)
     ow, oh = T.conv_out_shape(d)
@@ -17,7 +17,9 @@ def run(T, cfg, rng, spread=0.0):
     dy = rng.standard_normal((bs, oc * oh * ow)).astype(np.float32)
     if spread:
         x *= np.exp(spread * rng.standard_normal(x.shape)).astype(np.float32)
-    b = rng.standard_normal(oc).astype(np.float32)
+    for a, e in zip((x, w, dy), scale):
+        a *= np.float32(2.0 ** e)
+    b = rng.standard_normal(oc).astype(np.float32) * np.float32(2.0 ** (scale[0] + scale[1]))
     xd, wd, dyd, bd = (T.to_device(a) for a in (x, w, dy, b))
     y, dx, dw, db = T.DevBuf(dy.shape), T.DevBuf(x.shape), T.DevBuf(w.shape), T.DevBuf((oc,))
     T.conv2d_fwd(d, bs, xd, wd, bd, y)
@@ -79,12 +81,16 @@ def test_fc_matches_oracle(T, O, W, cfg):
         net.close()
 
 
-@pytest.mark.parametrize("spread", [0.0, 3.0])
-def test_no_further_from_float64_than_fp32_sums(T, spread):
+@pytest.mark.parametrize("spread, scale", [
+    (0.0, (0, 0, 0)), (3.0, (0, 0, 0)),
+    # powers of two of x, w and dy: operands whose lowest bits are far below the smallest normal bf16
+    (0.0, (-116, 0, 0)), (0.0, (0, -116, 0)), (0.0, (0, 0, -116)), (0.0, (-118, 30, 30)), (0.0, (-60, -50, -58)),
+])
+def test_no_further_from_float64_than_fp32_sums(T, spread, scale):
     import torch
     cfg = (64, 64, 32, 3, 64, True, 16)
     iw, ih, ic, k, oc, _, bs = cfg
-    (x, w, b, dy), got = run(T, cfg, np.random.default_rng(4), spread)
+    (x, w, b, dy), got = run(T, cfg, np.random.default_rng(4), spread, scale)
     xt = torch.from_numpy(x).double().reshape(bs, ic, ih, iw).requires_grad_()
     wt = torch.from_numpy(w).double().reshape(oc, ic, k, k).requires_grad_()
     y = torch.nn.functional.conv2d(xt, wt, torch.from_numpy(b).double(), padding=1)
@@ -96,3 +102,22 @@ def test_no_further_from_float64_than_fp32_sums(T, spread):
         # measure 2.2e-7 to 3.0e-7 here)
         assert np.linalg.norm(e) <= 2.0e-7 * np.linalg.norm(r), (name, np.linalg.norm(e) / np.linalg.norm(r))
         assert abs(e.mean()) <= 2e-8 * np.sqrt(np.mean(r * r)), (name, e.mean())
+
+
+@pytest.mark.parametrize("scale", [(-120, 0), (0, -120), (-60, -52)])
+def test_fc_of_tiny_operands(T, W, scale):
+    ni, no, bs = 1024, 1024, 512
+    rng = np.random.default_rng(16)
+    x = rng.standard_normal((bs, ni)).astype(np.float32) * np.float32(2.0 ** scale[0])
+    w = rng.uniform(-0.2, 0.2, ni * no).astype(np.float32) * np.float32(2.0 ** scale[1])
+    net = T.Net(W.build_layers(T, [("fc", ni, no)]), bs, 0)
+    net.set_param(0, 0, w)
+    net.set_param(0, 1, np.zeros(no, np.float32))
+    xd, wd, dx = T.to_device(x), T.to_device(w), T.DevBuf(x.shape)
+    net.forward(bs, xd)
+    T.fc_bwd(ni, no, True, bs, xd, wd, xd, dx, None, None)   # (square: x stands for dy)
+    w64 = w.astype(np.float64).reshape(ni, no)
+    for got, want, name in ((net.layer_out(0, bs), x @ w64, "y"), (dx.numpy(), x @ w64.T, "dx")):
+        # (a sum of 1024 products rounded after each: sqrt(1024) half-ulps, 9.5e-7)
+        assert np.linalg.norm(got - want) <= 5.0e-7 * np.linalg.norm(want), name
+    net.close()

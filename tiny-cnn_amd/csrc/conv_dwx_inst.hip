@@ -126,7 +126,7 @@ __global__ void __launch_bounds__(dwx_threads(RW), dwx_threads(RW) / 256) conv_d
 
   // every other 16-pixel group of dY is staged with its sign turned (split_bf16.h); a thread's
   // words lie in groups of the same parity
-  const float dsign = (tid & 15) >> 2 & 1 ? -1.0f : 1.0f;
+  const float dsign = (tid & 15) >> 2 & 1 ? -X3_SCALE : X3_SCALE;
 
   floatx4 rx[XI], rd[DI];
   auto load4 = [](auto desc, unsigned off, unsigned keep) {
@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(dwx_threads(RW), dwx_threads(RW) / 256) conv_d
       if (xrow[i] < 0) continue;
       int slot = head + xrow[i];
       slot -= slot >= NR ? NR : 0;
-      store4(xl + slot * XROW + xlds[i], NCI * XPX, rx[i]);
+      store4(xl + slot * XROW + xlds[i], NCI * XPX, rx[i] * X3_SCALE);
     }
 #pragma unroll
     for (int i = 0; i < DI; ++i) {

@@ -82,7 +82,7 @@ __device__ __forceinline__ void pack_x3(const PackPlan &j, const int e) {
   float v[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) v[k] = src[static_cast<size_t>(min(kc0 + k, KC - 1)) * step];
-  const float sign = x3_sign(g * rs + t);
+  const float sign = X3_SCALE * x3_sign(g * rs + t);
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     const int kc = kc0 + k, co = j.flip ? kc : m, ci = j.flip ? m : kc;

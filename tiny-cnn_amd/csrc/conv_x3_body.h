@@ -146,7 +146,7 @@ __device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, const int
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           uint32_t p3[X3_PARTS];
-          split_pair(rin[i][2 * c][k], rin[i][2 * c + 1][k], p3);
+          split_pair(X3_SCALE * rin[i][2 * c][k], X3_SCALE * rin[i][2 * c + 1][k], p3);
 #pragma unroll
           for (int p = 0; p < X3_PARTS; ++p) part[p][c] = p3[p];
         }

@@ -437,7 +437,7 @@ __device__ __forceinline__ void opt_part_store(uint16_t *wx, const uint32_t rs, 
   const uint32_t step = (kc >> 4) * rs + tap;
   const size_t pad = x3_mc_pad(mc), unit = step * X3_PARTS;
   uint32_t part[X3_PARTS];
-  split_pair(x3_sign(step) * v, 0.0f, part);
+  split_pair(X3_SCALE * x3_sign(step) * v, 0.0f, part);
 #pragma unroll
   for (int p = 0; p < X3_PARTS; ++p)
     wx[(((unit + p) * 2 + ((kc >> 3) & 1)) * pad + m) * 8 + (kc & 7)] = static_cast<uint16_t>(part[p]);

@@ -79,7 +79,7 @@ struct FxSide {
   // TURN: with the sign turned (the first operand's words carry the sign of their step)
   template <bool TURN>
   __device__ __forceinline__ void stage(uintx4 *lds, int tid) {
-    constexpr float sign = TURN ? -1.0f : 1.0f;
+    constexpr float sign = TURN ? -X3_SCALE : X3_SCALE;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int e = tid + FX_NT * i;

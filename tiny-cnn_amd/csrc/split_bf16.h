@@ -16,8 +16,10 @@
 // and its negative, which is subtracted, so that the biases cancel (without that, a weight gradient
 // over 65536 pixels had a mean error of 5e-7 of its size).
 //
-// Range: bf16 has fp32's exponent range; parts below the smallest denormal (for |x| < 2^-110) are
-// lost, an infinite operand gives NaN where fp32 would give an infinity or NaN.
+// Range, low end: the third part of a float below 2^-110 would lie below bf16's normal numbers. Both
+// operands are split times X3_SCALE, at which every part of every float, denormals included, is a
+// normal bf16, and the addition behind a step's products takes the scale out again (powers of two:
+// not a bit of an ordinary sum changes).
 #pragma once
 #include "common.h"
 
@@ -30,6 +32,8 @@ typedef float floatx16_x3 __attribute__((ext_vector_type(16)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 
 constexpr int X3_PARTS = 3;  // h, m, l
+constexpr float X3_SCALE   = 0x1p24f;   // of both operands when they are split
+constexpr float X3_UNSCALE = 0x1p-48f;  // of a product of the two
 
 // two floats to packed bf16 (round to nearest even), the first in the low half
 __device__ __forceinline__ uint32_t pack_bf16(const float a, const float b) {
@@ -39,7 +43,7 @@ __device__ __forceinline__ uint32_t pack_bf16(const float a, const float b) {
 __device__ __forceinline__ float low_bf16(const uint32_t p) { return __uint_as_float(p << 16); }
 __device__ __forceinline__ float high_bf16(const uint32_t p) { return __uint_as_float(p & 0xffff0000u); }
 
-// the three parts of two floats
+// the three parts of two floats (X3_SCALE times the operands)
 __device__ __forceinline__ void split_pair(const float a, const float b, uint32_t (&part)[X3_PARTS]) {
   part[0]        = pack_bf16(a, b);
   const float ra = a - low_bf16(part[0]), rb = b - high_bf16(part[0]);
@@ -47,8 +51,8 @@ __device__ __forceinline__ void split_pair(const float a, const float b, uint32_
   part[2]        = pack_bf16(ra - low_bf16(part[1]), rb - high_bf16(part[1]));
 }
 
-// acc[i][j] += sign * (a[i] * b[j]) over the 16*KS reduction indices of KS steps, smallest products
-// first; sign is 1 or -1
+// acc[i][j] += sign * (a[i] * b[j]) of the unscaled operands over the 16*KS reduction indices of KS
+// steps, smallest products first; sign is 1 or -1
 template <int TM, int TN, int KS>
 __device__ __forceinline__ void mfma_x3(floatx16_x3 (&acc)[TM][TN], const bf16x8 (&a)[KS][TM][X3_PARTS],
                                         const bf16x8 (&b)[KS][TN][X3_PARTS], const float sign) {
@@ -68,7 +72,7 @@ __device__ __forceinline__ void mfma_x3(floatx16_x3 (&acc)[TM][TN], const bf16x8
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_fmaf(sum[j][r], sign, acc[i][j][r]);
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_fmaf(sum[j][r], sign * X3_UNSCALE, acc[i][j][r]);
       asm volatile("" : "+v"(acc[i][j]));  // (here and now: deferred, the sums pile up in memory)
     }
   }
