@@ -1444,8 +1444,8 @@ int conv2d_fwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
   if (prepacked && prepacked.kind != conv_packed_kind(d, batch, 0))
     return set_error(TDH_ERR_INVALID, "conv2d_fwd: filters packed for another kernel");
   if (prepacked)
-    return conv_s1_run(g.R, g.S, batch, g.C, g.Kc, 0, x, w, nullptr, d->has_bias ? b : nullptr, y, g.H,
-                       g.W, g.OH, g.OW, g.pad_h, g.pad_w, ActGrad(), "conv_fwd_s1", prepacked, act_out,
+    return conv_s1_run(g.R, g.S, batch, g.C, g.Kc, 0, x, w, d->tbl ? tbl_resident : nullptr, d->has_bias ? b : nullptr,
+                       y, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w, ActGrad(), "conv_fwd_s1", prepacked, act_out,
                        act_kind, pool);
   const int ohw = g.OH * g.OW, crs = g.C * g.R * g.S;
   const uint8_t *tbl_dev;
@@ -1591,8 +1591,8 @@ int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
   // (packed for another kernel than the one that runs now: it packs for itself)
   if (prepacked_dx.kind != conv_packed_kind(d, batch, 1)) prepacked_dx = PackedFilters();
   if (dx && prepacked_dx) {
-    TDH_TRY(conv_s1_run(g.R, g.S, batch, g.C, g.Kc, 1, dy, w, nullptr, nullptr, dx, g.OH, g.OW, g.H,
-                        g.W, g.R - 1 - g.pad_h, g.S - 1 - g.pad_w, dx_act, "conv_dx_s1", prepacked_dx));
+    TDH_TRY(conv_s1_run(g.R, g.S, batch, g.C, g.Kc, 1, dy, w, d->tbl ? tbl_resident : nullptr, nullptr, dx, g.OH, g.OW,
+                        g.H, g.W, g.R - 1 - g.pad_h, g.S - 1 - g.pad_w, dx_act, "conv_dx_s1", prepacked_dx));
     dx = nullptr;
     if (!dw && !db) return TDH_OK;
   }

@@ -76,6 +76,7 @@ int conv_bwd_pair_run(int R, int S, int batch, int C, int Kc, int H, int W, int 
   }
   ConvS1Args &a = p.args;
   a.in = dy; a.wp = wp; a.bias = nullptr; a.out = dx; a.ag = dx_act;
+  a.w = w; a.tbl = nullptr; a.flip = 1;
   a.act_out = nullptr; a.act_kind = TDH_ACT_NONE;
   a.pool_out = nullptr; a.pool_argmax = nullptr; a.pool_act_out = nullptr;
   if (p.splits > 1) {

@@ -57,6 +57,37 @@ __device__ __forceinline__ void add_taps(floatx16 *acc, const bf16x8 (&d)[X3_PAR
   if constexpr (S > 1) add_taps<AT + 1, S - 1>(acc + 1, d, w, sign);
 }
 
+// The wave's blocks once more in fp32, if a sum in them is infinite or NaN (split_bf16.h), over the slice's
+// rows and its TC columns: lane l brings output channel co and input channel ci, l%32 of their blocks,
+// at pixel p + l/32.
+template <int S, int TC, int RPS>
+__device__ __forceinline__ void dwx_redo_exceptional(const DwxArgs &a, floatx16 (&acc)[S], const int lane, const int co,
+                                                     const int ci, const int fy, const int x0, const int slice) {
+  if (!x3_exceptional<16 * S>([&](int e) { return acc[e / 16][e % 16]; })) return;
+#pragma unroll
+  for (int fx = 0; fx < S; ++fx) acc[fx] = floatx16{};
+  const int end = min(a.chunks_total, (slice + 1) * a.chunks_per_slice);
+#pragma unroll 1
+  for (int chunk = slice * a.chunks_per_slice; chunk < end; ++chunk) {
+    const int img = chunk / a.chunks_per_image, y0 = RPS * (chunk % a.chunks_per_image);
+    const float *dy = a.dy + (static_cast<size_t>(img) * a.Kc + co) * a.OH * a.OW;
+    const float *x  = a.x + (static_cast<size_t>(img) * a.C + ci) * a.H * a.W;
+#pragma unroll 2
+    for (int p = lane >> 5; p < 64; p += 2) {
+      const int oy = y0 + p / TC, ox = x0 + p % TC, iy = oy + fy - a.ph;
+      const bool on = oy < a.OH && ox < a.OW;
+      const float d = on && co < a.Kc ? dy[oy * a.OW + ox] : 0.0f;
+#pragma unroll
+      for (int fx = 0; fx < S; ++fx) {
+        const int ix  = ox + fx - a.pw;
+        const bool in = on && ci < a.C && static_cast<unsigned>(iy) < static_cast<unsigned>(a.H) &&
+                        static_cast<unsigned>(ix) < static_cast<unsigned>(a.W);
+        acc[fx] = __builtin_amdgcn_mfma_f32_32x32x2f32(d, in ? x[iy * a.W + ix] : 0.0f, acc[fx], 0, 0, 0);
+      }
+    }
+  }
+}
+
 template <int RW, int S, int TC, int COB, int CIB, int SHIFT, bool VEC>
 __global__ void __launch_bounds__(dwx_threads(RW), dwx_threads(RW) / 256) conv_dwx_kernel(const DwxArgs a) {
   constexpr int RPS  = 64 / TC;                     // output rows a step
@@ -266,13 +297,21 @@ __global__ void __launch_bounds__(dwx_threads(RW), dwx_threads(RW) / 256) conv_d
     __syncthreads();
   }
   if (ks == 0 && fy0 + fy < a.R) {
+    if (KS > 1) {
+#pragma unroll
+      for (int fx = 0; fx < S; ++fx)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+#pragma unroll
+          for (int k = 1; k < KS; ++k)
+            acc[fx][r] += red[((((k - 1) * COB * CIB * RW + mine) * S + fx) * 16 + r) * 64 + lane];
+    }
+    dwx_redo_exceptional<S, TC, RPS>(a, acc, lane, co0 + 32 * cob + l32, ci0 + 32 * cib + l32, fy0 + fy, x0, slice);
 #pragma unroll
     for (int fx = 0; fx < S; ++fx)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        float v = acc[fx][r];
-#pragma unroll
-        for (int k = 1; k < KS; ++k) v += red[((((k - 1) * COB * CIB * RW + mine) * S + fx) * 16 + r) * 64 + lane];
+        const float v = acc[fx][r];
         const int co = co0 + 32 * cob + 8 * (r >> 2) + 4 * half + (r & 3), ci = ci0 + 32 * cib + l32;
         if (co < a.Kc && ci < a.C) out[static_cast<size_t>(co) * crs + ci * a.RS + (fy0 + fy) * S + fx] = v;
       }

@@ -38,6 +38,11 @@ __host__ __device__ constexpr float x3_sign(int u) { return u & 1 ? -1.0f : 1.0f
 struct ConvS1Args {
   const float *in;
   const void *wp;              // filters: floats [tap][kc][m], or the parts of conv_x3_inst.hip
+  // what wp was packed from, for sums that the three-part kernel computes again: OIHW filters, the
+  // connection table they are masked by (or null), and whether this is dX (taps reversed)
+  const float *w;
+  const uint8_t *tbl;
+  int flip;
   const float *bias;
   float *out;
   ActGrad ag;

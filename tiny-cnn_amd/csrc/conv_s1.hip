@@ -339,9 +339,9 @@ int conv_pack_filters(const PackJob *jobs, int n) {
 }
 
 // Runs out = conv(in, repack(w)) (+ bias) (* act'(y)); the caller has checked applicability
-// and reserved conv_s1_workspace_bytes of scratch. flip = 0: forward, 1: dX. prepacked: the
-// result of conv_pack_filters for this filter, when the caller already has it in the layout of the
-// kernel that runs (w is not read then).
+// and reserved conv_s1_workspace_bytes of scratch. flip = 0: forward, 1: dX. w: the filters, masked by
+// tbl_dev unless null. prepacked: the result of conv_pack_filters for them, when the caller already
+// has it in the layout of the kernel that runs.
 int conv_s1_run(int R, int S, int batch, int C, int Kc, int flip, const float *in, const float *w,
                 const uint8_t *tbl_dev, const float *bias, float *out, int IH, int IW, int OH,
                 int OW, int ph, int pw, ActGrad ag, const char *tag, PackedFilters prepacked,
@@ -364,6 +364,7 @@ int conv_s1_run(int R, int S, int batch, int C, int Kc, int flip, const float *i
     wp = fresh;
   }
   p.args.in = in; p.args.wp = wp; p.args.bias = bias;
+  p.args.w = w; p.args.tbl = tbl_dev; p.args.flip = flip;
   p.args.out = out; p.args.ag = ag;
   p.args.act_out = act_out; p.args.act_kind = act_kind;
   p.args.pool_out     = pool ? pool->out : nullptr;

@@ -25,6 +25,54 @@ typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 
 constexpr unsigned X3_NOWHERE = 0x80000000u;  // past the end of every tile's images
 
+// The wave's blocks once more in fp32, if a sum in them is infinite or NaN (split_bf16.h): lane l brings
+// channel l%32 of a filter block and pixel l%32 of a pixel block, for the reduction channel kc + l/32.
+template <int R, int S, int TC, int TM, int TN>
+__device__ __forceinline__ void x3_redo_exceptional(const ConvS1Args &a, floatx16 (&acc)[TM][TN], const int wn,
+                                                    const int lane, const int img0, const int y0, const int x0,
+                                                    const int m0, const int kc_lo, const int kc_hi) {
+  constexpr int LOG_TC = TC == 64 ? 6 : TC == 32 ? 5 : TC == 16 ? 4 : 3;
+  if (!x3_exceptional<16 * TM * TN>([&](int e) { return acc[e / (16 * TN)][e / 16 % TN][e % 16]; })) return;
+  int img[TN], iy[TN], ix[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int q = (wn * TN + j) * 32 + (lane & 31);
+    img[j] = img0 + (q >> (a.log_tr + LOG_TC));
+    iy[j]  = y0 + ((q >> LOG_TC) & (a.TR - 1)) - a.ph;
+    ix[j]  = x0 + (q & (TC - 1)) - a.pw;
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = floatx16{};
+#pragma unroll 1
+  for (int kc0 = kc_lo; kc0 < kc_hi; kc0 += 2) {
+    const int kc = kc0 + (lane >> 5);
+#pragma unroll 1
+    for (int fy = 0; fy < R; ++fy)
+#pragma unroll
+      for (int fx = 0; fx < S; ++fx) {
+        float w[TM], x[TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const int m = m0 + 32 * i + (lane & 31), t = fy * S + fx;
+          const bool on = kc < kc_hi && m < a.MC && (!a.tbl || a.tbl[a.flip ? m * a.KC + kc : kc * a.MC + m]);
+          w[i] = on ? a.w[static_cast<size_t>(a.flip ? kc * a.MC + m : m * a.KC + kc) * (R * S) + (a.flip ? R * S - 1 - t : t)] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const bool in = kc < kc_hi && img[j] < a.batch && static_cast<unsigned>(iy[j] + fy) < static_cast<unsigned>(a.IH) &&
+                          static_cast<unsigned>(ix[j] + fx) < static_cast<unsigned>(a.IW);
+          x[j] = in ? a.in[((static_cast<size_t>(img[j]) * a.KC + kc) * a.IH + iy[j] + fy) * a.IW + ix[j] + fx] : 0.0f;
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[i], x[j], acc[i][j], 0, 0, 0);
+      }
+  }
+}
+
 // the workgroup at (bx, by, bz) of the grid. BY_TAPS: the four waves share the
 // workgroup's 32 channels x 128 pixels (TM = TN = 1) by filter taps instead of by pixels
 template <int R, int S, int TC, int TM, int TN, bool VEC, bool BY_TAPS>
@@ -221,6 +269,7 @@ __device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, const int
 #pragma unroll
       for (int k = 0; k < 4; ++k) sum[0][0][4 * r + k] = v[k];
     }
+    x3_redo_exceptional<R, S, TC, 1, 1>(a, sum, wn, lane, img0, y0, x0, m0, kc_lo, kc_hi);
     s1_epilogue<TC, 1, 1>(a, sum, wn, lane, img0, y0, x0, m0, bz);
     return;
   } else {
@@ -274,6 +323,7 @@ __device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, const int
         for (int p = 0; p < X3_PARTS; ++p) wf[0][i][p] = wf[1][i][p];
     }
   }
+  x3_redo_exceptional<R, S, TC, TM, TN>(a, acc, wn, lane, img0, y0, x0, m0, kc_lo, kc_hi);
   s1_epilogue<TC, TM, TN>(a, acc, wn, lane, img0, y0, x0, m0, bz);
   }
 }

@@ -179,6 +179,30 @@ fc_x3_kernel(const float *__restrict__ A, const float *__restrict__ B, const int
     if (k0 + FX_BK < kend) step(k0 + FX_BK, std::integral_constant<int, 1>());
   }
 
+  // the wave's blocks once more in fp32, if a sum in them is infinite or NaN (split_bf16.h): lane l
+  // brings row and column l%32 of the blocks at index k + l/32
+  if (x3_exceptional<64>([&](int e) { return acc[e / 32][e / 16 % 2][e % 16]; })) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] = floatx16{};
+#pragma unroll 2
+    for (int k = kbeg; k < kend; k += 2) {
+      const bool on = k + half < kend;
+      float av[2], bv[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int m = m0 + 64 * wm + 32 * i + l32, n = n0 + 64 * wn + 32 * i + l32;
+        av[i] = on && m < M ? A[static_cast<size_t>(m) * lda + k + half] : 0.0f;
+        bv[i] = on && n < N ? B[B_KC ? static_cast<size_t>(n) * ldb + k + half : static_cast<size_t>(k + half) * ldb + n] : 0.0f;
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+    }
+  }
+
   // D[i][j] of a block: reg r of lane l at row 8*(r/4) + 4*(l/32) + r%4, column l%32
 #pragma unroll
   for (int j = 0; j < 2; ++j) {

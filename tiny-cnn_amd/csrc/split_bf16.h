@@ -20,6 +20,12 @@
 // operands are split times X3_SCALE, at which every part of every float, denormals included, is a
 // normal bf16, and the addition behind a step's products takes the scale out again (powers of two:
 // not a bit of an ordinary sum changes).
+// High end: an operand that is infinite, NaN or above 2^104, and a sum above 2^80, leaves an infinity or
+// NaN in every sum that it is part of, where fp32 would give one, or a number. Each wave looks at its
+// finished sums, and where one is infinite or NaN (x3_exceptional) it computes its whole tile again with
+// v_mfma_f32_32x32x2_f32, operands straight from memory. Finite sums pay one multiplication each for
+// the look. us with every input NaN, against ordinary inputs: convolution 32 -> 64 of 64x64, batch 64,
+// forward and backward 918 / 227; 4096 x 4096 fully-connected layer, batch 256 556 / 343.
 #pragma once
 #include "common.h"
 
@@ -82,6 +88,15 @@ __device__ __forceinline__ void mfma_x3(floatx16_x3 (&acc)[TM][TN], const bf16x8
                                         const bf16x8 (&b)[TN][X3_PARTS], const float sign) {
   mfma_x3<TM, TN, 1>(acc, reinterpret_cast<const bf16x8(&)[1][TM][X3_PARTS]>(a),
                      reinterpret_cast<const bf16x8(&)[1][TN][X3_PARTS]>(b), sign);
+}
+
+// whether any lane of the wave has an infinite or NaN element: 0 * infinity and 0 * NaN are NaN
+template <int N, class Get>
+__device__ __forceinline__ bool x3_exceptional(const Get &element) {
+  float probe = 0.0f;
+#pragma unroll
+  for (int e = 0; e < N; ++e) probe = __builtin_fmaf(element(e), 0.0f, probe);
+  return __builtin_expect(__any(!(probe == 0.0f)) != 0, 0);
 }
 
 }  // namespace
