@@ -24,9 +24,9 @@ def check(got, want, what):
 
 
 def plant(a, rng, rows):
-    """Exceptional values in as many rows of a."""
+    """Exceptional values in as many rows of a (the largest one times an ordinary value does not overflow)."""
     flat = a.reshape(-1, a.shape[-1])
-    for row, v in zip(rng.choice(len(flat), rows, replace=False), [np.inf, -np.inf, np.nan, 3.2e38, -2.5e32, 1e-41]):
+    for row, v in zip(rng.choice(len(flat), rows, replace=False), [np.inf, -np.inf, np.nan, 3e37, -2.5e32, 1e-41]):
         flat[row, rng.integers(a.shape[-1])] = v
 
 
@@ -65,8 +65,15 @@ THREE_PART = [
 ]
 
 
+FEW_TILES = [
+    (12, 12, 5, 5, 9, True, 1),         # 225 and 125 indices: a last block of one and of thirteen
+    (9, 7, 3, 3, 16, False, 1),         # 35 output pixels
+    (10, 9, 24, 3, 8, True, 3),
+]
+
+
 @pytest.mark.parametrize("where", ["x", "w", "dy"])
-@pytest.mark.parametrize("cfg", THREE_PART)
+@pytest.mark.parametrize("cfg", THREE_PART + FEW_TILES)
 def test_convolution(T, cfg, where):
     iw, ih, ic, k, oc, same, bs = cfg
     rng = np.random.default_rng(31)
@@ -84,6 +91,25 @@ def test_convolution(T, cfg, where):
     want = conv64(x, w, b, dy, *((k // 2, k // 2) if same else (0, 0)))
     for g, r, name in zip(out, want, ("y", "dx", "dw", "db")):
         check(g.numpy(), r, f"{cfg} {name}")
+
+
+def test_ends_of_short_reductions(T):
+    """The kernels for a few tiles fill the last block of 16 indices with the first weight and the last pixel, times
+    zero: an infinity there reaches the sums that it is a part of, as an infinity."""
+    iw, ih, ic, k, oc, bs = 9, 7, 5, 3, 9, 1
+    rng = np.random.default_rng(34)
+    d = T.conv_desc(iw, ih, ic, k, k, oc, pad_same=True)
+    x = rng.uniform(0.5, 1, (bs, ic, ih, iw)).astype(np.float32)
+    w = rng.uniform(0.5, 1, (oc, ic, k, k)).astype(np.float32)
+    dy = rng.uniform(0.5, 1, (bs, oc, ih, iw)).astype(np.float32)
+    b = np.zeros(oc, np.float32)
+    w[0, 0, 0, 0] = x[-1, 2, -1, -1] = np.inf
+    out = [T.DevBuf((n,)) for n in (dy.size, x.size, w.size, oc)]
+    xd, wd, dyd = (T.to_device(a.ravel()) for a in (x, w, dy))
+    T.conv2d_fwd(d, bs, xd, wd, T.to_device(b), out[0])
+    T.conv2d_bwd(d, bs, xd, wd, dyd, *out[1:])
+    for g, r, name in zip(out, conv64(x, w, b, dy, 1, 1), ("y", "dx", "dw", "db")):
+        check(g.numpy(), r, name)
 
 
 @pytest.mark.parametrize("where", ["x", "w"])

@@ -112,7 +112,7 @@ __device__ __forceinline__ void direct_dx(const BwdDirectArgs &a, int4 *tab, flo
           const int4 e  = tab[16 * (b0 + WAVES * i) + 4 * g + j];
           const bool in = (rows >> (e.y & 31) & cols >> (e.y >> 8)) & 1u;
           const float v = dyp[in ? at + e.x : 0];
-          wv[i][j]      = wr[e.z];
+          wv[i][j]      = e.y == 31 ? 0.0f : wr[e.z];   // (past the end: 0 times an infinite weight is NaN)
           yv[i][j]      = in ? v : 0.0f;
         }
       }
@@ -180,7 +180,7 @@ __device__ __forceinline__ void direct_dw(const BwdDirectArgs &a, float *red, co
             av[i][j]      = p + j < a.pixels ? v : 0.0f;
           }
           const int iy  = static_cast<int>(oy) * a.sh + y0, ix = static_cast<int>(ox + (QUAD ? j : 0)) * a.sw + x0;
-          const bool in = inner && static_cast<unsigned>(iy) < static_cast<unsigned>(a.H) &&
+          const bool in = inner && p + j < a.pixels && static_cast<unsigned>(iy) < static_cast<unsigned>(a.H) &&
                           static_cast<unsigned>(ix) < static_cast<unsigned>(a.W);
           const float v = xc[in ? static_cast<size_t>(img) * a.C * hw + iy * a.W + ix : 0];
           bv[i][j]      = in ? v : rim;
