@@ -56,10 +56,10 @@ THREE_PART = [
     # in_w, in_h, in_c, k, out_c, same, batch
     (64, 12, 16, 3, 64, True, 86),      # tiles of 64 columns, one chunk of channels
     (66, 17, 33, 3, 65, True, 26),      # scalar loads, channels past a chunk and a tile
-    (30, 30, 64, 3, 40, False, 20),     # no padding
-    (15, 33, 48, 3, 96, True, 33),      # tiles of 16 columns
-    (53, 50, 20, 5, 40, True, 7),       # 5x5: dW in groups of filter rows
-    (40, 40, 50, 1, 70, True, 12),      # 1x1
+    (30, 30, 64, 3, 40, False, 70),     # no padding
+    (15, 33, 48, 3, 96, True, 90),      # tiles of 16 columns
+    (53, 50, 20, 5, 40, True, 20),      # 5x5: dW in groups of filter rows
+    (40, 40, 50, 1, 70, True, 26),      # 1x1
     (16, 16, 32, 5, 32, True, 21),      # dX shared by filter taps, in the launch with dW
     (8, 8, 32, 5, 64, True, 37),
 ]
@@ -86,8 +86,11 @@ def test_convolution(T, cfg, where):
     plant({"x": x, "w": w, "dy": dy}[where], rng, 6)
     out = [T.DevBuf((n,)) for n in (dy.size, x.size, w.size, oc)]
     xd, wd, dyd = (T.to_device(a.ravel()) for a in (x, w, dy))
+    T.profile_begin()
     T.conv2d_fwd(d, bs, xd, wd, T.to_device(b), out[0])
     T.conv2d_bwd(d, bs, xd, wd, dyd, *out[1:])
+    tags = {e["tag"].split()[0] for e in T.profile_end()}
+    assert tags & {"conv_bwd_pair", "conv_bwd_direct"} or cfg in THREE_PART and {"conv_fwd_x3", "conv_dx_x3"} <= tags, tags
     want = conv64(x, w, b, dy, *((k // 2, k // 2) if same else (0, 0)))
     for g, r, name in zip(out, want, ("y", "dx", "dw", "db")):
         check(g.numpy(), r, f"{cfg} {name}")
@@ -127,8 +130,10 @@ def test_fully_connected(T, W, dims, where):
     net.set_param(0, 0, w)
     net.set_param(0, 1, np.zeros(no, np.float32))
     xd, dx = T.to_device(x), T.DevBuf(x.shape)
+    T.profile_begin()
     net.forward(bs, xd)
     T.fc_bwd(ni, no, True, bs, xd, T.to_device(w.ravel()), T.to_device(dy), dx, None, None)
+    assert {"fc_fwd_x3", "fc_dx_x3"} <= {e["tag"].split()[0] for e in T.profile_end()}
     with np.errstate(invalid="ignore", over="ignore"):
         check(net.layer_out(0, bs), x.astype(np.float64) @ w.astype(np.float64), f"{dims} y")
         check(dx.numpy(), dy.astype(np.float64) @ w.astype(np.float64).T, f"{dims} dx")
@@ -150,7 +155,9 @@ def test_packed_filters_behind_a_connection_table(T, W):
     net.set_param(0, 1, b)
     x = rng.standard_normal((bs, ic, size, size)).astype(np.float32)
     plant(x, rng, 4)
+    T.profile_begin()
     net.forward(bs, T.to_device(x.reshape(bs, -1)))
+    assert any(e["tag"].startswith("conv_fwd_x3") for e in T.profile_end())
     w[~on] = 0
     dy = np.zeros((bs, oc, size, size), np.float32)
     check(net.layer_out(0, bs), conv64(x, w, b, dy, 1, 1)[0], "y")

@@ -52,6 +52,30 @@ def test_matches_oracle(T, O, cfg):
 
 
 @pytest.mark.parametrize("cfg", [
+    # (of the list above, the ones that have too few tiles there for the three-part kernels in both directions)
+    (50, 11, 40, 3, 24, False, 130),
+    (30, 30, 64, 3, 40, False, 70),
+    (53, 50, 20, 5, 40, True, 20),
+    (49, 50, 34, 5, 33, False, 24),
+    (40, 40, 50, 1, 70, True, 26),
+    (36, 30, 20, 7, 40, True, 33),
+])
+def test_every_window_against_float64(T, cfg):
+    import torch
+    iw, ih, ic, k, oc, same, bs = cfg
+    T.profile_begin()
+    (x, w, b, dy), got = run(T, cfg, np.random.default_rng(3))
+    tags = {e["tag"].split()[0] for e in T.profile_end()}
+    assert {"conv_fwd_x3", "conv_dx_x3"} <= tags, tags
+    xt = torch.from_numpy(x).double().reshape(bs, ic, ih, iw).requires_grad_()
+    wt = torch.from_numpy(w).double().reshape(oc, ic, k, k).requires_grad_()
+    y = torch.nn.functional.conv2d(xt, wt, torch.from_numpy(b).double(), padding=k // 2 if same else 0)
+    y.backward(torch.from_numpy(dy).double().reshape(y.shape))
+    for g, r, name in zip(got, (y, xt.grad, wt.grad), ("y", "dx", "dw")):
+        assert_close(g.ravel(), r.detach().numpy().ravel(), what=f"{cfg} {name}")
+
+
+@pytest.mark.parametrize("cfg", [
     # in, out, batch
     (4096, 1024, 64),      # tiles of 64 rows
     (1028, 1012, 260),     # ragged on every side, a last step of four indices

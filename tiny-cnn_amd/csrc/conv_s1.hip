@@ -376,7 +376,8 @@ int conv_s1_run(int R, int S, int batch, int C, int Kc, int flip, const float *i
     p.args.part = static_cast<float *>(part);
   }
   {
-    ProfScope prof(pool ? "conv_fwd_s1_pool" : tag, MC, batch * OH * OW, KC * R * S);
+    const char *name = !p.x3 ? (pool ? "conv_fwd_s1_pool" : tag) : pool ? "conv_fwd_x3_pool" : flip ? "conv_dx_x3" : "conv_fwd_x3";
+    ProfScope prof(name, MC, batch * OH * OW, KC * R * S);
     const bool vec = IW % 4 == 0 && aligned16(in) && (p.x3 || (MC % 4 == 0 && aligned16(wp)));
     if (p.x3 && vec)
       TDH_TRY(R == 1 ? x3_launch_1_vec(p) : R == 3 ? x3_launch_3_vec(p) : R == 5 ? x3_launch_5_vec(p) : x3_launch_7_vec(p));

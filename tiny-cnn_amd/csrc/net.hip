@@ -232,7 +232,11 @@ bool tiny_step_applies(const tdh_net *net, int loss_kind);
 // queued in time for 1 (the CIFAR-10-shape net, us a step replayed / launched: batch 16 115 / 114, 32 128 /
 // 123, 64 134 / 129, 128 164 / 158, 512 516 / 507), and a step on tensors that it has not seen, or
 // of another batch, starts without a capture. A layer comes to about two launches of 4 us; from
-// 5e7 FLOP a layer on its kernels take more.
+// 5e7 FLOP a layer on its kernels take more. Other nets beyond that line, none of which is slower
+// launched: the VGG-style stack on 32x32 images, batch 32 380 / 375, on 64x64, batch 4 337 / 332, batch 16 587 /
+// 587; six 3x3 layers of 32 channels of 24x24, batch 128 513 / 509; three 5x5 layers of 48 channels of 12x12,
+// batch 64 241 / 241, batch 256 628 / 623; 784-1000-1000-10 fully connected, batch 1024 273 / 268; 1024-4096-4096-10,
+// batch 64 286 / 281. Below it the two are within 1 % of each other, and a replay leaves the host free.
 bool step_outlasts_launches(const tdh_net *net, int loss_kind, int batch) {
   return !tiny_step_applies(net, loss_kind) && !net_forks(net, batch) &&
          net_forward_flop(net, batch) >= 5e7 * static_cast<double>(net->layers.size());
