@@ -81,10 +81,6 @@ def test_every_window_against_float64(T, cfg):
     (1028, 1012, 260),     # ragged on every side, a last step of four indices
     (2048, 64, 512),       # tiles of 64 columns
     (16384, 68, 132),      # a reduction of two steps and four indices
-    # (of the first three, forward and dX are left to other kernels: too few tiles)
-    (8192, 2048, 64),      # tiles of 64 rows
-    (1028, 1012, 520),     # ragged on every side
-    (4096, 64, 2048),      # tiles of 64 columns, dX with the shortest reduction
 ])
 def test_fc_matches_oracle(T, O, W, cfg):
     """dX as an operator, the forward product as a net's inference."""
@@ -149,33 +145,3 @@ def test_fc_of_tiny_operands(T, W, scale):
         # (a sum of 1024 products rounded after each: sqrt(1024) half-ulps, 9.5e-7)
         assert np.linalg.norm(got - want) <= 5.0e-7 * np.linalg.norm(want), name
     net.close()
-
-
-@pytest.mark.parametrize("dims", [(4096, 1024, 256), (512, 512, 32), (1024, 1024, 512), (300, 40, 200)])
-def test_operator_and_inference_are_one_product(T, W, dims):
-    ni, no, bs = dims
-    rng = np.random.default_rng(17)
-    x = rng.standard_normal((bs, ni)).astype(np.float32)
-    w = rng.uniform(-0.2, 0.2, ni * no).astype(np.float32)
-    b = rng.standard_normal(no).astype(np.float32)
-    net = T.Net(W.build_layers(T, [("fc", ni, no)]), bs, 0)
-    net.set_param(0, 0, w)
-    net.set_param(0, 1, b)
-    xd, y = T.to_device(x), T.DevBuf((bs, no))
-    net.forward(bs, xd)
-    T.fc_fwd(ni, no, True, bs, xd, T.to_device(w), T.to_device(b), y)
-    assert np.array_equal(y.numpy(), net.layer_out(0, bs))
-    net.close()
-    size, ic, oc, k, cb = 24, 20, 40, 3, max(1, bs // 8)
-    d = T.conv_desc(size, size, ic, k, k, oc, pad_same=True)
-    x = rng.standard_normal((cb, ic * size * size)).astype(np.float32)
-    w, b = rng.uniform(-0.2, 0.2, oc * ic * k * k).astype(np.float32), rng.standard_normal(oc).astype(np.float32)
-    xd, y = T.to_device(x), T.DevBuf((cb, oc * size * size))
-    T.conv2d_fwd(d, cb, xd, T.to_device(w), T.to_device(b), y)
-    for flags in (0, T.NET_GRAPH):
-        net = T.Net(W.build_layers(T, [("conv", size, size, ic, k, oc, True)]), cb, flags)
-        net.set_param(0, 0, w)
-        net.set_param(0, 1, b)
-        net.forward(cb, xd)
-        assert np.array_equal(y.numpy(), net.layer_out(0, cb))
-        net.close()

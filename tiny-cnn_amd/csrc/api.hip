@@ -590,6 +590,7 @@ int tdh_fc_fwd(int in, int out, int has_bias, int batch, const float *x, const f
                   static_cast<long>(batch) * out < (1L << 31),
                 "tdh_fc_fwd: tensor exceeds 2^31 elements");
   TDH_TRY(ws_begin(fc_workspace_bytes(in, out, batch)));
+  const KeepF32 keep(true);
   return fc_fwd(in, out, has_bias, batch, x, w, b, y);
 }
 

@@ -35,21 +35,18 @@ struct Context {
   // leave_split_sum: the caller of a convolution asks it to leave a split reduction to the
   // kernel that reads the result next; split_sum_left: one was left (left_split_sum())
   bool leave_split_sum = false, split_sum_left = false;
-  // Products keep to the fp32 matrix instructions, and to one order of their sums, while this is set:
-  // in the forward pass of a net's train step, and in the whole step of a net with batch normalization.
-  // Everything else, inference and the operators called one by one, takes whatever kernel is fastest.
-  // The three-part products of split_bf16.h and the kernels for a few tiles are no less precise, but
-  // they round differently, and there are two places where a train step turns roundings into something
-  // larger, so that a training run would take another course than it always has:
+  // Products keep to the fp32 matrix instructions while this is set. The three-part products of
+  // split_bf16.h are no less precise, but they round differently, and there are two places where a
+  // train step turns roundings into something larger, so that a training run would take another
+  // course than it always has:
   //  - its forward pass decides signs (relu) and maxima (max-pool), and with them where whole
   //    gradients go: one choice in a million changes, and the input gradient of the VGG-style
   //    stack by 1.6e-3 with it;
+  //    (A fully-connected product called as an operator may be the forward half of such a step: every
+  //    bias gradient hangs on its last bits through the activation behind it, and Adam makes a full
+  //    step of one that is nearly zero.)
   //  - the bias gradient of a convolution in front of a batch normalization is zero but for its
   //    rounding, and an optimizer that divides by the gradient's size makes full steps of that.
-  // A caller who builds a train step out of operators calls for each product by itself, and gets each
-  // as near to the exact one as it comes: 4096 x 4096 behind tanh, batch 256, relative distance from
-  // float64 with this set / not set: y 4.1e-7 / 1.0e-7, dx 2.0e-7 / 1.2e-7, dw 3.3e-7 / 2.9e-7, the weights
-  // after an Adam step 9.1e-7 / 6.5e-7; layers of 25 to 4377 inputs y 0.8-2.8e-7 / 0.7-2.8e-7.
   bool keep_f32 = false;
   // two more streams (default priority) for work that branches off the main one inside a
   // captured train step; created on first use
@@ -64,7 +61,8 @@ struct StreamSwap {
 };
 
 Context &ctx();
-// Products inside the scope keep to fp32 (see Context::keep_f32).
+// Products inside the scope keep to fp32 instructions and to one order of their sums whatever the
+// batch's size (see Context::keep_f32).
 struct KeepF32 {
   const bool was;
   explicit KeepF32(bool on) : was(ctx().keep_f32) { ctx().keep_f32 = was || on; }

@@ -5,7 +5,8 @@
 //   forward  y[b][o]  = x[b][i] W[i][o]     A rows along k, B rows along n
 //   dX       dx[b][i] = dy[b][o] W[i][o]    both along k
 //
-// (Not the forward product of a train step, see Context::keep_f32.)
+// (Inference and dX only: the bias gradients of a train step hang on the last bits of its forward
+// product and of its weights, and Adam makes a full step of one that is nearly zero.)
 //
 // A workgroup of four wave64 owns 64*WM x 64*WN elements, a wave 64 x 64 of them (four accumulator
 // blocks). Per step of 32 reduction indices the tile's 16-byte words are loaded while the step
