@@ -57,35 +57,89 @@ __device__ __forceinline__ void add_taps(floatx16 *acc, const bf16x8 (&d)[X3_PAR
   if constexpr (S > 1) add_taps<AT + 1, S - 1>(acc + 1, d, w, sign);
 }
 
-// The wave's blocks once more in fp32, if a sum in them is infinite or NaN (split_bf16.h), over the slice's
-// rows and its TC columns: lane l brings output channel co and input channel ci, l%32 of their blocks,
-// at pixel p + l/32.
+// The wave's infinite and NaN sums once more in fp32 (split_bf16.h), over the slice's rows and its TC
+// columns: lane l brings output channel co and input channel ci, l%32 of their blocks, at pixel
+// p + l/32. Eight pixels are asked for together.
 template <int S, int TC, int RPS>
 __device__ __forceinline__ void dwx_redo_exceptional(const DwxArgs &a, floatx16 (&acc)[S], const int lane, const int co,
                                                      const int ci, const int fy, const int x0, const int slice) {
-  if (!x3_exceptional<16 * S>([&](int e) { return acc[e / 16][e % 16]; })) return;
-#pragma unroll
-  for (int fx = 0; fx < S; ++fx) acc[fx] = floatx16{};
-  const int end = min(a.chunks_total, (slice + 1) * a.chunks_per_slice);
+  // (hidden from the compiler, which otherwise keeps the comparisons for the stores behind)
+  int rows = a.Kc - (co - (lane & 31)) - 4 * (lane >> 5);   // from this lane's first element
+  asm volatile("" : "+v"(rows));
+  x3_redo(acc, [&](int, int r) { return ci < a.C && 8 * (r >> 2) + (r & 3) < rows; }, [&](floatx16 (&sum)[S]) {
+    const int end = min(a.chunks_total, (slice + 1) * a.chunks_per_slice);
 #pragma unroll 1
-  for (int chunk = slice * a.chunks_per_slice; chunk < end; ++chunk) {
-    const int img = chunk / a.chunks_per_image, y0 = RPS * (chunk % a.chunks_per_image);
-    const float *dy = a.dy + (static_cast<size_t>(img) * a.Kc + co) * a.OH * a.OW;
-    const float *x  = a.x + (static_cast<size_t>(img) * a.C + ci) * a.H * a.W;
-#pragma unroll 2
-    for (int p = lane >> 5; p < 64; p += 2) {
-      const int oy = y0 + p / TC, ox = x0 + p % TC, iy = oy + fy - a.ph;
-      const bool on = oy < a.OH && ox < a.OW;
-      const float d = on && co < a.Kc ? dy[oy * a.OW + ox] : 0.0f;
+    for (int chunk = slice * a.chunks_per_slice; chunk < end; ++chunk) {
+      const int img = chunk / a.chunks_per_image, y0 = RPS * (chunk % a.chunks_per_image);
+      const float *dy = a.dy + (static_cast<size_t>(img) * a.Kc + (co < a.Kc ? co : 0)) * a.OH * a.OW;
+      const float *x  = a.x + (static_cast<size_t>(img) * a.C + (ci < a.C ? ci : 0)) * a.H * a.W;
+#pragma unroll 1
+      for (int p0 = lane >> 5; p0 < 64; p0 += 8) {
+        float d[4], v[4][S];
 #pragma unroll
-      for (int fx = 0; fx < S; ++fx) {
-        const int ix  = ox + fx - a.pw;
-        const bool in = on && ci < a.C && static_cast<unsigned>(iy) < static_cast<unsigned>(a.H) &&
-                        static_cast<unsigned>(ix) < static_cast<unsigned>(a.W);
-        acc[fx] = __builtin_amdgcn_mfma_f32_32x32x2f32(d, in ? x[iy * a.W + ix] : 0.0f, acc[fx], 0, 0, 0);
+        for (int k = 0; k < 4; ++k) {
+          const int p = p0 + 2 * k, oy = y0 + p / TC, ox = x0 + p % TC, iy = oy + fy - a.ph;
+          const bool on = oy < a.OH && ox < a.OW;
+          d[k] = on && co < a.Kc ? dy[oy * a.OW + ox] : 0.0f;
+#pragma unroll
+          for (int fx = 0; fx < S; ++fx) {
+            const int ix  = ox + fx - a.pw;
+            const bool in = on && ci < a.C && static_cast<unsigned>(iy) < static_cast<unsigned>(a.H) &&
+                            static_cast<unsigned>(ix) < static_cast<unsigned>(a.W);
+            v[k][fx] = in ? x[iy * a.W + ix] : 0.0f;
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int fx = 0; fx < S; ++fx) sum[fx] = __builtin_amdgcn_mfma_f32_32x32x2f32(d[k], v[k][fx], sum[fx], 0, 0, 0);
+      }
+      if (x3_all_nan(sum)) return;
+      if (chunk == slice * a.chunks_per_slice) {
+        // A NaN anywhere in dY's channel makes NaN of all of that channel's sums: the channels that still
+        // have a number are looked through, a step of 64 pixels to a load, as far as an image goes (a
+        // few channels with a NaN here and there would take the loop around this one through all
+        // of it: 64 images of 64x64, 128 -> 128 channels, 970 us, so 358).
+        uint32_t need = 0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          bool number = false;
+#pragma unroll
+          for (int fx = 0; fx < S; ++fx) number = number || sum[fx][r] == sum[fx][r];
+          const uint64_t lanes = __ballot(number);
+          const int row        = 8 * (r >> 2) + (r & 3);   // of lanes 0-31; lanes 32-63 hold row + 4
+          need |= (static_cast<uint32_t>(lanes) != 0 ? 1u : 0u) << row | ((lanes >> 32) != 0 ? 1u : 0u) << (row + 4);
+        }
+        uint32_t nan_rows = 0;
+        while (need) {
+          const int row = __builtin_ctz(need), channel = co - (lane & 31) + row;
+          need &= need - 1;
+          for (int c0 = chunk; c0 < min(end, chunk + a.chunks_per_image); c0 += 8) {
+            bool nan = false;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+              const int c = min(c0 + k, end - 1), i = c / a.chunks_per_image;
+              const int oy = RPS * (c - i * a.chunks_per_image) + lane / TC, ox = x0 + lane % TC;
+              const float d = oy < a.OH && ox < a.OW && channel < a.Kc
+                                ? a.dy[(static_cast<size_t>(i) * a.Kc + channel) * a.OH * a.OW + oy * a.OW + ox] : 0.0f;
+              nan = nan || d != d;
+            }
+            if (__any(nan)) {
+              nan_rows |= 1u << row;
+              break;
+            }
+          }
+        }
+        nan_rows >>= 4 * (lane >> 5);
+#pragma unroll
+        for (int fx = 0; fx < S; ++fx)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (nan_rows >> (8 * (r >> 2) + (r & 3)) & 1u) sum[fx][r] = __builtin_nanf("");
+        if (x3_all_nan(sum)) return;
       }
     }
-  }
+  });
 }
 
 template <int RW, int S, int TC, int COB, int CIB, int SHIFT, bool VEC>

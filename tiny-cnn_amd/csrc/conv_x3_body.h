@@ -25,52 +25,63 @@ typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 
 constexpr unsigned X3_NOWHERE = 0x80000000u;  // past the end of every tile's images
 
-// The wave's blocks once more in fp32, if a sum in them is infinite or NaN (split_bf16.h): lane l brings
-// channel l%32 of a filter block and pixel l%32 of a pixel block, for the reduction channel kc + l/32.
+// The wave's infinite and NaN sums once more in fp32 (split_bf16.h): lane l brings channel l%32 of a
+// filter block and pixel l%32 of a pixel block, for the reduction channel kc + l/32.
 template <int R, int S, int TC, int TM, int TN>
 __device__ __forceinline__ void x3_redo_exceptional(const ConvS1Args &a, floatx16 (&acc)[TM][TN], const int wn,
                                                     const int lane, const int img0, const int y0, const int x0,
                                                     const int m0, const int kc_lo, const int kc_hi) {
   constexpr int LOG_TC = TC == 64 ? 6 : TC == 32 ? 5 : TC == 16 ? 4 : 3;
-  if (!x3_exceptional<16 * TM * TN>([&](int e) { return acc[e / (16 * TN)][e / 16 % TN][e % 16]; })) return;
-  int img[TN], iy[TN], ix[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int q = (wn * TN + j) * 32 + (lane & 31);
-    img[j] = img0 + (q >> (a.log_tr + LOG_TC));
-    iy[j]  = y0 + ((q >> LOG_TC) & (a.TR - 1)) - a.ph;
-    ix[j]  = x0 + (q & (TC - 1)) - a.pw;
-  }
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = floatx16{};
+  // (hidden from the compiler, which otherwise keeps this function's comparisons and addresses for the stores behind)
+  int rows = a.MC - (m0 + 4 * (lane >> 5)), pix = wn * TN * 32 + (lane & 31);
+  asm volatile("" : "+v"(rows), "+v"(pix));
+  auto place = [&](int j, int &img, int &oy, int &ox) {
+    const int q = pix + 32 * j;
+    img = img0 + (q >> (a.log_tr + LOG_TC));
+    oy  = y0 + ((q >> LOG_TC) & (a.TR - 1));
+    ox  = x0 + (q & (TC - 1));
+    return img < a.batch && oy < a.OH && ox < a.OW;
+  };
+  x3_redo(reinterpret_cast<floatx16(&)[TM * TN]>(acc), [&](int b, int r) {
+    int img, oy, ox;
+    return place(b % TN, img, oy, ox) && 32 * (b / TN) + 8 * (r >> 2) + (r & 3) < rows;
+  }, [&](floatx16 (&sum)[TM * TN]) {
 #pragma unroll 1
-  for (int kc0 = kc_lo; kc0 < kc_hi; kc0 += 2) {
-    const int kc = kc0 + (lane >> 5);
+    for (int kc0 = kc_lo; kc0 < kc_hi; kc0 += 2) {
+      const int kc = kc0 + (lane >> 5);
 #pragma unroll 1
-    for (int fy = 0; fy < R; ++fy)
-#pragma unroll
-      for (int fx = 0; fx < S; ++fx) {
-        float w[TM], x[TN];
+      for (int fy0 = 0; fy0 < R; ++fy0) {
+        float wv[TM][S], xv[TN][S];
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
-          const int m = m0 + 32 * i + (lane & 31), t = fy * S + fx;
+          const int m   = m0 + 32 * i + (lane & 31);
           const bool on = kc < kc_hi && m < a.MC && (!a.tbl || a.tbl[a.flip ? m * a.KC + kc : kc * a.MC + m]);
-          w[i] = on ? a.w[static_cast<size_t>(a.flip ? kc * a.MC + m : m * a.KC + kc) * (R * S) + (a.flip ? R * S - 1 - t : t)] : 0.0f;
+          const float *w = a.w + static_cast<size_t>(on ? (a.flip ? kc * a.MC + m : m * a.KC + kc) : 0) * (R * S);
+#pragma unroll
+          for (int t = 0; t < S; ++t) wv[i][t] = on ? w[a.flip ? R * S - 1 - fy0 * S - t : fy0 * S + t] : 0.0f;
         }
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-          const bool in = kc < kc_hi && img[j] < a.batch && static_cast<unsigned>(iy[j] + fy) < static_cast<unsigned>(a.IH) &&
-                          static_cast<unsigned>(ix[j] + fx) < static_cast<unsigned>(a.IW);
-          x[j] = in ? a.in[((static_cast<size_t>(img[j]) * a.KC + kc) * a.IH + iy[j] + fy) * a.IW + ix[j] + fx] : 0.0f;
+          int img, oy, ox;
+          const bool pixel = place(j, img, oy, ox) && kc < kc_hi;
+          const float *in  = a.in + (static_cast<size_t>(pixel ? img : 0) * a.KC + (pixel ? kc : 0)) * a.IH * a.IW;
+#pragma unroll
+          for (int t = 0; t < S; ++t) {
+            const int iy = oy - a.ph + fy0, ix = ox - a.pw + t;
+            const bool inside = pixel && static_cast<unsigned>(iy) < static_cast<unsigned>(a.IH) &&
+                                static_cast<unsigned>(ix) < static_cast<unsigned>(a.IW);
+            xv[j][t] = inside ? in[iy * a.IW + ix] : 0.0f;
+          }
         }
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+        for (int t = 0; t < S; ++t)
 #pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[i], x[j], acc[i][j], 0, 0, 0);
+          for (int b = 0; b < TM * TN; ++b)
+            sum[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[b / TN][t], xv[b % TN][t], sum[b], 0, 0, 0);
       }
-  }
+      if (x3_all_nan(sum)) return;
+    }
+  });
 }
 
 // the workgroup at (bx, by, bz) of the grid. BY_TAPS: the four waves share the

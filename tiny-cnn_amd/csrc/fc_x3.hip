@@ -179,28 +179,35 @@ fc_x3_kernel(const float *__restrict__ A, const float *__restrict__ B, const int
     if (k0 + FX_BK < kend) step(k0 + FX_BK, std::integral_constant<int, 1>());
   }
 
-  // the wave's blocks once more in fp32, if a sum in them is infinite or NaN (split_bf16.h): lane l
-  // brings row and column l%32 of the blocks at index k + l/32
-  if (x3_exceptional<64>([&](int e) { return acc[e / 32][e / 16 % 2][e % 16]; })) {
+  // the wave's infinite and NaN sums once more in fp32 (split_bf16.h): lane l brings row and column l%32
+  // of the blocks at index k + l/32; eight indices are asked for together
+  {
+    // (hidden from the compiler, which otherwise keeps the comparisons for the stores below)
+    int rows = M - (m0 + 64 * wm + 4 * half), cols = N - (n0 + 64 * wn + l32);   // from this lane's first element
+    asm volatile("" : "+v"(rows), "+v"(cols));
+    x3_redo(reinterpret_cast<floatx16(&)[4]>(acc), [&](int b, int r) {
+      return 32 * (b % 2) < cols && 32 * (b / 2) + 8 * (r >> 2) + (r & 3) < rows;
+    }, [&](floatx16 (&sum)[4]) {
+#pragma unroll 1
+      for (int k0 = kbeg; k0 < kend; k0 += 8) {
+        float av[4][2], bv[4][2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+        for (int s = 0; s < 4; ++s) {
+          const int k = k0 + 2 * s + half;
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = floatx16{};
-#pragma unroll 2
-    for (int k = kbeg; k < kend; k += 2) {
-      const bool on = k + half < kend;
-      float av[2], bv[2];
+          for (int i = 0; i < 2; ++i) {
+            const int m = m0 + 64 * wm + 32 * i + l32, n = n0 + 64 * wn + 32 * i + l32;
+            av[s][i] = k < kend && m < M ? A[static_cast<size_t>(m) * lda + k] : 0.0f;
+            bv[s][i] = k < kend && n < N ? B[B_KC ? static_cast<size_t>(n) * ldb + k : static_cast<size_t>(k) * ldb + n] : 0.0f;
+          }
+        }
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int m = m0 + 64 * wm + 32 * i + l32, n = n0 + 64 * wn + 32 * i + l32;
-        av[i] = on && m < M ? A[static_cast<size_t>(m) * lda + k + half] : 0.0f;
-        bv[i] = on && n < N ? B[B_KC ? static_cast<size_t>(n) * ldb + k + half : static_cast<size_t>(k + half) * ldb + n] : 0.0f;
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int b = 0; b < 4; ++b) sum[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[s][b / 2], bv[s][b % 2], sum[b], 0, 0, 0);
+        if (x3_all_nan(sum)) return;
       }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[j], acc[i][j], 0, 0, 0);
-    }
+    });
   }
 
   // D[i][j] of a block: reg r of lane l at row 8*(r/4) + 4*(l/32) + r%4, column l%32

@@ -22,10 +22,12 @@
 // not a bit of an ordinary sum changes).
 // High end: an operand that is infinite, NaN or above 2^104, and a sum above 2^80, leaves an infinity or
 // NaN in every sum that it is part of, where fp32 would give one, or a number. Each wave looks at its
-// finished sums, and where one is infinite or NaN (x3_exceptional) it computes its whole tile again with
-// v_mfma_f32_32x32x2_f32, operands straight from memory. Finite sums pay one multiplication each for
-// the look. us with every input NaN, against ordinary inputs: convolution 32 -> 64 of 64x64, batch 64,
-// forward and backward 918 / 227; 4096 x 4096 fully-connected layer, batch 256 556 / 343.
+// finished sums, and those that are infinite or NaN are computed again with v_mfma_f32_32x32x2_f32,
+// operands straight from memory, until each of them is NaN or complete (x3_redo): in a net that has
+// diverged that is after some operands. Finite sums pay one multiplication each for the look. us with
+// every input NaN / with ordinary ones: convolution 32 -> 64 of 64x64, batch 64, forward and backward 269 /
+// 223; a step of the VGG-style stack after it has diverged (all weights of three layers NaN, 7 of 128
+// filters of the fourth) / on finite values 4600 / 4340.
 #pragma once
 #include "common.h"
 
@@ -90,13 +92,42 @@ __device__ __forceinline__ void mfma_x3(floatx16_x3 (&acc)[TM][TN], const bf16x8
                      reinterpret_cast<const bf16x8(&)[1][TN][X3_PARTS]>(b), sign);
 }
 
-// whether any lane of the wave has an infinite or NaN element: 0 * infinity and 0 * NaN are NaN
-template <int N, class Get>
-__device__ __forceinline__ bool x3_exceptional(const Get &element) {
-  float probe = 0.0f;
+template <int N>
+__device__ __forceinline__ bool x3_all_nan(const floatx16_x3 (&sum)[N]) {
+  bool all = true;
 #pragma unroll
-  for (int e = 0; e < N; ++e) probe = __builtin_fmaf(element(e), 0.0f, probe);
-  return __builtin_expect(__any(!(probe == 0.0f)) != 0, 0);
+  for (int b = 0; b < N; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) all = all && sum[b][r] != sum[b][r];
+  return __all(all) != 0;
+}
+// A wave's N blocks of finished sums: the elements that are in use (element r of block b: used(b, r)) and
+// infinite or NaN are computed once more. add_up(sum) adds all their products to sum, or stops when
+// x3_all_nan(sum). The other elements stay as they are; in sum they are NaN.
+template <int N, class Used, class AddUp>
+__device__ __forceinline__ void x3_redo(floatx16_x3 (&acc)[N], const Used &used, const AddUp &add_up) {
+  float probe = 0.0f;   // 0 * infinity and 0 * NaN are NaN
+#pragma unroll
+  for (int b = 0; b < N; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(acc[b][r], 0.0f, probe);
+  if (__builtin_expect(__any(!(probe == 0.0f)) == 0, 1)) return;
+  uint32_t bad[N];
+  floatx16_x3 sum[N];
+#pragma unroll
+  for (int b = 0; b < N; ++b) {
+    bad[b] = 0;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      bad[b] |= (used(b, r) && !(__builtin_fabsf(acc[b][r]) <= 3.402823466e+38f) ? 1u : 0u) << r;
+      sum[b][r] = bad[b] >> r & 1u ? 0.0f : __builtin_nanf("");
+    }
+  }
+  add_up(sum);
+#pragma unroll
+  for (int b = 0; b < N; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[b][r] = bad[b] >> r & 1u ? sum[b][r] : acc[b][r];
 }
 
 }  // namespace
