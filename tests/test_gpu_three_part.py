@@ -81,6 +81,10 @@ def test_every_window_against_float64(T, cfg):
     (1028, 1012, 260),     # ragged on every side, a last step of four indices
     (2048, 64, 512),       # tiles of 64 columns
     (16384, 68, 132),      # a reduction of two steps and four indices
+    # (of the first three, forward and dX are left to other kernels: too few tiles)
+    (8192, 2048, 64),      # tiles of 64 rows
+    (1028, 1012, 520),     # ragged on every side
+    (4096, 64, 2048),      # tiles of 64 columns, dX with the shortest reduction
 ])
 def test_fc_matches_oracle(T, O, W, cfg):
     """dX as an operator, the forward product as a net's inference."""
@@ -91,7 +95,10 @@ def test_fc_matches_oracle(T, O, W, cfg):
     b = rng.standard_normal(no).astype(np.float32)
     dy = rng.standard_normal((bs, no)).astype(np.float32)
     xd, dx = T.to_device(x), T.DevBuf(x.shape)
+    T.profile_begin()
     T.fc_bwd(ni, no, True, bs, xd, T.to_device(w), T.to_device(dy), dx, None, None)
+    tags = {e["tag"].split()[0] for e in T.profile_end()}
+    assert "fc_dx_x3" in tags or cfg in ((4096, 1024, 64), (1028, 1012, 260), (2048, 64, 512)), tags
     assert_close(dx.numpy(), O.fc_bwd(x, w, dy)[0], what=f"{cfg} dx")
     want = O.fc_fwd(x, w, b)
     for flags, act in ((0, False), (T.NET_FUSE_ACT_GRAD, True)):
@@ -145,3 +152,21 @@ def test_fc_of_tiny_operands(T, W, scale):
         # (a sum of 1024 products rounded after each: sqrt(1024) half-ulps, 9.5e-7)
         assert np.linalg.norm(got - want) <= 5.0e-7 * np.linalg.norm(want), name
     net.close()
+
+
+@pytest.mark.parametrize("batch", [4, 32, 64])
+def test_convolution_operator_and_inference_are_one_product(T, W, batch):
+    size, ic, oc, k = 24, 20, 40, 3
+    rng = np.random.default_rng(17)
+    d = T.conv_desc(size, size, ic, k, k, oc, pad_same=True)
+    x = rng.standard_normal((batch, ic * size * size)).astype(np.float32)
+    w, b = rng.uniform(-0.2, 0.2, oc * ic * k * k).astype(np.float32), rng.standard_normal(oc).astype(np.float32)
+    xd, y = T.to_device(x), T.DevBuf((batch, oc * size * size))
+    T.conv2d_fwd(d, batch, xd, T.to_device(w), T.to_device(b), y)
+    for flags in (0, T.NET_GRAPH):
+        net = T.Net(W.build_layers(T, [("conv", size, size, ic, k, oc, True)]), batch, flags)
+        net.set_param(0, 0, w)
+        net.set_param(0, 1, b)
+        net.forward(batch, xd)
+        assert np.array_equal(y.numpy(), net.layer_out(0, batch))
+        net.close()

@@ -42,11 +42,17 @@ struct Context {
   //  - its forward pass decides signs (relu) and maxima (max-pool), and with them where whole
   //    gradients go: one choice in a million changes, and the input gradient of the VGG-style
   //    stack by 1.6e-3 with it;
-  //    (A fully-connected product called as an operator may be the forward half of such a step: every
-  //    bias gradient hangs on its last bits through the activation behind it, and Adam makes a full
-  //    step of one that is nearly zero.)
   //  - the bias gradient of a convolution in front of a batch normalization is zero but for its
   //    rounding, and an optimizer that divides by the gradient's size makes full steps of that.
+  // So it is set in the forward pass of a net's train step, in the whole step of a net with batch
+  // normalization, and in tdh_fc_fwd. That one because of a third such place, in steps that a caller
+  // builds out of operators: Adam divides by sqrt(v + 1e-8), so a bias gradient that cancels to less than
+  // 1e-4 passes its last bits on to the bias 10^4-fold, and it has them from the forward product by way
+  // of the activation. 4096 outputs, batch 256: gradients of order 1, 0.4 of them below 1e-4 on average;
+  // with the other kernels one run in six ended with biases 5e-5 away (largest 3e-3), outputs being
+  // four times nearer to float64. tdh_conv2d_fwd is free: a convolution has as many biases as channels and
+  // sums their gradients over the pixels as well (64 channels of 64x64, batch 64: 1e-4 of them on
+  // average). Inference decides nothing, and is free everywhere.
   bool keep_f32 = false;
   // two more streams (default priority) for work that branches off the main one inside a
   // captured train step; created on first use
@@ -61,7 +67,7 @@ struct StreamSwap {
 };
 
 Context &ctx();
-// Products inside the scope keep to fp32 instructions and to one order of their sums whatever the
+// Products inside the scope keep to fp32 instructions, and to one order of their sums whatever the
 // batch's size (see Context::keep_f32).
 struct KeepF32 {
   const bool was;

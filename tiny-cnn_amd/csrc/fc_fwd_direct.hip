@@ -8,8 +8,8 @@
 // and its output's column of the same four rows of W (64 bytes a row of the tile). Four blocks'
 // loads are under way before the first product. The waves' sums meet in LDS, one thread finishes
 // one output; with at most 16 outputs a workgroup has whole rows and takes the softmax as well.
-// us, kernels before / here, one sample: 1024 -> 64 7.1 / 4.0, 64 -> 10 4.9 / 3.2; 32 samples, 512 -> 512
-// 20.0 / 3.6.
+// us in a net's inference, kernels before / here, one sample: 1024 -> 64 7.1 / 4.0, 64 -> 10 4.9 / 3.2; 32 samples,
+// 512 -> 512 20.0 / 3.6. (tdh_fc_fwd does not come here, see Context::keep_f32.)
 // Bound: latency, and for large layers the read of W.
 //
 // Reference: fully_connected_op_internal.h:13-37 (forward), softmax_layer.h:36-55.
