@@ -171,7 +171,7 @@ int tdh_conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const floa
  * (TDH_ERR_UNSUPPORTED) for a descriptor with a connection table. Same
  * arguments, kernels and results as tdh_conv2d_bwd (a shape whose three-part kernels would not fit
  * runs the fp32 ones instead), but the kernels' scratch (split partial
- * sums, repacked filters) lies in a static 64 MiB device array that the library holds on every
+ * sums, packed filters) lies in a static 64 MiB device array that the library holds on every
  * device it is initialised on, and the call allocates and frees nothing. A shape whose scratch
  * need exceeds the array is refused with TDH_ERR_INVALID (the message states both sizes); use
  * tdh_conv2d_bwd for it. All calls on one GPU share that GPU's array: calls are ordered by the
