@@ -1,0 +1,108 @@
+"""Forward convolution and dX by the kernel that takes any window, stride and size: against float64 where its tiles, chunks of
+channels and phases end, and with infinities, NaN and the largest floats among the operands."""
+import numpy as np
+import pytest
+
+from conftest import assert_close
+from test_gpu_exceptional_values import check, plant
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(x, w, b, dy, same, stride, dilation=(1, 1)):
+    """y and dx in float64, a tap at a time. What lies outside the image, or outside the output, is a zero that is multiplied like
+    any other value; padding::same puts k // 2 zeros in front."""
+    x, w, dy = (a.astype(np.float64) for a in (x, w, dy))
+    (ih, iw), (oh, ow), (kh, kw) = x.shape[2:], dy.shape[2:], w.shape[2:]
+    (sh, sw), (eh, ew), (ph, pw) = stride, dilation, [k // 2 if same else 0 for k in (kh, kw)]
+
+    def gather(a, rows, cols):
+        inside = (rows >= 0) & (rows < a.shape[2]), (cols >= 0) & (cols < a.shape[3])
+        g = np.zeros(a.shape[:2] + (len(rows), len(cols)))
+        g[:, :, np.flatnonzero(inside[0])[:, None], np.flatnonzero(inside[1])] = a[:, :, rows[inside[0]][:, None], cols[inside[1]]]
+        return g.reshape(a.shape[:2] + (-1,))
+
+    y, dx = np.zeros(dy.shape), np.zeros(x.shape)
+    with np.errstate(invalid="ignore", over="ignore"):
+        for ky in range(kh):
+            for kx in range(kw):
+                y += np.matmul(w[:, :, ky, kx], gather(x, np.arange(oh) * sh + ky * eh - ph, np.arange(ow) * sw + kx * ew - pw)).reshape(y.shape)
+                iy, ix = (np.flatnonzero((np.arange(n) + p - k) % s == 0) for n, p, k, s in ((ih, ph, ky, sh), (iw, pw, kx, sw)))
+                part = np.matmul(w[:, :, ky, kx].T, gather(dy, (iy + ph - ky) // sh, (ix + pw - kx) // sw))
+                dx[:, :, iy[:, None], ix] += part.reshape(dx.shape[:2] + (len(iy), len(ix)))
+        return y + b.astype(np.float64).reshape(1, -1, 1, 1), dx
+
+
+CASES = [
+    # in_w, in_h, in_c, kw, kh, out_c, same, (sh, sw), batch; the directions that take the kernel
+    (45, 37, 21, 5, 5, 45, False, (2, 2), 19, "fb"),   # 9, 6, 6 and 4 taps a phase, a last group of 5 channels
+    (31, 91, 3, 7, 7, 20, True, (2, 2), 40, "fb"),     # three channels: reductions of one group
+    (17, 15, 79, 7, 7, 4, True, (1, 1), 60, "fb"),     # tiles of several images, several chunks
+    (26, 32, 9, 3, 3, 69, True, (1, 1), 40, "b"),      # dX of 9 channels
+    (34, 21, 58, 5, 5, 3, False, (1, 1), 92, "f"),     # 3 of 16 rows in use
+    (50, 47, 40, 3, 2, 130, True, (3, 1), 24, "fb"),   # unequal strides and window sides, channels past two workgroups
+    (21, 20, 70, 3, 3, 65, True, (2, 1), 33, "fb"),
+    (96, 5, 33, 1, 7, 40, True, (2, 2), 60, "b"),      # one column of taps: phases without a tap
+    (65, 40, 26, 5, 5, 30, True, (1, 1), 12, "b"),     # in the place of the stride-1 kernel
+    (9, 9, 64, 3, 3, 64, False, (2, 2), 300, "fb"),    # images of 16 outputs
+]
+
+
+def operands(T, cfg, rng):
+    iw, ih, ic, kw, kh, oc, same, (sh, sw), bs = cfg[:9]
+    d = T.conv_desc(iw, ih, ic, kw, kh, oc, pad_same=same, w_stride=sw, h_stride=sh)
+    ow, oh = T.conv_out_shape(d)
+    x = rng.standard_normal((bs, ic, ih, iw)).astype(np.float32)
+    w = rng.uniform(-0.3, 0.3, (oc, ic, kh, kw)).astype(np.float32)
+    return d, x, w, rng.standard_normal(oc).astype(np.float32), rng.standard_normal((bs, oc, oh, ow)).astype(np.float32)
+
+
+def run(T, d, x, w, b, dy):
+    y, dx = T.to_device(np.full(dy.size, 7, np.float32)), T.to_device(np.full(x.size, 7, np.float32))
+    xd, wd, bd, dyd = (T.to_device(a.ravel()) for a in (x, w, b, dy))
+    T.profile_begin()
+    T.conv2d_fwd(d, len(x), xd, wd, bd, y)
+    T.conv2d_bwd(d, len(x), xd, wd, dyd, dx, None, None)
+    tags = {e["tag"].split()[0] for e in T.profile_end()}
+    return y.numpy(), dx.numpy(), "".join(k for k, t in (("f", "conv_fwd_any_x3"), ("b", "conv_dx_any_x3")) if t in tags)
+
+
+@pytest.mark.parametrize("cfg", CASES)
+def test_against_float64(T, cfg):
+    d, x, w, b, dy = operands(T, cfg, np.random.default_rng(41))
+    y, dx, taken = run(T, d, x, w, b, dy)
+    assert taken == cfg[9]
+    for got, want, name in zip((y, dx), reference(x, w, b, dy, cfg[6], cfg[7]), ("y", "dx")):
+        assert_close(got, want.ravel(), what=f"{cfg} {name}")
+        # No further from float64 than a sum in fp32: K terms in order, each addition rounding to 2^-24 of a partial sum
+        # that grows as a random walk, leave 2^-24 sqrt(K / 6) of the result; six bits under that and 2^-23 of the parts.
+        k = cfg[3] * cfg[4] * cfg[2 if name == "y" else 5] / (1 if name == "y" else cfg[7][0] * cfg[7][1])
+        assert np.linalg.norm(got - want.ravel()) <= 2 ** -24 * (2 + np.sqrt(k / 6)) * np.linalg.norm(want)
+
+
+def test_dilation(T):
+    iw, ih, ic, k, oc, bs = 40, 33, 20, 3, 40, 30
+    rng = np.random.default_rng(42)
+    d = T.conv_desc(iw, ih, ic, k, k, oc, pad_same=False, w_stride=2, h_stride=1, w_dilation=3, h_dilation=2)
+    ow, oh = T.conv_out_shape(d)
+    x = rng.standard_normal((bs, ic, ih, iw)).astype(np.float32)
+    w = rng.uniform(-0.3, 0.3, (oc, ic, k, k)).astype(np.float32)
+    b = rng.standard_normal(oc).astype(np.float32)
+    y = T.DevBuf((bs * oc * oh * ow,))
+    T.profile_begin()
+    T.conv2d_fwd(d, bs, T.to_device(x.ravel()), T.to_device(w.ravel()), T.to_device(b), y)
+    assert any(e["tag"].startswith("conv_fwd_any_x3") for e in T.profile_end())
+    want = reference(x, w, b, np.zeros((bs, oc, oh, ow), np.float32), False, (1, 2), (2, 3))[0]
+    assert_close(y.numpy(), want.ravel(), what="y")
+
+
+@pytest.mark.parametrize("where", ["x", "w", "dy"])
+@pytest.mark.parametrize("cfg", [CASES[0], CASES[9]])
+def test_exceptional_values(T, cfg, where):
+    rng = np.random.default_rng(43)
+    d, x, w, b, dy = operands(T, cfg, rng)
+    plant({"x": x, "w": w, "dy": dy}[where], rng, 6)
+    y, dx, taken = run(T, d, x, w, b, dy)
+    assert taken == "fb"
+    for got, want, name in zip((y, dx), reference(x, w, b, dy, cfg[6], cfg[7]), ("y", "dx")):
+        check(got, want, f"{cfg} {name}")

@@ -476,6 +476,7 @@ bool conv_s1_fuses_pool(int R, int S, int batch, int KC, int MC, int IH, int IW,
 bool conv_s1_single_pass(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW,
                          int ph, int pw);
 // conv_packed_kind / conv_packed_bytes of a shape this file runs
+double conv_s1_fill(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw);
 int conv_s1_packed_kind(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw);
 size_t conv_s1_packed_bytes(int kind, int RS, int KC, int MC);
 // conv_dw.hip: stride-1 weight gradient from LDS-staged tiles (3x3 and 5x5 windows)
@@ -489,6 +490,19 @@ size_t conv_dw_halo_run_workspace_bytes(int R, int S, int batch, int C, int Kc, 
 int conv_dw_halo_run(int R, int S, int batch, int C, int Kc, const float *x, const float *dy,
                      float *dw, int H, int W, int OH, int OW, int ph, int pw, int accumulate,
                      float *db = nullptr);
+// conv_any.hip: forward pass and dX of any window, stride and size, on three-part operands
+struct ConvShape {
+  int batch, C, Kc, H, W, OH, OW, R, S, sh, sw, dh, dw, ph, pw;
+};
+// the kernel that would compute dX otherwise: the generic GEMM, a first layer's, a stride-1 kernel with poorly filled tiles
+enum AnyOver { ANY_OVER_GENERIC, ANY_OVER_FIRST, ANY_OVER_STRIDE1 };
+bool conv_any_fwd_applicable(const ConvShape &c);   // in the place of the generic GEMM
+bool conv_any_dx_applicable(const ConvShape &c, AnyOver over);
+size_t conv_any_fwd_workspace_bytes(const ConvShape &c);
+size_t conv_any_dx_workspace_bytes(const ConvShape &c);
+int conv_any_fwd_run(const ConvShape &c, const float *x, const float *w, const float *bias, float *out, float *act_out,
+                     int act_kind);
+int conv_any_dx_run(const ConvShape &c, const float *dy, const float *w, float *dx, ActGrad ag);
 // conv_bwd_direct.hip: any of dX, dW and db of a layer that is a few small tiles, as one launch
 bool conv_bwd_direct_applicable(int batch, int C, int Kc, int H, int W, int OH, int OW, int R, int S);
 int conv_bwd_direct_run(int batch, int C, int Kc, const float *x, const float *w, const float *dy, float *dx, float *dw,

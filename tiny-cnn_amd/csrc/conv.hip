@@ -1133,6 +1133,21 @@ static bool fwd_direct_applies(const ConvGeom &g, int batch) {
   return conv_fwd_direct_applicable(batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.R, g.S);
 }
 
+static ConvShape shape_of(const ConvGeom &g, int batch) {
+  return {batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.R, g.S, g.sh, g.sw, g.dh, g.dw, g.pad_h, g.pad_w};
+}
+// Gradients of too few workgroups for the three-part stride-1 kernel take the fp32 one, unless its tiles are less
+// than four fifths full (columns come in 8 to 64, channels in 32 or 64): then the kernel of any size, dX in us
+// there / here, packing included: 65x40, 26 -> 30, 5x5, 12 images 45 / 25, 43x31, 94 -> 74, 3x3, 6 images 40 /
+// 25, 19x89, 64 -> 21, 3x3, 11 images 26 / 16. (The forward product would gain as much; there the operator's and
+// a net's inference are one product, and the net's may take the layers behind along.)
+constexpr double ANY_FILL = 0.8;
+// (a train step, which adds to its gradients, has the same bits with filters that the net has packed for the stride-1 kernel)
+static bool dx_any_over_stride1(const ConvGeom &g, int batch, int accumulate) {
+  return !accumulate && conv_s1_fill(g.R, g.S, batch, g.Kc, g.C, g.OH, g.OW, g.H, g.W, g.R - 1 - g.pad_h, g.S - 1 - g.pad_w) < ANY_FILL &&
+         conv_any_dx_applicable(shape_of(g, batch), ANY_OVER_STRIDE1);
+}
+
 static bool fwd_small_applies(const ConvGeom &g, int batch) {
   // (small windows over many channels are short reductions as well, but no first layers)
   if (g.C >= 16 && g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 &&
@@ -1200,6 +1215,7 @@ size_t conv2d_workspace_bytes(const tdh_conv_desc *d, int batch) {
   total += first_both_workspace_bytes(d, g, batch);
   if (g.sh == 1 && g.sw == 1)
     total += conv_dw_halo_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
+  total += conv_any_fwd_workspace_bytes(shape_of(g, batch)) + conv_any_dx_workspace_bytes(shape_of(g, batch));
   if (g.sh == 1 && g.sw == 1) {  // LDS-halo kernel: repacked filters and split partial sums
     total += conv_s1_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, 0, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
     total += conv_s1_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, 1, g.OH, g.OW, g.H, g.W,
@@ -1224,15 +1240,24 @@ size_t conv2d_bwd_workspace_bytes(const tdh_conv_desc *d, int batch, const float
   DxsPlan dxs;
   DxPhases ph;
   int columns = 0, longest = 0;
-  if (dx && !small_cin_dx_plan(g, dxs)) {
-    if (g.sh == 1 && g.sw == 1 &&
-        conv_s1_applicable(g.R, g.S, batch, g.Kc, g.C, g.OH, g.OW, g.H, g.W, g.R - 1 - g.pad_h, g.S - 1 - g.pad_w))
-      total += conv_s1_run_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, 1, g.OH, g.OW, g.H, g.W, g.R - 1 - g.pad_h,
-                                           g.S - 1 - g.pad_w);
-    else if (dx_phases(g, batch, ph, &columns, &longest))
-      total += gemm_workspace_bytes(g.C, columns, longest, true);
-    else
-      total += gemm_workspace_bytes(g.C, batch * g.H * g.W, g.Kc * g.R * g.S, true);
+  const bool first = small_cin_dx_plan(g, dxs);
+  if (dx && first && conv_any_dx_applicable(shape_of(g, batch), ANY_OVER_FIRST)) {
+    total += conv_any_dx_workspace_bytes(shape_of(g, batch));
+  } else if (dx && !first) {
+    const bool stride1 = g.sh == 1 && g.sw == 1 &&
+                         conv_s1_applicable(g.R, g.S, batch, g.Kc, g.C, g.OH, g.OW, g.H, g.W, g.R - 1 - g.pad_h, g.S - 1 - g.pad_w);
+    size_t most = 0;
+    if (stride1 ? dx_any_over_stride1(g, batch, accumulate) : conv_any_dx_applicable(shape_of(g, batch), ANY_OVER_GENERIC))
+      most = conv_any_dx_workspace_bytes(shape_of(g, batch));
+    // (filters that the caller has packed keep to the stride-1 kernel)
+    if (stride1)
+      most = std::max(most, conv_s1_run_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, 1, g.OH, g.OW, g.H, g.W, g.R - 1 - g.pad_h,
+                                                        g.S - 1 - g.pad_w));
+    else if (!most && dx_phases(g, batch, ph, &columns, &longest))
+      most = gemm_workspace_bytes(g.C, columns, longest, true);
+    else if (!most)
+      most = gemm_workspace_bytes(g.C, batch * g.H * g.W, g.Kc * g.R * g.S, true);
+    total += most;
   }
   if (dw && dw_small_applies(d, g, batch) && dy_aligned)
     return total + conv_dw_small_workspace_bytes(batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.R, g.S, g.sh, g.sw, g.dh, g.dw,
@@ -1462,6 +1487,8 @@ int conv2d_fwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
     return conv_s1_run(g.R, g.S, batch, g.C, g.Kc, 0, x, w_eff, nullptr,
                        d->has_bias ? b : nullptr, y, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w,
                        ActGrad(), "conv_fwd_s1", PackedFilters(), act_out, act_kind, pool);
+  if (conv_any_fwd_applicable(shape_of(g, batch)))
+    return conv_any_fwd_run(shape_of(g, batch), x, w_eff, d->has_bias ? b : nullptr, y, act_out, act_kind);
   StridedOperand A{w_eff, crs, 1, g.Kc};
   FwdInputOperand B{x, g, batch * ohw};
   if (act_out) {  // the pointwise activation layer that follows leaves the same kernel
@@ -1603,18 +1630,23 @@ int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
   TDH_TRY(prepare_table(d, g, w, tbl_resident, &tbl_dev, &w_eff));
   DxsPlan dxs;
   int phase_columns = 0, phase_k = 0;
+  const bool dx_stride1 = dx && g.sh == 1 && g.sw == 1 &&
+                          conv_s1_applicable(g.R, g.S, batch, g.Kc, g.C, g.OH, g.OW, g.H, g.W, g.R - 1 - g.pad_h,
+                                             g.S - 1 - g.pad_w);
   if (dx && small_cin_dx_plan(g, dxs) && !(reinterpret_cast<uintptr_t>(dy) & 15) &&
       first_dx_mfma<false>(g, batch, dy, w_eff, dx, dx_act, PoolGather(), true)) {
     ProfScope prof("conv_dx_first_mfma", g.C, batch * g.H * g.W, g.Kc * g.R * g.S);
     first_dx_mfma<false>(g, batch, dy, w_eff, dx, dx_act, PoolGather(), false);
     TDH_LAUNCH_CHECK();
+  } else if (dx && (small_cin_dx_plan(g, dxs) ? conv_any_dx_applicable(shape_of(g, batch), ANY_OVER_FIRST)
+                    : dx_stride1              ? dx_any_over_stride1(g, batch, accumulate)
+                                              : conv_any_dx_applicable(shape_of(g, batch), ANY_OVER_GENERIC))) {
+    TDH_TRY(conv_any_dx_run(shape_of(g, batch), dy, w_eff, dx, dx_act));
   } else if (dx && small_cin_dx_plan(g, dxs)) {
     ProfScope prof("conv_dx_small_cin", g.C, batch * g.H * g.W, g.Kc * g.R * g.S);
     launch_small_cin_dx_window<false>(g, dxs, batch, dy, w_eff, dx, dx_act, PoolGather());
     TDH_LAUNCH_CHECK();
-  } else if (dx && g.sh == 1 && g.sw == 1 &&
-             conv_s1_applicable(g.R, g.S, batch, g.Kc, g.C, g.OH, g.OW, g.H, g.W,
-                                g.R - 1 - g.pad_h, g.S - 1 - g.pad_w)) {
+  } else if (dx && dx_stride1) {
     TDH_TRY(conv_s1_run(g.R, g.S, batch, g.C, g.Kc, 1, dy, w_eff, nullptr, nullptr, dx, g.OH,
                         g.OW, g.H, g.W, g.R - 1 - g.pad_h, g.S - 1 - g.pad_w, dx_act,
                         "conv_dx_s1"));

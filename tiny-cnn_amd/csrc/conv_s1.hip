@@ -261,6 +261,14 @@ bool conv_s1_applicable(int R, int S, int batch, int KC, int MC, int IH, int IW,
   return make_plan(R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw).ok;
 }
 
+// The share of its tiles' outputs that exist, of the fp32 kernel's; 1 where another one runs.
+double conv_s1_fill(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw) {
+  const S1Plan p = make_plan(R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw);
+  if (!p.ok || p.x3) return 1.0;
+  const double in_tiles = 128.0 * p.tn * p.grid.x * (32.0 * p.tm * p.grid.y);
+  return static_cast<double>(batch) * OH * OW * MC / in_tiles;
+}
+
 int conv_s1_packed_kind(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw) {
   const S1Plan p = make_plan(R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw);
   return !p.ok ? CONV_PACK_NONE : p.x3 ? CONV_PACK_X3 : CONV_PACK_F32;
