@@ -1,4 +1,4 @@
-"""Forward convolution and dX by the kernel that takes any window, stride and size: against float64 where its tiles, chunks of
+"""Forward convolution, dX and dW by the kernels that take any window, stride and size: against float64 where its tiles, chunks of
 channels and phases end, and with infinities, NaN and the largest floats among the operands."""
 import numpy as np
 import pytest
@@ -106,3 +106,65 @@ def test_exceptional_values(T, cfg, where):
     assert taken == "fb"
     for got, want, name in zip((y, dx), reference(x, w, b, dy, cfg[6], cfg[7]), ("y", "dx")):
         check(got, want, f"{cfg} {name}")
+
+
+DW_CASES = [
+    # as above, and what the launch is called with gradients stored and added (a train step keeps db apart)
+    (45, 37, 21, 5, 5, 45, False, (2, 2), 19, "conv_dw_db_any", "conv_dw_any"),
+    (59, 30, 46, 5, 5, 3, False, (1, 1), 40, "conv_dw_db_any", "conv_dw_any"),     # channels shared by two tiles of columns
+    (31, 91, 3, 7, 7, 20, True, (2, 2), 260, "conv_dw_db_any", "conv_dw_any"),     # one or two channels a tile
+    (23, 19, 33, 7, 3, 70, True, (3, 1), 60, "conv_dw_db_any", "conv_dw_any"),     # two workgroups of output channels
+    (12, 11, 85, 1, 7, 3, True, (2, 2), 600, "conv_dw_db_any", "conv_dw_any"),     # several images a chunk
+    (12, 11, 85, 5, 5, 3, True, (1, 1), 200, "conv_dw_db_any", "conv_dw_any"),
+    (22, 20, 32, 3, 3, 3, False, (2, 2), 900, "conv_dw_any", "conv_dw_any"),       # 288 columns: db is no part of the tiles
+]
+
+
+def weight_gradient(x, dy, kh, kw, same, stride):
+    x, dy = x.astype(np.float64), dy.astype(np.float64)
+    (oh, ow), (sh, sw), (ph, pw) = dy.shape[2:], stride, [k // 2 if same else 0 for k in (kh, kw)]
+    xp = np.zeros(x.shape[:2] + (x.shape[2] + 2 * kh + sh, x.shape[3] + 2 * kw + sw))
+    xp[:, :, ph:ph + x.shape[2], pw:pw + x.shape[3]] = x
+    dw = np.zeros((dy.shape[1], x.shape[1], kh, kw))
+    flat = dy.transpose(1, 0, 2, 3).reshape(dy.shape[1], -1)
+    with np.errstate(invalid="ignore", over="ignore"):
+        for ky in range(kh):
+            for kx in range(kw):
+                part = xp[:, :, ky:ky + (oh - 1) * sh + 1:sh, kx:kx + (ow - 1) * sw + 1:sw]
+                dw[:, :, ky, kx] = np.matmul(flat, part.transpose(0, 2, 3, 1).reshape(-1, x.shape[1]))
+        return dw, dy.sum(axis=(0, 2, 3))
+
+
+@pytest.mark.parametrize("accumulate", [0, 1])
+@pytest.mark.parametrize("cfg", DW_CASES)
+def test_weight_gradient_against_float64(T, cfg, accumulate):
+    rng = np.random.default_rng(44)
+    d, x, w, b, dy = operands(T, cfg, rng)
+    before = rng.standard_normal(w.size + b.size).astype(np.float32)
+    dw, db = T.to_device(before[:w.size].copy()), T.to_device(before[w.size:].copy())
+    T.profile_begin()
+    T.conv2d_bwd(d, len(x), T.to_device(x.ravel()), T.to_device(w.ravel()), T.to_device(dy.ravel()), None, dw, db, accumulate)
+    tags = {e["tag"].split()[0] for e in T.profile_end()}
+    assert cfg[9 + accumulate] in tags, tags
+    want = weight_gradient(x, dy, cfg[4], cfg[3], cfg[6], cfg[7])
+    for got, ref, old, name in zip((dw.numpy(), db.numpy()), want, (before[:w.size], before[w.size:]), ("dw", "db")):
+        ref = ref.ravel() + (old if accumulate else 0)
+        assert_close(got, ref, what=f"{cfg} {name}")
+        # K products in order in at least 64 slices: the bound of the sums above for K / 64 terms and for 64
+        k = dy.size / dy.shape[1]
+        assert np.linalg.norm(got - ref) <= 2 ** -24 * (3 + np.sqrt(k / 64 / 6) + np.sqrt(64 / 6)) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("where", ["x", "dy"])
+def test_weight_gradient_of_exceptional_values(T, where):
+    cfg = (59, 30, 46, 5, 5, 3, False, (1, 1), 13)   # (18590 pixels: a last piece of 14)
+    rng = np.random.default_rng(45)
+    d, x, w, b, dy = operands(T, cfg, rng)
+    plant({"x": x, "dy": dy}[where], rng, 6)
+    (x if where == "x" else dy)[-1, 2, -1, -1] = np.inf
+    dw, db = T.DevBuf((w.size,)), T.DevBuf((b.size,))
+    T.profile_begin()
+    T.conv2d_bwd(d, len(x), T.to_device(x.ravel()), T.to_device(w.ravel()), T.to_device(dy.ravel()), None, dw, db)
+    assert any(e["tag"].startswith("conv_dw_db_any") for e in T.profile_end())
+    for got, ref, name in zip((dw.numpy(), db.numpy()), weight_gradient(x, dy, 5, 5, False, (1, 1)), ("dw", "db")):
+        check(got, ref, name)

@@ -493,6 +493,10 @@ int conv_dw_halo_run(int R, int S, int batch, int C, int Kc, const float *x, con
 // conv_any.hip: forward pass and dX of any window, stride and size, on three-part operands
 struct ConvShape {
   int batch, C, Kc, H, W, OH, OW, R, S, sh, sw, dh, dw, ph, pw;
+  bool operator==(const ConvShape &o) const {
+    return batch == o.batch && C == o.C && Kc == o.Kc && H == o.H && W == o.W && OH == o.OH && OW == o.OW && R == o.R &&
+           S == o.S && sh == o.sh && sw == o.sw && dh == o.dh && dw == o.dw && ph == o.ph && pw == o.pw;
+  }
 };
 // the kernel that would compute dX otherwise: the generic GEMM, a first layer's, a stride-1 kernel with poorly filled tiles
 enum AnyOver { ANY_OVER_GENERIC, ANY_OVER_FIRST, ANY_OVER_STRIDE1 };
@@ -503,6 +507,11 @@ size_t conv_any_dx_workspace_bytes(const ConvShape &c);
 int conv_any_fwd_run(const ConvShape &c, const float *x, const float *w, const float *bias, float *out, float *act_out,
                      int act_kind);
 int conv_any_dx_run(const ConvShape &c, const float *dy, const float *w, float *dx, ActGrad ag);
+// conv_dw_any.hip: dW (and db as column C*R*S) of any window, stride and size, as slices [slice][Kc][columns]
+bool conv_dw_any_applicable(const ConvShape &c, bool with_db);
+size_t conv_dw_any_workspace_bytes(const ConvShape &c, bool with_db);
+size_t conv_dw_any_most_bytes(const ConvShape &c, bool with_db);
+int conv_dw_any_run(const ConvShape &c, const float *x, const float *dy, bool with_db, const float **partial, int *slices);
 // conv_bwd_direct.hip: any of dX, dW and db of a layer that is a few small tiles, as one launch
 bool conv_bwd_direct_applicable(int batch, int C, int Kc, int H, int W, int OH, int OW, int R, int S);
 int conv_bwd_direct_run(int batch, int C, int Kc, const float *x, const float *w, const float *dy, float *dx, float *dw,

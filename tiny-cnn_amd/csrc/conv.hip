@@ -1215,6 +1215,7 @@ size_t conv2d_workspace_bytes(const tdh_conv_desc *d, int batch) {
   total += first_both_workspace_bytes(d, g, batch);
   if (g.sh == 1 && g.sw == 1)
     total += conv_dw_halo_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
+  total += conv_dw_any_most_bytes(shape_of(g, batch), true);
   total += conv_any_fwd_workspace_bytes(shape_of(g, batch)) + conv_any_dx_workspace_bytes(shape_of(g, batch));
   if (g.sh == 1 && g.sw == 1) {  // LDS-halo kernel: repacked filters and split partial sums
     total += conv_s1_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, 0, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
@@ -1267,6 +1268,8 @@ size_t conv2d_bwd_workspace_bytes(const tdh_conv_desc *d, int batch, const float
     if (g.sh == 1 && g.sw == 1 &&
         conv_dw_halo_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w))
       total += conv_dw_halo_run_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, x, dy, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
+    else if (conv_dw_any_applicable(shape_of(g, batch), dw_takes_db(d, crs, db, accumulate)))
+      total += conv_dw_any_workspace_bytes(shape_of(g, batch), dw_takes_db(d, crs, db, accumulate));
     else
       total += gemm_workspace_bytes(g.Kc, crs + (dw_takes_db(d, crs, db, accumulate) ? 1 : 0), batch * ohw, true);
   }
@@ -1698,6 +1701,17 @@ int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
       TDH_TRY(conv_dw_halo_run(g.R, g.S, batch, g.C, g.Kc, x, dy, dw, g.H, g.W, g.OH, g.OW, g.pad_h,
                                g.pad_w, accumulate, db));
       db = nullptr;
+    } else if (conv_dw_any_applicable(shape_of(g, batch), with_db)) {
+      const float *partial;
+      int slices;
+      TDH_TRY(conv_dw_any_run(shape_of(g, batch), x, dy, with_db, &partial, &slices));
+      if (with_db) {
+        TDH_TRY(launch_splitk_reduce(partial, slices, g.Kc, crs + 1, EpiDwDb{dw, db, crs, accumulate}, "conv_dw_splitk_reduce"));
+        db = nullptr;
+      } else {
+        TDH_TRY(launch_splitk_reduce(partial, slices, g.Kc, crs, EpiRowMajor{dw, crs, nullptr, ActGrad(), accumulate},
+                                     "conv_dw_splitk_reduce"));
+      }
     } else if (with_db) {
       EpiDwDb epi{dw, db, crs, accumulate};
       TDH_TRY((launch_gemm<true, true>(A, B, epi, g.Kc, crs + 1, batch * ohw, true, "conv_dw_db_gemm",

@@ -259,7 +259,10 @@ __global__ void __launch_bounds__(256, 2) conv_any_kernel(const AnyArgs a) {
 #pragma unroll
       for (int q = 0; q < ITEMS; ++q)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v[q][k] = load(first[q] + k < left ? off[q] : ANY_NOWHERE, 4 * (c0 + first[q] + k) * ihw);
+        for (int k = 0; k < 8; ++k) {
+          const bool there = first[q] + k < left;   // (the same for all lanes)
+          v[q][k] = load(there ? off[q] : ANY_NOWHERE, there ? 4 * (c0 + first[q] + k) * ihw : 0);
+        }
 #pragma unroll
       for (int q = 0; q < ITEMS; ++q) {
         uintx4 part[X3_PARTS];
@@ -472,7 +475,7 @@ AnyPlan plan_tile(const AnyArgs &base, int batch, int mb, int nb, int wk) {
   return p;
 }
 
-AnyPlan make_any_plan(const AnyArgs &base, int batch) {
+AnyPlan best_tile(const AnyArgs &base, int batch) {
   const int mb = any_mb(base.M);
   AnyPlan best{};
   static const int tiles[7][2] = {{1, 4}, {2, 4}, {4, 4}, {1, 1}, {2, 2}, {2, 1}, {4, 1}};
@@ -533,6 +536,27 @@ bool backward_args(const ConvShape &c, AnyArgs &a) {
       p.cw = p.pw;
     }
   return a.phases > 0;
+}
+
+// (functions of the shape alone; the last of each is kept, because a call asks for it more than once)
+const AnyPlan &forward_plan(const ConvShape &c) {
+  static thread_local ConvShape shape{};
+  static thread_local AnyPlan plan{};
+  if (!(shape == c)) {
+    shape = c;
+    plan  = best_tile(forward_args(c), c.batch);
+  }
+  return plan;
+}
+const AnyPlan &backward_plan(const ConvShape &c) {
+  static thread_local ConvShape shape{};
+  static thread_local AnyPlan plan{};
+  if (!(shape == c)) {
+    AnyArgs a;
+    shape = c;
+    plan  = c.dh == 1 && c.dw == 1 && backward_args(c, a) ? best_tile(a, c.batch) : AnyPlan{};
+  }
+  return plan;
 }
 
 void finish_args(AnyArgs &a) {
@@ -603,13 +627,12 @@ double generic_us(double products) { return 11.0 + products / 16e6; }
 
 bool conv_any_fwd_applicable(const ConvShape &c) {
   if (ctx().keep_f32) return false;
-  const AnyPlan p = make_any_plan(forward_args(c), c.batch);
+  const AnyPlan &p = forward_plan(c);
   return p.ok && p.cost + ANY_PACK_US < generic_us(static_cast<double>(c.batch) * c.OH * c.OW * ceil_div(c.Kc, 32) * 32 * c.C * c.R * c.S);
 }
 bool conv_any_dx_applicable(const ConvShape &c, AnyOver over) {
-  AnyArgs a;
-  if (ctx().keep_f32 || c.dh != 1 || c.dw != 1 || !backward_args(c, a)) return false;
-  const AnyPlan p = make_any_plan(a, c.batch);
+  if (ctx().keep_f32) return false;
+  const AnyPlan &p = backward_plan(c);
   if (!p.ok) return false;
   const double pixels = static_cast<double>(c.batch) * c.H * c.W, k = static_cast<double>(c.Kc) * c.R * c.S / (c.sh * c.sw);
   switch (over) {
@@ -628,16 +651,14 @@ size_t conv_any_dx_workspace_bytes(const ConvShape &c) { return ws_align(any_pac
 
 int conv_any_fwd_run(const ConvShape &c, const float *x, const float *w, const float *bias, float *out, float *act_out,
                      int act_kind) {
-  AnyPlan p = make_any_plan(forward_args(c), c.batch);
+  AnyPlan p = forward_plan(c);
   if (!p.ok) return set_error(TDH_ERR_INVALID, "conv_any_fwd_run: no plan for this shape");
   finish_args(p.args);
   p.args.in = x; p.args.w = w; p.args.bias = bias; p.args.out = out; p.args.act_out = act_out; p.args.act_kind = act_kind;
   return run_any(p, "conv_fwd_any_x3", c.Kc, c.batch * c.OH * c.OW, c.C * c.R * c.S);
 }
 int conv_any_dx_run(const ConvShape &c, const float *dy, const float *w, float *dx, ActGrad ag) {
-  AnyArgs a;
-  AnyPlan p{};
-  if (c.dh == 1 && c.dw == 1 && backward_args(c, a)) p = make_any_plan(a, c.batch);
+  AnyPlan p = backward_plan(c);
   if (!p.ok) return set_error(TDH_ERR_INVALID, "conv_any_dx_run: no plan for this shape");
   finish_args(p.args);
   p.args.in = dy; p.args.w = w; p.args.out = dx; p.args.ag = ag;
