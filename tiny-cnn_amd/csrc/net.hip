@@ -236,9 +236,12 @@ bool tiny_step_applies(const tdh_net *net, int loss_kind);
 // launched: the VGG-style stack on 32x32 images, batch 32 380 / 375, on 64x64, batch 4 337 / 332, batch 16 587 /
 // 587; six 3x3 layers of 32 channels of 24x24, batch 128 513 / 509; three 5x5 layers of 48 channels of 12x12,
 // batch 64 241 / 241, batch 256 628 / 623; 784-1000-1000-10 fully connected, batch 1024 273 / 268; 1024-4096-4096-10,
-// batch 64 286 / 281. Below it the two are within 1 % of each other, and a replay leaves the host free.
+// batch 64 286 / 281. Below it the two are within 1 % of each other, and a replay leaves the host free. The step of a
+// workgroup per sample (tiny_net.hip) is three launches of 40, 9 and 5 us at least, whatever the net and the batch:
+// LeNet-5, batch 16 58.6 / 54.8, fed from the host in batches of 13 66.9 / 60.2 and of 221 136.6 / 128.3.
 bool step_outlasts_launches(const tdh_net *net, int loss_kind, int batch) {
-  return !tiny_step_applies(net, loss_kind) && !net_forks(net, batch) &&
+  if (tiny_step_applies(net, loss_kind)) return true;
+  return !net_forks(net, batch) &&
          net_forward_flop(net, batch) >= 5e7 * static_cast<double>(net->layers.size());
 }
 
