@@ -298,6 +298,14 @@ bool conv_dw_gives_db(const tdh_conv_desc *d, int batch);
 size_t batchnorm_workspace_bytes(int channels, int batch);
 int batchnorm_fwd(int channels, int spatial, int batch, float eps, int train, const float *x,
                   float *mean, float *variance, float *stddev, float *y);
+bool batchnorm_takes_pool(int channels, int spatial, int act_kind, const tdh_pool_desc *d);
+int batchnorm_act_pool_fwd(int channels, int spatial, int batch, float eps, int train, const float *x, float *mean,
+                           float *variance, float *stddev, float *y, int act_kind, float slope, float *act,
+                           const tdh_pool_desc *d, float *pooled, int32_t *argmax);
+// d_act: null where nobody reads the gradient of the activation's output
+int batchnorm_act_pool_bwd(int channels, int spatial, int batch, const float *y, const float *stddev, int act_kind,
+                           float slope, const float *act, const tdh_pool_desc *d, const float *dpool, const int32_t *argmax,
+                           float *d_act, float *d_norm, float *dx);
 int batchnorm_bwd(int channels, int spatial, int batch, const float *y, const float *dy,
                   const float *stddev, float *dx);
 // the running averages of up to BN_MOVING_MAX layers a launch

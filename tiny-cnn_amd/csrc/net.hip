@@ -427,6 +427,13 @@ bool pool_read_by_conv(tdh_net *net, int r, int batch) {
          conv_bwd_reads_pooled(&conv.spec.conv, &net->layers[r].spec.pool, batch);
 }
 
+// Layers i, i + 1 and i + 2 are a batch normalization, a rectifier and the 2x2 max-pool that norm.hip takes along.
+bool block_of_batchnorm(const tdh_net *net, int i) {
+  const tdh_layer &bn = net->layers[i].spec, &act = net->layers[i + 1].spec, &pool = net->layers[i + 2].spec;
+  return bn.kind == TDH_L_BATCHNORM && act.kind == TDH_L_ACT && pool.kind == TDH_L_MAXPOOL &&
+         batchnorm_takes_pool(bn.bn_channels, bn.bn_spatial, act.act, &pool.pool);
+}
+
 // The 2x2 max-pool in front of layer i (behind a folded activation, nothing folded into the pool
 // itself) that the dX epilogue of layer i can route its gradient through: its index, or -1.
 int pool_in_front(tdh_net *net, int i, PoolScatter *through) {
@@ -582,7 +589,7 @@ int forward(tdh_net *net, int batch, const float *x, const float *xent_t = nullp
       {
         const PackedFilters wp = packed_filters(L, batch, 0);
         const bool has_wp = static_cast<bool>(wp);
-        const bool fuse = (net->flags & TDH_NET_FUSE_ACT_GRAD) != 0;
+        // (with or without TDH_NET_FUSE_ACT_GRAD, which decides what a train step may leave unwritten)
         auto pointwise = [&](int k) {
           return k < n && net->layers[k].spec.kind == TDH_L_ACT && is_pointwise_act(net->layers[k].spec.act);
         };
@@ -591,13 +598,13 @@ int forward(tdh_net *net, int batch, const float *x, const float *xent_t = nullp
         int last = i;
         float *act_out = nullptr;
         int act_kind   = TDH_ACT_NONE;
-        if (fuse && pointwise(i + 1) && conv_fwd_applies_act(&s.conv, batch, has_wp)) {
+        if (pointwise(i + 1) && conv_fwd_applies_act(&s.conv, batch, has_wp)) {
           last     = i + 1;
           act_out  = net->layers[last].out;
           act_kind = net->layers[last].spec.act;
         }
         PoolFuse pf{nullptr, nullptr, nullptr, TDH_ACT_NONE};
-        if (fuse && !(pointwise(i + 1) && last == i) && last + 1 < n &&
+        if (!(pointwise(i + 1) && last == i) && last + 1 < n &&
             net->layers[last + 1].spec.kind == TDH_L_MAXPOOL &&
             conv_fwd_fuses_pool(&s.conv, &net->layers[last + 1].spec.pool, batch, has_wp)) {
           ++last;
@@ -612,11 +619,10 @@ int forward(tdh_net *net, int batch, const float *x, const float *xent_t = nullp
         }
         {
           // nothing behind the convolution left its kernel and a max-pool reads the result
-          LeaveSplitSum leave(ctx(), fuse && last == i && i + 1 < n &&
-                                         net->layers[i + 1].spec.kind == TDH_L_MAXPOOL);
+          LeaveSplitSum leave(ctx(), last == i && i + 1 < n && net->layers[i + 1].spec.kind == TDH_L_MAXPOOL);
           // (the backward pass reads the outputs of the layers that left the kernel, never the
           // convolution's own: the gradients of the pointwise activations are functions of y)
-          const bool own_out = !(training && ((pf.out && !act_out) ||
+          const bool own_out = !((net->flags & TDH_NET_FUSE_ACT_GRAD) && training && ((pf.out && !act_out) ||
                                               (act_out && conv_fwd_out_optional(&s.conv, batch, has_wp))));
           if (!own_out) net->out_unwritten[i] = 1;
           TDH_TRY(conv2d_fwd(&s.conv, batch, in, L.w, L.b, own_out ? L.out : nullptr, L.tbl_dev, wp, act_out, act_kind,
@@ -644,7 +650,7 @@ int forward(tdh_net *net, int batch, const float *x, const float *xent_t = nullp
                                   tail->target.dx, tail->target.fold));
           if (softmax_behind) ++i;
         } else
-        if ((net->flags & TDH_NET_FUSE_ACT_GRAD) && i + 1 < n && net->layers[i + 1].spec.kind == TDH_L_ACT &&
+        if (i + 1 < n && net->layers[i + 1].spec.kind == TDH_L_ACT &&
             (is_pointwise_act(net->layers[i + 1].spec.act) ||
              (!xent_t && net->layers[i + 1].spec.act == TDH_ACT_SOFTMAX &&
               fc_fwd_direct_applies_softmax(s.fc_in, s.fc_out, batch)))) {
@@ -657,7 +663,7 @@ int forward(tdh_net *net, int batch, const float *x, const float *xent_t = nullp
         }
         break;
       case TDH_L_MAXPOOL:
-        if ((net->flags & TDH_NET_FUSE_ACT_GRAD) && i + 1 < n && net->layers[i + 1].spec.kind == TDH_L_ACT &&
+        if (i + 1 < n && net->layers[i + 1].spec.kind == TDH_L_ACT &&
             is_pointwise_act(net->layers[i + 1].spec.act)) {
           // the activation layer behind the pool leaves the same kernel
           TDH_TRY(maxpool_fwd(&s.pool, batch, in, L.out, L.argmax, net->layers[i + 1].out,
@@ -671,6 +677,16 @@ int forward(tdh_net *net, int batch, const float *x, const float *xent_t = nullp
       case TDH_L_BATCHNORM: {  // batch_normalization_layer.h:127-169
         const int train = !net->test_phase;
         TDH_TRY(ws_begin(batchnorm_workspace_bytes(s.bn_channels, batch)));
+        if (i + 2 < n && block_of_batchnorm(net, i) &&
+            !(i + 3 < n && net->layers[i + 3].spec.kind == TDH_L_ACT &&
+              is_pointwise_act(net->layers[i + 3].spec.act))) {  // (which the pool's own kernel would take along)
+          const tdh_net::Layer &A = net->layers[i + 1], &P = net->layers[i + 2];
+          TDH_TRY(batchnorm_act_pool_fwd(s.bn_channels, s.bn_spatial, batch, s.bn_eps, train, in,
+                                         train ? L.bn_mean_cur : L.bn_mean, train ? L.bn_var_cur : L.bn_var, L.bn_stddev,
+                                         L.out, A.spec.act, A.spec.act_p[0], A.out, &P.spec.pool, P.out, P.argmax));
+          i += 2;
+          break;
+        }
         TDH_TRY(batchnorm_fwd(s.bn_channels, s.bn_spatial, batch, s.bn_eps, train, in,
                               train ? L.bn_mean_cur : L.bn_mean, train ? L.bn_var_cur : L.bn_var, L.bn_stddev,
                               L.out));
@@ -1335,6 +1351,19 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
           net->dx_unwritten[i] = 1;
           through_pool = PoolGather{L.dout, L.argmax};
           through_pool_for = i - 1;
+          break;
+        }
+        if (i >= 2 && block_of_batchnorm(net, i - 2)) {
+          // through the rectifier to the sums of the batch normalization in front of it, and its dX
+          TDH_TRY(finish_split_sum());
+          tdh_net::Layer &A = net->layers[i - 1], &N = net->layers[i - 2];
+          const DxTarget in_front = dx_target(net, i - 2);
+          if (in_front.fold.kind != TDH_ACT_NONE) return set_error(TDH_ERR_INVALID, "batch-norm behind a folded activation");
+          TDH_TRY(ws_begin(batchnorm_workspace_bytes(N.spec.bn_channels, batch)));
+          TDH_TRY(batchnorm_act_pool_bwd(N.spec.bn_channels, N.spec.bn_spatial, batch, N.out, N.bn_stddev, A.spec.act,
+                                         A.spec.act_p[0], A.out, &s.pool, L.dout, L.argmax, A.grad_folded ? nullptr : A.dout,
+                                         N.dout, in_front.dx));
+          i -= 2;
           break;
         }
         TDH_TRY(maxpool_bwd(&s.pool, batch, L.dout, L.argmax, dx, fold, L.out));
