@@ -1315,7 +1315,7 @@ __global__ void __launch_bounds__(256) splitk_reduce_multi_kernel(const ReduceJo
   int j = 0;
   while (j + 1 < jobs.n && jobs.first_block[j + 1] <= static_cast<int>(blockIdx.x)) ++j;
   const ReduceJob &r = jobs.job[j];
-  splitk_reduce_block(r.partial, r.splits, r.M, r.N, r.epi, static_cast<int>(blockIdx.x) - jobs.first_block[j], sm);
+  splitk_reduce_block<false>(r.partial, r.splits, r.M, r.N, r.epi, static_cast<int>(blockIdx.x) - jobs.first_block[j], sm);
 }
 
 static std::vector<ReduceJob> &deferred_reduces() {

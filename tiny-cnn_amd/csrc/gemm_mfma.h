@@ -502,7 +502,7 @@ gemm_mfma_kernel(const AOp a_op, const BOp b_op, const Epi epi, const int M, con
 constexpr int REDUCE_OUTPUTS = 32;
 constexpr int REDUCE_GROUPS  = 8;
 
-template <class Epi>
+template <bool MANY, class Epi>
 __device__ __forceinline__ void splitk_reduce_block(const float *__restrict__ partial, const int splits,
                                                     const int M, const int N, const Epi &epi,
                                                     const int block, float (*sm)[REDUCE_OUTPUTS]) {
@@ -512,8 +512,19 @@ __device__ __forceinline__ void splitk_reduce_block(const float *__restrict__ pa
   const size_t mn = static_cast<size_t>(M) * N;
   float s = 0.0f;
   if (idx < M * N) {
-    // eight slices per trip: the loads are issued together, the adds keep slice order
+    // Eight slices per trip: the loads are issued together, the adds keep slice order. Very many slices of few sums
+    // are bound by the trips alone: thirty-two (1040 slices of 648 sums 9.2 us / 6.3). MANY: not in the launch of several layers' sums,
+    // which the registers cost more (256 slices of 18432 sums 4.5 / 4.8).
+    // What is left goes in one trip as well (a slice past the last repeats it and is dropped).
     int z = g;
+    if (MANY && splits >= 64 * REDUCE_GROUPS)
+      for (; z + 31 * REDUCE_GROUPS < splits; z += 32 * REDUCE_GROUPS) {
+        float v[32];
+#pragma unroll
+        for (int u = 0; u < 32; ++u) v[u] = partial[(z + u * REDUCE_GROUPS) * mn + idx];
+#pragma unroll
+        for (int u = 0; u < 32; ++u) s += v[u];
+      }
     for (; z + 7 * REDUCE_GROUPS < splits; z += 8 * REDUCE_GROUPS) {
       float v[8];
 #pragma unroll
@@ -521,7 +532,15 @@ __device__ __forceinline__ void splitk_reduce_block(const float *__restrict__ pa
 #pragma unroll
       for (int u = 0; u < 8; ++u) s += v[u];
     }
-    for (; z < splits; z += REDUCE_GROUPS) s += partial[z * mn + idx];
+    if (MANY && z < splits) {
+      float v[7];
+#pragma unroll
+      for (int u = 0; u < 7; ++u) v[u] = partial[min(z + u * REDUCE_GROUPS, splits - 1) * mn + idx];
+#pragma unroll
+      for (int u = 0; u < 7; ++u) s = z + u * REDUCE_GROUPS < splits ? s + v[u] : s;
+    }
+    if (!MANY)
+      for (; z < splits; z += REDUCE_GROUPS) s += partial[z * mn + idx];
   }
   sm[g][o] = s;
   __syncthreads();
@@ -539,7 +558,7 @@ __global__ void __launch_bounds__(256)
 splitk_reduce_kernel(const float *__restrict__ partial, const int splits, const int M, const int N,
                      const Epi epi) {
   __shared__ float sm[REDUCE_GROUPS][REDUCE_OUTPUTS];
-  splitk_reduce_block(partial, splits, M, N, epi, blockIdx.x, sm);
+  splitk_reduce_block<true>(partial, splits, M, N, epi, blockIdx.x, sm);
 }
 
 // The same sums for a large result (N a multiple of four): a thread owns four neighbouring
