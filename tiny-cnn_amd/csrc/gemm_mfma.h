@@ -513,11 +513,11 @@ __device__ __forceinline__ void splitk_reduce_block(const float *__restrict__ pa
   float s = 0.0f;
   if (idx < M * N) {
     // Eight slices per trip: the loads are issued together, the adds keep slice order. Very many slices of few sums
-    // are bound by the trips alone: thirty-two (1040 slices of 648 sums 9.2 us / 6.3). MANY: not in the launch of several layers' sums,
-    // which the registers cost more (256 slices of 18432 sums 4.5 / 4.8).
-    // What is left goes in one trip as well (a slice past the last repeats it and is dropped).
+    // are bound by the trips alone: thirty-two, and what is left in one (a slice past the last repeats it and is
+    // dropped): 1040 slices of 648 sums 9.2 us / 6.3. MANY: an instance of its own, because its registers cost the
+    // others more (5 slices of 375436 sums 7.4 / 11.1).
     int z = g;
-    if (MANY && splits >= 64 * REDUCE_GROUPS)
+    if (MANY)
       for (; z + 31 * REDUCE_GROUPS < splits; z += 32 * REDUCE_GROUPS) {
         float v[32];
 #pragma unroll
@@ -538,9 +538,9 @@ __device__ __forceinline__ void splitk_reduce_block(const float *__restrict__ pa
       for (int u = 0; u < 7; ++u) v[u] = partial[min(z + u * REDUCE_GROUPS, splits - 1) * mn + idx];
 #pragma unroll
       for (int u = 0; u < 7; ++u) s = z + u * REDUCE_GROUPS < splits ? s + v[u] : s;
+      z = splits;
     }
-    if (!MANY)
-      for (; z < splits; z += REDUCE_GROUPS) s += partial[z * mn + idx];
+    for (; z < splits; z += REDUCE_GROUPS) s += partial[z * mn + idx];
   }
   sm[g][o] = s;
   __syncthreads();
@@ -553,12 +553,12 @@ __device__ __forceinline__ void splitk_reduce_block(const float *__restrict__ pa
   }
 }
 
-template <class Epi>
+template <bool MANY, class Epi>
 __global__ void __launch_bounds__(256)
 splitk_reduce_kernel(const float *__restrict__ partial, const int splits, const int M, const int N,
                      const Epi epi) {
   __shared__ float sm[REDUCE_GROUPS][REDUCE_OUTPUTS];
-  splitk_reduce_block<true>(partial, splits, M, N, epi, blockIdx.x, sm);
+  splitk_reduce_block<MANY>(partial, splits, M, N, epi, blockIdx.x, sm);
 }
 
 // The same sums for a large result (N a multiple of four): a thread owns four neighbouring
@@ -740,8 +740,11 @@ int launch_splitk_reduce(const float *partial, int splits, int M, int N, const E
   if (N % 4 == 0 && static_cast<long>(M) * N >= REDUCE_WIDE_MIN && (reinterpret_cast<uintptr_t>(partial) & 15u) == 0)
     TDH_LAUNCH((splitk_reduce_wide_kernel<Epi>), dim3(static_cast<unsigned>(ceil_div_sz(static_cast<size_t>(M) * N / 4, 256))),
                dim3(256), 0, ctx().stream, partial, splits, M, N, epi);
+  else if (splits >= 64 * REDUCE_GROUPS)
+    TDH_LAUNCH((splitk_reduce_kernel<true, Epi>), dim3(ceil_div(M * N, REDUCE_OUTPUTS)), dim3(256), 0,
+               ctx().stream, partial, splits, M, N, epi);
   else
-    TDH_LAUNCH((splitk_reduce_kernel<Epi>), dim3(ceil_div(M * N, REDUCE_OUTPUTS)), dim3(256), 0,
+    TDH_LAUNCH((splitk_reduce_kernel<false, Epi>), dim3(ceil_div(M * N, REDUCE_OUTPUTS)), dim3(256), 0,
                ctx().stream, partial, splits, M, N, epi);
   TDH_LAUNCH_CHECK();
   return TDH_OK;
