@@ -381,6 +381,7 @@ bool conv_bwd_pairs(const tdh_conv_desc *d, int batch, const float *x = nullptr,
 // the forward kernel of this convolution can also compute the max-pool layer `pool` behind it
 bool conv_fwd_fuses_pool(const tdh_conv_desc *d, const tdh_pool_desc *pool, int batch, bool prepacked);
 // ... and the pointwise activation of this kind behind that pool
+bool conv_fwd_packs_along(const tdh_conv_desc *d, int batch);
 bool conv_fwd_pool_applies_act(const tdh_conv_desc *d, int batch, bool prepacked, int act_kind);
 // the forward kernel of this layer can leave `y` out (null) when it writes the activation layer
 // or the pool behind the convolution itself
@@ -421,6 +422,11 @@ struct PackJob {
 };
 constexpr int CONV_PACK_JOBS = 16;
 int conv_pack_filters(const PackJob *jobs, int n);
+// The same, left to the next launch of a first convolution (conv_fwd_small.hip), which takes up to CONV_PACK_JOBS along:
+// in front of whoever reads them, conv_pack_finish launches what is left.
+void conv_pack_leave(const PackJob *jobs, int n);
+bool conv_packs_left();
+int conv_pack_finish();
 // (conv.hip) the kind that the backward pass of this layer reads when dX is computed together with dW
 // (x, dy: as in conv_bwd_pairs)
 int conv_bwd_packed_kind(const tdh_conv_desc *d, int batch, const float *x = nullptr, const float *dy = nullptr);

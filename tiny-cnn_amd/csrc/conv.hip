@@ -1431,6 +1431,12 @@ bool conv_fwd_out_optional(const tdh_conv_desc *d, int batch, bool prepacked) {
          conv_s1_single_pass(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
 }
 
+// this layer's forward kernel takes filters to pack along (conv_pack_leave)
+bool conv_fwd_packs_along(const tdh_conv_desc *d, int batch) {
+  const ConvGeom g = make_geom(d);
+  return !fwd_direct_applies(g, batch) && fwd_small_applies(g, batch);
+}
+
 bool conv_fwd_pool_applies_act(const tdh_conv_desc *d, int batch, bool prepacked, int act_kind) {
   const ConvGeom g = make_geom(d);
   // the direct and the first-layer kernel apply any pointwise kind, the stride-1 kernel relu

@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <cfloat>
 
+#include "conv_pack.h"
 #include "gemm_mfma.h"
 
 namespace tdh {
@@ -42,7 +43,31 @@ struct FwdSmallArgs {
   int rows_in, pitch, plane;
   int crs, x_floats;
   FastDiv div_pitch, div_rows_in, div_col_tiles;
+  int batch, workgroups;     // of the convolution
+  int pack_threads;
 };
+
+// Workgroups in front of the convolution's own pack filters that later layers read: in a net whose
+// weights may have been written since the last call that is a launch less. A packing workgroup holds as many registers as
+// one of the convolution, two to a CU, so it is no more than half hidden: first convolution of the CIFAR-10-shape net at
+// batch 128 14.9 us and the packing 5.0 in launches of their own, together 18.9 (packing behind the
+// convolution 19.5), the step 161.6 / 160.6, inference of 1000 images 245 / 234. No more
+// than 192: a thread of them writes several pieces rather than 500 workgroups (23 us).
+constexpr int FWD_SMALL_PACKERS = 192;
+struct NoPacks {};
+template <class Packs>
+__device__ __forceinline__ bool fwd_small_packs(const FwdSmallArgs &a, const Packs &packs) {
+  if constexpr (std::is_same_v<Packs, PackJobs>) {
+    if (blockIdx.x >= gridDim.x - a.workgroups) return false;
+    // (whole pieces of a job's 256 threads: of three waves two work)
+    const int threads = blockDim.x < 256 ? 128 : 256;
+    if (static_cast<int>(threadIdx.x) >= threads) return true;
+    const int step = (gridDim.x - a.workgroups) * threads;
+    for (int t = blockIdx.x * threads + threadIdx.x; t < a.pack_threads; t += step) pack_any(packs, t);
+    return true;
+  }
+  return false;
+}
 
 // the value of lane l ^ 1 (a swap inside lane pairs, done by the DPP path of a move)
 __device__ __forceinline__ float lane_xor1(const float v) {
@@ -151,18 +176,18 @@ __device__ __forceinline__ void fwd_small_stage(const FwdSmallArgs &a, float *xs
   }
 }
 
-template <int NS>
-__global__ void __launch_bounds__(256, 2) conv_fwd_small_kernel(const FwdSmallArgs a) {
+template <int NS, class Packs>
+__global__ void __launch_bounds__(256, 2) conv_fwd_small_kernel(const FwdSmallArgs a, const Packs packs) {
   extern __shared__ __align__(16) float lds[];
+  if (fwd_small_packs(a, packs)) return;
   float *xs = lds;
   float *ws = lds + a.x_floats;  // [32][crs], rows past Cout are zero
   float *bs = ws + 32 * a.crs;   // [32] bias, zero past Cout or without bias
   int *offs = reinterpret_cast<int *>(bs + 32);  // [2*NS] patch offset of k (0 past K)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // (an image's bands share rows: they go to one XCD)
-  const int wg = xcd_compact_id(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z),
-                                gridDim.x * gridDim.y * gridDim.z);
-  const int bandi = wg % gridDim.x, img = (wg / gridDim.x) % gridDim.y, co0 = (wg / (gridDim.x * gridDim.y)) * 32;
+  const int wg = xcd_compact_id(blockIdx.x - (gridDim.x - a.workgroups), a.workgroups);
+  const int bandi = wg % a.bands, img = (wg / a.bands) % a.batch, co0 = (wg / (a.bands * a.batch)) * 32;
   const int oy0 = bandi * a.band;
   const int nthr = blockDim.x;  // one wave per tile of the band, two to four waves
 
@@ -290,18 +315,18 @@ __global__ void __launch_bounds__(256, 2) conv_fwd_small_kernel(const FwdSmallAr
 // everything that depends on the tile is kept in scalar registers (the wave index is read from
 // the first lane for that), a lane adds one offset of its own that is computed once, and no
 // store has a condition.
-template <int NS>
-__global__ void __launch_bounds__(256, 2) conv_fwd_small_full_kernel(const FwdSmallArgs a) {
+template <int NS, class Packs>
+__global__ void __launch_bounds__(256, 2) conv_fwd_small_full_kernel(const FwdSmallArgs a, const Packs packs) {
   extern __shared__ __align__(16) float lds[];
+  if (fwd_small_packs(a, packs)) return;
   float *xs = lds;
   float *ws = lds + a.x_floats;
   float *bs = ws + 32 * a.crs;
   int *offs = reinterpret_cast<int *>(bs + 32);
   const int tid = threadIdx.x, lane = tid & 63;
   // (an image's bands share rows: they go to one XCD)
-  const int wg = xcd_compact_id(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z),
-                                gridDim.x * gridDim.y * gridDim.z);
-  const int bandi = wg % gridDim.x, img = (wg / gridDim.x) % gridDim.y, co0 = (wg / (gridDim.x * gridDim.y)) * 32;
+  const int wg = xcd_compact_id(blockIdx.x - (gridDim.x - a.workgroups), a.workgroups);
+  const int bandi = wg % a.bands, img = (wg / a.bands) % a.batch, co0 = (wg / (a.bands * a.batch)) * 32;
   const int oy0 = bandi * a.band;
   const int nthr = blockDim.x;
   fwd_small_stage<NS>(a, xs, ws, bs, offs, img, co0, oy0, tid, nthr);
@@ -417,7 +442,6 @@ struct FwdSmallPlan {
   FwdSmallArgs a;
   int ns;  // k-steps, rounded up to the next instantiated count
   size_t lds_bytes;
-  dim3 grid;
   bool ok;
 };
 
@@ -469,28 +493,40 @@ FwdSmallPlan make_fwd_small_plan(int batch, int C, int Kc, int H, int W, int OH,
   a.div_rows_in   = FastDiv(a.rows_in);
   a.div_col_tiles = FastDiv(a.col_tiles);
   p.lds_bytes = lds_floats(best) * sizeof(float);
-  p.grid      = dim3(a.bands, batch, co_tiles);
+  const long workgroups = static_cast<long>(a.bands) * batch * co_tiles;
+  if (workgroups > (1L << 30)) return p;
+  a.batch      = batch;
+  a.workgroups = static_cast<int>(workgroups);
   p.ok        = true;
   return p;
 }
 
-template <int NS>
-int launch_fwd_small(const FwdSmallPlan &p) {
+template <int NS, class Packs>
+int launch_fwd_small(const FwdSmallPlan &p, const Packs &packs, int pack_blocks) {
   const int tiles = (p.a.band / 2) * p.a.col_tiles;
   const FwdSmallArgs &a = p.a;
   const bool full = a.OH % a.band == 0 && a.band % 2 == 0 && a.OW % 32 == 0 && a.Kc % 32 == 0 && !a.act_out &&
                     (a.pool_act_kind == TDH_ACT_RELU || a.pool_act_kind == TDH_ACT_NONE || !a.pool_act_out) &&
                     static_cast<long long>(a.Kc) * a.OH * a.OW < (1LL << 30);
-  if (full) {
-    TDH_LAUNCH((conv_fwd_small_full_kernel<NS>), p.grid, dim3(64 * std::min(4, std::max(2, tiles))), p.lds_bytes,
-               ctx().stream, p.a);
-    TDH_LAUNCH_CHECK();
-    return TDH_OK;
-  }
-  TDH_LAUNCH((conv_fwd_small_kernel<NS>), p.grid, dim3(64 * std::min(4, std::max(2, tiles))), p.lds_bytes,
-             ctx().stream, p.a);
+  const dim3 block(64 * std::min(4, std::max(2, tiles)));
+  const dim3 grid(a.workgroups + std::min(block.x < 256 ? 2 * pack_blocks : pack_blocks, FWD_SMALL_PACKERS));
+  if (full)
+    TDH_LAUNCH((conv_fwd_small_full_kernel<NS, Packs>), grid, block, p.lds_bytes, ctx().stream, p.a, packs);
+  else
+    TDH_LAUNCH((conv_fwd_small_kernel<NS, Packs>), grid, block, p.lds_bytes, ctx().stream, p.a, packs);
   TDH_LAUNCH_CHECK();
   return TDH_OK;
+}
+template <class Packs>
+int launch_fwd_small_ns(const FwdSmallPlan &p, const Packs &packs, int pack_blocks) {
+  switch (p.ns) {
+    case 8: return launch_fwd_small<8>(p, packs, pack_blocks);
+    case 16: return launch_fwd_small<16>(p, packs, pack_blocks);
+    case 24: return launch_fwd_small<24>(p, packs, pack_blocks);
+    case 32: return launch_fwd_small<32>(p, packs, pack_blocks);
+    case 40: return launch_fwd_small<40>(p, packs, pack_blocks);
+    default: return launch_fwd_small<48>(p, packs, pack_blocks);
+  }
 }
 
 }  // namespace
@@ -518,14 +554,16 @@ int conv_fwd_small_run(int batch, int C, int Kc, const float *x, const float *w,
     p.a.pool_act_kind = pool->act_kind;
   }
   ProfScope prof(pool ? "conv_fwd_small_pool" : "conv_fwd_small", Kc, batch * OH * OW, p.a.crs);
-  switch (p.ns) {
-    case 8: return launch_fwd_small<8>(p);
-    case 16: return launch_fwd_small<16>(p);
-    case 24: return launch_fwd_small<24>(p);
-    case 32: return launch_fwd_small<32>(p);
-    case 40: return launch_fwd_small<40>(p);
-    default: return launch_fwd_small<48>(p);
-  }
+  std::vector<PackJob> jobs = take_left_packs();
+  if (jobs.empty()) return launch_fwd_small_ns(p, NoPacks(), 0);
+  PackJobs packs;
+  int blocks   = 0;
+  double bytes = 0.0;
+  const int here = std::min<int>(CONV_PACK_JOBS, static_cast<int>(jobs.size()));
+  plan_packs(jobs.data(), here, &packs, &blocks, &bytes);
+  p.a.pack_threads = 256 * blocks;
+  conv_pack_leave(jobs.data() + here, static_cast<int>(jobs.size()) - here);
+  return launch_fwd_small_ns(p, packs, blocks);
 }
 
 }  // namespace tdh

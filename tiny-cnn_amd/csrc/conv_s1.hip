@@ -1,10 +1,10 @@
 // conv_s1.hip — host side of the stride-1 convolution (forward and dX) on the LDS-halo MFMA
 // kernel of conv_s1_inst.hip: tile choice, filter repacking, split-K reduction.
 #include <algorithm>
-#include <climits>
+#include <utility>
+#include <vector>
 
-#include "conv_s1.h"
-#include "split_bf16.h"
+#include "conv_pack.h"
 
 namespace tdh {
 
@@ -39,83 +39,7 @@ int launch_split_reduce(const SplitSum &sum, int plane, float *act_out, int act_
   return TDH_OK;
 }
 
-// The filters of several layers in one launch: job k owns the workgroups [first_block[k],
-// first_block[k+1]). A launch of its own in every pass whose caller may have written the weights: bound by
-// latency, so nothing is divided and a thread's loads are asked for together. us for 5x5, 32 -> 32 and
-// 32 -> 64 channels, both directions' copies: one thread per weight with scattered stores 5.9.
-// (A single job goes as a kernel of its own, with a tenth of the arguments and no search.)
-struct PackPlan : PackJob {
-  FastDiv div_rs, div_m, div_kc;
-};
-struct PackJobs {
-  PackPlan job[CONV_PACK_JOBS];
-  int first_block[CONV_PACK_JOBS];   // (past the last job: INT_MAX)
-};
-
-// wp[t][kc][m]: forward (flip = 0): kc = ci, m = co, t as is; dX (flip = 1): kc = co, m = ci,
-// tap reversed. An optional connection table zeroes unconnected (ci, co) pairs. e: element of wp.
-__device__ __forceinline__ void pack_f32(const PackPlan &j, const int e) {
-  const int rs = j.R * j.S;
-  if (e >= j.C * j.Kc * rs) return;
-  uint32_t rest, m, t, kc;
-  j.div_m.divmod(e, rest, m);
-  j.div_kc.divmod(rest, t, kc);
-  const int co = j.flip ? kc : m, ci = j.flip ? m : kc;
-  const float v = j.w[(static_cast<size_t>(co) * j.C + ci) * rs + (j.flip ? rs - 1 - t : t)];
-  static_cast<float *>(j.wp)[e] = j.tbl && !j.tbl[ci * j.Kc + co] ? 0.0f : v;
-}
-
-// The filters of the three-part kernel: unit ((g*rs + t)*3 + part)*2 + half)*mc_pad + m holds the
-// parts of channels 16g + 8*half .. +7 of row m (zero beyond the tensor), with the sign of step
-// g*rs + t. A thread writes the
-// three units of eight channels.
-__device__ __forceinline__ void pack_x3(const PackPlan &j, const int e) {
-  const int rs = j.R * j.S, KC = j.flip ? j.Kc : j.C, MC = j.flip ? j.C : j.Kc, mc_pad = j.div_m.d;
-  uint32_t rest, m, g, t;
-  j.div_m.divmod(e, rest, m);
-  const int half = rest & 1;
-  j.div_rs.divmod(rest >> 1, g, t);
-  if (static_cast<int>(g) * 16 >= KC) return;
-  const int step = (j.flip ? j.C : 1) * rs, kc0 = 16 * g + 8 * half;   // floats from one channel to the next
-  const float *src = j.w + static_cast<size_t>(j.flip ? min(static_cast<int>(m), MC - 1) : min(static_cast<int>(m), MC - 1) * j.C) * rs +
-                     (j.flip ? rs - 1 - t : t);
-  float v[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) v[k] = src[static_cast<size_t>(min(kc0 + k, KC - 1)) * step];
-  const float sign = X3_SCALE * x3_sign(g * rs + t);
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int kc = kc0 + k, co = j.flip ? kc : m, ci = j.flip ? m : kc;
-    const bool in = kc < KC && static_cast<int>(m) < MC && (!j.tbl || j.tbl[ci * j.Kc + co]);
-    v[k] = in ? sign * v[k] : 0.0f;
-  }
-  uint32_t part[X3_PARTS][4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    uint32_t p3[X3_PARTS];
-    split_pair(v[2 * k], v[2 * k + 1], p3);
-#pragma unroll
-    for (int p = 0; p < X3_PARTS; ++p) part[p][k] = p3[p];
-  }
-  uint4 *wp = static_cast<uint4 *>(j.wp);
-#pragma unroll
-  for (int p = 0; p < X3_PARTS; ++p)
-    wp[((static_cast<size_t>(g * rs + t) * X3_PARTS + p) * 2 + half) * mc_pad + m] =
-      make_uint4(part[p][0], part[p][1], part[p][2], part[p][3]);
-}
-
-__device__ __forceinline__ void pack_one(const PackPlan &j, const int e) {
-  if (j.kind == CONV_PACK_X3)
-    pack_x3(j, e);
-  else
-    pack_f32(j, e);
-}
-__global__ void __launch_bounds__(256) pack_filters_kernel(const PackJobs jobs) {
-  int k = 0;
-#pragma unroll
-  for (int i = 1; i < CONV_PACK_JOBS; ++i) k += jobs.first_block[i] <= static_cast<int>(blockIdx.x) ? 1 : 0;
-  pack_one(jobs.job[k], (static_cast<int>(blockIdx.x) - jobs.first_block[k]) * 256 + threadIdx.x);
-}
+__global__ void __launch_bounds__(256) pack_filters_kernel(const PackJobs jobs) { pack_any(jobs, blockIdx.x * 256 + threadIdx.x); }
 __global__ void __launch_bounds__(256) pack_filter_kernel(const PackPlan j) { pack_one(j, blockIdx.x * 256 + threadIdx.x); }
 
 int pow2_ceil(int v) {
@@ -317,25 +241,31 @@ size_t conv_s1_run_workspace_bytes(int R, int S, int batch, int C, int Kc, int f
   return p.ok ? plan_workspace_bytes(p, R * S) : 0;
 }
 
+void plan_packs(const PackJob *jobs, int n, PackJobs *p, int *blocks, double *bytes) {
+  *blocks = 0;
+  *bytes  = 0.0;
+  for (int k = 0; k < CONV_PACK_JOBS; ++k) {
+    p->first_block[k] = k < n ? *blocks : INT_MAX;
+    if (k >= n) continue;
+    PackPlan &j = p->job[k];
+    static_cast<PackJob &>(j) = jobs[k];
+    const bool x3 = j.kind == CONV_PACK_X3;
+    const int rs = j.R * j.S, KC = j.flip ? j.Kc : j.C, MC = j.flip ? j.C : j.Kc;
+    j.div_rs = FastDiv(rs);
+    j.div_m  = FastDiv(x3 ? x3_mc_pad(MC) : MC);
+    j.div_kc = FastDiv(KC);
+    *blocks += ceil_div(x3 ? ceil_div(KC, 16) * rs * 2 * x3_mc_pad(MC) : rs * KC * MC, 256);
+    *bytes += (x3 ? 10.0 : 8.0) * rs * KC * MC;
+  }
+}
+
 int conv_pack_filters(const PackJob *jobs, int n) {
   for (int at = 0; at < n; at += CONV_PACK_JOBS) {
     PackJobs p;
     const int here = std::min(CONV_PACK_JOBS, n - at);
-    int blocks     = 0;
-    double bytes   = 0.0;
-    for (int k = 0; k < CONV_PACK_JOBS; ++k) {
-      p.first_block[k] = k < here ? blocks : INT_MAX;
-      if (k >= here) continue;
-      PackPlan &j = p.job[k];
-      static_cast<PackJob &>(j) = jobs[at + k];
-      const bool x3 = j.kind == CONV_PACK_X3;
-      const int rs = j.R * j.S, KC = j.flip ? j.Kc : j.C, MC = j.flip ? j.C : j.Kc;
-      j.div_rs = FastDiv(rs);
-      j.div_m  = FastDiv(x3 ? x3_mc_pad(MC) : MC);
-      j.div_kc = FastDiv(KC);
-      blocks += ceil_div(x3 ? ceil_div(KC, 16) * rs * 2 * x3_mc_pad(MC) : rs * KC * MC, 256);
-      bytes += (x3 ? 10.0 : 8.0) * rs * KC * MC;
-    }
+    int blocks;
+    double bytes;
+    plan_packs(jobs + at, here, &p, &blocks, &bytes);
     ProfScope prof("conv_repack_weights", bytes, WORK_BYTE);
     if (here == 1)
       TDH_LAUNCH(pack_filter_kernel, dim3(blocks), dim3(256), 0, ctx().stream, p.job[0]);
@@ -344,6 +274,16 @@ int conv_pack_filters(const PackJob *jobs, int n) {
     TDH_LAUNCH_CHECK();
   }
   return TDH_OK;
+}
+
+// Jobs that the next launch of a first convolution takes along.
+static thread_local std::vector<PackJob> left_packs;
+void conv_pack_leave(const PackJob *jobs, int n) { left_packs.assign(jobs, jobs + n); }
+bool conv_packs_left() { return !left_packs.empty(); }
+std::vector<PackJob> take_left_packs() { return std::exchange(left_packs, {}); }
+int conv_pack_finish() {
+  const std::vector<PackJob> jobs = take_left_packs();
+  return conv_pack_filters(jobs.data(), static_cast<int>(jobs.size()));
 }
 
 // Runs out = conv(in, repack(w)) (+ bias) (* act'(y)); the caller has checked applicability

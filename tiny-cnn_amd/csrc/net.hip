@@ -524,7 +524,8 @@ const std::vector<uint8_t> &copies_read(tdh_net *net, int batch, const float *x,
 }
 
 // Packs the copies that the pass reads and that do not hold the weights as they are, in one launch.
-int pack_copies(tdh_net *net, int batch, const float *x, bool training) {
+// leave: a forward pass follows, whose first layer's kernel takes the jobs along if it can.
+int pack_copies(tdh_net *net, int batch, const float *x, bool training, bool leave) {
   const std::vector<uint8_t> &reads = copies_read(net, batch, x, training);
   std::vector<PackJob> jobs;
   for (size_t i = 0; i < net->layers.size(); ++i) {
@@ -535,6 +536,13 @@ int pack_copies(tdh_net *net, int batch, const float *x, bool training) {
       jobs.push_back(PackJob{L.w, d.tbl ? L.tbl_dev : nullptr, L.copy[c], d.in_c, d.out_c, d.k_h, d.k_w,
                              c >= 2 ? CONV_PACK_X3 : CONV_PACK_F32, c & 1});
       L.current[c] = true;
+    }
+  }
+  if (leave && !jobs.empty() && net->layers[0].spec.kind == TDH_L_CONV && !reads[0]) {
+    const KeepF32 keep(training);
+    if (conv_fwd_packs_along(&net->layers[0].spec.conv, batch)) {
+      conv_pack_leave(jobs.data(), static_cast<int>(jobs.size()));
+      return TDH_OK;
     }
   }
   return conv_pack_filters(jobs.data(), static_cast<int>(jobs.size()));
@@ -580,6 +588,14 @@ int forward(tdh_net *net, int batch, const float *x, const float *xent_t = nullp
   const float *in = x;
   const int n     = static_cast<int>(net->layers.size());
   net->out_unwritten.assign(n, 0);
+  struct Packs {   // what the first layer did not take along although it could have (an error in between): not packed
+    tdh_net *net;
+    ~Packs() {
+      if (!conv_packs_left()) return;
+      conv_pack_leave(nullptr, 0);
+      for (tdh_net::Layer &L : net->layers) forget_copies(L);
+    }
+  } packs{net};
   for (int i = 0; i < n; ++i) {
     tdh_net::Layer &L  = net->layers[i];
     const tdh_layer &s = L.spec;
@@ -628,6 +644,7 @@ int forward(tdh_net *net, int batch, const float *x, const float *xent_t = nullp
           TDH_TRY(conv2d_fwd(&s.conv, batch, in, L.w, L.b, own_out ? L.out : nullptr, L.tbl_dev, wp, act_out, act_kind,
                              pf.out ? &pf : nullptr));
         }
+        if (conv_packs_left()) TDH_TRY(conv_pack_finish());   // (more jobs than a launch takes)
         i = last;
       }
         break;
@@ -1047,7 +1064,7 @@ int tdh_net_forward(tdh_net *net, int batch, const float *x) {
   TDH_REQUIRE_INIT();
   TDH_CHECK_ARG(net && x && batch > 0 && batch <= net->max_batch, "tdh_net_forward: bad argument");
   distrust_copies(net);
-  TDH_TRY(pack_copies(net, batch, x, /*training=*/false));
+  TDH_TRY(pack_copies(net, batch, x, /*training=*/false, /*leave=*/true));
   return forward(net, batch, x);
 }
 
@@ -1094,7 +1111,7 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
     after_update(net, keep_packs);
     return post_update(net);
   }
-  TDH_TRY(pack_copies(net, batch, x, /*training=*/true));
+  TDH_TRY(pack_copies(net, batch, x, /*training=*/true, /*leave=*/true));
   Context &c = ctx();
   struct KeepScratch {  // hands out disjoint scratch pieces for the whole backward pass
     Context &c;
@@ -1474,7 +1491,7 @@ static int train_steps(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, int
   key.test_phase = net->test_phase;
   key.packs      = net->weights_out && !tiny;
   if (!key.packs && !tiny)
-    for (int s = 0; s < n_steps; ++s) TDH_TRY(pack_copies(net, batch, xs[s], /*training=*/true));
+    for (int s = 0; s < n_steps; ++s) TDH_TRY(pack_copies(net, batch, xs[s], /*training=*/true, /*leave=*/false));
   // (only steps that advance the powers take turns between the two buffers)
   const bool powers_move = opt && do_update && (opt->kind == TDH_OPT_ADAM || opt->kind == TDH_OPT_ADAMAX);
   key.powers_at = powers_move ? net->powers_at : 0;
