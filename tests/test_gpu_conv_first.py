@@ -1,0 +1,100 @@
+"""A net's first convolution with what leaves its kernel (activation, 2x2 max-pool, the activation behind that, and the
+filters of later layers it packs along), against the operators of the layers: the same bits."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def conv64(x, w, b, k, stride, pad):
+    batch, ci, h, wd = x.shape
+    x = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (pad, pad), (pad, pad)))
+    oh, ow = (h + 2 * pad - k) // stride + 1, (wd + 2 * pad - k) // stride + 1
+    y = np.zeros((batch, w.shape[0], oh, ow)) + b.astype(np.float64)[None, :, None, None]
+    for r in range(k):
+        for s in range(k):
+            part = x[:, :, r:r + stride * oh:stride, s:s + stride * ow:stride]
+            y += np.tensordot(w[:, :, r, s].astype(np.float64), part, (1, 1)).transpose(1, 0, 2, 3)
+    return y
+
+
+@pytest.mark.parametrize("between,behind", [(None, "relu"), ("relu", None), (None, "tanh"), ("sigmoid", "relu"), ("relu", "tanh")])
+@pytest.mark.parametrize("w,h,ci,k,co,batch", [
+    (32, 32, 3, 5, 32, 128),    # whole tiles
+    (64, 6, 1, 3, 64, 200),     # two column tiles, a last band of fewer rows
+    (34, 30, 3, 5, 33, 90),     # a column tile of two, a channel tile of one
+    (30, 14, 2, 3, 36, 260),
+    (14, 12, 3, 5, 5, 300),
+    (66, 34, 6, 4, 4, 64),      # all 96 taps
+])
+def test_first_convolution_is_its_layers(T, w, h, ci, k, co, batch, between, behind):
+    rng = np.random.default_rng(61)
+    same = k % 2 == 1
+    ow, oh = (w, h) if same else (w - k + 1, h - k + 1)
+    if ow % 2 or oh % 2:
+        w, h, ow, oh = w + ow % 2, h + oh % 2, ow + ow % 2, oh + oh % 2
+    d = T.conv_desc(w, h, ci, k, k, co, pad_same=same)
+    x = rng.standard_normal((batch, ci, h, w)).astype(np.float32)
+    wt = rng.uniform(-0.3, 0.3, (co, ci, k, k)).astype(np.float32)
+    b = rng.standard_normal(co).astype(np.float32)
+    xd, n = T.to_device(x), co * ow * oh
+    y, a, p, q = T.DevBuf((batch, n)), T.DevBuf((batch, n)), T.DevBuf((batch, n // 4)), T.DevBuf((batch, n // 4))
+    argmax = T.DevBuf((batch, n // 4), np.int32)
+    T.profile_begin()
+    T.conv2d_fwd(d, batch, xd, T.to_device(wt), T.to_device(b), y)
+    assert any(r["tag"].startswith("conv_fwd_small ") for r in T.profile_end())
+    ref = conv64(x, wt, b, k, 1, k // 2 if same else 0)
+    bound = 2.0 ** -24 * (ci * k * k + 2) * (np.abs(x).max() * np.abs(wt).reshape(co, -1).sum(1) + np.abs(b))
+    assert (np.abs(y.numpy().reshape(ref.shape) - ref) <= bound[None, :, None, None]).all()
+
+    layers, want = [T.L_conv(w, h, ci, k, co, pad_same=same)], [y]
+    if between:
+        T.act_fwd(between, batch, n, y, a)
+        layers, want = layers + [T.L_act(between)], want + [a]
+    T.maxpool_fwd(T.pool_desc(ow, oh, co, 2, stride_w=2, stride_h=2), batch, want[-1], p, argmax)
+    layers, want = layers + [T.L_maxpool(ow, oh, co, 2, 2)], want + [p]
+    if behind:
+        T.act_fwd(behind, batch, n // 4, p, q)
+        layers, want = layers + [T.L_act(behind)], want + [q]
+    net = T.Net(layers, batch, 0)
+    net.set_param(0, 0, wt.ravel())
+    net.set_param(0, 1, b)
+    net.forward(batch, xd)
+    for i, buf in enumerate(want):
+        assert np.array_equal(net.layer_out(i, batch).ravel(), buf.numpy().ravel()), i
+    assert np.array_equal(net.layer_argmax(len(layers) - (2 if behind else 1), batch).ravel(), argmax.numpy().ravel())
+    net.close()
+
+
+@pytest.mark.parametrize("convs", [1, 2, 11])    # (one job, several, more than a launch takes along)
+def test_filters_packed_along_are_those_written_last(T, convs):
+    rng = np.random.default_rng(62)
+    batch, hw, c = 64, 16, 32
+    layers = [T.L_conv(hw, hw, 3, 5, c, pad_same=True), T.L_act("relu")]
+    layers += [T.L_conv(hw, hw, c, 3, c, pad_same=True) for _ in range(convs)]
+    x, t = T.to_device(rng.standard_normal((batch, 3 * hw * hw)).astype(np.float32)), T.DevBuf((batch, c * hw * hw), zero=True)
+    weights = [[rng.uniform(-0.1, 0.1, c * (3 * 25 if i == 0 else 9 * c)).astype(np.float32) for i in range(convs + 1)] for _ in (0, 1)]
+    at = [0] + list(range(2, convs + 2))
+
+    def results(net):
+        net.forward(batch, x)
+        out = [net.layer_out(len(layers) - 1, batch).copy()]
+        net.clear_grads()
+        net.train_step(None, "mse", batch, x, t, do_update=False)
+        return out + [net.layer_grad(i, 0).copy() for i in at]
+
+    net = T.Net(layers, batch, T.NET_FUSE_ACT_GRAD)
+    views = [T.DevBuf.view(T.lib().tdh_net_param(net.h, i, 0), (net.param_size(i, 0),)) for i in at]   # (never trusted again)
+    got = []
+    for ws in weights:
+        for view, v in zip(views, ws):
+            view.upload(v)
+        got.append(results(net))
+    net.close()
+    for ws, have in zip(weights, got):
+        fresh = T.Net(layers, batch, T.NET_FUSE_ACT_GRAD)
+        for i, v in zip(at, ws):
+            fresh.set_param(i, 0, v)
+        for i, (a, b) in enumerate(zip(have, results(fresh))):
+            assert np.array_equal(a, b), i
+        fresh.close()

@@ -28,6 +28,7 @@ namespace tdh {
 namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef int intx4 __attribute__((ext_vector_type(4)));
 
 struct FwdSmallArgs {
   const float *x, *w, *bias;
@@ -48,11 +49,9 @@ struct FwdSmallArgs {
 };
 
 // Workgroups in front of the convolution's own pack filters that later layers read: in a net whose
-// weights may have been written since the last call that is a launch less. A packing workgroup holds as many registers as
-// one of the convolution, two to a CU, so it is no more than half hidden: first convolution of the CIFAR-10-shape net at
-// batch 128 14.9 us and the packing 5.0 in launches of their own, together 18.9 (packing behind the
-// convolution 19.5), the step 161.6 / 160.6, inference of 1000 images 245 / 234. No more
-// than 192: a thread of them writes several pieces rather than 500 workgroups (23 us).
+// weights may have been written since the last call that is a launch less, and beside four workgroups of the convolution on a CU
+// it costs little: first convolution of the CIFAR-10-shape net at batch 128 15.0 us, with 590 KB of
+// filters 15.8 (a launch of its own 5.0). No more than 192: a thread of them writes several pieces rather than 500 workgroups.
 constexpr int FWD_SMALL_PACKERS = 192;
 struct NoPacks {};
 template <class Packs>
@@ -74,20 +73,21 @@ __device__ __forceinline__ float lane_xor1(const float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));
 }
 
-// act_apply on the 16 values of an accumulator block; the choice is made once, not per value
-__device__ __forceinline__ void act_apply16(const int kind, float (&v)[16]) {
+// act_apply on the values of an accumulator block; the choice is made once, not per value
+template <int N>
+__device__ __forceinline__ void act_apply_each(const int kind, float (&v)[N]) {
   switch (kind) {
     case TDH_ACT_RELU:
 #pragma unroll
-      for (int i = 0; i < 16; ++i) v[i] = act_apply(TDH_ACT_RELU, v[i]);
+      for (int i = 0; i < N; ++i) v[i] = act_apply(TDH_ACT_RELU, v[i]);
       break;
     case TDH_ACT_TANH:
 #pragma unroll
-      for (int i = 0; i < 16; ++i) v[i] = act_apply(TDH_ACT_TANH, v[i]);
+      for (int i = 0; i < N; ++i) v[i] = act_apply(TDH_ACT_TANH, v[i]);
       break;
     case TDH_ACT_SIGMOID:
 #pragma unroll
-      for (int i = 0; i < 16; ++i) v[i] = act_apply(TDH_ACT_SIGMOID, v[i]);
+      for (int i = 0; i < N; ++i) v[i] = act_apply(TDH_ACT_SIGMOID, v[i]);
       break;
     default: break;
   }
@@ -171,167 +171,44 @@ __device__ __forceinline__ void fwd_small_stage(const FwdSmallArgs &a, float *xs
         const int ky = tap / a.S, kx = tap - ky * a.S;
         o = ci * a.plane + ky * a.dh * a.pitch + kx * a.dw;
       }
-      offs[tid] = max(o, 0);
+      offs[(tid & 1) * NS + (tid >> 1)] = max(o, 0);
     }
   }
 }
 
-template <int NS, class Packs>
-__global__ void __launch_bounds__(256, 2) conv_fwd_small_kernel(const FwdSmallArgs a, const Packs packs) {
+// Stores of a tile that has every channel and every pixel of its 32 x 2 x 32, or less: a value's address is
+// a scalar offset of the tile plus one offset of the lane that is computed once, and what does not exist
+// has a lane offset behind the buffer (guards, 64-bit addresses and saved exec masks were most of 25 vector
+// instructions per MFMA).
+constexpr uint32_t FWD_SMALL_NOWHERE = 0xfffffff0u;   // past the end of any 32 planes
+template <bool STREAM, class T>
+__device__ __forceinline__ void fwd_small_store(const T v, const __amdgpu_buffer_rsrc_t to, const uint32_t lane, const uint32_t tile) {
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), to, lane, tile, STREAM ? 2 : 0);
+}
+
+// PLAIN: the channels are a multiple of 32 and each activation is relu or none.
+// Registers are what keeps workgroups from a CU: with patch offsets and biases read again per tile instead of held, and
+// patch values a group of four steps ahead instead of eight, 176 -> 114 of them and two -> four workgroups. us for 3 -> 32 channels, 5x5, 32x32 with
+// a pool and relu behind, batch 1000 with y: 92 -> 77; of three to four workgroups and the stores above, 3 -> 64 channels, 3x3, 128x128, batch 64
+// 91 -> 75, 1 -> 32, 5x5, 28x28, batch 256 17.6 -> 12.6, 1 -> 6, 5x5, 70x50, batch 64 20.6 -> 14.6.
+template <int NS, class Packs, bool PLAIN>
+__global__ void __launch_bounds__(256, PLAIN ? 4 : 3) conv_fwd_small_kernel(const FwdSmallArgs a, const Packs packs) {
   extern __shared__ __align__(16) float lds[];
   if (fwd_small_packs(a, packs)) return;
   float *xs = lds;
   float *ws = lds + a.x_floats;  // [32][crs], rows past Cout are zero
   float *bs = ws + 32 * a.crs;   // [32] bias, zero past Cout or without bias
-  int *offs = reinterpret_cast<int *>(bs + 32);  // [2*NS] patch offset of k (0 past K)
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // (an image's bands share rows: they go to one XCD)
-  const int wg = xcd_compact_id(blockIdx.x - (gridDim.x - a.workgroups), a.workgroups);
-  const int bandi = wg % a.bands, img = (wg / a.bands) % a.batch, co0 = (wg / (a.bands * a.batch)) * 32;
-  const int oy0 = bandi * a.band;
-  const int nthr = blockDim.x;  // one wave per tile of the band, two to four waves
-
-  fwd_small_stage<NS>(a, xs, ws, bs, offs, img, co0, oy0, tid, nthr);
-  __syncthreads();
-
-  // ---- per-lane constants: the lane's column of the filter matrix
-  // (k = 2*s + half), the bias of its 16 output channels
-  const int nl = lane & 31, half = lane >> 5;
-  float areg[NS];
-#pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    const int k = 2 * s + half;
-    areg[s]     = k < a.crs ? ws[nl * a.crs + k] : 0.0f;
-  }
-  const int *offh = offs + half;  // the offsets stay in LDS: one broadcast read per k-step
-  float bias_r[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    bias_r[i] = bs[(i >> 2) * 8 + half * 4 + (i & 3)];
-  }
-
-  const int ohw = a.OH * a.OW;
-  const int POH = a.OH >> 1, POW = a.OW >> 1;
-  const int tiles = (a.band >> 1) * a.col_tiles;
-#pragma unroll 1
-  for (int tile = wave; tile < tiles; tile += (nthr >> 6)) {
-    const int rp = a.div_col_tiles.div(tile), ct = tile - rp * a.col_tiles;
-    const int r = 2 * rp, c = 32 * ct + nl;  // band-relative upper row, column
-    const float *xb0 = xs + r * a.sh * a.pitch + c * a.sw;
-    const float *xb1 = xb0 + a.sh * a.pitch;
-    floatx16 acc0, acc1;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc0[i] = acc1[i] = 0.0f;
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const int o = offh[2 * s];
-      acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(areg[s], xb0[o], acc0, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(areg[s], xb1[o], acc1, 0, 0, 0);
-    }
-
-    // ---- epilogue: reg i of lane l holds channel 8*(i/4) + 4*(l/32) + i%4 at column l%32
-    const int oy = oy0 + r, ox = c;
-    const bool ok0 = oy < a.OH && ox < a.OW, ok1 = oy + 1 < a.OH && ox < a.OW;
-    const size_t pbase = static_cast<size_t>(img) * a.Kc * ohw + oy * a.OW + ox;
-    const int mlo = co0 + half * 4;  // channel of reg i: mlo + 8*(i/4) + i%4
-    float v0[16], v1[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      v0[i] = acc0[i] + bias_r[i];
-      v1[i] = acc1[i] + bias_r[i];
-    }
-    if (a.out) {  // (null: the layers behind leave this kernel too and nobody reads the convolution's own output)
-      float *o = a.out + pbase;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int m = mlo + (i >> 2) * 8 + (i & 3);
-        if (ok0 && m < a.Kc) o[m * ohw] = v0[i];
-        if (ok1 && m < a.Kc) o[m * ohw + a.OW] = v1[i];
-      }
-    }
-    if (a.act_out) {
-      act_apply16(a.act_kind, v0);
-      act_apply16(a.act_kind, v1);
-      float *o = a.act_out + pbase;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int m = mlo + (i >> 2) * 8 + (i & 3);
-        if (ok0 && m < a.Kc) o[m * ohw] = v0[i];
-        if (ok1 && m < a.Kc) o[m * ohw + a.OW] = v1[i];
-      }
-    }
-    if (a.pool_out) {
-      // the window of an even lane in scan order: its own value, its right neighbour's, and the
-      // same two of the row below; every lane runs the exchange, even lanes keep the result
-      int sel[16];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float w4[4] = {v0[i], lane_xor1(v0[i]), v1[i], lane_xor1(v1[i])};
-        float best = -FLT_MAX;
-        sel[i]     = -1;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (w4[j] > best) {
-            best   = w4[j];
-            sel[i] = j;
-          }
-        v0[i] = best;
-      }
-      const bool anchor = ok0 && !(nl & 1);
-      const size_t pobase = static_cast<size_t>(img) * a.Kc * (POH * POW) + (oy >> 1) * POW + (ox >> 1);
-      if (anchor) {
-        float *o   = a.pool_out + pobase;
-        int32_t *g = a.pool_argmax + pobase;
-        const int pix = oy * a.OW + ox;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int m = mlo + (i >> 2) * 8 + (i & 3);
-          if (m < a.Kc) {
-            o[m * (POH * POW)] = v0[i];
-            g[m * (POH * POW)] = sel[i] < 0 ? 0 : m * ohw + pix + (sel[i] >> 1) * a.OW + (sel[i] & 1);
-          }
-        }
-      }
-      if (a.pool_act_out) {
-        act_apply16(a.pool_act_kind, v0);
-        if (anchor) {
-          float *o = a.pool_act_out + pobase;
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int m = mlo + (i >> 2) * 8 + (i & 3);
-            if (m < a.Kc) o[m * (POH * POW)] = v0[i];
-          }
-        }
-      }
-    }
-  }
-}
-
-// The same tiles for a layer where nothing needs a guard or a choice per value: every band has
-// whole row pairs, the width is a multiple of 32 columns, the channels a multiple of 32, there is
-// no activation between convolution and pool, and the activation behind the pool is relu or
-// none. These tiles are bound by the vector instructions around the MFMAs (about 25 per MFMA
-// in the kernel above, guards, 64-bit addresses and saved exec masks most of them), so here
-// everything that depends on the tile is kept in scalar registers (the wave index is read from
-// the first lane for that), a lane adds one offset of its own that is computed once, and no
-// store has a condition.
-template <int NS, class Packs>
-__global__ void __launch_bounds__(256, 2) conv_fwd_small_full_kernel(const FwdSmallArgs a, const Packs packs) {
-  extern __shared__ __align__(16) float lds[];
-  if (fwd_small_packs(a, packs)) return;
-  float *xs = lds;
-  float *ws = lds + a.x_floats;
-  float *bs = ws + 32 * a.crs;
-  int *offs = reinterpret_cast<int *>(bs + 32);
+  int *offs = reinterpret_cast<int *>(bs + 32);  // [2][NS] patch offset of k = 2s, 2s + 1 (0 past K)
   const int tid = threadIdx.x, lane = tid & 63;
   // (an image's bands share rows: they go to one XCD)
   const int wg = xcd_compact_id(blockIdx.x - (gridDim.x - a.workgroups), a.workgroups);
   const int bandi = wg % a.bands, img = (wg / a.bands) % a.batch, co0 = (wg / (a.bands * a.batch)) * 32;
   const int oy0 = bandi * a.band;
-  const int nthr = blockDim.x;
+  const int nthr = blockDim.x;  // one wave per tile of the band, two to four waves
   fwd_small_stage<NS>(a, xs, ws, bs, offs, img, co0, oy0, tid, nthr);
   __syncthreads();
 
+  // the lane's column of the filter matrix (k = 2*s + half)
   const int nl = lane & 31, half = lane >> 5;
   float areg[NS];
 #pragma unroll
@@ -339,52 +216,57 @@ __global__ void __launch_bounds__(256, 2) conv_fwd_small_full_kernel(const FwdSm
     const int k = 2 * s + half;
     areg[s]     = k < a.crs ? ws[nl * a.crs + k] : 0.0f;
   }
-  // the patch offset of every k-step: the same for all tiles of the wave
-  int o[NS];
-#pragma unroll
-  for (int s = 0; s < NS; ++s) o[s] = offs[2 * s + half];
-  float bias_r[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) bias_r[i] = bs[(i >> 2) * 8 + half * 4 + (i & 3)];
 
   const uint32_t ohw = a.OH * a.OW, OW = a.OW, POW = a.OW >> 1, pohw = (a.OH >> 1) * POW;
   const uint32_t tiles = (a.band >> 1) * a.col_tiles;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = __builtin_amdgcn_readfirstlane(nthr >> 6);
   // the lane's own part of every address: its channel group and its column
-  const uint32_t lane_out = half * 4 * ohw + nl, lane_pool = half * 4 * pohw + (nl >> 1);
-  const bool even  = !(nl & 1);
-  const bool pool  = a.pool_out != nullptr;
+  // (of two neighbours, which share a window, the odd one pools the next channel)
+  const bool even = !(nl & 1);
+  const uint32_t lane_out = half * 4 * ohw + nl, lane_window = even ? lane_out : lane_out - 1 + ohw;
+  const uint32_t lane_pool = half * 4 * pohw + (nl >> 1) + (even ? 0 : pohw);
   const float floor_v = a.pool_act_kind == TDH_ACT_RELU ? 0.0f : -INFINITY;  // relu as a max
-  float *out_img        = a.out + (static_cast<size_t>(img) * a.Kc + co0) * ohw;
-  float *pool_img       = a.pool_out + (static_cast<size_t>(img) * a.Kc + co0) * pohw;
-  float *pool_act_img   = a.pool_act_out + (static_cast<size_t>(img) * a.Kc + co0) * pohw;
-  int32_t *argmax_img   = a.pool_argmax + (static_cast<size_t>(img) * a.Kc + co0) * pohw;
+  const int channels  = PLAIN ? 32 : min(32, a.Kc - co0);
+  auto planes = [&](auto *p, const uint32_t plane) {   // the planes of the workgroup's channels
+    return __builtin_amdgcn_make_buffer_rsrc(p ? p + (static_cast<size_t>(img) * a.Kc + co0) * plane : nullptr, 0,
+                                             p ? 4u * channels * plane : 0u, 0x00027000);
+  };
+  const auto out = planes(a.out, ohw), act_out = planes(a.act_out, ohw), pool_out = planes(a.pool_out, pohw),
+             pool_argmax = planes(a.pool_argmax, pohw), pool_act_out = planes(a.pool_act_out, pohw);
 #pragma unroll 1
   for (uint32_t tile = wave; tile < tiles; tile += nwaves) {
     const uint32_t rp = a.div_col_tiles.div(tile), ct = tile - rp * a.col_tiles;
     const uint32_t r = 2 * rp, c0 = 32 * ct;
+    if (oy0 + r >= static_cast<uint32_t>(a.OH)) break;   // (so that a tile's offset is always inside its planes)
     const float *xb0 = xs + r * a.sh * a.pitch + (c0 + nl) * a.sw;
     const float *xb1 = xb0 + a.sh * a.pitch;
     floatx16 acc0, acc1;
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc0[i] = acc1[i] = 0.0f;
-    // The patch values of eight k-steps are read while the products of the eight before them
-    // run: read and product one after the other would wait for LDS in every step.
-    constexpr int G = 8;
-    static_assert(NS % G == 0, "k-steps come in groups");
+    // The patch values of four k-steps are read while the products of the four before them
+    // run, and their offsets a group earlier: read and product one after the other would wait for LDS in every step.
+    constexpr int G = 4;
+    static_assert(NS % G == 0 && NS >= 2 * G, "k-steps come in groups");
+    int from = half * NS;
+    asm volatile("" : "+v"(from));   // (not held over the tiles)
+    intx4 o[2];
     float b0[2][G], b1[2][G];
-    auto read_patch = [&](int g, int to) {
+    auto read_offsets = [&](int g) { o[g & 1] = *reinterpret_cast<const intx4 *>(offs + from + g * G); };
+    auto read_patch = [&](int g) {
 #pragma unroll
       for (int j = 0; j < G; ++j) {
-        b0[to][j] = xb0[o[g * G + j]];
-        b1[to][j] = xb1[o[g * G + j]];
+        b0[g & 1][j] = xb0[o[g & 1][j]];
+        b1[g & 1][j] = xb1[o[g & 1][j]];
       }
     };
-    read_patch(0, 0);
+    read_offsets(0);
+    read_offsets(1);
+    read_patch(0);
 #pragma unroll
     for (int g = 0; g < NS / G; ++g) {
       const int cur = g & 1;
-      if (g + 1 < NS / G) read_patch(g + 1, cur ^ 1);
+      if (g + 1 < NS / G) read_patch(g + 1);
+      if (g + 2 < NS / G) read_offsets(g + 2);
 #pragma unroll
       for (int j = 0; j < G; ++j) {
         acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(areg[g * G + j], b0[cur][j], acc0, 0, 0, 0);
@@ -396,42 +278,84 @@ __global__ void __launch_bounds__(256, 2) conv_fwd_small_full_kernel(const FwdSm
     const uint32_t oy = oy0 + r;
     const uint32_t first = oy * OW + c0;  // of the tile inside a channel plane
     float v0[16], v1[16];
+    int at_bias = half * 4;
+    asm volatile("" : "+v"(at_bias));
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      v0[i] = acc0[i] + bias_r[i];
-      v1[i] = acc1[i] + bias_r[i];
+      const float bias = bs[at_bias + (i >> 2) * 8 + (i & 3)];
+      v0[i] = acc0[i] + bias;
+      v1[i] = acc1[i] + bias;
     }
-    if (a.out) {
+    const bool in = c0 + nl < OW && oy < static_cast<uint32_t>(a.OH);
+    const uint32_t lane0 = in ? 4 * lane_out : FWD_SMALL_NOWHERE;
+    const uint32_t lane1 = in && oy + 1 < static_cast<uint32_t>(a.OH) ? 4 * (lane_out + OW) : FWD_SMALL_NOWHERE;
+    // the lane holds channel c of register i (scalar: the first of the two halves'); of a channel that does not exist, nothing is in reach
+    auto here  = [&](int c, uint32_t lane) { return PLAIN || c + 4 * half < channels ? lane : FWD_SMALL_NOWHERE; };
+    auto plane = [&](int c, uint32_t size) { return PLAIN || c < channels ? c * size : 0u; };
+    auto write = [&](auto stream, const auto to) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        float *o = out_img + (((i >> 2) * 8 + (i & 3)) * ohw + first);  // scalar
-        o[lane_out]        = v0[i];
-        (o + OW)[lane_out] = v1[i];
+        const int c = (i >> 2) * 8 + (i & 3);
+        fwd_small_store<decltype(stream)::value>(v0[i], to, here(c, lane0), 4 * (plane(c, ohw) + first));
+        fwd_small_store<decltype(stream)::value>(v1[i], to, here(c, lane1), 4 * (plane(c, ohw) + first));
       }
+    };
+    if (a.out) {
+      // (what is pooled here no kernel reads next: 86 us / 77 for 131 MB of it)
+      if (a.pool_out)
+        write(std::true_type(), out);
+      else
+        write(std::false_type(), out);
     }
-    if (pool) {
-      // as above: the window of an even lane in scan order, strict '>', start value lowest();
+    if (a.act_out) {
+      if (PLAIN) {
+        if (a.act_kind == TDH_ACT_RELU) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            v0[i] = act_apply(TDH_ACT_RELU, v0[i]);
+            v1[i] = act_apply(TDH_ACT_RELU, v1[i]);
+          }
+        }
+      } else {
+        act_apply_each(a.act_kind, v0);
+        act_apply_each(a.act_kind, v1);
+      }
+      write(std::false_type(), act_out);
+    }
+    if (a.pool_out) {
+      // the window of two neighbours in scan order, strict '>', start value lowest();
       // where: the winner's distance from the window's first element (0, 1, OW, OW + 1), -1 when
       // no value beat the start value
       const uint32_t pfirst = (oy >> 1) * POW + (c0 >> 1);
+      const uint32_t lane_p = in ? 4 * lane_pool : FWD_SMALL_NOWHERE;
+      float best[8];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float w4[4] = {v0[i], lane_xor1(v0[i]), v1[i], lane_xor1(v1[i])};
+      for (int i = 0; i < 16; i += 2) {
+        const float l0 = lane_xor1(v0[i + 1]), r0 = lane_xor1(v0[i]), l1 = lane_xor1(v1[i + 1]), r1 = lane_xor1(v1[i]);
+        const float w4[4] = {even ? v0[i] : l0, even ? r0 : v0[i + 1], even ? v1[i] : l1, even ? r1 : v1[i + 1]};
         const int at[4]   = {0, 1, static_cast<int>(OW), static_cast<int>(OW) + 1};
-        float best = -FLT_MAX;
-        int where  = -1;
+        float &b  = best[i >> 1];
+        b         = -FLT_MAX;
+        int where = -1;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (w4[j] > best) {
-            best  = w4[j];
+          if (w4[j] > b) {
+            b     = w4[j];
             where = at[j];
           }
-        const uint32_t ch     = (i >> 2) * 8 + (i & 3);
-        const uint32_t chfirst = (co0 + ch) * ohw + first;  // scalar: flat CHW index of the tile's first element
-        if (even) {
-          (pool_img + (ch * pohw + pfirst))[lane_pool]   = best;
-          (argmax_img + (ch * pohw + pfirst))[lane_pool] = where < 0 ? 0 : static_cast<int>(chfirst + lane_out) + where;
-          if (a.pool_act_out) (pool_act_img + (ch * pohw + pfirst))[lane_pool] = best > floor_v ? best : floor_v;
+        const int c = (i >> 2) * 8 + (i & 3);
+        const uint32_t to = here(c + (even ? 0 : 1), lane_p), tile_p = 4 * (plane(c, pohw) + pfirst);
+        const uint32_t cfirst = (co0 + c) * ohw + first;  // scalar: flat CHW index of the tile's first element
+        fwd_small_store<false>(b, pool_out, to, tile_p);
+        fwd_small_store<false>(where < 0 ? 0 : static_cast<int>(cfirst + lane_window) + where, pool_argmax, to, tile_p);
+        if (PLAIN && a.pool_act_out) fwd_small_store<false>(b > floor_v ? b : floor_v, pool_act_out, to, tile_p);
+      }
+      if (!PLAIN && a.pool_act_out) {
+        act_apply_each(a.pool_act_kind, best);
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) {
+          const int c = (i >> 2) * 8 + (i & 3);
+          fwd_small_store<false>(best[i >> 1], pool_act_out, here(c + (even ? 0 : 1), lane_p), 4 * (plane(c, pohw) + pfirst));
         }
       }
     }
@@ -457,6 +381,8 @@ FwdSmallPlan make_fwd_small_plan(int batch, int C, int Kc, int H, int W, int OH,
   a.C = C; a.Kc = Kc; a.H = H; a.W = W; a.OH = OH; a.OW = OW;
   a.R = R; a.S = S; a.sh = sh; a.sw = sw; a.dh = dh; a.dw = dw; a.ph = ph; a.pw = pw;
   a.crs = C * R * S;
+  // (a workgroup's 32 planes are one buffer)
+  if (static_cast<long long>(OH) * OW >= 1LL << 25) return p;
   if (a.crs > 96 || batch < 1 || batch > 65535 || OH < 1 || OW < 1) return p;
   p.ns = ((a.crs + 1) / 2 + 7) / 8 * 8;
   a.col_tiles = ceil_div(OW, 32);
@@ -505,15 +431,13 @@ template <int NS, class Packs>
 int launch_fwd_small(const FwdSmallPlan &p, const Packs &packs, int pack_blocks) {
   const int tiles = (p.a.band / 2) * p.a.col_tiles;
   const FwdSmallArgs &a = p.a;
-  const bool full = a.OH % a.band == 0 && a.band % 2 == 0 && a.OW % 32 == 0 && a.Kc % 32 == 0 && !a.act_out &&
-                    (a.pool_act_kind == TDH_ACT_RELU || a.pool_act_kind == TDH_ACT_NONE || !a.pool_act_out) &&
-                    static_cast<long long>(a.Kc) * a.OH * a.OW < (1LL << 30);
+  auto plain = [](int kind) { return kind == TDH_ACT_RELU || kind == TDH_ACT_NONE; };
   const dim3 block(64 * std::min(4, std::max(2, tiles)));
   const dim3 grid(a.workgroups + std::min(block.x < 256 ? 2 * pack_blocks : pack_blocks, FWD_SMALL_PACKERS));
-  if (full)
-    TDH_LAUNCH((conv_fwd_small_full_kernel<NS, Packs>), grid, block, p.lds_bytes, ctx().stream, p.a, packs);
+  if (a.Kc % 32 == 0 && (!a.act_out || plain(a.act_kind)) && (!a.pool_act_out || plain(a.pool_act_kind)))
+    TDH_LAUNCH((conv_fwd_small_kernel<NS, Packs, true>), grid, block, p.lds_bytes, ctx().stream, p.a, packs);
   else
-    TDH_LAUNCH((conv_fwd_small_kernel<NS, Packs>), grid, block, p.lds_bytes, ctx().stream, p.a, packs);
+    TDH_LAUNCH((conv_fwd_small_kernel<NS, Packs, false>), grid, block, p.lds_bytes, ctx().stream, p.a, packs);
   TDH_LAUNCH_CHECK();
   return TDH_OK;
 }
