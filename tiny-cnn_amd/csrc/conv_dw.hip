@@ -31,7 +31,8 @@
 // WK row-group sums are added pairwise through LDS and the workgroup writes one slice
 // [slice][co][ci][tap]; splitk_reduce_kernel adds the slices in order.
 //
-// 5x5 windows: 25 accumulators do not fit one wave, so the filter rows go to different
+// 5x5 windows: 25 accumulators do not fit one wave, so the filter rows (of 3x3 windows too, where the
+// chip has room for them) go to different
 // WORKGROUPS (grid z = channel block x filter row) and the kernel runs as a 1x5 window whose
 // input rows are shifted by the filter row. Such a window needs no halo rows, so on small
 // images a chunk holds TI whole images stacked as rows.
@@ -382,6 +383,7 @@ __global__ void __launch_bounds__(DWI_NT, 2) conv_dw_img_kernel(const DwImgArgs 
 struct DwHaloPlan {
   bool ok;
   int tc, wco, wk, wfy, nt;
+  int window;      // filter rows (3 or 5)
   int rows_block;  // filter rows one workgroup covers
   DwHaloArgs args;
   size_t lds_bytes;
@@ -409,6 +411,7 @@ DwHaloPlan make_dw_plan(int R, int S, int batch, int C, int Kc, int H, int W, in
   p.wco = Kc > 32 ? 2 : 1;
   p.wk  = 4 / p.wco;
   p.nt = 64 * p.wco * p.wk * p.wfy;
+  p.window     = R;
   p.rows_block = five ? 1 : R;
   DwHaloArgs &a = p.args;
   a.batch = batch; a.C = C; a.Kc = Kc; a.H = H; a.W = W; a.OH = OH; a.OW = OW; a.ph = ph; a.pw = pw;
@@ -432,7 +435,8 @@ DwHaloPlan make_dw_plan(int R, int S, int batch, int C, int Kc, int H, int W, in
   a.chunks_total  = a.TI > 1 ? ceil_div(batch, a.TI) : batch * row_chunks;
   a.div_rowchunks = FastDiv(row_chunks);
   a.div_oh        = FastDiv(OH);
-  const int co_blocks = ceil_div(Kc, 32 * p.wco), ci_blocks = ceil_div(C, 32) * (R / p.rows_block);
+  const int co_blocks = ceil_div(Kc, 32 * p.wco);
+  int ci_blocks       = ceil_div(C, 32) * (R / p.rows_block);
   const long base = static_cast<long>(a.tiles_x) * co_blocks * ci_blocks;
   // one workgroup per CU; a slice should still cover a few chunks so that its prologue and
   // its partial tile are paid for
@@ -440,6 +444,14 @@ DwHaloPlan make_dw_plan(int R, int S, int batch, int C, int Kc, int H, int W, in
   slices = std::min<long>(slices, std::max(1, a.chunks_total / 2));
   a.chunks_per_slice = ceil_div(a.chunks_total, static_cast<int>(slices));
   p.slices           = ceil_div(a.chunks_total, a.chunks_per_slice);
+  // A 3x3 window whose slices leave compute units idle: a workgroup per filter row as well, of the same slices (a tap has a
+  // sum of its own either way, in the same order). us with the rows together / apart: 15x15, 24 -> 48, batch 37 (37
+  // workgroups / 111) 28.5 / 15.6; 24x24, 16 -> 32, batch 16 28.5 / 13.5; 10x10, 32 -> 64, batch 64 29.5 / 16.1.
+  if (p.rows_block == 3 && 3 * base * p.slices <= 256) {
+    p.rows_block = 1;
+    ci_blocks *= 3;
+    a.plane_p = (4 * (tr * nq)) | 1;
+  }
   const int nacc = (p.rows_block / p.wfy) * S;
   const size_t stage_floats = static_cast<size_t>(32 * p.wco) * a.dyp + 32 * static_cast<size_t>(a.plane_p);
   const size_t red_floats   = static_cast<size_t>(p.wk / 2) * p.wco * nacc * 16 * 64;
@@ -474,6 +486,8 @@ int launch_dw_inst(const DwHaloPlan &p) {
 
 template <int TC, bool VEC>
 int launch_dw_tc(const DwHaloPlan &p) {
+  if (p.rows_block == 1 && p.window == 3)
+    return p.wco == 2 ? launch_dw_inst<1, 3, TC, 2, 2, 1, 3, VEC>(p) : launch_dw_inst<1, 3, TC, 1, 4, 1, 3, VEC>(p);
   if (p.rows_block == 1)
     return p.wco == 2 ? launch_dw_inst<1, 5, TC, 2, 2, 1, 5, VEC>(p) : launch_dw_inst<1, 5, TC, 1, 4, 1, 5, VEC>(p);
   if (p.wco == 2) return launch_dw_inst<3, 3, TC, 2, 2, 1, 3, VEC>(p);
