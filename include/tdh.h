@@ -326,8 +326,8 @@ int tdh_net_update_weights(tdh_net *net, tdh_opt *opt);
 /* nodes::clear_grads (tiny_dnn/nodes.h:118-122): zeroes every weight and bias gradient */
 int tdh_net_clear_grads(tdh_net *net);
 /* device views valid until the net is destroyed. The weights may be written through them between any
- * two calls: once a convolution's weights have been asked for here, a TDH_NET_GRAPH net packs the
- * filters that a pass or step reads anew in every call (one launch of a few microseconds), where it
+ * two calls: once a convolution's weights have been asked for here, a net packs the filters
+ * that a pass or step reads anew in every call (one launch of a few microseconds at most), where it
  * otherwise keeps packed copies beside the weights. To look at weights, or to set them now and then,
  * tdh_net_get_param and tdh_net_set_param cost the following calls nothing. */
 float *tdh_net_param(tdh_net *net, int layer, int which);

@@ -24,8 +24,8 @@ struct tdh_net {
     // set where the optimizer table is built: the tensor's entry there has the small blocks
     // (OPT_SUM_ELEMS_PER_BLOCK) that let the optimizer kernel add up K-split partial slices
     bool w_sums_in_opt = false, b_sums_in_opt = false;
-    // Copies of the filters in the layouts that the stride-1 kernels read (stride-1 conv layers of a
-    // TDH_NET_GRAPH net; null: no kernel of this layer reads that one). current: it holds the
+    // Copies of the filters in the layouts that the stride-1 kernels read (stride-1 conv layers;
+    // null: no kernel of this layer reads that one). current: it holds the
     // weights as they are; kept: the optimizer kernel writes the new weights into it as well,
     // which it does for the copies that train steps read.
     enum Copy { FWD_F32, DX_F32, FWD_X3, DX_X3, COPIES };
@@ -799,8 +799,7 @@ int tdh_net_create(const tdh_layer *layers, int n_layers, int max_batch, int fla
       if ((rc = net_alloc(net, ceil_div_sz(act, sizeof(float)), &p, true))) break;
       L.mask = reinterpret_cast<uint8_t *>(p);
     }
-    if ((flags & TDH_NET_GRAPH) && L.spec.kind == TDH_L_CONV && L.spec.conv.w_stride == 1 &&
-        L.spec.conv.h_stride == 1) {
+    if (L.spec.kind == TDH_L_CONV && L.spec.conv.w_stride == 1 && L.spec.conv.h_stride == 1) {
       // (one buffer: an allocation takes the host some 100 us)
       auto padded = [](size_t floats) { return ceil_div_sz(floats, 64) * 64; };
       size_t at[2] = {0, 0}, total = 2 * padded(L.w_size);
