@@ -945,7 +945,7 @@ int fc_two_layer_tail(int in, int hidden, int out, int has_bias1, int has_bias2,
 size_t fc_workspace_bytes(int in, int out, int batch) {
   return std::max(gemm_workspace_bytes(batch, out, in, true), fc_x3_workspace_bytes(batch, out, in)) +
          std::max(gemm_workspace_bytes(batch, in, out, true), fc_x3_workspace_bytes(batch, in, out)) +
-         gemm_workspace_bytes(in, out, batch, true);
+         std::max(gemm_workspace_bytes(in, out, batch, true), fc_x3_workspace_bytes(in, out, batch));
 }
 
 int fc_fwd(int in, int out, int has_bias, int batch, const float *x, const float *w,
@@ -957,15 +957,15 @@ int fc_fwd(int in, int out, int has_bias, int batch, const float *x, const float
   if (act_out) {  // the pointwise activation layer that follows leaves the same kernel
     EpiRowMajorAct epi{y, out, has_bias ? b : nullptr, act_out, act_kind};
     if (small_fc_applies(batch, out, in)) return launch_small_fc(A, B, epi, batch, out, in, "fc_fwd_small");
-    if (fc_x3_applies(batch, out, in, x, w, in, out))
+    if (fc_x3_applies(FX_A_K_B_N, batch, out, in, x, w, in, out))
       return fc_x3_run_act(x, w, in, out, epi, batch, out, in, "fc_fwd_x3", "fc_fwd_splitk_reduce");
     return launch_gemm<true, false, false, true>(A, B, epi, batch, out, in, true, "fc_fwd_gemm",
                                                 "fc_fwd_splitk_reduce");
   }
   EpiRowMajor epi{y, out, has_bias ? b : nullptr, ActGrad(), 0};
   if (small_fc_applies(batch, out, in)) return launch_small_fc(A, B, epi, batch, out, in, "fc_fwd_small");
-  if (fc_x3_applies(batch, out, in, x, w, in, out))
-    return fc_x3_run(false, x, w, in, out, epi, batch, out, in, "fc_fwd_x3", "fc_fwd_splitk_reduce");
+  if (fc_x3_applies(FX_A_K_B_N, batch, out, in, x, w, in, out))
+    return fc_x3_run(FX_A_K_B_N, x, w, in, out, epi, batch, out, in, "fc_fwd_x3", "fc_fwd_splitk_reduce");
   return launch_gemm<true, false, false, true>(A, B, epi, batch, out, in, true, "fc_fwd_gemm",
                                               "fc_fwd_splitk_reduce");
 }
@@ -1364,8 +1364,8 @@ int fc_bwd(int in, int out, int has_bias, int batch, const float *x, const float
     EpiRowMajor epi{dx, in, nullptr, dx_act, 0};
     if (small_fc_applies(batch, in, out)) {
       TDH_TRY(launch_small_fc(A, B, epi, batch, in, out, "fc_dx_small"));
-    } else if (fc_x3_applies(batch, in, out, dy, w, out, out)) {
-      TDH_TRY(fc_x3_run(true, dy, w, out, out, epi, batch, in, out, "fc_dx_x3", "fc_dx_splitk_reduce"));
+    } else if (fc_x3_applies(FX_A_K_B_K, batch, in, out, dy, w, out, out)) {
+      TDH_TRY(fc_x3_run(FX_A_K_B_K, dy, w, out, out, epi, batch, in, out, "fc_dx_x3", "fc_dx_splitk_reduce"));
     } else if (fc_dx_tile_applies(in, out, batch, dy, w)) {
       ProfScope prof("fc_dx_tile", batch, in, out);
       FcDxTile f{dy, w, dx, dx_act, batch, in, out, ceil_div(batch, 64), ceil_div(in, 64), 0};
@@ -1382,6 +1382,8 @@ int fc_bwd(int in, int out, int has_bias, int batch, const float *x, const float
     EpiRowMajor epi{dw, out, nullptr, ActGrad(), accumulate};
     if (small_fc_applies(in, out, batch)) {
       TDH_TRY(launch_small_fc(A, B, epi, in, out, batch, "fc_dw_small"));
+    } else if (fc_x3_applies(FX_A_M_B_N, in, out, batch, x, dy, in, out)) {
+      TDH_TRY(fc_x3_run(FX_A_M_B_N, x, dy, in, out, epi, in, out, batch, "fc_dw_x3", "fc_dw_splitk_reduce"));
     } else if (fc_dw_direct_applies(in, out, batch, x, dy, dw)) {
       ProfScope prof("fc_dw_direct", in, out, batch);
       const FcDwDirect f{x, dy, dw, batch, in, out, accumulate};

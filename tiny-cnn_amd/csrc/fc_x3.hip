@@ -4,9 +4,10 @@
 //
 //   forward  y[b][o]  = x[b][i] W[i][o]     A rows along k, B rows along n
 //   dX       dx[b][i] = dy[b][o] W[i][o]    both along k
+//   dW       dW[i][o] = x[b][i] dy[b][o]    A rows along m, B rows along n
 //
-// (Inference and dX only: the bias gradients of a train step hang on the last bits of its forward
-// product and of its weights, and Adam makes a full step of one that is nearly zero.)
+// (Not the forward product of a train step: the bias gradients of a train step hang on the last bits of it
+// and of the weights, and Adam makes a full step of one that is nearly zero.)
 //
 // A workgroup of four wave64 owns 64*WM x 64*WN elements, a wave 64 x 64 of them (four accumulator
 // blocks). Per step of 32 reduction indices the tile's 16-byte words are loaded while the step
@@ -20,7 +21,8 @@
 // instructions; the two hardly overlap), HBM where one matrix is narrow.
 // us, fp32 kernels / here: 4096 x 4096, batch 256 forward 107 / 67, dX 87 / 71; 6000 x 4096, batch 512
 // 258 / 161, 234 / 179; 131072 x 256, batch 64 69 / 43, 65 / 47. Loading two steps ahead changed
-// nothing.
+// nothing, nor did tiles of 256 x 128 whose next step is split between the products of this one (dX of 4096 x 4096, batch 1024 199 and
+// 203): what is left is what the chip's power allows.
 #include "gemm_mfma.h"
 #include "split_bf16.h"
 
@@ -114,12 +116,12 @@ struct FxSide {
   }
 };
 
-template <int WM, int WN, bool B_KC, class Epi>
+template <int WM, int WN, bool A_KC, bool B_KC, class Epi>
 __global__ void __launch_bounds__(FX_NT, 2)
 fc_x3_kernel(const float *__restrict__ A, const float *__restrict__ B, const int lda, const int ldb, const Epi epi,
              const int M, const int N, const int K, const int k_per_split, float *__restrict__ partial) {
   constexpr int BM = 64 * WM, BN = 64 * WN;
-  using SideA = FxSide<BM, true>;
+  using SideA = FxSide<BM, A_KC>;
   using SideB = FxSide<BN, B_KC>;
   __shared__ uintx4 a_lds[SideA::UNITS], b_lds[SideB::UNITS];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -133,7 +135,7 @@ fc_x3_kernel(const float *__restrict__ A, const float *__restrict__ B, const int
   const int m0 = by * BM, n0 = bx * BN;
   const int kbeg = bz * k_per_split, kend = min(K, kbeg + k_per_split);
 
-  const auto da = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), 0, 4u * M * lda, 0x00027000);
+  const auto da = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), 0, 4u * (A_KC ? M : K) * lda, 0x00027000);
   const auto db = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(B), 0, 4u * (B_KC ? N : K) * ldb, 0x00027000);
   SideA sa;
   SideB sb;
@@ -197,7 +199,7 @@ fc_x3_kernel(const float *__restrict__ A, const float *__restrict__ B, const int
 #pragma unroll
           for (int i = 0; i < 2; ++i) {
             const int m = m0 + 64 * wm + 32 * i + l32, n = n0 + 64 * wn + 32 * i + l32;
-            av[s][i] = k < kend && m < M ? A[static_cast<size_t>(m) * lda + k] : 0.0f;
+            av[s][i] = k < kend && m < M ? A[A_KC ? static_cast<size_t>(m) * lda + k : static_cast<size_t>(k) * lda + m] : 0.0f;
             bv[s][i] = k < kend && n < N ? B[B_KC ? static_cast<size_t>(n) * ldb + k : static_cast<size_t>(k) * ldb + n] : 0.0f;
           }
         }
@@ -262,14 +264,14 @@ FxPlan fx_plan(int M, int N, int K) {
   return p;
 }
 
-template <bool B_KC, class Epi>
+template <bool A_KC, bool B_KC, class Epi>
 int launch_fx(const FxPlan &p, const float *A, const float *B, int lda, int ldb, const Epi &epi, int M, int N, int K,
               float *partial) {
   const dim3 grid(ceil_div(N, 64 * p.wn), ceil_div(M, 64 * p.wm), p.splits);
   switch (p.wm) {
-    case 1: TDH_LAUNCH((fc_x3_kernel<1, 4, B_KC, Epi>), grid, dim3(FX_NT), 0, ctx().stream, A, B, lda, ldb, epi, M, N, K, p.k_per_split, partial); break;
-    case 2: TDH_LAUNCH((fc_x3_kernel<2, 2, B_KC, Epi>), grid, dim3(FX_NT), 0, ctx().stream, A, B, lda, ldb, epi, M, N, K, p.k_per_split, partial); break;
-    default: TDH_LAUNCH((fc_x3_kernel<4, 1, B_KC, Epi>), grid, dim3(FX_NT), 0, ctx().stream, A, B, lda, ldb, epi, M, N, K, p.k_per_split, partial); break;
+    case 1: TDH_LAUNCH((fc_x3_kernel<1, 4, A_KC, B_KC, Epi>), grid, dim3(FX_NT), 0, ctx().stream, A, B, lda, ldb, epi, M, N, K, p.k_per_split, partial); break;
+    case 2: TDH_LAUNCH((fc_x3_kernel<2, 2, A_KC, B_KC, Epi>), grid, dim3(FX_NT), 0, ctx().stream, A, B, lda, ldb, epi, M, N, K, p.k_per_split, partial); break;
+    default: TDH_LAUNCH((fc_x3_kernel<4, 1, A_KC, B_KC, Epi>), grid, dim3(FX_NT), 0, ctx().stream, A, B, lda, ldb, epi, M, N, K, p.k_per_split, partial); break;
   }
   TDH_LAUNCH_CHECK();
   return TDH_OK;
@@ -277,8 +279,13 @@ int launch_fx(const FxPlan &p, const float *A, const float *B, int lda, int ldb,
 
 }  // namespace
 
-bool fc_x3_applies(int M, int N, int K, const float *A, const float *B, int lda, int ldb) {
-  if (ctx().keep_f32 || M % 4 || N % 4 || K % 4 || lda % 4 || ldb % 4 || K < 64) return false;
+// dW: its result is written once however few samples there are, and the fp32 kernels (fc.hip) have less in front of their
+// products. us there / here: 4096 x 4096 of 64 samples 31 / 39, 256 87 / 75 (one after the other for 10 ms, with dX and an
+// optimizer between them, no different), 1024 309 / 212; 6000 x 4096 of 512 239 / 177; 784 x 1024 of 512 23 / 21; 512 x 512
+// of 4000 37 / 28; 2048 x 2048 of 128 21 / 22; 131072 x 256 of 64 57 / 72.
+constexpr int FX_DW_SAMPLES = 384;
+bool fc_x3_applies(FxRows rows, int M, int N, int K, const float *A, const float *B, int lda, int ldb) {
+  if (ctx().keep_f32 || M % 4 || N % 4 || (rows != FX_A_M_B_N && K % 4) || lda % 4 || ldb % 4 || K < (rows == FX_A_M_B_N ? FX_DW_SAMPLES : 64)) return false;
   if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15) return false;
   if (static_cast<long>(M) * K >= (1L << 29) || static_cast<long>(N) * K >= (1L << 29)) return false;
   return fx_plan(M, N, K).ok;
@@ -290,7 +297,7 @@ size_t fc_x3_workspace_bytes(int M, int N, int K) {
 }
 
 template <class Epi>
-static int run_fx(bool b_along_k, const float *A, const float *B, int lda, int ldb, const Epi &epi, int M, int N, int K,
+static int run_fx(FxRows rows, const float *A, const float *B, int lda, int ldb, const Epi &epi, int M, int N, int K,
                   const char *tag, const char *reduce_tag) {
   const FxPlan p = fx_plan(M, N, K);
   float *partial = nullptr;
@@ -302,20 +309,21 @@ static int run_fx(bool b_along_k, const float *A, const float *B, int lda, int l
   {
     ProfScope prof(tag, M, N, K);
     if constexpr (std::is_same<Epi, EpiRowMajorAct>::value)
-      TDH_TRY((launch_fx<false>(p, A, B, lda, ldb, epi, M, N, K, partial)));
+      TDH_TRY((launch_fx<true, false>(p, A, B, lda, ldb, epi, M, N, K, partial)));
     else
-      TDH_TRY(b_along_k ? (launch_fx<true>(p, A, B, lda, ldb, epi, M, N, K, partial))
-                        : (launch_fx<false>(p, A, B, lda, ldb, epi, M, N, K, partial)));
+      TDH_TRY(rows == FX_A_K_B_K   ? (launch_fx<true, true>(p, A, B, lda, ldb, epi, M, N, K, partial))
+              : rows == FX_A_K_B_N ? (launch_fx<true, false>(p, A, B, lda, ldb, epi, M, N, K, partial))
+                                   : (launch_fx<false, false>(p, A, B, lda, ldb, epi, M, N, K, partial)));
   }
   return p.splits > 1 ? launch_splitk_reduce(partial, p.splits, M, N, epi, reduce_tag) : TDH_OK;
 }
-int fc_x3_run(bool b_along_k, const float *A, const float *B, int lda, int ldb, const EpiRowMajor &epi, int M, int N, int K,
+int fc_x3_run(FxRows rows, const float *A, const float *B, int lda, int ldb, const EpiRowMajor &epi, int M, int N, int K,
               const char *tag, const char *reduce_tag) {
-  return run_fx(b_along_k, A, B, lda, ldb, epi, M, N, K, tag, reduce_tag);
+  return run_fx(rows, A, B, lda, ldb, epi, M, N, K, tag, reduce_tag);
 }
 int fc_x3_run_act(const float *A, const float *B, int lda, int ldb, const EpiRowMajorAct &epi, int M, int N, int K,
                   const char *tag, const char *reduce_tag) {
-  return run_fx(false, A, B, lda, ldb, epi, M, N, K, tag, reduce_tag);
+  return run_fx(FX_A_K_B_N, A, B, lda, ldb, epi, M, N, K, tag, reduce_tag);
 }
 
 }  // namespace tdh

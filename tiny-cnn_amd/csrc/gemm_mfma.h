@@ -193,11 +193,11 @@ __device__ __forceinline__ const Op &bind_tile(const Op &op, int) { return op; }
 template <class Op>
 __device__ __forceinline__ int tile_k(const Op &, int, int K) { return K; }
 
-// fc_x3.hip: products of plain matrices with three-part operands, A rows along k, B rows along k or
-// n; lda, ldb: floats from row to row
-bool fc_x3_applies(int M, int N, int K, const float *A, const float *B, int lda, int ldb);
+// fc_x3.hip: products of plain matrices with three-part operands, their rows along these; lda, ldb: floats from row to row
+enum FxRows { FX_A_K_B_K, FX_A_K_B_N, FX_A_M_B_N };
+bool fc_x3_applies(FxRows rows, int M, int N, int K, const float *A, const float *B, int lda, int ldb);
 size_t fc_x3_workspace_bytes(int M, int N, int K);
-int fc_x3_run(bool b_along_k, const float *A, const float *B, int lda, int ldb, const EpiRowMajor &epi, int M, int N, int K,
+int fc_x3_run(FxRows rows, const float *A, const float *B, int lda, int ldb, const EpiRowMajor &epi, int M, int N, int K,
               const char *tag, const char *reduce_tag);
 int fc_x3_run_act(const float *A, const float *B, int lda, int ldb, const EpiRowMajorAct &epi, int M, int N, int K,
                   const char *tag, const char *reduce_tag);
