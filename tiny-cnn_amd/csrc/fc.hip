@@ -959,6 +959,8 @@ int fc_fwd(int in, int out, int has_bias, int batch, const float *x, const float
     if (small_fc_applies(batch, out, in)) return launch_small_fc(A, B, epi, batch, out, in, "fc_fwd_small");
     if (fc_x3_applies(FX_A_K_B_N, batch, out, in, x, w, in, out))
       return fc_x3_run_act(x, w, in, out, epi, batch, out, in, "fc_fwd_x3", "fc_fwd_splitk_reduce");
+    if (fc_f32_applies(batch, out, in, x, w))
+      return fc_f32_run_act(x, w, epi, batch, out, in, "fc_fwd_f32", "fc_fwd_splitk_reduce");
     return launch_gemm<true, false, false, true>(A, B, epi, batch, out, in, true, "fc_fwd_gemm",
                                                 "fc_fwd_splitk_reduce");
   }
@@ -966,6 +968,8 @@ int fc_fwd(int in, int out, int has_bias, int batch, const float *x, const float
   if (small_fc_applies(batch, out, in)) return launch_small_fc(A, B, epi, batch, out, in, "fc_fwd_small");
   if (fc_x3_applies(FX_A_K_B_N, batch, out, in, x, w, in, out))
     return fc_x3_run(FX_A_K_B_N, x, w, in, out, epi, batch, out, in, "fc_fwd_x3", "fc_fwd_splitk_reduce");
+  if (fc_f32_applies(batch, out, in, x, w))
+    return fc_f32_run(x, w, epi, batch, out, in, "fc_fwd_f32", "fc_fwd_splitk_reduce");
   return launch_gemm<true, false, false, true>(A, B, epi, batch, out, in, true, "fc_fwd_gemm",
                                               "fc_fwd_splitk_reduce");
 }

@@ -199,6 +199,11 @@ bool fc_x3_applies(FxRows rows, int M, int N, int K, const float *A, const float
 size_t fc_x3_workspace_bytes(int M, int N, int K);
 int fc_x3_run(FxRows rows, const float *A, const float *B, int lda, int ldb, const EpiRowMajor &epi, int M, int N, int K,
               const char *tag, const char *reduce_tag);
+// fc_f32.hip: C = A B of plain matrices in fp32 with the bits of launch_gemm, A rows along k, B rows along n
+bool fc_f32_applies(int M, int N, int K, const float *A, const float *B);
+int fc_f32_run(const float *A, const float *B, const EpiRowMajor &epi, int M, int N, int K, const char *tag, const char *reduce_tag);
+int fc_f32_run_act(const float *A, const float *B, const EpiRowMajorAct &epi, int M, int N, int K, const char *tag,
+                   const char *reduce_tag);
 int fc_x3_run_act(const float *A, const float *B, int lda, int ldb, const EpiRowMajorAct &epi, int M, int N, int K,
                   const char *tag, const char *reduce_tag);
 
