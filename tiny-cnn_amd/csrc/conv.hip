@@ -790,7 +790,7 @@ conv_dx_first_mfma_kernel(const float *__restrict__ dy, const float *__restrict_
     f4 sq[POOLED ? 1 : DXM_MAXCH];
     if constexpr (POOLED) {
       // by words of four windows: the kernel is cold code, and a thread's single windows were 32 loads and 64
-      // stores of it (5x5, 3 -> 32 channels of 32x32, batch 128: 7.8 us of 25.4 in front of the products, now 5.6 of 23)
+      // stores of it (5x5, 3 -> 32 channels of 32x32, batch 128: 7.8 us of 25.4 in front of the products, now 6.4 of 23.8)
 #pragma unroll
       for (int i = 0; i < G::WPT; ++i) {
         int c, pr, col;

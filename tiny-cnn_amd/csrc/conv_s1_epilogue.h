@@ -81,19 +81,27 @@ __device__ __forceinline__ void s1_epilogue(const ConvS1Args &a, const floatx16 
       }
       if constexpr (TC <= 16) {
         if (!a.part && a.pool_out) {
-          // A 32-pixel block is whole rows of TC pixels, the first one even: the window of the
-          // lane with an even row and column is its own value, lane^1's, lane^TC's and
-          // lane^(TC+1)'s, scanned in that order with strict '>' from lowest()
-          // (maxpool_op_internal.h:17-47). Every lane runs the exchange, the anchors store.
-          const bool anchor = !(lane & 1) && !(lane & TC);
+          // A 32-pixel block is whole rows of TC pixels, the first one even: a window belongs to four lanes, l, l^1, l^TC and
+          // l^(TC+1) in scan order. They turn their 4 x 4 values of four channels and each pools the channel of its place, with
+          // strict '>' from lowest() (maxpool_op_internal.h:17-47): a quarter of the code, which runs once, cold, and of the
+          // stores of a lane that pools every channel and leaves three idle (16x16, 32 -> 32, 5x5: fp32,
+          // batch 128, without y 22.2 / 20.8; three parts, batch 1000, with y 80 / 70).
+          const bool right = lane & 1, below = lane & TC;
           const int pw2 = a.OW >> 1, pohw = (a.OH >> 1) * pw2;
           const size_t pobase = static_cast<size_t>(img) * a.MC * pohw + (oy >> 1) * pw2 + (ox >> 1);
-          const int pix = oy * a.OW + ox;
+          const int pix = (oy & ~1) * a.OW + (ox & ~1);
 #pragma unroll
-          for (int rr = 0; rr < 16; ++rr) {
-            const int m = mb + 8 * (rr >> 2) + (rr & 3);
-            const float right = s1_lane_xor1(v[rr]);
-            const float w4[4] = {v[rr], right, s1_lane_xor<TC>(v[rr]), s1_lane_xor<TC>(right)};
+          for (int g = 0; g < 4; ++g) {
+            float l[2], r2[2];   // this row's two values of channel 2k + right
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+              const float v0 = v[4 * g + 2 * k], v1 = v[4 * g + 2 * k + 1];
+              const float from1 = s1_lane_xor1(v1), from0 = s1_lane_xor1(v0);
+              l[k]  = right ? from1 : v0;
+              r2[k] = right ? v1 : from0;
+            }
+            const float l0 = s1_lane_xor<TC>(l[0]), r0 = s1_lane_xor<TC>(r2[0]), l1 = s1_lane_xor<TC>(l[1]), r1 = s1_lane_xor<TC>(r2[1]);
+            const float w4[4] = {below ? l1 : l[0], below ? r1 : r2[0], below ? l[1] : l0, below ? r2[1] : r0};
             float best = -3.402823466e+38f;
             int sel    = -1;
 #pragma unroll
@@ -102,7 +110,8 @@ __device__ __forceinline__ void s1_epilogue(const ConvS1Args &a, const floatx16 
                 best = w4[k];
                 sel  = k;
               }
-            if (anchor && m < a.MC) {
+            const int m = mb + 8 * g + (right ? 1 : 0) + (below ? 2 : 0);
+            if (m < a.MC) {
               const size_t at = pobase + static_cast<size_t>(m) * pohw;
               a.pool_out[at]    = best;
               a.pool_argmax[at] = sel < 0 ? 0 : m * ohw + pix + (sel >> 1) * a.OW + (sel & 1);
