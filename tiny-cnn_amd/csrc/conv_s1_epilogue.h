@@ -85,7 +85,7 @@ __device__ __forceinline__ void s1_epilogue(const ConvS1Args &a, const floatx16 
           // l^(TC+1) in scan order. They turn their 4 x 4 values of four channels and each pools the channel of its place, with
           // strict '>' from lowest() (maxpool_op_internal.h:17-47): a quarter of the code, which runs once, cold, and of the
           // stores of a lane that pools every channel and leaves three idle (16x16, 32 -> 32, 5x5: fp32,
-          // batch 128, without y 22.2 / 20.8; three parts, batch 1000, with y 80 / 70).
+          // batch 128, without y 22.2 / 20.8; three parts, batch 1000, with y 80 / 75).
           const bool right = lane & 1, below = lane & TC;
           const int pw2 = a.OW >> 1, pohw = (a.OH >> 1) * pw2;
           const size_t pobase = static_cast<size_t>(img) * a.MC * pohw + (oy >> 1) * pw2 + (ox >> 1);
