@@ -98,3 +98,21 @@ def test_filters_packed_along_are_those_written_last(T, convs):
         for i, (a, b) in enumerate(zip(have, results(fresh))):
             assert np.array_equal(a, b), i
         fresh.close()
+
+
+def test_more_work_items_than_a_grid_has_in_one_direction(T):
+    """65535 images of 513 blocks of channels, a workgroup of two waves each: more than 2^32 work-items."""
+    rng = np.random.default_rng(65)
+    k, co, batch = 3, 32 * 513, 65535
+    x = rng.standard_normal((batch, 1, k, k)).astype(np.float32)
+    wt = rng.uniform(-0.3, 0.3, (co, 1, k, k)).astype(np.float32)
+    b = rng.standard_normal(co).astype(np.float32)
+    y = T.DevBuf((batch * co,))
+    T.profile_begin()
+    T.conv2d_fwd(T.conv_desc(k, k, 1, k, k, co), batch, T.to_device(x), T.to_device(wt), T.to_device(b), y)
+    assert any(r["tag"].startswith("conv_fwd_small ") for r in T.profile_end())
+    bound = 2.0 ** -24 * (k * k + 2) * (np.abs(x).max() * np.abs(wt).reshape(co, -1).sum(1) + np.abs(b))
+    for i in (0, 1, 4095, 32768, 65533, 65534):
+        got = T.DevBuf.view(y.ptr.value + 4 * i * co, (co,)).numpy()
+        want = wt.reshape(co, -1).astype(np.float64) @ x[i].ravel().astype(np.float64) + b
+        assert (np.abs(got - want) <= bound).all(), i

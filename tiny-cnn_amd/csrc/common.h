@@ -146,6 +146,10 @@ void prof_launch_events(hipEvent_t *start, hipEvent_t *stop);  // nulls outside 
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 inline size_t ceil_div_sz(size_t a, size_t b) { return (a + b - 1) / b; }
 
+// Workgroups of up to 256 threads that a launch may have in one direction: at 2^32 work-items the number wraps, and
+// the launch does a part of the work without an error.
+constexpr int GRID_X_MAX = (1 << 24) - 1;
+
 // Workgroups are handed to the eight XCDs (each with its own L2) round-robin in launch order.
 // This renumbers a workgroup's linear id so that ids that are neighbours after the renumbering,
 // which is how the kernels below give neighbouring pieces of one image to their workgroups, run

@@ -434,7 +434,7 @@ AnyPlan plan_tile(const AnyArgs &base, int batch, int mb, int nb, int wk) {
   }
   const int all = ceil_div(a.KC, 8), m_tiles = ceil_div(a.M, 16 * mb);
   const long blocks = tiles * m_tiles;
-  if (tiles >= (1L << 31) || m_tiles > 65535) return p;
+  if (tiles > GRID_X_MAX || m_tiles > 65535) return p;
   auto bytes = [&](int groups) {
     return 16 * static_cast<size_t>(groups) * plane * X3_PARTS + 8 * static_cast<size_t>(groups) * most_taps;
   };

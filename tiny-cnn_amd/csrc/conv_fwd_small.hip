@@ -45,7 +45,7 @@ struct FwdSmallArgs {
   int crs, x_floats;
   FastDiv div_pitch, div_rows_in, div_col_tiles;
   int batch, workgroups;     // of the convolution
-  int pack_threads;
+  int packers, pack_threads; // workgroups in front of them
 };
 
 // Workgroups in front of the convolution's own pack filters that later layers read: in a net whose
@@ -55,14 +55,14 @@ struct FwdSmallArgs {
 constexpr int FWD_SMALL_PACKERS = 192;
 struct NoPacks {};
 template <class Packs>
-__device__ __forceinline__ bool fwd_small_packs(const FwdSmallArgs &a, const Packs &packs) {
+__device__ __forceinline__ bool fwd_small_packs(const FwdSmallArgs &a, const Packs &packs, const int id) {
   if constexpr (std::is_same_v<Packs, PackJobs>) {
-    if (blockIdx.x >= gridDim.x - a.workgroups) return false;
+    if (id >= a.packers) return false;
     // (whole pieces of a job's 256 threads: of three waves two work)
     const int threads = blockDim.x < 256 ? 128 : 256;
     if (static_cast<int>(threadIdx.x) >= threads) return true;
-    const int step = (gridDim.x - a.workgroups) * threads;
-    for (int t = blockIdx.x * threads + threadIdx.x; t < a.pack_threads; t += step) pack_any(packs, t);
+    const int step = a.packers * threads;
+    for (int t = id * threads + threadIdx.x; t < a.pack_threads; t += step) pack_any(packs, t);
     return true;
   }
   return false;
@@ -194,14 +194,16 @@ __device__ __forceinline__ void fwd_small_store(const T v, const __amdgpu_buffer
 template <int NS, class Packs, bool PLAIN>
 __global__ void __launch_bounds__(256, PLAIN ? 4 : 3) conv_fwd_small_kernel(const FwdSmallArgs a, const Packs packs) {
   extern __shared__ __align__(16) float lds[];
-  if (fwd_small_packs(a, packs)) return;
+  const int id = blockIdx.x + gridDim.x * blockIdx.y;
+  if (id >= a.packers + a.workgroups) return;   // (the last row of a grid of several)
+  if (fwd_small_packs(a, packs, id)) return;
   float *xs = lds;
   float *ws = lds + a.x_floats;  // [32][crs], rows past Cout are zero
   float *bs = ws + 32 * a.crs;   // [32] bias, zero past Cout or without bias
   int *offs = reinterpret_cast<int *>(bs + 32);  // [2][NS] patch offset of k = 2s, 2s + 1 (0 past K)
   const int tid = threadIdx.x, lane = tid & 63;
   // (an image's bands share rows: they go to one XCD)
-  const int wg = xcd_compact_id(blockIdx.x - (gridDim.x - a.workgroups), a.workgroups);
+  const int wg = xcd_compact_id(id - a.packers, a.workgroups);
   const int bandi = wg % a.bands, img = (wg / a.bands) % a.batch, co0 = (wg / (a.bands * a.batch)) * 32;
   const int oy0 = bandi * a.band;
   const int nthr = blockDim.x;  // one wave per tile of the band, two to four waves
@@ -430,14 +432,17 @@ FwdSmallPlan make_fwd_small_plan(int batch, int C, int Kc, int H, int W, int OH,
 template <int NS, class Packs>
 int launch_fwd_small(const FwdSmallPlan &p, const Packs &packs, int pack_blocks) {
   const int tiles = (p.a.band / 2) * p.a.col_tiles;
-  const FwdSmallArgs &a = p.a;
+  FwdSmallArgs a = p.a;
   auto plain = [](int kind) { return kind == TDH_ACT_RELU || kind == TDH_ACT_NONE; };
   const dim3 block(64 * std::min(4, std::max(2, tiles)));
-  const dim3 grid(a.workgroups + std::min(block.x < 256 ? 2 * pack_blocks : pack_blocks, FWD_SMALL_PACKERS));
+  a.packers = std::min(block.x < 256 ? 2 * pack_blocks : pack_blocks, FWD_SMALL_PACKERS);
+  // (a grid takes less than 2^32 work-items in one direction)
+  const int total = a.packers + a.workgroups, rows = ceil_div(total, GRID_X_MAX);
+  const dim3 grid(ceil_div(total, rows), rows);
   if (a.Kc % 32 == 0 && (!a.act_out || plain(a.act_kind)) && (!a.pool_act_out || plain(a.pool_act_kind)))
-    TDH_LAUNCH((conv_fwd_small_kernel<NS, Packs, true>), grid, block, p.lds_bytes, ctx().stream, p.a, packs);
+    TDH_LAUNCH((conv_fwd_small_kernel<NS, Packs, true>), grid, block, p.lds_bytes, ctx().stream, a, packs);
   else
-    TDH_LAUNCH((conv_fwd_small_kernel<NS, Packs, false>), grid, block, p.lds_bytes, ctx().stream, p.a, packs);
+    TDH_LAUNCH((conv_fwd_small_kernel<NS, Packs, false>), grid, block, p.lds_bytes, ctx().stream, a, packs);
   TDH_LAUNCH_CHECK();
   return TDH_OK;
 }
