@@ -3,6 +3,8 @@ filters of later layers it packs along), against the operators of the layers: th
 import numpy as np
 import pytest
 
+from test_gpu_exceptional_values import check
+
 pytestmark = pytest.mark.gpu
 
 
@@ -98,6 +100,44 @@ def test_filters_packed_along_are_those_written_last(T, convs):
         for i, (a, b) in enumerate(zip(have, results(fresh))):
             assert np.array_equal(a, b), i
         fresh.close()
+
+
+@pytest.mark.parametrize("w,h,ci,k,co,batch", [
+    (32, 32, 3, 5, 32, 128),    # 75 taps of 80
+    (28, 28, 1, 5, 33, 256),    # 25 of 32
+    (30, 20, 3, 3, 20, 160),    # 27 of 32
+    (40, 24, 6, 4, 16, 100),    # all 96
+])
+def test_what_fills_up_the_taps_is_no_part_of_a_sum(T, w, h, ci, k, co, batch):
+    """Infinities and NaN under the first tap of the first channel, whose place the taps that fill up a block of 16 take."""
+    rng = np.random.default_rng(63)
+    same = k % 2 == 1
+    ow, oh = (w, h) if same else (w - k + 1, h - k + 1)
+    ow, oh = ow - ow % 2, oh - oh % 2
+    w, h = (ow, oh) if same else (ow + k - 1, oh + k - 1)
+    d = T.conv_desc(w, h, ci, k, k, co, pad_same=same)
+    x = rng.standard_normal((batch, ci, h, w)).astype(np.float32)
+    for i, v in enumerate([np.inf, -np.inf, np.nan, np.inf, 3e37]):
+        x[rng.integers(batch), 0, rng.integers(h), rng.integers(w)] = v
+        x[i, 0, 0, 0] = v
+    wt = rng.uniform(0.1, 0.3, (co, ci, k, k)).astype(np.float32) * rng.choice([-1, 1], (co, ci, k, k)).astype(np.float32)
+    b = rng.standard_normal(co).astype(np.float32)
+    xd, n = T.to_device(x), co * ow * oh
+    y, p, argmax = T.DevBuf((batch, n)), T.DevBuf((batch, n // 4)), T.DevBuf((batch, n // 4), np.int32)
+    T.profile_begin()
+    T.conv2d_fwd(d, batch, xd, T.to_device(wt), T.to_device(b), y)
+    assert any(r["tag"].startswith("conv_fwd_small ") for r in T.profile_end())
+    with np.errstate(invalid="ignore"):
+        check(y.numpy(), conv64(x, wt, b, k, 1, k // 2 if same else 0), "y")
+    T.maxpool_fwd(T.pool_desc(ow, oh, co, 2, stride_w=2, stride_h=2), batch, y, p, argmax)
+    net = T.Net([T.L_conv(w, h, ci, k, co, pad_same=same), T.L_maxpool(ow, oh, co, 2, 2)], batch, 0)
+    net.set_param(0, 0, wt.ravel())
+    net.set_param(0, 1, b)
+    net.forward(batch, xd)
+    assert np.array_equal(net.layer_out(0, batch).ravel(), y.numpy().ravel(), equal_nan=True)
+    assert np.array_equal(net.layer_out(1, batch).ravel(), p.numpy().ravel(), equal_nan=True)
+    assert np.array_equal(net.layer_argmax(1, batch).ravel(), argmax.numpy().ravel())
+    net.close()
 
 
 def test_more_work_items_than_a_grid_has_in_one_direction(T):

@@ -269,6 +269,10 @@ __global__ void __launch_bounds__(256, PLAIN ? 4 : 3) conv_fwd_small_kernel(cons
       const int cur = g & 1;
       if (g + 1 < NS / G) read_patch(g + 1);
       if (g + 2 < NS / G) read_offsets(g + 2);
+      if (g >= NS / G - 2 && 2 * G * (g + 1) > a.crs)   // (indices past the last tap: no infinity or NaN of the word they read)
+#pragma unroll
+        for (int j = 0; j < G; ++j)
+          if (2 * (g * G + j) + half >= a.crs) b0[cur][j] = b1[cur][j] = 0.0f;
 #pragma unroll
       for (int j = 0; j < G; ++j) {
         acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(areg[g * G + j], b0[cur][j], acc0, 0, 0, 0);
