@@ -140,6 +140,27 @@ def test_what_fills_up_the_taps_is_no_part_of_a_sum(T, w, h, ci, k, co, batch):
     net.close()
 
 
+@pytest.mark.parametrize("co", [3, 33])
+def test_planes_of_more_than_a_descriptor(T, co):
+    """2^25 pixels of 32 channels are 4 GiB, more than one buffer descriptor reaches."""
+    rng = np.random.default_rng(64)
+    w, h, k = 2050, 16500, 3
+    assert w * h > 1 << 25
+    x = rng.standard_normal((1, 1, h, w)).astype(np.float32)
+    wt = rng.uniform(-0.3, 0.3, (co, 1, k, k)).astype(np.float32)
+    b = rng.standard_normal(co).astype(np.float32)
+    y = T.DevBuf((co * h * w,))
+    T.profile_begin()
+    T.conv2d_fwd(T.conv_desc(w, h, 1, k, k, co, pad_same=True), 1, T.to_device(x), T.to_device(wt), T.to_device(b), y)
+    assert any(r["tag"].startswith("conv_fwd_small ") for r in T.profile_end())
+    bound = 2.0 ** -24 * (k * k + 2) * (np.abs(x).max() * np.abs(wt).reshape(co, -1).sum(1) + np.abs(b))
+    for row in (1, 8191, h - 2):
+        want = conv64(x[:, :, row - 1:row + 2], wt, b, k, 1, 1)[0, :, 1]
+        for c in range(co):
+            got = T.DevBuf.view(y.ptr.value + 4 * (c * h + row) * w, (w,)).numpy()
+            assert (np.abs(got - want[c]) <= bound[c]).all(), (row, c)
+
+
 def test_more_work_items_than_a_grid_has_in_one_direction(T):
     """65535 images of 513 blocks of channels, a workgroup of two waves each: more than 2^32 work-items."""
     rng = np.random.default_rng(65)

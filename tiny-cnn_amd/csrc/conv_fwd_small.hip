@@ -44,6 +44,7 @@ struct FwdSmallArgs {
   int rows_in, pitch, plane;
   int crs, x_floats;
   FastDiv div_pitch, div_rows_in, div_col_tiles;
+  int co_step;               // output channels of a workgroup
   int batch, workgroups;     // of the convolution
   int packers, pack_threads; // workgroups in front of them
 };
@@ -204,7 +205,7 @@ __global__ void __launch_bounds__(256, PLAIN ? 4 : 3) conv_fwd_small_kernel(cons
   const int tid = threadIdx.x, lane = tid & 63;
   // (an image's bands share rows: they go to one XCD)
   const int wg = xcd_compact_id(id - a.packers, a.workgroups);
-  const int bandi = wg % a.bands, img = (wg / a.bands) % a.batch, co0 = (wg / (a.bands * a.batch)) * 32;
+  const int bandi = wg % a.bands, img = (wg / a.bands) % a.batch, co0 = (wg / (a.bands * a.batch)) * (PLAIN ? 32 : a.co_step);
   const int oy0 = bandi * a.band;
   const int nthr = blockDim.x;  // one wave per tile of the band, two to four waves
   fwd_small_stage<NS>(a, xs, ws, bs, offs, img, co0, oy0, tid, nthr);
@@ -228,7 +229,7 @@ __global__ void __launch_bounds__(256, PLAIN ? 4 : 3) conv_fwd_small_kernel(cons
   const uint32_t lane_out = half * 4 * ohw + nl, lane_window = even ? lane_out : lane_out - 1 + ohw;
   const uint32_t lane_pool = half * 4 * pohw + (nl >> 1) + (even ? 0 : pohw);
   const float floor_v = a.pool_act_kind == TDH_ACT_RELU ? 0.0f : -INFINITY;  // relu as a max
-  const int channels  = PLAIN ? 32 : min(32, a.Kc - co0);
+  const int channels  = PLAIN ? 32 : min(a.co_step, a.Kc - co0);
   auto planes = [&](auto *p, const uint32_t plane) {   // the planes of the workgroup's channels
     return __builtin_amdgcn_make_buffer_rsrc(p ? p + (static_cast<size_t>(img) * a.Kc + co0) * plane : nullptr, 0,
                                              p ? 4u * channels * plane : 0u, 0x00027000);
@@ -387,14 +388,19 @@ FwdSmallPlan make_fwd_small_plan(int batch, int C, int Kc, int H, int W, int OH,
   a.C = C; a.Kc = Kc; a.H = H; a.W = W; a.OH = OH; a.OW = OW;
   a.R = R; a.S = S; a.sh = sh; a.sw = sw; a.dh = dh; a.dw = dw; a.ph = ph; a.pw = pw;
   a.crs = C * R * S;
-  // (a workgroup's 32 planes are one buffer)
-  if (static_cast<long long>(OH) * OW >= 1LL << 25) return p;
+  // A workgroup's planes are one buffer, with FWD_SMALL_NOWHERE behind it: of planes of 2^25 pixels and more it takes
+  // fewer than 32 (1 input channel of 2050x16500, 3x3, us by the general kernel / here: to 3 channels 1015 / 636,
+  // to 33 3619 / 2155).
+  auto buffer = [&](int channels) { return 4LL * std::min(channels, Kc) * OH * OW; };
+  a.co_step = 32;
+  while (a.co_step > 1 && buffer(a.co_step) > FWD_SMALL_NOWHERE) a.co_step /= 2;
+  if (buffer(a.co_step) > FWD_SMALL_NOWHERE) return p;
   if (a.crs > 96 || batch < 1 || batch > 65535 || OH < 1 || OW < 1) return p;
   p.ns = ((a.crs + 1) / 2 + 7) / 8 * 8;
   a.col_tiles = ceil_div(OW, 32);
   a.pitch     = (a.col_tiles * 32 - 1) * sw + (S - 1) * dw + 1;
   a.pitch |= 1;
-  const int co_tiles = ceil_div(Kc, 32);
+  const int co_tiles = ceil_div(Kc, a.co_step);
   if (co_tiles > 65535) return p;
   const int cus  = ctx().compute_units > 0 ? ctx().compute_units : 256;
   const int OH2  = (OH + 1) & ~1;
@@ -443,7 +449,7 @@ int launch_fwd_small(const FwdSmallPlan &p, const Packs &packs, int pack_blocks)
   // (a grid takes less than 2^32 work-items in one direction)
   const int total = a.packers + a.workgroups, rows = ceil_div(total, GRID_X_MAX);
   const dim3 grid(ceil_div(total, rows), rows);
-  if (a.Kc % 32 == 0 && (!a.act_out || plain(a.act_kind)) && (!a.pool_act_out || plain(a.pool_act_kind)))
+  if (a.Kc % 32 == 0 && a.co_step == 32 && (!a.act_out || plain(a.act_kind)) && (!a.pool_act_out || plain(a.pool_act_kind)))
     TDH_LAUNCH((conv_fwd_small_kernel<NS, Packs, true>), grid, block, p.lds_bytes, ctx().stream, a, packs);
   else
     TDH_LAUNCH((conv_fwd_small_kernel<NS, Packs, false>), grid, block, p.lds_bytes, ctx().stream, a, packs);
