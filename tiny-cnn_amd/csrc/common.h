@@ -500,6 +500,7 @@ size_t conv_s1_packed_bytes(int kind, int RS, int KC, int MC);
 // conv_dw.hip: stride-1 weight gradient from LDS-staged tiles (3x3 and 5x5 windows)
 bool conv_dw_halo_applicable(int R, int S, int batch, int C, int Kc, int H, int W, int OH, int OW,
                              int ph, int pw);
+bool conv_dw_halo_f32_applicable(int R, int S, int batch, int C, int Kc, int H, int W, int OH, int OW, int ph, int pw);
 size_t conv_dw_halo_workspace_bytes(int R, int S, int batch, int C, int Kc, int H, int W, int OH,
                                     int OW, int ph, int pw);
 // ... of the kernel that conv_dw_halo_run takes for these tensors
@@ -542,8 +543,9 @@ int conv_bwd_pair_run(int R, int S, int batch, int C, int Kc, int H, int W, int 
                       float *db, int accumulate);
 size_t conv_bwd_pair_workspace_bytes(int R, int S, int batch, int C, int Kc, int H, int W, int ph, int pw);
 // workspace bytes the op may ask for, whichever of its kernels runs (so a net can reserve it before
-// graph capture), and what one call of conv2d_bwd without packed filters takes
-size_t conv2d_workspace_bytes(const tdh_conv_desc *d, int batch);
+// graph capture; f32_gradients: of a net whose steps keep to fp32), and what one call of conv2d_bwd without
+// packed filters takes
+size_t conv2d_workspace_bytes(const tdh_conv_desc *d, int batch, bool f32_gradients = false);
 size_t conv2d_declared_bytes(const tdh_conv_desc *d, int batch);
 size_t conv2d_bwd_workspace_bytes(const tdh_conv_desc *d, int batch, const float *x, const float *dy, bool dx, bool dw,
                                   bool db, int accumulate);

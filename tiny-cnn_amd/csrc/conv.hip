@@ -1213,7 +1213,7 @@ size_t conv2d_declared_bytes(const tdh_conv_desc *d, int batch) {
   return total;
 }
 
-size_t conv2d_workspace_bytes(const tdh_conv_desc *d, int batch) {
+size_t conv2d_workspace_bytes(const tdh_conv_desc *d, int batch, bool f32_gradients) {
   const ConvGeom g = make_geom(d);
   const int ohw = g.OH * g.OW, crs = g.C * g.R * g.S;
   size_t total = 0;
@@ -1231,7 +1231,10 @@ size_t conv2d_workspace_bytes(const tdh_conv_desc *d, int batch) {
   total += first_both_workspace_bytes(d, g, batch);
   if (g.sh == 1 && g.sw == 1)
     total += conv_dw_halo_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
-  total += conv_dw_any_most_bytes(shape_of(g, batch), true);
+  // (nothing for a kernel that the dispatch does not come to, at this batch or a smaller one: it may take up to 1024 slices)
+  const bool halo = g.sh == 1 && g.sw == 1 &&
+                    conv_dw_halo_f32_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
+  if (!f32_gradients && !halo && !d->tbl) total += conv_dw_any_most_bytes(shape_of(g, batch), true);
   total += conv_any_fwd_workspace_bytes(shape_of(g, batch)) + conv_any_dx_workspace_bytes(shape_of(g, batch));
   if (g.sh == 1 && g.sw == 1) {  // LDS-halo kernel: repacked filters and split partial sums
     total += conv_s1_workspace_bytes(g.R, g.S, batch, g.C, g.Kc, 0, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);

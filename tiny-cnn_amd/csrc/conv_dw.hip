@@ -598,6 +598,11 @@ bool conv_dw_halo_applicable(int R, int S, int batch, int C, int Kc, int H, int 
          make_dw_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw).ok;
 }
 
+// the fp32 kernel's part of it: a shape that has a plan at one batch has one at every smaller batch
+bool conv_dw_halo_f32_applicable(int R, int S, int batch, int C, int Kc, int H, int W, int OH, int OW, int ph, int pw) {
+  return make_dw_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw).ok;
+}
+
 size_t conv_dw_halo_workspace_bytes(int R, int S, int batch, int C, int Kc, int H, int W, int OH,
                                     int OW, int ph, int pw) {
   const DwxPlan x3   = make_dwx_plan(R, S, batch, C, Kc, H, W, OH, OW, ph, pw);

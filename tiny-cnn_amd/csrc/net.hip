@@ -601,7 +601,7 @@ int forward(tdh_net *net, int batch, const float *x, const float *xent_t = nullp
     const tdh_layer &s = L.spec;
     switch (s.kind) {
       case TDH_L_CONV:
-        TDH_TRY(ws_begin(conv2d_workspace_bytes(&s.conv, batch)));
+        TDH_TRY(ws_begin(conv2d_workspace_bytes(&s.conv, batch, has_batchnorm(net))));
       {
         const PackedFilters wp = packed_filters(L, batch, 0);
         const bool has_wp = static_cast<bool>(wp);
@@ -821,7 +821,7 @@ int tdh_net_create(const tdh_layer *layers, int n_layers, int max_batch, int fla
       if ((rc = tdh_memcpy_h2d(L.tbl_dev, L.tbl.data(), L.tbl.size()))) break;
     }
     size_t need = 0;
-    if (L.spec.kind == TDH_L_CONV) need = conv2d_workspace_bytes(&L.spec.conv, max_batch);
+    if (L.spec.kind == TDH_L_CONV) need = conv2d_workspace_bytes(&L.spec.conv, max_batch, has_batchnorm(net));
     if (L.spec.kind == TDH_L_FC) need = fc_workspace_bytes(L.spec.fc_in, L.spec.fc_out, max_batch);
     if (L.spec.kind == TDH_L_AVEPOOL) need = avepool_workspace_bytes(&L.spec.pool, max_batch);
     if (L.spec.kind == TDH_L_BATCHNORM) need = batchnorm_workspace_bytes(L.spec.bn_channels, max_batch);
@@ -1226,7 +1226,7 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
     }
     switch (s.kind) {
       case TDH_L_CONV:
-        TDH_TRY(ws_begin((forked || as_forked ? 3 : 1) * conv2d_workspace_bytes(&s.conv, batch)));
+        TDH_TRY(ws_begin((forked || as_forked ? 3 : 1) * conv2d_workspace_bytes(&s.conv, batch, has_batchnorm(net))));
       {
         const PoolGather *gp = i == through_pool_for ? &through_pool : nullptr;
         const PackedFilters wp = conv_pair ? packed_as(L, CONV_PACK_X3, 1) : packed_filters(L, batch, 1);
