@@ -695,13 +695,12 @@ struct DxmGeom {
   static constexpr int RPW       = 4 / NMB;            // rows of the band a wave owns
   static constexpr int TILE_ROWS = DXM_WAVES * RPW;
   static constexpr int TROWS     = TILE_ROWS + KR - 1;
-  // floats per staged channel: the rows, a spare word for stores that fall outside the tile,
-  // padded to 16 (mod 32) so that four channels' rows lie in different banks
-  static constexpr int PLANE   = ((TROWS * OW + 1 + 15) / 32) * 32 + 16;
-  static constexpr int PER_ROW = POOLED ? OW / 2 : OW / 4;  // staging positions per row of them
-  static constexpr int NPOS    = (POOLED ? TROWS / 2 + 1 : TROWS) * PER_ROW;
+  // floats per staged channel: the rows, padded to 16 (mod 32) so that four channels' rows lie in different banks
+  static constexpr int PLANE   = ((TROWS * OW + 15) / 32) * 32 + 16;
+  // not pooled: staging positions, and channels per thread
+  static constexpr int PER_ROW = OW / 4, NPOS = TROWS * PER_ROW;
   static constexpr int GROUPS  = DXM_NT / NPOS;
-  static constexpr int CPT     = (DXM_MCH + GROUPS - 1) / GROUPS;  // channels per thread
+  static constexpr int CPT     = (DXM_MCH + GROUPS - 1) / GROUPS;
   // pooled: words of four windows, of a row of them and of a channel, a thread's share
   static constexpr int WPR = OW / 8, WPC = (TROWS / 2 + 1) * WPR, WORDS = DXM_MCH * WPC, WPT = (WORDS + DXM_NT - 1) / DXM_NT;
   static constexpr int WROW    = 4 * KR * KR;          // staged filter floats per output channel
@@ -709,7 +708,7 @@ struct DxmGeom {
   static constexpr int GATHER  = DXM_WAVES * RPW * OW * 17;
   static constexpr int STAGE   = DXM_MCH * PLANE + WL;
   static constexpr int LDS_FLOATS = STAGE > GATHER ? STAGE : GATHER;
-  static constexpr bool FITS = GROUPS >= 1 && CPT <= DXM_MAXCH && LDS_FLOATS * 4 <= 64 * 1024;
+  static constexpr bool FITS = (POOLED || (GROUPS >= 1 && CPT <= DXM_MAXCH)) && LDS_FLOATS * 4 <= 64 * 1024;
 };
 
 template <int KR, int KS, int NMB, bool POOLED, int DWNT = 0>
@@ -1608,7 +1607,8 @@ int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
   const ConvGeom g = make_geom(d);
   const int ohw = g.OH * g.OW, crs = g.C * g.R * g.S;
   if (dy_pool) {
-    // only the two first-layer kernels read the gradient this way, and they leave nothing over
+    // only the first-layer kernels read the gradient this way, and they leave nothing over: the matrix-core ones by words
+    // of four windows, the others by two
     tdh_pool_desc over{};
     over.in_w = g.OW; over.in_h = g.OH; over.in_c = g.Kc;
     over.pool_w = over.pool_h = over.stride_w = over.stride_h = 2;
@@ -1616,14 +1616,17 @@ int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
         (reinterpret_cast<uintptr_t>(dy_pool->g) & 7) || (reinterpret_cast<uintptr_t>(dy_pool->argmax) & 7) ||
         (db && !dw))
       return set_error(TDH_ERR_INVALID, "conv2d_bwd: the pooled gradient cannot be read for this layer");
-    if (dx && dw && conv_bwd_one_launch(d, batch, true))
+    const bool words = !((reinterpret_cast<uintptr_t>(dy_pool->g) | reinterpret_cast<uintptr_t>(dy_pool->argmax)) & 15);
+    if (dx && dw && words && conv_bwd_one_launch(d, batch, true))
       return run_first_both<true>(g, batch, x, nullptr, w, dx, dw, db, accumulate, dx_act, *dy_pool);
     DxsPlan dxs;
     small_cin_dx_plan(g, dxs);
     if (dx) {
-      if (first_dx_mfma<true>(g, batch, nullptr, w, dx, dx_act, *dy_pool, true)) {
+      if (words && first_dx_mfma<true>(g, batch, nullptr, w, dx, dx_act, *dy_pool, true)) {
         ProfScope prof("conv_dx_first_mfma", g.C, batch * g.H * g.W, g.Kc * g.R * g.S);
         first_dx_mfma<true>(g, batch, nullptr, w, dx, dx_act, *dy_pool, false);
+      } else if (!dxs.pooled_ok) {
+        return set_error(TDH_ERR_INVALID, "conv2d_bwd: the pooled gradient of this layer is read by aligned words");
       } else {
         ProfScope prof("conv_dx_small_cin", g.C, batch * g.H * g.W, g.Kc * g.R * g.S);
         launch_small_cin_dx_window<true>(g, dxs, batch, nullptr, w, dx, dx_act, *dy_pool);
