@@ -168,3 +168,17 @@ def test_weight_gradient_of_exceptional_values(T, where):
     assert any(e["tag"].startswith("conv_dw_db_any") for e in T.profile_end())
     for got, ref, name in zip((dw.numpy(), db.numpy()), weight_gradient(x, dy, 5, 5, False, (1, 1)), ("dw", "db")):
         check(got, ref, name)
+
+
+@pytest.mark.parametrize("cfg", [
+    # (us of the forward product by the generic kernel / by the one of any size)
+    (94, 10, 92, 1, 1, 11, True, (1, 1), 54, False),    # 14 / 28
+    (70, 59, 65, 1, 5, 56, False, (2, 2), 23, False),   # 33 / 53
+    (29, 82, 86, 3, 1, 2, False, (2, 2), 59, False),    # 26 / 39
+    (44, 43, 2, 7, 7, 39, True, (2, 2), 72, False),     # 17 / 24
+    (41, 70, 74, 7, 7, 6, True, (2, 2), 120, True),     # 717 / 311
+    (19, 74, 31, 7, 5, 2, True, (1, 1), 97, True),      # 211 / 73
+])
+def test_forward_product_takes_the_faster_kernel(T, cfg):
+    d, x, w, b, dy = operands(T, cfg, np.random.default_rng(46))
+    assert ("f" in run(T, d, x, w, b, dy)[2]) == cfg[9]

@@ -28,7 +28,7 @@
 // Reference: conv2d_op_internal.h:13-74 (forward), :79-158 (backward).
 #include <algorithm>
 
-#include "common.h"
+#include "gemm_mfma.h"
 #include "split_bf16.h"
 
 namespace tdh {
@@ -468,9 +468,12 @@ AnyPlan plan_tile(const AnyArgs &base, int batch, int mb, int nb, int wk) {
   const int by_lds    = static_cast<int>(160 * 1024 / p.lds_bytes);
   const int by_regs   = mb == 1 || mb * nb <= 4 ? 4 : 2;
   const int resident  = std::max(1, std::min(by_lds, by_regs));
-  const double full   = static_cast<double>(blocks) / 256;
-  const double at_once = std::min<double>(resident, std::ceil(full));
-  p.cost = 0.9 + std::max(1.0, full / resident) * std::max(alone + (at_once - 1) * shared * 0.36, at_once * shared);
+  // (whole rounds: 520 workgroups of which a compute unit holds two take twice the time of 512. 35x42, 125 -> 82, 3x3, stride
+  // 2, 11 images: 22 us estimated without, 44 in fact)
+  auto round = [&](double at_once) { return std::max(alone + (at_once - 1) * shared * 0.36, at_once * shared); };
+  const double whole = std::floor(static_cast<double>(blocks) / (256 * resident));
+  const double left  = std::ceil(static_cast<double>(blocks) / 256 - whole * resident);
+  p.cost = 0.9 + whole * round(resident) + (left > 0 ? round(left) : 0.0);
   p.ok = true;
   return p;
 }
@@ -621,14 +624,16 @@ int run_any(AnyPlan &p, const char *tag, int m, int n, int k) {
 
 }  // namespace
 
-// us of the packing launch, and of the generic kernel on `products` (rows of 32) with their split sums
+// us of the packing launch, and of the generic kernel on `products` (rows of 32) of a dX with their split sums
 constexpr double ANY_PACK_US = 5.0;
 double generic_us(double products) { return 11.0 + products / 16e6; }
 
 bool conv_any_fwd_applicable(const ConvShape &c) {
   if (ctx().keep_f32) return false;
+  // Of 1600 shapes (5 to 1150 us) this takes 1215; 51 of those are over 3 % faster by the generic kernel, 34 of the others here, and
+  // in all it is 97987 us there, 54671 here, 54325 with the faster one of each. 94x10, 92 -> 11, 1x1, 54 images 14 us there, 28 here.
   const AnyPlan &p = forward_plan(c);
-  return p.ok && p.cost + ANY_PACK_US < generic_us(static_cast<double>(c.batch) * c.OH * c.OW * ceil_div(c.Kc, 32) * 32 * c.C * c.R * c.S);
+  return p.ok && p.cost + ANY_PACK_US < gathered_gemm_us(c.Kc, c.batch * c.OH * c.OW, c.C * c.R * c.S);
 }
 bool conv_any_dx_applicable(const ConvShape &c, AnyOver over) {
   if (ctx().keep_f32) return false;
@@ -636,7 +641,10 @@ bool conv_any_dx_applicable(const ConvShape &c, AnyOver over) {
   if (!p.ok) return false;
   const double pixels = static_cast<double>(c.batch) * c.H * c.W, k = static_cast<double>(c.Kc) * c.R * c.S / (c.sh * c.sw);
   switch (over) {
-    // (a reduction of a few steps is all staging)
+    // A reduction of a few steps is all staging, of which the estimate knows too little. Of the shapes that it alone would
+    // take, how many are over 3 % slower here / there, and all of them in us, there / here: strided, k under 12 257 / 9
+    // (2251 / 2545), 24 to 48 40 / 149 (3436 / 2812), 48 to 96 4 / 192 (5249 / 3345); stride 1, k of 24 to 48 34 / 21 (686 /
+    // 731), 48 to 96 12 / 42 (973 / 845), 96 to 192 8 / 55 (1436 / 1055).
     case ANY_OVER_GENERIC:
       return k >= (c.sh * c.sw > 1 ? 48 : 96) && p.cost + ANY_PACK_US < generic_us(pixels * ceil_div(c.C, 32) * 32 * k);
     // The vector-ALU kernel is built for windows of 3 and 5; 7x7, us there / here: 41x40, 3 -> 105, 101 images 379 /

@@ -486,14 +486,14 @@ int launch_dw_inst(const DwHaloPlan &p) {
 
 template <int TC, bool VEC>
 int launch_dw_tc(const DwHaloPlan &p) {
-  if (p.rows_block == 1 && p.window == 3)
-    return p.wco == 2 ? launch_dw_inst<1, 3, TC, 2, 2, 1, 3, VEC>(p) : launch_dw_inst<1, 3, TC, 1, 4, 1, 3, VEC>(p);
-  if (p.rows_block == 1)
+  if (p.window == 5)
     return p.wco == 2 ? launch_dw_inst<1, 5, TC, 2, 2, 1, 5, VEC>(p) : launch_dw_inst<1, 5, TC, 1, 4, 1, 5, VEC>(p);
-  if (p.wco == 2) return launch_dw_inst<3, 3, TC, 2, 2, 1, 3, VEC>(p);
-  // 8 columns x 4 row groups would stage 17 words a thread; the plan leaves that tile out
+  if (p.wco == 2)
+    return p.rows_block == 1 ? launch_dw_inst<1, 3, TC, 2, 2, 1, 3, VEC>(p) : launch_dw_inst<3, 3, TC, 2, 2, 1, 3, VEC>(p);
+  // 8 columns x 4 row groups would stage 17 words a thread with the filter rows together; the plan leaves that tile out
+  constexpr int TC1 = TC == 8 ? 16 : TC;
   if (TC == 8) return set_error(TDH_ERR_INVALID, "conv_dw_halo_run: tile not built");
-  return launch_dw_inst<3, 3, (TC == 8 ? 16 : TC), 1, 4, 1, 3, VEC>(p);
+  return p.rows_block == 1 ? launch_dw_inst<1, 3, TC1, 1, 4, 1, 3, VEC>(p) : launch_dw_inst<3, 3, TC1, 1, 4, 1, 3, VEC>(p);
 }
 
 template <bool VEC>
