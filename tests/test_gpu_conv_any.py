@@ -182,3 +182,16 @@ def test_weight_gradient_of_exceptional_values(T, where):
 def test_forward_product_takes_the_faster_kernel(T, cfg):
     d, x, w, b, dy = operands(T, cfg, np.random.default_rng(46))
     assert ("f" in run(T, d, x, w, b, dy)[2]) == cfg[9]
+
+
+@pytest.mark.parametrize("cfg", [
+    # (us of dX by the stride-1 kernel / by the one of any size)
+    (59, 13, 51, 5, 5, 139, True, (1, 1), 2, False),   # 22 / 56
+    (55, 7, 23, 3, 3, 157, True, (1, 1), 8, False),    # 16 / 31
+    (77, 9, 94, 5, 5, 113, False, (1, 1), 2, False),   # 30 / 51
+    (43, 31, 94, 3, 3, 74, True, (1, 1), 6, True),     # 40 / 25
+    (19, 89, 64, 3, 3, 21, True, (1, 1), 11, True),    # 26 / 16
+])
+def test_input_gradient_of_poorly_filled_tiles_takes_the_faster_kernel(T, cfg):
+    d, x, w, b, dy = operands(T, cfg, np.random.default_rng(47))
+    assert ("b" in run(T, d, x, w, b, dy)[2]) == cfg[9]

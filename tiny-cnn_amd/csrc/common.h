@@ -494,7 +494,7 @@ bool conv_s1_fuses_pool(int R, int S, int batch, int KC, int MC, int IH, int IW,
 bool conv_s1_single_pass(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW,
                          int ph, int pw);
 // conv_packed_kind / conv_packed_bytes of a shape this file runs
-double conv_s1_fill(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw);
+double conv_s1_fill(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw, double *us);
 int conv_s1_packed_kind(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw);
 size_t conv_s1_packed_bytes(int kind, int RS, int KC, int MC);
 // conv_dw.hip: stride-1 weight gradient from LDS-staged tiles (3x3 and 5x5 windows)
@@ -520,7 +520,7 @@ struct ConvShape {
 // the kernel that would compute dX otherwise: the generic GEMM, a first layer's, a stride-1 kernel with poorly filled tiles
 enum AnyOver { ANY_OVER_GENERIC, ANY_OVER_FIRST, ANY_OVER_STRIDE1 };
 bool conv_any_fwd_applicable(const ConvShape &c);   // in the place of the generic GEMM
-bool conv_any_dx_applicable(const ConvShape &c, AnyOver over);
+bool conv_any_dx_applicable(const ConvShape &c, AnyOver over, double other_us = 0.0);   // (other_us: ANY_OVER_STRIDE1's estimate of itself)
 size_t conv_any_fwd_workspace_bytes(const ConvShape &c);
 size_t conv_any_dx_workspace_bytes(const ConvShape &c);
 int conv_any_fwd_run(const ConvShape &c, const float *x, const float *w, const float *bias, float *out, float *act_out,

@@ -1152,15 +1152,18 @@ static ConvShape shape_of(const ConvGeom &g, int batch) {
   return {batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.R, g.S, g.sh, g.sw, g.dh, g.dw, g.pad_h, g.pad_w};
 }
 // Gradients of too few workgroups for the three-part stride-1 kernel take the fp32 one, unless its tiles are less
-// than four fifths full (columns come in 8 to 64, channels in 32 or 64): then the kernel of any size, dX in us
-// there / here, packing included: 65x40, 26 -> 30, 5x5, 12 images 45 / 25, 43x31, 94 -> 74, 3x3, 6 images 40 /
-// 25, 19x89, 64 -> 21, 3x3, 11 images 26 / 16. (The forward product would gain as much; there the operator's and
+// than four fifths full (columns come in 8 to 64, channels in 32 or 64) and the kernel of any size is estimated to be the
+// faster one. dX in us there / here, packing included: 65x40, 26 -> 30, 5x5, 12 images 45 / 25, 43x31, 94 -> 74, 3x3, 6
+// images 40 / 25, 19x89, 64 -> 21, 3x3, 11 images 26 / 16, but 59x13, 51 -> 139, 5x5, 2 images 22 / 56. Of 800
+// such shapes 617 go there, 27 of them over 3 % slower than here (all 800 would be 162): 24266 us / 18356 in all. (The forward product would gain as much; there the operator's and
 // a net's inference are one product, and the net's may take the layers behind along.)
 constexpr double ANY_FILL = 0.8;
 // (a train step, which adds to its gradients, has the same bits with filters that the net has packed for the stride-1 kernel)
 static bool dx_any_over_stride1(const ConvGeom &g, int batch, int accumulate) {
-  return !accumulate && conv_s1_fill(g.R, g.S, batch, g.Kc, g.C, g.OH, g.OW, g.H, g.W, g.R - 1 - g.pad_h, g.S - 1 - g.pad_w) < ANY_FILL &&
-         conv_any_dx_applicable(shape_of(g, batch), ANY_OVER_STRIDE1);
+  double us = 0.0;
+  return !accumulate &&
+         conv_s1_fill(g.R, g.S, batch, g.Kc, g.C, g.OH, g.OW, g.H, g.W, g.R - 1 - g.pad_h, g.S - 1 - g.pad_w, &us) < ANY_FILL &&
+         conv_any_dx_applicable(shape_of(g, batch), ANY_OVER_STRIDE1, us);
 }
 
 static bool fwd_small_applies(const ConvGeom &g, int batch) {

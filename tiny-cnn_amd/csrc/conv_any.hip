@@ -635,7 +635,7 @@ bool conv_any_fwd_applicable(const ConvShape &c) {
   const AnyPlan &p = forward_plan(c);
   return p.ok && p.cost + ANY_PACK_US < gathered_gemm_us(c.Kc, c.batch * c.OH * c.OW, c.C * c.R * c.S);
 }
-bool conv_any_dx_applicable(const ConvShape &c, AnyOver over) {
+bool conv_any_dx_applicable(const ConvShape &c, AnyOver over, double other_us) {
   if (ctx().keep_f32) return false;
   const AnyPlan &p = backward_plan(c);
   if (!p.ok) return false;
@@ -650,7 +650,7 @@ bool conv_any_dx_applicable(const ConvShape &c, AnyOver over) {
     // The vector-ALU kernel is built for windows of 3 and 5; 7x7, us there / here: 41x40, 3 -> 105, 101 images 379 /
     // 219, 32x49, 2 -> 38, 6 images 54 / 23, but 53x31, 4 -> 12, 54 images 29 / 36
     case ANY_OVER_FIRST: return !(c.R == c.S && (c.R == 3 || c.R == 5)) && c.R * c.S > 9 && (k >= 1000 || c.batch <= 4);
-    default: return true;
+    default: return p.cost + ANY_PACK_US < other_us;
   }
 }
 // (the packed filters: the same whatever the tile)

@@ -1,6 +1,7 @@
 // conv_s1.hip — host side of the stride-1 convolution (forward and dX) on the LDS-halo MFMA
 // kernel of conv_s1_inst.hip: tile choice, filter repacking, split-K reduction.
 #include <algorithm>
+#include <cmath>
 #include <utility>
 #include <vector>
 
@@ -185,10 +186,19 @@ bool conv_s1_applicable(int R, int S, int batch, int KC, int MC, int IH, int IW,
   return make_plan(R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw).ok;
 }
 
-// The share of its tiles' outputs that exist, of the fp32 kernel's; 1 where another one runs.
-double conv_s1_fill(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw) {
+// The share of its tiles' outputs that exist, of the fp32 kernel's (1 where another one runs), and the estimated us of that
+// kernel with its packing and split sum: whole rounds of the workgroups, fitted to 800 shapes of poorly filled tiles
+// (12 % rms).
+double conv_s1_fill(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw, double *us) {
+  *us = 0.0;
   const S1Plan p = make_plan(R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw);
   if (!p.ok || p.x3) return 1.0;
+  const double products = p.args.kc_split * R * S / 2 * p.tm * p.tn * 64 / 2400.0;   // of a workgroup, us of its matrix instructions
+  const double full     = static_cast<double>(p.grid.x) * p.grid.y * p.splits / 256;
+  const int resident    = p.lds_bytes <= 80 * 1024 ? 2 : 1;
+  auto round = [&](double at_once) { return 2.8 + 1.6 * products * at_once; };
+  const double whole = std::floor(full / resident), left = std::ceil(full - whole * resident);
+  *us = 6.4 + whole * round(resident) + (left > 0 ? round(left) : 0.0) + (p.splits > 1 ? 0.6 : 0.0);
   const double in_tiles = 128.0 * p.tn * p.grid.x * (32.0 * p.tm * p.grid.y);
   return static_cast<double>(batch) * OH * OW * MC / in_tiles;
 }
