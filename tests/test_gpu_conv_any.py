@@ -191,7 +191,12 @@ def test_forward_product_takes_the_faster_kernel(T, cfg):
     (77, 9, 94, 5, 5, 113, False, (1, 1), 2, False),   # 30 / 51
     (43, 31, 94, 3, 3, 74, True, (1, 1), 6, True),     # 40 / 25
     (19, 89, 64, 3, 3, 21, True, (1, 1), 11, True),    # 26 / 16
+    # (... by the vector kernel of a first layer)
+    (70, 25, 3, 4, 4, 127, True, (1, 1), 83, False),   # 104 / 160
+    (29, 61, 2, 7, 5, 110, True, (1, 1), 76, False),   # 164 / 261
+    (41, 40, 3, 7, 7, 105, True, (1, 1), 101, True),   # 379 / 219
+    (18, 15, 1, 7, 7, 116, True, (1, 1), 1, True),     # 155 / 29
 ])
-def test_input_gradient_of_poorly_filled_tiles_takes_the_faster_kernel(T, cfg):
+def test_input_gradient_takes_the_faster_kernel(T, cfg):
     d, x, w, b, dy = operands(T, cfg, np.random.default_rng(47))
     assert ("b" in run(T, d, x, w, b, dy)[2]) == cfg[9]

@@ -647,9 +647,16 @@ bool conv_any_dx_applicable(const ConvShape &c, AnyOver over, double other_us) {
     // 731), 48 to 96 12 / 42 (973 / 845), 96 to 192 8 / 55 (1436 / 1055).
     case ANY_OVER_GENERIC:
       return k >= (c.sh * c.sw > 1 ? 48 : 96) && p.cost + ANY_PACK_US < generic_us(pixels * ceil_div(c.C, 32) * 32 * k);
-    // The vector-ALU kernel is built for windows of 3 and 5; 7x7, us there / here: 41x40, 3 -> 105, 101 images 379 /
-    // 219, 32x49, 2 -> 38, 6 images 54 / 23, but 53x31, 4 -> 12, 54 images 29 / 36
-    case ANY_OVER_FIRST: return !(c.R == c.S && (c.R == 3 || c.R == 5)) && c.R * c.S > 9 && (k >= 1000 || c.batch <= 4);
+    // The vector-ALU kernel is built for windows of 3 and 5. Of 1600 shapes with others, how many are over 3 % slower here / there,
+    // and all of them in us, there / here: k from 1000 on and more than 4 images 66 / 397 (43746 / 26527; of the 444 that its
+    // estimate leaves 47, and 26141 in all), up to 4 images 7 / 293 (16911 / 5403: a workgroup's chain of channels there), the
+    // rest, which stay, 200 / 566 (15470 / 12622).
+    case ANY_OVER_FIRST: {
+      // (20 % rms over those 476)
+      const double vector_us = 19 + 0.55 * c.Kc + pixels * c.Kc * 1e-6 * (0.39 * c.R * c.S - 7.3);
+      return !(c.R == c.S && (c.R == 3 || c.R == 5)) && c.R * c.S > 9 &&
+             (c.batch <= 4 || (k >= 1000 && p.cost + ANY_PACK_US < vector_us));
+    }
     default: return p.cost + ANY_PACK_US < other_us;
   }
 }
