@@ -200,3 +200,18 @@ def test_forward_product_takes_the_faster_kernel(T, cfg):
 def test_input_gradient_takes_the_faster_kernel(T, cfg):
     d, x, w, b, dy = operands(T, cfg, np.random.default_rng(47))
     assert ("b" in run(T, d, x, w, b, dy)[2]) == cfg[9]
+
+
+@pytest.mark.parametrize("cfg", [
+    # (us of dW and db by the generic kernel / by the one of any size)
+    (52, 71, 24, 3, 3, 114, True, (2, 2), 47, False),   # 56 / 97, 68 with whole rounds in the choice of its tile
+    (65, 19, 123, 3, 5, 109, True, (1, 1), 21, False),  # 157 / 222, 176
+    (59, 56, 46, 5, 5, 3, True, (1, 1), 69, True),      # 286 / 141
+    (48, 85, 55, 7, 7, 12, True, (1, 1), 26, True),     # 362 / 155
+])
+def test_weight_gradient_takes_the_faster_kernel(T, cfg):
+    d, x, w, b, dy = operands(T, cfg, np.random.default_rng(48))
+    dw, db = T.DevBuf((w.size,)), T.DevBuf((b.size,))
+    T.profile_begin()
+    T.conv2d_bwd(d, len(x), T.to_device(x.ravel()), T.to_device(w.ravel()), T.to_device(dy.ravel()), None, dw, db)
+    assert any(e["tag"].startswith("conv_dw_db_any") for e in T.profile_end()) == cfg[9]

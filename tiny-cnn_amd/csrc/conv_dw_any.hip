@@ -16,7 +16,7 @@
 // Reference: conv2d_op_internal.h:79-158.
 #include <algorithm>
 
-#include "common.h"
+#include "gemm_mfma.h"
 
 namespace tdh {
 
@@ -269,10 +269,11 @@ DwAnyPlan plan_tile(const ConvShape &c, bool with_db, int nb, int ch, int rounds
                         chunks * (0.048 * slots * channels / 8 + 0.071 * dy_trips);
   const double alone  = 2.0 + stage + std::max(mfma, steps * 0.044);
   const double at     = std::max<double>(1, std::min<double>(4, 160 * 1024 / p.lds_bytes));
+  // (whole rounds: 600 workgroups of which a compute unit holds two take the time of 768)
   const double full   = static_cast<double>(p.slices) * n_tiles * m_tiles / 256;
-  const double once   = std::min(at, std::ceil(full));
-  p.cost = 1.0 + std::max(1.0, full / at) * std::max(alone + (once - 1) * 0.82 * shared, once * shared) +
-           4.6 + 0.665 * 4e-6 * p.slices * a.M * a.N;
+  auto round = [&](double once) { return std::max(alone + (once - 1) * 0.82 * shared, once * shared); };
+  const double whole = std::floor(full / at), left = std::ceil(full - whole * at);
+  p.cost = 1.0 + whole * round(at) + (left > 0 ? round(left) : 0.0) + 4.6 + 0.665 * 4e-6 * p.slices * a.M * a.N;
   p.ok = true;
   return p;
 }
@@ -329,16 +330,18 @@ int launch_mb(const DwAnyPlan &p) {
 
 }  // namespace
 
-// Against the generic GEMM with its split reduction, of which one workgroup gathers every input word of its 32
-// columns by itself: its time is close to 10 us and 26 million products (of whole tiles) a us. Both us: 59x56, 46 ->
-// 3, 5x5, 69 images 286 / 141; 48x85, 55 -> 12, 7x7, 26 images 362 / 155; 45x37, 21 -> 45, 5x5, stride 2, 19 images
-// 19.4 / 17.4; 71x46, 1 -> 152, 1x1, 81 images 63 / 113 (two columns: the tile is empty), stays there.
+// Against the generic GEMM with its split reduction, of which one workgroup gathers every input word of its columns by itself.
+// Both us: 59x56, 46 -> 3, 5x5, 69 images 286 / 141; 48x85, 55 -> 12, 7x7, 26 images 362 / 155; 45x37, 21 -> 45, 5x5, stride 2,
+// 19 images 19.4 / 17.4; 71x46, 1 -> 152, 1x1, 81 images 63 / 113 (two columns: the tile is empty), stays there, and so does
+// 52x71, 24 -> 114, 3x3, stride 2, 47 images 56 / 68. Of 1600 shapes (7 to 440 us) this takes 620; 57 of those are over 3 % slower
+// here, 184 of the others there, and in all it is 32378 us there, 28560 here, 28209 with the faster one of each.
+// In fp32 like the GEMM, but in another order of its sums: a step that keeps to fp32 (Context::keep_f32) has the order it
+// always had.
 bool conv_dw_any_applicable(const ConvShape &c, bool with_db) {
   if (ctx().keep_f32 || c.dh != 1 || c.dw != 1) return false;
   const DwAnyPlan &p = make_plan(c, with_db);
-  const double products = static_cast<double>(c.batch) * c.OH * c.OW * ceil_div(c.Kc, 32) * 32 *
-                          (ceil_div(c.C * c.R * c.S + (with_db ? 1 : 0), 32) * 32);
-  return p.ok && p.cost < 10.0 + products / 26e6;
+  // (the estimate as it turns out at the tile it chooses: 10 % rms)
+  return p.ok && 1.03 * p.cost - 2.0 < 0.87 * gathered_gemm_us(c.Kc, c.C * c.R * c.S + (with_db ? 1 : 0), c.batch * c.OH * c.OW);
 }
 size_t conv_dw_any_workspace_bytes(const ConvShape &c, bool with_db) {
   if (!conv_dw_any_applicable(c, with_db)) return 0;
