@@ -215,3 +215,71 @@ def test_weight_gradient_takes_the_faster_kernel(T, cfg):
     T.profile_begin()
     T.conv2d_bwd(d, len(x), T.to_device(x.ravel()), T.to_device(w.ravel()), T.to_device(dy.ravel()), None, dw, db)
     assert any(e["tag"].startswith("conv_dw_db_any") for e in T.profile_end()) == cfg[9]
+
+
+NET = dict(w=45, h=37, ci=3, mid=21, co=45, k=5, batch=19)   # 3x3 to 21 channels, then 5x5 at stride 2 to 45: ragged everywhere
+
+
+def tags_of(T, f):
+    T.profile_begin()
+    f()
+    return {e["tag"].split()[0] for e in T.profile_end()}
+
+
+@pytest.mark.parametrize("exceptional", [False, True])
+@pytest.mark.parametrize("kind", ["relu", "tanh", "sigmoid"])
+def test_inference_writes_the_activation_behind_it(T, kind, exceptional):
+    """A net's forward pass takes the pointwise activation along: the bits of the two operators, and float64."""
+    n, rng = NET, np.random.default_rng(51)
+    d, x, w, b, dy = operands(T, (n["w"], n["h"], n["mid"], n["k"], n["k"], n["co"], False, (2, 2), n["batch"]), rng)
+    if exceptional:
+        plant(x, rng, 6)
+    net = T.Net([T.L_conv(n["w"], n["h"], n["mid"], n["k"], n["co"], stride=2), T.L_act(kind)], n["batch"], T.NET_FUSE_ACT_GRAD)
+    net.set_param(0, 0, w.ravel())
+    net.set_param(0, 1, b)
+    xd, y, a = T.to_device(x), T.DevBuf((dy.size,)), T.DevBuf((dy.size,))
+    tags = tags_of(T, lambda: net.forward(n["batch"], xd))
+    assert "conv_fwd_any_x3" in tags and not any(t.startswith("act") for t in tags), tags
+    T.conv2d_fwd(d, n["batch"], xd, T.to_device(w.ravel()), T.to_device(b), y)
+    T.act_fwd(kind, n["batch"], dy.size // n["batch"], y, a)
+    assert np.array_equal(net.layer_out(0, n["batch"]).ravel(), y.numpy(), equal_nan=True)
+    assert np.array_equal(net.layer_out(1, n["batch"]).ravel(), a.numpy(), equal_nan=True)
+    check(y.numpy(), reference(x, w, b, dy, False, (2, 2))[0], kind)
+    net.close()
+
+
+@pytest.mark.parametrize("exceptional", [False, True])
+@pytest.mark.parametrize("kind", ["relu", "tanh", "sigmoid"])
+def test_input_gradient_folds_the_activation_in_front(T, kind, exceptional):
+    """A train step's dX through the activation between two convolutions, against float64 on the step's own outputs."""
+    n, rng = NET, np.random.default_rng(52)
+    _, x, w0, b0, _ = operands(T, (n["w"], n["h"], n["ci"], 3, 3, n["mid"], True, (1, 1), n["batch"]), rng)
+    _, _, w1, b1, dy = operands(T, (n["w"], n["h"], n["mid"], n["k"], n["k"], n["co"], False, (2, 2), n["batch"]), rng)
+    layers = [T.L_conv(n["w"], n["h"], n["ci"], 3, n["mid"], pad_same=True), T.L_act(kind),
+              T.L_conv(n["w"], n["h"], n["mid"], n["k"], n["co"], stride=2)]
+    net = T.Net(layers, n["batch"], T.NET_FUSE_ACT_GRAD)
+    for i, w, b in ((0, w0, b0), (2, w1, b1)):
+        net.set_param(i, 0, w.ravel())
+        net.set_param(i, 1, b)
+    t = rng.standard_normal(dy.shape).astype(np.float32)
+    if exceptional:
+        plant(t, rng, 4)   # (infinities and NaN of dY: sums that are computed again, then multiplied by the activation's gradient)
+    tags = tags_of(T, lambda: net.train_step(None, "mse", n["batch"], T.to_device(x), T.to_device(t), do_update=False))
+    assert "conv_dx_any_x3" in tags and not any(g.startswith("act_bwd") for g in tags), tags
+    a, y = net.layer_out(1, n["batch"]).reshape(n["batch"], n["mid"], n["h"], n["w"]), net.layer_out(2, n["batch"]).reshape(dy.shape)
+    dy = ((y - t) * np.float32(2.0 / (dy.size // n["batch"]))).astype(np.float32)
+    a64 = a.astype(np.float64)
+    factor = {"relu": (a64 > 0) * 1.0, "tanh": 1 - a64 * a64, "sigmoid": a64 * (1 - a64)}[kind]
+    with np.errstate(invalid="ignore"):
+        want = reference(a, w1, b1, dy, False, (2, 2))[1] * factor
+    got = net.layer_dx(1, n["batch"]).ravel()
+    if exceptional:
+        assert not np.isfinite(got).all()
+        on = factor.ravel() != 0   # (behind a rectifier that is off: 0, or NaN where the sum is not finite)
+        check(got[on], want.ravel()[on], kind)
+        assert np.array_equal(got[~on], want.ravel()[~on], equal_nan=True)
+    else:
+        assert_close(got, want.ravel(), what=kind)
+        k = n["k"] ** 2 * n["co"] / 4
+        assert np.linalg.norm(got - want.ravel()) <= 2 ** -24 * (6 + np.sqrt(k / 6)) * np.linalg.norm(want)
+    net.close()

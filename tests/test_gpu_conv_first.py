@@ -68,10 +68,10 @@ def test_first_convolution_is_its_layers(T, w, h, ci, k, co, batch, between, beh
     net.close()
 
 
-@pytest.mark.parametrize("convs", [1, 2, 11])    # (one job, several, more than a launch takes along)
+@pytest.mark.parametrize("convs", [1, 2, 17])    # (filters to pack: one, several, more than the 16 that a launch takes along)
 def test_filters_packed_along_are_those_written_last(T, convs):
     rng = np.random.default_rng(62)
-    batch, hw, c = 64, 16, 32
+    batch, hw, c = 128, 16, 32
     layers = [T.L_conv(hw, hw, 3, 5, c, pad_same=True), T.L_act("relu")]
     layers += [T.L_conv(hw, hw, c, 3, c, pad_same=True) for _ in range(convs)]
     x, t = T.to_device(rng.standard_normal((batch, 3 * hw * hw)).astype(np.float32)), T.DevBuf((batch, c * hw * hw), zero=True)
@@ -79,10 +79,15 @@ def test_filters_packed_along_are_those_written_last(T, convs):
     at = [0] + list(range(2, convs + 2))
 
     def results(net):
-        net.forward(batch, x)
-        out = [net.layer_out(len(layers) - 1, batch).copy()]
-        net.clear_grads()
-        net.train_step(None, "mse", batch, x, t, do_update=False)
+        out = []
+        for run, jobs in ((lambda: net.forward(batch, x), convs),
+                          (lambda: net.train_step(None, "mse", batch, x, t, do_update=False), 2 * convs)):
+            net.clear_grads()
+            T.profile_begin()
+            run()
+            tags = {e["tag"].split()[0] for e in T.profile_end()}
+            assert "conv_fwd_small" in tags and ("conv_repack_weights" in tags) == (jobs > 16), tags
+            out.append(net.layer_out(len(layers) - 1, batch).copy())
         return out + [net.layer_grad(i, 0).copy() for i in at]
 
     net = T.Net(layers, batch, T.NET_FUSE_ACT_GRAD)

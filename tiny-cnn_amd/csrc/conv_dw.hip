@@ -678,7 +678,8 @@ int conv_dw_halo_run(int R, int S, int batch, int C, int Kc, const float *x, con
     ProfScope prof(db ? "conv_dw_db_x3" : "conv_dw_x3", Kc, crs, batch * OH * OW);
     TDH_TRY(R == 5 ? dwx_launch_5_scalar(x3) : vec ? dwx_launch_3_vec(x3) : dwx_launch_3_scalar(x3));
   } else {
-    ProfScope prof(db ? "conv_dw_db_halo" : "conv_dw_halo", Kc, crs, batch * OH * OW);
+    const bool rows = !im.ok && p.window == 3 && p.rows_block == 1;
+    ProfScope prof(rows ? (db ? "conv_dw_db_rows" : "conv_dw_rows") : db ? "conv_dw_db_halo" : "conv_dw_halo", Kc, crs, batch * OH * OW);
     if (im.ok) {
       im.args.x = x; im.args.dy = dy;
       im.args.partial = static_cast<float *>(part); im.args.partial_db = static_cast<float *>(part_db);
