@@ -93,7 +93,7 @@ class NetWorkload:
 
 
 class ConvBwdWorkload:
-    """configs[1]: conv2d backward, batch 64, 32x64x64 -> 64 channels, 3x3, pad same."""
+    """conv2d backward, batch 64, 32x64x64 -> 64 channels, 3x3, pad same."""
 
     def __init__(self, T, W, name="conv2d_bwd_b64", batch=64):
         self.T = T
@@ -111,7 +111,7 @@ class ConvBwdWorkload:
 
 
 class FcBwdWorkload:
-    """configs[2]: tanh-grad -> FC backward (dX, dW, db) -> Adam on W and b, batch 256."""
+    """tanh-grad -> FC backward (dX, dW, db) -> Adam on W and b, batch 256."""
 
     def __init__(self, T, W, name="fc_bwd_adam_b256", batch=256, n=4096):
         self.T = T
@@ -393,7 +393,7 @@ def main():
         "one_step_per_call": None if res["single_step_calls_ms"] is None else
         {"ms_per_step": round(res["single_step_calls_ms"], 4),
          "samples_per_s": round(wl.samples / (res["single_step_calls_ms"] * 1e-3), 2),
-         "note": "the same steps through tdh_net_train_step, one captured graph replayed per step"},
+         "note": "the same steps through tdh_net_train_step, replayed from a captured graph or launched, as the net does by itself"},
         "roofline": dict(res["kernels"][0]) if res["kernels"] else None,
         "kernels": res["kernels"],
     }

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 def test_config2_conv_backward_full_size(T, W):
-    """batch 64, 32x64x64 -> 64 channels, 3x3, pad same, stride 1."""
+    """Batch 64, 32x64x64 -> 64 channels, 3x3, pad same, stride 1."""
     (hw, _, c, k, oc), x, w, dy = W.conv_bwd_case()
     bs = x.shape[0]
     d = T.conv_desc(hw, hw, c, k, k, oc, pad_same=True)
@@ -108,7 +108,7 @@ def test_large_fc_input_gradient_from_untransposed_tiles(T, bs, ni, no):
 
 
 def test_config3_fc_backward_adam_full_size(T, O, W):
-    """batch 256, 4096 -> 4096, tanh, Adam on W and b."""
+    """Batch 256, 4096 -> 4096, tanh, Adam on W and b."""
     x, w, b, dy = W.fc_bwd_case()
     bs, n = x.shape[0], 4096
     xd, wd, bd = T.to_device(x), T.to_device(w), T.to_device(b)
@@ -147,7 +147,7 @@ def test_config3_fc_backward_adam_full_size(T, O, W):
 
 
 def test_config4_full_batch_step_properties(T, W):
-    """configs[3] at batch 128: a step changes every parameter, stays finite, and the loss
+    """The CIFAR-10-shape net at batch 128: a step changes every parameter, stays finite, and the loss
     gradient rows sum to zero (softmax + cross-entropy)."""
     spec, params, x, t, batch, loss, opt_kind, opt_kw = W.make_batch("cifar10_cnn_b128")
     net = T.Net(W.build_layers(T, spec), batch, 1)
@@ -175,7 +175,7 @@ def test_config4_full_batch_step_properties(T, W):
 
 
 def test_config5_vgg_full_size_one_step(T, W):
-    """configs[4] at its full size (batch 64, 3x128x128): one momentum step; spot-check the
+    """The VGG-style stack at its full size (batch 64, 3x128x128): one momentum step; spot-check the
     big fully-connected gradient (131072 x 256) against float64 and the first conv's bias
     gradient against a host sum."""
     spec, params, x, t, batch, loss, opt_kind, opt_kw = W.make_batch("vgg_stack_b64")
@@ -248,7 +248,7 @@ def _pool2x2_scan(x4):
 
 
 def test_config5_vgg_batch64_every_conv_layer_and_both_execution_modes(T, W):
-    """configs[4] as it is benchmarked (batch 64, 3x128x128). Unfused (flags 0), where every
+    """The VGG-style stack as it is benchmarked (batch 64, 3x128x128). Unfused (flags 0), where every
     tensor of the step is in memory: sampled dW taps and dX positions of all four convolutions
     against float64 dot products over the whole batch, every bias gradient against a float64
     sum, both max-pools against a numpy scan (indices exact). Then one momentum step fused and

@@ -174,7 +174,7 @@ def check_every_layer(net, ref, spec, batch, name, fused, passes=1, cancelling_d
 
 
 def test_cifar_net_at_the_benchmarked_batch_and_flags_matches_oracle(T, O, W):
-    """configs[3] exactly as bench.py runs it: batch 128, folded activation gradients, the step
+    """The CIFAR-10-shape net exactly as bench.py runs it: batch 128, folded activation gradients, the step
     captured into a graph (at this batch one chain of launches: the first layer's three gradients
     from one launch, every weight gradient's split sums left to the optimizer kernel). Every
     layer's output, argmax, dW, db and dX, then the parameters after each of two Adam steps."""
@@ -201,7 +201,7 @@ def test_cifar_net_at_the_benchmarked_batch_and_flags_matches_oracle(T, O, W):
 
 @pytest.mark.parametrize("flags", [1, 3])
 def test_vgg_layers_at_full_image_size_match_oracle(T, O, W, flags):
-    """configs[4] at its real 3x128x128 input (every convolution at the tile plans of the full
+    """The VGG-style stack at its real 3x128x128 input (every convolution at the tile plans of the full
     workload's image size), batch 2. The net as a whole: every output and argmax, and every
     gradient behind the last relu element whose sign differs (see relu_sign_flips). Then every
     convolution, max-pool and fully-connected layer's backward pass on its own, fed with the

@@ -385,8 +385,9 @@ bool conv_bwd_pairs(const tdh_conv_desc *d, int batch, const float *x = nullptr,
 // the forward kernel of this convolution can also compute the max-pool layer `pool` behind it
 bool conv_fwd_fuses_pool(const tdh_conv_desc *d, const tdh_pool_desc *pool, int batch, bool prepacked);
 // ... and the pointwise activation of this kind behind that pool
-bool conv_fwd_packs_along(const tdh_conv_desc *d, int batch);
 bool conv_fwd_pool_applies_act(const tdh_conv_desc *d, int batch, bool prepacked, int act_kind);
+// ... and take filters along that later layers read packed (conv_pack_leave)
+bool conv_fwd_packs_along(const tdh_conv_desc *d, int batch);
 // the forward kernel of this layer can leave `y` out (null) when it writes the activation layer
 // or the pool behind the convolution itself
 bool conv_fwd_out_optional(const tdh_conv_desc *d, int batch, bool prepacked);
@@ -493,8 +494,9 @@ bool conv_s1_fuses_pool(int R, int S, int batch, int KC, int MC, int IH, int IW,
 // one pass over the reduction channels: the kernel's epilogue is the only writer of `out`
 bool conv_s1_single_pass(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW,
                          int ph, int pw);
-// conv_packed_kind / conv_packed_bytes of a shape this file runs
+// how full its fp32 tiles are, and the estimated us of that kernel
 double conv_s1_fill(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw, double *us);
+// conv_packed_kind / conv_packed_bytes of a shape this file runs
 int conv_s1_packed_kind(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw);
 size_t conv_s1_packed_bytes(int kind, int RS, int KC, int MC);
 // conv_dw.hip: stride-1 weight gradient from LDS-staged tiles (3x3 and 5x5 windows)

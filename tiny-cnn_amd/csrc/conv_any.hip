@@ -454,8 +454,8 @@ AnyPlan plan_tile(const AnyArgs &base, int batch, int mb, int nb, int wk) {
   a.m_pad     = m_tiles * 16 * mb;
   p.pack_bytes = any_pack_bytes(a.M, a.KC, std::min(a.wm, a.wk));
   if (p.pack_bytes >= (1u << 31)) return p;
-  // Estimated us, from stamps inside the kernel and 240 shapes at every tile (10 to 1400 us; the chosen tile is
-  // 3 % off the best one, the estimate 15 %): what a workgroup waits for by itself, what the workgroups
+  // Estimated us, from stamps inside the kernel and 240 shapes at every tile (10 to 1400 us; over 400 others the chosen tile
+  // is 3 % off the best one, the estimate 16 %): what a workgroup waits for by itself, what the workgroups
   // of a compute unit share, and how many of them run at once.
   const double chunks = ceil_div(all, groups);
   const double steps  = chunks * ceil_div(groups * static_cast<int>(most_taps), 4 * wk);

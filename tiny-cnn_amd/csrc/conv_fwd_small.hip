@@ -10,10 +10,11 @@
 // the band in LDS (zero-filled where the window leaves the image) and the filter slice, and a
 // wave then computes tiles of 2 rows x 32 columns x 32 channels, one accumulator block per row:
 // per k-step and row one LDS read at patch[pixel] + offset(k) and one v_mfma_f32_32x32x2_f32
-// (A lane = (co, k), B lane = (pixel, k)). A lane so holds both rows of its column, and the 2x2
-// pooling window of an even lane is completed by its right neighbour: the max-pool (with its
-// argmax record and the activation behind it) costs a lane swap in the epilogue and needs no
-// kernel or pass over y of its own. Stores of y are whole rows of 32 floats per channel.
+// (A lane = (co, k), B lane = (pixel, k); indices past the last tap are zeros on both sides). A lane so
+// holds both rows of its column, and two neighbours share a 2x2 pooling window: they exchange the values of
+// two channels and pool one each. The max-pool (with its argmax record and the activation behind it) costs
+// those lane swaps in the epilogue and needs no kernel or pass over y of its own. Stores of y are whole
+// rows of 32 floats per channel.
 //
 // Reference: conv2d_op_internal.h:13-74 (forward), maxpool_op_internal.h:17-47 (window scan:
 // row by row, strict '>', start value lowest()).
@@ -189,9 +190,10 @@ __device__ __forceinline__ void fwd_small_store(const T v, const __amdgpu_buffer
 
 // PLAIN: the channels are a multiple of 32 and each activation is relu or none.
 // Registers are what keeps workgroups from a CU: with patch offsets and biases read again per tile instead of held, and
-// patch values a group of four steps ahead instead of eight, 176 -> 114 of them and two -> four workgroups. us for 3 -> 32 channels, 5x5, 32x32 with
-// a pool and relu behind, batch 1000 with y: 92 -> 77; of three to four workgroups and the stores above, 3 -> 64 channels, 3x3, 128x128, batch 64
-// 91 -> 75, 1 -> 32, 5x5, 28x28, batch 256 17.6 -> 12.6, 1 -> 6, 5x5, 70x50, batch 64 20.6 -> 14.6.
+// patch values a group of four steps ahead instead of eight, 176 -> 112 of them for 5x5 on three channels and two -> four
+// workgroups. The kernel's us for 3 -> 32 channels, 5x5, 32x32 with a pool and relu behind, batch 1000, y past the caches: 101 -> 79; of three to four workgroups
+// and the stores above, 3 -> 64 channels, 3x3, 128x128, batch 64 68 -> 59, 1 -> 32, 5x5, 28x28, batch 256 17.5 -> 13.1, 1 -> 6,
+// 5x5, 70x50, batch 64 26 -> 18.
 template <int NS, class Packs, bool PLAIN>
 __global__ void __launch_bounds__(256, PLAIN ? 4 : 3) conv_fwd_small_kernel(const FwdSmallArgs a, const Packs packs) {
   extern __shared__ __align__(16) float lds[];

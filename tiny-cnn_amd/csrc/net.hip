@@ -238,7 +238,8 @@ bool tiny_step_applies(const tdh_net *net, int loss_kind);
 // batch 64 241 / 241, batch 256 628 / 623; 784-1000-1000-10 fully connected, batch 1024 273 / 268; 1024-4096-4096-10,
 // batch 64 286 / 281. Below it the two are within 1 % of each other, and a replay leaves the host free. The step of a
 // workgroup per sample (tiny_net.hip) is three launches of 40, 9 and 5 us at least, whatever the net and the batch:
-// LeNet-5, batch 16 58.6 / 54.8, fed from the host in batches of 13 66.9 / 60.2 and of 221 136.6 / 128.3.
+// LeNet-5, batch 16 58.6 / 54.8, fed from the host in batches of 13 66.9 / 60.2 and of 221 136.6 / 128.3; the call
+// takes the host 14 to 19 / 11.
 bool step_outlasts_launches(const tdh_net *net, int loss_kind, int batch) {
   if (tiny_step_applies(net, loss_kind)) return true;
   return !net_forks(net, batch) &&
@@ -998,7 +999,7 @@ static int post_update(tdh_net *net) {
 int tdh_net_update_weights(tdh_net *net, tdh_opt *opt) {
   TDH_REQUIRE_INIT();
   TDH_CHECK_ARG(net && opt, "tdh_net_update_weights: null argument");
-  // the optimizer kernel keeps the packed filter copies of a graph net current, as in a step
+  // the optimizer kernel keeps the packed filter copies current, as in a step
   TDH_TRY(launch_opt_update_multi(opt, net->opt_table, net->opt_tensors, net->opt_blocks, net->opt_params, 1.0f, 1,
                                   nullptr, nullptr, nullptr, net->opt_table_host.data(), !net->weights_out));
   after_update(net, !net->weights_out);

@@ -18,7 +18,7 @@ import numpy as np
 
 
 def lenet5():
-    """LeNet-5-style net, 1x32x32 input (configs[0])."""
+    """LeNet-5-style net, 1x32x32 input."""
     return [("conv", 32, 32, 1, 5, 6, False), ("act", "tanh"), ("avepool", 28, 28, 6, 2),
             ("conv", 14, 14, 6, 5, 16, False), ("act", "tanh"), ("avepool", 10, 10, 16, 2),
             ("conv", 5, 5, 16, 5, 120, False), ("act", "tanh"), ("fc", 120, 10)]
@@ -41,7 +41,7 @@ def lenet5_mnist():
 
 
 def cifar10_cnn():
-    """CIFAR-10-shape CNN of examples/cifar10/train.cpp:26-42 (configs[3])."""
+    """CIFAR-10-shape CNN of examples/cifar10/train.cpp:26-42."""
     return [("conv", 32, 32, 3, 5, 32, True), ("maxpool", 32, 32, 32, 2), ("act", "relu"),
             ("conv", 16, 16, 32, 5, 32, True), ("maxpool", 16, 16, 32, 2), ("act", "relu"),
             ("conv", 8, 8, 32, 5, 64, True), ("maxpool", 8, 8, 64, 2), ("act", "relu"),
@@ -49,7 +49,7 @@ def cifar10_cnn():
 
 
 def vgg_stack(size=128):
-    """VGG-style block stack, 3 x size x size input (configs[4] at size=128)."""
+    """VGG-style block stack, 3 x size x size input."""
     h = size // 2
     q = size // 4
     return [("conv", size, size, 3, 3, 64, True), ("act", "relu"),
@@ -171,7 +171,7 @@ def make_batch(name, batch=None, size=None):
 
 
 def conv_bwd_case(batch=64, c=32, hw=64, oc=64, k=3, seed=1235):
-    """single conv2d backward, pad same, stride 1. Returns (dims, x, w, dy)."""
+    """Single conv2d backward, pad same, stride 1. Returns (dims, x, w, dy)."""
     rng = np.random.Generator(np.random.Philox(seed))
     x = rng.standard_normal((batch, c * hw * hw)).astype(np.float32)
     dy = rng.standard_normal((batch, oc * hw * hw)).astype(np.float32)
@@ -181,7 +181,7 @@ def conv_bwd_case(batch=64, c=32, hw=64, oc=64, k=3, seed=1235):
 
 
 def fc_bwd_case(batch=256, n_in=4096, n_out=4096, seed=1236):
-    """configs[2]: FC backward + Adam. Returns (x, w, b, dy); the layer is followed by tanh."""
+    """FC backward + Adam. Returns (x, w, b, dy); the layer is followed by tanh."""
     rng = np.random.Generator(np.random.Philox(seed))
     x = rng.uniform(-1.0, 1.0, (batch, n_in)).astype(np.float32)
     bound = math.sqrt(6.0 / (n_in + n_out))
