@@ -33,6 +33,12 @@ def reference(x, w, b, dy, same, stride, dilation=(1, 1)):
         return y + b.astype(np.float64).reshape(1, -1, 1, 1), dx
 
 
+def within_fp32_sum(got, want, size):
+    """A sum in fp32, each addition rounding to 2^-24 of a partial sum that grows as a random walk, is 0.64 * 2^-24 of
+    the sum of absolute products (size) away, rms; no element is twelve times as far."""
+    return (np.abs(got.ravel() - want.ravel()) <= 8 * 2.0 ** -24 * size.ravel()).all()
+
+
 CASES = [
     # in_w, in_h, in_c, kw, kh, out_c, same, (sh, sw), batch; the directions that take the kernel
     (45, 37, 21, 5, 5, 45, False, (2, 2), 19, "fb"),   # 9, 6, 6 and 4 taps a phase, a last group of 5 channels
@@ -72,8 +78,10 @@ def test_against_float64(T, cfg):
     d, x, w, b, dy = operands(T, cfg, np.random.default_rng(41))
     y, dx, taken = run(T, d, x, w, b, dy)
     assert taken == cfg[9]
-    for got, want, name in zip((y, dx), reference(x, w, b, dy, cfg[6], cfg[7]), ("y", "dx")):
+    sizes = reference(*(np.abs(a) for a in (x, w, b, dy)), cfg[6], cfg[7])
+    for got, want, size, name in zip((y, dx), reference(x, w, b, dy, cfg[6], cfg[7]), sizes, ("y", "dx")):
         assert_close(got, want.ravel(), what=f"{cfg} {name}")
+        assert within_fp32_sum(got, want, size), name
         # No further from float64 than a sum in fp32: K terms in order, each addition rounding to 2^-24 of a partial sum
         # that grows as a random walk, leave 2^-24 sqrt(K / 6) of the result; six bits under that and 2^-23 of the parts.
         k = cfg[3] * cfg[4] * cfg[2 if name == "y" else 5] / (1 if name == "y" else cfg[7][0] * cfg[7][1])
@@ -147,8 +155,10 @@ def test_weight_gradient_against_float64(T, cfg, accumulate):
     tags = {e["tag"].split()[0] for e in T.profile_end()}
     assert cfg[9 + accumulate] in tags, tags
     want = weight_gradient(x, dy, cfg[4], cfg[3], cfg[6], cfg[7])
-    for got, ref, old, name in zip((dw.numpy(), db.numpy()), want, (before[:w.size], before[w.size:]), ("dw", "db")):
+    sizes = weight_gradient(np.abs(x), np.abs(dy), cfg[4], cfg[3], cfg[6], cfg[7])
+    for got, ref, size, old, name in zip((dw.numpy(), db.numpy()), want, sizes, (before[:w.size], before[w.size:]), ("dw", "db")):
         ref = ref.ravel() + (old if accumulate else 0)
+        assert within_fp32_sum(got, ref, size.ravel() + (np.abs(old) if accumulate else 0)), name
         assert_close(got, ref, what=f"{cfg} {name}")
         # K products in order in at least 64 slices: the bound of the sums above for K / 64 terms and for 64
         k = dy.size / dy.shape[1]
