@@ -1,0 +1,55 @@
+"""The small net's step where it begins with a convolution, activations and pools, and a second convolution: the front
+and the back of its chain run a channel a workgroup while there is a compute unit for each. Every tensor against the
+oracle, at the ends of those kernels' tiles and on both sides of the line between the two forms."""
+import numpy as np
+import pytest
+
+from conftest import assert_close
+from test_gpu_sample_step import FUSE, SAMPLE, build
+
+pytestmark = pytest.mark.gpu
+
+TABLE = [[(2 * ci + co) % 3 != 0 for co in range(9)] for ci in range(5)]
+NETS = {
+    # a first plane of more pixels than threads; rows of the second one that are no multiple of four, in two chunks of units
+    "wide": ([("conv", 40, 38, 1, 3, 4, True), ("act", "tanh"), ("maxpool", 40, 38, 4, 2), ("act", "sigmoid"),
+              ("conv", 20, 19, 4, 5, 8, True), ("act", "tanh"), ("maxpool", 20, 19, 8, 3),
+              ("fc", 8 * 6 * 6, 5)], "mse", "sgd"),
+    # five layers in front (one more than travel ahead), table behind, windows clipped by the edge
+    "deep_front": ([("conv", 17, 15, 3, 5, 5, True), ("act", "tanh"), ("act", "sigmoid"), ("maxpool", 17, 15, 5, 2),
+                    ("act", "tanh"), ("act", "leaky_relu", (0.2, 0.0)), ("conv", 8, 7, 5, 3, 9, False, TABLE),
+                    ("act", "tanh"), ("fc", 9 * 6 * 5, 4), ("act", "softmax")], "ce_multiclass", "momentum"),
+    # 64 output channels are the most that the back kernel sums over; 65 stay in one launch
+    "k64": ([("conv", 9, 9, 2, 3, 3, False), ("conv", 7, 7, 3, 3, 64, True), ("act", "tanh"), ("fc", 64 * 49, 3)], "mse", "adagrad"),
+    "k65": ([("conv", 9, 9, 2, 3, 3, False), ("conv", 7, 7, 3, 3, 65, True), ("act", "tanh"), ("fc", 65 * 49, 3)], "mse", "adagrad"),
+    # an average pool of odd height behind it, two channels
+    "two": ([("conv", 12, 10, 1, 5, 2, False), ("act", "sigmoid"), ("avepool", 8, 6, 2, 2), ("conv", 4, 3, 2, 3, 4, True),
+             ("fc", 48, 6), ("act", "sigmoid")], "ce", "adam"),
+}
+ENDS = {"wide": 64, "deep_front": 51, "k64": 85, "k65": None, "two": 128}   # the largest batch of the split form
+
+
+@pytest.mark.parametrize("name", list(NETS))
+@pytest.mark.parametrize("batch", [1, 3, "last", "past"])
+def test_every_tensor_matches_oracle(T, O, W, name, batch):
+    split = ENDS[name] is not None
+    if not isinstance(batch, int):
+        if not split:
+            pytest.skip("this net has one form")
+        split, batch = batch == "last", ENDS[name] + (batch == "past")
+    spec, params, x, t, batch, loss, kind, _, net, ref = build(T, O, W, name, batch, SAMPLE | FUSE, nets=NETS)
+    xd, td = T.to_device(x), T.to_device(t)
+    T.profile_begin()
+    net.train_step(None, loss, batch, xd, td, do_update=False)
+    tags = {e["tag"].split()[0] for e in T.profile_end()}
+    assert ("tiny_net_front" in tags) == ("tiny_net_back" in tags) == split, tags
+    ref.train_step(O.opt_desc(kind), loss, x, t, do_update=False)
+    for i, l in enumerate(spec):
+        assert_close(net.layer_out(i, batch), ref.layer_out(i, batch), what=f"layer {i} output")
+        assert_close(net.layer_dx(i, batch), ref.layer_dx(i, batch), what=f"layer {i} dX")
+        if l[0] == "maxpool":
+            assert np.array_equal(net.layer_argmax(i, batch).astype(np.int64), ref.layer_argmax(i, batch))
+        if net.param_size(i, 0):
+            assert_close(net.layer_grad(i, 0), ref.layer_dw(i), what=f"layer {i} dW")
+            assert_close(net.layer_grad(i, 1), ref.layer_db(i), what=f"layer {i} db")
+    net.close()

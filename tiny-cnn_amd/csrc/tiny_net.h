@@ -59,6 +59,9 @@ struct TinyJob {
 struct TinyPlan {
   TinyLayer l[TINY_MAX_LAYERS];
   int n, in_size;
+  // the second convolution, where the layers in front of it run a channel a workgroup (tiny_net.hip), or 0;
+  // LDS of those launches: floats behind the input in front, and offsets behind the framed dY
+  int split, front_floats, back_scratch, back_planes, back_floats;
   int lds_g0, lds_g1, lds_w, lds_pad, lds_floats;   // lds_pad: the zero-framed dY
   int n_mfma, mfma_layers[TINY_MAX_LAYERS];   // the layers with operands to stage for the matrix cores
   int mf_ahead;                // the layer (> 0) whose filters wait in registers until the layer in front of it runs, or -1

@@ -1172,23 +1172,27 @@ TN_INLINE void conv_bwd_param_matvec(const TinyLayer *__restrict__ Lp, const flo
     for (int co = threadIdx.x; co < nb; co += NT) gb[co] = dy[co];
 }
 
-// One workgroup per sample. LDS: the sample's input, every layer's output, two gradient buffers,
-// the staging area.
+// One workgroup per sample, from layer m on (0, or the plan's split). LDS: its input, every layer's output, two gradient
+// buffers, the staging area.
 __global__ void __launch_bounds__(TN_THREADS)
-tiny_net_step_kernel(const TinyPlan *__restrict__ plan, const int loss, const int softmax_xent,
+tiny_net_step_kernel(const TinyPlan *__restrict__ plan, const int m, const int loss, const int softmax_xent,
                      const float *__restrict__ x, const float *__restrict__ t) {
   extern __shared__ float lds[];
-  const int s = blockIdx.x, n = plan->n, in_size = plan->in_size;
+  const int s = blockIdx.x, n = plan->n, in_size = plan->l[m].in_size;
   float *wl = lds + plan->lds_w;   // where partial sums of split layers meet (TINY_SCRATCH_FLOATS)
   // (one layer's filters for the matrix cores are asked for here, in front of the sample's input,
   // and put in LDS while the layer in front of that layer runs: no layer waits for them)
   const int ahead = plan->mf_ahead;
   float ahead_w[MFMA_AHEAD] = {0.0f, 0.0f, 0.0f, 0.0f}, ahead_b = 0.0f;
   if (ahead > 0) mfma_filters_load(&plan->l[ahead], 0, ahead_w, ahead_b);
-  fill_lds<TN_THREADS>(lds, x + static_cast<size_t>(s) * in_size, in_size);
+  fill_lds<TN_THREADS>(lds + plan->l[m].lds_in, (m ? plan->l[m - 1].out : x) + static_cast<size_t>(s) * in_size, in_size);
   stage_mfma_operands(plan, lds, ahead);
+  if (m && ahead == m) {   // (there is no layer in front of it here)
+    mfma_filters_store(&plan->l[m], 0, ahead_w, ahead_b, lds);
+    mfma_tables(&plan->l[m], lds);
+  }
   lds_barrier();
-  for (int li = 0; li < n; ++li) {
+  for (int li = m; li < n; ++li) {
     const TinyLayer *__restrict__ L = &plan->l[li];
     if (li + 1 == ahead) {
       mfma_filters_store(&plan->l[ahead], 0, ahead_w, ahead_b, lds);
@@ -1261,7 +1265,7 @@ tiny_net_step_kernel(const TinyPlan *__restrict__ plan, const int loss, const in
   }
   __syncthreads();   // (also: the max-pool records written to memory above are read back below)
   // input gradients only: the parameter-gradient kernel reads what this loop leaves in memory
-  const int last_bwd = (plan->first_dx_as_job || plan->skip_first_dx) ? 1 : 0;
+  const int last_bwd = m ? m + 1 : (plan->first_dx_as_job || plan->skip_first_dx) ? 1 : 0;
   for (int li = first_bwd; li >= last_bwd; --li) {
     const TinyLayer *__restrict__ L = &plan->l[li];
     const int kind = L->kind, in_sz = L->in_size;
@@ -1304,6 +1308,301 @@ tiny_net_step_kernel(const TinyPlan *__restrict__ plan, const int loss, const in
     float *sw = ga;
     ga = gb;
     gb = sw;
+  }
+}
+
+// ------------------------------------------------------------- the two ends of the chain, spread out
+// One workgroup per sample leaves most of the chip idle at the batches of such nets, and the first
+// convolution's block and the way back to it are half of its time. Where a net begins with
+//   convolution (3x3 or 5x5), pointwise activations and pools, convolution (3x3 or 5x5, stride 1)
+// (TinyPlan::split is the index of the second one), everything in front of the second convolution
+// keeps to one channel: a workgroup takes one channel of a sample through it, forward in a launch in
+// front of the step kernel, and in a launch behind it from the second convolution's dX back to the
+// gradient of the first one's output. Bound: latency, a launch and some three trips to memory each.
+// LeNet-5, batch 16, us: one launch 40.1; here 4.5 + 21.8 + 7.8 (which batches: launch_tiny_step).
+constexpr int TF_THREADS = 1024;   // front, at most
+constexpr int TB_THREADS = 1024;   // back
+
+// the sums of channel co, a lane a pixel, filters as scalar operands (as conv_fwd_scalar adds them up)
+template <int R, int S, bool PAD>
+TN_INLINE void conv_front(const TinyLayer *__restrict__ Lp, const float *in, float *out, float *__restrict__ gout,
+                          const int co) {
+  const int C = Lp->C, H = Lp->H, W = Lp->W, K = Lp->K, OH = Lp->OH, OW = Lp->OW;
+  const int sh = Lp->sh, sw = Lp->sw, ph = Lp->ph, pw = Lp->pw;
+  const FastDiv d_ow = Lp->d_ow;
+  const float *__restrict__ w = Lp->w;
+  const uint8_t *__restrict__ tbl = Lp->tbl;
+  constexpr int taps = R * S;
+  const int plane = OH * OW;
+  const float bias = Lp->has_bias ? ((ScalarFloats)Lp->b)[co] : 0.0f;
+  for (int p = threadIdx.x; p < plane; p += blockDim.x) {
+    uint32_t oy, ox;
+    d_ow.divmod(p, oy, ox);
+    const int y0 = static_cast<int>(oy) * sh - ph, x0 = static_cast<int>(ox) * sw - pw;
+    float acc = 0.0f;
+    for (int ci = 0; ci < C; ++ci) {
+      if (tbl && !tbl[ci * K + co]) continue;
+      const float *ip = in + ci * H * W + y0 * W + x0;
+      const ScalarFloats wq = (ScalarFloats)(w + static_cast<size_t>(co * C + ci) * taps);
+      float sum = 0.0f;
+#pragma unroll
+      for (int wy = 0; wy < R; ++wy)
+#pragma unroll
+        for (int wx = 0; wx < S; ++wx) {
+          float v;
+          if (PAD) {
+            const bool ok = static_cast<unsigned>(y0 + wy) < static_cast<unsigned>(H) &&
+                            static_cast<unsigned>(x0 + wx) < static_cast<unsigned>(W);
+            v = ip[ok ? wy * W + wx : -(y0 * W + x0)];
+            v = ok ? v : 0.0f;
+          } else {
+            v = ip[wy * W + wx];
+          }
+          sum = __builtin_fmaf(wq[wy * S + wx], v, sum);
+        }
+      acc += sum;
+    }
+    const float v = Lp->has_bias ? acc + bias : acc;
+    out[p]  = v;
+    gout[p] = v;
+  }
+}
+
+__global__ void __launch_bounds__(TF_THREADS)
+tiny_net_front_kernel(const TinyPlan *__restrict__ plan, const int m, const int in_size, const float *__restrict__ x) {
+  extern __shared__ float lds[];
+  const int s = blockIdx.x, co = blockIdx.y, nt = blockDim.x;
+  for (int base = threadIdx.x; base < in_size; base += 4 * nt) {
+    float v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = x[static_cast<size_t>(s) * in_size + min(base + j * nt, in_size - 1)];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (base + j * nt < in_size) lds[base + j * nt] = v[j];
+  }
+  const TinyLayer *__restrict__ L = &plan->l[0];
+  int plane  = L->OH * L->OW;
+  float *cur = lds + in_size, *g0 = L->out + static_cast<size_t>(s) * L->out_size + co * plane;
+  lds_barrier();
+  const bool pad = L->ph != 0 || L->pw != 0;
+  if (L->R == 5) pad ? conv_front<5, 5, true>(L, lds, cur, g0, co) : conv_front<5, 5, false>(L, lds, cur, g0, co);
+  else pad ? conv_front<3, 3, true>(L, lds, cur, g0, co) : conv_front<3, 3, false>(L, lds, cur, g0, co);
+  for (int li = 1; li < m; ++li) {
+    L = &plan->l[li];
+    lds_barrier();
+    if (L->kind == TDH_L_ACT) {
+      const int act = L->act;
+      const float p0 = L->p0;
+      float *gout = L->out + static_cast<size_t>(s) * L->out_size + co * plane;
+      for (int i = threadIdx.x; i < plane; i += nt) {
+        const float v = tn_act_fwd(act, p0, cur[i]);
+        cur[i]  = v;
+        gout[i] = v;
+      }
+      continue;
+    }
+    const int H = L->H, W = L->W, OH = L->OH, OW = L->OW, R = L->R, S = L->S, sh = L->sh, sw = L->sw, oplane = OH * OW;
+    const bool most = L->kind == TDH_L_MAXPOOL;
+    const FastDiv d_ow = L->d_ow;
+    const size_t at = static_cast<size_t>(s) * L->out_size + co * oplane;
+    const float weight = most ? 0.0f : L->w[co] * L->scale, bias = most ? 0.0f : L->b[co];
+    float *nxt = cur + plane;
+    for (int o = threadIdx.x; o < oplane; o += nt) {
+      uint32_t oy, ox;
+      d_ow.divmod(o, oy, ox);
+      const int x0 = ox * sw, y0 = oy * sh;
+      const float *win = cur + y0 * W + x0;
+      float v;
+      if (most) {   // maxpool_fwd
+        const int dxmax = min(S, W - x0), dymax = min(R, H - y0);
+        int idx = 0;
+        v = -FLT_MAX;
+        for (int wy = 0; wy < dymax; ++wy)
+          for (int wx = 0; wx < dxmax; ++wx)
+            if (win[wy * W + wx] > v) {
+              v   = win[wy * W + wx];
+              idx = (H * co + y0 + wy) * W + x0 + wx;
+            }
+        L->argmax[at + o] = idx;
+      } else {      // avepool_fwd
+        v = 0.0f;
+        if (x0 + S <= W && y0 + R <= H)
+          for (int wy = 0; wy < R; ++wy)
+            for (int wx = 0; wx < S; ++wx) v += win[wy * W + wx];
+        v *= weight;
+        v += bias;
+      }
+      nxt[o]         = v;
+      L->out[at + o] = v;
+    }
+    cur   = nxt;
+    plane = oplane;
+  }
+}
+
+// dX of the second convolution for channel ci, [H][W], from the zero-framed dY. A lane takes four
+// neighbouring pixels of a row, whose taps share eight values of a framed row; the waves are chunks of
+// 64 such units x `parts` ranges of output channels, whose sums meet in `scratch` ([part][chunk][4][64]).
+// connected: bit b stands for the output channel c_lo + b of this wave's range
+struct BackSplit {
+  int units_w, chunks, parts, per_part;
+};
+__host__ __device__ inline BackSplit back_split(const int H, const int W, const int K) {
+  BackSplit b;
+  b.units_w  = (W + 3) >> 2;
+  b.chunks   = (H * b.units_w + 63) >> 6;
+  b.parts    = min(max(TB_THREADS / 64 / b.chunks, 1), K);
+  b.per_part = (K + b.parts - 1) / b.parts;
+  return b;
+}
+template <int R, int S>
+TN_INLINE void conv_back_dx(const TinyLayer *__restrict__ Lp, const BackSplit b, const float *framed, float *dx,
+                            float *__restrict__ gdx, float *scratch, const int ci, const int kp, const int c_lo,
+                            const int c_hi, const uint64_t connected) {
+  const int C = Lp->C, H = Lp->H, W = Lp->W;
+  const float *__restrict__ w = Lp->w;
+  constexpr int taps = R * S;
+  const int PW = W + S - 1, PP = (H + R - 1) * PW, lane = threadIdx.x & 63, units = H * b.units_w;
+  const int step = b.parts > 1 ? b.chunks : TB_THREADS / 64;
+  if (kp < b.parts)
+    for (int chunk = wave_index() - kp * step; chunk < b.chunks; chunk += step) {   // (one trip where parts > 1)
+      const int unit = min((chunk << 6) + lane, units - 1);
+      const int iy = unit / b.units_w, ix = (unit - iy * b.units_w) << 2;
+      // (a row's last unit may reach up to three values past the row: of the next row, or of `scratch`)
+      const float *dp = framed + c_lo * PP + iy * PW + ix;
+      float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      for (int co = c_lo; co < c_hi; ++co, dp += PP) {
+        if (!(connected >> (co - c_lo) & 1)) continue;
+        const ScalarFloats wq = (ScalarFloats)(w + static_cast<size_t>(co * C + ci) * taps);
+        float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int wy = 0; wy < R; ++wy) {
+          float v[S + 3];
+#pragma unroll
+          for (int k = 0; k < S + 3; ++k) v[k] = dp[(R - 1 - wy) * PW + k];
+#pragma unroll
+          for (int wx = 0; wx < S; ++wx)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) sum[k] = __builtin_fmaf(wq[wy * S + wx], v[k + S - 1 - wx], sum[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) acc[k] += sum[k];
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) scratch[((kp * b.chunks + chunk) * 4 + k) * 64 + lane] = acc[k];
+    }
+  lds_barrier();
+  const FastDiv d_w = Lp->d_w;
+  for (int p = threadIdx.x; p < H * W; p += TB_THREADS) {
+    uint32_t iy, ix;
+    d_w.divmod(p, iy, ix);
+    const int unit = static_cast<int>(iy) * b.units_w + (static_cast<int>(ix) >> 2);
+    const float *part = scratch + ((unit >> 6) * 4 + (ix & 3)) * 64 + (unit & 63);
+    float v = part[0];
+    for (int o = 1; o < b.parts; ++o) v += part[o * b.chunks * 256];
+    dx[p]  = v;
+    gdx[p] = v;
+  }
+}
+
+// (everything from memory is asked for first: the gradient, the filters' cache lines, the table, and
+// the outputs of the activations on the way)
+__global__ void __launch_bounds__(TB_THREADS)
+tiny_net_back_kernel(const TinyPlan *__restrict__ plan, const int m) {
+  extern __shared__ float lds[];
+  constexpr int AHEAD = 4;   // gradients a thread holds, and layers whose outputs it does
+  const int s = blockIdx.x, ci = blockIdx.y, n = plan->n, tid = threadIdx.x;
+  const TinyLayer *__restrict__ L = &plan->l[m];
+  const int K = L->K, H = L->H, W = L->W, R = L->R, S = L->S, OW = L->OW, out_size = L->out_size, taps = R * S;
+  const float *gdy = (m == n - 1 ? plan->dloss : plan->l[m + 1].dx) + static_cast<size_t>(s) * out_size;
+  float dy[AHEAD];
+#pragma unroll
+  for (int j = 0; j < AHEAD; ++j) dy[j] = gdy[min(tid + TB_THREADS * j, out_size - 1)];
+  int plane = H * W;
+  const BackSplit b = back_split(H, W, K);
+  const int kp = b.parts > 1 ? wave_index() / b.chunks : 0;
+  const int c_lo = min(K, kp * b.per_part), c_hi = kp < b.parts ? min(K, c_lo + b.per_part) : c_lo;
+  float y[AHEAD];
+  int p_li = plane;
+#pragma unroll
+  for (int j = 0; j < AHEAD; ++j) {
+    y[j] = 0.0f;
+    const TinyLayer *__restrict__ A = &plan->l[max(m - 1 - j, 0)];
+    if (m - 1 - j < 1) continue;
+    if (A->kind == TDH_L_ACT) y[j] = A->out[static_cast<size_t>(s) * A->out_size + ci * p_li + min(tid, p_li - 1)];
+    else p_li = A->H * A->W;
+  }
+  uint64_t connected = ~0ull;
+  if (L->tbl) connected = __ballot((tid & 63) < c_hi - c_lo && L->tbl[ci * K + min(c_lo + (tid & 63), K - 1)] != 0);
+  int touch = 0;
+  for (int co = c_lo; co < c_hi; ++co) {
+    typedef const int __attribute__((address_space(4))) *ScalarInts;
+    const ScalarInts line = (ScalarInts)(L->w + static_cast<size_t>(co * L->C + ci) * taps);
+    touch |= line[0] | line[taps - 1];
+  }
+  float *framed = lds, *scratch = lds + plan->back_scratch, *cur = lds + plan->back_planes;
+  float *gdx = L->dx + static_cast<size_t>(s) * L->in_size + ci * plane;
+  // dY into its frame of zeros
+  const int PW = W + S - 1, PP = (H + R - 1) * PW, corner = (R - 1 - L->ph) * PW + S - 1 - L->pw;
+  const FastDiv d_oplane = L->d_oplane, d_ow = L->d_ow;
+  for (int i = tid; i < K * PP; i += TB_THREADS) framed[i] = 0.0f;
+  asm volatile("" ::"s"(touch));
+  lds_barrier();
+  auto place = [&](int e, float v) {
+    uint32_t co, r, oy, ox;
+    d_oplane.divmod(e, co, r);
+    d_ow.divmod(r, oy, ox);
+    framed[co * PP + corner + oy * PW + ox] = v;
+  };
+#pragma unroll
+  for (int j = 0; j < AHEAD; ++j)
+    if (tid + TB_THREADS * j < out_size) place(tid + TB_THREADS * j, dy[j]);
+  for (int e = tid + TB_THREADS * AHEAD; e < out_size; e += TB_THREADS) place(e, gdy[e]);
+  lds_barrier();
+  if (R == 5) conv_back_dx<5, 5>(L, b, framed, cur, gdx, scratch, ci, kp, c_lo, c_hi, connected);
+  else conv_back_dx<3, 3>(L, b, framed, cur, gdx, scratch, ci, kp, c_lo, c_hi, connected);
+  for (int li = m - 1; li >= 1; --li) {
+    L = &plan->l[li];
+    lds_barrier();
+    if (L->kind == TDH_L_ACT) {
+      const int act = L->act, j = m - 1 - li;
+      const float p0 = L->p0;
+      const size_t at = static_cast<size_t>(s) * L->out_size + ci * plane;
+      const float *out = L->out + at;
+      float *g = L->dx + at;
+      const float first = j == 0 ? y[0] : j == 1 ? y[1] : j == 2 ? y[2] : y[3];
+      for (int i = tid; i < plane; i += TB_THREADS) {
+        const float v = tn_act_bwd(act, p0, i == tid && j < AHEAD ? first : out[i], cur[i]);
+        cur[i] = v;
+        g[i]   = v;
+      }
+      continue;
+    }
+    const int H = L->H, W = L->W, OH = L->OH, OW = L->OW, R = L->R, S = L->S, sh = L->sh, sw = L->sw, iplane = H * W;
+    const bool most = L->kind == TDH_L_MAXPOOL, two = R == 2 && S == 2 && sh == 2 && sw == 2;
+    const FastDiv d_w = L->d_w;
+    const int32_t *argmax = most ? L->argmax + static_cast<size_t>(s) * L->out_size + ci * plane : nullptr;
+    const float weight = most ? 0.0f : L->w[ci] * L->scale;
+    float *nxt = cur + plane, *g = L->dx + static_cast<size_t>(s) * L->in_size + ci * iplane;
+    for (int e = tid; e < iplane; e += TB_THREADS) {
+      uint32_t yy, xx;
+      d_w.divmod(e, yy, xx);
+      const int iy = yy, ix = xx;
+      float v;
+      if (most) {   // maxpool_bwd
+        const int ox = min(OW - 1, two ? ix >> 1 : ix / sw), oy = min(OH - 1, two ? iy >> 1 : iy / sh);
+        const bool covered = ix < ox * sw + S && iy < oy * sh + R;
+        const int outi = covered ? oy * OW + ox : 0;
+        v = covered && argmax[outi] == ci * iplane + e ? cur[outi] : 0.0f;
+      } else {      // avepool_bwd_dx
+        const int ox = two ? ix >> 1 : ix < S ? 0 : (ix - S + sw) / sw, oy = two ? iy >> 1 : iy < R ? 0 : (iy - R + sh) / sh;
+        v = weight * cur[oy * OW + ox];
+      }
+      nxt[e] = v;
+      g[e]   = v;
+    }
+    cur   = nxt;
+    plane = iplane;
   }
 }
 
@@ -1392,9 +1691,38 @@ int tiny_prepare() {
                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(TINY_LDS_MAX_BYTES)));
     TDH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&tiny_net_param_kernel),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(TINY_LDS_MAX_BYTES)));
+    for (const void *k : {reinterpret_cast<const void *>(&tiny_net_front_kernel), reinterpret_cast<const void *>(&tiny_net_back_kernel)})
+      TDH_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(TINY_LDS_MAX_BYTES)));
     attr_set = true;
   }
   return TDH_OK;
+}
+
+// Whether the net begins with what the front and back kernels take, and their LDS
+static void plan_split(TinyPlan &P) {
+  P.split = 0;
+  const TinyLayer &F = P.l[0];
+  if (F.kind != TDH_L_CONV || !((F.R == 5 && F.S == 5) || (F.R == 3 && F.S == 3)) || conv_is_matvec(F) ||
+      !(P.first_dx_as_job || P.skip_first_dx))
+    return;
+  int m = 1;
+  size_t front = F.OH * F.OW, back = 0;
+  for (; m < P.n; ++m) {
+    const TinyLayer &L = P.l[m];
+    if (L.kind == TDH_L_ACT && L.act != TDH_ACT_SOFTMAX) continue;
+    if (L.kind != TDH_L_MAXPOOL && L.kind != TDH_L_AVEPOOL) break;
+    front += L.OH * L.OW;
+    back += L.H * L.W;
+  }
+  if (m == P.n || !P.l[m].dx_framed || P.l[m].K > 64) return;   // (64: conv_back_dx)
+  const TinyLayer &L = P.l[m];
+  P.back_scratch = (conv_framed_floats(L) + 3) & ~3;
+  const BackSplit b = back_split(L.H, L.W, L.K);
+  P.back_planes  = P.back_scratch + b.parts * b.chunks * 256;
+  P.back_floats  = P.back_planes + static_cast<int>(back) + L.H * L.W;
+  P.front_floats = static_cast<int>(front);
+  if (std::max(static_cast<size_t>(P.back_floats), P.in_size + front) * sizeof(float) > TINY_LDS_MAX_BYTES) return;
+  P.split = m;
 }
 
 int tiny_build_jobs(TinyPlan &P) {
@@ -1413,6 +1741,7 @@ int tiny_build_jobs(TinyPlan &P) {
     }
   }
   P.first_dx_as_job = P.l[0].dx_framed && P.n > 1 && !P.skip_first_dx;
+  plan_split(P);
   for (int i = 0; i < P.n; ++i) {
     const TinyLayer &L = P.l[i];
     if (i == 0 && P.first_dx_as_job) {
@@ -1502,10 +1831,33 @@ int tiny_build_jobs(TinyPlan &P) {
 
 int launch_tiny_step(const TinyPlan &plan, const TinyPlan *dev_plan, int loss, int softmax_xent, int batch,
                      const float *x, const float *t) {
-  ProfScope prof("tiny_net_step", plan.flop_per_sample * batch * (2.0 / 3.0), WORK_FLOP);
-  TDH_LAUNCH(tiny_net_step_kernel, dim3(batch), dim3(TN_THREADS), plan.lds_floats * sizeof(float), ctx().stream,
-             dev_plan, loss, softmax_xent, x, t);
-  TDH_LAUNCH_CHECK();
+  // The ends of the chain a channel a workgroup while there is a compute unit for each. LeNet-5 at 16 / 32 / 64 /
+  // 120 samples, us for the three launches and for the step kernel alone: 34.5 / 40.1, 35.5 / 40.2, 40.8 / 40.3, 52.4 /
+  // 43.1: with several workgroups a compute unit, each of which frames all of dY for its one channel, they lose.
+  const TinyLayer &F = plan.l[0], &M = plan.l[plan.split];
+  const int m = plan.split && batch * std::max(F.K, M.C) <= 256 ? plan.split : 0;
+  const double front_flop = m ? 2.0 * F.out_size * F.C * F.R * F.S * batch : 0.0;
+  const double back_flop  = m ? 2.0 * M.out_size * M.C * M.R * M.S * batch : 0.0;
+  if (m) {
+    ProfScope prof("tiny_net_front", front_flop, WORK_FLOP);
+    // (a pixel a thread, in whole waves)
+    const int plane = F.OH * F.OW, rounds = ceil_div(plane, TF_THREADS), threads = 64 * ceil_div(plane, 64 * rounds);
+    TDH_LAUNCH(tiny_net_front_kernel, dim3(batch, F.K), dim3(threads), (plan.in_size + plan.front_floats) * sizeof(float),
+               ctx().stream, dev_plan, m, plan.in_size, x);
+    TDH_LAUNCH_CHECK();
+  }
+  {
+    ProfScope prof("tiny_net_step", plan.flop_per_sample * batch * (2.0 / 3.0) - front_flop - back_flop, WORK_FLOP);
+    TDH_LAUNCH(tiny_net_step_kernel, dim3(batch), dim3(TN_THREADS), plan.lds_floats * sizeof(float), ctx().stream,
+               dev_plan, m, loss, softmax_xent, x, t);
+    TDH_LAUNCH_CHECK();
+  }
+  if (m) {
+    ProfScope prof("tiny_net_back", back_flop, WORK_FLOP);
+    TDH_LAUNCH(tiny_net_back_kernel, dim3(batch, M.C), dim3(TB_THREADS), plan.back_floats * sizeof(float), ctx().stream,
+               dev_plan, m);
+    TDH_LAUNCH_CHECK();
+  }
   return TDH_OK;
 }
 
