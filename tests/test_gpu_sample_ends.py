@@ -53,3 +53,54 @@ def test_every_tensor_matches_oracle(T, O, W, name, batch):
             assert_close(net.layer_grad(i, 0), ref.layer_dw(i), what=f"layer {i} dW")
             assert_close(net.layer_grad(i, 1), ref.layer_db(i), what=f"layer {i} db")
     net.close()
+
+
+# nets whose parameter gradients take every road: channel pairs of 3x3 and 5x5 windows, of any window and stride, outer
+# products in words and one by one, average pools, tables
+PARAM_NETS = {
+    "wide": NETS["wide"], "deep_front": NETS["deep_front"], "two": NETS["two"],
+    "any_window": ([("conv", 14, 13, 2, 4, 5, False), ("act", "tanh"), ("avepool", 11, 10, 5, 1), ("conv", 11, 10, 5, 2, 6, False),
+                    ("act", "sigmoid"), ("fc", 6 * 90, 7)], "mse", "adam"),
+    "fc": ([("fc", 37, 24), ("act", "tanh"), ("fc", 24, 36), ("act", "sigmoid"), ("fc", 36, 5)], "mse", "adam"),
+    "matvec": ([("conv", 5, 5, 3, 5, 8, False, [[(ci + co) % 2 == 0 for co in range(8)] for ci in range(3)]), ("act", "tanh"),
+                ("fc", 8, 3)], "mse", "adam"),
+}
+
+
+@pytest.mark.parametrize("kind", ["sgd", "momentum", "adam", "adagrad", "rmsprop", "adamax", "nesterov"])
+@pytest.mark.parametrize("name,batch", [("wide", 16), ("deep_front", 32), ("deep_front", 33), ("two", 1), ("any_window", 31),
+                                        ("any_window", 50), ("fc", 32), ("fc", 70), ("matvec", 17), ("matvec", 100)])
+def test_gradients_and_updates_of_one_group_and_of_several(T, O, W, name, batch, kind):
+    """Up to 32 samples the launch that adds up the gradients updates; larger batches leave slices. Gradients against the
+    oracle; updates, of a step that adds to the gradients of a pass without one, against the layer-by-layer step."""
+    spec, params, x, t, batch, loss, _, _, net, ref = build(T, O, W, name, batch, SAMPLE | FUSE, nets=PARAM_NETS)
+    *_, replay, _ = build(T, O, W, name, batch, SAMPLE | FUSE | 2, nets=PARAM_NETS)
+    *_, layered, _ = build(T, O, W, name, batch, FUSE, nets=PARAM_NETS)
+    xd, td = T.to_device(x), T.to_device(t)
+    alpha = {"sgd": 1e-3, "momentum": 1e-3, "nesterov": 1e-3}.get(kind, 1e-2)
+    opts = [T.opt_desc(kind, alpha=alpha) for _ in range(3)]
+    for m in (net, replay, layered):
+        m.train_step(None, loss, batch, xd, td, do_update=False)
+    ref.train_step(O.opt_desc(kind), loss, x, t, do_update=False)
+    grads = {(i, w): (ref.layer_dw(i) if w == 0 else ref.layer_db(i)).copy() for i, w, _ in params}
+    for (i, w), want in grads.items():
+        assert_close(net.layer_grad(i, w), want, what=f"gradient {i}.{w}")
+    for k, m in enumerate((net, replay, layered)):
+        for _ in range(2):
+            m.train_step(opts[k], loss, batch, xd, td)
+    divides = kind in ("adam", "adagrad", "rmsprop", "adamax")
+    for i, w, a in params:
+        got, want = net.get_param(i, w), layered.get_param(i, w)
+        assert np.array_equal(got, replay.get_param(i, w))
+        if divides:
+            # a gradient's relative error of 1e-4 (of its tensor's rms) moves a weight by up to alpha times itself over the
+            # gradient's own size: elements below a hundredth of the rms are left out, the others get 1e-2 of a step
+            g = np.abs(grads[(i, w)].ravel())
+            on = g > 1e-2 * np.sqrt(np.mean(g * g))
+            assert np.abs(got.ravel() - want.ravel())[on].max(initial=0.0) <= 2 * 2 * 1e-2 * alpha, f"{kind} parameter {i}.{w}"
+        else:
+            assert_close(got, want, what=f"{kind} parameter {i}.{w}")
+        assert not net.layer_grad(i, w).any()
+    assert opts[0].b1_t == opts[1].b1_t == opts[2].b1_t and opts[0].b2_t == opts[1].b2_t == opts[2].b2_t
+    for m in (net, replay, layered):
+        m.close()

@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "common.h"
+#include "opt_update.h"
 #include "conv_s1.h"
 #include "split_bf16.h"
 
@@ -346,46 +347,6 @@ softmax_fwd_xent_kernel(const float *__restrict__ x, const float *__restrict__ t
 }
 
 // --------------------------------------------------------------- optimizers
-// tiny_dnn/optimizers/optimizer.h; g = merged * grad_scale is layer::update_weight's
-// diff (tiny_dnn/layers/layer.h:668-673). Scalars that the reference derives once per
-// call from its float members (1 - b1_t, ...) arrive precomputed in float.
-struct OptScalars {
-  float alpha, lambda, mu, b1, b2, eps, omb1, omb2, omb1t, omb2t, grad_scale;
-  double adamax_lr;  // alpha / (1.0 - b1_t), evaluated in double as the reference does
-};
-
-template <int KIND>
-__device__ __forceinline__ void opt_one(float g, float &w, float &s0, float &s1,
-                                        const OptScalars &p) {
-  g *= p.grad_scale;
-  if (KIND == TDH_OPT_SGD) {  // :185-188
-    w = w - p.alpha * (g + p.lambda * w);
-  } else if (KIND == TDH_OPT_MOMENTUM) {  // :205-213
-    const float V = p.mu * s0 - p.alpha * (g + w * p.lambda);
-    w += V;
-    s0 = V;
-  } else if (KIND == TDH_OPT_NESTEROV) {  // :231-239
-    const float V = p.mu * s0 - p.alpha * (g + w * p.lambda);
-    w += (-p.mu) * s0 + (1 + p.mu) * V;
-    s0 = V;
-  } else if (KIND == TDH_OPT_ADAM) {  // :112-127, eps inside the square root
-    s0 = p.b1 * s0 + p.omb1 * g;
-    s1 = p.b2 * s1 + p.omb2 * g * g;
-    w -= p.alpha * (s0 / p.omb1t) / sqrtf((s1 / p.omb2t) + p.eps);
-  } else if (KIND == TDH_OPT_ADAGRAD) {  // :60-66
-    s0 += g * g;
-    w -= p.alpha * g / (sqrtf(s0) + p.eps);
-  } else if (KIND == TDH_OPT_RMSPROP) {  // :81-88
-    s0 = p.mu * s0 + (1 - p.mu) * g * g;
-    w -= p.alpha * g / sqrtf(s0 + p.eps);
-  } else if (KIND == TDH_OPT_ADAMAX) {  // :153-165
-    s0 = p.b1 * s0 + p.omb1 * g;
-    s1 = fmaxf(p.b2 * s1, fabsf(g));
-    w  = static_cast<float>(static_cast<double>(w) -
-                           p.adamax_lr * static_cast<double>(s0 / (s1 + p.eps)));
-  }
-}
-
 template <int KIND, int NSTATE>
 __global__ void __launch_bounds__(EW_THREADS)
 opt_kernel(const float *__restrict__ g, float *__restrict__ w, float *__restrict__ s0,
@@ -827,8 +788,7 @@ int launch_opt_update(tdh_opt *o, size_t n, const float *g, float grad_scale, fl
   p.grad_scale = grad_scale;
   p.adamax_lr  = static_cast<double>(o->alpha) / (1.0 - static_cast<double>(o->b1_t));
   int rc = TDH_OK;
-  const int nstate = (o->kind == TDH_OPT_SGD) ? 0
-                     : (o->kind == TDH_OPT_ADAM || o->kind == TDH_OPT_ADAMAX) ? 2 : 1;
+  const int nstate = opt_states(o->kind);
   if (n > 0) {
     if (nstate >= 1 && !s0) return set_error(TDH_ERR_INVALID, "optimizer %d needs state s0", o->kind);
     if (nstate >= 2 && !s1) return set_error(TDH_ERR_INVALID, "optimizer %d needs state s1", o->kind);
@@ -845,12 +805,7 @@ int launch_opt_update(tdh_opt *o, size_t n, const float *g, float grad_scale, fl
   }
   if (rc != TDH_OK) return rc;
   // the reference advances the powers once per update() call, whatever the tensor size
-  if (o->kind == TDH_OPT_ADAM) {
-    o->b1_t *= o->b1;
-    o->b2_t *= o->b2;
-  } else if (o->kind == TDH_OPT_ADAMAX) {
-    o->b1_t *= o->b1;
-  }
+  opt_advance(o, 1);
   return TDH_OK;
 }
 
@@ -885,21 +840,14 @@ int launch_opt_update_multi(tdh_opt *o, const OptTensor *dev_table, int n_tensor
         if (pend.sum[q].g == host_table[k].g) idx.pend_of[k] = static_cast<int8_t>(q);
     }
   }
-  OptScalars p;
-  p.alpha = o->alpha; p.lambda = o->lambda; p.mu = o->mu; p.b1 = o->b1; p.b2 = o->b2;
-  p.eps = o->eps;
-  p.omb1 = 1.0f - o->b1; p.omb2 = 1.0f - o->b2;
-  p.omb1t = p.omb2t = 0.0f;
-  p.grad_scale = grad_scale;
-  p.adamax_lr  = 0.0;
+  const OptScalars p = opt_scalars(*o, grad_scale);
   static const char *const tags[] = {"opt_sgd_multi", "opt_momentum_multi", "opt_adam_multi",
                                      "opt_adagrad_multi", "opt_rmsprop_multi", "opt_adamax_multi",
                                      "opt_nesterov_multi"};
   TDH_CHECK_ARG(o->kind >= 0 && o->kind <= TDH_OPT_NESTEROV, "optimizer kind %d is not supported",
                 o->kind);
-  const int advance = o->kind == TDH_OPT_ADAM ? 2 : o->kind == TDH_OPT_ADAMAX ? 1 : 0;
-  const int nstate = (o->kind == TDH_OPT_SGD) ? 0
-                     : (o->kind == TDH_OPT_ADAM || o->kind == TDH_OPT_ADAMAX) ? 2 : 1;
+  const int advance = opt_powers(o->kind);
+  const int nstate = opt_states(o->kind);
   // gradient read (+ cleared), weight read+write, states read+write
   ProfScope prof(tags[o->kind], (12.0 + 8.0 * nstate + (zero_grad ? 4.0 : 0.0)) * total_params + pending_bytes,
                  WORK_BYTE);
@@ -918,14 +866,7 @@ int launch_opt_update_multi(tdh_opt *o, const OptTensor *dev_table, int n_tensor
   }
 #undef TDH_LAUNCH_MULTI
   TDH_LAUNCH_CHECK();
-  for (int j = 0; j < n_tensors; ++j) {
-    if (o->kind == TDH_OPT_ADAM) {
-      o->b1_t *= o->b1;
-      o->b2_t *= o->b2;
-    } else if (o->kind == TDH_OPT_ADAMAX) {
-      o->b1_t *= o->b1;
-    }
-  }
+  opt_advance(o, n_tensors);
   return TDH_OK;
 }
 

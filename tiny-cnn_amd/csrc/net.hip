@@ -260,6 +260,7 @@ int build_tiny_plan(tdh_net *net) {
   P.n       = n;
   P.in_size = static_cast<int>(net->layers[0].in_size);
   size_t lds = net->layers[0].in_size, gmax = net->layers[0].in_size, slice_floats = 0;
+  const auto slices_of = [](size_t len, int count) { return ceil_div_sz(len * count, 4) * 4; };   // (16-byte aligned slices)
   int tensors = 0;
   for (int i = 0; i < n; ++i) {
     const tdh_net::Layer &L = net->layers[i];
@@ -327,8 +328,6 @@ int build_tiny_plan(tdh_net *net) {
       default: return TDH_OK;   // batch normalization, dropout: the layer-by-layer step
     }
     tensors += (L.w_size ? 1 : 0) + (L.b_size ? 1 : 0);
-    slice_floats += (ceil_div_sz(L.w_size * static_cast<size_t>(net->max_batch), 4) * 4) +
-                    (ceil_div_sz(L.b_size * static_cast<size_t>(net->max_batch), 4) * 4);   // (16-byte aligned slices)
   }
   P.lds_g0 = static_cast<int>(lds);
   P.lds_g1 = static_cast<int>(lds + gmax);
@@ -339,11 +338,23 @@ int build_tiny_plan(tdh_net *net) {
   P.lds_floats = static_cast<int>(lds);
   P.dloss      = net->layers[n - 1].dout;
   P.mse_factor = 2.0f / static_cast<float>(net->layers[n - 1].out_size);
-  if (tensors > TINY_MAX_TENSORS || slice_floats > (64u << 20)) return TDH_OK;
-  TDH_TRY(tiny_build_jobs(P));   // (adds the framed dY's LDS to the plan's)
+  if (tensors > TINY_MAX_TENSORS) return TDH_OK;
+  TDH_TRY(tiny_layout(P));
   if (std::max(P.lds_floats, P.lds_job_floats) * sizeof(float) > TINY_LDS_MAX_BYTES) return TDH_OK;
+  const int split_batch = std::min(tiny_most_split(P), net->max_batch);   // (whose back kernel leaves slices per sample)
+  int groups[TINY_MAX_LAYERS];
+  for (int i = 0; i < n; ++i) {
+    groups[i] = 1;
+    for (int b = 1; b <= net->max_batch; ++b) groups[i] = std::max(groups[i], tiny_groups(P, i, b));
+    const int parts = groups[i] + (i < P.split ? split_batch : 0);
+    slice_floats += slices_of(net->layers[i].w_size, parts) + slices_of(net->layers[i].b_size, parts) + 8;
+  }
+  slice_floats += slices_of(net->layers[0].w_size, 1);
+  if (slice_floats > (64u << 20)) return TDH_OK;
   float *slices = nullptr;
   TDH_TRY(net_alloc(net, slice_floats, &slices, false));
+  P.first_w = slices;
+  slices += slices_of(net->layers[0].w_size, 1);
   TinyMerge &M = net->tiny_merge;
   std::memset(&M, 0, sizeof(M));
   int blocks = 0;
@@ -357,17 +368,30 @@ int build_tiny_plan(tdh_net *net) {
       M.slices[M.n] = slices;
       M.g[M.n]      = which ? L.db : L.dw;
       M.len[M.n]    = static_cast<int>(len);
+      M.layer[M.n]  = i;
       M.first_block[M.n] = blocks;
       blocks += ceil_div(static_cast<int>(len), 256);
       ++M.n;
-      slices += ceil_div_sz(len * static_cast<size_t>(net->max_batch), 4) * 4;
+      slices += slices_of(len, groups[i]);
+      if (i < P.split) {
+        (which ? T.pb_part : T.pw_part) = slices;
+        slices += slices_of(len, split_batch);
+      }
     }
+    T.tw.index = T.tb.index = -1;
+    for (size_t j = 0; j < net->opt_table_host.size(); ++j) {
+      const OptTensor &o = net->opt_table_host[j];
+      if (L.w_size && o.g == L.dw) T.tw = TinyTensor{o.g, o.w, o.s0, o.s1, static_cast<int>(j)};
+      if (L.b_size && o.g == L.db) T.tb = TinyTensor{o.g, o.w, o.s0, o.s1, static_cast<int>(j)};
+    }
+    if ((L.w_size && T.tw.index < 0) || (L.b_size && T.tb.index < 0)) return TDH_OK;
   }
   M.first_block[M.n] = blocks;
   for (int i = 0; i < n; ++i) {
     TinyLayer &T = P.l[i];
     const auto fd = [](int v) { return FastDiv(static_cast<uint32_t>(v > 0 ? v : 1)); };
-    T.d_oplane = fd(T.OH * T.OW); T.d_ow = fd(T.OW); T.d_iplane = fd(T.H * T.W); T.d_w = fd(T.W);
+    T.d_oplane = fd(T.OH * T.OW); T.d_ow = fd(T.OW); T.d_oh = fd(T.OH); T.d_quads = fd((T.OW + 3) / 4);
+    T.d_vquads = fd((T.OH + 3) / 4); T.d_iplane = fd(T.H * T.W); T.d_w = fd(T.W);
     T.d_taps = fd(T.R * T.S); T.d_s = fd(T.S); T.d_c = fd(T.C); T.d_out = fd(T.out_size);
     T.d_nk = fd(T.C * T.R * T.S);
   }
@@ -1079,17 +1103,28 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
                         bool keep_packs, bool forked = false) {
   const KeepF32 keep_f32(has_batchnorm(net));
   if (tiny_step_applies(net, loss_kind)) {
-    // a small net: one workgroup per sample runs forward, loss and the input gradients out of
-    // LDS, a second launch computes every sample's weight and bias gradients, a third adds
-    // those slices in sample order, the fourth is the optimizer (tiny_net.hip)
+    // a small net: forward, loss and the input gradients out of LDS, a workgroup per sample (the ends of that chain
+    // a workgroup per channel where there is room), then the parameter gradients over the batch (tiny_net.hip)
     const tdh_layer &closing = net->layers.back().spec;
     const int softmax_xent = closing.kind == TDH_L_ACT && closing.act == TDH_ACT_SOFTMAX;
     net->dx_unwritten.assign(net->layers.size(), 0);   // everything is written to memory as well
     if (net_skips_input_grad(net)) net->dx_unwritten[0] = 1;
     net->out_unwritten.assign(net->layers.size(), 0);
     TDH_TRY(launch_tiny_step(net->tiny, net->tiny_dev, loss_kind, softmax_xent, batch, x, t));
-    TDH_TRY(launch_tiny_params(net->tiny, net->tiny_dev, batch, x));
-    // the samples' slices: added to the gradient tensors in sample order by a launch of their
+    // One group of samples: the same launch is the update, unless copies of filters hang on it that only the optimizer's
+    // kernel writes.
+    bool may_update = do_update, updated = false;
+    for (const OptTensor &o : net->opt_table_host)
+      for (const void *copy : o.packed) may_update = may_update && !(keep_packs && copy);
+    TDH_TRY(launch_tiny_params(net->tiny, net->tiny_dev, batch, x, may_update ? opt : nullptr, net->opt_tensors, powers_in,
+                               powers_out, &updated));
+    if (updated) {
+      after_update(net, keep_packs);
+      return post_update(net);
+    }
+    for (int j = 0; j < net->tiny_merge.n; ++j)
+      net->tiny_merge.count[j] = tiny_groups(net->tiny, net->tiny_merge.layer[j], batch);
+    // the groups' slices: added to the gradient tensors in order by a launch of their
     // own when the step stops there; otherwise the optimizer adds them up as it does the split
     // sums of the layer-by-layer step (it clears the gradient tensors afterwards either way)
     const TinyMerge &M = net->tiny_merge;
@@ -1101,9 +1136,9 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
       for (const tdh_net::Layer &L : net->layers)
         if ((M.g[j] == L.dw && L.w_sums_in_opt) || (M.g[j] == L.db && L.b_sums_in_opt)) small_blocks = true;
       to_optimizer = small_blocks;
-      pending.sum[pending.n++] = {M.slices[j], M.g[j], static_cast<uint32_t>(batch), static_cast<uint32_t>(M.len[j])};
+      pending.sum[pending.n++] = {M.slices[j], M.g[j], static_cast<uint32_t>(M.count[j]), static_cast<uint32_t>(M.len[j])};
     }
-    if (!to_optimizer) TDH_TRY(launch_tiny_merge(net->tiny_merge, batch));
+    if (!to_optimizer) TDH_TRY(launch_tiny_merge(net->tiny_merge));
     if (!do_update) return TDH_OK;
     TDH_TRY(launch_opt_update_multi(opt, net->opt_table, net->opt_tensors, net->opt_blocks, net->opt_params, 1.0f,
                                     1, powers_in, powers_out, to_optimizer ? &pending : nullptr,

@@ -10,8 +10,11 @@ constexpr int TINY_MAX_LAYERS     = 16;
 constexpr int TINY_MAX_TENSORS    = 2 * TINY_MAX_LAYERS;
 constexpr size_t TINY_LDS_MAX_BYTES = 152u << 10;  // of a compute unit's 160 KiB
 constexpr int TINY_SCRATCH_FLOATS = 4096;          // LDS where the partial sums of a split layer meet
-constexpr int TINY_MAX_JOBS       = 256;           // pieces of the parameter-gradient kernel's work per sample
 
+struct TinyTensor {
+  float *g, *w, *s0, *s1;
+  int index;                   // in the optimizer's table
+};
 struct TinyLayer {
   int kind, act;               // TDH_L_*, TDH_ACT_* (activation layers)
   float p0;                    // leaky relu's slope
@@ -24,15 +27,18 @@ struct TinyLayer {
   float *out;                  // memory: this layer's output [batch][out_size]
   float *dx;                   // memory: gradient w.r.t. this layer's input [batch][in_size]
   int32_t *argmax;             // memory: max-pool records [batch][out_size]
-  float *gw, *gb;              // memory: per-sample gradient slices [batch][nw], [batch][nb]
+  float *gw, *gb;              // memory: a gradient slice per group of samples, [group][nw], [group][nb]
+  float *pw_part, *pb_part;    // memory, layers in front of TinyPlan::split: what the back kernel leaves per sample
+  TinyTensor tw, tb;           // weights and bias, as the optimizer has them
+  int dw_chunk, dw_quads;      // parameter gradients: samples in LDS at a time; whether four pixels go together
   int nw, nb;
   int lds_in, lds_out;         // where the layer's input and output live in LDS (floats)
   // divisions by the layer's sizes as multiply-high + shift
-  FastDiv d_oplane, d_ow, d_iplane, d_w, d_taps, d_s, d_c, d_out, d_nk;
+  FastDiv d_oplane, d_ow, d_oh, d_quads, d_vquads, d_iplane, d_w, d_taps, d_s, d_c, d_out, d_nk;
   // the unrolled input gradient of a stride-1 3x3 / 5x5 convolution reads dY from a zero-framed copy,
   // [K][H + R - 1][W + S - 1] floats in LDS; 0 when the layer takes the general loops
   int dx_framed;
-  FastDiv d_pplane, d_pw;
+  FastDiv d_pplane, d_pw, d_pw4;
   // A stride-1 convolution's forward product without padding on the matrix cores (conv_mfma in
   // tiny_net.hip): where in LDS the step kernel keeps the filters as [co][k] (k = (ci, tap), rows
   // padded with zeros), the input offset of every k and a copy of the bias; -1: the scalar loops
@@ -47,39 +53,30 @@ struct TinyLayer {
   int mf_dx_w, mf_dx_ko, mf_dx_d;
 };
 
-// One workgroup's share of the parameter-gradient kernel for one sample: the units
-// [base, base + count) of a layer's weight-gradient work (the bias gradient goes with base 0,
-// except that of a convolution that is not a matrix-vector product, which is a job of its own),
-// or, for the first layer, the wave items [base, base + count) of its input gradient.
-struct TinyJob {
-  int16_t layer, what;         // what: 0 = weight (/ bias) gradient, 1 = input gradient, 2 = bias gradient
-  int base, count;
-};
-
 struct TinyPlan {
   TinyLayer l[TINY_MAX_LAYERS];
   int n, in_size;
   // the second convolution, where the layers in front of it run a channel a workgroup (tiny_net.hip), or 0;
   // LDS of those launches: floats behind the input in front, and offsets behind the framed dY
-  int split, front_floats, back_scratch, back_planes, back_floats;
+  int split, front_floats, back_scratch, back_planes, back_sample, back_sample_floats, back_floats;
   int lds_g0, lds_g1, lds_w, lds_pad, lds_floats;   // lds_pad: the zero-framed dY
   int n_mfma, mfma_layers[TINY_MAX_LAYERS];   // the layers with operands to stage for the matrix cores
   int mf_ahead;                // the layer (> 0) whose filters wait in registers until the layer in front of it runs, or -1
   float mse_factor;            // 2 / outputs
   float *dloss;                // memory: gradient w.r.t. the net's output [batch][out_size]
   double flop_per_sample;
-  TinyJob jobs[TINY_MAX_JOBS];
-  int n_jobs;
-  int first_dx_as_job;         // the first layer's input gradient is among the jobs
+  int first_dx_as_job;         // the first layer's input gradient is computed beside the parameter gradients,
+  float *first_w;              // ... from this copy of its filters (memory), which the step kernel makes
   int skip_first_dx;           // nobody wants the gradient of the net's input: it is not computed
   int lds_job_floats;          // LDS of the parameter-gradient kernel
 };
 
-// the per-sample slices of every trainable tensor and the gradient tensor each is added to
+// the groups' slices of every trainable tensor and the gradient tensor each is added to
 struct TinyMerge {
   const float *slices[TINY_MAX_TENSORS];
   float *g[TINY_MAX_TENSORS];
-  int len[TINY_MAX_TENSORS];
+  int len[TINY_MAX_TENSORS], layer[TINY_MAX_TENSORS];
+  int count[TINY_MAX_TENSORS];                       // slices (of the batch in use)
   int first_block[TINY_MAX_TENSORS + 1];
   int n;
 };
@@ -91,13 +88,19 @@ int tiny_prepare();
 // this step's loss and whether the closing softmax folds into it
 int launch_tiny_step(const TinyPlan &plan, const TinyPlan *dev_plan, int loss, int softmax_xent, int batch,
                      const float *x, const float *t);
-// Cuts the parameter-gradient work of the plan's layers into jobs, decides which layers' input
-// gradients read a zero-framed dY and appends that area to the plan's LDS (lds_floats comes
-// in as the floats in use so far; the caller checks the result against TINY_LDS_MAX_BYTES).
-int tiny_build_jobs(TinyPlan &plan);
-// every layer's per-sample weight and bias gradient slices (and the first layer's input
-// gradient) from the outputs and gradients that launch_tiny_step left in memory
-int launch_tiny_params(const TinyPlan &plan, const TinyPlan *dev_plan, int batch, const float *x);
-int launch_tiny_merge(const TinyMerge &m, int batch);
+// Decides which layers' input gradients read a zero-framed dY, which products run on the matrix cores and
+// which layers the front and back kernels take, and appends what that needs to the plan's LDS (lds_floats
+// comes in as the floats in use so far; the caller checks the result against TINY_LDS_MAX_BYTES).
+int tiny_layout(TinyPlan &plan);
+// the largest batch that runs the front and back kernels (0: none)
+int tiny_most_split(const TinyPlan &plan);
+// groups of samples whose gradients of a layer leave a slice each
+int tiny_groups(const TinyPlan &plan, int layer, int batch);
+// Every layer's weight and bias gradients (and the first layer's input gradient) from the outputs and
+// gradients that launch_tiny_step left in memory. With `update` and one group of samples everywhere, the optimizer's step
+// on all tensors as well (powers_in, powers_out: as in launch_opt_update_multi; *updated), else the slices.
+int launch_tiny_params(const TinyPlan &plan, const TinyPlan *dev_plan, int batch, const float *x, tdh_opt *update,
+                       int n_tensors, const float *powers_in, float *powers_out, bool *updated);
+int launch_tiny_merge(const TinyMerge &m);
 
 }  // namespace tdh

@@ -1,19 +1,20 @@
-// tiny_net.hip — the whole train step of a small net in three launches, the optimizer's included.
+// tiny_net.hip — the whole train step of a small net in two to five launches, the optimizer's included.
 //
 // A net whose activations of one sample fit in LDS (LeNet-5: 15 k floats) spends its step in
 // launches, not in arithmetic: 24 kernels of 3-10 us on tensors of a few kilobytes. Here one
 // workgroup takes one sample through the chain that has to run in order: forward through every
 // layer with all layer outputs kept in LDS, the loss gradient, and the input gradients backward
-// through every layer, reading the filters through the caches. Layer outputs, input gradients
+// through every layer, reading the filters through the caches (tiny_net_step_kernel). Where the batch
+// leaves compute units for it, the ends of that chain run a channel a workgroup, in a launch in front
+// and one behind (tiny_net_front_kernel, tiny_net_back_kernel). Layer outputs, input gradients
 // and max-pool records are also written to the net's tensors in memory, so a caller sees what
 // the layer-by-layer path leaves. Nothing in that chain waits for a weight gradient, so those
-// are a second launch of many small workgroups, (piece of a layer's work) x (sample), that read
-// the layer's input and output gradient back from memory. What adds over the batch leaves that
-// kernel as one slice per sample ([sample][tensor], the layout of the reference's own
-// per-sample gradients, tiny_dnn/layers/layer.h:699-718). When the step ends with an update,
-// the optimizer's kernel adds the slices up on its way (the split sums it also takes from the
+// are a launch behind it, (piece of a layer's parameters) x (group of samples), that reads
+// the layer's input and output gradient back from memory (tiny_net_param_kernel). A batch of one
+// group is updated there; what larger ones leave as one slice per group ([group][tensor]) the
+// optimizer's kernel adds up on its way (the split sums it also takes from the
 // layer-by-layer step); a step that stops at the gradients adds them to the gradient tensors in
-// sample order, the order of edge::merge_grads (tiny_dnn/node.h:89-103), with a kernel of its own.
+// order, as edge::merge_grads does (tiny_dnn/node.h:89-103), with a kernel of its own.
 //
 // The arithmetic of each layer follows the reference's scalar kernels: convolution sums the
 // taps of one input channel, then adds channel sums in channel order, then the bias
@@ -22,8 +23,11 @@
 // gradient, a first layer's weight gradient, a fully-connected output) are split over a group
 // of neighbouring lanes and added with butterfly shuffles, a fixed tree.
 // Built with -ffp-contract=off like the other scalar kernels.
+#include <algorithm>
 #include <cfloat>
+#include <type_traits>
 
+#include "opt_update.h"
 #include "tiny_net.h"
 
 namespace tdh {
@@ -57,6 +61,20 @@ __device__ __forceinline__ float tn_act_bwd(int act, float p0, float y, float dy
 __device__ __forceinline__ float group_sum(float v, int group) {
   for (int off = group >> 1; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;
+}
+// sum over a wave, in lane 63, without LDS: rows of sixteen lanes, then the rows in order
+__device__ __forceinline__ float wave_sum_63(float v) {
+  auto step = [](float x, auto ctrl, auto rows) {
+    return x + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), ctrl(), rows(), 0xf, false));
+  };
+  using std::integral_constant;
+  constexpr integral_constant<int, 0xf> all;
+  v = step(v, integral_constant<int, 0x111>(), all);   // row_shr:1
+  v = step(v, integral_constant<int, 0x112>(), all);
+  v = step(v, integral_constant<int, 0x114>(), all);
+  v = step(v, integral_constant<int, 0x118>(), all);
+  v = step(v, integral_constant<int, 0x142>(), integral_constant<int, 0xa>());   // row_bcast:15
+  return step(v, integral_constant<int, 0x143>(), integral_constant<int, 0xc>());   // row_bcast:31
 }
 // lanes per value, so that `values` of them make at least two rounds of the workgroup busy
 // and no lane's share of `length` terms is empty
@@ -306,21 +324,6 @@ TN_INLINE void fc_bwd_dx(const TinyLayer *__restrict__ Lp, const float *dy, floa
     if (gdx) gdx[c] = acc;
   }
 }
-// dW[c][i] = in[c] * dy[i] for the elements [base, base + count), db = dy with base 0
-template <int NT>
-TN_INLINE void fc_bwd_param(const TinyLayer *__restrict__ Lp, const float *in, const float *dy,
-                            float *__restrict__ gw, float *__restrict__ gb, const int base, const int count) {
-  const int nb = Lp->nb;
-  const FastDiv d_out = Lp->d_out;
-  for (int e = base + threadIdx.x; e < base + count; e += NT) {
-    uint32_t c, i;
-    d_out.divmod(e, c, i);
-    gw[e] = in[c] * dy[i];
-  }
-  if (base == 0)
-    for (int i = threadIdx.x; i < nb; i += NT) gb[i] = dy[i];
-}
-
 // maxpool_op_internal.h:42-57: an input takes the gradient of the LAST window that contains it
 // when that window's record names it
 TN_INLINE void maxpool_bwd(const TinyLayer *__restrict__ Lp, const float *dy, const int32_t *gargmax, float *dx,
@@ -367,39 +370,6 @@ TN_INLINE void avepool_bwd_dx(const TinyLayer *__restrict__ Lp, const float *dy,
     if (gdx) gdx[e] = v;
   }
 }
-template <int NT>
-TN_INLINE void avepool_bwd_param(const TinyLayer *__restrict__ Lp, const float *in, const float *dy,
-                                 float *__restrict__ gw, float *__restrict__ gb) {
-  const int C = Lp->C, H = Lp->H, W = Lp->W, OH = Lp->OH, OW = Lp->OW, R = Lp->R, S = Lp->S, sh = Lp->sh, sw = Lp->sw;
-  const FastDiv d_ow = Lp->d_ow;
-  const float scale = Lp->scale;
-  const int oplane = OH * OW;
-  int g = 64;
-  while (g > 1 && (C * g > NT || g > oplane)) g >>= 1;
-  const int items = C * g, gs = __ffs(g) - 1;
-  for (int base = 0; base < items; base += NT) {
-    const int it = base + threadIdx.x, c = it >> gs, part = it & (g - 1);
-    float sw_ = 0.0f, sb = 0.0f;
-    if (it < items)
-      for (int o = part; o < oplane; o += g) {
-        uint32_t oy, ox;
-        d_ow.divmod(o, oy, ox);
-        const int x0 = ox * sw, y0 = oy * sh;
-        const float dv = dy[c * oplane + o];
-        sb += dv;
-        if (x0 + S <= W && y0 + R <= H)
-          for (int wy = 0; wy < R; ++wy)
-            for (int wx = 0; wx < S; ++wx) sw_ += in[(c * H + y0 + wy) * W + x0 + wx] * dv;
-      }
-    sw_ = group_sum(sw_, g);
-    sb  = group_sum(sb, g);
-    if (it < items && part == 0) {
-      gw[c] = sw_ * scale;
-      gb[c] = sb;
-    }
-  }
-}
-
 TN_INLINE void act_bwd(const TinyLayer *__restrict__ Lp, const float *y, const float *dy, float *dx,
                        float *__restrict__ gdx) {
   const int n = Lp->out_size, act = Lp->act;
@@ -434,25 +404,6 @@ TN_INLINE void stage_framed_dy(const TinyLayer *__restrict__ Lp, const Src *dy, 
     const float v = dy[in ? (co * OH + oy) * OW + ox : 0];
     framed[e] = in ? v : 0.0f;
   }
-}
-// the rows [py_lo, py_hi] of the copy only (a workgroup that computes a few rows of dX)
-template <int NT, typename Src>
-TN_INLINE void stage_framed_rows(const TinyLayer *__restrict__ Lp, const Src *dy, float *framed, const int py_lo,
-                                 const int py_hi) {
-  const int K = Lp->K, H = Lp->H, W = Lp->W, OH = Lp->OH, OW = Lp->OW, R = Lp->R, S = Lp->S;
-  const int PW = W + S - 1, PP = (H + R - 1) * PW, oy0 = R - 1 - Lp->ph, ox0 = S - 1 - Lp->pw;
-  const FastDiv d_pw = Lp->d_pw;
-  const int cells = (py_hi - py_lo + 1) * PW;
-  for (int co = 0; co < K; ++co)
-    for (int idx = threadIdx.x; idx < cells; idx += NT) {
-      uint32_t q, px;
-      d_pw.divmod(idx, q, px);
-      const int py = py_lo + static_cast<int>(q);
-      const int oy = py - oy0, ox = static_cast<int>(px) - ox0;
-      const bool in = static_cast<unsigned>(oy) < static_cast<unsigned>(OH) && static_cast<unsigned>(ox) < static_cast<unsigned>(OW);
-      const float v = dy[in ? (co * OH + oy) * OW + ox : 0];
-      framed[co * PP + py * PW + static_cast<int>(px)] = in ? v : 0.0f;
-    }
 }
 __host__ __device__ inline int conv_framed_floats(const TinyLayer &L) {
   return L.K * (L.H + L.R - 1) * (L.W + L.S - 1);
@@ -1067,111 +1018,6 @@ TN_INLINE void conv_bwd_dx_matvec(const TinyLayer *__restrict__ Lp, const float 
   }
 }
 
-// lanes that share one weight's sum over output rows in the parameter-gradient kernel
-__host__ __device__ inline int conv_param_group(const TinyLayer &L) {
-  int g = 32;
-  while (g > 1 && (32 * g > L.OH * L.OW || g > L.OH)) g >>= 1;   // 32 output pixels or more per lane
-  return g;
-}
-// this sample's dW and db of a convolution (conv2d_op_internal.h:130-179): a group of lanes per
-// weight; the lanes of a group take output rows in turn, a lane walks the pixels of its rows
-// whose window element lies inside the input, and the group adds up with butterfly shuffles.
-// (Lanes that take pixels in turn instead, neighbouring lanes on neighbouring words, run into no
-// bank conflicts but pay more for the bookkeeping per pixel: 13.1 against 10.4 us for LeNet-5.)
-// Units [base, base + count) of nw * group (weights x lanes); the bias gradient goes with base 0.
-template <int NT>
-TN_INLINE void conv_bwd_param_rows(const TinyLayer *__restrict__ Lp, const float *in, const float *dy,
-                                   float *__restrict__ gw, const int base0, const int count) {
-  const int H = Lp->H, W = Lp->W, K = Lp->K, OH = Lp->OH, OW = Lp->OW;
-  const int sh = Lp->sh, sw = Lp->sw, ph = Lp->ph, pw = Lp->pw;
-  const FastDiv d_taps = Lp->d_taps, d_s = Lp->d_s, d_c = Lp->d_c;
-  const uint8_t *__restrict__ tbl = Lp->tbl;
-  const int plane = OH * OW;
-  const bool unit = sh == 1 && sw == 1;
-  {
-    const int g = conv_param_group(*Lp), gs = __ffs(g) - 1, end = base0 + count;
-    for (int base = base0; base < end; base += NT) {
-      const int it = base + threadIdx.x, idx = it >> gs, part = it & (g - 1);
-      float sum = 0.0f;
-      if (it < end) {
-        uint32_t pair, tap, co, ci, wy, wx;
-        d_taps.divmod(idx, pair, tap);
-        d_c.divmod(pair, co, ci);
-        d_s.divmod(tap, wy, wx);
-        if (!tbl || tbl[ci * K + co]) {
-          // iy = oy*sh + wy - ph in [0, H), ix = ox*sw + wx - pw in [0, W)
-          const int yoff = static_cast<int>(wy) - ph, xoff = static_cast<int>(wx) - pw;
-          int oy_lo, oy_hi, ox_lo, ox_hi;
-          if (unit) {
-            oy_lo = max(0, -yoff); oy_hi = min(OH, H - yoff);
-            ox_lo = max(0, -xoff); ox_hi = min(OW, W - xoff);
-          } else {
-            oy_lo = yoff >= 0 ? 0 : (-yoff + sh - 1) / sh; oy_hi = min(OH, (H - 1 - yoff) / sh + 1);
-            ox_lo = xoff >= 0 ? 0 : (-xoff + sw - 1) / sw; ox_hi = min(OW, (W - 1 - xoff) / sw + 1);
-          }
-          const float *ip = in + ci * H * W + yoff * W + xoff;
-          const float *dp = dy + co * plane;
-          for (int oy = oy_lo + part; oy < oy_hi; oy += g) {
-            const float *ir = ip + oy * sh * W;
-            const float *dr = dp + oy * OW;
-            int ox = ox_lo;
-            if (unit) {
-              for (; ox + 4 <= ox_hi; ox += 4)
-                sum += ir[ox] * dr[ox] + ir[ox + 1] * dr[ox + 1] + ir[ox + 2] * dr[ox + 2] + ir[ox + 3] * dr[ox + 3];
-              for (; ox < ox_hi; ++ox) sum += ir[ox] * dr[ox];
-            } else {
-              for (; ox + 4 <= ox_hi; ox += 4)
-                sum += ir[ox * sw] * dr[ox] + ir[(ox + 1) * sw] * dr[ox + 1] + ir[(ox + 2) * sw] * dr[ox + 2] +
-                       ir[(ox + 3) * sw] * dr[ox + 3];
-              for (; ox < ox_hi; ++ox) sum += ir[ox * sw] * dr[ox];
-            }
-          }
-        }
-      }
-      sum = group_sum(sum, g);
-      if (it < end && part == 0) gw[idx] = sum;
-    }
-  }
-}
-// the bias gradient of such a convolution, a job of its own (beside the first units of the weight
-// gradient it made that workgroup the last of the launch to finish): every plane of dY, a group
-// of lanes a channel
-template <int NT>
-TN_INLINE void conv_bwd_param_bias(const TinyLayer *__restrict__ Lp, const float *dy, float *__restrict__ gb) {
-  const int nb = Lp->nb, plane = Lp->OH * Lp->OW;
-  {
-    int g = 64;
-    while (g > 1 && (nb * g > 2 * NT || g > plane)) g >>= 1;
-    const int total = nb * g, gs = __ffs(g) - 1;
-    for (int base = 0; base < total; base += NT) {
-      const int it = base + threadIdx.x, co = it >> gs, part = it & (g - 1);
-      float sum = 0.0f;
-      if (it < total)
-        for (int p = part; p < plane; p += g) sum += dy[co * plane + p];
-      sum = group_sum(sum, g);
-      if (it < total && part == 0) gb[co] = sum;
-    }
-  }
-}
-// the same for a convolution that is a matrix-vector product: dW[co][k] = in[k] * dY[co] for
-// the elements [base, base + count)
-template <int NT>
-TN_INLINE void conv_bwd_param_matvec(const TinyLayer *__restrict__ Lp, const float *in, const float *dy,
-                                     float *__restrict__ gw, float *__restrict__ gb, const int base, const int count) {
-  const int K = Lp->K, nb = Lp->nb;
-  const FastDiv d_taps = Lp->d_taps, d_nk = Lp->d_nk;
-  const uint8_t *__restrict__ tbl = Lp->tbl;
-  for (int e = base + threadIdx.x; e < base + count; e += NT) {
-    uint32_t co, k;
-    d_nk.divmod(e, co, k);
-    float v = in[k] * dy[co];
-    if (tbl && !tbl[d_taps.div(k) * K + co]) v = 0.0f;
-    gw[e] = v;
-  }
-  if (base == 0)
-    for (int co = threadIdx.x; co < nb; co += NT) gb[co] = dy[co];
-}
-
 // One workgroup per sample, from layer m on (0, or the plan's split). LDS: its input, every layer's output, two gradient
 // buffers, the staging area.
 __global__ void __launch_bounds__(TN_THREADS)
@@ -1309,6 +1155,9 @@ tiny_net_step_kernel(const TinyPlan *__restrict__ plan, const int m, const int l
     ga = gb;
     gb = sw;
   }
+  // (the launch that updates the first layer's filters also reads them, for the input gradient)
+  if (s == 0 && plan->first_dx_as_job)
+    for (int i = threadIdx.x; i < plan->l[0].nw; i += TN_THREADS) plan->first_w[i] = plan->l[0].w[i];
 }
 
 // ------------------------------------------------------------- the two ends of the chain, spread out
@@ -1322,6 +1171,7 @@ tiny_net_step_kernel(const TinyPlan *__restrict__ plan, const int m, const int l
 // LeNet-5, batch 16, us: one launch 40.1; here 4.5 + 21.8 + 7.8 (which batches: launch_tiny_step).
 constexpr int TF_THREADS = 1024;   // front, at most
 constexpr int TB_THREADS = 1024;   // back
+static_assert(TB_THREADS / 64 == 16, "sixteen shares of a pool's sums; a wave left over from five rows of three and from three of five");
 
 // the sums of channel co, a lane a pixel, filters as scalar operands (as conv_fwd_scalar adds them up)
 template <int R, int S, bool PAD>
@@ -1440,6 +1290,21 @@ tiny_net_front_kernel(const TinyPlan *__restrict__ plan, const int m, const int 
   }
 }
 
+// LDS words of 16 bytes: what a lane reads of a row starts on one (a stride of four floats from lane to lane would
+// put a wave's 4-byte reads on a quarter of the banks)
+__host__ __device__ inline int quad_pitch(const int columns) { return (columns + 3) & ~3; }
+template <int N>
+TN_INLINE void read_row(float (&v)[N], const float *row) {
+  const float4 *r = reinterpret_cast<const float4 *>(row);
+#pragma unroll
+  for (int k = 0; k < (N + 3) / 4; ++k) {
+    const float4 w = r[k];
+    v[4 * k] = w.x;
+    if (4 * k + 1 < N) v[4 * k + 1 < N ? 4 * k + 1 : 0] = w.y;
+    if (4 * k + 2 < N) v[4 * k + 2 < N ? 4 * k + 2 : 0] = w.z;
+    if (4 * k + 3 < N) v[4 * k + 3 < N ? 4 * k + 3 : 0] = w.w;
+  }
+}
 // dX of the second convolution for channel ci, [H][W], from the zero-framed dY. A lane takes four
 // neighbouring pixels of a row, whose taps share eight values of a framed row; the waves are chunks of
 // 64 such units x `parts` ranges of output channels, whose sums meet in `scratch` ([part][chunk][4][64]).
@@ -1462,13 +1327,12 @@ TN_INLINE void conv_back_dx(const TinyLayer *__restrict__ Lp, const BackSplit b,
   const int C = Lp->C, H = Lp->H, W = Lp->W;
   const float *__restrict__ w = Lp->w;
   constexpr int taps = R * S;
-  const int PW = W + S - 1, PP = (H + R - 1) * PW, lane = threadIdx.x & 63, units = H * b.units_w;
+  const int PW = quad_pitch(W + S - 1), PP = (H + R - 1) * PW, lane = threadIdx.x & 63, units = H * b.units_w;
   const int step = b.parts > 1 ? b.chunks : TB_THREADS / 64;
   if (kp < b.parts)
     for (int chunk = wave_index() - kp * step; chunk < b.chunks; chunk += step) {   // (one trip where parts > 1)
       const int unit = min((chunk << 6) + lane, units - 1);
       const int iy = unit / b.units_w, ix = (unit - iy * b.units_w) << 2;
-      // (a row's last unit may reach up to three values past the row: of the next row, or of `scratch`)
       const float *dp = framed + c_lo * PP + iy * PW + ix;
       float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
       for (int co = c_lo; co < c_hi; ++co, dp += PP) {
@@ -1478,8 +1342,7 @@ TN_INLINE void conv_back_dx(const TinyLayer *__restrict__ Lp, const BackSplit b,
 #pragma unroll
         for (int wy = 0; wy < R; ++wy) {
           float v[S + 3];
-#pragma unroll
-          for (int k = 0; k < S + 3; ++k) v[k] = dp[(R - 1 - wy) * PW + k];
+          read_row(v, dp + (R - 1 - wy) * PW);
 #pragma unroll
           for (int wx = 0; wx < S; ++wx)
 #pragma unroll
@@ -1505,10 +1368,98 @@ TN_INLINE void conv_back_dx(const TinyLayer *__restrict__ Lp, const BackSplit b,
   }
 }
 
-// (everything from memory is asked for first: the gradient, the filters' cache lines, the table, and
-// the outputs of the activations on the way)
+// Four neighbouring output pixels of a unit-stride convolution, from the four gradients d: acc[wy][wx] += d * X.
+// xr: X's row under filter row 0, at the first pixel's column with the padding in front (rows of xp floats, a multiple of
+// four); iy0, ix0: that row and column of the image. Products that do not exist (past the row's end, or outside the
+// input) are left out, not multiplied by zero: an infinity stays out of sums that it is no part of.
+template <int ROWS, int S, bool PAD>
+TN_INLINE void dw_quad(float (&acc)[ROWS][S], const float *xr, const int xp, const float (&d)[4], const int iy0, const int ix0,
+                       const int H, const int W, const int left) {
+  float v[ROWS][S + 3];
+#pragma unroll
+  for (int wy = 0; wy < ROWS; ++wy) {
+    const bool row = !PAD || static_cast<unsigned>(iy0 + wy) < static_cast<unsigned>(H);
+    read_row(v[wy], xr + (row ? wy * xp : -iy0 * xp));
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (k < left) {
+#pragma unroll
+      for (int wy = 0; wy < ROWS; ++wy) {
+        const bool row = !PAD || static_cast<unsigned>(iy0 + wy) < static_cast<unsigned>(H);
+#pragma unroll
+        for (int wx = 0; wx < S; ++wx) {
+          const float sum = __builtin_fmaf(d[k], v[wy][k + wx], acc[wy][wx]);
+          const bool in   = !PAD || (row && static_cast<unsigned>(ix0 + k + wx) < static_cast<unsigned>(W));
+          acc[wy][wx] = in ? sum : acc[wy][wx];
+        }
+      }
+    }
+}
+// floats of a staged row of X for it
+__host__ __device__ inline int dw_x_pitch(const TinyLayer *__restrict__ L) {
+  return quad_pitch(max(L->W + L->pw, quad_pitch(L->OW) + L->S - 1));
+}
+
+// This sample's part of a first convolution's dW and db, output channel co: a lane adds up the taps of four pixels of a
+// filter row at a time (16 / R waves a row), waves and lanes meet in `red` ((S + 1) floats a wave)
+template <int R, int S, bool PAD>
+TN_INLINE void conv_back_param(const TinyLayer *__restrict__ L, const float *x, const float *dy, const int s, const int co,
+                               float *red) {
+  constexpr int WAVES = TB_THREADS / 64, PER_ROW = WAVES / R, taps = R * S;
+  const int C = L->C, H = L->H, W = L->W, OH = L->OH, OW = L->OW, quads = (OW + 3) >> 2, units = OH * quads;
+  const int xp = dw_x_pitch(L), ph = L->ph, pw0 = L->pw;
+  const FastDiv d_quads = L->d_quads;
+  const int wave = wave_index(), wy = wave / PER_ROW, sub = wave - wy * PER_ROW, lane = threadIdx.x & 63;
+  float *pw = L->pw_part + static_cast<size_t>(s) * L->nw + static_cast<size_t>(co) * C * taps;
+  for (int ci = 0; ci < C; ++ci) {
+    float acc[1][S], db = 0.0f;
+#pragma unroll
+    for (int wx = 0; wx < S; ++wx) acc[0][wx] = 0.0f;
+    if (wy < R)
+      for (int i = sub * 64 + lane; i < units; i += 64 * PER_ROW) {
+        uint32_t oy, q;
+        d_quads.divmod(i, oy, q);
+        const int left  = OW - 4 * static_cast<int>(q), iy = static_cast<int>(oy) - ph + wy;
+        const float *dr = dy + oy * OW + 4 * q;
+        float d[4];
+        if ((OW & 3) == 0) {
+          read_row(d, dr);
+        } else {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) d[k] = dr[k < left ? k : 0];
+        }
+        dw_quad<1, S, PAD>(acc, x + (ci * H + iy) * xp + 4 * q, xp, d, iy, 4 * static_cast<int>(q) - pw0, H, W, left);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) db += k < left ? d[k] : 0.0f;
+      }
+#pragma unroll
+    for (int wx = 0; wx < S; ++wx) acc[0][wx] = wave_sum_63(acc[0][wx]);
+    db = wave_sum_63(db);
+    if (lane == 63) {
+#pragma unroll
+      for (int wx = 0; wx < S; ++wx) red[wave * (S + 1) + wx] = acc[0][wx];
+      red[wave * (S + 1) + S] = db;
+    }
+    lds_barrier();
+    // thread: filter row tid / (S + 1), column tid % (S + 1); of the last column, the bias gradient, row 0 alone
+    const int row = threadIdx.x / (S + 1), col = threadIdx.x - row * (S + 1);
+    if (row < R) {
+      float v = 0.0f;
+#pragma unroll
+      for (int k = 0; k < PER_ROW; ++k) v += red[(row * PER_ROW + k) * (S + 1) + col];
+      const bool on = !L->tbl || L->tbl[ci * L->K + co];
+      if (col < S) pw[ci * taps + row * S + col] = on ? v : 0.0f;
+      else if (row == 0 && ci == 0 && L->nb) L->pb_part[static_cast<size_t>(s) * L->nb + co] = v;
+    }
+    lds_barrier();
+  }
+}
+
+// (everything from memory is asked for first: the gradient, the filters' cache lines, the table, the
+// outputs of the layers on the way, and the sample)
 __global__ void __launch_bounds__(TB_THREADS)
-tiny_net_back_kernel(const TinyPlan *__restrict__ plan, const int m) {
+tiny_net_back_kernel(const TinyPlan *__restrict__ plan, const int m, const float *__restrict__ x) {
   extern __shared__ float lds[];
   constexpr int AHEAD = 4;   // gradients a thread holds, and layers whose outputs it does
   const int s = blockIdx.x, ci = blockIdx.y, n = plan->n, tid = threadIdx.x;
@@ -1522,16 +1473,21 @@ tiny_net_back_kernel(const TinyPlan *__restrict__ plan, const int m) {
   const BackSplit b = back_split(H, W, K);
   const int kp = b.parts > 1 ? wave_index() / b.chunks : 0;
   const int c_lo = min(K, kp * b.per_part), c_hi = kp < b.parts ? min(K, c_lo + b.per_part) : c_lo;
-  float y[AHEAD];
+  // y[j]: this channel of the output of layer m - 1 - j
+  float y[AHEAD], xv[AHEAD];
   int p_li = plane;
 #pragma unroll
   for (int j = 0; j < AHEAD; ++j) {
     y[j] = 0.0f;
     const TinyLayer *__restrict__ A = &plan->l[max(m - 1 - j, 0)];
-    if (m - 1 - j < 1) continue;
-    if (A->kind == TDH_L_ACT) y[j] = A->out[static_cast<size_t>(s) * A->out_size + ci * p_li + min(tid, p_li - 1)];
-    else p_li = A->H * A->W;
+    if (m - 1 - j < 0) continue;
+    y[j] = A->out[static_cast<size_t>(s) * A->out_size + ci * p_li + min(tid, p_li - 1)];
+    if (A->kind != TDH_L_ACT) p_li = A->H * A->W;
   }
+  const int in_size = plan->in_size;
+  x += static_cast<size_t>(s) * in_size;
+#pragma unroll
+  for (int j = 0; j < AHEAD; ++j) xv[j] = x[min(tid + TB_THREADS * j, in_size - 1)];
   uint64_t connected = ~0ull;
   if (L->tbl) connected = __ballot((tid & 63) < c_hi - c_lo && L->tbl[ci * K + min(c_lo + (tid & 63), K - 1)] != 0);
   int touch = 0;
@@ -1540,10 +1496,11 @@ tiny_net_back_kernel(const TinyPlan *__restrict__ plan, const int m) {
     const ScalarInts line = (ScalarInts)(L->w + static_cast<size_t>(co * L->C + ci) * taps);
     touch |= line[0] | line[taps - 1];
   }
-  float *framed = lds, *scratch = lds + plan->back_scratch, *cur = lds + plan->back_planes;
+  float *framed = lds, *scratch = lds + plan->back_scratch, *cur = lds + plan->back_planes, *sample = lds + plan->back_sample;
+  float *pool_sums = sample + plan->back_sample_floats;
   float *gdx = L->dx + static_cast<size_t>(s) * L->in_size + ci * plane;
   // dY into its frame of zeros
-  const int PW = W + S - 1, PP = (H + R - 1) * PW, corner = (R - 1 - L->ph) * PW + S - 1 - L->pw;
+  const int PW = quad_pitch(W + S - 1), PP = (H + R - 1) * PW, corner = (R - 1 - L->ph) * PW + S - 1 - L->pw;
   const FastDiv d_oplane = L->d_oplane, d_ow = L->d_ow;
   for (int i = tid; i < K * PP; i += TB_THREADS) framed[i] = 0.0f;
   asm volatile("" ::"s"(touch));
@@ -1558,6 +1515,18 @@ tiny_net_back_kernel(const TinyPlan *__restrict__ plan, const int m) {
   for (int j = 0; j < AHEAD; ++j)
     if (tid + TB_THREADS * j < out_size) place(tid + TB_THREADS * j, dy[j]);
   for (int e = tid + TB_THREADS * AHEAD; e < out_size; e += TB_THREADS) place(e, gdy[e]);
+  const TinyLayer *__restrict__ F = &plan->l[0];
+  const FastDiv d_w0 = F->d_w;
+  const int xp = dw_x_pitch(F), pw0 = F->pw;
+  auto put = [&](int e, float v) {
+    uint32_t row, col;
+    d_w0.divmod(e, row, col);
+    sample[row * xp + col + pw0] = v;
+  };
+#pragma unroll
+  for (int j = 0; j < AHEAD; ++j)
+    if (tid + TB_THREADS * j < in_size) put(tid + TB_THREADS * j, xv[j]);
+  for (int e = tid + TB_THREADS * AHEAD; e < in_size; e += TB_THREADS) put(e, x[e]);
   lds_barrier();
   if (R == 5) conv_back_dx<5, 5>(L, b, framed, cur, gdx, scratch, ci, kp, c_lo, c_hi, connected);
   else conv_back_dx<3, 3>(L, b, framed, cur, gdx, scratch, ci, kp, c_lo, c_hi, connected);
@@ -1583,7 +1552,12 @@ tiny_net_back_kernel(const TinyPlan *__restrict__ plan, const int m) {
     const FastDiv d_w = L->d_w;
     const int32_t *argmax = most ? L->argmax + static_cast<size_t>(s) * L->out_size + ci * plane : nullptr;
     const float weight = most ? 0.0f : L->w[ci] * L->scale;
-    float *nxt = cur + plane, *g = L->dx + static_cast<size_t>(s) * L->in_size + ci * iplane;
+    float *nxt = cur + quad_pitch(plane), *g = L->dx + static_cast<size_t>(s) * L->in_size + ci * iplane;
+    const int j_in = m - li;
+    const float *in = plan->l[li - 1].out + static_cast<size_t>(s) * L->in_size + ci * iplane;
+    const float first = j_in == 1 ? y[1] : j_in == 2 ? y[2] : y[3];
+    float pw = 0.0f, pb = 0.0f;   // an average pool's own gradients
+    for (int o = tid; o < plane && !most; o += TB_THREADS) pb += cur[o];
     for (int e = tid; e < iplane; e += TB_THREADS) {
       uint32_t yy, xx;
       d_w.divmod(e, yy, xx);
@@ -1596,89 +1570,577 @@ tiny_net_back_kernel(const TinyPlan *__restrict__ plan, const int m) {
         v = covered && argmax[outi] == ci * iplane + e ? cur[outi] : 0.0f;
       } else {      // avepool_bwd_dx
         const int ox = two ? ix >> 1 : ix < S ? 0 : (ix - S + sw) / sw, oy = two ? iy >> 1 : iy < R ? 0 : (iy - R + sh) / sh;
-        v = weight * cur[oy * OW + ox];
+        const float d = cur[oy * OW + ox];
+        v = weight * d;
+        pw = __builtin_fmaf(e == tid && j_in < AHEAD ? first : in[e], d, pw);
       }
       nxt[e] = v;
       g[e]   = v;
     }
+    if (!most) {   // (a wave's share; they are added up behind the last layer)
+      pw = wave_sum_63(pw);
+      pb = wave_sum_63(pb);
+      if ((tid & 63) == 63) {
+        pool_sums[32 * li + (tid >> 6)]      = pw;
+        pool_sums[32 * li + 16 + (tid >> 6)] = pb;
+      }
+    }
     cur   = nxt;
     plane = iplane;
   }
-}
-
-// The parameter gradients of one sample, a job per workgroup: the layer's input and the gradient
-// of its output come back from memory into LDS (the step kernel wrote both), then the job's
-// units run as they would in one workgroup.
-constexpr int TP_THREADS = 256;
-__global__ void __launch_bounds__(TP_THREADS)
-tiny_net_param_kernel(const TinyPlan *__restrict__ plan, const float *__restrict__ x) {
-  extern __shared__ float lds[];
-  const TinyJob job = plan->jobs[blockIdx.y];
-  const int s = blockIdx.x, n = plan->n, li = job.layer;
-  const TinyLayer *__restrict__ L = &plan->l[li];
-  const int in_sz = L->in_size, out_sz = L->out_size, kind = L->kind;
-  const float *gin = (li == 0 ? x : plan->l[li - 1].out) + static_cast<size_t>(s) * in_sz;
-  const float *gdy = (li == n - 1 ? plan->dloss : plan->l[li + 1].dx) + static_cast<size_t>(s) * out_sz;
-  if (job.what == 1) {   // the first layer's dX from a framed dY: dY goes from memory straight into its frame
-    float *framed = lds;
-    float *gdx = L->dx + static_cast<size_t>(s) * in_sz;
-    // the rows of the frame that this job's pixels read: its items are chunks of 64 pixels of
-    // one block of channels, or else everything
-    const int plane = L->H * L->W, chunks = (plane + 63) >> 6, last = job.base + job.count - 1;
-    int py_lo = 0, py_hi = L->H + L->R - 2;
-    if (job.base / chunks == last / chunks) {
-      const int p_lo = (job.base % chunks) << 6, p_hi = min(plane - 1, ((last % chunks) << 6) + 63);
-      py_lo = static_cast<int>(L->d_w.div(p_lo));
-      py_hi = static_cast<int>(L->d_w.div(p_hi)) + L->R - 1;
-    }
-    stage_framed_rows<TP_THREADS>(L, gdy, framed, py_lo, py_hi);
-    lds_barrier();
-    if (L->R == 5) conv_bwd_dx_scalar_any<5, 5, TP_THREADS>(L, framed, nullptr, gdx, nullptr, job.base, job.base + job.count, 1);
-    else conv_bwd_dx_scalar_any<3, 3, TP_THREADS>(L, framed, nullptr, gdx, nullptr, job.base, job.base + job.count, 1);
-    return;
-  }
-  if (job.what == 2) {   // a convolution's bias gradient: dY alone
-    fill_lds<TP_THREADS>(lds, gdy, out_sz);
-    lds_barrier();
-    conv_bwd_param_bias<TP_THREADS>(L, lds, L->gb + static_cast<size_t>(s) * L->nb);
-    return;
-  }
-  float *in = lds, *dy = lds + ((in_sz + 3) & ~3);
-  fill_lds<TP_THREADS>(in, gin, in_sz);
-  // (a convolution's weight-gradient units name the output channels whose gradient planes they read)
-  int dy_lo = 0, dy_n = out_sz;
-  if (kind == TDH_L_CONV && !conv_is_matvec(*L)) {
-    const int gs = __ffs(conv_param_group(*L)) - 1, plane = L->OH * L->OW;
-    const int co_lo = static_cast<int>(L->d_nk.div(job.base >> gs));
-    const int co_hi = static_cast<int>(L->d_nk.div((job.base + job.count - 1) >> gs));
-    dy_lo = co_lo * plane;
-    dy_n  = (co_hi - co_lo + 1) * plane;
-  }
-  fill_lds<TP_THREADS>(dy + dy_lo, gdy + dy_lo, dy_n);
   lds_barrier();
-  float *gw = L->gw + static_cast<size_t>(s) * L->nw;
-  float *gb = L->gb ? L->gb + static_cast<size_t>(s) * L->nb : nullptr;
-  switch (kind) {
-    case TDH_L_CONV:
-      if (conv_is_matvec(*L)) conv_bwd_param_matvec<TP_THREADS>(L, in, dy, gw, gb, job.base, job.count);
-      else conv_bwd_param_rows<TP_THREADS>(L, in, dy, gw, job.base, job.count);
-      break;
-    case TDH_L_FC: fc_bwd_param<TP_THREADS>(L, in, dy, gw, gb, job.base, job.count); break;
-    case TDH_L_AVEPOOL: avepool_bwd_param<TP_THREADS>(L, in, dy, gw, gb); break;
-    default: break;
+  if (tid >= TB_THREADS - 64)   // (the last wave has no filter row below)
+    for (int li = 1; li < m; ++li) {
+      L = &plan->l[li];
+      if (L->kind != TDH_L_AVEPOOL) continue;
+      const float sum = group_sum(pool_sums[32 * li + (tid & 31)], 16);
+      if ((tid & 63) == 0) L->pw_part[static_cast<size_t>(s) * L->nw + ci] = sum * L->scale;
+      if ((tid & 63) == 16) L->pb_part[static_cast<size_t>(s) * L->nb + ci] = sum;
+    }
+  L = &plan->l[0];
+  const bool pad = L->ph != 0 || L->pw != 0;
+  if (L->R == 5) pad ? conv_back_param<5, 5, true>(L, sample, cur, s, ci, scratch) : conv_back_param<5, 5, false>(L, sample, cur, s, ci, scratch);
+  else pad ? conv_back_param<3, 3, true>(L, sample, cur, s, ci, scratch) : conv_back_param<3, 3, false>(L, sample, cur, s, ci, scratch);
+}
+
+// ------------------------------------------------------------- the parameter gradients
+// One launch over the whole batch: a workgroup owns some of a layer's parameters and adds up their
+// gradients over all samples of its group (tiny_groups), from the layer inputs and output
+// gradients that the launches in front left in memory. A batch of one group updates its parameters right
+// there; the groups of a larger one leave a slice each ([group][tensor]) for the optimizer's kernel, or for
+// tiny_net_merge_kernel. Behind those workgroups come the ones of the first layer's input gradient, which
+// nothing waits for either. Bound: latency (kernel arguments, the layer's sizes, one trip for the operands, the sums).
+// us, a slice per sample and the optimizer's launch / here: LeNet-5, batch 16 9.2 + 5.0 / 7.8 (and 2 in the back kernel), 32
+// 14.6 + 7.3 / 11.1, 64 24.4 + 7.4 / 15.3 + 5.6, 120 40.0 + 12.9 / 25.9 + 6.8, 300 86.4 + 20.6 / 55.9 + 9.3.
+constexpr int TP_THREADS = 512, TP_WAVES = TP_THREADS / 64;
+enum { TP_CONV, TP_OUTER, TP_OUTER4, TP_COLUMNS, TP_POOL, TP_SLICES_W, TP_SLICES_B };   // what a range of workgroups does
+constexpr int TP_RANGES = 2 * TINY_MAX_LAYERS;
+struct TinyRanges {
+  int first[TP_RANGES];     // first workgroup; past the last range larger than any
+  int job[TP_RANGES];       // layer * 8 + TP_*
+  int per_group[TP_RANGES]; // workgroups per group of samples
+  int size[TP_RANGES];      // samples of a group
+};
+// What becomes of a finished gradient: KIND < 0: a slice; else that optimizer's update (elementwise.hip,
+// opt_multi_kernel). A kernel for each: with a choice at every update in one kernel, its code was 200 KB, and
+// a workgroup waited for instructions.
+struct TinyUpdate {
+  OptScalars p;
+  float b1_t, b2_t;
+  const float *powers_in;
+  float *powers_out;
+  int n_tensors;
+};
+struct TinyTarget {
+  float *g, *w, *s0, *s1, *slice;
+  OptScalars p;
+};
+struct TinyOld {
+  float g, w, s0, s1;
+};
+template <int KIND>
+TN_INLINE TinyTarget tn_target(const TinyUpdate &u, const TinyLayer *__restrict__ L, const bool bias, const int group) {
+  TinyTarget t;
+  if (KIND < 0) {
+    t.slice = bias ? L->gb + static_cast<size_t>(group) * L->nb : L->gw + static_cast<size_t>(group) * L->nw;
+    return t;
+  }
+  const TinyTensor &e = bias ? L->tb : L->tw;
+  t.g = e.g; t.w = e.w; t.s0 = e.s0; t.s1 = e.s1;
+  t.p = u.p;
+  if (opt_powers(KIND) == 0) return t;
+  // the reference multiplies b1_t by b1 after every update() call (optimizer.h:125-126)
+  float p1 = u.powers_in ? u.powers_in[0] : u.b1_t, p2 = u.powers_in ? u.powers_in[1] : u.b2_t;
+  for (int i = 0; i < e.index; ++i) {
+    p1 *= u.p.b1;
+    p2 *= u.p.b2;
+  }
+  t.p.omb1t     = 1.0f - p1;
+  t.p.omb2t     = 1.0f - p2;
+  t.p.adamax_lr = static_cast<double>(u.p.alpha) / (1.0 - static_cast<double>(p1));
+  return t;
+}
+// what the update of element e needs, asked for before the gradient is computed
+template <int KIND>
+TN_INLINE TinyOld tn_old(const TinyTarget &t, const int e, const bool on) {
+  TinyOld o = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (KIND < 0 || !on) return o;
+  o.g = t.g[e];
+  o.w = t.w[e];
+  if (opt_states(KIND) >= 1) o.s0 = t.s0[e];
+  if (opt_states(KIND) >= 2) o.s1 = t.s1[e];
+  return o;
+}
+template <int KIND>
+TN_INLINE void tn_finish(const TinyTarget &t, TinyOld o, const int e, const float value) {
+  if constexpr (KIND < 0) {
+    t.slice[e] = value;
+  } else {
+    opt_one<KIND>(value + o.g, o.w, o.s0, o.s1, t.p);   // (o.g: what passes without an update left there)
+    t.w[e] = o.w;
+    if (opt_states(KIND) >= 1) t.s0[e] = o.s0;
+    if (opt_states(KIND) >= 2) t.s1[e] = o.s1;
+    t.g[e] = 0.0f;
   }
 }
 
-// g[i] += slice[0][i] + slice[1][i] + ... in sample order (edge::merge_grads, node.h:89-103)
+// One plane of the layer's input and one of its output gradient, of ns samples, into LDS, all of a trip's
+// reads before its first store
+TN_INLINE void stage_planes(const TinyLayer *__restrict__ L, float *xl, const float *__restrict__ x, const int x_stride, float *dl,
+                            const float *__restrict__ d, const int d_stride, const int ns) {
+  const int x_plane = L->H * L->W, d_plane = L->OH * L->OW, nx = ns * x_plane, total = nx + ns * d_plane;
+  const FastDiv d_x = L->d_iplane, d_d = L->d_oplane;
+  const bool vec = ((x_plane | x_stride | d_plane | d_stride) & 3) == 0 &&
+                   ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(d)) & 15u) == 0;
+  auto from = [&](int e) {
+    const bool of_x  = e < nx;
+    const uint32_t i = of_x ? e : e - nx;
+    const uint32_t s = of_x ? d_x.div(i) : d_d.div(i);
+    return of_x ? x + static_cast<size_t>(s) * (x_stride - x_plane) + i : d + static_cast<size_t>(s) * (d_stride - d_plane) + i;
+  };
+  if (vec) {
+    constexpr int AHEAD = 4;
+    for (int base = 4 * threadIdx.x; base < total; base += 4 * AHEAD * TP_THREADS) {
+      float4 v[AHEAD];
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) v[j] = *reinterpret_cast<const float4 *>(from(min(base + 4 * j * TP_THREADS, total - 4)));
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) {
+        const int e = base + 4 * j * TP_THREADS;
+        if (e < total) *reinterpret_cast<float4 *>(e < nx ? xl + e : dl + e - nx) = v[j];
+      }
+    }
+  } else {
+    constexpr int AHEAD = 12;
+    for (int base = threadIdx.x; base < total; base += AHEAD * TP_THREADS) {
+      float v[AHEAD];
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) v[j] = *from(min(base + j * TP_THREADS, total - 1));
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) {
+        const int e = base + j * TP_THREADS;
+        if (e < total) *(e < nx ? xl + e : dl + e - nx) = v[j];
+      }
+    }
+  }
+}
+// sum over the workgroup, in every thread of its first wave; `red`: TP_WAVES floats of LDS that nobody else uses
+TN_INLINE float workgroup_sum(float v, float *red) {
+  v = wave_sum_63(v);
+  if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6] = v;
+  lds_barrier();
+  v = red[0];
+#pragma unroll
+  for (int k = 1; k < TP_WAVES; ++k) v += red[k];
+  return v;
+}
+
+// What the functions below need of a layer, asked for at once (left to their first uses, its scalar loads are four trips
+// to memory, one behind the other)
+TN_INLINE void at_hand(const TinyLayer *__restrict__ L) {
+  const FastDiv a = L->d_iplane, b = L->d_oplane, d = L->d_ow, e = L->d_vquads;
+  asm volatile("" ::"s"(L->C), "s"(L->H), "s"(L->W), "s"(L->K), "s"(L->OH), "s"(L->OW), "s"(L->ph), "s"(L->pw), "s"(L->nb), "s"(L->nw),
+               "s"(L->dw_chunk), "s"(L->tbl), "s"(L->gw), "s"(L->gb), "s"(L->tw.g), "s"(L->tw.w), "s"(L->tw.s0), "s"(L->tw.s1),
+               "s"(L->tw.index));
+  asm volatile("" ::"s"(L->tb.g), "s"(L->tb.w), "s"(L->tb.s0), "s"(L->tb.s1), "s"(L->tb.index), "s"(a.mul), "s"(a.shift), "s"(b.mul),
+               "s"(b.shift), "s"(d.mul), "s"(d.shift), "s"(d.d), "s"(e.mul), "s"(e.shift), "s"(e.d));
+}
+// dW of a channel pair (and, with the first input channel, the output channel's bias gradient), over the samples
+// [s_beg, s_end), `chunk` of them in LDS at a time. A thread adds up the taps of four output pixels below each other at
+// a time (neighbouring lanes read neighbouring columns, whatever the row's length); the waves' sums meet in LDS.
+template <int KIND, int R, int S, bool PAD>
+TN_INLINE void conv_param_pair(const TinyLayer *__restrict__ L, const float *__restrict__ gin, const int in_sz,
+                               const float *__restrict__ gdy, const int out_sz, const int s_beg, const int s_end,
+                               const int co, const int ci, const int group, const TinyUpdate &u, float *lds) {
+  constexpr int taps = R * S;
+  at_hand(L);
+  const bool connected = !L->tbl || L->tbl[ci * L->K + co];
+  const int tap = threadIdx.x, e = (co * L->C + ci) * taps + tap;
+  const bool mine = tap < taps, mine_b = tap == taps && ci == 0 && L->nb;
+  const TinyTarget tw = tn_target<KIND>(u, L, false, group), tb = tn_target<KIND>(u, L, true, group);
+  const TinyOld old_w = tn_old<KIND>(tw, e, mine), old_b = tn_old<KIND>(tb, co, mine_b);
+  const int H = L->H, W = L->W, OH = L->OH, OW = L->OW, plane = OH * OW, iplane = H * W, chunk = L->dw_chunk;
+  const int ph = L->ph, pw = L->pw, quads = (OH + 3) >> 2;
+  const FastDiv d_ow = L->d_ow, d_quads = L->d_vquads;
+  float acc[R][S], db = 0.0f;
+#pragma unroll
+  for (int wy = 0; wy < R; ++wy)
+#pragma unroll
+    for (int wx = 0; wx < S; ++wx) acc[wy][wx] = 0.0f;
+  float *xl = lds, *dl = lds + quad_pitch(chunk * iplane);
+  for (int s0 = s_beg; s0 < s_end; s0 += chunk) {
+    const int ns = min(chunk, s_end - s0);
+    if (s0 > s_beg) lds_barrier();
+    stage_planes(L, xl, gin + static_cast<size_t>(s0) * in_sz + ci * iplane, in_sz, dl,
+                 gdy + static_cast<size_t>(s0) * out_sz + co * plane, out_sz, ns);
+    lds_barrier();
+    const int units = ns * quads * OW;
+    for (int i = threadIdx.x; i < units; i += TP_THREADS) {
+      uint32_t line, ox, s, q;
+      d_ow.divmod(i, line, ox);
+      d_quads.divmod(line, s, q);
+      const int oy = 4 * static_cast<int>(q), left = OH - oy, iy0 = oy - ph, ix0 = static_cast<int>(ox) - pw;
+      const float *dr = dl + s * plane + oy * OW + ox, *xr = xl + s * iplane + iy0 * W + ix0;
+      float d[4], v[R + 3][S];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) d[k] = dr[k < left ? k * OW : 0];
+      // (rows behind the last one that a live pixel needs: some row that exists)
+#pragma unroll
+      for (int r = 0; r < R + 3; ++r) {
+        const bool row = PAD ? static_cast<unsigned>(iy0 + r) < static_cast<unsigned>(H) : r < left + R - 1;
+#pragma unroll
+        for (int wx = 0; wx < S; ++wx) {
+          const bool in = row && (!PAD || static_cast<unsigned>(ix0 + wx) < static_cast<unsigned>(W));
+          v[r][wx] = xr[in ? r * W + wx : -(iy0 * W + ix0)];
+        }
+      }
+      // Products that do not exist (past the last row, or outside the input) are left out, not multiplied by zero: an
+      // infinity stays out of sums that it is no part of.
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (k < left) {
+#pragma unroll
+          for (int wy = 0; wy < R; ++wy)
+#pragma unroll
+            for (int wx = 0; wx < S; ++wx) {
+              const float sum = __builtin_fmaf(d[k], v[k + wy][wx], acc[wy][wx]);
+              const bool in   = !PAD || (static_cast<unsigned>(iy0 + k + wy) < static_cast<unsigned>(H) &&
+                                       static_cast<unsigned>(ix0 + wx) < static_cast<unsigned>(W));
+              acc[wy][wx] = in ? sum : acc[wy][wx];
+            }
+          db += d[k];
+        }
+    }
+  }
+#pragma unroll
+  for (int wy = 0; wy < R; ++wy)
+#pragma unroll
+    for (int wx = 0; wx < S; ++wx) acc[wy][wx] = wave_sum_63(acc[wy][wx]);
+  db = wave_sum_63(db);
+  lds_barrier();
+  if ((threadIdx.x & 63) == 63) {
+    float *red = lds + wave_index() * (taps + 1);
+#pragma unroll
+    for (int wy = 0; wy < R; ++wy)
+#pragma unroll
+      for (int wx = 0; wx < S; ++wx) red[wy * S + wx] = acc[wy][wx];
+    red[taps] = db;
+  }
+  lds_barrier();
+  if (tap > taps) return;
+  float sum = lds[tap];
+#pragma unroll
+  for (int k = 1; k < TP_WAVES; ++k) sum += lds[k * (taps + 1) + tap];
+  if (mine) tn_finish<KIND>(tw, old_w, e, connected ? sum : 0.0f);
+  if (mine_b) tn_finish<KIND>(tb, old_b, co, sum);
+}
+// the same for any window and stride: a group of lanes per weight, a lane takes output rows in turn and walks the
+// pixels whose window element lies inside the input
+template <int KIND>
+TN_INLINE void conv_param_pair_any(const TinyLayer *__restrict__ L, const float *__restrict__ gin, const int in_sz,
+                                   const float *__restrict__ gdy, const int out_sz, const int s_beg, const int s_end,
+                                   const int co, const int ci, const int group, const TinyUpdate &u, float *lds) {
+  const int H = L->H, W = L->W, OH = L->OH, OW = L->OW, plane = OH * OW, iplane = H * W, chunk = L->dw_chunk;
+  const int sh = L->sh, sw = L->sw, taps = L->R * L->S, C = L->C;
+  const FastDiv d_oh = L->d_oh, d_s = L->d_s;
+  const bool connected = !L->tbl || L->tbl[ci * L->K + co];
+  const TinyTarget tw = tn_target<KIND>(u, L, false, group), tb = tn_target<KIND>(u, L, true, group);
+  float *xl = lds, *dl = lds + quad_pitch(chunk * iplane);
+  int g = 64;
+  while (g > 1 && taps * g > TP_THREADS) g >>= 1;
+  const int part = threadIdx.x & (g - 1);
+  float db = 0.0f;
+  for (int t0 = 0; t0 < taps; t0 += TP_THREADS / g) {
+    const int tap = t0 + threadIdx.x / g, e = (co * C + ci) * taps + tap;
+    const bool mine = tap < taps;
+    const TinyOld old_w = tn_old<KIND>(tw, e, mine && part == 0);
+    uint32_t wy, wx;
+    d_s.divmod(mine ? tap : 0, wy, wx);
+    // iy = oy*sh + wy - ph in [0, H), ix = ox*sw + wx - pw in [0, W)
+    const int yoff = static_cast<int>(wy) - L->ph, xoff = static_cast<int>(wx) - L->pw;
+    const int ox_lo = xoff >= 0 ? 0 : (-xoff + sw - 1) / sw, ox_hi = W - 1 - xoff < 0 ? 0 : min(OW, (W - 1 - xoff) / sw + 1);
+    float sum = 0.0f;
+    for (int s0 = s_beg; s0 < s_end; s0 += chunk) {
+      const int ns = min(chunk, s_end - s0);
+      lds_barrier();
+      stage_planes(L, xl, gin + static_cast<size_t>(s0) * in_sz + ci * iplane, in_sz, dl,
+                   gdy + static_cast<size_t>(s0) * out_sz + co * plane, out_sz, ns);
+      lds_barrier();
+      if (mine && connected)
+        for (int row = part; row < ns * OH; row += g) {
+          uint32_t s, oy;
+          d_oh.divmod(row, s, oy);
+          const int iy = static_cast<int>(oy) * sh + yoff;
+          if (static_cast<unsigned>(iy) >= static_cast<unsigned>(H)) continue;
+          const float *xr = xl + s * iplane + iy * W + xoff, *dr = dl + row * OW;
+          for (int ox = ox_lo; ox < ox_hi; ++ox) sum = __builtin_fmaf(xr[ox * sw], dr[ox], sum);
+        }
+      if (t0 == 0 && ci == 0)
+        for (int i = threadIdx.x; i < ns * plane; i += TP_THREADS) db += dl[i];
+    }
+    sum = group_sum(sum, g);
+    if (mine && part == 0) tn_finish<KIND>(tw, old_w, e, sum);
+  }
+  if (ci == 0 && L->nb) {
+    lds_barrier();
+    db = workgroup_sum(db, lds);
+    if (threadIdx.x == 0) tn_finish<KIND>(tb, tn_old<KIND>(tb, co, true), co, db);
+  }
+}
+// A fully-connected layer, or a convolution that is one: a weight is the sum over the samples of one input times one
+// output gradient. V weights a thread, neighbours along the faster index (V = 4: its rows are whole, aligned words).
+template <int KIND, int V>
+TN_INLINE void outer_param(const TinyLayer *__restrict__ L, const float *__restrict__ gin, const int in_sz,
+                           const float *__restrict__ gdy, const int out_sz, const int s_beg, const int s_end,
+                           const int block, const int group, const TinyUpdate &u) {
+  const bool conv = L->kind == TDH_L_CONV;   // [co][k], or [input][output]
+  const float *fast = conv ? gin : gdy, *slow = conv ? gdy : gin;
+  const int fast_stride = conv ? in_sz : out_sz, slow_stride = conv ? out_sz : in_sz, nw = L->nw;
+  const int e = (block * TP_THREADS + static_cast<int>(threadIdx.x)) * V;
+  if (e >= nw) return;
+  uint32_t r, c;
+  if (conv) L->d_nk.divmod(e, r, c);
+  else L->d_out.divmod(e, r, c);
+  const TinyTarget t = tn_target<KIND>(u, L, false, group);
+  TinyOld old[V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) old[k] = tn_old<KIND>(t, e + k, true);
+  float sum[V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) sum[k] = 0.0f;
+  constexpr int AHEAD = 16;
+  for (int s0 = s_beg; s0 < s_end; s0 += AHEAD) {
+    float f[AHEAD][V], d[AHEAD];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) {
+      const size_t s = min(s0 + j, s_end - 1);
+      const float *fp = fast + s * fast_stride + c;
+      if (V == 4) {
+        const float4 v = *reinterpret_cast<const float4 *>(fp);
+        f[j][0] = v.x; f[j][1 % V] = v.y; f[j][2 % V] = v.z; f[j][3 % V] = v.w;
+      } else {
+        f[j][0] = fp[0];
+      }
+      d[j] = slow[s * slow_stride + r];
+    }
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+      if (s0 + j < s_end) {
+#pragma unroll
+        for (int k = 0; k < V; ++k) sum[k] = __builtin_fmaf(f[j][k], d[j], sum[k]);
+      }
+  }
+  const uint8_t *tbl = L->tbl;
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    if (conv && tbl && !tbl[L->d_taps.div(c + k) * L->K + r]) sum[k] = 0.0f;
+    tn_finish<KIND>(t, old[k], e + k, sum[k]);
+  }
+}
+// element e of n: the sum over the samples of src[sample][stride]
+template <int KIND>
+TN_INLINE void column_param(const float *__restrict__ src, const size_t stride, const int n, const int s_beg, const int s_end,
+                            const int block, const TinyTarget &t) {
+  const int e = block * TP_THREADS + threadIdx.x;
+  if (e >= n) return;
+  const TinyOld old = tn_old<KIND>(t, e, true);
+  constexpr int AHEAD = 16;
+  float sum = 0.0f;
+  for (int s0 = s_beg; s0 < s_end; s0 += AHEAD) {
+    float v[AHEAD];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) v[j] = src[min(s0 + j, s_end - 1) * stride + e];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) sum += s0 + j < s_end ? v[j] : 0.0f;
+  }
+  tn_finish<KIND>(t, old, e, sum);
+}
+// an average pool's channel (average_pooling_layer.h:58-106): dW = scale * sum of (window sum * dY), db = sum of dY
+template <int KIND>
+TN_INLINE void pool_param(const TinyLayer *__restrict__ L, const float *__restrict__ gin, const int in_sz,
+                          const float *__restrict__ gdy, const int out_sz, const int s_beg, const int s_end, const int c,
+                          const int group, const TinyUpdate &u, float *lds) {
+  const int H = L->H, W = L->W, OW = L->OW, plane = L->OH * OW, iplane = H * W, R = L->R, S = L->S, chunk = L->dw_chunk;
+  const FastDiv d_oplane = L->d_oplane, d_ow = L->d_ow;
+  float *xl = lds, *dl = lds + quad_pitch(chunk * iplane);
+  float dw = 0.0f, db = 0.0f;
+  for (int s0 = s_beg; s0 < s_end; s0 += chunk) {
+    const int ns = min(chunk, s_end - s0);
+    lds_barrier();
+    stage_planes(L, xl, gin + static_cast<size_t>(s0) * in_sz + c * iplane, in_sz, dl,
+                 gdy + static_cast<size_t>(s0) * out_sz + c * plane, out_sz, ns);
+    lds_barrier();
+    for (int i = threadIdx.x; i < ns * plane; i += TP_THREADS) {
+      uint32_t s, r, oy, ox;
+      d_oplane.divmod(i, s, r);
+      d_ow.divmod(r, oy, ox);
+      const int x0 = ox * L->sw, y0 = oy * L->sh;
+      const float d = dl[i], *win = xl + s * iplane + y0 * W + x0;
+      db += d;
+      if (x0 + S <= W && y0 + R <= H)
+        for (int wy = 0; wy < R; ++wy)
+          for (int wx = 0; wx < S; ++wx) dw = __builtin_fmaf(win[wy * W + wx], d, dw);
+    }
+  }
+  lds_barrier();
+  dw = workgroup_sum(dw, lds);
+  db = workgroup_sum(db, lds + TP_WAVES);
+  if (threadIdx.x == 0) {
+    const TinyTarget tw = tn_target<KIND>(u, L, false, group), tb = tn_target<KIND>(u, L, true, group);
+    tn_finish<KIND>(tw, tn_old<KIND>(tw, c, true), c, dw * L->scale);
+    tn_finish<KIND>(tb, tn_old<KIND>(tb, c, true), c, db);
+  }
+}
+
+// The first layer's dX of one sample and input channel, a band of `rows` rows: dY's rows under it go into their frame
+// of zeros, a lane takes four pixels (conv_back_dx), the waves share the output channels.
+struct DxBand {
+  int rows, bands, floats;   // floats of LDS
+};
+__host__ __device__ inline DxBand dx_band(const TinyLayer &L) {
+  const int units_w = (L.W + 3) >> 2;
+  DxBand b;
+  b.rows   = units_w >= 64 ? 1 : min(64 / units_w, L.H);
+  b.bands  = (L.H + b.rows - 1) / b.rows;
+  b.floats = L.K * (b.rows + L.R - 1) * quad_pitch(L.W + L.S - 1) + 4 + TP_THREADS * 4;
+  return b;
+}
+template <int R, int S>
+TN_INLINE void conv_dx_band(const TinyLayer *__restrict__ L, const float *__restrict__ w, const float *__restrict__ gdy,
+                            float *__restrict__ gdx, const int ci, const int band, float *lds) {
+  const int C = L->C, H = L->H, W = L->W, K = L->K, OH = L->OH, OW = L->OW, PW = quad_pitch(W + S - 1), units_w = (W + 3) >> 2;
+  const int full = units_w >= 64 ? 1 : min(64 / units_w, H), y0 = band * full, rows = min(full, H - y0);
+  const int fr = rows + R - 1, PP = fr * PW, cells = K * PP, oy0 = y0 - (R - 1 - L->ph), ox0 = -(S - 1 - L->pw);
+  const FastDiv d_pw = L->d_pw4;
+  const uint8_t *__restrict__ tbl = L->tbl;
+  constexpr int AHEAD = 8;
+  for (int base = threadIdx.x; base < cells; base += AHEAD * TP_THREADS) {
+    float v[AHEAD];
+    bool in[AHEAD];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) {
+      uint32_t line, px;
+      d_pw.divmod(min(base + j * TP_THREADS, cells - 1), line, px);
+      const int co = static_cast<int>(line) / fr, oy = oy0 + static_cast<int>(line) - co * fr, ox = ox0 + static_cast<int>(px);
+      in[j] = static_cast<unsigned>(oy) < static_cast<unsigned>(OH) && static_cast<unsigned>(ox) < static_cast<unsigned>(OW);
+      v[j]  = gdy[in[j] ? (co * OH + oy) * OW + ox : 0];
+    }
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+      if (base + j * TP_THREADS < cells) lds[base + j * TP_THREADS] = in[j] ? v[j] : 0.0f;
+  }
+  lds_barrier();
+  constexpr int taps = R * S;
+  const int lane = threadIdx.x & 63, wave = wave_index(), units = rows * units_w;
+  float *scratch = lds + cells + 4;            // (a row's last read may pass its end)
+  for (int u0 = 0; u0 < units; u0 += 64) {     // (one trip unless a row has more units than a wave lanes)
+    const int unit = min(u0 + lane, units - 1), iy = unit / units_w, ix = (unit - iy * units_w) << 2;
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int co = wave; co < K; co += TP_WAVES) {
+      if (tbl && !tbl[ci * K + co]) continue;
+      const ScalarFloats wq = (ScalarFloats)(w + static_cast<size_t>(co * C + ci) * taps);
+      const float *dp = lds + co * PP + iy * PW + ix;
+      float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int wy = 0; wy < R; ++wy) {
+        float v[S + 3];
+        read_row(v, dp + (R - 1 - wy) * PW);
+#pragma unroll
+        for (int wx = 0; wx < S; ++wx)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) sum[k] = __builtin_fmaf(wq[wy * S + wx], v[k + S - 1 - wx], sum[k]);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc[k] += sum[k];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) scratch[(wave * 64 + lane) * 4 + k] = acc[k];
+    lds_barrier();
+    // thread: pixel tid%4 of unit u0 + tid/4, of the first 64
+    const int mine = u0 + (threadIdx.x >> 2), my = mine / units_w, mx = ((mine - my * units_w) << 2) + (threadIdx.x & 3);
+    if (threadIdx.x < 256 && mine < units && mx < W) {
+      float v = scratch[threadIdx.x];
+#pragma unroll
+      for (int k = 1; k < TP_WAVES; ++k) v += scratch[256 * k + threadIdx.x];
+      gdx[(y0 + my) * W + mx] = v;
+    }
+    lds_barrier();
+  }
+}
+
+template <int KIND>
+__global__ void __launch_bounds__(TP_THREADS, 4)
+tiny_net_param_kernel(const TinyPlan *__restrict__ plan, const float *__restrict__ x, const TinyRanges ranges,
+                      const TinyUpdate u, const int batch, const int param_blocks) {
+  extern __shared__ float lds[];
+  if (KIND >= 0 && opt_powers(KIND) > 0 && u.powers_in && blockIdx.x == 0 && threadIdx.x == 0) {   // (as opt_multi_kernel)
+    float q1 = u.powers_in[0], q2 = u.powers_in[1];
+    for (int i = 0; i < u.n_tensors; ++i) {
+      q1 *= u.p.b1;
+      if (opt_powers(KIND) == 2) q2 *= u.p.b2;
+    }
+    u.powers_out[0] = q1;
+    u.powers_out[1] = q2;
+  }
+  const int n = plan->n;
+  int id = blockIdx.x;
+  if (id >= param_blocks) {   // workgroups (band, input channel, sample), samples fastest
+    id -= param_blocks;
+    const TinyLayer *__restrict__ L = &plan->l[0];
+    const int rest = id / batch, s = id - rest * batch, ci = rest % L->C, band = rest / L->C;
+    const float *gdy = plan->l[1].dx + static_cast<size_t>(s) * L->out_size;
+    float *gdx = L->dx + static_cast<size_t>(s) * L->in_size + ci * L->H * L->W;
+    if (L->R == 5) conv_dx_band<5, 5>(L, plan->first_w, gdy, gdx, ci, band, lds);
+    else conv_dx_band<3, 3>(L, plan->first_w, gdy, gdx, ci, band, lds);
+    return;
+  }
+  int first = 0, job = ranges.job[0], per_group = ranges.per_group[0], size = ranges.size[0];
+#pragma unroll
+  for (int k = 1; k < TP_RANGES; ++k) {   // (indices known to the compiler: the argument stays in scalar registers)
+    const bool on = ranges.first[k] <= id;
+    first     = on ? ranges.first[k] : first;
+    job       = on ? ranges.job[k] : job;
+    per_group = on ? ranges.per_group[k] : per_group;
+    size      = on ? ranges.size[k] : size;
+  }
+  const int li = job >> 3, what = job & 7, group = (id - first) / per_group, block = id - first - group * per_group;
+  const TinyLayer *__restrict__ L = &plan->l[li];
+  const int in_sz = L->in_size, out_sz = L->out_size;
+  const float *gin = li == 0 ? x : plan->l[li - 1].out;
+  const float *gdy = li == n - 1 ? plan->dloss : plan->l[li + 1].dx;
+  const int s_beg = group * size, s_end = min(batch, s_beg + size);
+  switch (what) {
+    case TP_CONV: {
+      const int co = L->d_c.div(block), ci = block - co * L->C;
+      const bool pad = L->ph != 0 || L->pw != 0;
+      if (!L->dw_quads) conv_param_pair_any<KIND>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, co, ci, group, u, lds);
+      else if (L->R == 5) {
+        if (pad) conv_param_pair<KIND, 5, 5, true>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, co, ci, group, u, lds);
+        else conv_param_pair<KIND, 5, 5, false>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, co, ci, group, u, lds);
+      } else {
+        if (pad) conv_param_pair<KIND, 3, 3, true>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, co, ci, group, u, lds);
+        else conv_param_pair<KIND, 3, 3, false>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, co, ci, group, u, lds);
+      }
+    } break;
+    case TP_OUTER: outer_param<KIND, 1>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, block, group, u); break;
+    case TP_OUTER4: outer_param<KIND, 4>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, block, group, u); break;
+    case TP_COLUMNS: column_param<KIND>(gdy, out_sz, L->nb, s_beg, s_end, block, tn_target<KIND>(u, L, true, group)); break;
+    case TP_POOL: pool_param<KIND>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, block, group, u, lds); break;
+    case TP_SLICES_W: column_param<KIND>(L->pw_part, L->nw, L->nw, s_beg, s_end, block, tn_target<KIND>(u, L, false, group)); break;
+    default: column_param<KIND>(L->pb_part, L->nb, L->nb, s_beg, s_end, block, tn_target<KIND>(u, L, true, group)); break;
+  }
+}
+
+// g[i] += slice[0][i] + slice[1][i] + ... in the order of the groups (edge::merge_grads, node.h:89-103)
 __global__ void __launch_bounds__(256)
-tiny_net_merge_kernel(const TinyMerge m, const int batch) {
+tiny_net_merge_kernel(const TinyMerge m) {
   int j = 0;
   while (j + 1 < m.n && m.first_block[j + 1] <= static_cast<int>(blockIdx.x)) ++j;
   const int i = (static_cast<int>(blockIdx.x) - m.first_block[j]) * 256 + threadIdx.x;
   if (i >= m.len[j]) return;
   const float *p = m.slices[j] + i;
   float sum = p[0];
-  for (int s = 1; s < batch; ++s) sum += p[static_cast<size_t>(s) * m.len[j]];
+  for (int s = 1; s < m.count[j]; ++s) sum += p[static_cast<size_t>(s) * m.len[j]];
   m.g[j][i] += sum;
 }
 
@@ -1689,9 +2151,12 @@ int tiny_prepare() {
   if (!attr_set) {
     TDH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&tiny_net_step_kernel),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(TINY_LDS_MAX_BYTES)));
-    TDH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&tiny_net_param_kernel),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(TINY_LDS_MAX_BYTES)));
-    for (const void *k : {reinterpret_cast<const void *>(&tiny_net_front_kernel), reinterpret_cast<const void *>(&tiny_net_back_kernel)})
+    const auto of = [](auto k) { return reinterpret_cast<const void *>(k); };
+    for (const void *k : {of(&tiny_net_front_kernel), of(&tiny_net_back_kernel), of(&tiny_net_param_kernel<-1>),
+                          of(&tiny_net_param_kernel<TDH_OPT_SGD>), of(&tiny_net_param_kernel<TDH_OPT_MOMENTUM>),
+                          of(&tiny_net_param_kernel<TDH_OPT_NESTEROV>), of(&tiny_net_param_kernel<TDH_OPT_ADAM>),
+                          of(&tiny_net_param_kernel<TDH_OPT_ADAGRAD>), of(&tiny_net_param_kernel<TDH_OPT_RMSPROP>),
+                          of(&tiny_net_param_kernel<TDH_OPT_ADAMAX>)})
       TDH_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(TINY_LDS_MAX_BYTES)));
     attr_set = true;
   }
@@ -1703,7 +2168,7 @@ static void plan_split(TinyPlan &P) {
   P.split = 0;
   const TinyLayer &F = P.l[0];
   if (F.kind != TDH_L_CONV || !((F.R == 5 && F.S == 5) || (F.R == 3 && F.S == 3)) || conv_is_matvec(F) ||
-      !(P.first_dx_as_job || P.skip_first_dx))
+      F.sh != 1 || F.sw != 1 || !(P.first_dx_as_job || P.skip_first_dx))
     return;
   int m = 1;
   size_t front = F.OH * F.OW, back = 0;
@@ -1712,53 +2177,46 @@ static void plan_split(TinyPlan &P) {
     if (L.kind == TDH_L_ACT && L.act != TDH_ACT_SOFTMAX) continue;
     if (L.kind != TDH_L_MAXPOOL && L.kind != TDH_L_AVEPOOL) break;
     front += L.OH * L.OW;
-    back += L.H * L.W;
+    back += quad_pitch(L.H * L.W);
   }
   if (m == P.n || !P.l[m].dx_framed || P.l[m].K > 64) return;   // (64: conv_back_dx)
   const TinyLayer &L = P.l[m];
-  P.back_scratch = (conv_framed_floats(L) + 3) & ~3;
+  P.back_scratch = L.K * (L.H + L.R - 1) * quad_pitch(L.W + L.S - 1) + 4;   // (a row's last read may pass its end)
   const BackSplit b = back_split(L.H, L.W, L.K);
   P.back_planes  = P.back_scratch + b.parts * b.chunks * 256;
-  P.back_floats  = P.back_planes + static_cast<int>(back) + L.H * L.W;
+  P.back_sample  = P.back_planes + static_cast<int>(back) + quad_pitch(L.H * L.W);
+  P.back_sample_floats = F.C * F.H * dw_x_pitch(&F);
+  P.back_floats  = P.back_sample + P.back_sample_floats + 32 * m;
   P.front_floats = static_cast<int>(front);
   if (std::max(static_cast<size_t>(P.back_floats), P.in_size + front) * sizeof(float) > TINY_LDS_MAX_BYTES) return;
   P.split = m;
 }
 
-int tiny_build_jobs(TinyPlan &P) {
-  // units of work per layer and the units one workgroup takes: a lane's item for the grouped
-  // sums, sixteen elements per lane for the element-wise products, a wave's item for the dX
-  struct Piece { int layer, what, units, per_job; };
-  Piece pieces[2 * TINY_MAX_LAYERS + 1];
-  int n_pieces = 0;
-  size_t lds = 0, framed = 0;
+int tiny_layout(TinyPlan &P) {
+  size_t framed = 0, lds = 26 * TP_WAVES;   // (conv_param_pair's sums)
   for (int i = 0; i < P.n; ++i) {
     TinyLayer &L = P.l[i];
     L.dx_framed = L.kind == TDH_L_CONV && conv_dx_shape_is_framed(L) && L.dx != nullptr;
     if (L.dx_framed) {
       L.d_pplane = FastDiv(static_cast<uint32_t>((L.H + L.R - 1) * (L.W + L.S - 1)));
       L.d_pw     = FastDiv(static_cast<uint32_t>(L.W + L.S - 1));
+      L.d_pw4    = FastDiv(static_cast<uint32_t>(quad_pitch(L.W + L.S - 1)));
     }
   }
   P.first_dx_as_job = P.l[0].dx_framed && P.n > 1 && !P.skip_first_dx;
-  plan_split(P);
   for (int i = 0; i < P.n; ++i) {
-    const TinyLayer &L = P.l[i];
-    if (i == 0 && P.first_dx_as_job) {
-      pieces[n_pieces++] = {i, 1, conv_dx_scalar_items(L), TP_THREADS / 64};
-      lds = std::max(lds, static_cast<size_t>(conv_framed_floats(L)));
-    } else if (L.dx_framed) {
-      framed = std::max(framed, static_cast<size_t>(conv_framed_floats(L)));
-    }
-    if (!L.nw) continue;
-    lds = std::max(lds, static_cast<size_t>(((L.in_size + 3) & ~3) + ((L.out_size + 3) & ~3)));
-    if (L.kind == TDH_L_CONV && !conv_is_matvec(L)) {
-      pieces[n_pieces++] = {i, 0, L.nw * conv_param_group(L), TP_THREADS};
-      if (L.nb) pieces[n_pieces++] = {i, 2, 1, 1};
-    }
-    else if (L.kind == TDH_L_CONV || L.kind == TDH_L_FC) pieces[n_pieces++] = {i, 0, L.nw, 16 * TP_THREADS};
-    else pieces[n_pieces++] = {i, 0, 1, 1};
+    TinyLayer &L = P.l[i];
+    L.dw_chunk = 512;   // (what needs no LDS)
+    if (i == 0 && P.first_dx_as_job) lds = std::max(lds, static_cast<size_t>(dx_band(L).floats));
+    else if (L.dx_framed) framed = std::max(framed, static_cast<size_t>(conv_framed_floats(L)));
+    if (!L.nw || L.kind == TDH_L_FC || conv_is_matvec(L)) continue;
+    // planes of the input and the output gradient: as many samples at a time as fit 48 KB
+    L.dw_quads = L.kind == TDH_L_CONV && L.sh == 1 && L.sw == 1 && ((L.R == 5 && L.S == 5) || (L.R == 3 && L.S == 3));
+    const int planes = L.H * L.W + L.OH * L.OW;
+    L.dw_chunk = std::min(std::max(12288 / planes, 1), 32);
+    lds = std::max(lds, static_cast<size_t>(L.dw_chunk) * planes + 4);
   }
+  plan_split(P);
   P.lds_pad = P.lds_floats;
   P.lds_floats += static_cast<int>(framed);
   // operands of the products that run on the matrix cores, while LDS has room for them
@@ -1808,34 +2266,28 @@ int tiny_build_jobs(TinyPlan &P) {
       P.lds_floats = at + rows * cols;
     }
   }
-  for (int scale = 1;; scale *= 2) {
-    int jobs = 0;
-    for (int q = 0; q < n_pieces; ++q) jobs += ceil_div(pieces[q].units, pieces[q].per_job * scale);
-    if (jobs > TINY_MAX_JOBS) continue;
-    P.n_jobs = 0;
-    for (int q = 0; q < n_pieces; ++q) {
-      const int per = pieces[q].per_job * scale;
-      for (int base = 0; base < pieces[q].units; base += per) {
-        TinyJob &J = P.jobs[P.n_jobs++];
-        J.layer = static_cast<int16_t>(pieces[q].layer);
-        J.what  = static_cast<int16_t>(pieces[q].what);
-        J.base  = base;
-        J.count = std::min(per, pieces[q].units - base);
-      }
-    }
-    break;
-  }
   P.lds_job_floats = static_cast<int>(lds);
   return TDH_OK;
 }
 
+// The ends of the chain a channel a workgroup while there is a compute unit for each. LeNet-5's step, us, with them / one
+// workgroup per sample throughout: 16 samples 46.6 / 56.4, 32 48.7 / 57.9, 42 57.4 / 60.1, 44 64.0 / 61.3, 64 67.2 / 64.8, 104 82.8 /
+// 73.5: with several workgroups a compute unit, each of which frames all of dY for its one channel, they lose.
+int tiny_most_split(const TinyPlan &plan) { return plan.split ? 256 / std::max(plan.l[0].K, plan.l[plan.split].C) : 0; }
+static bool tiny_splits(const TinyPlan &plan, int batch) { return batch <= tiny_most_split(plan); }
+// A batch of up to 32 samples is one group, whose workgroups update; the groups of a larger one are of 16, which
+// the optimizer's kernel has to add up either way (64 samples in groups of 32: 58 us instead of 16, the first layer's
+// workgroups being few and long; as many samples as fit LDS at a time is what a layer's group is limited to).
+int tiny_groups(const TinyPlan &plan, int layer, int batch) {
+  const TinyLayer &L = plan.l[layer];
+  const int most = batch <= 32 ? 32 : 16;
+  return ceil_div(batch, tiny_splits(plan, batch) && layer < plan.split ? most : std::min(L.dw_chunk, most));
+}
+
 int launch_tiny_step(const TinyPlan &plan, const TinyPlan *dev_plan, int loss, int softmax_xent, int batch,
                      const float *x, const float *t) {
-  // The ends of the chain a channel a workgroup while there is a compute unit for each. LeNet-5 at 16 / 32 / 64 /
-  // 120 samples, us for the three launches and for the step kernel alone: 34.5 / 40.1, 35.5 / 40.2, 40.8 / 40.3, 52.4 /
-  // 43.1: with several workgroups a compute unit, each of which frames all of dY for its one channel, they lose.
   const TinyLayer &F = plan.l[0], &M = plan.l[plan.split];
-  const int m = plan.split && batch * std::max(F.K, M.C) <= 256 ? plan.split : 0;
+  const int m = tiny_splits(plan, batch) ? plan.split : 0;
   const double front_flop = m ? 2.0 * F.out_size * F.C * F.R * F.S * batch : 0.0;
   const double back_flop  = m ? 2.0 * M.out_size * M.C * M.R * M.S * batch : 0.0;
   if (m) {
@@ -1855,29 +2307,87 @@ int launch_tiny_step(const TinyPlan &plan, const TinyPlan *dev_plan, int loss, i
   if (m) {
     ProfScope prof("tiny_net_back", back_flop, WORK_FLOP);
     TDH_LAUNCH(tiny_net_back_kernel, dim3(batch, M.C), dim3(TB_THREADS), plan.back_floats * sizeof(float), ctx().stream,
-               dev_plan, m);
+               dev_plan, m, x);
     TDH_LAUNCH_CHECK();
   }
   return TDH_OK;
 }
 
-int launch_tiny_params(const TinyPlan &plan, const TinyPlan *dev_plan, int batch, const float *x) {
-  if (plan.n_jobs == 0) return TDH_OK;
-  ProfScope prof("tiny_net_param_grads", plan.flop_per_sample * batch * (1.0 / 3.0), WORK_FLOP);
-  // (x counts the samples: consecutive workgroups go to different XCDs, and this way each XCD
-  // gets every job of the samples that fall to it rather than every sample of a few jobs)
-  TDH_LAUNCH(tiny_net_param_kernel, dim3(batch, plan.n_jobs), dim3(TP_THREADS), plan.lds_job_floats * sizeof(float),
-             ctx().stream, dev_plan, x);
-  TDH_LAUNCH_CHECK();
+int launch_tiny_params(const TinyPlan &plan, const TinyPlan *dev_plan, int batch, const float *x, tdh_opt *update,
+                       int n_tensors, const float *powers_in, float *powers_out, bool *updated) {
+  TinyRanges r;
+  int n = 0, blocks = 0;
+  bool one_group = true;
+  auto add = [&](int layer, int what, int count) {
+    const int groups = tiny_groups(plan, layer, batch);
+    r.first[n]     = blocks;
+    r.job[n]       = layer * 8 + what;
+    r.per_group[n] = count;
+    r.size[n++]    = ceil_div(batch, groups);
+    blocks += count * groups;
+    one_group = one_group && groups == 1;
+  };
+  const int m = tiny_splits(plan, batch) ? plan.split : 0;
+  for (int pass = 0; pass < 2; ++pass)   // (the convolutions first: they take longest)
+    for (int i = 0; i < plan.n; ++i) {
+      const TinyLayer &L = plan.l[i];
+      const bool pair = L.kind == TDH_L_CONV && !conv_is_matvec(L);
+      if (!L.nw || pair != (pass == 0)) continue;
+      if (i < m) {   // left by the back kernel, sample by sample
+        add(i, TP_SLICES_W, ceil_div(L.nw, TP_THREADS));
+        if (L.nb) add(i, TP_SLICES_B, ceil_div(L.nb, TP_THREADS));
+      } else if (pair) {
+        add(i, TP_CONV, L.K * L.C);
+      } else if (L.kind == TDH_L_AVEPOOL) {
+        add(i, TP_POOL, L.C);
+      } else {
+        const bool conv = L.kind == TDH_L_CONV;
+        const int fast = conv ? L.in_size : L.out_size;
+        const bool vec = fast % 4 == 0 && (i > 0 || !conv || (reinterpret_cast<uintptr_t>(x) & 15u) == 0);
+        add(i, vec ? TP_OUTER4 : TP_OUTER, ceil_div(L.nw, (vec ? 4 : 1) * TP_THREADS));
+        if (L.nb) add(i, TP_COLUMNS, ceil_div(L.nb, TP_THREADS));
+      }
+    }
+  for (int k = n; k < TP_RANGES; ++k) {
+    r.first[k] = 0x7fffffff;
+    r.job[k] = r.per_group[k] = r.size[k] = 0;
+  }
+  const int dx_blocks = plan.first_dx_as_job ? dx_band(plan.l[0]).bands * plan.l[0].C * batch : 0;
+  TinyUpdate u;
+  *updated = update && one_group;
+  if (*updated) {
+    u.p = opt_scalars(*update, 1.0f);
+    u.n_tensors = n_tensors;
+    u.b1_t = update->b1_t; u.b2_t = update->b2_t;
+    u.powers_in = powers_in; u.powers_out = powers_out;
+  }
+  if (blocks + dx_blocks > 0) {
+    ProfScope prof("tiny_net_param_grads", plan.flop_per_sample * batch * (1.0 / 3.0), WORK_FLOP);
+    void (*kernel)(const TinyPlan *, const float *, TinyRanges, TinyUpdate, int, int) = tiny_net_param_kernel<-1>;
+    if (*updated) switch (update->kind) {
+      case TDH_OPT_SGD: kernel = tiny_net_param_kernel<TDH_OPT_SGD>; break;
+      case TDH_OPT_MOMENTUM: kernel = tiny_net_param_kernel<TDH_OPT_MOMENTUM>; break;
+      case TDH_OPT_NESTEROV: kernel = tiny_net_param_kernel<TDH_OPT_NESTEROV>; break;
+      case TDH_OPT_ADAM: kernel = tiny_net_param_kernel<TDH_OPT_ADAM>; break;
+      case TDH_OPT_ADAGRAD: kernel = tiny_net_param_kernel<TDH_OPT_ADAGRAD>; break;
+      case TDH_OPT_RMSPROP: kernel = tiny_net_param_kernel<TDH_OPT_RMSPROP>; break;
+      case TDH_OPT_ADAMAX: kernel = tiny_net_param_kernel<TDH_OPT_ADAMAX>; break;
+      default: return set_error(TDH_ERR_INVALID, "optimizer kind %d is not supported", update->kind);
+    }
+    TDH_LAUNCH(kernel, dim3(blocks + dx_blocks), dim3(TP_THREADS), plan.lds_job_floats * sizeof(float),
+               ctx().stream, dev_plan, x, r, u, batch, blocks);
+    TDH_LAUNCH_CHECK();
+  }
+  if (*updated) opt_advance(update, n_tensors);
   return TDH_OK;
 }
 
-int launch_tiny_merge(const TinyMerge &m, int batch) {
+int launch_tiny_merge(const TinyMerge &m) {
   if (m.n == 0) return TDH_OK;
   double bytes = 0.0;
-  for (int j = 0; j < m.n; ++j) bytes += 4.0 * m.len[j] * (batch + 2);
+  for (int j = 0; j < m.n; ++j) bytes += 4.0 * m.len[j] * (m.count[j] + 2);
   ProfScope prof("tiny_net_merge_grads", bytes, WORK_BYTE);
-  TDH_LAUNCH(tiny_net_merge_kernel, dim3(m.first_block[m.n]), dim3(256), 0, ctx().stream, m, batch);
+  TDH_LAUNCH(tiny_net_merge_kernel, dim3(m.first_block[m.n]), dim3(256), 0, ctx().stream, m);
   TDH_LAUNCH_CHECK();
   return TDH_OK;
 }
