@@ -527,12 +527,10 @@ size_t conv_any_fwd_workspace_bytes(const ConvShape &c);
 size_t conv_any_dx_workspace_bytes(const ConvShape &c);
 int conv_any_fwd_run(const ConvShape &c, const float *x, const float *w, const float *bias, float *out, float *act_out,
                      int act_kind);
-int conv_any_dx_run(const ConvShape &c, const float *dy, const float *w, float *dx, ActGrad ag);
 // conv_dw_any.hip: dW (and db as column C*R*S) of any window, stride and size, as slices [slice][Kc][columns]
 bool conv_dw_any_applicable(const ConvShape &c, bool with_db);
 size_t conv_dw_any_workspace_bytes(const ConvShape &c, bool with_db);
 size_t conv_dw_any_most_bytes(const ConvShape &c, bool with_db);
-int conv_dw_any_run(const ConvShape &c, const float *x, const float *dy, bool with_db, const float **partial, int *slices);
 // conv_bwd_direct.hip: any of dX, dW and db of a layer that is a few small tiles, as one launch
 bool conv_bwd_direct_applicable(int batch, int C, int Kc, int H, int W, int OH, int OW, int R, int S);
 int conv_bwd_direct_run(int batch, int C, int Kc, const float *x, const float *w, const float *dy, float *dx, float *dw,

@@ -15,7 +15,7 @@
 #include <algorithm>
 #include <vector>
 
-#include "gemm_mfma.h"
+#include "conv_any.h"
 
 namespace tdh {
 
@@ -135,20 +135,6 @@ struct DwInputOperand {
                     static_cast<unsigned>(ix) < static_cast<unsigned>(g.W);
     return ok ? x[k.base + f.coff + iy * g.W + ix] : f.outside;
   }
-};
-
-// dW with the bias gradient as column crs
-struct EpiDwDb {
-  float *dw, *db;
-  int crs, accumulate;
-  struct Col {
-    int n;
-  };
-  __device__ __forceinline__ float *at(int m, const Col &c) const { return c.n < crs ? dw + m * crs + c.n : db + m; }
-  __device__ __forceinline__ Col col(int n) const { return {n}; }
-  __device__ __forceinline__ float prior(int m, const Col &c) const { return accumulate ? *at(m, c) : 0.0f; }
-  __device__ __forceinline__ void store(int m, const Col &c, float v, float before) const { *at(m, c) = v + before; }
-  __device__ __forceinline__ void store(int m, const Col &c, float v) const { store(m, c, v, prior(m, c)); }
 };
 
 // dX A operand: m = ci, k = (co, ky, kx) -> w[co][ci][ky][kx]
@@ -1604,6 +1590,41 @@ static int run_first_both(const ConvGeom &g, int batch, const float *x, const fl
   return flush_deferred_reduces();
 }
 
+// Whether dW of this call runs on conv_dw_any_kernel (the branches of conv2d_bwd in front of it, in its order).
+static bool dw_goes_any(const tdh_conv_desc *d, const ConvGeom &g, int batch, const float *dy, const float *db, int accumulate) {
+  if (d->tbl || (dw_small_applies(d, g, batch) && !(reinterpret_cast<uintptr_t>(dy) & 15))) return false;
+  if (g.sh == 1 && g.sw == 1 && conv_dw_halo_applicable(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w))
+    return false;
+  return conv_dw_any_applicable(shape_of(g, batch), dw_takes_db(d, g.C * g.R * g.S, db != nullptr, accumulate));
+}
+
+// dX and dW on the kernels of any window: dW's launch packs the filters for dX, and dX's adds up dW's slices. 45x37, 21 ->
+// 45, 5x5, stride 2, 19 images, with the forward call: 49.4 us in six launches, 43.9 in four.
+static int run_any_both(const tdh_conv_desc *d, const ConvGeom &g, int batch, const float *x, const float *w, const float *dy,
+                        float *dx, float *dw, float *db, int accumulate, ActGrad dx_act) {
+  const ConvShape shape = shape_of(g, batch);
+  const int crs = g.C * g.R * g.S;
+  const bool with_db = dw_takes_db(d, crs, db != nullptr, accumulate);
+  AnyPack pack;
+  TDH_TRY(conv_any_dx_pack(shape, w, &pack));
+  const float *partial;
+  int slices;
+  TDH_TRY(conv_dw_any_run(shape, x, dy, with_db, &partial, &slices, &pack));
+  AnySums sums{};
+  sums.partial = partial; sums.splits = slices;
+  sums.M = g.Kc; sums.N = crs + (with_db ? 1 : 0);
+  sums.epi = EpiDwDb{dw, db, crs, accumulate};
+  // Very many slices, which launch_splitk_reduce has another kernel for, stay with it, and so do sums of more than three workgroups a
+  // compute unit, each of which would hold a place of dX's: forward, dX and dW of 51x50, 128 -> 150, 3x3, stride 2, 20 images (1351
+  // workgroups) 304 us along, 298 apart; 33x29, 40 -> 41, 7x7, 11 images (628) 99 / 107.
+  sums.blocks      = ceil_div(sums.M * sums.N, ANY_SUMS);
+  const bool along = slices < 64 * REDUCE_GROUPS && sums.blocks <= 768;
+  if (!along) sums.blocks = 0;
+  TDH_TRY(conv_any_dx_run(shape, dy, w, dx, dx_act, &pack, &sums));
+  if (!along) TDH_TRY(launch_splitk_reduce(partial, slices, sums.M, sums.N, sums.epi, "conv_dw_splitk_reduce"));
+  return db && !with_db ? launch_rowsum(dy, batch, g.Kc, g.OH * g.OW, db, accumulate) : TDH_OK;
+}
+
 int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w, const float *dy,
                float *dx, float *dw, float *db, int accumulate, ActGrad dx_act,
                const uint8_t *tbl_resident, PackedFilters prepacked_dx, const PoolGather *dy_pool) {
@@ -1675,7 +1696,9 @@ int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
   } else if (dx && (small_cin_dx_plan(g, dxs) ? conv_any_dx_applicable(shape_of(g, batch), ANY_OVER_FIRST)
                     : dx_stride1              ? dx_any_over_stride1(g, batch, accumulate)
                                               : conv_any_dx_applicable(shape_of(g, batch), ANY_OVER_GENERIC))) {
-    TDH_TRY(conv_any_dx_run(shape_of(g, batch), dy, w_eff, dx, dx_act));
+    if (dw && !ctx().defer_reduce && dw_goes_any(d, g, batch, dy, db, accumulate))
+      return run_any_both(d, g, batch, x, w_eff, dy, dx, dw, db, accumulate, dx_act);
+    TDH_TRY(conv_any_dx_run(shape_of(g, batch), dy, w_eff, dx, dx_act, nullptr, nullptr));
   } else if (dx && small_cin_dx_plan(g, dxs)) {
     ProfScope prof("conv_dx_small_cin", g.C, batch * g.H * g.W, g.Kc * g.R * g.S);
     launch_small_cin_dx_window<false>(g, dxs, batch, dy, w_eff, dx, dx_act, PoolGather());
@@ -1735,7 +1758,7 @@ int conv2d_bwd(const tdh_conv_desc *d, int batch, const float *x, const float *w
     } else if (conv_dw_any_applicable(shape_of(g, batch), with_db)) {
       const float *partial;
       int slices;
-      TDH_TRY(conv_dw_any_run(shape_of(g, batch), x, dy, with_db, &partial, &slices));
+      TDH_TRY(conv_dw_any_run(shape_of(g, batch), x, dy, with_db, &partial, &slices, nullptr));
       if (with_db) {
         TDH_TRY(launch_splitk_reduce(partial, slices, g.Kc, crs + 1, EpiDwDb{dw, db, crs, accumulate}, "conv_dw_splitk_reduce"));
         db = nullptr;

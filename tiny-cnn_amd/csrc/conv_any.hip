@@ -28,15 +28,14 @@
 // Reference: conv2d_op_internal.h:13-74 (forward), :79-158 (backward).
 #include <algorithm>
 
-#include "gemm_mfma.h"
-#include "split_bf16.h"
+#include "conv_any.h"
 
 namespace tdh {
 
 namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
+typedef uintx4_any uintx4;
 
 constexpr int ANY_MAX_PHASES = 4;
 constexpr uint32_t ANY_NOWHERE = 0x80000000u;   // past the end of every tile's images
@@ -75,34 +74,7 @@ struct AnyArgs {
   AnyPhase p[ANY_MAX_PHASES];
 };
 
-// The filters in parts: thread = (group, tap, m).
-__global__ void __launch_bounds__(256)
-any_pack_kernel(const float *__restrict__ w, uintx4 *__restrict__ wp, const int M, const int KC, const int m_pad,
-                const int rs, const int wm, const int wk, const int total, const FastDiv div_m, const FastDiv div_rs) {
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  if (e >= total) return;
-  uint32_t gt, m, g, t;
-  div_m.divmod(e, gt, m);
-  div_rs.divmod(gt, g, t);
-  float v[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int kc  = 8 * static_cast<int>(g) + k;
-    const bool on = static_cast<int>(m) < M && kc < KC;
-    const float f = w[on ? static_cast<size_t>(m) * wm + static_cast<size_t>(kc) * wk + t : 0];
-    v[k]          = on ? f * X3_SCALE : 0.0f;
-  }
-  uintx4 part[X3_PARTS];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    uint32_t p3[X3_PARTS];
-    split_pair(v[2 * c], v[2 * c + 1], p3);
-#pragma unroll
-    for (int p = 0; p < X3_PARTS; ++p) part[p][c] = p3[p];
-  }
-#pragma unroll
-  for (int p = 0; p < X3_PARTS; ++p) wp[(static_cast<size_t>(gt) * X3_PARTS + p) * m_pad + m] = part[p];
-}
+__global__ void __launch_bounds__(256) any_pack_kernel(const AnyPack p) { any_pack_block(p, blockIdx.x); }
 
 // One output once more in fp32, for sums that the three parts leave infinite or NaN.
 __device__ __forceinline__ float any_redo(const AnyArgs &a, const AnyPhase &ph, const int m, const int img,
@@ -127,12 +99,18 @@ __device__ __forceinline__ float any_redo(const AnyArgs &a, const AnyPhase &ph, 
 
 // MB x NB: blocks of 16 channels x 16 pixels of a wave; WK waves share the units, 4 / WK the pixels.
 template <int MB, int NB, int WK>
-__global__ void __launch_bounds__(256, 2) conv_any_kernel(const AnyArgs a) {
+__global__ void __launch_bounds__(256, 2) conv_any_kernel(const AnyArgs a, const AnySums sums) {
   constexpr int WN    = 4 / WK;
   constexpr int PIX   = WN * NB * 16;
   constexpr int ITEMS = 2;           // patch words a thread has under way
   constexpr int DEPTH = WK == 4 && MB * NB <= 6 ? 2 : 1;   // (few steps, and filters fresh from another XCD)
   extern __shared__ __align__(16) uintx4 any_lds[];
+  if (static_cast<int>(blockIdx.x) >= sums.first_x) {   // (behind the tiles)
+    const int block = (static_cast<int>(blockIdx.x) - sums.first_x) * gridDim.y + blockIdx.y;
+    if (block < sums.blocks)
+      any_sums_block(sums, block, reinterpret_cast<float(*)[ANY_SUMS]>(any_lds));
+    return;
+  }
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kw = wave % WK, nw = wave / WK;
   const int col = lane & 15, quarter = lane >> 4;
@@ -571,7 +549,7 @@ void finish_args(AnyArgs &a) {
 }
 
 template <int MB, int NB, int WK>
-int launch_any_inst(const AnyPlan &p) {
+int launch_any_inst(const AnyPlan &p, const AnySums &sums) {
   auto kernel = conv_any_kernel<MB, NB, WK>;
   if (p.lds_bytes > 64 * 1024) {
     static size_t raised = 0;
@@ -581,45 +559,63 @@ int launch_any_inst(const AnyPlan &p) {
       raised = p.lds_bytes;
     }
   }
-  TDH_LAUNCH(kernel, p.grid, dim3(256), p.lds_bytes, ctx().stream, p.args);
+  const unsigned extra = ceil_div(sums.blocks, static_cast<int>(p.grid.y));
+  TDH_LAUNCH(kernel, dim3(p.grid.x + extra, p.grid.y), dim3(256), p.lds_bytes, ctx().stream, p.args, sums);
   TDH_LAUNCH_CHECK();
   return TDH_OK;
 }
 template <int MB>
-int launch_any_mb(const AnyPlan &p) {
+int launch_any_mb(const AnyPlan &p, const AnySums &sums) {
   switch (10 * p.nb + p.wk) {
-    case 14: return launch_any_inst<MB, 1, 4>(p);
-    case 24: return launch_any_inst<MB, 2, 4>(p);
-    case 44: return launch_any_inst<MB, 4, 4>(p);
-    case 11: return launch_any_inst<MB, 1, 1>(p);
-    case 22: return launch_any_inst<MB, 2, 2>(p);
-    case 21: return launch_any_inst<MB, 2, 1>(p);
-    default: return launch_any_inst<MB, 4, 1>(p);
+    case 14: return launch_any_inst<MB, 1, 4>(p, sums);
+    case 24: return launch_any_inst<MB, 2, 4>(p, sums);
+    case 44: return launch_any_inst<MB, 4, 4>(p, sums);
+    case 11: return launch_any_inst<MB, 1, 1>(p, sums);
+    case 22: return launch_any_inst<MB, 2, 2>(p, sums);
+    case 21: return launch_any_inst<MB, 2, 1>(p, sums);
+    default: return launch_any_inst<MB, 4, 1>(p, sums);
   }
 }
-int launch_any(const AnyPlan &p) {
+int launch_any(const AnyPlan &p, const AnySums &sums) {
   switch (p.mb) {
-    case 1: return launch_any_mb<1>(p);
-    case 2: return launch_any_mb<2>(p);
-    case 3: return launch_any_mb<3>(p);
-    default: return launch_any_mb<4>(p);
+    case 1: return launch_any_mb<1>(p, sums);
+    case 2: return launch_any_mb<2>(p, sums);
+    case 3: return launch_any_mb<3>(p, sums);
+    default: return launch_any_mb<4>(p, sums);
   }
 }
 
-int run_any(AnyPlan &p, const char *tag, int m, int n, int k) {
+// the packing of a plan's filters, into scratch
+int any_pack_of(const AnyPlan &p, const float *w, AnyPack *pack) {
+  const AnyArgs &a = p.args;
+  void *wp = nullptr;
+  TDH_TRY(ws_take(p.pack_bytes, &wp));
+  const int rs = std::min(a.wm, a.wk);
+  pack->w = w; pack->wp = static_cast<uintx4 *>(wp);
+  pack->M = a.M; pack->KC = a.KC; pack->m_pad = a.m_pad; pack->wm = a.wm; pack->wk = a.wk;
+  pack->total  = ceil_div(a.KC, 8) * rs * a.m_pad;
+  pack->blocks = ceil_div(pack->total, 256);
+  pack->div_m = FastDiv(a.m_pad); pack->div_rs = FastDiv(rs);
+  return TDH_OK;
+}
+
+int run_any(AnyPlan &p, const char *tag, int m, int n, int k, const AnyPack *packed, const AnySums *with) {
   AnyArgs &a = p.args;
-  {
-    void *wp = nullptr;
-    TDH_TRY(ws_take(p.pack_bytes, &wp));
-    const int rs = std::min(a.wm, a.wk), total = ceil_div(a.KC, 8) * rs * a.m_pad;
-    ProfScope prof("conv_any_pack", 4.0 * a.M * a.KC * rs + static_cast<double>(p.pack_bytes), WORK_BYTE);
-    TDH_LAUNCH(any_pack_kernel, dim3(ceil_div(total, 256)), dim3(256), 0, ctx().stream, a.w, static_cast<uintx4 *>(wp), a.M,
-               a.KC, a.m_pad, rs, a.wm, a.wk, total, FastDiv(a.m_pad), FastDiv(rs));
+  AnyPack pack;
+  if (packed) {
+    pack = *packed;
+  } else {
+    TDH_TRY(any_pack_of(p, a.w, &pack));
+    ProfScope prof("conv_any_pack", 4.0 * a.M * a.KC * std::min(a.wm, a.wk) + static_cast<double>(p.pack_bytes), WORK_BYTE);
+    TDH_LAUNCH(any_pack_kernel, dim3(pack.blocks), dim3(256), 0, ctx().stream, pack);
     TDH_LAUNCH_CHECK();
-    a.wp = wp;
   }
+  a.wp = pack.wp;
+  AnySums sums{};
+  if (with) sums = *with;
+  sums.first_x = static_cast<int>(p.grid.x);
   ProfScope prof(tag, m, n, k);
-  return launch_any(p);
+  return launch_any(p, sums);
 }
 
 }  // namespace
@@ -670,14 +666,20 @@ int conv_any_fwd_run(const ConvShape &c, const float *x, const float *w, const f
   if (!p.ok) return set_error(TDH_ERR_INVALID, "conv_any_fwd_run: no plan for this shape");
   finish_args(p.args);
   p.args.in = x; p.args.w = w; p.args.bias = bias; p.args.out = out; p.args.act_out = act_out; p.args.act_kind = act_kind;
-  return run_any(p, "conv_fwd_any_x3", c.Kc, c.batch * c.OH * c.OW, c.C * c.R * c.S);
+  return run_any(p, "conv_fwd_any_x3", c.Kc, c.batch * c.OH * c.OW, c.C * c.R * c.S, nullptr, nullptr);
 }
-int conv_any_dx_run(const ConvShape &c, const float *dy, const float *w, float *dx, ActGrad ag) {
+int conv_any_dx_pack(const ConvShape &c, const float *w, AnyPack *pack) {
+  const AnyPlan &p = backward_plan(c);
+  if (!p.ok) return set_error(TDH_ERR_INVALID, "conv_any_dx_pack: no plan for this shape");
+  return any_pack_of(p, w, pack);
+}
+int conv_any_dx_run(const ConvShape &c, const float *dy, const float *w, float *dx, ActGrad ag, const AnyPack *packed,
+                    const AnySums *with) {
   AnyPlan p = backward_plan(c);
   if (!p.ok) return set_error(TDH_ERR_INVALID, "conv_any_dx_run: no plan for this shape");
   finish_args(p.args);
   p.args.in = dy; p.args.w = w; p.args.out = dx; p.args.ag = ag;
-  return run_any(p, "conv_dx_any_x3", c.C, c.batch * c.H * c.W, std::max(1, c.Kc * c.R * c.S / (c.sh * c.sw)));
+  return run_any(p, "conv_dx_any_x3", c.C, c.batch * c.H * c.W, std::max(1, c.Kc * c.R * c.S / (c.sh * c.sw)), packed, with);
 }
 
 }  // namespace tdh

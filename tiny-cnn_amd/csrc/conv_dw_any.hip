@@ -16,7 +16,7 @@
 // Reference: conv2d_op_internal.h:79-158.
 #include <algorithm>
 
-#include "gemm_mfma.h"
+#include "conv_any.h"
 
 namespace tdh {
 
@@ -42,7 +42,12 @@ struct DwAnyArgs {
 
 // MB blocks of 16 channels; NB blocks of 16 columns to each of the four waves; CH pixels a chunk
 template <int MB, int NB, int CH>
-__global__ void __launch_bounds__(256, 2) conv_dw_any_kernel(const DwAnyArgs a) {
+__global__ void __launch_bounds__(256, 2) conv_dw_any_kernel(const DwAnyArgs a, const AnyPack pack) {
+  if (static_cast<int>(blockIdx.x) >= pack.first_x) {   // (behind the slices)
+    const int block = ((static_cast<int>(blockIdx.x) - pack.first_x) * gridDim.y + blockIdx.y) * gridDim.z + blockIdx.z;
+    if (block < pack.blocks) any_pack_block(pack, block);
+    return;
+  }
   constexpr int DYP = CH + 4;        // (sixteen channels' 16-byte reads cover all banks)
   constexpr int ROWS = 256 / CH;     // channels of dY staged side by side
   extern __shared__ __align__(16) int dwa_lds[];
@@ -297,7 +302,7 @@ const DwAnyPlan &make_plan(const ConvShape &c, bool with_db) {
 }
 
 template <int MB, int NB, int CH>
-int launch_inst(const DwAnyPlan &p) {
+int launch_inst(const DwAnyPlan &p, const AnyPack &pack) {
   auto kernel = conv_dw_any_kernel<MB, NB, CH>;
   if (p.lds_bytes > 64 * 1024) {
     static size_t raised = 0;
@@ -307,24 +312,25 @@ int launch_inst(const DwAnyPlan &p) {
       raised = p.lds_bytes;
     }
   }
-  TDH_LAUNCH(kernel, p.grid, dim3(256), p.lds_bytes, ctx().stream, p.args);
+  const unsigned extra = ceil_div(pack.blocks, static_cast<int>(p.grid.y * p.grid.z));
+  TDH_LAUNCH(kernel, dim3(p.grid.x + extra, p.grid.y, p.grid.z), dim3(256), p.lds_bytes, ctx().stream, p.args, pack);
   TDH_LAUNCH_CHECK();
   return TDH_OK;
 }
 template <int MB, int NB>
-int launch_nb(const DwAnyPlan &p) {
+int launch_nb(const DwAnyPlan &p, const AnyPack &pack) {
   switch (p.ch) {
-    case 64: return launch_inst<MB, NB, 64>(p);
-    case 128: return launch_inst<MB, NB, 128>(p);
-    default: return launch_inst<MB, NB, 256>(p);
+    case 64: return launch_inst<MB, NB, 64>(p, pack);
+    case 128: return launch_inst<MB, NB, 128>(p, pack);
+    default: return launch_inst<MB, NB, 256>(p, pack);
   }
 }
 template <int MB>
-int launch_mb(const DwAnyPlan &p) {
+int launch_mb(const DwAnyPlan &p, const AnyPack &pack) {
   switch (p.nb) {
-    case 1: return launch_nb<MB, 1>(p);
-    case 2: return launch_nb<MB, 2>(p);
-    default: return launch_nb<MB, 4>(p);
+    case 1: return launch_nb<MB, 1>(p, pack);
+    case 2: return launch_nb<MB, 2>(p, pack);
+    default: return launch_nb<MB, 4>(p, pack);
   }
 }
 
@@ -355,7 +361,8 @@ size_t conv_dw_any_most_bytes(const ConvShape &c, bool with_db) {
   const long slices  = std::min<long>((static_cast<long>(c.batch) * c.OH * c.OW + 63) / 64, std::max(1L, 1024 / tiles));
   return ws_align(sizeof(float) * static_cast<size_t>(slices) * c.Kc * columns);
 }
-int conv_dw_any_run(const ConvShape &c, const float *x, const float *dy, bool with_db, const float **partial, int *slices) {
+int conv_dw_any_run(const ConvShape &c, const float *x, const float *dy, bool with_db, const float **partial, int *slices,
+                    const AnyPack *pack) {
   DwAnyPlan p = make_plan(c, with_db);
   if (!p.ok) return set_error(TDH_ERR_INVALID, "conv_dw_any_run: no plan for this shape");
   DwAnyArgs &a = p.args;
@@ -366,12 +373,15 @@ int conv_dw_any_run(const ConvShape &c, const float *x, const float *dy, bool wi
   a.div_sx = FastDiv(c.sw); a.div_rs = FastDiv(c.R * c.S); a.div_s = FastDiv(c.S);
   *partial = a.partial;
   *slices  = p.slices;
+  AnyPack side{};
+  if (pack) side = *pack;
+  side.first_x = static_cast<int>(p.grid.x);
   ProfScope prof(with_db ? "conv_dw_db_any" : "conv_dw_any", a.M, a.N, a.pixels);
   switch (p.mb) {
-    case 1: return launch_mb<1>(p);
-    case 2: return launch_mb<2>(p);
-    case 3: return launch_mb<3>(p);
-    default: return launch_mb<4>(p);
+    case 1: return launch_mb<1>(p, side);
+    case 2: return launch_mb<2>(p, side);
+    case 3: return launch_mb<3>(p, side);
+    default: return launch_mb<4>(p, side);
   }
 }
 

@@ -500,6 +500,20 @@ gemm_mfma_kernel(const AOp a_op, const BOp b_op, const Epi epi, const int M, con
   }
 }
 
+// dW with the bias gradient as column crs
+struct EpiDwDb {
+  float *dw, *db;
+  int crs, accumulate;
+  struct Col {
+    int n;
+  };
+  __device__ __forceinline__ float *at(int m, const Col &c) const { return c.n < crs ? dw + m * crs + c.n : db + m; }
+  __device__ __forceinline__ Col col(int n) const { return {n}; }
+  __device__ __forceinline__ float prior(int m, const Col &c) const { return accumulate ? *at(m, c) : 0.0f; }
+  __device__ __forceinline__ void store(int m, const Col &c, float v, float before) const { *at(m, c) = v + before; }
+  __device__ __forceinline__ void store(int m, const Col &c, float v) const { store(m, c, v, prior(m, c)); }
+};
+
 // Adds the K-split partial tiles and applies the epilogue. A workgroup owns 32 consecutive
 // outputs; its eight 32-lane groups each add every eighth slice (g, g+8, ...) and the eight
 // group sums are then added in group order, so the summation tree depends on the split
