@@ -104,3 +104,47 @@ def test_gradients_and_updates_of_one_group_and_of_several(T, O, W, name, batch,
     assert opts[0].b1_t == opts[1].b1_t == opts[2].b1_t and opts[0].b2_t == opts[1].b2_t == opts[2].b2_t
     for m in (net, replay, layered):
         m.close()
+
+
+HELD_NETS = {
+    # 16 rows a thread are the most: 24 pieces of a row, 16 ranges of channels
+    "k256": ([("conv", 8, 8, 6, 3, 8, False), ("act", "tanh"), ("maxpool", 6, 6, 8, 2), ("conv", 3, 3, 8, 3, 256, False),
+              ("act", "relu"), ("fc", 256, 5), ("act", "softmax")], "ce_multiclass", "sgd"),
+    "k257": ([("conv", 8, 8, 6, 3, 8, False), ("act", "tanh"), ("maxpool", 6, 6, 8, 2), ("conv", 3, 3, 8, 3, 257, False),
+              ("act", "relu"), ("fc", 257, 5), ("act", "softmax")], "ce_multiclass", "sgd"),
+    # one output channel; two activations in front, the nearer one in a phase of its own
+    "k1": ([("conv", 8, 8, 6, 3, 8, False), ("act", "tanh"), ("act", "sigmoid"), ("conv", 6, 6, 8, 6, 1, False),
+            ("fc", 1, 2)], "mse", "sgd"),
+    # no layer between the two; rows of 392 values in 128 lanes, an uneven last range of channels
+    "direct": ([("conv", 9, 9, 6, 3, 8, False), ("conv", 7, 7, 8, 7, 61, False), ("act", "tanh"), ("act", "leaky_relu", (0.1, 0.0)),
+                ("fc", 61, 9), ("act", "tanh"), ("fc", 9, 3), ("act", "sigmoid")], "mse", "adam"),
+    # a split net whose second convolution's gradient takes the scratch area next; one row more than a wave of pieces
+    "behind": ([("conv", 14, 14, 1, 3, 6, False), ("act", "tanh"), ("conv", 12, 12, 6, 3, 16, False), ("act", "sigmoid"),
+                ("avepool", 10, 10, 16, 2), ("act", "tanh"), ("conv", 5, 5, 16, 5, 20, False),
+                ("fc", 20, 4)], "mse", "momentum"),
+    "act_only": ([("conv", 8, 8, 2, 3, 6, False), ("act", "tanh"), ("conv", 6, 6, 6, 3, 13, False), ("act", "tanh"),
+                  ("conv", 4, 4, 13, 4, 33, False), ("act", "tanh"), ("fc", 33, 4)], "mse", "adagrad"),
+    # rows that are no multiple of four values
+    "odd": ([("conv", 8, 8, 6, 3, 9, False), ("act", "tanh"), ("maxpool", 6, 6, 9, 2), ("conv", 3, 3, 9, 3, 12, False),
+             ("act", "tanh"), ("fc", 12, 3)], "mse", "sgd"),
+}
+
+
+@pytest.mark.parametrize("batch", [1, 5, 90])
+@pytest.mark.parametrize("name", list(HELD_NETS))
+def test_filters_held_in_registers(T, O, W, name, batch):
+    """Every tensor of nets with a convolution whose window is its whole input, against the oracle; two passes, so that the
+    second one runs on what the first one left behind."""
+    spec, params, x, t, batch, loss, kind, _, net, ref = build(T, O, W, name, batch, SAMPLE | FUSE, nets=HELD_NETS)
+    xd, td = T.to_device(x), T.to_device(t)
+    opt = T.opt_desc(kind, alpha=1e-3)
+    net.train_step(opt, loss, batch, xd, td)
+    ref.train_step(O.opt_desc(kind, alpha=1e-3), loss, x, t)
+    net.train_step(None, loss, batch, xd, td, do_update=False)
+    ref.train_step(O.opt_desc(kind), loss, x, t, do_update=False)
+    for i, l in enumerate(spec):
+        assert_close(net.layer_out(i, batch), ref.layer_out(i, batch), what=f"layer {i} output")
+        assert_close(net.layer_dx(i, batch), ref.layer_dx(i, batch), what=f"layer {i} dX")
+        if net.param_size(i, 0):
+            assert_close(net.layer_grad(i, 0), ref.layer_dw(i), what=f"layer {i} dW")
+    net.close()

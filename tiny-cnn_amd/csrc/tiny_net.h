@@ -62,6 +62,9 @@ struct TinyPlan {
   int lds_g0, lds_g1, lds_w, lds_pad, lds_floats;   // lds_pad: the zero-framed dY
   int n_mfma, mfma_layers[TINY_MAX_LAYERS];   // the layers with operands to stage for the matrix cores
   int mf_ahead;                // the layer (> 0) whose filters wait in registers until the layer in front of it runs, or -1
+  // the layer whose filters wait in registers from layer held_from on (held_chain), or 0; how they lie there (Held)
+  int held, held_from, held_shift, held_rows;   // (held_from: a convolution on the matrix cores)
+  FastDiv d_held_rows;
   float mse_factor;            // 2 / outputs
   float *dloss;                // memory: gradient w.r.t. the net's output [batch][out_size]
   double flop_per_sample;

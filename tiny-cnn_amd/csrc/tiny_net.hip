@@ -76,6 +76,17 @@ __device__ __forceinline__ float wave_sum_63(float v) {
   v = step(v, integral_constant<int, 0x142>(), integral_constant<int, 0xa>());   // row_bcast:15
   return step(v, integral_constant<int, 0x143>(), integral_constant<int, 0xc>());   // row_bcast:31
 }
+// sum over each sixteen lanes, in all of them
+__device__ __forceinline__ float row_sum(float v) {
+  auto step = [](float x, auto ctrl) {
+    return x + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), ctrl(), 0xf, 0xf, false));
+  };
+  using std::integral_constant;
+  v = step(v, integral_constant<int, 0x128>());   // row_ror:8
+  v = step(v, integral_constant<int, 0x124>());
+  v = step(v, integral_constant<int, 0x122>());
+  return step(v, integral_constant<int, 0x121>());
+}
 // lanes per value, so that `values` of them make at least two rounds of the workgroup busy
 // and no lane's share of `length` terms is empty
 __device__ __forceinline__ int group_for(int values, int length) {
@@ -115,6 +126,51 @@ __device__ __forceinline__ void fill_lds(float *dst, const float *__restrict__ s
 // stay LDS addresses.
 #define TN_INLINE __device__ __forceinline__
 
+// Where a layer's outputs go, and those of a pointwise activation behind it that runs in the same phase (later layers
+// read that one's outputs only)
+struct FwdOut {
+  float *out, *gout;      // LDS: what the next layer reads; memory: this layer's
+  int act;                // the activation's, or TDH_ACT_NONE
+  float p0, *gact;
+  __device__ __forceinline__ void operator()(const int i, float v) const {
+    gout[i] = v;
+    if (act != TDH_ACT_NONE) {
+      v = tn_act_fwd(act, p0, v);
+      gact[i] = v;
+    }
+    out[i] = v;
+  }
+};
+// The same on the way back: a gradient with respect to a layer's input (gdx: its place in memory, or NULL), and through
+// the activation in front of that layer
+struct BwdOut {
+  float *dx, *gdx;
+  int act;
+  float p0, *gact;
+  const float *y;         // the activation's outputs
+  __device__ __forceinline__ void operator()(const int i, float v) const {
+    if (gdx) gdx[i] = v;
+    if (act != TDH_ACT_NONE) {
+      v = tn_act_bwd(act, p0, y[i], v);
+      if (gact) gact[i] = v;
+    }
+    dx[i] = v;
+  }
+};
+TN_INLINE FwdOut fwd_out(const TinyPlan *__restrict__ plan, float *lds, const int li, const int s, const bool with_act) {
+  const TinyLayer *L = &plan->l[li], *A = with_act ? L + 1 : L;   // (a pointwise activation has its input's size)
+  const size_t at = static_cast<size_t>(s) * L->out_size;
+  return {lds + A->lds_out, L->out + at, with_act ? A->act : TDH_ACT_NONE, A->p0, A->out + at};
+}
+TN_INLINE BwdOut bwd_out(const TinyPlan *__restrict__ plan, const float *lds, float *dx, const int li, const int s,
+                         const bool with_act) {
+  const TinyLayer *L = &plan->l[li], *A = with_act ? L - 1 : L;
+  const size_t at = static_cast<size_t>(s) * L->in_size;
+  return {dx, L->dx ? L->dx + at : nullptr, with_act ? A->act : TDH_ACT_NONE, A->p0, A->dx ? A->dx + at : nullptr, lds + A->lds_out};
+}
+__host__ __device__ inline bool is_pointwise(const TinyLayer &L) { return L.kind == TDH_L_ACT && L.act != TDH_ACT_SOFTMAX; }
+__host__ __device__ inline bool is_pool(const TinyLayer &L) { return L.kind == TDH_L_MAXPOOL || L.kind == TDH_L_AVEPOOL; }
+
 // ------------------------------------------------------------------ forward
 TN_INLINE void conv_fwd(const TinyLayer *__restrict__ Lp, const float *in, float *out, float *__restrict__ gout) {
   const int C = Lp->C, H = Lp->H, W = Lp->W, K = Lp->K, OH = Lp->OH, OW = Lp->OW, R = Lp->R, S = Lp->S;
@@ -148,7 +204,7 @@ TN_INLINE void conv_fwd(const TinyLayer *__restrict__ Lp, const float *in, float
 
 // fully_connected_op_internal.h:15-36: out[i] = sum_c W[c*out + i] * in[c] + b[i]; the sum over
 // c is split over a group of lanes
-TN_INLINE void fc_fwd(const TinyLayer *__restrict__ Lp, const float *in, float *out, float *__restrict__ gout) {
+TN_INLINE void fc_fwd(const TinyLayer *__restrict__ Lp, const float *in, const FwdOut out) {
   const int n_out = Lp->out_size, n_in = Lp->in_size, has_bias = Lp->has_bias;
   const float *__restrict__ w = Lp->w;
   const float *__restrict__ b = Lp->b;
@@ -161,15 +217,14 @@ TN_INLINE void fc_fwd(const TinyLayer *__restrict__ Lp, const float *in, float *
     sum = group_sum(sum, g);
     if (it < total && part == 0) {
       if (has_bias) sum += b[i];
-      out[i]  = sum;
-      gout[i] = sum;
+      out(i, sum);
     }
   }
 }
 
 // max_pooling_layer.h:195-222 + maxpool_op_internal.h:16-40: windows clipped at the edges,
 // strict '>' from lowest(), the record is the flat CHW input index (0 when nothing wins)
-TN_INLINE void maxpool_fwd(const TinyLayer *__restrict__ Lp, const float *in, float *out, float *__restrict__ gout,
+TN_INLINE void maxpool_fwd(const TinyLayer *__restrict__ Lp, const float *in, const FwdOut out,
                            int32_t *__restrict__ gargmax) {
   const int C = Lp->C, H = Lp->H, W = Lp->W, OH = Lp->OH, OW = Lp->OW, R = Lp->R, S = Lp->S, sh = Lp->sh, sw = Lp->sw;
   const FastDiv d_plane = Lp->d_oplane, d_ow = Lp->d_ow;
@@ -191,14 +246,13 @@ TN_INLINE void maxpool_fwd(const TinyLayer *__restrict__ Lp, const float *in, fl
           idx  = j;
         }
       }
-    out[o]     = best;
-    gout[o]    = best;
+    out(o, best);
     gargmax[o] = idx;
   }
 }
 
 // average_pooling_layer.h:25-55: value = sum(window) * (W[c] * scale) + b[c]
-TN_INLINE void avepool_fwd(const TinyLayer *__restrict__ Lp, const float *in, float *out, float *__restrict__ gout) {
+TN_INLINE void avepool_fwd(const TinyLayer *__restrict__ Lp, const float *in, const FwdOut out) {
   const int C = Lp->C, H = Lp->H, W = Lp->W, OH = Lp->OH, OW = Lp->OW, R = Lp->R, S = Lp->S, sh = Lp->sh, sw = Lp->sw;
   const FastDiv d_plane = Lp->d_oplane, d_ow = Lp->d_ow;
   const float scale = Lp->scale;
@@ -217,8 +271,7 @@ TN_INLINE void avepool_fwd(const TinyLayer *__restrict__ Lp, const float *in, fl
     const float weight = w[c] * scale;
     value *= weight;
     value += b[c];
-    out[o]  = value;
-    gout[o] = value;
+    out(o, value);
   }
 }
 
@@ -305,7 +358,7 @@ TN_INLINE void conv_bwd_dx(const TinyLayer *__restrict__ Lp, const float *dy, fl
 }
 
 // fully_connected_op_internal.h:38-71
-TN_INLINE void fc_bwd_dx(const TinyLayer *__restrict__ Lp, const float *dy, float *dx, float *__restrict__ gdx) {
+TN_INLINE void fc_bwd_dx(const TinyLayer *__restrict__ Lp, const float *dy, const BwdOut dx) {
   const int n_out = Lp->out_size, n_in = Lp->in_size;
   const float *__restrict__ w = Lp->w;
   for (int c = threadIdx.x; c < n_in; c += TN_THREADS) {
@@ -320,14 +373,12 @@ TN_INLINE void fc_bwd_dx(const TinyLayer *__restrict__ Lp, const float *dy, floa
       for (int j = 0; j < 8; ++j) acc += dy[i + j] * wv[j];
     }
     for (; i < n_out; ++i) acc += dy[i] * wr[i];
-    dx[c] = acc;
-    if (gdx) gdx[c] = acc;
+    dx(c, acc);
   }
 }
 // maxpool_op_internal.h:42-57: an input takes the gradient of the LAST window that contains it
 // when that window's record names it
-TN_INLINE void maxpool_bwd(const TinyLayer *__restrict__ Lp, const float *dy, const int32_t *gargmax, float *dx,
-                           float *__restrict__ gdx) {
+TN_INLINE void maxpool_bwd(const TinyLayer *__restrict__ Lp, const float *dy, const int32_t *gargmax, const BwdOut dx) {
   const int C = Lp->C, H = Lp->H, W = Lp->W, OH = Lp->OH, OW = Lp->OW, R = Lp->R, S = Lp->S, sh = Lp->sh, sw = Lp->sw;
   const FastDiv d_plane = Lp->d_iplane, d_w = Lp->d_w;
   const int total = C * H * W;
@@ -338,14 +389,12 @@ TN_INLINE void maxpool_bwd(const TinyLayer *__restrict__ Lp, const float *dy, co
     const int ox = min(OW - 1, static_cast<int>(xx) / sw), oy = min(OH - 1, static_cast<int>(yy) / sh);
     const bool covered = (static_cast<int>(xx) < ox * sw + S) && (static_cast<int>(yy) < oy * sh + R);
     const int outi = covered ? (OH * c + oy) * OW + ox : 0;
-    const float v  = (gargmax[outi] == e) ? dy[outi] : 0.0f;
-    dx[e] = v;
-    if (gdx) gdx[e] = v;
+    dx(e, (gargmax[outi] == e) ? dy[outi] : 0.0f);
   }
 }
 
 // average_pooling_layer.h:58-106
-TN_INLINE void avepool_bwd_dx(const TinyLayer *__restrict__ Lp, const float *dy, float *dx, float *__restrict__ gdx) {
+TN_INLINE void avepool_bwd_dx(const TinyLayer *__restrict__ Lp, const float *dy, const BwdOut dx) {
   const int C = Lp->C, H = Lp->H, W = Lp->W, OH = Lp->OH, OW = Lp->OW, R = Lp->R, S = Lp->S, sh = Lp->sh, sw = Lp->sw;
   const FastDiv d_plane = Lp->d_iplane, d_w = Lp->d_w;
   const float scale = Lp->scale;
@@ -365,9 +414,7 @@ TN_INLINE void avepool_bwd_dx(const TinyLayer *__restrict__ Lp, const float *dy,
       oy = static_cast<int>(iy) < R ? 0 : (static_cast<int>(iy) - R + sh) / sh;
     }
     const float weight = w[c] * scale;
-    const float v      = weight * dy[(c * OH + oy) * OW + ox];
-    dx[e] = v;
-    if (gdx) gdx[e] = v;
+    dx(e, weight * dy[(c * OH + oy) * OW + ox]);
   }
 }
 TN_INLINE void act_bwd(const TinyLayer *__restrict__ Lp, const float *y, const float *dy, float *dx,
@@ -643,10 +690,9 @@ constexpr int MFMA_AHEAD = 4;   // filter values a thread holds for the layer wh
 __host__ __device__ inline int mfma_steps(const int n_k) { return ((n_k + 15) >> 4) << 2; }
 // (a row pitch of 4 * odd floats: sixteen rows read 16 bytes each from different banks, two rows a bank group)
 __host__ __device__ inline int mfma_pitch(const int n_k) { return (4 * mfma_steps(n_k)) | 4; }
-template <int T>
+template <int T, typename Out>
 TN_INLINE void conv_mfma(const float *src, const float *a, const int *koff, const int M, const int n_k,
-                         const int plane, const FastDiv d_row, const int src_pitch, const float *bias,
-                         float *out, float *__restrict__ gout) {
+                         const int plane, const FastDiv d_row, const int src_pitch, const float *bias, const Out out) {
   const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
   const int steps = mfma_steps(n_k), pitch = mfma_pitch(n_k), groups = steps >> 2;
   const int m_tiles = (M + 15) >> 4, p_tiles = (plane + 15) >> 4, p_items = (p_tiles + T - 1) / T;
@@ -703,14 +749,69 @@ TN_INLINE void conv_mfma(const float *src, const float *a, const int *koff, cons
 #pragma unroll
       for (int j = 0; j < T; ++j) {
         const int p = (pi * T + j) * 16 + r;
-        if (p < plane) {
-          const float v = bias ? acc[j][i] + bv : acc[j][i];
-          out[m * plane + p] = v;
-          if (gout) gout[m * plane + p] = v;
-        }
+        if (p < plane) out(m * plane + p, bias ? acc[j][i] + bv : acc[j][i]);
       }
     }
   }
+}
+// The same with a tile a wave where there are fewer tiles than waves: `splits` waves take a tile, a range of k each, and
+// leave their sums in `scratch` ([split][tile][i][lane]), from where all threads take the outputs: the chain of a tile's
+// products is shorter, and what follows them (an activation) has all the workgroup's lanes. LeNet-5's second convolution
+// with the tanh behind it, 7 tiles: 3.9 us, in two phases of whole tiles 4.6.
+TN_INLINE void conv_mfma_split(const TinyLayer *__restrict__ L, const float *src, const float *a, const int *koff,
+                               const float *bias, const FwdOut out, float *scratch) {
+  const int M = L->K, n_k = L->C * L->R * L->S, plane = L->OH * L->OW, src_pitch = L->W;
+  const FastDiv d_plane = L->d_oplane, d_row = L->d_ow;
+  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  const int steps = mfma_steps(n_k), pitch = mfma_pitch(n_k), groups = steps >> 2;
+  const int p_tiles = (plane + 15) >> 4, tiles = ((M + 15) >> 4) * p_tiles;
+  int log_splits = 0;
+  while ((2 << log_splits) * tiles <= TN_WAVES && (2 << log_splits) <= groups) ++log_splits;
+  const int splits = 1 << log_splits, item = wave_index();
+  if (item < tiles << log_splits) {
+    int part = 0, mt = 0, pt = item;   // (at most sixteen items: no divisions)
+    while (pt >= tiles) { pt -= tiles; ++part; }
+    while (pt >= p_tiles) { pt -= p_tiles; ++mt; }
+    const int share = (groups + splits - 1) >> log_splits, g0 = part * share, g1 = min(groups, g0 + share);
+    const int k_left = n_k - q * steps;   // this lane's steps from k_left on are padding
+    uint32_t py, px;
+    d_row.divmod(min(pt * 16 + r, plane - 1), py, px);
+    const float *sp  = src + static_cast<int>(py) * src_pitch + static_cast<int>(px);
+    const float4 *a4 = reinterpret_cast<const float4 *>(a + min(mt * 16 + r, M - 1) * pitch + q * steps);
+    const int4 *k4   = reinterpret_cast<const int4 *>(koff + q * steps);
+    tn_f4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = acc0;   // (two chains)
+    for (int g = g0; g < g1; ++g) {
+      const int4 ko   = k4[g];
+      const float4 ac = a4[g];
+      const float bc[4] = {sp[ko.x], sp[ko.y], sp[ko.z], sp[ko.w]};
+      const int st = 4 * g;   // (a zero filter value times an infinity would be a NaN)
+      acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(ac.x, st < k_left ? bc[0] : 0.0f, acc0, 0, 0, 0);
+      acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(ac.y, st + 1 < k_left ? bc[1] : 0.0f, acc1, 0, 0, 0);
+      acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(ac.z, st + 2 < k_left ? bc[2] : 0.0f, acc0, 0, 0, 0);
+      acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(ac.w, st + 3 < k_left ? bc[3] : 0.0f, acc1, 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) scratch[(item * 4 + i) * 64 + lane] = acc0[i] + acc1[i];
+  }
+  lds_barrier();
+  for (int e = threadIdx.x; e < M * plane; e += TN_THREADS) {
+    uint32_t m, p;
+    d_plane.divmod(e, m, p);
+    const int tile = (m >> 4) * p_tiles + (p >> 4);
+    const float *sum = scratch + (tile * 4 + (m & 3)) * 64 + ((m >> 2) & 3) * 16 + (p & 15);
+    float v = sum[0];
+    for (int o = 1; o < splits; ++o) v += sum[o * tiles * 256];
+    out(e, bias ? v + bias[m] : v);
+  }
+}
+// the forward pass of a layer with operands in LDS
+TN_INLINE void conv_fwd_mfma(const TinyLayer *__restrict__ L, const float *lds, float *scratch, const FwdOut out) {
+  const float *in = lds + L->lds_in, *fa = lds + L->mf_fwd_w, *fb = L->has_bias ? lds + L->mf_fwd_b : nullptr;
+  const int *fk = reinterpret_cast<const int *>(lds + L->mf_fwd_ko);
+  const int K = L->K, n_k = L->C * L->R * L->S, plane = L->OH * L->OW;
+  // (several pixel tiles a wave when there are more tiles than waves)
+  if (((K + 15) >> 4) * ((plane + 15) >> 4) > TN_WAVES) conv_mfma<4>(in, fa, fk, K, n_k, plane, L->d_ow, L->W, fb, out);
+  else conv_mfma_split(L, in, fa, fk, fb, out, scratch);
 }
 // The operand and the offset table of the input gradient described at TinyLayer::mf_dx_w, from
 // the filter values the thread still holds (mfma_filters_load: value j is element
@@ -733,10 +834,8 @@ TN_INLINE void mfma_dx_operand_store(const TinyLayer *__restrict__ L, const floa
     a[(ci * S + wx) * pitch + co * R + wy] = (tbl && !tbl[ci * K + co]) ? 0.0f : v[j];
   }
   const int pad = pitch - n_k;
-  for (int idx = threadIdx.x; idx < rows * pad; idx += TN_THREADS) {
-    const int row = idx / pad;
-    a[row * pitch + n_k + idx - row * pad] = 0.0f;
-  }
+  for (int row = threadIdx.x >> 5; row < rows; row += TN_THREADS / 32)   // (pad <= 20)
+    if (static_cast<int>(threadIdx.x & 31) < pad) a[row * pitch + n_k + (threadIdx.x & 31)] = 0.0f;
   for (int k = threadIdx.x; k < k4; k += TN_THREADS) {
     const int co = k / R, wy = k - co * R;
     ko[k] = k < n_k ? co * PP + (R - 1 - wy) * PW : 0;
@@ -771,17 +870,18 @@ TN_INLINE void mfma_filters_load(const TinyLayer *__restrict__ L, const int e0, 
 }
 TN_INLINE void mfma_filters_store(const TinyLayer *__restrict__ L, const int e0, const float (&v)[MFMA_AHEAD],
                                   const float bias, float *lds) {
-  const int K = L->K, taps = L->R * L->S, n_k = L->C * taps, nw = K * n_k, pitch = mfma_pitch(n_k);
+  const int K = L->K, n_k = L->C * L->R * L->S, nw = K * n_k, pitch = mfma_pitch(n_k);
   const uint8_t *__restrict__ tbl = L->tbl;
   float *fa = lds + L->mf_fwd_w;
 #pragma unroll
   for (int j = 0; j < MFMA_AHEAD; ++j) {
     const int e = e0 + j * TN_THREADS + threadIdx.x;
     if (e >= nw) continue;
-    uint32_t co, k, ci, t;
+    uint32_t co, k;
     L->d_nk.divmod(e, co, k);
-    L->d_taps.divmod(k, ci, t);
-    fa[co * pitch + k] = (tbl && !tbl[ci * K + co]) ? 0.0f : v[j];
+    bool on = true;
+    if (tbl) on = tbl[L->d_taps.div(k) * K + co];
+    fa[co * pitch + k] = on ? v[j] : 0.0f;
   }
   if (e0 == 0 && L->has_bias && static_cast<int>(threadIdx.x) < K) lds[L->mf_fwd_b + threadIdx.x] = bias;
 }
@@ -791,10 +891,9 @@ TN_INLINE void mfma_tables(const TinyLayer *__restrict__ L, float *lds) {
   const int n_k = L->C * taps, pitch = mfma_pitch(n_k), k4 = 4 * mfma_steps(n_k), pad = pitch - n_k;
   float *fa = lds + L->mf_fwd_w;
   int *ko   = reinterpret_cast<int *>(lds + L->mf_fwd_ko);
-  for (int idx = threadIdx.x; idx < K * pad; idx += TN_THREADS) {
-    const int row = idx / pad;
-    fa[row * pitch + n_k + idx - row * pad] = 0.0f;
-  }
+  // (pad <= 20)
+  for (int row = threadIdx.x >> 5; row < K; row += TN_THREADS / 32)
+    if (static_cast<int>(threadIdx.x & 31) < pad) fa[row * pitch + n_k + (threadIdx.x & 31)] = 0.0f;
   for (int k = threadIdx.x; k < k4; k += TN_THREADS) {
     uint32_t ci, t, wy, wx;
     L->d_taps.divmod(min(k, n_k - 1), ci, t);
@@ -803,11 +902,11 @@ TN_INLINE void mfma_tables(const TinyLayer *__restrict__ L, float *lds) {
   }
 }
 // every layer but the one whose filters travel in registers (`ahead`, or -1): when the kernel starts
-TN_INLINE void stage_mfma_operands(const TinyPlan *__restrict__ plan, float *lds, const int ahead) {
+TN_INLINE void stage_mfma_operands(const TinyPlan *__restrict__ plan, float *lds, const int m, const int ahead) {
   const int n = plan->n_mfma;
   for (int q = 0; q < n; ++q) {   // (the plan lists them: walking every layer is a scalar load and a wait each)
     const int li = plan->mfma_layers[q];
-    if (li == ahead) continue;
+    if (li == ahead || li < m) continue;
     const TinyLayer *__restrict__ L = &plan->l[li];
     mfma_tables(L, lds);
     const int nw = L->K * L->C * L->R * L->S;
@@ -1018,6 +1117,222 @@ TN_INLINE void conv_bwd_dx_matvec(const TinyLayer *__restrict__ Lp, const float 
   }
 }
 
+// The same product with its filters held in registers: read once, while the layers in front run, and used on the way
+// forward and on the way back. A thread holds the filter values of four neighbouring k for HELD_ROWS output channels or
+// fewer: `span` threads (a power of two) lie along k, and each of the TN_THREADS / span ranges of channels is theirs.
+// Forward a wave adds up its channels' sums with the lanes of two channels swapped into one register (sixteen sums in 40
+// instructions), and the waves' sums meet in scratch; back a thread sums its channels alone and the ranges meet.
+// LeNet-5's 120 x 400 (190 KB, which a compute unit takes 1.3 us to read), 16 samples, us: forward 1.7 with the tanh
+// behind it, back 1.5; asked for when they were needed, 4.6 (and 0.6 the tanh) and 3.2.
+constexpr int HELD_ROWS = 16;
+struct Held {
+  int shift, rows;   // 1 << shift threads along k; channels a thread holds
+};
+// (host; a division costs the sixteen waves of the kernel half a microsecond)
+inline Held held_shape(const TinyLayer &L) {
+  const int n_k4 = (L.C * L.R * L.S) >> 2;
+  int shift = 6;
+  while ((1 << shift) < n_k4) ++shift;
+  const int parts = TN_THREADS >> shift;
+  return {shift, parts ? ceil_div(L.K, parts) : L.K};
+}
+TN_INLINE void held_load(const TinyLayer *__restrict__ L, const Held h, float4 (&w)[HELD_ROWS], float &bias) {
+  const int K = L->K, n_k4 = (L->C * L->R * L->S) >> 2;
+  const int c0 = (wave_index() >> (h.shift - 6)) * h.rows, span = 1 << h.shift;
+  const int k = min(static_cast<int>(threadIdx.x) & (span - 1), n_k4 - 1);
+  const float4 *__restrict__ w4 = reinterpret_cast<const float4 *>(L->w);
+#pragma unroll
+  for (int r = 0; r < HELD_ROWS; ++r) w[r] = w4[static_cast<size_t>(min(c0 + min(r, h.rows - 1), K - 1)) * n_k4 + k];
+  bias = L->has_bias ? L->b[min(static_cast<int>(threadIdx.x), K - 1)] : 0.0f;
+}
+TN_INLINE void held_fwd(const TinyLayer *__restrict__ L, const Held h, const FastDiv d_rows, const float4 (&w)[HELD_ROWS], const float bias,
+                        const float *in, const FwdOut out, float *scratch) {
+  const int K = L->K, n_k4 = (L->C * L->R * L->S) >> 2, lane = threadIdx.x & 63;
+  const int k = static_cast<int>(threadIdx.x) & ((1 << h.shift) - 1);
+  float p[HELD_ROWS];
+#pragma unroll
+  for (int r = 0; r < HELD_ROWS; ++r) p[r] = 0.0f;
+  if (k < n_k4) {
+    const float4 xv = reinterpret_cast<const float4 *>(in)[k];
+#pragma unroll
+    for (int r = 0; r < HELD_ROWS; ++r) p[r] = (w[r].x * xv.x + w[r].y * xv.y) + (w[r].z * xv.z + w[r].w * xv.w);
+  }
+  // register j of each sixteen lanes, the g-th of the wave: the sum of row j + HELD_ROWS / 4 * g
+#pragma unroll
+  for (int r = 0; r < HELD_ROWS / 2; ++r) {
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[r]), __float_as_uint(p[r + HELD_ROWS / 2]), false, false);
+    p[r] = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+  }
+  const int j = lane & 15;
+  float mine = 0.0f;
+#pragma unroll
+  for (int r = 0; r < HELD_ROWS / 4; ++r) {
+    const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(p[r]), __float_as_uint(p[r + HELD_ROWS / 4]), false, false);
+    p[r] = row_sum(__uint_as_float(sw[0]) + __uint_as_float(sw[1]));
+    if (j == r) mine = p[r];
+  }
+  if (j < HELD_ROWS / 4) scratch[wave_index() * HELD_ROWS + HELD_ROWS / 4 * (lane >> 4) + j] = mine;
+  const bool has_bias = L->has_bias;
+  lds_barrier();
+  for (int co = threadIdx.x; co < K; co += TN_THREADS) {
+    uint32_t part, r;
+    d_rows.divmod(co, part, r);
+    const int waves = 1 << (h.shift - 6);
+    const float *q  = scratch + part * waves * HELD_ROWS + r;
+    float sum = q[0];
+    for (int v = 1; v < waves; ++v) sum += q[v * HELD_ROWS];
+    out(co, has_bias ? sum + (co < TN_THREADS ? bias : L->b[co]) : sum);
+  }
+}
+TN_INLINE void held_bwd(const TinyLayer *__restrict__ L, const Held h, const float4 (&w)[HELD_ROWS], const float *dy,
+                        const BwdOut dx, float *scratch) {
+  const int K = L->K, n_k = L->C * L->R * L->S, parts = TN_THREADS >> h.shift;
+  const int c0 = (wave_index() >> (h.shift - 6)) * h.rows;
+  const int rows = min(h.rows, K - c0);   // (negative in a range past the last channel)
+  const float dr = dy[min(c0 + static_cast<int>(threadIdx.x & (HELD_ROWS - 1)), K - 1)];   // lane r: row r's
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int r = 0; r < HELD_ROWS; ++r) {
+    const float d = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(dr), r));
+    if (r < rows) {   // (the whole wave)
+      acc.x += w[r].x * d; acc.y += w[r].y * d; acc.z += w[r].z * d; acc.w += w[r].w * d;
+    }
+  }
+  reinterpret_cast<float4 *>(scratch)[threadIdx.x] = acc;
+  lds_barrier();
+  for (int k = threadIdx.x; k < n_k; k += TN_THREADS) {
+    float sum = 0.0f;
+    for (int q0 = 0; q0 < parts; q0 += 4) {   // (four reads in flight)
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = scratch[(min(q0 + j, parts - 1) << (h.shift + 2)) + k];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (q0 + j < parts) sum += v[j];
+    }
+    dx(k, sum);
+  }
+}
+static_assert(4 * TN_THREADS <= TINY_SCRATCH_FLOATS, "four sums a thread");
+
+// The loss gradient with respect to the net's output (loss_function.h:28-36, 120-150); with a
+// closing softmax and cross_entropy_multiclass the gradient with respect to the softmax's
+// INPUT in closed form, y * sum(t) - t, and the softmax layer's own backward pass is skipped.
+// Returns the first layer to go back through.
+TN_INLINE int loss_gradient(const TinyPlan *__restrict__ plan, const float *lds, const int s, const int loss, const int softmax_xent,
+                            const float *__restrict__ t, float *ga) {
+  const int n = plan->n;
+  const TinyLayer *__restrict__ last = &plan->l[n - 1];
+  const int n_out = last->out_size;
+  const float *y  = lds + last->lds_out;
+  const float *tr = t + static_cast<size_t>(s) * n_out;
+  if (softmax_xent) {
+    float st = 0.0f;  // (every thread adds up the same few targets, in order)
+    for (int j = 0; j < n_out; ++j) st += tr[j];
+    float *gdz = last->dx + static_cast<size_t>(s) * n_out;
+    for (int j = threadIdx.x; j < n_out; j += TN_THREADS) {
+      const float v = fmaf(y[j], st, -tr[j]);
+      ga[j]  = v;
+      gdz[j] = v;
+    }
+    return n - 2;
+  }
+  const float mse_factor = plan->mse_factor;
+  float *gdl = plan->dloss + static_cast<size_t>(s) * n_out;
+  for (int j = threadIdx.x; j < n_out; j += TN_THREADS) {
+    float v;
+    if (loss == TDH_LOSS_MSE) v = mse_factor * (y[j] - tr[j]);
+    else if (loss == TDH_LOSS_CE_MULTICLASS) v = -tr[j] / y[j];
+    else v = (y[j] - tr[j]) / (y[j] * (1.0f - y[j]));
+    ga[j]  = v;
+    gdl[j] = v;
+  }
+  return n - 1;
+}
+
+// From the convolution in front of TinyPlan::held to the end of the net and back to that convolution's output: the
+// activation behind a layer runs in the layer's own phase, forward and back (a phase is half a microsecond of barrier and
+// layer sizes before its first value), with the filters of `held` in registers throughout. Only the kinds that
+// tiny_layout lets through are in these loops, so that the other layers' registers are free for the filters. Returns
+// with the gradient with respect to that convolution's output in `ga`.
+// LeNet-5, 16 samples: the kernel 21.8 us without this, 17.3 with it (with 512 threads and twice the filters each, 19).
+TN_INLINE void held_chain(const TinyPlan *__restrict__ plan, float *lds, const int s, const int loss,
+                          const int softmax_xent, const float *__restrict__ t, const int last_bwd, const float (&ahead_w)[MFMA_AHEAD],
+                          const float4 (&w)[HELD_ROWS], const float bias, float *&ga, float *&gb) {
+  const int n = plan->n, held = plan->held, from = plan->held_from;
+  const TinyLayer *__restrict__ H = &plan->l[held];
+  float *wl = lds + plan->lds_w;
+  const Held shape{plan->held_shift, plan->held_rows};
+  {
+    const bool act = is_pointwise(plan->l[from + 1]);
+    conv_fwd_mfma(&plan->l[from], lds, wl, fwd_out(plan, lds, from, s, act));
+    lds_barrier();
+    for (int li = from + 1 + act; li < held;) {
+      const TinyLayer *__restrict__ L = &plan->l[li];
+      const float *in = lds + L->lds_in;
+      const bool with = is_pool(*L) && is_pointwise(L[1]);
+      const FwdOut out = fwd_out(plan, lds, li, s, with);
+      if (L->kind == TDH_L_MAXPOOL) maxpool_fwd(L, in, out, L->argmax + static_cast<size_t>(s) * L->out_size);
+      else if (L->kind == TDH_L_AVEPOOL) avepool_fwd(L, in, out);
+      else act_fwd(L, in, out.out, out.gout);
+      lds_barrier();
+      li += 1 + with;
+    }
+  }
+  {
+    const bool act = held + 1 < n && is_pointwise(H[1]);
+    held_fwd(H, shape, plan->d_held_rows, w, bias, lds + H->lds_in, fwd_out(plan, lds, held, s, act), wl);
+    lds_barrier();
+    for (int li = held + 1 + act; li < n;) {
+      const TinyLayer *__restrict__ L = &plan->l[li];
+      const float *in = lds + L->lds_in;
+      const bool with = L->kind == TDH_L_FC && li + 1 < n && is_pointwise(L[1]);
+      const FwdOut out = fwd_out(plan, lds, li, s, with);
+      if (L->kind == TDH_L_FC) fc_fwd(L, in, out);
+      else if (L->act == TDH_ACT_SOFTMAX) softmax_fwd(L, in, out.out, out.gout);
+      else act_fwd(L, in, out.out, out.gout);
+      lds_barrier();
+      li += 1 + with;
+    }
+  }
+  int li = loss_gradient(plan, lds, s, loss, softmax_xent, t, ga);
+  __syncthreads();   // (also: the max-pool records written to memory above are read back below)
+  auto next = [&](const int done) {
+    lds_barrier();
+    float *sw = ga;
+    ga = gb;
+    gb = sw;
+    li -= done;
+  };
+  while (li > held) {
+    const TinyLayer *__restrict__ L = &plan->l[li];
+    const bool with = L->kind == TDH_L_FC && is_pointwise(L[-1]);   // (`held` is a convolution, so L[-1] lies behind it)
+    const BwdOut dx = bwd_out(plan, lds, gb, li, s, with);
+    if (L->kind == TDH_L_FC) fc_bwd_dx(L, ga, dx);
+    else act_bwd(L, lds + L->lds_out, ga, gb, dx.gdx);
+    next(1 + with);
+  }
+  // (the scratch area takes the filters of `from` for its input gradient while the layer behind it runs: there the
+  // gradient of `held`, which also meets in that area, stops short of it)
+  const int ahead = plan->mf_ahead;
+  const bool operand = ahead == from && ahead >= last_bwd && plan->l[from].mf_dx_w >= 0;
+  {
+    const bool with = held - 1 > from + operand && is_pointwise(H[-1]);
+    held_bwd(H, shape, w, ga, bwd_out(plan, lds, gb, held, s, with), wl);
+    next(1 + with);
+  }
+  while (li > from) {
+    const TinyLayer *__restrict__ L = &plan->l[li];
+    const bool with = is_pool(*L) && is_pointwise(L[-1]);
+    if (operand && li - with == from + 1) mfma_dx_operand_store(&plan->l[from], ahead_w, lds);
+    const BwdOut dx = bwd_out(plan, lds, gb, li, s, with);
+    if (L->kind == TDH_L_MAXPOOL) maxpool_bwd(L, ga, L->argmax + static_cast<size_t>(s) * L->out_size, dx);
+    else if (L->kind == TDH_L_AVEPOOL) avepool_bwd_dx(L, ga, dx);
+    else act_bwd(L, lds + L->lds_out, ga, gb, dx.gdx);
+    next(1 + with);
+  }
+}
+
 // One workgroup per sample, from layer m on (0, or the plan's split). LDS: its input, every layer's output, two gradient
 // buffers, the staging area.
 __global__ void __launch_bounds__(TN_THREADS)
@@ -1029,96 +1344,97 @@ tiny_net_step_kernel(const TinyPlan *__restrict__ plan, const int m, const int l
   // (one layer's filters for the matrix cores are asked for here, in front of the sample's input,
   // and put in LDS while the layer in front of that layer runs: no layer waits for them)
   const int ahead = plan->mf_ahead;
-  float ahead_w[MFMA_AHEAD] = {0.0f, 0.0f, 0.0f, 0.0f}, ahead_b = 0.0f;
+  float ahead_w[MFMA_AHEAD] = {}, ahead_b = 0.0f;
   if (ahead > 0) mfma_filters_load(&plan->l[ahead], 0, ahead_w, ahead_b);
-  fill_lds<TN_THREADS>(lds + plan->l[m].lds_in, (m ? plan->l[m - 1].out : x) + static_cast<size_t>(s) * in_size, in_size);
-  stage_mfma_operands(plan, lds, ahead);
-  if (m && ahead == m) {   // (there is no layer in front of it here)
-    mfma_filters_store(&plan->l[m], 0, ahead_w, ahead_b, lds);
-    mfma_tables(&plan->l[m], lds);
-  }
-  lds_barrier();
-  for (int li = m; li < n; ++li) {
-    const TinyLayer *__restrict__ L = &plan->l[li];
-    if (li + 1 == ahead) {
-      mfma_filters_store(&plan->l[ahead], 0, ahead_w, ahead_b, lds);
-      mfma_tables(&plan->l[ahead], lds);
-    }
-    const int kind = L->kind, out_size = L->out_size;
-    const float *in = lds + L->lds_in;
-    float *out      = lds + L->lds_out;
-    float *gout     = L->out + static_cast<size_t>(s) * out_size;
-    switch (kind) {
-      case TDH_L_CONV:
-        if (conv_is_matvec(*L)) {
-          if (!L->tbl && ((L->C * L->R * L->S) & 3) == 0 && (L->lds_in & 3) == 0) conv_fwd_matvec4(L, in, out, gout);
-          else conv_fwd_matvec(L, in, out, gout);
-        }
-        else if (L->mf_fwd_w >= 0) {
-          const float *fa = lds + L->mf_fwd_w, *fb = L->has_bias ? lds + L->mf_fwd_b : nullptr;
-          const int *fk = reinterpret_cast<const int *>(lds + L->mf_fwd_ko);
-          const int n_k = L->C * L->R * L->S, plane = L->OH * L->OW;
-          // (several pixel tiles a wave when there are more tiles than waves)
-          if (((L->K + 15) >> 4) * ((plane + 15) >> 4) > TN_WAVES) conv_mfma<4>(in, fa, fk, L->K, n_k, plane, L->d_ow, L->W, fb, out, gout);
-          else conv_mfma<1>(in, fa, fk, L->K, n_k, plane, L->d_ow, L->W, fb, out, gout);
-        }
-        else if (L->R == 5 && L->S == 5 && L->ph == 0 && L->pw == 0) conv_fwd_scalar_any<5, 5, false>(L, in, out, gout, wl);
-        else if (L->R == 5 && L->S == 5) conv_fwd_scalar_any<5, 5, true>(L, in, out, gout, wl);
-        else if (L->R == 3 && L->S == 3 && L->ph == 0 && L->pw == 0) conv_fwd_scalar_any<3, 3, false>(L, in, out, gout, wl);
-        else if (L->R == 3 && L->S == 3) conv_fwd_scalar_any<3, 3, true>(L, in, out, gout, wl);
-        else conv_fwd(L, in, out, gout);
-        break;
-      case TDH_L_FC: fc_fwd(L, in, out, gout); break;
-      case TDH_L_MAXPOOL: maxpool_fwd(L, in, out, gout, L->argmax + static_cast<size_t>(s) * out_size); break;
-      case TDH_L_AVEPOOL: avepool_fwd(L, in, out, gout); break;
-      default:
-        if (L->act == TDH_ACT_SOFTMAX) softmax_fwd(L, in, out, gout);
-        else act_fwd(L, in, out, gout);
-        break;
+  const float *src = (m ? plan->l[m - 1].out : x) + static_cast<size_t>(s) * in_size;
+  float *dst       = lds + plan->l[m].lds_in;
+  const int held = plan->held, generic = held ? plan->held_from : n;
+  float4 held_w[HELD_ROWS];
+  float held_b, touch = 0.0f;
+  if (held && generic == m) {
+    // (memory answers in order: what the first phases wait for is asked for in front of the held filters, what the last
+    // ones read behind them: those lines then lie in the cache)
+    float v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = src[min(j * TN_THREADS + static_cast<int>(threadIdx.x), in_size - 1)];
+    held_load(&plan->l[held], Held{plan->held_shift, plan->held_rows}, held_w, held_b);
+    touch = t[static_cast<size_t>(s) * plan->l[n - 1].out_size + min(static_cast<int>(threadIdx.x), plan->l[n - 1].out_size - 1)];
+    const TinyLayer *__restrict__ F = &plan->l[min(held + 1 + (held + 1 < n && is_pointwise(plan->l[held + 1])), n - 1)];
+    if (F->kind == TDH_L_FC) touch += F->w[min(32 * static_cast<int>(threadIdx.x), F->nw - 1)];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j * TN_THREADS + static_cast<int>(threadIdx.x) < in_size) dst[j * TN_THREADS + threadIdx.x] = v[j];
+    if (in_size > 4 * TN_THREADS) fill_lds<TN_THREADS>(dst + 4 * TN_THREADS, src + 4 * TN_THREADS, in_size - 4 * TN_THREADS);
+    stage_mfma_operands(plan, lds, m, ahead);
+    if (m && ahead == m) {   // (there is no layer in front of it here)
+      mfma_filters_store(&plan->l[m], 0, ahead_w, ahead_b, lds);
+      mfma_tables(&plan->l[m], lds);
     }
     lds_barrier();
-  }
-  // the loss gradient with respect to the net's output (loss_function.h:28-36, 120-150); with a
-  // closing softmax and cross_entropy_multiclass the gradient with respect to the softmax's
-  // INPUT in closed form, y * sum(t) - t, and the softmax layer's own backward pass is skipped
-  float *ga = lds + plan->lds_g0, *gb = lds + plan->lds_g1;
-  const TinyLayer *__restrict__ last = &plan->l[n - 1];
-  const int n_out = last->out_size;
-  const float *y  = lds + last->lds_out;
-  const float *tr = t + static_cast<size_t>(s) * n_out;
-  int first_bwd   = n - 1;
-  if (softmax_xent) {
-    float st = 0.0f;  // (every thread adds up the same few targets, in order)
-    for (int j = 0; j < n_out; ++j) st += tr[j];
-    float *gdz = last->dx + static_cast<size_t>(s) * n_out;
-    for (int j = threadIdx.x; j < n_out; j += TN_THREADS) {
-      const float v = fmaf(y[j], st, -tr[j]);
-      ga[j]  = v;
-      gdz[j] = v;
-    }
-    first_bwd = n - 2;
   } else {
-    const float mse_factor = plan->mse_factor;
-    float *gdl = plan->dloss + static_cast<size_t>(s) * n_out;
-    for (int j = threadIdx.x; j < n_out; j += TN_THREADS) {
-      float v;
-      if (loss == TDH_LOSS_MSE) v = mse_factor * (y[j] - tr[j]);
-      else if (loss == TDH_LOSS_CE_MULTICLASS) v = -tr[j] / y[j];
-      else v = (y[j] - tr[j]) / (y[j] * (1.0f - y[j]));
-      ga[j]  = v;
-      gdl[j] = v;
+    fill_lds<TN_THREADS>(dst, src, in_size);
+    stage_mfma_operands(plan, lds, m, ahead);
+    if (m && ahead == m) {
+      mfma_filters_store(&plan->l[m], 0, ahead_w, ahead_b, lds);
+      mfma_tables(&plan->l[m], lds);
     }
+    lds_barrier();
+    for (int li = m; li < generic; ++li) {
+      const TinyLayer *__restrict__ L = &plan->l[li];
+      if (li + 1 == ahead) {
+        mfma_filters_store(&plan->l[ahead], 0, ahead_w, ahead_b, lds);
+        mfma_tables(&plan->l[ahead], lds);
+      }
+      const int kind = L->kind, out_size = L->out_size;
+      const float *in = lds + L->lds_in;
+      float *out      = lds + L->lds_out;
+      float *gout     = L->out + static_cast<size_t>(s) * out_size;
+      const FwdOut plain = fwd_out(plan, lds, li, s, false);
+      switch (kind) {
+        case TDH_L_CONV:
+          if (conv_is_matvec(*L)) {
+            if (!L->tbl && ((L->C * L->R * L->S) & 3) == 0 && (L->lds_in & 3) == 0) conv_fwd_matvec4(L, in, out, gout);
+            else conv_fwd_matvec(L, in, out, gout);
+          }
+          else if (L->mf_fwd_w >= 0) conv_fwd_mfma(L, lds, wl, plain);
+          else if (L->R == 5 && L->S == 5 && L->ph == 0 && L->pw == 0) conv_fwd_scalar_any<5, 5, false>(L, in, out, gout, wl);
+          else if (L->R == 5 && L->S == 5) conv_fwd_scalar_any<5, 5, true>(L, in, out, gout, wl);
+          else if (L->R == 3 && L->S == 3 && L->ph == 0 && L->pw == 0) conv_fwd_scalar_any<3, 3, false>(L, in, out, gout, wl);
+          else if (L->R == 3 && L->S == 3) conv_fwd_scalar_any<3, 3, true>(L, in, out, gout, wl);
+          else conv_fwd(L, in, out, gout);
+          break;
+        case TDH_L_FC: fc_fwd(L, in, plain); break;
+        case TDH_L_MAXPOOL: maxpool_fwd(L, in, plain, L->argmax + static_cast<size_t>(s) * out_size); break;
+        case TDH_L_AVEPOOL: avepool_fwd(L, in, plain); break;
+        default:
+          if (L->act == TDH_ACT_SOFTMAX) softmax_fwd(L, in, out, gout);
+          else act_fwd(L, in, out, gout);
+          break;
+      }
+      lds_barrier();
+    }
+    if (held) held_load(&plan->l[held], Held{plan->held_shift, plan->held_rows}, held_w, held_b);
   }
-  __syncthreads();   // (also: the max-pool records written to memory above are read back below)
-  // input gradients only: the parameter-gradient kernel reads what this loop leaves in memory
+  asm volatile("" ::"v"(touch));
+  float *ga = lds + plan->lds_g0, *gb = lds + plan->lds_g1;
+  // input gradients only: the parameter-gradient kernel reads what this leaves in memory
   const int last_bwd = m ? m + 1 : (plan->first_dx_as_job || plan->skip_first_dx) ? 1 : 0;
+  int first_bwd;
+  if (held) {
+    held_chain(plan, lds, s, loss, softmax_xent, t, last_bwd, ahead_w, held_w, held_b, ga, gb);
+    first_bwd = generic;
+  } else {
+    first_bwd = loss_gradient(plan, lds, s, loss, softmax_xent, t, ga);
+    __syncthreads();   // (also: the max-pool records written to memory above are read back below)
+  }
   for (int li = first_bwd; li >= last_bwd; --li) {
     const TinyLayer *__restrict__ L = &plan->l[li];
     const int kind = L->kind, in_sz = L->in_size;
     // (the layer in front of this one in memory order is the next to run: its operand goes into
     // the scratch area now, which this phase does not use when that is so; see tiny_build_jobs)
-    if (li - 1 == ahead && ahead > 0 && plan->l[ahead].mf_dx_w >= 0) mfma_dx_operand_store(&plan->l[ahead], ahead_w, lds);
+    if (li - 1 == ahead && ahead >= last_bwd && plan->l[ahead].mf_dx_w >= 0) mfma_dx_operand_store(&plan->l[ahead], ahead_w, lds);
     float *gdx = L->dx ? L->dx + static_cast<size_t>(s) * in_sz : nullptr;
+    const BwdOut plain = bwd_out(plan, lds, gb, li, s, false);
     switch (kind) {
       case TDH_L_CONV:
         if (conv_is_matvec(*L)) {
@@ -1137,7 +1453,7 @@ tiny_net_step_kernel(const TinyPlan *__restrict__ plan, const int m, const int l
             float *dd = lds + L->mf_dx_d;
             const int PW = L->W + L->S - 1, cols = L->H * PW;
             conv_mfma<2>(framed, lds + L->mf_dx_w, reinterpret_cast<const int *>(lds + L->mf_dx_ko), L->C * L->S,
-                         L->K * L->R, cols, L->d_pw, PW, nullptr, dd, nullptr);
+                         L->K * L->R, cols, L->d_pw, PW, nullptr, [dd](const int i, const float v) { dd[i] = v; });
             lds_barrier();
             mfma_dx_gather(L, dd, gb, gdx);
           }
@@ -1145,9 +1461,9 @@ tiny_net_step_kernel(const TinyPlan *__restrict__ plan, const int m, const int l
           else conv_bwd_dx_scalar_any<3, 3, TN_THREADS>(L, framed, gb, gdx, wl, 0, items * parts, parts);
         }
         break;
-      case TDH_L_FC: fc_bwd_dx(L, ga, gb, gdx); break;
-      case TDH_L_MAXPOOL: maxpool_bwd(L, ga, L->argmax + static_cast<size_t>(s) * L->out_size, gb, gdx); break;
-      case TDH_L_AVEPOOL: avepool_bwd_dx(L, ga, gb, gdx); break;
+      case TDH_L_FC: fc_bwd_dx(L, ga, plain); break;
+      case TDH_L_MAXPOOL: maxpool_bwd(L, ga, L->argmax + static_cast<size_t>(s) * L->out_size, plain); break;
+      case TDH_L_AVEPOOL: avepool_bwd_dx(L, ga, plain); break;
       default: act_bwd(L, lds + L->lds_out, ga, gb, gdx); break;
     }
     lds_barrier();
@@ -1168,7 +1484,7 @@ tiny_net_step_kernel(const TinyPlan *__restrict__ plan, const int m, const int l
 // keeps to one channel: a workgroup takes one channel of a sample through it, forward in a launch in
 // front of the step kernel, and in a launch behind it from the second convolution's dX back to the
 // gradient of the first one's output. Bound: latency, a launch and some three trips to memory each.
-// LeNet-5, batch 16, us: one launch 40.1; here 4.5 + 21.8 + 7.8 (which batches: launch_tiny_step).
+// LeNet-5, batch 16, us: one launch 34; here 4.5 + 17.3 + 7.8 (which batches: launch_tiny_step).
 constexpr int TF_THREADS = 1024;   // front, at most
 constexpr int TB_THREADS = 1024;   // back
 static_assert(TB_THREADS / 64 == 16, "sixteen shares of a pool's sums; a wave left over from five rows of three and from three of five");
@@ -2265,6 +2581,24 @@ int tiny_layout(TinyPlan &P) {
       L.mf_dx_d  = at;
       P.lds_floats = at + rows * cols;
     }
+  }
+  // A matrix-vector layer whose filters a workgroup holds in registers while everything behind them runs: its rows are a
+  // multiple of 16 bytes, in front of it lie pools and activations behind a product on the matrix cores, and behind
+  // it fully-connected layers and activations (the loops that run meanwhile know no other kinds)
+  P.held = P.held_from = 0;
+  for (int h = 1; h < P.n; ++h) {
+    const TinyLayer &L = P.l[h];
+    if (L.kind != TDH_L_CONV || !conv_is_matvec(L) || L.tbl || ((L.C * L.R * L.S) & 3) || (L.lds_in & 3) ||
+        (reinterpret_cast<uintptr_t>(L.w) & 15) || (1 << held_shape(L).shift) > TN_THREADS || held_shape(L).rows > HELD_ROWS)
+      continue;
+    int from = h - 1, end = h + 1;
+    while (from > 0 && (is_pointwise(P.l[from]) || is_pool(P.l[from]))) --from;
+    while (end < P.n && (P.l[end].kind == TDH_L_FC || P.l[end].kind == TDH_L_ACT)) ++end;
+    if (P.l[from].mf_fwd_w < 0 || end < P.n || from < P.split) continue;
+    P.held = h; P.held_from = from;
+    P.held_shift  = held_shape(L).shift;
+    P.held_rows   = held_shape(L).rows;
+    P.d_held_rows = FastDiv(static_cast<uint32_t>(P.held_rows));
   }
   P.lds_job_floats = static_cast<int>(lds);
   return TDH_OK;
