@@ -32,6 +32,15 @@ constexpr size_t x3_pack_bytes(int RS, int KC, int MC) {
   return static_cast<size_t>((KC + 15) / 16) * RS * 6 * x3_mc_pad(MC) * 16;
 }
 
+// The first pixel, in the workgroup's tile of rows of TC pixels, of accumulator block b = wave * TN + j. Blocks are 32 pixels in
+// a row; where rows are longer, two blocks of a wave that follow each other are the same columns of two rows, so that
+// a lane holds both rows of its column and two lanes a 2x2 pooling window. (Not in the three-part kernel, whose waves read
+// 0.5 % slower that way: 32 -> 64 channels, 3x3, 64x64, batch 64, forward, dX and dW 219.3 us / 220.3.)
+template <int TC, int TN>
+__host__ __device__ constexpr int s1_block_pixel(const int b) {
+  return TC == 64 && TN % 2 == 0 ? ((b >> 2) * 2 + (b & 1)) * 64 + ((b >> 1) & 1) * 32 : 32 * b;
+}
+
 // the sign of step u's products (chunk, tap): the packed filters carry it
 __host__ __device__ constexpr float x3_sign(int u) { return u & 1 ? -1.0f : 1.0f; }
 
@@ -49,8 +58,8 @@ struct ConvS1Args {
   float *act_out;              // forward: act(out) of the pointwise activation layer that follows
   int act_kind;
   // forward: the 2x2 / stride-2 max-pool layer behind the convolution (or behind act_out) and
-  // the relu behind that pool, all null when the pool runs as a kernel of its own. Only tiles
-  // whose 32-pixel blocks hold whole pool windows (rows of 8 or 16 pixels, no split) take it.
+  // the relu behind that pool, all null when the pool runs as a kernel of its own. Only waves
+  // whose blocks hold whole pool windows (rows of 8 or 16 pixels, or an even number of blocks in rows of 32 and, in fp32, 64; no split) take it.
   float *pool_out;
   int32_t *pool_argmax;        // flat CHW index inside the sample of the pool's input
   float *pool_act_out;         // max(pool_out, 0), or null

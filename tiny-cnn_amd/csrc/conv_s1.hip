@@ -217,13 +217,13 @@ bool conv_s1_single_pass(int R, int S, int batch, int KC, int MC, int IH, int IW
   return p.ok && p.splits == 1;
 }
 
-// A 32-pixel accumulator block must hold whole 2x2 windows: rows of 8 or 16 pixels (tile rows
-// come in powers of two and start at even image rows), even image sizes, and one pass over the
-// reduction channels (the partial sums of a split have no maximum yet).
+// A wave must hold whole 2x2 windows: in a 32-pixel accumulator block (rows of 8 or 16 pixels; tile rows
+// come in powers of two and start at even image rows) or in two of them (s1_block_pixel), with even image sizes and
+// one pass over the reduction channels (the partial sums of a split have no maximum yet).
 bool conv_s1_fuses_pool(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW,
                         int ph, int pw) {
   const S1Plan p = make_plan(R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw);
-  return p.ok && p.splits == 1 && p.tc <= 16 && p.args.TR >= 2 && OH % 2 == 0 && OW % 2 == 0 &&
+  return p.ok && p.splits == 1 && (p.tc <= 16 || (p.tn % 2 == 0 && !(p.x3 && p.tc == 64))) && p.args.TR >= 2 && OH % 2 == 0 && OW % 2 == 0 &&
          static_cast<long>(MC) * OH * OW < (1L << 31);
 }
 

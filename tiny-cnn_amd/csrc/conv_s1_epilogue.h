@@ -20,16 +20,106 @@ __device__ __forceinline__ float s1_lane_xor(const float v) {
   return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (X << 10) | 0x1F));
 }
 
+// The forward pass with a 2x2 max-pool behind it where blocks j and j + 1 of a wave are two rows (s1_block_pixel): a lane
+// holds both rows of its column, two neighbours share a window, exchange the values of two channels and pool one each,
+// with strict '>' from lowest() in scan order (maxpool_op_internal.h:17-47). The pool's own kernel is bound by the read of
+// the activation, which no kernel reads next once the pool is made here: y and it go past the caches. us of
+// convolution and pool, apart / here: 64 -> 64 channels, 3x3, 128x128, batch 64 748 / 697, 128 -> 128, 64x64 655 / 620 (stores that
+// stay in the caches 703 and 628).
 template <int TC, int TM, int TN>
+__device__ __forceinline__ void s1_epilogue_pool_rows(const ConvS1Args &a, const floatx16 (&acc)[TM][TN], const int wn,
+                                                      const int lane, const int img0, const int y0, const int x0, const int m0) {
+  constexpr int LOG_TC = TC == 64 ? 6 : 5;
+  const int ohw = a.OH * a.OW, pw2 = a.OW >> 1, pohw = (a.OH >> 1) * pw2;
+  const bool right = lane & 1;
+#pragma unroll
+  for (int j = 0; j < TN; j += 2) {
+    const int q   = s1_block_pixel<TC, TN>(wn * TN + j) + (lane & 31);
+    const int img = img0 + (q >> (a.log_tr + LOG_TC));
+    const int oy = y0 + ((q >> LOG_TC) & (a.TR - 1)), ox = x0 + (q & (TC - 1));
+    if (img >= a.batch || oy >= a.OH || ox >= a.OW) continue;   // (even sizes: both rows, and both lanes of a window)
+    const size_t pbase  = static_cast<size_t>(img) * a.MC * ohw + oy * a.OW + ox;
+    const size_t pobase = static_cast<size_t>(img) * a.MC * pohw + (oy >> 1) * pw2 + (ox >> 1);
+    const int pix = oy * a.OW + (ox & ~1);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int mb = m0 + 32 * i + 4 * (lane >> 5);
+      float v0[16], v1[16];
+#pragma unroll
+      for (int rr = 0; rr < 16; ++rr) {
+        v0[rr] = acc[i][j][rr];
+        v1[rr] = acc[i][j + 1][rr];
+      }
+      if (a.bias) {
+#pragma unroll
+        for (int rr = 0; rr < 16; ++rr) {
+          const float b = a.bias[min(mb + 8 * (rr >> 2) + (rr & 3), a.MC - 1)];
+          v0[rr] += b;
+          v1[rr] += b;
+        }
+      }
+      auto write = [&](float *to) {
+#pragma unroll
+        for (int rr = 0; rr < 16; ++rr) {
+          const int m = mb + 8 * (rr >> 2) + (rr & 3);
+          if (m < a.MC) {
+            float *p = to + pbase + static_cast<size_t>(m) * ohw;
+            __builtin_nontemporal_store(v0[rr], p);
+            __builtin_nontemporal_store(v1[rr], p + a.OW);
+          }
+        }
+      };
+      if (a.out) write(a.out);
+      if (a.act_out) {
+#pragma unroll
+        for (int rr = 0; rr < 16; ++rr) {
+          v0[rr] = act_apply(a.act_kind, v0[rr]);
+          v1[rr] = act_apply(a.act_kind, v1[rr]);
+        }
+        write(a.act_out);
+      }
+#pragma unroll
+      for (int rr = 0; rr < 16; rr += 2) {
+        const float l0 = s1_lane_xor1(v0[rr + 1]), r0 = s1_lane_xor1(v0[rr]);
+        const float l1 = s1_lane_xor1(v1[rr + 1]), r1 = s1_lane_xor1(v1[rr]);
+        const float w4[4] = {right ? l0 : v0[rr], right ? v0[rr + 1] : r0, right ? l1 : v1[rr], right ? v1[rr + 1] : r1};
+        float best = -3.402823466e+38f;
+        int sel    = -1;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (w4[k] > best) {
+            best = w4[k];
+            sel  = k;
+          }
+        const int m = mb + 8 * (rr >> 2) + (rr & 3) + (right ? 1 : 0);
+        if (m < a.MC) {
+          const size_t at = pobase + static_cast<size_t>(m) * pohw;
+          a.pool_out[at]    = best;
+          a.pool_argmax[at] = sel < 0 ? 0 : m * ohw + pix + (sel >> 1) * a.OW + (sel & 1);
+          if (a.pool_act_out) a.pool_act_out[at] = best > 0.0f ? best : 0.0f;
+        }
+      }
+    }
+  }
+}
+
+// ROWS: the wave's blocks lie as s1_block_pixel<TC, TN> has them, else one after the other
+template <int TC, int TM, int TN, bool ROWS = true>
 __device__ __forceinline__ void s1_epilogue(const ConvS1Args &a, const floatx16 (&acc)[TM][TN], const int wn,
                                             const int lane, const int img0, const int y0, const int x0,
                                             const int m0, const int bz) {
   constexpr int LOG_TC = TC == 64 ? 6 : TC == 32 ? 5 : TC == 16 ? 4 : 3;
   // reg r of lane l holds channel 8*(r/4) + 4*(l/32) + r%4, pixel l%32
   const int ohw = a.OH * a.OW;
+  if constexpr (ROWS && TC >= 32 && TN % 2 == 0) {
+    if (a.pool_out) {   // (forward, unsplit)
+      s1_epilogue_pool_rows<TC, TM, TN>(a, acc, wn, lane, img0, y0, x0, m0);
+      return;
+    }
+  }
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    const int q   = (wn * TN + j) * 32 + (lane & 31);
+    const int q   = s1_block_pixel<TC, ROWS ? TN : 1>(wn * TN + j) + (lane & 31);
     const int ti  = q >> (a.log_tr + LOG_TC);
     const int r   = (q >> LOG_TC) & (a.TR - 1);
     const int c   = q & (TC - 1);

@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(256, 2) conv_s1_kernel(const ConvS1Args a) {
   int boff[TN];
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    const int q  = (wn * TN + j) * 32 + (lane & 31);
+    const int q  = s1_block_pixel<TC, TN>(wn * TN + j) + (lane & 31);
     const int ti = q >> (a.log_tr + LOG_TC);
     const int r  = (q >> LOG_TC) & (a.TR - 1);
     const int c  = q & (TC - 1);
