@@ -182,3 +182,42 @@ def test_more_work_items_than_a_grid_has_in_one_direction(T):
         got = T.DevBuf.view(y.ptr.value + 4 * i * co, (co,)).numpy()
         want = wt.reshape(co, -1).astype(np.float64) @ x[i].ravel().astype(np.float64) + b
         assert (np.abs(got - want) <= bound).all(), i
+
+
+@pytest.mark.parametrize("w,h,ci,k,co,batch,same", [
+    (128, 9, 3, 3, 17, 4, True),     # rows of 128, the last band of one row, a last chunk of one channel
+    (20, 21, 4, 3, 8, 9, True),
+    (26, 19, 2, 3, 5, 9, False),     # rows of 24 outputs, two in front of the first that is read
+    (40, 13, 1, 5, 9, 6, True),
+    (44, 30, 4, 5, 30, 3, False),    # rows of 40 outputs from the first one on
+    (200, 31, 3, 3, 9, 12, True),    # a band of one row
+])
+def test_dx_of_words_is_that_of_elements(T, w, h, ci, k, co, batch, same):
+    """dX reads rows of a multiple of four outputs by words where they are aligned, else by elements: the same bits, and the
+    same as a correlation in 64 bits (the error of a sum of k * k * co products)."""
+    rng = np.random.default_rng(5)
+    ow, oh = (w, h) if same else (w - k + 1, h - k + 1)
+    d = T.conv_desc(w, h, ci, k, k, co, pad_same=same)
+    wt = rng.uniform(-0.3, 0.3, (co, ci, k, k)).astype(np.float32)
+    dy = rng.standard_normal((batch, co, oh, ow)).astype(np.float32)
+    moved = T.DevBuf((dy.size + 1,))
+    moved.upload(np.concatenate([[0], dy.ravel()]).astype(np.float32))
+    x, got = T.to_device(rng.standard_normal((batch, ci, h, w)).astype(np.float32)), []
+    for g in (T.to_device(dy), T.DevBuf.view(moved.ptr.value + 4, dy.shape)):
+        dx = T.DevBuf((batch, ci, h, w))
+        T.profile_begin()
+        T.conv2d_bwd(d, batch, x, T.to_device(wt), g, dx, T.DevBuf(wt.shape), T.DevBuf((co,)))
+        tags = [r["tag"].split()[0] for r in T.profile_end()]
+        assert "conv_dx_small_cin" in tags, tags
+        got.append(dx.numpy())
+    assert np.array_equal(*got)
+    p = k // 2 if same else 0
+    want, size = np.zeros((2, batch, ci, h + 2 * p, w + 2 * p))
+    dy, wt = dy.astype(np.float64), wt.astype(np.float64)
+    for ky in range(k):
+        for kx in range(k):
+            at = (slice(None), slice(None), slice(ky, ky + oh), slice(kx, kx + ow))
+            want[at] += np.einsum("bohw,oc->bchw", dy, wt[:, :, ky, kx])
+            size[at] += np.einsum("bohw,oc->bchw", np.abs(dy), np.abs(wt[:, :, ky, kx]))
+    inner = (slice(None), slice(None), slice(p, p + h), slice(p, p + w))
+    assert np.all(np.abs(got[0] - want[inner]) <= 2.0**-24 * (k * k * co + 2) * size[inner])

@@ -410,14 +410,23 @@ struct DxsPlan {
 // A thread stages pool windows instead of tile elements: one gradient and one argmax record per
 // window, and writes the window's four elements into the tile (the gradient where the record
 // names the element, else zero; windows outside the image give the zero halo).
-template <int KR, int KS, int CIN, bool POOLED>
+// SHIFT >= 0: rows of a multiple of four outputs, staged as 16-byte words; the tile then starts SHIFT columns in front of the
+// first one that is read, at a multiple of four, and the weights are scalar operands straight from memory (a wave has one
+// output channel at a time).
+// Bound: vector instructions (108 multiply-adds a lane and channel for 3x3 on three channels; staged by elements, a
+// chunk's 20 loads with their addresses and stores are as many again, and the weights nine of fifteen LDS reads a
+// channel). 3 <- 64 channels, 3x3, 128x128, batch 64: 111 us by elements, 84 by words. (Scalar weights and elements: 3 <- 24,
+// 3x3, 30x30, batch 37 9.1 us, with the weights in LDS 8.8; the few workgroups wait for each channel's.)
+template <int KR, int KS, int CIN, bool POOLED, int SHIFT = -1>
 __global__ void __launch_bounds__(DXS_NT)
 conv_dx_small_cin_kernel(const float *__restrict__ dy, const float *__restrict__ w,
                          float *__restrict__ dx, const ConvGeom g, const DxsPlan p,
                          const ActGrad ag, const PoolGather pooled) {
   extern __shared__ __align__(16) float smem[];
   const int R = KR ? KR : g.R, S = KS ? KS : g.S;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  constexpr bool WORDS = SHIFT >= 0, SCALAR_W = WORDS;
+  typedef const float __attribute__((address_space(4))) *ScalarFloats;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wg  = xcd_compact_id(blockIdx.x, gridDim.x);  // (an image's bands share rows: one XCD)
   const int img = wg / p.bands;
   const int y0  = (wg - img * p.bands) * p.tile_rows;
@@ -445,17 +454,17 @@ conv_dx_small_cin_kernel(const float *__restrict__ dy, const float *__restrict__
 
   // staging plan, the same for every chunk: element e = tid + DXS_NT*j of the chunk tile ->
   // channel inside the chunk and offset inside that channel's plane (-1: outside the image)
-  constexpr int NS = POOLED ? 1 : DXS_MAX_STAGE, NP = POOLED ? DXS_MAX_PSTAGE : 1;
-  float stage[NS];
+  constexpr int NS = POOLED ? 1 : WORDS ? DXS_MAX_STAGE / 4 : DXS_MAX_STAGE, NP = POOLED ? DXS_MAX_PSTAGE : 1;
+  std::conditional_t<WORDS, float4, float> stage[NS];
   int soff[NS], sch[NS];
   if (!POOLED) {
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
       const uint32_t e = tid + DXS_NT * j;
       uint32_t c, rem, r, q;
-      p.div_tile.divmod(e, c, rem);
+      p.div_tile.divmod(e, c, rem);    // (in words where those are staged)
       p.div_tcols.divmod(rem, r, q);
-      const int oy = oy0 + static_cast<int>(r), ox = ox0 + static_cast<int>(q);
+      const int oy = oy0 + static_cast<int>(r), ox = WORDS ? ox0 - SHIFT + 4 * static_cast<int>(q) : ox0 + static_cast<int>(q);
       const bool in = static_cast<unsigned>(oy) < static_cast<unsigned>(g.OH) &&
                       static_cast<unsigned>(ox) < static_cast<unsigned>(g.OW);
       sch[j]  = static_cast<int>(c);
@@ -522,14 +531,22 @@ conv_dx_small_cin_kernel(const float *__restrict__ dy, const float *__restrict__
         prec[j] = live ? rec_img[co0 * pohw + poff[j]] - (co0 * ohw + pflat[j]) : -1;
       }
     } else {
+      if constexpr (WORDS) {
 #pragma unroll
-      for (int j = 0; j < NS; ++j)
-        stage[j] = (soff[j] >= 0 && sch[j] < nco) ? base[soff[j]] : 0.0f;
+        for (int j = 0; j < NS; ++j)
+          stage[j] = (soff[j] >= 0 && sch[j] < nco) ? *reinterpret_cast<const float4 *>(base + soff[j]) : make_float4(0.f, 0.f, 0.f, 0.f);
+      } else {
+#pragma unroll
+        for (int j = 0; j < NS; ++j)
+          stage[j] = (soff[j] >= 0 && sch[j] < nco) ? base[soff[j]] : 0.0f;
+      }
     }
+    if constexpr (!SCALAR_W) {
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int e = tid + DXS_NT * k;
-      wreg[k]     = e < nco * rs ? load_w(co0, e) : make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int k = 0; k < 2; ++k) {
+        const int e = tid + DXS_NT * k;
+        wreg[k]     = e < nco * rs ? load_w(co0, e) : make_float4(0.f, 0.f, 0.f, 0.f);
+      }
     }
   };
 
@@ -549,15 +566,21 @@ conv_dx_small_cin_kernel(const float *__restrict__ dy, const float *__restrict__
 #pragma unroll
       for (int j = 0; j < NS; ++j) {
         const int e = tid + DXS_NT * j;
-        if (e < DXS_CO_CHUNK * tsz) tile[e] = stage[j];
+        if constexpr (WORDS) {
+          if (4 * e < DXS_CO_CHUNK * tsz) reinterpret_cast<float4 *>(tile)[e] = stage[j];
+        } else {
+          if (e < DXS_CO_CHUNK * tsz) tile[e] = stage[j];
+        }
       }
     }
+    if constexpr (!SCALAR_W) {
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int e = tid + DXS_NT * k;
-      if (e < nco * rs) wl[e] = wreg[k];
+      for (int k = 0; k < 2; ++k) {
+        const int e = tid + DXS_NT * k;
+        if (e < nco * rs) wl[e] = wreg[k];
+      }
+      for (int e = tid + 2 * DXS_NT; e < nco * rs; e += DXS_NT) wl[e] = load_w(co0, e);  // larger windows
     }
-    for (int e = tid + 2 * DXS_NT; e < nco * rs; e += DXS_NT) wl[e] = load_w(co0, e);  // larger windows
     __syncthreads();
     if (co0 + DXS_CO_CHUNK < g.Kc) fetch(co0 + DXS_CO_CHUNK);  // in flight during the math
 
@@ -568,7 +591,10 @@ conv_dx_small_cin_kernel(const float *__restrict__ dy, const float *__restrict__
       const float *t   = tile + c * tsz + toff;
       const float4 *wc = wl + c * rs;
       if (KR != 0) {
-        constexpr int NV = (DXS_PX + (KS ? KS : 1) - 1 + 3) / 4;  // 16-byte words per filter row
+        constexpr int FROM = WORDS ? SHIFT : 0;
+        constexpr int NV   = (FROM + DXS_PX + (KS ? KS : 1) - 1 + 3) / 4;  // 16-byte words per filter row
+        // (channels of the instance, which is the layer's own count for a known window)
+        const ScalarFloats ws = (ScalarFloats)(w + static_cast<size_t>(co0 + c) * (CIN * KR * KS));
 #pragma unroll
         for (int fy = 0; fy < KR; ++fy) {
           float v[4 * NV];
@@ -579,12 +605,18 @@ conv_dx_small_cin_kernel(const float *__restrict__ dy, const float *__restrict__
           }
 #pragma unroll
           for (int fx = 0; fx < KS; ++fx) {
-            const float4 wq  = wc[fy * KS + fx];
-            const float wa[4] = {wq.x, wq.y, wq.z, wq.w};
+            float wa[4];
+            if constexpr (SCALAR_W) {
+#pragma unroll
+              for (int ci = 0; ci < CIN; ++ci) wa[ci] = ws[(ci + 1) * (KR * KS) - 1 - fy * KS - fx];   // (flipped)
+            } else {
+              const float4 wq = wc[fy * KS + fx];
+              wa[0] = wq.x; wa[1] = wq.y; wa[2] = wq.z; wa[3] = wq.w;
+            }
 #pragma unroll
             for (int ci = 0; ci < CIN; ++ci)
 #pragma unroll
-              for (int i = 0; i < DXS_PX; ++i) acc[ci][i] += wa[ci] * v[i + fx];
+              for (int i = 0; i < DXS_PX; ++i) acc[ci][i] += wa[ci] * v[FROM + i + fx];
           }
         }
       } else {
@@ -1106,10 +1138,49 @@ static bool small_cin_dx_plan(const ConvGeom &g, DxsPlan &p) {
   return p.lds_bytes <= 64 * 1024;
 }
 
+// the columns in front of the first one read, staged as words, or -1
+static int small_cin_words(const ConvGeom &g, const float *dy, DxsPlan &p) {
+  const int ox0 = g.pad_w - (g.S - 1), shift = ((ox0 % 4) + 4) % 4;
+  if (g.OW % 4 != 0 || (reinterpret_cast<uintptr_t>(dy) & 15) || (g.OH * g.OW) % 4 != 0) return -1;
+  const int words = ceil_div(shift + DXS_PX * p.gw + g.S - 1, 4);
+  if (DXS_CO_CHUNK * p.trows * words > DXS_MAX_STAGE / 4 * DXS_NT) return -1;
+  p.tcols     = 4 * words;
+  p.div_tcols = FastDiv(words);
+  p.div_tile  = FastDiv(p.trows * words);
+  const size_t stage_floats = static_cast<size_t>(DXS_CO_CHUNK) * p.trows * p.tcols;
+  const size_t red_floats   = static_cast<size_t>(DXS_WAVES) * DXS_MAX_CIN * 64 * DXS_PX;
+  p.lds_bytes = sizeof(float) * std::max(stage_floats, red_floats);
+  return shift;
+}
+template <int KR, int CIN, int SHIFT>
+static void launch_small_cin_dx_words(const ConvGeom &g, const DxsPlan &p, int batch, const float *dy, const float *w, float *dx,
+                                      ActGrad ag) {
+  TDH_LAUNCH((conv_dx_small_cin_kernel<KR, KR, CIN, false, SHIFT>), dim3(batch * p.bands), dim3(DXS_NT), p.lds_bytes,
+             ctx().stream, dy, w, dx, g, p, ag, PoolGather());
+}
+
 template <int KR, int KS, bool POOLED>
-static void launch_small_cin_dx(const ConvGeom &g, const DxsPlan &p, int batch, const float *dy,
+static void launch_small_cin_dx(const ConvGeom &g, const DxsPlan &plan, int batch, const float *dy,
                                 const float *w, float *dx, ActGrad ag, PoolGather pooled) {
+  DxsPlan p = plan;
   const dim3 grid(batch * p.bands), block(DXS_NT);
+  if constexpr (KR != 0 && !POOLED) {
+    // the two paddings there are
+    constexpr int same = (4 - KR / 2) % 4, valid = (8 - (KR - 1)) % 4;
+    const int shift = small_cin_words(g, dy, p);
+    if (shift == same || shift == valid) {
+#define TDH_DXS(CIN_) (shift == same ? launch_small_cin_dx_words<KR, CIN_, same>(g, p, batch, dy, w, dx, ag) \
+                                     : launch_small_cin_dx_words<KR, CIN_, valid>(g, p, batch, dy, w, dx, ag))
+      switch (g.C) {
+        case 1: TDH_DXS(1); return;
+        case 2: TDH_DXS(2); return;
+        case 3: TDH_DXS(3); return;
+        default: TDH_DXS(4); return;
+      }
+#undef TDH_DXS
+    }
+    p = plan;
+  }
   switch (KR ? g.C : DXS_MAX_CIN) {
     case 1: TDH_LAUNCH((conv_dx_small_cin_kernel<KR, KS, 1, POOLED>), grid, block, p.lds_bytes, ctx().stream, dy, w, dx, g, p, ag, pooled); break;
     case 2: TDH_LAUNCH((conv_dx_small_cin_kernel<KR, KS, 2, POOLED>), grid, block, p.lds_bytes, ctx().stream, dy, w, dx, g, p, ag, pooled); break;
