@@ -1233,3 +1233,26 @@ def test_weights_written_by_their_address_are_the_ones_used(T, O, W, flags, batc
         for i in convs:
             assert_close(net.get_param(i, 0), ref.weight(i), what=f"turn {turn} weights {i}")
     net.close()
+
+
+@pytest.mark.parametrize("batch", [1, 7, 300])
+@pytest.mark.parametrize("act", ["tanh", "relu", "sigmoid", "leaky_relu"])
+def test_dropout_and_the_activation_in_front_on_the_way_back(T, W, act, batch):
+    """A pointwise activation in front of a dropout layer leaves that layer's launch; the gradients of both, bit for bit."""
+    spec = [("fc", 12, 37), ("act", act, (0.2, 0.0)) if act == "leaky_relu" else ("act", act), ("dropout", 0.3), ("fc", 37, 5)]
+    rng = np.random.default_rng(11)
+    for flags in (0, T.NET_FUSE_ACT_GRAD):
+        net = T.Net(W.build_layers(T, spec), batch, flags)
+        for i, which, a in W.init_params(spec, "xavier", rng):
+            net.set_param(i, which, a)
+        mask = T.dropout_mask(T.Mt19937(5), 0.3, batch, 37)
+        net.set_dropout_mask(2, mask)
+        net.train_step(None, "mse", batch, T.to_device(rng.standard_normal((batch, 12)).astype(np.float32)),
+                       T.to_device(rng.standard_normal((batch, 5)).astype(np.float32)), do_update=False)
+        one, y = np.float32(1), net.layer_out(1, batch).reshape(batch, 37)
+        g = np.asarray(mask).reshape(batch, 37).astype(np.float32) * net.layer_dx(3, batch).reshape(batch, 37)
+        assert np.array_equal(net.layer_dx(2, batch).reshape(batch, 37), g)
+        want = {"tanh": lambda: g * (one - y * y), "relu": lambda: g * (y > 0).astype(np.float32),
+                "sigmoid": lambda: g * y * (one - y), "leaky_relu": lambda: g * np.where(y > 0, one, np.float32(0.2))}[act]()
+        assert np.array_equal(net.layer_dx(1, batch).reshape(batch, 37), want)
+        net.close()

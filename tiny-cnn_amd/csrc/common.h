@@ -326,6 +326,8 @@ struct BnMovingJobs {
 int batchnorm_update_moving(const BnMoving *jobs, int n);
 int dropout_fwd(size_t total, int train, float scale, const uint8_t *mask, const float *x, float *y);
 int dropout_bwd(size_t total, const uint8_t *mask, const float *dy, float *dx);
+// act: tanh, relu or sigmoid, with outputs y
+int dropout_act_bwd(size_t total, const uint8_t *mask, const float *dy, float *dx, int act, const float *y, float *act_dx);
 size_t rowsum_workspace_bytes(int outer, int rows, int cols);
 // out[c] (+)= sum_s src[s*cols + c]
 int launch_colsum(const float *src, int rows, int cols, float *out, int accumulate);

@@ -1181,6 +1181,7 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
   tdh_net::Layer &last = net->layers[n - 1];
   int first_bwd        = n - 1;
   int tail_done        = -1;     // this layer already has the gradient of its input
+  int act_done         = -1;     // an activation layer whose backward pass the dropout layer behind it did
   int pool_done        = -1;     // a max-pool layer whose backward pass the layer behind it did
   PoolGather through_pool;       // a max-pool layer whose backward pass the convolution in front
   int through_pool_for = -1;     // does while it reads its output gradient: that convolution
@@ -1425,7 +1426,7 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
         TDH_TRY(avepool_bwd(&s.pool, batch, in, L.w, L.dout, dx, L.dw, L.db, 1, fold));
         break;
       case TDH_L_ACT:
-        if (!L.grad_folded)
+        if (!L.grad_folded && i != act_done)
           TDH_TRY(launch_act_bwd(s.act, s.act_p, batch, static_cast<int>(L.out_size), in, L.out, L.dout, dx));
         break;
       case TDH_L_BATCHNORM:  // batch_normalization_layer.h:87-125
@@ -1434,8 +1435,15 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
         if (fold.kind != TDH_ACT_NONE) return set_error(TDH_ERR_INVALID, "batch-norm behind a folded activation");
         break;
       case TDH_L_DROPOUT:    // dropout_layer.h:62-82
-        TDH_TRY(dropout_bwd(L.out_size * static_cast<size_t>(batch), L.mask, L.dout, dx));
         if (fold.kind != TDH_ACT_NONE) return set_error(TDH_ERR_INVALID, "dropout behind a folded activation");
+        if (const tdh_net::Layer &A = net->layers[i - 1]; A.spec.kind == TDH_L_ACT && is_pointwise_act(A.spec.act) && !A.grad_folded) {
+          // the activation in front leaves the same kernel
+          const DxTarget through = dx_target(net, i - 1);
+          TDH_TRY(dropout_act_bwd(L.out_size * static_cast<size_t>(batch), L.mask, L.dout, dx, A.spec.act, A.out, through.dx));
+          act_done = i - 1;
+          break;
+        }
+        TDH_TRY(dropout_bwd(L.out_size * static_cast<size_t>(batch), L.mask, L.dout, dx));
         break;
     }
   }

@@ -335,6 +335,18 @@ dropout_bwd_kernel(const uint8_t *__restrict__ mask, const float *__restrict__ d
   dx[i] = static_cast<float>(mask[i]) * dy[i];
 }
 
+// The same, and through the pointwise activation in front of the dropout layer (tanh_layer.h:30-38, relu_layer.h:31-39,
+// sigmoid_layer.h:30-38, on its output y). Bound: a launch; of 37 x 64 values 1.9 and 2.2 us apart, 2.2 together, and the step of that net 1.4 % less.
+__global__ void __launch_bounds__(NT)
+dropout_act_bwd_kernel(const uint8_t *__restrict__ mask, const float *__restrict__ dy, const size_t total,
+                       float *__restrict__ dx, const int act, const float *__restrict__ y, float *__restrict__ act_dx) {
+  const size_t i = static_cast<size_t>(blockIdx.x) * NT + threadIdx.x;
+  if (i >= total) return;
+  const float g = static_cast<float>(mask[i]) * dy[i], v = y[i];
+  dx[i]     = g;
+  act_dx[i] = act == TDH_ACT_TANH ? g * (1.0f - v * v) : act == TDH_ACT_RELU ? g * (v > 0.0f ? 1.0f : 0.0f) : g * v * (1.0f - v);
+}
+
 int bn_groups(int batch) { return batch < 64 ? batch : 64; }
 
 // The elementwise passes: about 2048 workgroups where the tensor is large enough, and at least
@@ -501,6 +513,14 @@ int dropout_fwd(size_t total, int train, float scale, const uint8_t *mask, const
   ProfScope prof("dropout_fwd", (train ? 9.0 : 8.0) * total, WORK_BYTE);
   TDH_LAUNCH(dropout_fwd_kernel, dim3(static_cast<unsigned>(ceil_div_sz(total, NT))),
                      dim3(NT), 0, ctx().stream, train ? mask : nullptr, scale, x, total, y);
+  TDH_LAUNCH_CHECK();
+  return TDH_OK;
+}
+
+int dropout_act_bwd(size_t total, const uint8_t *mask, const float *dy, float *dx, int act, const float *y, float *act_dx) {
+  ProfScope prof("dropout_act_bwd", 17.0 * total, WORK_BYTE);
+  TDH_LAUNCH(dropout_act_bwd_kernel, dim3(static_cast<unsigned>(ceil_div_sz(total, NT))), dim3(NT), 0, ctx().stream, mask, dy,
+             total, dx, act, y, act_dx);
   TDH_LAUNCH_CHECK();
   return TDH_OK;
 }
