@@ -52,3 +52,31 @@ def test_exceptional_weight_gradient(T, value):
     assert (np.isfinite(got) == fits).all()
     rows = np.setdiff1d(np.arange(n_in), (7, 1023))
     assert np.abs(got[rows] - want[rows]).max() <= 2.0 ** -24 * 24 * (np.abs(x[:, rows]).T @ np.abs(dy)).max()
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("n_in,n_out,batch,slices", [
+    (4096, 4096, 256, True),
+    (3000, 3000, 100, True),       # the last 1024 sums and the last 32 columns in part
+    (2052, 4100, 130, False),      # dX on the fp32 kernel
+    (4096, 4096, 63, False),       # too few outputs for the sums of this form
+    (4096, 2050, 96, False),       # rows that dX cannot read by words
+])
+def test_sums_in_the_weight_gradients_launch(T, n_in, n_out, batch, slices, accumulate):
+    """dX and dW of one call: dW's launch adds up dX's slices and the columns of dY. The bits of each by itself, and the bias
+    gradient's error (the additions of its column)."""
+    rng = np.random.default_rng(83)
+    x, w, dy = (T.to_device(rng.standard_normal(s).astype(np.float32)) for s in ((batch, n_in), (n_in, n_out), (batch, n_out)))
+    before = [rng.standard_normal(s).astype(np.float32) for s in ((n_in, n_out), (n_out,))]
+    dw, db, alone = T.to_device(before[0]), T.to_device(before[1]), T.to_device(before[0])
+    dx, single = T.DevBuf((batch, n_in)), T.DevBuf((batch, n_in))
+    T.profile_begin()
+    T.fc_bwd(n_in, n_out, True, batch, x, w, dy, dx, dw, db, accumulate=accumulate)
+    tags = [r["tag"].split()[0] for r in T.profile_end()]
+    assert ("fc_dw_direct_sums" in tags) == slices and "bias_grad_colsum" not in tags, tags
+    T.fc_bwd(n_in, n_out, True, batch, x, w, dy, single, None, None)
+    T.fc_bwd(n_in, n_out, False, batch, x, w, dy, None, alone, None, accumulate=accumulate)
+    assert np.array_equal(dx.numpy(), single.numpy())
+    assert np.array_equal(dw.numpy(), alone.numpy())
+    d, prior = dy.numpy().astype(np.float64), before[1].astype(np.float64) * accumulate
+    assert (np.abs(db.numpy() - (d.sum(0) + prior)) <= 2.0 ** -24 * (batch + 2) * (np.abs(d).sum(0) + np.abs(prior))).all()

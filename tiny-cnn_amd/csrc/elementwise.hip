@@ -9,6 +9,7 @@
 #include "common.h"
 #include "opt_update.h"
 #include "conv_s1.h"
+#include "gemm_mfma.h"
 #include "split_bf16.h"
 
 namespace tdh {
@@ -648,29 +649,7 @@ __global__ void __launch_bounds__(EW_THREADS)
 colsum_kernel(const float *__restrict__ src, const int rows, const int cols,
               float *__restrict__ out, const int accumulate) {
   __shared__ float sm[8][32];
-  const int cl = threadIdx.x & 31, g = threadIdx.x >> 5;
-  const int c  = blockIdx.x * 32 + cl;
-  float s = 0.0f;
-  if (c < cols) {
-    // eight loads in flight, added in row order (one at a time each add waits a trip to memory)
-    int r = g;
-    for (; r + 56 < rows; r += 64) {
-      float v[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] = src[static_cast<size_t>(r + 8 * k) * cols + c];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) s += v[k];
-    }
-    for (; r < rows; r += 8) s += src[static_cast<size_t>(r) * cols + c];
-  }
-  sm[g][cl] = s;
-  __syncthreads();
-  if (g == 0 && c < cols) {
-    float t = sm[0][cl];
-#pragma unroll
-    for (int i = 1; i < 8; ++i) t += sm[i][cl];
-    out[c] = accumulate ? out[c] + t : t;
-  }
+  colsum_block(src, rows, cols, out, accumulate, blockIdx.x, sm);
 }
 
 }  // namespace

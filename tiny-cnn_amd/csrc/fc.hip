@@ -991,10 +991,17 @@ int fc_fwd(int in, int out, int has_bias, int batch, const float *x, const float
 constexpr int FDW_WM = 2, FDW_WN = 2;     // waves of a workgroup along the two
 constexpr int FDW_DEPTH = 4;              // sample pairs per group of loads
 
+// In front of the products, shared out evenly over the workgroups: the slices of dX (whose launch was the one before) added
+// up, and the bias gradient's column sums. 4096 x 4096, batch 256, us: launches of their own 8.6 + 4.8, here 7.5 of the kernel's
+// (half of the workgroups behind their products instead, so that the other one on a compute unit has the matrix cores
+// meanwhile: no different); 3000 x 3000, batch 100, the layer's forward, backward and update 154.5 / 150.
 struct FcDwDirect {
   const float *x, *dy;
   float *dw;
   int batch, in, out, accumulate;
+  LeftSums sums;             // (sum_blocks of 1024 outputs, or 0)
+  float *db;
+  int sum_blocks, db_blocks; // (db_blocks of 32 columns, or 0)
 };
 
 typedef float fdw_x16 __attribute__((ext_vector_type(16)));
@@ -1007,8 +1014,20 @@ fc_dw_direct_kernel(const FcDwDirect f) {
   constexpr int FDW_TM = 32 * CA, FDW_TN = 32 * CB;
   typedef float avec __attribute__((ext_vector_type(CA)));
   typedef float bvec __attribute__((ext_vector_type(CB)));
+  static_assert(64 * FDW_WM * FDW_WN == 256, "the sums are for 256 threads");
+  __shared__ float col_sums[8][32];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = lane & 31, h = lane >> 5;
+  const unsigned self = blockIdx.x + gridDim.x * blockIdx.y, all = gridDim.x * gridDim.y;
+  {
+    auto first = [&](unsigned i, int blocks) { return static_cast<unsigned>(static_cast<unsigned long long>(i) * blocks / all); };
+    for (unsigned u = first(self, f.sum_blocks); u < first(self + 1, f.sum_blocks); ++u)
+      splitk_reduce_wide(f.sums.partial, f.sums.splits, f.sums.M, f.sums.N, f.sums.epi, u);
+    for (unsigned u = first(self, f.db_blocks); u < first(self + 1, f.db_blocks); ++u) {
+      colsum_block(f.dy, f.batch, f.out, f.db, f.accumulate, u, col_sums);
+      __syncthreads();   // (the next one's)
+    }
+  }
   // Workgroups go to the eight XCDs (each with its own L2) round-robin in launch order. Each
   // XCD gets a compact block of the tile grid (a quarter of the rows x half of the columns
   // where the grid divides so, else a run of consecutive tiles), so that the panels its
@@ -1097,8 +1116,7 @@ fc_dw_direct_kernel(const FcDwDirect f) {
 
   // reg r of lane l of block (c, d): input i0 + CA*(8*(r/4) + 4*(l/32) + r%4) + c, output
   // o0 + 2*(l%32) + d; the two blocks d leave as one 8-byte store
-  if (!b_ok) return;
-  float *out = f.dw + o0 + CB * m;
+  float *out = f.dw + (b_ok ? o0 + CB * m : 0);
   // (rows past the layer's inputs are read and written at row i0, with what row i0 holds:
   // loads and stores without conditions, sixteen loads in flight when the sums are added to
   // what the gradient held)
@@ -1115,7 +1133,7 @@ fc_dw_direct_kernel(const FcDwDirect f) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int i = i0 + CA * (8 * (r >> 2) + 4 * h + (r & 3)) + c;
-      if (i >= f.in) continue;
+      if (i >= f.in || !b_ok) continue;
       bvec v;
 #pragma unroll
       for (int d = 0; d < CB; ++d) v[d] = f.accumulate ? old[r][d] + acc[c][d][r] : acc[c][d][r];
@@ -1362,6 +1380,10 @@ int fc_bwd(int in, int out, int has_bias, int batch, const float *x, const float
     TDH_LAUNCH_CHECK();
     return TDH_OK;
   }
+  // dW straight from memory also adds up what dX leaves in slices, and the bias gradient
+  const bool dw_direct = dw && !small_fc_applies(in, out, batch) && !fc_x3_applies(FX_A_M_B_N, in, out, batch, x, dy, in, out) &&
+                         fc_dw_direct_applies(in, out, batch, x, dy, dw);
+  LeftSums left{};
   if (dx) {
     StridedOperand A{dy, out, 1, batch};  // dY[s][k]
     StridedOperand B{w, out, 1, in};      // W[n][k], k contiguous
@@ -1369,7 +1391,8 @@ int fc_bwd(int in, int out, int has_bias, int batch, const float *x, const float
     if (small_fc_applies(batch, in, out)) {
       TDH_TRY(launch_small_fc(A, B, epi, batch, in, out, "fc_dx_small"));
     } else if (fc_x3_applies(FX_A_K_B_K, batch, in, out, dy, w, out, out)) {
-      TDH_TRY(fc_x3_run(FX_A_K_B_K, dy, w, out, out, epi, batch, in, out, "fc_dx_x3", "fc_dx_splitk_reduce"));
+      TDH_TRY(fc_x3_run(FX_A_K_B_K, dy, w, out, out, epi, batch, in, out, "fc_dx_x3", "fc_dx_splitk_reduce",
+                        dw_direct ? &left : nullptr));
     } else if (fc_dx_tile_applies(in, out, batch, dy, w)) {
       ProfScope prof("fc_dx_tile", batch, in, out);
       FcDxTile f{dy, w, dx, dx_act, batch, in, out, ceil_div(batch, 64), ceil_div(in, 64), 0};
@@ -1388,9 +1411,10 @@ int fc_bwd(int in, int out, int has_bias, int batch, const float *x, const float
       TDH_TRY(launch_small_fc(A, B, epi, in, out, batch, "fc_dw_small"));
     } else if (fc_x3_applies(FX_A_M_B_N, in, out, batch, x, dy, in, out)) {
       TDH_TRY(fc_x3_run(FX_A_M_B_N, x, dy, in, out, epi, in, out, batch, "fc_dw_x3", "fc_dw_splitk_reduce"));
-    } else if (fc_dw_direct_applies(in, out, batch, x, dy, dw)) {
-      ProfScope prof("fc_dw_direct", in, out, batch);
-      const FcDwDirect f{x, dy, dw, batch, in, out, accumulate};
+    } else if (dw_direct) {
+      ProfScope prof(left.partial ? "fc_dw_direct_sums" : "fc_dw_direct", in, out, batch);
+      const FcDwDirect f{x, dy, dw, batch, in, out, accumulate, left, db, left.partial ? ceil_div(batch * in, REDUCE_WIDE_OUTPUTS) : 0,
+                         bias_grad ? ceil_div(out, 32) : 0};
       TDH_LAUNCH((fc_dw_direct_kernel<4, 2>), dim3(ceil_div(out, 64 * FDW_WN), ceil_div(in, 128 * FDW_WM)),
                  dim3(64 * FDW_WM * FDW_WN), 0, ctx().stream, f);
       TDH_LAUNCH_CHECK();
@@ -1398,7 +1422,7 @@ int fc_bwd(int in, int out, int has_bias, int batch, const float *x, const float
       TDH_TRY((launch_gemm<false, false, true, true>(A, B, epi, in, out, batch, true, "fc_dw_gemm",
                                                    "fc_dw_splitk_reduce")));
   }
-  if (db && has_bias) TDH_TRY(launch_colsum(dy, batch, out, db, accumulate));
+  if (bias_grad && !dw_direct) TDH_TRY(launch_colsum(dy, batch, out, db, accumulate));
   return TDH_OK;
 }
 

@@ -298,7 +298,7 @@ size_t fc_x3_workspace_bytes(int M, int N, int K) {
 
 template <class Epi>
 static int run_fx(FxRows rows, const float *A, const float *B, int lda, int ldb, const Epi &epi, int M, int N, int K,
-                  const char *tag, const char *reduce_tag) {
+                  const char *tag, const char *reduce_tag, LeftSums *leave = nullptr) {
   const FxPlan p = fx_plan(M, N, K);
   float *partial = nullptr;
   if (p.splits > 1) {
@@ -315,11 +315,17 @@ static int run_fx(FxRows rows, const float *A, const float *B, int lda, int ldb,
               : rows == FX_A_K_B_N ? (launch_fx<true, false>(p, A, B, lda, ldb, epi, M, N, K, partial))
                                    : (launch_fx<false, false>(p, A, B, lda, ldb, epi, M, N, K, partial)));
   }
+  if constexpr (std::is_same<Epi, EpiRowMajor>::value) {
+    if (leave && p.splits > 1 && !ctx().defer_reduce && N % 4 == 0 && static_cast<long>(M) * N >= REDUCE_WIDE_MIN) {
+      *leave = LeftSums{partial, p.splits, M, N, epi};   // (the order of the wide kernel, which would add them up)
+      return TDH_OK;
+    }
+  }
   return p.splits > 1 ? launch_splitk_reduce(partial, p.splits, M, N, epi, reduce_tag) : TDH_OK;
 }
 int fc_x3_run(FxRows rows, const float *A, const float *B, int lda, int ldb, const EpiRowMajor &epi, int M, int N, int K,
-              const char *tag, const char *reduce_tag) {
-  return run_fx(rows, A, B, lda, ldb, epi, M, N, K, tag, reduce_tag);
+              const char *tag, const char *reduce_tag, LeftSums *leave) {
+  return run_fx(rows, A, B, lda, ldb, epi, M, N, K, tag, reduce_tag, leave);
 }
 int fc_x3_run_act(const float *A, const float *B, int lda, int ldb, const EpiRowMajorAct &epi, int M, int N, int K,
                   const char *tag, const char *reduce_tag) {

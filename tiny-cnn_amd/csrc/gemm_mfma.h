@@ -86,6 +86,34 @@ struct StridedOperand {
   }
 };
 
+// The sums of 32 columns of a matrix of `rows` rows, by 256 threads: eight share a column's rows, sm is [8][32] in LDS.
+__device__ __forceinline__ void colsum_block(const float *__restrict__ src, const int rows, const int cols, float *__restrict__ out,
+                                             const int accumulate, const int block, float (&sm)[8][32]) {
+  const int cl = threadIdx.x & 31, g = threadIdx.x >> 5;
+  const int c  = block * 32 + cl;
+  float s = 0.0f;
+  if (c < cols) {
+    // eight loads in flight, added in row order (one at a time each add waits a trip to memory)
+    int r = g;
+    for (; r + 56 < rows; r += 64) {
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = src[static_cast<size_t>(r + 8 * k) * cols + c];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s += v[k];
+    }
+    for (; r < rows; r += 8) s += src[static_cast<size_t>(r) * cols + c];
+  }
+  sm[g][cl] = s;
+  __syncthreads();
+  if (g == 0 && c < cols) {
+    float t = sm[0][cl];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) t += sm[i][cl];
+    out[c] = accumulate ? out[c] + t : t;
+  }
+}
+
 // ------------------------------------------------------------------ epilogues
 // out[m*ld + n] = (accumulate ? out : 0) + (v + bias_n[n]) * act'(y[m*ld + n])
 struct EpiRowMajor {
@@ -197,8 +225,15 @@ __device__ __forceinline__ int tile_k(const Op &, int, int K) { return K; }
 enum FxRows { FX_A_K_B_K, FX_A_K_B_N, FX_A_M_B_N };
 bool fc_x3_applies(FxRows rows, int M, int N, int K, const float *A, const float *B, int lda, int ldb);
 size_t fc_x3_workspace_bytes(int M, int N, int K);
+// the slices of a product that another launch adds up (splitk_reduce_wide), or none
+struct LeftSums {
+  const float *partial;
+  int splits, M, N;
+  EpiRowMajor epi;
+};
+// (leave: may be null)
 int fc_x3_run(FxRows rows, const float *A, const float *B, int lda, int ldb, const EpiRowMajor &epi, int M, int N, int K,
-              const char *tag, const char *reduce_tag);
+              const char *tag, const char *reduce_tag, LeftSums *leave = nullptr);
 // fc_f32.hip: C = A B of plain matrices in fp32 with the bits of launch_gemm, A rows along k, B rows along n
 bool fc_f32_applies(int M, int N, int K, const float *A, const float *B);
 int fc_f32_run(const float *A, const float *B, const EpiRowMajor &epi, int M, int N, int K, const char *tag, const char *reduce_tag);
@@ -585,13 +620,13 @@ splitk_reduce_kernel(const float *__restrict__ partial, const int splits, const 
 // goes to group z % 8 and the groups are added in order, so the result is the one of the
 // kernel above bit for bit; that kernel gives a workgroup 32 outputs, which for a million
 // outputs and eight slices is 32768 workgroups of one load a thread.
+constexpr int REDUCE_WIDE_OUTPUTS = 1024;   // of 256 threads
 template <class Epi>
-__global__ void __launch_bounds__(256)
-splitk_reduce_wide_kernel(const float *__restrict__ partial, const int splits, const int M, const int N,
-                          const Epi epi) {
+__device__ __forceinline__ void splitk_reduce_wide(const float *__restrict__ partial, const int splits, const int M, const int N,
+                                                   const Epi &epi, const unsigned block) {
   typedef float f4 __attribute__((ext_vector_type(4)));
   const size_t mn = static_cast<size_t>(M) * N;
-  const size_t idx = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
+  const size_t idx = (static_cast<size_t>(block) * 256 + threadIdx.x) * 4;
   if (idx >= mn) return;
   f4 s[REDUCE_GROUPS];
 #pragma unroll
@@ -618,6 +653,12 @@ splitk_reduce_wide_kernel(const float *__restrict__ partial, const int splits, c
   }
 #pragma unroll
   for (int e = 0; e < 4; ++e) epi.store(m, c[e], t[e], before[e]);
+}
+template <class Epi>
+__global__ void __launch_bounds__(256)
+splitk_reduce_wide_kernel(const float *__restrict__ partial, const int splits, const int M, const int N,
+                          const Epi epi) {
+  splitk_reduce_wide(partial, splits, M, N, epi, blockIdx.x);
 }
 constexpr long REDUCE_WIDE_MIN = 1L << 18;  // outputs from which the wide kernel is launched
 
