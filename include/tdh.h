@@ -276,10 +276,11 @@ enum {
   TDH_NET_FUSE_ACT_GRAD = 1, /* fold activation gradients into the next layer's dX epilogue */
   TDH_NET_GRAPH         = 2, /* replay the step as a captured HIP graph */
   /* A net whose activations of one sample fit in a workgroup's local memory (LeNet-5) trains in
-   * three launches: one workgroup per sample runs forward, the loss gradient and the input
-   * gradients of every layer; a second launch computes every sample's weight and bias
-   * gradients; the optimizer launch adds those up and updates (a step without an update adds
-   * them to the gradient tensors in sample order instead, edge::merge_grads,
+   * two to five launches: one workgroup per sample runs forward, the loss gradient and the input
+   * gradients of the layers (the first block and the way back to it, a channel a workgroup, in launches of
+   * their own for small batches); one launch computes the weight and bias gradients over the batch and, up to 32
+   * samples, updates; larger batches leave a slice per group of samples, which the optimizer launch adds up (a step
+   * without an update adds to the gradient tensors in sample order instead, edge::merge_grads,
    * tiny_dnn/node.h:89-103). Every layer output, input gradient and max-pool record is still
    * written to memory. Nets that do not qualify (size, batch normalization, dropout, a softmax
    * that is not the closing layer of a cross_entropy_multiclass net) ignore the flag. */

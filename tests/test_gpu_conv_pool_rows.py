@@ -28,7 +28,7 @@ def test_pool_of_rows_as_its_own_kernel(T, W, width, height, in_c, out_c, window
     w = rng.uniform(-0.3, 0.3, out_c * in_c * window * window).astype(np.float32)
     b = np.linspace(-0.2, 0.2, out_c, dtype=np.float32)
     x = T.to_device(rng.standard_normal((batch, width * height * in_c)).astype(np.float32))
-    net = T.Net(W.build_layers(T, spec), batch, 0)
+    net = T.Net(W.build_layers(T, spec), batch, T.NET_FUSE_ACT_GRAD if form == "train" and not act else 0)
     net.set_param(0, 0, w)
     net.set_param(0, 1, b)
     pool = 2 if act else 1

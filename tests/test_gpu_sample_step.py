@@ -1,7 +1,7 @@
 """TDH_NET_SAMPLE_STEP: a small net trains with one workgroup per sample (forward, loss gradient
-and the input gradients in one launch out of LDS), a launch for every sample's weight and bias
-gradients, and the optimizer launch that adds them up (a step without an update adds them in
-sample order with a launch of its own). Against the oracle (every layer output, input gradient,
+and the input gradients in one launch out of LDS, for small batches with the ends of that chain in
+two more), a launch for the weight and bias gradients over the batch, which updates, or leaves slices
+that the optimizer launch adds up (a step without an update adds them with a launch of its own). Against the oracle (every layer output, input gradient,
 max-pool record, weight and bias gradient; updated weights over several steps), against the
 layer-by-layer step of the same library, against tiny-dnn's own fit (tests/golden/net_steps.npz),
 and replayed from a captured graph bit for bit."""

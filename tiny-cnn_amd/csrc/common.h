@@ -393,6 +393,8 @@ bool conv_fwd_packs_along(const tdh_conv_desc *d, int batch);
 // the forward kernel of this layer can leave `y` out (null) when it writes the activation layer
 // or the pool behind the convolution itself
 bool conv_fwd_out_optional(const tdh_conv_desc *d, int batch, bool prepacked);
+// a train step may leave the convolution's own output unwritten where the pool directly behind it leaves its kernel
+bool conv_fwd_pool_replaces_out(const tdh_conv_desc *d, int batch, bool prepacked);
 // conv_fwd_direct.hip: forward pass of a layer that is a few small tiles, with the layers behind it
 bool conv_fwd_direct_applicable(int batch, int C, int Kc, int H, int W, int OH, int OW, int R, int S);
 int conv_fwd_direct_run(int batch, int C, int Kc, const float *x, const float *w, const float *bias, float *out, int H, int W,
@@ -493,6 +495,8 @@ int conv_s1_run(int R, int S, int batch, int C, int Kc, int flip, const float *i
 // a relu behind that pool); `out` may then be null
 bool conv_s1_fuses_pool(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW,
                         int ph, int pw);
+// its tiles are rows of 8 or 16 pixels
+bool conv_s1_short_rows(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw);
 // one pass over the reduction channels: the kernel's epilogue is the only writer of `out`
 bool conv_s1_single_pass(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW,
                          int ph, int pw);

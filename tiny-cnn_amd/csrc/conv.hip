@@ -1502,6 +1502,13 @@ bool conv_fwd_fuses_pool(const tdh_conv_desc *d, const tdh_pool_desc *pool, int 
          conv_s1_fuses_pool(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
 }
 
+// with the pool alone behind it (in longer rows the convolution's own output is what a train step has always left there)
+bool conv_fwd_pool_replaces_out(const tdh_conv_desc *d, int batch, bool prepacked) {
+  const ConvGeom g = make_geom(d);
+  if (!prepacked && (fwd_direct_applies(g, batch) || fwd_small_applies(g, batch))) return true;
+  return conv_s1_short_rows(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
+}
+
 bool conv_fwd_out_optional(const tdh_conv_desc *d, int batch, bool prepacked) {
   const ConvGeom g = make_geom(d);
   if (!prepacked && (fwd_direct_applies(g, batch) || fwd_small_applies(g, batch))) return true;

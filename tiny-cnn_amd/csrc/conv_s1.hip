@@ -227,6 +227,12 @@ bool conv_s1_fuses_pool(int R, int S, int batch, int KC, int MC, int IH, int IW,
          static_cast<long>(MC) * OH * OW < (1L << 31);
 }
 
+// tiles of rows of 8 or 16 pixels
+bool conv_s1_short_rows(int R, int S, int batch, int KC, int MC, int IH, int IW, int OH, int OW, int ph, int pw) {
+  const S1Plan p = make_plan(R, S, batch, KC, MC, IH, IW, OH, OW, ph, pw);
+  return p.ok && p.tc <= 16;
+}
+
 // packed filters and the partial sums of a split
 size_t plan_workspace_bytes(const S1Plan &p, int RS) {
   const size_t packed = ws_align(conv_s1_packed_bytes(p.x3 ? CONV_PACK_X3 : CONV_PACK_F32, RS, p.args.KC, p.args.MC));

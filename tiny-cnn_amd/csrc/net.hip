@@ -237,9 +237,9 @@ bool tiny_step_applies(const tdh_net *net, int loss_kind);
 // 587; six 3x3 layers of 32 channels of 24x24, batch 128 513 / 509; three 5x5 layers of 48 channels of 12x12,
 // batch 64 241 / 241, batch 256 628 / 623; 784-1000-1000-10 fully connected, batch 1024 273 / 268; 1024-4096-4096-10,
 // batch 64 286 / 281. Below it the two are within 1 % of each other, and a replay leaves the host free. The step of a
-// workgroup per sample (tiny_net.hip) is three launches of 40, 9 and 5 us at least, whatever the net and the batch:
-// LeNet-5, batch 16 58.6 / 54.8, fed from the host in batches of 13 66.9 / 60.2 and of 221 136.6 / 128.3; the call
-// takes the host 14 to 19 / 11.
+// workgroup per sample (tiny_net.hip) is two to five launches of 4 to 40 us, whatever the net and the batch (with the
+// three of 40, 9 and 5 that it once was, LeNet-5, batch 16 58.6 / 54.8, fed from the host in batches of 13 66.9 / 60.2 and of 221
+// 136.6 / 128.3; the call takes the host 14 to 19 / 11).
 bool step_outlasts_launches(const tdh_net *net, int loss_kind, int batch) {
   if (tiny_step_applies(net, loss_kind)) return true;
   return !net_forks(net, batch) &&
@@ -663,7 +663,7 @@ int forward(tdh_net *net, int batch, const float *x, const float *xent_t = nullp
           LeaveSplitSum leave(ctx(), last == i && i + 1 < n && net->layers[i + 1].spec.kind == TDH_L_MAXPOOL);
           // (the backward pass reads the outputs of the layers that left the kernel, never the
           // convolution's own: the gradients of the pointwise activations are functions of y)
-          const bool own_out = !((net->flags & TDH_NET_FUSE_ACT_GRAD) && training && ((pf.out && !act_out) ||
+          const bool own_out = !((net->flags & TDH_NET_FUSE_ACT_GRAD) && training && ((pf.out && !act_out && conv_fwd_pool_replaces_out(&s.conv, batch, has_wp)) ||
                                               (act_out && conv_fwd_out_optional(&s.conv, batch, has_wp))));
           if (!own_out) net->out_unwritten[i] = 1;
           TDH_TRY(conv2d_fwd(&s.conv, batch, in, L.w, L.b, own_out ? L.out : nullptr, L.tbl_dev, wp, act_out, act_kind,

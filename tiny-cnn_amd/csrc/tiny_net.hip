@@ -1484,7 +1484,7 @@ tiny_net_step_kernel(const TinyPlan *__restrict__ plan, const int m, const int l
 // keeps to one channel: a workgroup takes one channel of a sample through it, forward in a launch in
 // front of the step kernel, and in a launch behind it from the second convolution's dX back to the
 // gradient of the first one's output. Bound: latency, a launch and some three trips to memory each.
-// LeNet-5, batch 16, us: one launch 34; here 4.5 + 17.3 + 7.8 (which batches: launch_tiny_step).
+// LeNet-5, batch 16, us: here 4.5 + 17.3 + 7.8, and the whole step 40.7 where in one launch it is 52.1 (which batches: launch_tiny_step).
 constexpr int TF_THREADS = 1024;   // front, at most
 constexpr int TB_THREADS = 1024;   // back
 static_assert(TB_THREADS / 64 == 16, "sixteen shares of a pool's sums; a wave left over from five rows of three and from three of five");
@@ -2605,8 +2605,8 @@ int tiny_layout(TinyPlan &P) {
 }
 
 // The ends of the chain a channel a workgroup while there is a compute unit for each. LeNet-5's step, us, with them / one
-// workgroup per sample throughout: 16 samples 46.6 / 56.4, 32 48.7 / 57.9, 42 57.4 / 60.1, 44 64.0 / 61.3, 64 67.2 / 64.8, 104 82.8 /
-// 73.5: with several workgroups a compute unit, each of which frames all of dY for its one channel, they lose.
+// workgroup per sample throughout: 16 samples 40.7 / 52.1, 32 43.1 / 54.0, 42 50.7 / 55.8, 44 57.4 / 56.4, 64 60.6 / 61.4, 104 77.1 /
+// 70.7: with several workgroups a compute unit, each of which frames all of dY for its one channel, they lose.
 int tiny_most_split(const TinyPlan &plan) { return plan.split ? 256 / std::max(plan.l[0].K, plan.l[plan.split].C) : 0; }
 static bool tiny_splits(const TinyPlan &plan, int batch) { return batch <= tiny_most_split(plan); }
 // A batch of up to 32 samples is one group, whose workgroups update; the groups of a larger one are of 16, which
