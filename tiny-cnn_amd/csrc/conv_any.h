@@ -15,7 +15,7 @@ struct AnyPack {
   const float *w;
   uintx4_any *wp;
   int M, KC, m_pad, wm, wk, total;
-  int blocks, first_x;   // workgroups; the first of them along a larger grid's x
+  int blocks, first;     // workgroups; the number of the first of them in a larger launch
   FastDiv div_m, div_rs;
 };
 // slices [splits][M][N] of a weight gradient, added up by gemm_mfma.h's tree

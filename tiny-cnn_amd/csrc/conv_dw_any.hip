@@ -37,24 +37,31 @@ struct DwAnyArgs {
   int plane;                 // words of one channel's staged rows
   int pixels, per;           // of the batch, of a slice
   int x_at, dy_at;           // words of LDS in front of the staged tensors
+  FastDiv div_slices, div_n_tiles;   // of a workgroup's number where others follow: slices, then tiles of columns, then tiles of channels
   FastDiv div_pix, div_nx, div_hv, div_pw, div_sx, div_rs, div_s;
 };
 
-// MB blocks of 16 channels; NB blocks of 16 columns to each of the four waves; CH pixels a chunk
-template <int MB, int NB, int CH>
+// MB blocks of 16 channels; NB blocks of 16 columns to each of the four waves; CH pixels a chunk. PACK: workgroups behind the
+// slices' pack filters (an instance of its own, as in conv_any_kernel).
+template <int MB, int NB, int CH, bool PACK>
 __global__ void __launch_bounds__(256, 2) conv_dw_any_kernel(const DwAnyArgs a, const AnyPack pack) {
-  if (static_cast<int>(blockIdx.x) >= pack.first_x) {   // (behind the slices)
-    const int block = ((static_cast<int>(blockIdx.x) - pack.first_x) * gridDim.y + blockIdx.y) * gridDim.z + blockIdx.z;
-    if (block < pack.blocks) any_pack_block(pack, block);
+  if (PACK && static_cast<int>(blockIdx.x) >= pack.first) {
+    any_pack_block(pack, static_cast<int>(blockIdx.x) - pack.first);
     return;
+  }
+  uint32_t slice = blockIdx.x, n_tile = blockIdx.y, m_tile = blockIdx.z;
+  if (PACK) {
+    uint32_t tile;
+    a.div_slices.divmod(blockIdx.x, tile, slice);
+    a.div_n_tiles.divmod(tile, m_tile, n_tile);
   }
   constexpr int DYP = CH + 4;        // (sixteen channels' 16-byte reads cover all banks)
   constexpr int ROWS = 256 / CH;     // channels of dY staged side by side
   extern __shared__ __align__(16) int dwa_lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, quarter = lane >> 4;
-  const int n0 = blockIdx.y * (64 * NB), m0 = blockIdx.z * (16 * MB);
-  const int first = blockIdx.x * a.per, end = min(first + a.per, a.pixels);
+  const int n0 = static_cast<int>(n_tile) * (64 * NB), m0 = static_cast<int>(m_tile) * (16 * MB);
+  const int first = static_cast<int>(slice) * a.per, end = min(first + a.per, a.pixels);
   int *pos   = dwa_lds;                                       // [CH]
   float *dys = reinterpret_cast<float *>(dwa_lds) + a.dy_at;  // [16 * MB][DYP]
   float *xs  = reinterpret_cast<float *>(dwa_lds) + a.x_at;   // [channel][plane]
@@ -199,7 +206,7 @@ __global__ void __launch_bounds__(256, 2) conv_dw_any_kernel(const DwAnyArgs a, 
     }
   }
 
-  float *to = a.partial + static_cast<size_t>(blockIdx.x) * a.M * a.N;
+  float *to = a.partial + static_cast<size_t>(slice) * a.M * a.N;
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -217,7 +224,7 @@ struct DwAnyPlan {
   bool ok;
   int mb, nb, ch, slices;
   size_t lds_bytes;
-  dim3 grid;
+  int n_tiles, m_tiles;
   DwAnyArgs args;
   double cost;
 };
@@ -261,7 +268,7 @@ DwAnyPlan plan_tile(const ConvShape &c, bool with_db, int nb, int ch, int rounds
   a.per    = std::max(a.per, 64);
   p.slices = ceil_div(a.pixels, a.per);
   if (n_tiles > 65535 || m_tiles > 65535) return p;
-  p.grid = dim3(p.slices, n_tiles, m_tiles);
+  p.n_tiles = n_tiles; p.m_tiles = m_tiles;
   // Estimated us with the reduction, fitted to 92 shapes at every tile (8 to 460 us; over 400 others the chosen tile is 2 % off
   // the best one): what a workgroup waits for by itself, what the workgroups of a
   // compute unit share, and how many of them run at once.
@@ -301,9 +308,9 @@ const DwAnyPlan &make_plan(const ConvShape &c, bool with_db) {
   return best;
 }
 
-template <int MB, int NB, int CH>
-int launch_inst(const DwAnyPlan &p, const AnyPack &pack) {
-  auto kernel = conv_dw_any_kernel<MB, NB, CH>;
+template <int MB, int NB, int CH, bool PACK>
+int launch_pack(const DwAnyPlan &p, const AnyPack &pack) {
+  auto kernel = conv_dw_any_kernel<MB, NB, CH, PACK>;
   if (p.lds_bytes > 64 * 1024) {
     static size_t raised = 0;
     if (p.lds_bytes > raised) {
@@ -312,10 +319,14 @@ int launch_inst(const DwAnyPlan &p, const AnyPack &pack) {
       raised = p.lds_bytes;
     }
   }
-  const unsigned extra = ceil_div(pack.blocks, static_cast<int>(p.grid.y * p.grid.z));
-  TDH_LAUNCH(kernel, dim3(p.grid.x + extra, p.grid.y, p.grid.z), dim3(256), p.lds_bytes, ctx().stream, p.args, pack);
+  const dim3 grid = PACK ? dim3(pack.first + pack.blocks) : dim3(p.slices, p.n_tiles, p.m_tiles);
+  TDH_LAUNCH(kernel, grid, dim3(256), p.lds_bytes, ctx().stream, p.args, pack);
   TDH_LAUNCH_CHECK();
   return TDH_OK;
+}
+template <int MB, int NB, int CH>
+int launch_inst(const DwAnyPlan &p, const AnyPack &pack) {
+  return pack.blocks ? launch_pack<MB, NB, CH, true>(p, pack) : launch_pack<MB, NB, CH, false>(p, pack);
 }
 template <int MB, int NB>
 int launch_nb(const DwAnyPlan &p, const AnyPack &pack) {
@@ -375,7 +386,13 @@ int conv_dw_any_run(const ConvShape &c, const float *x, const float *dy, bool wi
   *slices  = p.slices;
   AnyPack side{};
   if (pack) side = *pack;
-  side.first_x = static_cast<int>(p.grid.x);
+  // (Behind all of the products' workgroups: those are planned as whole rounds of the chip, and a few in between
+  // push as many of the last ones into a round of their own. us, dX, dW and db, packing apart / in between / behind: 13x50, 38 -> 155,
+  // 7x7, stride 2, 54 images 137 / 186 / 134; 93x67, 10 -> 133, 7x7, 44 images 1106 / 1326 / 1100; 31x93, 33 -> 2, 7x7, 82 images
+  // 264 / 325 / 261; 45x37, 21 -> 45, 5x5, stride 2, 19 images 34.8 / 27.7 / 27.9.)
+  side.first    = p.slices * p.n_tiles * p.m_tiles;
+  a.div_slices  = FastDiv(p.slices);
+  a.div_n_tiles = FastDiv(p.n_tiles);
   ProfScope prof(with_db ? "conv_dw_db_any" : "conv_dw_any", a.M, a.N, a.pixels);
   switch (p.mb) {
     case 1: return launch_mb<1>(p, side);
