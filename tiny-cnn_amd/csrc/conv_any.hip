@@ -97,15 +97,17 @@ __device__ __forceinline__ float any_redo(const AnyArgs &a, const AnyPhase &ph, 
   return sum;
 }
 
-// MB x NB: blocks of 16 channels x 16 pixels of a wave; WK waves share the units, 4 / WK the pixels.
-template <int MB, int NB, int WK>
+// MB x NB: blocks of 16 channels x 16 pixels of a wave; WK waves share the units, 4 / WK the pixels. SUMS: workgroups behind the
+// tiles add up dW's slices. (An instance of its own: the look at whether there are any, a scalar load in front of everything else, takes 0.4 us
+// of 10 to 30. dX of 12x82, 10 <- 60, 3x3, 14 images 13.1 us without it, 13.5 with.)
+template <int MB, int NB, int WK, bool SUMS>
 __global__ void __launch_bounds__(256, 2) conv_any_kernel(const AnyArgs a, const AnySums sums) {
   constexpr int WN    = 4 / WK;
   constexpr int PIX   = WN * NB * 16;
   constexpr int ITEMS = 2;           // patch words a thread has under way
   constexpr int DEPTH = WK == 4 && MB * NB <= 6 ? 2 : 1;   // (few steps, and filters fresh from another XCD)
   extern __shared__ __align__(16) uintx4 any_lds[];
-  if (static_cast<int>(blockIdx.x) >= sums.first_x) {   // (behind the tiles)
+  if (SUMS && static_cast<int>(blockIdx.x) >= sums.first_x) {
     const int block = (static_cast<int>(blockIdx.x) - sums.first_x) * gridDim.y + blockIdx.y;
     if (block < sums.blocks)
       any_sums_block(sums, block, reinterpret_cast<float(*)[ANY_SUMS]>(any_lds));
@@ -548,9 +550,9 @@ void finish_args(AnyArgs &a) {
   }
 }
 
-template <int MB, int NB, int WK>
-int launch_any_inst(const AnyPlan &p, const AnySums &sums) {
-  auto kernel = conv_any_kernel<MB, NB, WK>;
+template <int MB, int NB, int WK, bool SUMS>
+int launch_any_sums(const AnyPlan &p, const AnySums &sums) {
+  auto kernel = conv_any_kernel<MB, NB, WK, SUMS>;
   if (p.lds_bytes > 64 * 1024) {
     static size_t raised = 0;
     if (p.lds_bytes > raised) {
@@ -563,6 +565,10 @@ int launch_any_inst(const AnyPlan &p, const AnySums &sums) {
   TDH_LAUNCH(kernel, dim3(p.grid.x + extra, p.grid.y), dim3(256), p.lds_bytes, ctx().stream, p.args, sums);
   TDH_LAUNCH_CHECK();
   return TDH_OK;
+}
+template <int MB, int NB, int WK>
+int launch_any_inst(const AnyPlan &p, const AnySums &sums) {
+  return sums.blocks ? launch_any_sums<MB, NB, WK, true>(p, sums) : launch_any_sums<MB, NB, WK, false>(p, sums);
 }
 template <int MB>
 int launch_any_mb(const AnyPlan &p, const AnySums &sums) {
