@@ -418,7 +418,7 @@ AnyPlan plan_tile(const AnyArgs &base, int batch, int mb, int nb, int wk) {
   auto bytes = [&](int groups) {
     return 16 * static_cast<size_t>(groups) * plane * X3_PARTS + 8 * static_cast<size_t>(groups) * most_taps;
   };
-  const size_t sums = static_cast<size_t>(wk) * 16 * mb * pix * sizeof(float);
+  const size_t sums = std::max<size_t>(static_cast<size_t>(wk) * 16 * mb * pix, REDUCE_GROUPS * ANY_SUMS) * sizeof(float);   // (and any_sums_block's)
   if (plane <= 0 || bytes(1) > ANY_LDS_MAX || sums > ANY_LDS_MAX) return p;
   // two workgroups a compute unit where there are that many
   const size_t room = blocks > 256 ? 78 * 1024 : ANY_LDS_MAX;
