@@ -1696,7 +1696,7 @@ static int run_any_both(const tdh_conv_desc *d, const ConvGeom &g, int batch, co
   // compute unit, each of which would hold a place of dX's: forward, dX and dW of 51x50, 128 -> 150, 3x3, stride 2, 20 images (1351
   // workgroups) 304 us along, 298 apart; 33x29, 40 -> 41, 7x7, 11 images (628) 99 / 107.
   sums.blocks      = ceil_div(sums.M * sums.N, ANY_SUMS);
-  const bool along = slices < 64 * REDUCE_GROUPS && sums.blocks <= 768;
+  const bool along = slices < 64 * REDUCE_GROUPS && sums.blocks <= 768 && conv_any_dx_has_room(shape, sums.blocks);
   if (!along) sums.blocks = 0;
   TDH_TRY(conv_any_dx_run(shape, dy, w, dx, dx_act, &pack, &sums));
   if (!along) TDH_TRY(launch_splitk_reduce(partial, slices, sums.M, sums.N, sums.epi, "conv_dw_splitk_reduce"));

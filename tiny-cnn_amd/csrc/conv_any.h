@@ -26,6 +26,8 @@ struct AnySums {
   EpiDwDb epi;
 };
 int conv_any_dx_pack(const ConvShape &c, const float *w, AnyPack *pack);
+// whether dX's launch can be that many workgroups larger
+bool conv_any_dx_has_room(const ConvShape &c, int blocks);
 // packed: the filters are (or will be, by a launch in front) packed; with: sums to take along
 int conv_any_dx_run(const ConvShape &c, const float *dy, const float *w, float *dx, ActGrad ag, const AnyPack *packed,
                     const AnySums *with);

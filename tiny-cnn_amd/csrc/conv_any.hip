@@ -679,6 +679,10 @@ int conv_any_dx_pack(const ConvShape &c, const float *w, AnyPack *pack) {
   if (!p.ok) return set_error(TDH_ERR_INVALID, "conv_any_dx_pack: no plan for this shape");
   return any_pack_of(p, w, pack);
 }
+bool conv_any_dx_has_room(const ConvShape &c, int blocks) {
+  const AnyPlan &p = backward_plan(c);
+  return p.ok && static_cast<long>(p.grid.x) + blocks <= GRID_X_MAX;
+}
 int conv_any_dx_run(const ConvShape &c, const float *dy, const float *w, float *dx, ActGrad ag, const AnyPack *packed,
                     const AnySums *with) {
   AnyPlan p = backward_plan(c);
