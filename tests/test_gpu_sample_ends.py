@@ -62,6 +62,11 @@ PARAM_NETS = {
     "any_window": ([("conv", 14, 13, 2, 4, 5, False), ("act", "tanh"), ("avepool", 11, 10, 5, 1), ("conv", 11, 10, 5, 2, 6, False),
                     ("act", "sigmoid"), ("fc", 6 * 90, 7)], "mse", "adam"),
     "fc": ([("fc", 37, 24), ("act", "tanh"), ("fc", 24, 36), ("act", "sigmoid"), ("fc", 36, 5)], "mse", "adam"),
+    # many channel pairs of small planes, a wave a pair: blocks of input channels that overlap, a table, one block of two channels
+    "many_pairs": ([("conv", 9, 8, 3, 3, 11, True), ("act", "tanh"), ("conv", 9, 8, 11, 3, 40, True,
+                    [[(ci + 2 * co) % 3 != 0 for co in range(40)] for ci in range(11)]), ("act", "sigmoid"),
+                    ("fc", 40 * 72, 4)], "mse", "adam"),
+    "many_pairs_5x5": ([("conv", 9, 8, 2, 5, 120, False), ("act", "tanh"), ("fc", 120 * 20, 3)], "mse", "adam"),
     "matvec": ([("conv", 5, 5, 3, 5, 8, False, [[(ci + co) % 2 == 0 for co in range(8)] for ci in range(3)]), ("act", "tanh"),
                 ("fc", 8, 3)], "mse", "adam"),
 }
@@ -69,9 +74,9 @@ PARAM_NETS = {
 
 @pytest.mark.parametrize("kind", ["sgd", "momentum", "adam", "adagrad", "rmsprop", "adamax", "nesterov"])
 @pytest.mark.parametrize("name,batch", [("wide", 16), ("deep_front", 32), ("deep_front", 33), ("two", 1), ("any_window", 31),
-                                        ("any_window", 50), ("fc", 32), ("fc", 70), ("matvec", 17), ("matvec", 100)])
+                                        ("any_window", 50), ("fc", 32), ("fc", 64), ("fc", 70), ("matvec", 17), ("matvec", 100)])
 def test_gradients_and_updates_of_one_group_and_of_several(T, O, W, name, batch, kind):
-    """Up to 32 samples the launch that adds up the gradients updates; larger batches leave slices. Gradients against the
+    """Small batches are updated by the launch that adds up the gradients; larger ones leave slices. Gradients against the
     oracle; updates, of a step that adds to the gradients of a pass without one, against the layer-by-layer step."""
     spec, params, x, t, batch, loss, _, _, net, ref = build(T, O, W, name, batch, SAMPLE | FUSE, nets=PARAM_NETS)
     *_, replay, _ = build(T, O, W, name, batch, SAMPLE | FUSE | 2, nets=PARAM_NETS)
@@ -104,6 +109,97 @@ def test_gradients_and_updates_of_one_group_and_of_several(T, O, W, name, batch,
     assert opts[0].b1_t == opts[1].b1_t == opts[2].b1_t and opts[0].b2_t == opts[1].b2_t == opts[2].b2_t
     for m in (net, replay, layered):
         m.close()
+
+
+def roads_of(T, step):
+    T.profile_begin()
+    step()
+    return {e["tag"].split()[0] for e in T.profile_end()}
+
+
+@pytest.mark.parametrize("name,batch,road", [("many_pairs", 65, "waves"), ("many_pairs", 200, "waves"), ("many_pairs", 12, None),
+                                             ("many_pairs_5x5", 100, "waves"), ("any_window", 9, "any")])
+def test_gradients_of_many_pairs_and_of_any_window(T, O, W, name, batch, road):
+    spec, params, x, t, batch, loss, kind, _, net, ref = build(T, O, W, name, batch, SAMPLE | FUSE, nets=PARAM_NETS)
+    xd, td = T.to_device(x), T.to_device(t)
+    tags = roads_of(T, lambda: net.train_step(None, loss, batch, xd, td, do_update=False))
+    assert "tiny_net_param_grads" + ("_" + road if road else "") in tags, tags
+    ref.train_step(O.opt_desc(kind), loss, x, t, do_update=False)
+    for i, w, _ in params:
+        assert_close(net.layer_grad(i, w), ref.layer_dw(i) if w == 0 else ref.layer_db(i), what=f"gradient {i}.{w}")
+    opt = T.opt_desc(kind, alpha=1e-3)
+    tags = roads_of(T, lambda: net.train_step(opt, loss, batch, xd, td))
+    assert any(tag.startswith("opt_") for tag in tags) == (batch > 12 or road == "any"), tags
+    net.close()
+
+
+@pytest.mark.parametrize("batch", [1, 6, 40])
+def test_strided_convolutions_match_oracle(T, O, batch):
+    """Windows and strides that no fast form takes, one of them behind a 3x3 window of stride 1 (the first layer's dX and a
+    channel pair's gradients beside them)."""
+    def layers(L):
+        return [L.L_conv(13, 12, 2, 3, 5, pad_same=True), L.L_act("tanh"), L.L_conv(13, 12, 5, 4, 6, stride=2), L.L_act("sigmoid"),
+                L.L_conv(5, 5, 6, 3, 7, pad_same=True, stride=3, has_bias=False), L.L_act("tanh"), L.L_fc(7 * 4, 3)]
+
+    rng = np.random.default_rng(5)
+    net, ref = T.Net(layers(T), batch, SAMPLE | FUSE), O.OracleNet(layers(O), batch)
+    for i, which, n in net.params():
+        a = rng.uniform(-0.4, 0.4, n).astype(np.float32)
+        net.set_param(i, which, a)
+        (ref.weight(i) if which == 0 else ref.bias(i))[:] = a
+    x = rng.standard_normal((batch, net.in_size())).astype(np.float32)
+    t = rng.uniform(-0.8, 0.8, (batch, net.out_size())).astype(np.float32)
+    tags = roads_of(T, lambda: net.train_step(None, "mse", batch, T.to_device(x), T.to_device(t), do_update=False))
+    assert "tiny_net_param_grads_any" in tags, tags
+    ref.train_step(O.opt_desc("sgd"), "mse", x, t, do_update=False)
+    for i in range(net.n):
+        assert_close(net.layer_out(i, batch), ref.layer_out(i, batch), what=f"layer {i} output")
+        assert_close(net.layer_dx(i, batch), ref.layer_dx(i, batch), what=f"layer {i} dX")
+    for i, w, _ in net.params():
+        assert_close(net.layer_grad(i, w), ref.layer_dw(i) if w == 0 else ref.layer_db(i), what=f"gradient {i}.{w}")
+    net.close()
+
+
+@pytest.mark.parametrize("k,same,in_c,out_c", [(3, False, 2, 4), (3, True, 2, 4), (5, True, 1, 3), (5, False, 2, 3), (3, True, 9, 40)])
+@pytest.mark.parametrize("batch", [3, 90])
+def test_infinities_stay_out_of_sums_that_they_are_no_part_of(T, O, k, same, in_c, out_c, batch):
+    """Minus infinity at corners of the input: relu makes a zero of what they reach, so that the first layer's weight gradient has a NaN
+    (infinity times zero) exactly where one of them meets an output pixel, in the oracle's sums as well."""
+    w, h = 10, 9
+    ow, oh = (w, h) if same else (w - k + 1, h - k + 1)
+
+    def layers(L):
+        return [L.L_conv(w, h, in_c, k, out_c, pad_same=same), L.L_act("relu"), L.L_conv(ow, oh, out_c, 3, 5, pad_same=True),
+                L.L_act("tanh"), L.L_fc(5 * ow * oh, 2)]
+
+    rng = np.random.default_rng(8)
+    net, ref = T.Net(layers(T), batch, SAMPLE | FUSE), O.OracleNet(layers(O), batch)
+    for i, which, n in net.params():
+        a = rng.uniform(0.05, 0.4, n).astype(np.float32) if i == 0 else rng.uniform(-0.3, 0.3, n).astype(np.float32)
+        net.set_param(i, which, a)
+        (ref.weight(i) if which == 0 else ref.bias(i))[:] = a
+    x = rng.standard_normal((batch, in_c, h, w)).astype(np.float32)
+    x[0, 0, 0, 0] = x[1, in_c - 1, h - 1, w - 1] = x[2, 0, 0, w - 1] = -np.inf
+    x = x.reshape(batch, -1)
+    t = rng.uniform(-0.8, 0.8, (batch, 2)).astype(np.float32)
+    tags = roads_of(T, lambda: net.train_step(None, "mse", batch, T.to_device(x), T.to_device(t), do_update=False))
+    assert {"tiny_net_step"} <= tags and any(tag.startswith("tiny_net_param_grads") for tag in tags), tags
+    ref.train_step(O.opt_desc("sgd"), "mse", x, t, do_update=False)
+
+    def same_values(got, want, what):
+        got, want = np.asarray(got).ravel(), np.asarray(want).ravel()
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want)), what
+        on = np.isfinite(want)
+        assert_close(got[on], want[on], what=what)
+
+    for i in range(net.n):
+        same_values(net.layer_out(i, batch), ref.layer_out(i, batch), f"layer {i} output")
+        same_values(net.layer_dx(i, batch), ref.layer_dx(i, batch), f"layer {i} dX")
+    for i, which, _ in net.params():
+        same_values(net.layer_grad(i, which), ref.layer_dw(i) if which == 0 else ref.layer_db(i), f"gradient {i}.{which}")
+    dw = ref.layer_dw(0)
+    assert np.isnan(dw).any() and np.isfinite(dw).any()   # (the test's point)
+    net.close()
 
 
 HELD_NETS = {

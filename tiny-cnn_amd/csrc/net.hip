@@ -343,9 +343,12 @@ int build_tiny_plan(tdh_net *net) {
   if (std::max(P.lds_floats, P.lds_job_floats) * sizeof(float) > TINY_LDS_MAX_BYTES) return TDH_OK;
   const int split_batch = std::min(tiny_most_split(P), net->max_batch);   // (whose back kernel leaves slices per sample)
   int groups[TINY_MAX_LAYERS];
+  std::fill(groups, groups + n, 1);
+  for (int b = 1; b <= net->max_batch; ++b) {
+    const TinyGroups g = tiny_groups(P, b);
+    for (int i = 0; i < n; ++i) groups[i] = std::max(groups[i], g.count(i, b));
+  }
   for (int i = 0; i < n; ++i) {
-    groups[i] = 1;
-    for (int b = 1; b <= net->max_batch; ++b) groups[i] = std::max(groups[i], tiny_groups(P, i, b));
     const int parts = groups[i] + (i < P.split ? split_batch : 0);
     slice_floats += slices_of(net->layers[i].w_size, parts) + slices_of(net->layers[i].b_size, parts) + 8;
   }
@@ -390,7 +393,7 @@ int build_tiny_plan(tdh_net *net) {
   for (int i = 0; i < n; ++i) {
     TinyLayer &T = P.l[i];
     const auto fd = [](int v) { return FastDiv(static_cast<uint32_t>(v > 0 ? v : 1)); };
-    T.d_oplane = fd(T.OH * T.OW); T.d_ow = fd(T.OW); T.d_oh = fd(T.OH); T.d_quads = fd((T.OW + 3) / 4);
+    T.d_oplane = fd(T.OH * T.OW); T.d_ow = fd(T.OW); T.d_quads = fd((T.OW + 3) / 4);
     T.d_vquads = fd((T.OH + 3) / 4); T.d_iplane = fd(T.H * T.W); T.d_w = fd(T.W);
     T.d_taps = fd(T.R * T.S); T.d_s = fd(T.S); T.d_c = fd(T.C); T.d_out = fd(T.out_size);
     T.d_nk = fd(T.C * T.R * T.S);
@@ -1113,17 +1116,18 @@ static int enqueue_step(tdh_net *net, tdh_opt *opt, int loss_kind, int batch, co
     TDH_TRY(launch_tiny_step(net->tiny, net->tiny_dev, loss_kind, softmax_xent, batch, x, t));
     // One group of samples: the same launch is the update, unless copies of filters hang on it that only the optimizer's
     // kernel writes.
-    bool may_update = do_update, updated = false;
+    const TinyGroups groups = tiny_groups(net->tiny, batch);
+    bool updates = do_update && groups.one;
     for (const OptTensor &o : net->opt_table_host)
-      for (const void *copy : o.packed) may_update = may_update && !(keep_packs && copy);
-    TDH_TRY(launch_tiny_params(net->tiny, net->tiny_dev, batch, x, may_update ? opt : nullptr, net->opt_tensors, powers_in,
-                               powers_out, &updated));
-    if (updated) {
+      for (const void *copy : o.packed) updates = updates && !(keep_packs && copy);
+    TDH_TRY(launch_tiny_params(net->tiny, net->tiny_dev, groups, batch, x, updates ? opt : nullptr, net->opt_tensors, powers_in,
+                               powers_out));
+    if (updates) {
       after_update(net, keep_packs);
       return post_update(net);
     }
     for (int j = 0; j < net->tiny_merge.n; ++j)
-      net->tiny_merge.count[j] = tiny_groups(net->tiny, net->tiny_merge.layer[j], batch);
+      net->tiny_merge.count[j] = groups.count(net->tiny_merge.layer[j], batch);
     // the groups' slices: added to the gradient tensors in order by a launch of their
     // own when the step stops there; otherwise the optimizer adds them up as it does the split
     // sums of the layer-by-layer step (it clears the gradient tensors afterwards either way)

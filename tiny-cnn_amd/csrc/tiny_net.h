@@ -30,11 +30,11 @@ struct TinyLayer {
   float *gw, *gb;              // memory: a gradient slice per group of samples, [group][nw], [group][nb]
   float *pw_part, *pb_part;    // memory, layers in front of TinyPlan::split: what the back kernel leaves per sample
   TinyTensor tw, tb;           // weights and bias, as the optimizer has them
-  int dw_chunk, dw_quads;      // parameter gradients: samples in LDS at a time; whether four pixels go together
+  int dw_chunk, dw_chunk_waves;   // parameter gradients: samples in LDS at a time, with a workgroup or a wave a channel pair (0: not so)
   int nw, nb;
   int lds_in, lds_out;         // where the layer's input and output live in LDS (floats)
   // divisions by the layer's sizes as multiply-high + shift
-  FastDiv d_oplane, d_ow, d_oh, d_quads, d_vquads, d_iplane, d_w, d_taps, d_s, d_c, d_out, d_nk;
+  FastDiv d_oplane, d_ow, d_quads, d_vquads, d_iplane, d_iplanes, d_cblocks, d_w, d_taps, d_s, d_c, d_out, d_nk;
   // the unrolled input gradient of a stride-1 3x3 / 5x5 convolution reads dY from a zero-framed copy,
   // [K][H + R - 1][W + S - 1] floats in LDS; 0 when the layer takes the general loops
   int dx_framed;
@@ -97,13 +97,20 @@ int launch_tiny_step(const TinyPlan &plan, const TinyPlan *dev_plan, int loss, i
 int tiny_layout(TinyPlan &plan);
 // the largest batch that runs the front and back kernels (0: none)
 int tiny_most_split(const TinyPlan &plan);
-// groups of samples whose gradients of a layer leave a slice each
-int tiny_groups(const TinyPlan &plan, int layer, int batch);
+// How a batch's parameter gradients are split: samples of a layer's group, each of which leaves a slice; whether there is one group
+// everywhere (which may be updated at once)
+struct TinyGroups {
+  int size[TINY_MAX_LAYERS];
+  bool waves[TINY_MAX_LAYERS];   // a wave a channel pair
+  bool one;
+  int count(int layer, int batch) const { return ceil_div(batch, size[layer]); }
+};
+TinyGroups tiny_groups(const TinyPlan &plan, int batch);
 // Every layer's weight and bias gradients (and the first layer's input gradient) from the outputs and
-// gradients that launch_tiny_step left in memory. With `update` and one group of samples everywhere, the optimizer's step
-// on all tensors as well (powers_in, powers_out: as in launch_opt_update_multi; *updated), else the slices.
-int launch_tiny_params(const TinyPlan &plan, const TinyPlan *dev_plan, int batch, const float *x, tdh_opt *update,
-                       int n_tensors, const float *powers_in, float *powers_out, bool *updated);
+// gradients that launch_tiny_step left in memory. With `update` (one group everywhere) the optimizer's step
+// on all tensors as well (powers_in, powers_out: as in launch_opt_update_multi), else the slices.
+int launch_tiny_params(const TinyPlan &plan, const TinyPlan *dev_plan, const TinyGroups &groups, int batch, const float *x,
+                       tdh_opt *update, int n_tensors, const float *powers_in, float *powers_out);
 int launch_tiny_merge(const TinyMerge &m);
 
 }  // namespace tdh

@@ -26,6 +26,7 @@
 #include <algorithm>
 #include <cfloat>
 #include <type_traits>
+#include <vector>
 
 #include "opt_update.h"
 #include "tiny_net.h"
@@ -1932,11 +1933,11 @@ tiny_net_back_kernel(const TinyPlan *__restrict__ plan, const int m, const float
 // us, a slice per sample and the optimizer's launch / here: LeNet-5, batch 16 9.2 + 5.0 / 7.8 (and 2 in the back kernel), 32
 // 14.6 + 7.3 / 11.1, 64 24.4 + 7.4 / 15.3 + 5.6, 120 40.0 + 12.9 / 25.9 + 6.8, 300 86.4 + 20.6 / 55.9 + 9.3.
 constexpr int TP_THREADS = 512, TP_WAVES = TP_THREADS / 64;
-enum { TP_CONV, TP_OUTER, TP_OUTER4, TP_COLUMNS, TP_POOL, TP_SLICES_W, TP_SLICES_B };   // what a range of workgroups does
+enum { TP_CONV, TP_CONV_WAVES, TP_ROWS, TP_BIAS, TP_OUTER, TP_OUTER4, TP_COLUMNS, TP_POOL, TP_SLICES_W, TP_SLICES_B };   // what a range of workgroups does
 constexpr int TP_RANGES = 2 * TINY_MAX_LAYERS;
 struct TinyRanges {
   int first[TP_RANGES];     // first workgroup; past the last range larger than any
-  int job[TP_RANGES];       // layer * 8 + TP_*
+  int job[TP_RANGES];       // layer * 16 + TP_*
   int per_group[TP_RANGES]; // workgroups per group of samples
   int size[TP_RANGES];      // samples of a group
 };
@@ -2003,12 +2004,13 @@ TN_INLINE void tn_finish(const TinyTarget &t, TinyOld o, const int e, const floa
   }
 }
 
-// One plane of the layer's input and one of its output gradient, of ns samples, into LDS, all of a trip's
-// reads before its first store
-TN_INLINE void stage_planes(const TinyLayer *__restrict__ L, float *xl, const float *__restrict__ x, const int x_stride, float *dl,
-                            const float *__restrict__ d, const int d_stride, const int ns) {
-  const int x_plane = L->H * L->W, d_plane = L->OH * L->OW, nx = ns * x_plane, total = nx + ns * d_plane;
-  const FastDiv d_x = L->d_iplane, d_d = L->d_oplane;
+// x_plane values of the layer's input (one of its planes, or some that follow each other) and one plane of its output
+// gradient, of ns samples, into LDS, all of a trip's reads before its first store
+TN_INLINE void stage_planes(const TinyLayer *__restrict__ L, float *xl, const float *__restrict__ x, const int x_stride,
+                            const int x_plane, const FastDiv d_x, float *dl, const float *__restrict__ d, const int d_stride,
+                            const int ns) {
+  const int d_plane = L->OH * L->OW, nx = ns * x_plane, total = nx + ns * d_plane;
+  const FastDiv d_d = L->d_oplane;
   const bool vec = ((x_plane | x_stride | d_plane | d_stride) & 3) == 0 &&
                    ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(d)) & 15u) == 0;
   auto from = [&](int e) {
@@ -2065,41 +2067,51 @@ TN_INLINE void at_hand(const TinyLayer *__restrict__ L) {
                "s"(b.shift), "s"(d.mul), "s"(d.shift), "s"(d.d), "s"(e.mul), "s"(e.shift), "s"(e.d));
 }
 // dW of a channel pair (and, with the first input channel, the output channel's bias gradient), over the samples
-// [s_beg, s_end), `chunk` of them in LDS at a time. A thread adds up the taps of four output pixels below each other at
+// [s_beg, s_end), some of them in LDS at a time. A thread adds up the taps of four output pixels below each other at
 // a time (neighbouring lanes read neighbouring columns, whatever the row's length); the waves' sums meet in LDS.
-template <int KIND, int R, int S, bool PAD>
+// WAVES: a wave a pair, up to TP_WAVES input channels of one output channel side by side (`ci` is their block). A
+// workgroup's time is mostly its latency, so that many pairs of small planes are many rounds of the chip. 12x12, 3 -> 16 -> 32
+// channels, 3x3 (512 pairs of 6x6 planes behind a pool), the launch, us, a workgroup a pair / a wave: 64 samples 25.6 / 11.3, 256 88 / 29; LeNet-5's
+// 96 pairs of 14x14, 5x5, 33 samples 11 / 16, 256 47 / 37 (pair_split chooses).
+template <int KIND, int R, int S, bool PAD, bool WAVES>
 TN_INLINE void conv_param_pair(const TinyLayer *__restrict__ L, const float *__restrict__ gin, const int in_sz,
                                const float *__restrict__ gdy, const int out_sz, const int s_beg, const int s_end,
-                               const int co, const int ci, const int group, const TinyUpdate &u, float *lds) {
-  constexpr int taps = R * S;
+                               const int co, const int ci_or_block, const int group, const TinyUpdate &u, float *lds) {
+  constexpr int taps = R * S, TEAM = WAVES ? 64 : TP_THREADS;
   at_hand(L);
+  const int channels = WAVES ? min(L->C, TP_WAVES) : 1, tid = threadIdx.x & (TEAM - 1);
+  // (the last block of channels begins early enough to be whole, and leaves what the one in front of it has)
+  const int ci_first = WAVES ? min(ci_or_block * TP_WAVES, L->C - channels) : ci_or_block;
+  const int place = WAVES ? min(wave_index(), channels - 1) : 0, ci = ci_first + place;
+  const bool here = !WAVES || (wave_index() < channels && ci >= ci_or_block * TP_WAVES);
   const bool connected = !L->tbl || L->tbl[ci * L->K + co];
-  const int tap = threadIdx.x, e = (co * L->C + ci) * taps + tap;
-  const bool mine = tap < taps, mine_b = tap == taps && ci == 0 && L->nb;
+  const int tap = tid, e = (co * L->C + ci) * taps + tap;
+  const bool mine = here && tap < taps, mine_b = here && tap == taps && ci == 0 && L->nb;
   const TinyTarget tw = tn_target<KIND>(u, L, false, group), tb = tn_target<KIND>(u, L, true, group);
   const TinyOld old_w = tn_old<KIND>(tw, e, mine), old_b = tn_old<KIND>(tb, co, mine_b);
-  const int H = L->H, W = L->W, OH = L->OH, OW = L->OW, plane = OH * OW, iplane = H * W, chunk = L->dw_chunk;
+  const int H = L->H, W = L->W, OH = L->OH, OW = L->OW, plane = OH * OW, iplane = H * W;
+  const int chunk = WAVES ? L->dw_chunk_waves : L->dw_chunk, x_plane = channels * iplane;
   const int ph = L->ph, pw = L->pw, quads = (OH + 3) >> 2;
-  const FastDiv d_ow = L->d_ow, d_quads = L->d_vquads;
+  const FastDiv d_ow = L->d_ow, d_quads = L->d_vquads, d_x = WAVES ? L->d_iplanes : L->d_iplane;
   float acc[R][S], db = 0.0f;
 #pragma unroll
   for (int wy = 0; wy < R; ++wy)
 #pragma unroll
     for (int wx = 0; wx < S; ++wx) acc[wy][wx] = 0.0f;
-  float *xl = lds, *dl = lds + quad_pitch(chunk * iplane);
+  float *xl = lds, *dl = lds + quad_pitch(chunk * x_plane);
   for (int s0 = s_beg; s0 < s_end; s0 += chunk) {
     const int ns = min(chunk, s_end - s0);
     if (s0 > s_beg) lds_barrier();
-    stage_planes(L, xl, gin + static_cast<size_t>(s0) * in_sz + ci * iplane, in_sz, dl,
+    stage_planes(L, xl, gin + static_cast<size_t>(s0) * in_sz + ci_first * iplane, in_sz, x_plane, d_x, dl,
                  gdy + static_cast<size_t>(s0) * out_sz + co * plane, out_sz, ns);
     lds_barrier();
-    const int units = ns * quads * OW;
-    for (int i = threadIdx.x; i < units; i += TP_THREADS) {
+    const int units = here ? ns * quads * OW : 0;
+    for (int i = tid; i < units; i += TEAM) {
       uint32_t line, ox, s, q;
       d_ow.divmod(i, line, ox);
       d_quads.divmod(line, s, q);
       const int oy = 4 * static_cast<int>(q), left = OH - oy, iy0 = oy - ph, ix0 = static_cast<int>(ox) - pw;
-      const float *dr = dl + s * plane + oy * OW + ox, *xr = xl + s * iplane + iy0 * W + ix0;
+      const float *dr = dl + s * plane + oy * OW + ox, *xr = xl + s * x_plane + place * iplane + iy0 * W + ix0;
       float d[4], v[R + 3][S];
 #pragma unroll
       for (int k = 0; k < 4; ++k) d[k] = dr[k < left ? k * OW : 0];
@@ -2136,6 +2148,18 @@ TN_INLINE void conv_param_pair(const TinyLayer *__restrict__ L, const float *__r
 #pragma unroll
     for (int wx = 0; wx < S; ++wx) acc[wy][wx] = wave_sum_63(acc[wy][wx]);
   db = wave_sum_63(db);
+  if constexpr (WAVES) {
+    // (lane 63 has the sums, lane t finishes tap t)
+    float sum = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(db), 63));
+#pragma unroll
+    for (int t = 0; t < taps; ++t) {
+      const float v = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(acc[t / S][t % S]), 63));
+      sum = tap == t ? v : sum;
+    }
+    if (mine) tn_finish<KIND>(tw, old_w, e, connected ? sum : 0.0f);
+    if (mine_b) tn_finish<KIND>(tb, old_b, co, sum);
+    return;
+  }
   lds_barrier();
   if ((threadIdx.x & 63) == 63) {
     float *red = lds + wave_index() * (taps + 1);
@@ -2153,62 +2177,70 @@ TN_INLINE void conv_param_pair(const TinyLayer *__restrict__ L, const float *__r
   if (mine) tn_finish<KIND>(tw, old_w, e, connected ? sum : 0.0f);
   if (mine_b) tn_finish<KIND>(tb, old_b, co, sum);
 }
-// the same for any window and stride: a group of lanes per weight, a lane takes output rows in turn and walks the
-// pixels whose window element lies inside the input
-template <int KIND>
-TN_INLINE void conv_param_pair_any(const TinyLayer *__restrict__ L, const float *__restrict__ gin, const int in_sz,
-                                   const float *__restrict__ gdy, const int out_sz, const int s_beg, const int s_end,
-                                   const int co, const int ci, const int group, const TinyUpdate &u, float *lds) {
-  const int H = L->H, W = L->W, OH = L->OH, OW = L->OW, plane = OH * OW, iplane = H * W, chunk = L->dw_chunk;
-  const int sh = L->sh, sw = L->sw, taps = L->R * L->S, C = L->C;
-  const FastDiv d_oh = L->d_oh, d_s = L->d_s;
-  const bool connected = !L->tbl || L->tbl[ci * L->K + co];
-  const TinyTarget tw = tn_target<KIND>(u, L, false, group), tb = tn_target<KIND>(u, L, true, group);
-  float *xl = lds, *dl = lds + quad_pitch(chunk * iplane);
-  int g = 64;
-  while (g > 1 && taps * g > TP_THREADS) g >>= 1;
-  const int part = threadIdx.x & (g - 1);
-  float db = 0.0f;
-  for (int t0 = 0; t0 < taps; t0 += TP_THREADS / g) {
-    const int tap = t0 + threadIdx.x / g, e = (co * C + ci) * taps + tap;
-    const bool mine = tap < taps;
-    const TinyOld old_w = tn_old<KIND>(tw, e, mine && part == 0);
-    uint32_t wy, wx;
-    d_s.divmod(mine ? tap : 0, wy, wx);
+// dW of one sample for any window and stride: a group of lanes per weight, which take output rows in turn; a lane walks the
+// pixels of its rows whose window element lies inside the input, and the group adds up with butterfly shuffles. Workgroup
+// `block` has as many (weight, lane) units as threads. (A workgroup per channel pair over several samples, as above, is few and long
+// for wide windows, and short of work for small planes. 28x28, 1 -> 8, 7x7, pool, 8 -> 16, 4x4, the launch, us, so / here: 16 samples
+// 26.9 / 7.7, 64 28.5 / 15.7, 256 57 / 43; 28x28, 1 -> 8 -> 16 channels, stride 2, 16 samples 10.6 / 7.1, 256 38 / 22.)
+__host__ __device__ inline int conv_rows_lanes(const TinyLayer &L) {
+  int g = 32;
+  while (g > 1 && (32 * g > L.OH * L.OW || g > L.OH)) g >>= 1;   // 32 output pixels or more per lane
+  return g;
+}
+TN_INLINE void conv_param_rows(const TinyLayer *__restrict__ L, const float *__restrict__ gin, const float *__restrict__ gdy,
+                               const int block, float *__restrict__ slice, float *lds) {
+  const int H = L->H, W = L->W, K = L->K, OH = L->OH, OW = L->OW, sh = L->sh, sw = L->sw, plane = OH * OW;
+  const FastDiv d_taps = L->d_taps, d_s = L->d_s, d_c = L->d_c;
+  const uint8_t *__restrict__ tbl = L->tbl;
+  const int g = conv_rows_lanes(*L), gs = __ffs(g) - 1, end = L->nw << gs;
+  const int base = block * TP_THREADS, it = base + static_cast<int>(threadIdx.x), idx = min(it, end - 1) >> gs, part = it & (g - 1);
+  // (of dY, the planes of the output channels that these units are of)
+  const int co_lo = static_cast<int>(L->d_nk.div(base >> gs));
+  const int co_hi = static_cast<int>(L->d_nk.div((min(base + TP_THREADS, end) - 1) >> gs));
+  float *in = lds, *dy = lds + quad_pitch(L->in_size);
+  fill_lds<TP_THREADS>(in, gin, L->in_size);
+  fill_lds<TP_THREADS>(dy, gdy + co_lo * plane, (co_hi - co_lo + 1) * plane);
+  lds_barrier();
+  uint32_t pair, tap, co, ci, wy, wx;
+  d_taps.divmod(idx, pair, tap);
+  d_c.divmod(pair, co, ci);
+  d_s.divmod(tap, wy, wx);
+  float sum = 0.0f;
+  if (it < end && (!tbl || tbl[ci * K + co])) {
     // iy = oy*sh + wy - ph in [0, H), ix = ox*sw + wx - pw in [0, W)
     const int yoff = static_cast<int>(wy) - L->ph, xoff = static_cast<int>(wx) - L->pw;
+    const int oy_lo = yoff >= 0 ? 0 : (-yoff + sh - 1) / sh, oy_hi = H - 1 - yoff < 0 ? 0 : min(OH, (H - 1 - yoff) / sh + 1);
     const int ox_lo = xoff >= 0 ? 0 : (-xoff + sw - 1) / sw, ox_hi = W - 1 - xoff < 0 ? 0 : min(OW, (W - 1 - xoff) / sw + 1);
-    float sum = 0.0f;
-    for (int s0 = s_beg; s0 < s_end; s0 += chunk) {
-      const int ns = min(chunk, s_end - s0);
-      lds_barrier();
-      stage_planes(L, xl, gin + static_cast<size_t>(s0) * in_sz + ci * iplane, in_sz, dl,
-                   gdy + static_cast<size_t>(s0) * out_sz + co * plane, out_sz, ns);
-      lds_barrier();
-      if (mine && connected)
-        for (int row = part; row < ns * OH; row += g) {
-          uint32_t s, oy;
-          d_oh.divmod(row, s, oy);
-          const int iy = static_cast<int>(oy) * sh + yoff;
-          if (static_cast<unsigned>(iy) >= static_cast<unsigned>(H)) continue;
-          const float *xr = xl + s * iplane + iy * W + xoff, *dr = dl + row * OW;
-          for (int ox = ox_lo; ox < ox_hi; ++ox) sum = __builtin_fmaf(xr[ox * sw], dr[ox], sum);
-        }
-      if (t0 == 0 && ci == 0)
-        for (int i = threadIdx.x; i < ns * plane; i += TP_THREADS) db += dl[i];
+    const float *ip = in + (static_cast<int>(ci) * H + yoff) * W + xoff, *dp = dy + (static_cast<int>(co) - co_lo) * plane;
+    for (int oy = oy_lo + part; oy < oy_hi; oy += g) {
+      const float *ir = ip + oy * sh * W, *dr = dp + oy * OW;
+      int ox = ox_lo;
+      for (; ox + 4 <= ox_hi; ox += 4)
+        sum += ir[ox * sw] * dr[ox] + ir[(ox + 1) * sw] * dr[ox + 1] + ir[(ox + 2) * sw] * dr[ox + 2] + ir[(ox + 3) * sw] * dr[ox + 3];
+      for (; ox < ox_hi; ++ox) sum += ir[ox * sw] * dr[ox];
     }
-    sum = group_sum(sum, g);
-    if (mine && part == 0) tn_finish<KIND>(tw, old_w, e, sum);
   }
-  if (ci == 0 && L->nb) {
-    lds_barrier();
-    db = workgroup_sum(db, lds);
-    if (threadIdx.x == 0) tn_finish<KIND>(tb, tn_old<KIND>(tb, co, true), co, db);
+  sum = group_sum(sum, g);
+  if (it < end && part == 0) slice[idx] = sum;
+}
+// the bias gradient of such a convolution, a workgroup of its own: a group of lanes a channel
+TN_INLINE void conv_param_bias(const TinyLayer *__restrict__ L, const float *__restrict__ gdy, float *__restrict__ slice) {
+  const int nb = L->nb, plane = L->OH * L->OW;
+  int g = 64;
+  while (g > 1 && (nb * g > 2 * TP_THREADS || g > plane)) g >>= 1;
+  const int total = nb * g, gs = __ffs(g) - 1;
+  for (int base = 0; base < total; base += TP_THREADS) {
+    const int it = base + static_cast<int>(threadIdx.x), co = it >> gs, part = it & (g - 1);
+    float sum = 0.0f;
+    if (it < total)
+      for (int p = part; p < plane; p += g) sum += gdy[co * plane + p];
+    sum = group_sum(sum, g);
+    if (it < total && part == 0) slice[co] = sum;
   }
 }
 // A fully-connected layer, or a convolution that is one: a weight is the sum over the samples of one input times one
 // output gradient. V weights a thread, neighbours along the faster index (V = 4: its rows are whole, aligned words).
-template <int KIND, int V>
+template <int KIND, int V, int AHEAD>
 TN_INLINE void outer_param(const TinyLayer *__restrict__ L, const float *__restrict__ gin, const int in_sz,
                            const float *__restrict__ gdy, const int out_sz, const int s_beg, const int s_end,
                            const int block, const int group, const TinyUpdate &u) {
@@ -2227,7 +2259,6 @@ TN_INLINE void outer_param(const TinyLayer *__restrict__ L, const float *__restr
   float sum[V];
 #pragma unroll
   for (int k = 0; k < V; ++k) sum[k] = 0.0f;
-  constexpr int AHEAD = 16;
   for (int s0 = s_beg; s0 < s_end; s0 += AHEAD) {
     float f[AHEAD][V], d[AHEAD];
 #pragma unroll
@@ -2286,7 +2317,7 @@ TN_INLINE void pool_param(const TinyLayer *__restrict__ L, const float *__restri
   for (int s0 = s_beg; s0 < s_end; s0 += chunk) {
     const int ns = min(chunk, s_end - s0);
     lds_barrier();
-    stage_planes(L, xl, gin + static_cast<size_t>(s0) * in_sz + c * iplane, in_sz, dl,
+    stage_planes(L, xl, gin + static_cast<size_t>(s0) * in_sz + c * iplane, in_sz, iplane, L->d_iplane, dl,
                  gdy + static_cast<size_t>(s0) * out_sz + c * plane, out_sz, ns);
     lds_barrier();
     for (int i = threadIdx.x; i < ns * plane; i += TP_THREADS) {
@@ -2387,11 +2418,16 @@ TN_INLINE void conv_dx_band(const TinyLayer *__restrict__ L, const float *__rest
   }
 }
 
-template <int KIND>
-__global__ void __launch_bounds__(TP_THREADS, 4)
+// ROADS: what there is code for. TP_HAS_PAIRS: 3x3 or 5x5 windows of stride 1, and the first layer's dX; TP_HAS_WAVES: a wave a pair;
+// TP_HAS_ROWS: other windows. (All of it in one kernel, LeNet-5's step at 16 samples takes 41.1 us instead of 40.7: more scalars than
+// there are registers for.)
+constexpr int TP_HAS_PAIRS = 1, TP_HAS_WAVES = 2, TP_HAS_ROWS = 4;
+template <int KIND, int ROADS>
+__global__ void __launch_bounds__(TP_THREADS, ROADS & TP_HAS_PAIRS ? 4 : 6)
 tiny_net_param_kernel(const TinyPlan *__restrict__ plan, const float *__restrict__ x, const TinyRanges ranges,
                       const TinyUpdate u, const int batch, const int param_blocks) {
   extern __shared__ float lds[];
+  constexpr int AHEAD = ROADS & TP_HAS_PAIRS ? 16 : 4;   // samples that an outer product has in flight
   if (KIND >= 0 && opt_powers(KIND) > 0 && u.powers_in && blockIdx.x == 0 && threadIdx.x == 0) {   // (as opt_multi_kernel)
     float q1 = u.powers_in[0], q2 = u.powers_in[1];
     for (int i = 0; i < u.n_tensors; ++i) {
@@ -2403,7 +2439,7 @@ tiny_net_param_kernel(const TinyPlan *__restrict__ plan, const float *__restrict
   }
   const int n = plan->n;
   int id = blockIdx.x;
-  if (id >= param_blocks) {   // workgroups (band, input channel, sample), samples fastest
+  if ((ROADS & TP_HAS_PAIRS) && id >= param_blocks) {   // workgroups (band, input channel, sample), samples fastest
     id -= param_blocks;
     const TinyLayer *__restrict__ L = &plan->l[0];
     const int rest = id / batch, s = id - rest * batch, ci = rest % L->C, band = rest / L->C;
@@ -2422,27 +2458,43 @@ tiny_net_param_kernel(const TinyPlan *__restrict__ plan, const float *__restrict
     per_group = on ? ranges.per_group[k] : per_group;
     size      = on ? ranges.size[k] : size;
   }
-  const int li = job >> 3, what = job & 7, group = (id - first) / per_group, block = id - first - group * per_group;
+  const int li = job >> 4, what = job & 15, group = (id - first) / per_group, block = id - first - group * per_group;
   const TinyLayer *__restrict__ L = &plan->l[li];
   const int in_sz = L->in_size, out_sz = L->out_size;
   const float *gin = li == 0 ? x : plan->l[li - 1].out;
   const float *gdy = li == n - 1 ? plan->dloss : plan->l[li + 1].dx;
   const int s_beg = group * size, s_end = min(batch, s_beg + size);
   switch (what) {
-    case TP_CONV: {
-      const int co = L->d_c.div(block), ci = block - co * L->C;
-      const bool pad = L->ph != 0 || L->pw != 0;
-      if (!L->dw_quads) conv_param_pair_any<KIND>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, co, ci, group, u, lds);
-      else if (L->R == 5) {
-        if (pad) conv_param_pair<KIND, 5, 5, true>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, co, ci, group, u, lds);
-        else conv_param_pair<KIND, 5, 5, false>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, co, ci, group, u, lds);
-      } else {
-        if (pad) conv_param_pair<KIND, 3, 3, true>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, co, ci, group, u, lds);
-        else conv_param_pair<KIND, 3, 3, false>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, co, ci, group, u, lds);
+    case TP_CONV:
+    case TP_CONV_WAVES:
+      if constexpr (ROADS & TP_HAS_PAIRS) {
+        const bool waves = (ROADS & TP_HAS_WAVES) && what == TP_CONV_WAVES, pad = L->ph != 0 || L->pw != 0;
+        uint32_t co, ci;
+        (waves ? L->d_cblocks : L->d_c).divmod(block, co, ci);
+        const auto run = [&](auto window, auto padded) {
+          constexpr int R = decltype(window)::value;
+          constexpr bool PAD = decltype(padded)::value, MAY_WAVES = (ROADS & TP_HAS_WAVES) != 0;
+          if (waves) conv_param_pair<KIND, R, R, PAD, MAY_WAVES>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, co, ci, group, u, lds);
+          else conv_param_pair<KIND, R, R, PAD, false>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, co, ci, group, u, lds);
+        };
+        const std::integral_constant<int, 5> five;
+        const std::integral_constant<int, 3> three;
+        if (L->R == 5) pad ? run(five, std::true_type()) : run(five, std::false_type());
+        else pad ? run(three, std::true_type()) : run(three, std::false_type());
       }
-    } break;
-    case TP_OUTER: outer_param<KIND, 1>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, block, group, u); break;
-    case TP_OUTER4: outer_param<KIND, 4>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, block, group, u); break;
+      break;
+    // (groups of one sample, slices only)
+    case TP_ROWS:
+      if constexpr (ROADS & TP_HAS_ROWS)
+        conv_param_rows(L, gin + static_cast<size_t>(s_beg) * in_sz, gdy + static_cast<size_t>(s_beg) * out_sz, block,
+                        L->gw + static_cast<size_t>(group) * L->nw, lds);
+      break;
+    case TP_BIAS:
+      if constexpr (ROADS & TP_HAS_ROWS)
+        conv_param_bias(L, gdy + static_cast<size_t>(s_beg) * out_sz, L->gb + static_cast<size_t>(group) * L->nb);
+      break;
+    case TP_OUTER: outer_param<KIND, 1, AHEAD>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, block, group, u); break;
+    case TP_OUTER4: outer_param<KIND, 4, AHEAD>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, block, group, u); break;
     case TP_COLUMNS: column_param<KIND>(gdy, out_sz, L->nb, s_beg, s_end, block, tn_target<KIND>(u, L, true, group)); break;
     case TP_POOL: pool_param<KIND>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, block, group, u, lds); break;
     case TP_SLICES_W: column_param<KIND>(L->pw_part, L->nw, L->nw, s_beg, s_end, block, tn_target<KIND>(u, L, false, group)); break;
@@ -2465,15 +2517,33 @@ tiny_net_merge_kernel(const TinyMerge m) {
 
 }  // namespace
 
+// of an optimizer kind, or -1 for slices, which may be of every road
+static decltype(&tiny_net_param_kernel<-1, 0>) param_kernel(const int kind, const int roads) {
+  switch (kind) {
+    case -1:
+      return roads == TP_HAS_ROWS                     ? tiny_net_param_kernel<-1, TP_HAS_ROWS>
+             : roads & (TP_HAS_WAVES | TP_HAS_ROWS) ? tiny_net_param_kernel<-1, TP_HAS_PAIRS | TP_HAS_WAVES | TP_HAS_ROWS>
+                                                    : tiny_net_param_kernel<-1, TP_HAS_PAIRS>;
+    case TDH_OPT_SGD: return tiny_net_param_kernel<TDH_OPT_SGD, TP_HAS_PAIRS>;
+    case TDH_OPT_MOMENTUM: return tiny_net_param_kernel<TDH_OPT_MOMENTUM, TP_HAS_PAIRS>;
+    case TDH_OPT_NESTEROV: return tiny_net_param_kernel<TDH_OPT_NESTEROV, TP_HAS_PAIRS>;
+    case TDH_OPT_ADAM: return tiny_net_param_kernel<TDH_OPT_ADAM, TP_HAS_PAIRS>;
+    case TDH_OPT_ADAGRAD: return tiny_net_param_kernel<TDH_OPT_ADAGRAD, TP_HAS_PAIRS>;
+    case TDH_OPT_RMSPROP: return tiny_net_param_kernel<TDH_OPT_RMSPROP, TP_HAS_PAIRS>;
+    case TDH_OPT_ADAMAX: return tiny_net_param_kernel<TDH_OPT_ADAMAX, TP_HAS_PAIRS>;
+    default: return nullptr;
+  }
+}
+
 int tiny_prepare() {
   static bool attr_set = false;
   if (!attr_set) {
     const auto of = [](auto k) { return reinterpret_cast<const void *>(k); };
-    for (const void *k : {of(&tiny_net_step_kernel<false>), of(&tiny_net_step_kernel<true>), of(&tiny_net_front_kernel), of(&tiny_net_back_kernel), of(&tiny_net_param_kernel<-1>),
-                          of(&tiny_net_param_kernel<TDH_OPT_SGD>), of(&tiny_net_param_kernel<TDH_OPT_MOMENTUM>),
-                          of(&tiny_net_param_kernel<TDH_OPT_NESTEROV>), of(&tiny_net_param_kernel<TDH_OPT_ADAM>),
-                          of(&tiny_net_param_kernel<TDH_OPT_ADAGRAD>), of(&tiny_net_param_kernel<TDH_OPT_RMSPROP>),
-                          of(&tiny_net_param_kernel<TDH_OPT_ADAMAX>)})
+    std::vector<const void *> kernels = {of(&tiny_net_step_kernel<false>), of(&tiny_net_step_kernel<true>), of(&tiny_net_front_kernel),
+                                         of(&tiny_net_back_kernel)};
+    for (int kind = -1; kind <= TDH_OPT_NESTEROV; ++kind) kernels.push_back(of(param_kernel(kind, TP_HAS_PAIRS)));
+    for (int roads : {TP_HAS_ROWS, TP_HAS_PAIRS | TP_HAS_ROWS}) kernels.push_back(of(param_kernel(-1, roads)));
+    for (const void *k : kernels)
       TDH_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(TINY_LDS_MAX_BYTES)));
     attr_set = true;
   }
@@ -2509,6 +2579,11 @@ static void plan_split(TinyPlan &P) {
   P.split = m;
 }
 
+// convolutions whose weight gradients are added up sample by sample (conv_param_rows)
+static bool conv_by_rows(const TinyLayer &L) {
+  return L.kind == TDH_L_CONV && !conv_is_matvec(L) &&
+         !(L.sh == 1 && L.sw == 1 && ((L.R == 5 && L.S == 5) || (L.R == 3 && L.S == 3)));
+}
 int tiny_layout(TinyPlan &P) {
   size_t framed = 0, lds = 26 * TP_WAVES;   // (conv_param_pair's sums)
   for (int i = 0; i < P.n; ++i) {
@@ -2527,11 +2602,20 @@ int tiny_layout(TinyPlan &P) {
     if (i == 0 && P.first_dx_as_job) lds = std::max(lds, static_cast<size_t>(dx_band(L).floats));
     else if (L.dx_framed) framed = std::max(framed, static_cast<size_t>(conv_framed_floats(L)));
     if (!L.nw || L.kind == TDH_L_FC || conv_is_matvec(L)) continue;
+    if (conv_by_rows(L)) {
+      lds = std::max(lds, static_cast<size_t>(quad_pitch(L.in_size)) + L.out_size);
+      continue;
+    }
     // planes of the input and the output gradient: as many samples at a time as fit 48 KB
-    L.dw_quads = L.kind == TDH_L_CONV && L.sh == 1 && L.sw == 1 && ((L.R == 5 && L.S == 5) || (L.R == 3 && L.S == 3));
     const int planes = L.H * L.W + L.OH * L.OW;
     L.dw_chunk = std::min(std::max(12288 / planes, 1), 32);
     lds = std::max(lds, static_cast<size_t>(L.dw_chunk) * planes + 4);
+    if (L.kind != TDH_L_CONV || L.C == 1) continue;
+    const int channels = std::min(L.C, TP_WAVES), more = channels * L.H * L.W + L.OH * L.OW;
+    L.dw_chunk_waves = more > 12288 ? 0 : std::min(12288 / more, 32);
+    L.d_iplanes = FastDiv(static_cast<uint32_t>(channels * L.H * L.W));
+    L.d_cblocks = FastDiv(static_cast<uint32_t>(ceil_div(L.C, TP_WAVES)));
+    lds = std::max(lds, static_cast<size_t>(L.dw_chunk_waves) * more + 4);
   }
   plan_split(P);
   P.lds_pad = P.lds_floats;
@@ -2610,13 +2694,75 @@ int tiny_layout(TinyPlan &P) {
 // 70.7: with several workgroups a compute unit, each of which frames all of dY for its one channel, they lose.
 int tiny_most_split(const TinyPlan &plan) { return plan.split ? 256 / std::max(plan.l[0].K, plan.l[plan.split].C) : 0; }
 static bool tiny_splits(const TinyPlan &plan, int batch) { return batch <= tiny_most_split(plan); }
-// A batch of up to 32 samples is one group, whose workgroups update; the groups of a larger one are of 16, which
-// the optimizer's kernel has to add up either way (64 samples in groups of 32: 58 us instead of 16, the first layer's
-// workgroups being few and long; as many samples as fit LDS at a time is what a layer's group is limited to).
-int tiny_groups(const TinyPlan &plan, int layer, int batch) {
-  const TinyLayer &L = plan.l[layer];
-  const int most = batch <= 32 ? 32 : 16;
-  return ceil_div(batch, tiny_splits(plan, batch) && layer < plan.split ? most : std::min(L.dw_chunk, most));
+// How the parameter gradients of a batch are split. Estimated us of a layer of channel pairs, fitted to LeNet-5's and to layers of 12 to 512
+// pairs of 6x6 to 28x28 planes, 1 to 512 samples: whole rounds of 512 workgroups (two a compute unit, by their registers), each of which takes
+// its latency, another trip to memory for every further lot of samples in LDS, and its products; and a share of the time of the launch's other
+// workgroups. The step, us, with groups of 16 samples and a workgroup a pair / as chosen: LeNet-5, 33 samples 48.7 / 47.2, 256 100.9 / 91.3;
+// 28x28, 1 -> 8 -> 16 channels, 3x3, pools, 128 samples 77.6 / 71.8; 12x12, 3 -> 16 -> 32, 3x3, pools, 33 samples 70.7 / 61.1, 256 145 / 84; 28x28,
+// 1 -> 12, 5x5, pool, 64 samples 60.0 / 57.5.
+struct PairSplit {
+  int size, waves;   // samples of a group; a wave a pair instead of a workgroup
+  double us;
+};
+static PairSplit pair_split(const TinyLayer &L, const int batch, const int size, const int waves) {
+  const int chunk = waves ? L.dw_chunk_waves : L.dw_chunk, units = size * ((L.OH + 3) / 4) * L.OW;
+  const int workgroups = ceil_div(batch, size) * L.K * (waves ? ceil_div(L.C, TP_WAVES) : L.C);
+  const double each = 8.0 + 3.0 * (ceil_div(size, chunk) - 1) + 0.032 * L.R * L.S * ceil_div(units, waves ? 64 : TP_THREADS);
+  return {size, waves, ceil_div(workgroups, 512) * each + workgroups / 170.0};
+}
+// of groups of up to 32 samples, or of all of them
+static PairSplit best_pair_split(const TinyLayer &L, const int batch, const bool whole) {
+  PairSplit best = {0, 0, 0.0};
+  for (int waves = 0; waves <= (L.dw_chunk_waves > 0 && !whole); ++waves)
+    for (int size = whole ? batch : 4; size <= std::min(whole ? batch : 32, batch); size *= 2) {
+      const PairSplit p = pair_split(L, batch, size, waves);
+      if (!best.size || p.us < best.us) best = p;
+    }
+  if (!best.size) best = pair_split(L, batch, batch, 0);   // (fewer than four samples)
+  return best;
+}
+TinyGroups tiny_groups(const TinyPlan &plan, const int batch) {
+  TinyGroups g = {};
+  const int m = tiny_splits(plan, batch) ? plan.split : 0;
+  // One group is updated by the launch that adds it up, and the optimizer's launch, 5 us, left out: where no layer takes
+  // longer for it than that. (Outer products and column sums have sixteen samples at a time in flight, a trip to memory each; a step of
+  // 784-30-10 fully connected, us, in several groups / one: 33 samples 28.8 / 25.4, 64 29.1 / 26.6; of 64-64-10, 33 22.2 / 20.5, 64 22.3 / 21.7.)
+  bool pairs = false, pools = false, rows = false;
+  double one = 0.0, several = 0.0;
+  g.one = batch <= 64;
+  for (int i = 0; i < plan.n; ++i) {
+    const TinyLayer &L = plan.l[i];
+    if (!L.nw || i < m) continue;
+    if (conv_by_rows(L)) {
+      rows  = true;
+      g.one = false;
+    } else if (L.kind == TDH_L_CONV && !conv_is_matvec(L)) {
+      pairs   = true;
+      if (!g.one) continue;
+      one     = std::max(one, best_pair_split(L, batch, true).us);
+      several = std::max(several, best_pair_split(L, batch, false).us);
+    } else if (L.kind == TDH_L_AVEPOOL) {
+      pools = true;
+      g.one = g.one && batch <= L.dw_chunk;
+    }
+  }
+  g.one = g.one && one <= several + 5.0 && (batch <= 32 || !(pairs || pools || m));
+  for (int i = 0; i < plan.n; ++i) {
+    const TinyLayer &L = plan.l[i];
+    g.size[i] = g.one ? batch : std::min(batch, 16);
+    if (!L.nw || i < m) continue;
+    if (conv_by_rows(L)) {
+      g.size[i] = 1;
+    } else if (L.kind == TDH_L_CONV && !conv_is_matvec(L)) {
+      const PairSplit p = best_pair_split(L, batch, g.one);
+      g.size[i]  = p.size;
+      g.waves[i] = p.waves;
+    } else if (L.kind == TDH_L_AVEPOOL) {
+      g.size[i] = std::min(g.size[i], L.dw_chunk);
+      if (rows) g.size[i] = std::min(g.size[i], std::max(4, batch * L.C / 256));   // (whose others are of one sample)
+    }
+  }
+  return g;
 }
 
 int launch_tiny_step(const TinyPlan &plan, const TinyPlan *dev_plan, int loss, int softmax_xent, int batch,
@@ -2649,19 +2795,17 @@ int launch_tiny_step(const TinyPlan &plan, const TinyPlan *dev_plan, int loss, i
   return TDH_OK;
 }
 
-int launch_tiny_params(const TinyPlan &plan, const TinyPlan *dev_plan, int batch, const float *x, tdh_opt *update,
-                       int n_tensors, const float *powers_in, float *powers_out, bool *updated) {
+int launch_tiny_params(const TinyPlan &plan, const TinyPlan *dev_plan, const TinyGroups &groups, int batch, const float *x,
+                       tdh_opt *update, int n_tensors, const float *powers_in, float *powers_out) {
   TinyRanges r;
   int n = 0, blocks = 0;
-  bool one_group = true;
+  int roads = plan.first_dx_as_job ? TP_HAS_PAIRS : 0;
   auto add = [&](int layer, int what, int count) {
-    const int groups = tiny_groups(plan, layer, batch);
     r.first[n]     = blocks;
-    r.job[n]       = layer * 8 + what;
+    r.job[n]       = layer * 16 + what;
     r.per_group[n] = count;
-    r.size[n++]    = ceil_div(batch, groups);
-    blocks += count * groups;
-    one_group = one_group && groups == 1;
+    r.size[n++]    = groups.size[layer];
+    blocks += count * ceil_div(batch, groups.size[layer]);
   };
   const int m = tiny_splits(plan, batch) ? plan.split : 0;
   for (int pass = 0; pass < 2; ++pass)   // (the convolutions first: they take longest)
@@ -2672,8 +2816,14 @@ int launch_tiny_params(const TinyPlan &plan, const TinyPlan *dev_plan, int batch
       if (i < m) {   // left by the back kernel, sample by sample
         add(i, TP_SLICES_W, ceil_div(L.nw, TP_THREADS));
         if (L.nb) add(i, TP_SLICES_B, ceil_div(L.nb, TP_THREADS));
+      } else if (conv_by_rows(L)) {
+        add(i, TP_ROWS, ceil_div(L.nw * conv_rows_lanes(L), TP_THREADS));
+        if (L.nb) add(i, TP_BIAS, 1);
+        roads |= TP_HAS_ROWS;
       } else if (pair) {
-        add(i, TP_CONV, L.K * L.C);
+        const bool waves = groups.waves[i];
+        roads |= TP_HAS_PAIRS | (waves ? TP_HAS_WAVES : 0);
+        add(i, waves ? TP_CONV_WAVES : TP_CONV, L.K * (waves ? ceil_div(L.C, TP_WAVES) : L.C));
       } else if (L.kind == TDH_L_AVEPOOL) {
         add(i, TP_POOL, L.C);
       } else {
@@ -2690,31 +2840,21 @@ int launch_tiny_params(const TinyPlan &plan, const TinyPlan *dev_plan, int batch
   }
   const int dx_blocks = plan.first_dx_as_job ? dx_band(plan.l[0]).bands * plan.l[0].C * batch : 0;
   TinyUpdate u;
-  *updated = update && one_group;
-  if (*updated) {
+  if (update) {
     u.p = opt_scalars(*update, 1.0f);
     u.n_tensors = n_tensors;
     u.b1_t = update->b1_t; u.b2_t = update->b2_t;
     u.powers_in = powers_in; u.powers_out = powers_out;
   }
   if (blocks + dx_blocks > 0) {
-    ProfScope prof("tiny_net_param_grads", plan.flop_per_sample * batch * (1.0 / 3.0), WORK_FLOP);
-    void (*kernel)(const TinyPlan *, const float *, TinyRanges, TinyUpdate, int, int) = tiny_net_param_kernel<-1>;
-    if (*updated) switch (update->kind) {
-      case TDH_OPT_SGD: kernel = tiny_net_param_kernel<TDH_OPT_SGD>; break;
-      case TDH_OPT_MOMENTUM: kernel = tiny_net_param_kernel<TDH_OPT_MOMENTUM>; break;
-      case TDH_OPT_NESTEROV: kernel = tiny_net_param_kernel<TDH_OPT_NESTEROV>; break;
-      case TDH_OPT_ADAM: kernel = tiny_net_param_kernel<TDH_OPT_ADAM>; break;
-      case TDH_OPT_ADAGRAD: kernel = tiny_net_param_kernel<TDH_OPT_ADAGRAD>; break;
-      case TDH_OPT_RMSPROP: kernel = tiny_net_param_kernel<TDH_OPT_RMSPROP>; break;
-      case TDH_OPT_ADAMAX: kernel = tiny_net_param_kernel<TDH_OPT_ADAMAX>; break;
-      default: return set_error(TDH_ERR_INVALID, "optimizer kind %d is not supported", update->kind);
-    }
+    ProfScope prof(roads & TP_HAS_ROWS ? "tiny_net_param_grads_any" : roads & TP_HAS_WAVES ? "tiny_net_param_grads_waves" : "tiny_net_param_grads", plan.flop_per_sample * batch * (1.0 / 3.0), WORK_FLOP);
+    const auto kernel = param_kernel(update ? update->kind : -1, roads);
+    if (!kernel) return set_error(TDH_ERR_INVALID, "optimizer kind %d is not supported", update->kind);
     TDH_LAUNCH(kernel, dim3(blocks + dx_blocks), dim3(TP_THREADS), plan.lds_job_floats * sizeof(float),
                ctx().stream, dev_plan, x, r, u, batch, blocks);
     TDH_LAUNCH_CHECK();
   }
-  if (*updated) opt_advance(update, n_tensors);
+  if (update) opt_advance(update, n_tensors);
   return TDH_OK;
 }
 
