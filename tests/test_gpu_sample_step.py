@@ -179,6 +179,25 @@ def test_nets_that_do_not_qualify_ignore_the_flag(T, O, W):
             assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("spec,max_batch,per_sample", [
+    ("lenet5", 512, True),
+    ([("fc", 784, 160), ("act", "tanh"), ("fc", 160, 10)], 512, True),     # 127 k parameters: just within 2^26 reads of weights a batch
+    ([("fc", 784, 170), ("act", "tanh"), ("fc", 170, 10)], 512, False),
+    ([("fc", 784, 1000), ("act", "tanh"), ("fc", 1000, 1000), ("act", "tanh"), ("fc", 1000, 10)], 64, False),
+    ([("fc", 784, 1000), ("act", "tanh"), ("fc", 1000, 1000), ("act", "tanh"), ("fc", 1000, 10)], 32, True),
+])
+def test_many_weights_for_the_batch_go_layer_by_layer(T, W, spec, max_batch, per_sample):
+    """Every sample's workgroup reads all weights: with many of them (parameters x largest batch) the flag is ignored."""
+    net = T.Net(W.build_layers(T, W.lenet5() if spec == "lenet5" else spec), max_batch, SAMPLE | FUSE)
+    x, t = T.DevBuf((4, net.in_size())), T.DevBuf((4, net.out_size()))
+    T.fill_zero(x)
+    T.fill_zero(t)
+    T.profile_begin()
+    net.train_step(None, "mse", 4, x, t, do_update=False)
+    assert any(e["tag"].startswith("tiny_net_step") for e in T.profile_end()) == per_sample
+    net.close()
+
+
 def _random_small_net(rng):
     """A random net that the per-sample kernel takes: one to three convolutions (3x3 or 5x5, with
     and without padding, 1 to 12 channels), pools that leave rows or columns uncovered, every

@@ -248,8 +248,8 @@ bool step_outlasts_launches(const tdh_net *net, int loss_kind, int batch) {
 
 // The plan of the one-workgroup-per-sample step (tiny_net.hip) for a net that qualifies: at most
 // TINY_MAX_LAYERS layers of the kinds that kernel knows, every layer output of one sample and two
-// gradient buffers within a workgroup's LDS, little arithmetic per sample, and room for the
-// per-sample gradient slices. Leaves net->tiny_ok false otherwise: the layer-by-layer step runs.
+// gradient buffers within a workgroup's LDS, little arithmetic per sample, and few weights for
+// its batch. Leaves net->tiny_ok false otherwise: the layer-by-layer step runs.
 int build_tiny_plan(tdh_net *net) {
   net->tiny_ok = false;
   const int n = static_cast<int>(net->layers.size());
@@ -259,7 +259,7 @@ int build_tiny_plan(tdh_net *net) {
   std::memset(&P, 0, sizeof(P));
   P.n       = n;
   P.in_size = static_cast<int>(net->layers[0].in_size);
-  size_t lds = net->layers[0].in_size, gmax = net->layers[0].in_size, slice_floats = 0;
+  size_t lds = net->layers[0].in_size, gmax = net->layers[0].in_size, slice_floats = 0, weight_reads = 0;
   const auto slices_of = [](size_t len, int count) { return ceil_div_sz(len * count, 4) * 4; };   // (16-byte aligned slices)
   int tensors = 0;
   for (int i = 0; i < n; ++i) {
@@ -328,7 +328,15 @@ int build_tiny_plan(tdh_net *net) {
       default: return TDH_OK;   // batch normalization, dropout: the layer-by-layer step
     }
     tensors += (L.w_size ? 1 : 0) + (L.b_size ? 1 : 0);
+    weight_reads += slices_of(L.w_size, net->max_batch) + slices_of(L.b_size, net->max_batch);
   }
+  // Every sample's workgroup reads all weights, forward and on the way back, through the caches and in the loops of one compute unit; where that
+  // is much in all, the layer-by-layer step's products over the whole batch win. A step, us, a workgroup per sample / layer by layer: 784-300-10
+  // fully connected, 512 samples 281 / 94; 784-1000-10, 128 samples 330 / 80; 784-1000-1000-10, 64 samples 772 / 108; 100-400-400-10, 512
+  // samples 222 / 124; 28x28, 1 -> 8 -> 16, 3x3, pools, 784-300-10, 512 samples 460 / 203. On this side of the line: LeNet-5, 512 samples 155 / 493;
+  // the same with 400-250-10 behind its second pool 278 / 442; 784-30-10, 512 samples 61 / 73. (A net of fully-connected layers alone is
+  // slower so from some 80 k weights on, whatever the batch: 784-100-10, 64 samples 54 / 39, 784-300-10 141 / 54.)
+  if (weight_reads > (64u << 20)) return TDH_OK;
   P.lds_g0 = static_cast<int>(lds);
   P.lds_g1 = static_cast<int>(lds + gmax);
   lds += 2 * gmax;
@@ -353,7 +361,6 @@ int build_tiny_plan(tdh_net *net) {
     slice_floats += slices_of(net->layers[i].w_size, parts) + slices_of(net->layers[i].b_size, parts) + 8;
   }
   slice_floats += slices_of(net->layers[0].w_size, 1);
-  if (slice_floats > (64u << 20)) return TDH_OK;
   float *slices = nullptr;
   TDH_TRY(net_alloc(net, slice_floats, &slices, false));
   P.first_w = slices;
