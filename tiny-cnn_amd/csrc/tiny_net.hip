@@ -11,10 +11,10 @@
 // the layer-by-layer path leaves. Nothing in that chain waits for a weight gradient, so those
 // are a launch behind it, (piece of a layer's parameters) x (group of samples), that reads
 // the layer's input and output gradient back from memory (tiny_net_param_kernel). A batch of one
-// group is updated there; what larger ones leave as one slice per group ([group][tensor]) the
+// group is updated there; what several leave as one slice each ([group][tensor]) the
 // optimizer's kernel adds up on its way (the split sums it also takes from the
-// layer-by-layer step); a step that stops at the gradients adds them to the gradient tensors in
-// order, as edge::merge_grads does (tiny_dnn/node.h:89-103), with a kernel of its own.
+// layer-by-layer step); a step that stops at the gradients adds the slices to the gradient tensors in the groups'
+// order, as edge::merge_grads does with samples (tiny_dnn/node.h:89-103), with a kernel of its own.
 //
 // The arithmetic of each layer follows the reference's scalar kernels: convolution sums the
 // taps of one input channel, then adds channel sums in channel order, then the bias
@@ -438,12 +438,11 @@ constexpr int TN_WAVES = TN_THREADS / 64;
 // [K][H + R - 1][W + S - 1] with dY[co][0][0] at row R-1-ph, column S-1-pw, so that every tap of
 // every input pixel reads inside the copy and the loops hold no bounds test: the tap (wy, wx) of
 // input pixel (iy, ix) is the copy's element (iy + R-1 - wy, ix + S-1 - wx).
-template <int NT, typename Src>
-TN_INLINE void stage_framed_dy(const TinyLayer *__restrict__ Lp, const Src *dy, float *framed) {
+TN_INLINE void stage_framed_dy(const TinyLayer *__restrict__ Lp, const float *dy, float *framed) {
   const int K = Lp->K, H = Lp->H, W = Lp->W, OH = Lp->OH, OW = Lp->OW, R = Lp->R, S = Lp->S;
   const int PW = W + S - 1, PP = (H + R - 1) * PW, oy0 = R - 1 - Lp->ph, ox0 = S - 1 - Lp->pw;
   const FastDiv d_pplane = Lp->d_pplane, d_pw = Lp->d_pw;
-  for (int e = threadIdx.x; e < K * PP; e += NT) {
+  for (int e = threadIdx.x; e < K * PP; e += TN_THREADS) {
     uint32_t co, r, py, px;
     d_pplane.divmod(e, co, r);
     d_pw.divmod(r, py, px);
@@ -576,25 +575,23 @@ TN_INLINE void conv_fwd_scalar_any(const TinyLayer *__restrict__ Lp, const float
   }
 }
 
-// dX from the zero-framed dY (stage_framed_dy); the waves of a workgroup of NT threads take the
-// items [item0, item1) of items * parts in turn (item = part * items + block * chunks + chunk);
-// dx (LDS) may be NULL
-template <int R, int S, int NB, int NT, bool TBL>
+// dX from the zero-framed dY (stage_framed_dy); the waves take items * parts in turn
+// (item = part * items + block * chunks + chunk)
+template <int R, int S, int NB, bool TBL>
 TN_INLINE void conv_bwd_dx_scalar(const TinyLayer *__restrict__ Lp, const float *framed, float *dx,
-                                  float *__restrict__ gdx, float *scratch, const int item0, const int item1,
-                                  const int parts) {
+                                  float *__restrict__ gdx, float *scratch) {
   const int C = Lp->C, H = Lp->H, W = Lp->W, K = Lp->K;
   const FastDiv d_w = Lp->d_w;
   const float *__restrict__ w = Lp->w;
   const uint8_t *__restrict__ tbl = Lp->tbl;
   constexpr int taps = R * S;
   const int plane = H * W, chunks = (plane + 63) >> 6, blocks = (C + NB - 1) / NB, items = blocks * chunks;
-  const int PW = W + S - 1, PP = (H + R - 1) * PW, Kh = (K + parts - 1) / parts;
-  const int lane = threadIdx.x & 63;
-  for (int it0 = item0; it0 < item1; it0 += NT / 64) {
+  const int parts = scalar_parts(items, K, TN_WAVES), PW = W + S - 1, PP = (H + R - 1) * PW, Kh = (K + parts - 1) / parts;
+  const int total = items * parts, lane = threadIdx.x & 63;
+  for (int it0 = 0; it0 < total; it0 += TN_WAVES) {
     const int item = it0 + wave_index();
-    const bool active = item < item1;
-    const int it = active ? item : item0;
+    const bool active = item < total;
+    const int it = active ? item : 0;
     const int kp = it / items, rem = it - kp * items, blk = rem / chunks, chunk = rem - blk * chunks, ci0 = blk * NB;
     const int p = (chunk << 6) + lane;
     const bool live = p < plane;
@@ -647,30 +644,24 @@ TN_INLINE void conv_bwd_dx_scalar(const TinyLayer *__restrict__ Lp, const float 
 #pragma unroll
       for (int q = 0; q < NB; ++q)
         if (ci0 + q < C) {
-          if (dx) dx[(ci0 + q) * plane + p] = acc[q];
+          dx[(ci0 + q) * plane + p] = acc[q];
           if (gdx) gdx[(ci0 + q) * plane + p] = acc[q];
         }
     }
   }
 }
-// whole-wave items of the scalar dX
-__host__ __device__ inline int conv_dx_scalar_items(const TinyLayer &L) {
-  const int nb = scalar_block(L.C);
-  return ((L.C + nb - 1) / nb) * ((L.H * L.W + 63) >> 6);
-}
-template <int R, int S, int NT>
+template <int R, int S>
 TN_INLINE void conv_bwd_dx_scalar_any(const TinyLayer *__restrict__ Lp, const float *framed, float *dx,
-                                      float *__restrict__ gdx, float *scratch, const int item0, const int item1,
-                                      const int parts) {
+                                      float *__restrict__ gdx, float *scratch) {
   const int nb = scalar_block(Lp->C);
   if (Lp->tbl) {
-    if (nb == 1) conv_bwd_dx_scalar<R, S, 1, NT, true>(Lp, framed, dx, gdx, scratch, item0, item1, parts);
-    else if (nb == 3) conv_bwd_dx_scalar<R, S, 3, NT, true>(Lp, framed, dx, gdx, scratch, item0, item1, parts);
-    else conv_bwd_dx_scalar<R, S, 4, NT, true>(Lp, framed, dx, gdx, scratch, item0, item1, parts);
+    if (nb == 1) conv_bwd_dx_scalar<R, S, 1, true>(Lp, framed, dx, gdx, scratch);
+    else if (nb == 3) conv_bwd_dx_scalar<R, S, 3, true>(Lp, framed, dx, gdx, scratch);
+    else conv_bwd_dx_scalar<R, S, 4, true>(Lp, framed, dx, gdx, scratch);
   } else {
-    if (nb == 1) conv_bwd_dx_scalar<R, S, 1, NT, false>(Lp, framed, dx, gdx, scratch, item0, item1, parts);
-    else if (nb == 3) conv_bwd_dx_scalar<R, S, 3, NT, false>(Lp, framed, dx, gdx, scratch, item0, item1, parts);
-    else conv_bwd_dx_scalar<R, S, 4, NT, false>(Lp, framed, dx, gdx, scratch, item0, item1, parts);
+    if (nb == 1) conv_bwd_dx_scalar<R, S, 1, false>(Lp, framed, dx, gdx, scratch);
+    else if (nb == 3) conv_bwd_dx_scalar<R, S, 3, false>(Lp, framed, dx, gdx, scratch);
+    else conv_bwd_dx_scalar<R, S, 4, false>(Lp, framed, dx, gdx, scratch);
   }
 }
 
@@ -1435,7 +1426,7 @@ tiny_net_step_kernel(const TinyPlan *__restrict__ plan, const int m, const int l
     const TinyLayer *__restrict__ L = &plan->l[li];
     const int kind = L->kind, in_sz = L->in_size;
     // (the layer in front of this one in memory order is the next to run: its operand goes into
-    // the scratch area now, which this phase does not use when that is so; see tiny_build_jobs)
+    // the scratch area now, which this phase does not use when that is so; see tiny_layout)
     if (li - 1 == ahead && ahead >= last_bwd && plan->l[ahead].mf_dx_w >= 0) mfma_dx_operand_store(&plan->l[ahead], ahead_w, lds);
     float *gdx = L->dx ? L->dx + static_cast<size_t>(s) * in_sz : nullptr;
     const BwdOut plain = bwd_out(plan, lds, gb, li, s, false);
@@ -1448,9 +1439,8 @@ tiny_net_step_kernel(const TinyPlan *__restrict__ plan, const int m, const int l
         else if (!L->dx_framed) conv_bwd_dx(L, ga, gb, gdx);
         else {
           float *framed = lds + plan->lds_pad;
-          stage_framed_dy<TN_THREADS>(L, ga, framed);
+          stage_framed_dy(L, ga, framed);
           lds_barrier();
-          const int items = conv_dx_scalar_items(*L), parts = scalar_parts(items, L->K, TN_WAVES);
           if (L->mf_dx_w >= 0) {
             // (the operand was written into the scratch area while the layer behind ran; D has every
             // position of H framed rows as a column, so a column's offset is its index)
@@ -1461,8 +1451,8 @@ tiny_net_step_kernel(const TinyPlan *__restrict__ plan, const int m, const int l
             lds_barrier();
             mfma_dx_gather(L, dd, gb, gdx);
           }
-          else if (L->R == 5) conv_bwd_dx_scalar_any<5, 5, TN_THREADS>(L, framed, gb, gdx, wl, 0, items * parts, parts);
-          else conv_bwd_dx_scalar_any<3, 3, TN_THREADS>(L, framed, gb, gdx, wl, 0, items * parts, parts);
+          else if (L->R == 5) conv_bwd_dx_scalar_any<5, 5>(L, framed, gb, gdx, wl);
+          else conv_bwd_dx_scalar_any<3, 3>(L, framed, gb, gdx, wl);
         }
         break;
       case TDH_L_FC: fc_bwd_dx(L, ga, plain); break;
@@ -1488,7 +1478,7 @@ tiny_net_step_kernel(const TinyPlan *__restrict__ plan, const int m, const int l
 // keeps to one channel: a workgroup takes one channel of a sample through it, forward in a launch in
 // front of the step kernel, and in a launch behind it from the second convolution's dX back to the
 // gradient of the first one's output. Bound: latency, a launch and some three trips to memory each.
-// LeNet-5, batch 16, us: here 4.5 + 17.3 + 7.8, and the whole step 40.7 where in one launch it is 52.1 (which batches: launch_tiny_step).
+// LeNet-5, batch 16, us in a trace: front 5.0, step kernel 17.9, back 10.0, and the whole step 40.6 where in one launch it is 52.1 (which batches: tiny_most_split).
 constexpr int TF_THREADS = 1024;   // front, at most
 constexpr int TB_THREADS = 1024;   // back
 static_assert(TB_THREADS / 64 == 16, "sixteen shares of a pool's sums; a wave left over from five rows of three and from three of five");
@@ -1688,31 +1678,24 @@ TN_INLINE void conv_back_dx(const TinyLayer *__restrict__ Lp, const BackSplit b,
   }
 }
 
-// Four neighbouring output pixels of a unit-stride convolution, from the four gradients d: acc[wy][wx] += d * X.
-// xr: X's row under filter row 0, at the first pixel's column with the padding in front (rows of xp floats, a multiple of
-// four); iy0, ix0: that row and column of the image. Products that do not exist (past the row's end, or outside the
+// Four neighbouring output pixels of a unit-stride convolution and one filter row, from the four gradients d: acc[wx] += d * X.
+// xr: X's row under that filter row, at the first pixel's column with the padding in front (rows of xp floats, a multiple of
+// four); iy, ix0: that row and column of the image. Products that do not exist (past the row's end, or outside the
 // input) are left out, not multiplied by zero: an infinity stays out of sums that it is no part of.
-template <int ROWS, int S, bool PAD>
-TN_INLINE void dw_quad(float (&acc)[ROWS][S], const float *xr, const int xp, const float (&d)[4], const int iy0, const int ix0,
+template <int S, bool PAD>
+TN_INLINE void dw_quad(float (&acc)[S], const float *xr, const int xp, const float (&d)[4], const int iy, const int ix0,
                        const int H, const int W, const int left) {
-  float v[ROWS][S + 3];
-#pragma unroll
-  for (int wy = 0; wy < ROWS; ++wy) {
-    const bool row = !PAD || static_cast<unsigned>(iy0 + wy) < static_cast<unsigned>(H);
-    read_row(v[wy], xr + (row ? wy * xp : -iy0 * xp));
-  }
+  const bool row = !PAD || static_cast<unsigned>(iy) < static_cast<unsigned>(H);
+  float v[S + 3];
+  read_row(v, xr + (row ? 0 : -iy * xp));
 #pragma unroll
   for (int k = 0; k < 4; ++k)
     if (k < left) {
 #pragma unroll
-      for (int wy = 0; wy < ROWS; ++wy) {
-        const bool row = !PAD || static_cast<unsigned>(iy0 + wy) < static_cast<unsigned>(H);
-#pragma unroll
-        for (int wx = 0; wx < S; ++wx) {
-          const float sum = __builtin_fmaf(d[k], v[wy][k + wx], acc[wy][wx]);
-          const bool in   = !PAD || (row && static_cast<unsigned>(ix0 + k + wx) < static_cast<unsigned>(W));
-          acc[wy][wx] = in ? sum : acc[wy][wx];
-        }
+      for (int wx = 0; wx < S; ++wx) {
+        const float sum = __builtin_fmaf(d[k], v[k + wx], acc[wx]);
+        const bool in   = !PAD || (row && static_cast<unsigned>(ix0 + k + wx) < static_cast<unsigned>(W));
+        acc[wx] = in ? sum : acc[wx];
       }
     }
 }
@@ -1733,9 +1716,9 @@ TN_INLINE void conv_back_param(const TinyLayer *__restrict__ L, const float *x, 
   const int wave = wave_index(), wy = wave / PER_ROW, sub = wave - wy * PER_ROW, lane = threadIdx.x & 63;
   float *pw = L->pw_part + static_cast<size_t>(s) * L->nw + static_cast<size_t>(co) * C * taps;
   for (int ci = 0; ci < C; ++ci) {
-    float acc[1][S], db = 0.0f;
+    float acc[S], db = 0.0f;
 #pragma unroll
-    for (int wx = 0; wx < S; ++wx) acc[0][wx] = 0.0f;
+    for (int wx = 0; wx < S; ++wx) acc[wx] = 0.0f;
     if (wy < R)
       for (int i = sub * 64 + lane; i < units; i += 64 * PER_ROW) {
         uint32_t oy, q;
@@ -1749,16 +1732,16 @@ TN_INLINE void conv_back_param(const TinyLayer *__restrict__ L, const float *x, 
 #pragma unroll
           for (int k = 0; k < 4; ++k) d[k] = dr[k < left ? k : 0];
         }
-        dw_quad<1, S, PAD>(acc, x + (ci * H + iy) * xp + 4 * q, xp, d, iy, 4 * static_cast<int>(q) - pw0, H, W, left);
+        dw_quad<S, PAD>(acc, x + (ci * H + iy) * xp + 4 * q, xp, d, iy, 4 * static_cast<int>(q) - pw0, H, W, left);
 #pragma unroll
         for (int k = 0; k < 4; ++k) db += k < left ? d[k] : 0.0f;
       }
 #pragma unroll
-    for (int wx = 0; wx < S; ++wx) acc[0][wx] = wave_sum_63(acc[0][wx]);
+    for (int wx = 0; wx < S; ++wx) acc[wx] = wave_sum_63(acc[wx]);
     db = wave_sum_63(db);
     if (lane == 63) {
 #pragma unroll
-      for (int wx = 0; wx < S; ++wx) red[wave * (S + 1) + wx] = acc[0][wx];
+      for (int wx = 0; wx < S; ++wx) red[wave * (S + 1) + wx] = acc[wx];
       red[wave * (S + 1) + S] = db;
     }
     lds_barrier();
@@ -1784,7 +1767,7 @@ tiny_net_back_kernel(const TinyPlan *__restrict__ plan, const int m, const float
   constexpr int AHEAD = 4;   // gradients a thread holds, and layers whose outputs it does
   const int s = blockIdx.x, ci = blockIdx.y, n = plan->n, tid = threadIdx.x;
   const TinyLayer *__restrict__ L = &plan->l[m];
-  const int K = L->K, H = L->H, W = L->W, R = L->R, S = L->S, OW = L->OW, out_size = L->out_size, taps = R * S;
+  const int K = L->K, H = L->H, W = L->W, R = L->R, S = L->S, out_size = L->out_size, taps = R * S;
   const float *gdy = (m == n - 1 ? plan->dloss : plan->l[m + 1].dx) + static_cast<size_t>(s) * out_size;
   float dy[AHEAD];
 #pragma unroll
@@ -1930,8 +1913,8 @@ tiny_net_back_kernel(const TinyPlan *__restrict__ plan, const int m, const float
 // there; the groups of a larger one leave a slice each ([group][tensor]) for the optimizer's kernel, or for
 // tiny_net_merge_kernel. Behind those workgroups come the ones of the first layer's input gradient, which
 // nothing waits for either. Bound: latency (kernel arguments, the layer's sizes, one trip for the operands, the sums).
-// us, a slice per sample and the optimizer's launch / here: LeNet-5, batch 16 9.2 + 5.0 / 7.8 (and 2 in the back kernel), 32
-// 14.6 + 7.3 / 11.1, 64 24.4 + 7.4 / 15.3 + 5.6, 120 40.0 + 12.9 / 25.9 + 6.8, 300 86.4 + 20.6 / 55.9 + 9.3.
+// us, a slice per sample and the optimizer's launch / here: LeNet-5, batch 16 8.7 + 4.9 / 8.0 (and 2 in the back kernel), 64
+// 23.6 + 6.2 / 13.8 + 4.6, 128 40.2 + 9.6 / 21.8 + 5.4, 256 70.9 + 15.8 / 38.7 + 7.7.
 constexpr int TP_THREADS = 512, TP_WAVES = TP_THREADS / 64;
 enum { TP_CONV, TP_CONV_WAVES, TP_ROWS, TP_BIAS, TP_OUTER, TP_OUTER4, TP_COLUMNS, TP_POOL, TP_SLICES_W, TP_SLICES_B };   // what a range of workgroups does
 constexpr int TP_RANGES = 2 * TINY_MAX_LAYERS;
