@@ -278,12 +278,15 @@ enum {
   /* A net whose activations of one sample fit in a workgroup's local memory (LeNet-5) trains in
    * two to five launches: one workgroup per sample runs forward, the loss gradient and the input
    * gradients of the layers (the first block and the way back to it, a channel a workgroup, in launches of
-   * their own for small batches); one launch computes the weight and bias gradients over the batch and, up to 32
-   * samples, updates; larger batches leave a slice per group of samples, which the optimizer launch adds up (a step
-   * without an update adds to the gradient tensors in sample order instead, edge::merge_grads,
-   * tiny_dnn/node.h:89-103). Every layer output, input gradient and max-pool record is still
-   * written to memory. Nets that do not qualify (size, batch normalization, dropout, a softmax
-   * that is not the closing layer of a cross_entropy_multiclass net) ignore the flag. */
+   * their own for small batches); one launch computes the weight and bias gradients over groups of samples, whose
+   * sizes follow from the layers and the batch. Where one group of all samples is the faster way, as in most nets
+   * up to 16 or 32 samples, that launch updates as well; else every group leaves a slice, which the optimizer
+   * launch adds up. Inside a group the order of a sum is fixed but is not the samples'; the slices are added in
+   * the groups' order, also by a step without an update, which adds them to the gradient tensors
+   * (edge::merge_grads, tiny_dnn/node.h:89-103). Every layer output, input gradient and max-pool record is still
+   * written to memory. Nets that do not qualify (size, more than 2^26 parameters x max_batch, batch
+   * normalization, dropout, a softmax that is not the closing layer of a cross_entropy_multiclass net) ignore
+   * the flag. */
   TDH_NET_SAMPLE_STEP   = 4,
   /* Training never reads the gradient with respect to the net's input, which the reference
    * computes like every other (layer::backward of the first layer fills the gradient of its

@@ -415,8 +415,9 @@ struct DxsPlan {
 // output channel at a time).
 // Bound: vector instructions (108 multiply-adds a lane and channel for 3x3 on three channels; staged by elements, a
 // chunk's 20 loads with their addresses and stores are as many again, and the weights nine of fifteen LDS reads a
-// channel). 3 <- 64 channels, 3x3, 128x128, batch 64: 111 us by elements, 84 by words. (Scalar weights and elements: 3 <- 24,
-// 3x3, 30x30, batch 37 9.1 us, with the weights in LDS 8.8; the few workgroups wait for each channel's.)
+// channel). us by elements / words: 3 <- 64 channels, 3x3, 128x128, 64 images 111 / 84, one image 17.6 / 11.1; 3 <- 24, 28x28, 4 images
+// 8.7 / 6.0; 4 <- 16, 5x5, 64x64, 2 images 9.6 / 7.3: with words at any number of workgroups. (Scalar weights and elements: 3 <- 24,
+// 3x3, 30x30, 37 images 9.1 us, with the weights in LDS 8.8; the few workgroups wait for each channel's.)
 template <int KR, int KS, int CIN, bool POOLED, int SHIFT = -1>
 __global__ void __launch_bounds__(DXS_NT)
 conv_dx_small_cin_kernel(const float *__restrict__ dy, const float *__restrict__ w,
@@ -1504,7 +1505,8 @@ bool conv_fwd_fuses_pool(const tdh_conv_desc *d, const tdh_pool_desc *pool, int 
          conv_s1_fuses_pool(g.R, g.S, batch, g.C, g.Kc, g.H, g.W, g.OH, g.OW, g.pad_h, g.pad_w);
 }
 
-// with the pool alone behind it (in longer rows the convolution's own output is what a train step has always left there)
+// with the pool alone behind it (in rows of 8 and 16; in longer ones a train step's caller finds the convolution's own output, as it did
+// when the pool ran by itself there)
 bool conv_fwd_pool_replaces_out(const tdh_conv_desc *d, int batch, bool prepacked) {
   const ConvGeom g = make_geom(d);
   if (!prepacked && (fwd_direct_applies(g, batch) || fwd_small_applies(g, batch))) return true;
@@ -1695,8 +1697,8 @@ static int run_any_both(const tdh_conv_desc *d, const ConvGeom &g, int batch, co
   sums.M = g.Kc; sums.N = crs + (with_db ? 1 : 0);
   sums.epi = EpiDwDb{dw, db, crs, accumulate};
   // Very many slices, which launch_splitk_reduce has another kernel for, stay with it, and so do sums of more than three workgroups a
-  // compute unit, each of which would hold a place of dX's: forward, dX and dW of 51x50, 128 -> 150, 3x3, stride 2, 20 images (1351
-  // workgroups) 304 us along, 298 apart; 33x29, 40 -> 41, 7x7, 11 images (628) 99 / 107.
+  // compute unit, each of which holds a place of dX's. Drawn layers, dX, dW and db, apart over along: 38 of 250 to 768 workgroups 0.998 to 1.15,
+  // 29 of 800 to 2600 0.954 (51x50, 128 -> 150, 3x3, stride 2, 20 images: 176 us apart, 184 along) to 1.08, 26 of 3300 and more 0.73 to 1.02.
   sums.blocks      = ceil_div(sums.M * sums.N, ANY_SUMS);
   const bool along = slices < 64 * REDUCE_GROUPS && sums.blocks <= 768 && conv_any_dx_has_room(shape, sums.blocks);
   if (!along) sums.blocks = 0;

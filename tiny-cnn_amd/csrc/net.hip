@@ -902,7 +902,7 @@ int tdh_net_create(const tdh_layer *layers, int n_layers, int max_batch, int fla
         // weight gradients whose kernels may leave split sums to the optimizer: small blocks,
         // eight groups of lanes add the slices of OPT_SUM_ELEMS_PER_BLOCK elements
         // (and every tensor of a net that may run the workgroup-per-sample step, whose
-        // per-sample slices take the same way)
+        // slices of sample groups take the same way)
         t.block_elems = (((L.spec.kind == TDH_L_CONV || L.spec.kind == TDH_L_FC) && (flags & TDH_NET_GRAPH)) ||
                          (flags & TDH_NET_SAMPLE_STEP))
                           ? OPT_SUM_ELEMS_PER_BLOCK : OPT_MULTI_ELEMS_PER_BLOCK;
