@@ -66,3 +66,28 @@ def test_pool_of_rows_as_its_own_kernel(T, W, width, height, in_c, out_c, window
     record = (np.arange(out_c) * height * width)[None, :, None] + top[None, None, :] + (first >> 1) * width + (first & 1)
     assert np.array_equal(net.layer_argmax(pool, batch).ravel(), record.ravel())
     net.close()
+
+
+@pytest.mark.parametrize("window", [3, 5])
+def test_rows_of_64_take_no_longer_than_rows_of_32(T, W, window):
+    """A train step's forward pass of 32 channels or fewer, in tiles of 512 pixels: as many products in rows of either length.
+    (With the blocks of the wider rows in another order the kernel's registers went to memory: 1.13 and 1.27 times; else 1.00 and 1.02.)"""
+    us = {}
+    for width, batch in ((32, 256), (64, 64)):
+        layers = W.build_layers(T, [("conv", width, width, 32, window, 32, True)])
+        net = T.Net(layers, batch, 0)
+        for i, which, n in net.params():
+            net.set_param(i, which, np.linspace(-0.1, 0.1, n, dtype=np.float32))
+        x = T.to_device(np.linspace(-1, 1, batch * net.in_size(), dtype=np.float32).reshape(batch, -1))
+        t = T.DevBuf((batch, net.layer_out_size(0)), zero=True)
+        net.train_step(None, "mse", batch, x, t, do_update=False)
+        best = float("inf")
+        for _ in range(5):
+            T.profile_begin()
+            for _ in range(10):
+                net.train_step(None, "mse", batch, x, t, do_update=False)
+            best = min([best] + [e["avg_us"] for e in T.profile_end() if e["tag"].startswith("conv_fwd_s1")])
+        us[width] = best
+        net.close()
+    print(us)
+    assert us[64] < 1.08 * us[32], us

@@ -33,13 +33,17 @@ constexpr size_t x3_pack_bytes(int RS, int KC, int MC) {
 }
 
 // The first pixel, in the workgroup's tile of rows of TC pixels, of accumulator block b = wave * TN + j. Blocks are 32 pixels in
-// a row; where rows are longer, two blocks of a wave that follow each other are the same columns of two rows, so that
-// a lane holds both rows of its column and two lanes a 2x2 pooling window. (Not in the three-part kernel, whose waves read
+// a row, one after the other; where a row of 64 is two blocks and a wave has two, they are the same columns of two rows, so that a lane
+// holds both rows of its column and two lanes a 2x2 pooling window. A wave of four blocks of such rows holds two rows anyway (in any
+// other order the instance needs more than the 256 registers there are: 80 of them went to memory, and 24 -> 32 channels, 5x5, 96x96,
+// 16 images, tanh and the pool took 105 us instead of 89). (Not in the three-part kernel, whose waves read
 // 0.5 % slower that way: 32 -> 64 channels, 3x3, 64x64, batch 64, forward, dX and dW 219.3 us / 220.3.)
 template <int TC, int TN>
 __host__ __device__ constexpr int s1_block_pixel(const int b) {
-  return TC == 64 && TN % 2 == 0 ? ((b >> 2) * 2 + (b & 1)) * 64 + ((b >> 1) & 1) * 32 : 32 * b;
+  return TC == 64 && TN == 2 ? ((b >> 2) * 2 + (b & 1)) * 64 + ((b >> 1) & 1) * 32 : 32 * b;
 }
+// how many blocks further on in the wave the one below a block is
+constexpr int s1_block_below(const int TC, const int TN) { return TC == 64 && TN == 4 ? 2 : 1; }
 
 // the sign of step u's products (chunk, tap): the packed filters carry it
 __host__ __device__ constexpr float x3_sign(int u) { return u & 1 ? -1.0f : 1.0f; }

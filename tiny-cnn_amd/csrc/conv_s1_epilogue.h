@@ -20,7 +20,7 @@ __device__ __forceinline__ float s1_lane_xor(const float v) {
   return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (X << 10) | 0x1F));
 }
 
-// The forward pass with a 2x2 max-pool behind it where blocks j and j + 1 of a wave are two rows (s1_block_pixel): a lane
+// The forward pass with a 2x2 max-pool behind it where a wave holds two rows of a block's columns (s1_block_pixel, s1_block_below): a lane
 // holds both rows of its column, two neighbours share a window, exchange the values of two channels and pool one each,
 // with strict '>' from lowest() in scan order (maxpool_op_internal.h:17-47). The pool's own kernel is bound by the read of
 // the activation, which no kernel reads next once the pool is made here: y and it go past the caches. us of
@@ -33,7 +33,9 @@ __device__ __forceinline__ void s1_epilogue_pool_rows(const ConvS1Args &a, const
   const int ohw = a.OH * a.OW, pw2 = a.OW >> 1, pohw = (a.OH >> 1) * pw2;
   const bool right = lane & 1;
 #pragma unroll
-  for (int j = 0; j < TN; j += 2) {
+  for (int pair = 0; pair < TN / 2; ++pair) {
+    constexpr int BELOW = s1_block_below(TC, TN);
+    const int j   = BELOW == 1 ? 2 * pair : pair;
     const int q   = s1_block_pixel<TC, TN>(wn * TN + j) + (lane & 31);
     const int img = img0 + (q >> (a.log_tr + LOG_TC));
     const int oy = y0 + ((q >> LOG_TC) & (a.TR - 1)), ox = x0 + (q & (TC - 1));
@@ -48,7 +50,7 @@ __device__ __forceinline__ void s1_epilogue_pool_rows(const ConvS1Args &a, const
 #pragma unroll
       for (int rr = 0; rr < 16; ++rr) {
         v0[rr] = acc[i][j][rr];
-        v1[rr] = acc[i][j + 1][rr];
+        v1[rr] = acc[i][j + BELOW][rr];
       }
       if (a.bias) {
 #pragma unroll
