@@ -105,7 +105,8 @@ __device__ __forceinline__ void s1_epilogue_pool_rows(const ConvS1Args &a, const
   }
 }
 
-// ROWS: the wave's blocks lie as s1_block_pixel<TC, TN> has them, else one after the other
+// ROWS: the wave's blocks lie as s1_block_pixel<TC, TN> has them and the pool behind rows of 32 and 64 can be made here, else
+// the blocks lie one after the other
 template <int TC, int TM, int TN, bool ROWS = true>
 __device__ __forceinline__ void s1_epilogue(const ConvS1Args &a, const floatx16 (&acc)[TM][TN], const int wn,
                                             const int lane, const int img0, const int y0, const int x0,

@@ -33,10 +33,10 @@ __device__ __forceinline__ void x3_redo_exceptional(const ConvS1Args &a, floatx1
                                                     const int m0, const int kc_lo, const int kc_hi) {
   constexpr int LOG_TC = TC == 64 ? 6 : TC == 32 ? 5 : TC == 16 ? 4 : 3;
   // (hidden from the compiler, which otherwise keeps this function's comparisons and addresses for the stores behind)
-  int rows = a.MC - (m0 + 4 * (lane >> 5)), pix = lane & 31;
+  int rows = a.MC - (m0 + 4 * (lane >> 5)), pix = wn * TN * 32 + (lane & 31);
   asm volatile("" : "+v"(rows), "+v"(pix));
   auto place = [&](int j, int &img, int &oy, int &ox) {
-    const int q = pix + s1_block_pixel<TC, 1>(wn * TN + j);
+    const int q = pix + 32 * j;
     img = img0 + (q >> (a.log_tr + LOG_TC));
     oy  = y0 + ((q >> LOG_TC) & (a.TR - 1));
     ox  = x0 + (q & (TC - 1));
@@ -85,8 +85,9 @@ __device__ __forceinline__ void x3_redo_exceptional(const ConvS1Args &a, floatx1
 }
 
 // the workgroup at (bx, by, bz) of the grid. BY_TAPS: the four waves share the
-// workgroup's 32 channels x 128 pixels (TM = TN = 1) by filter taps instead of by pixels
-template <int R, int S, int TC, int TM, int TN, bool VEC, bool BY_TAPS>
+// workgroup's 32 channels x 128 pixels (TM = TN = 1) by filter taps instead of by pixels. POOL: with the max-pool behind
+// rows of 32 (shorter rows always can)
+template <int R, int S, int TC, int TM, int TN, bool VEC, bool BY_TAPS, bool POOL = false>
 __device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, const int bx, const int by, const int bz) {
   static_assert(!BY_TAPS || (TM == 1 && TN == 1), "a tile of 32 channels x 128 pixels");
   constexpr int RS     = R * S;
@@ -155,7 +156,7 @@ __device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, const int
   int bpix[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    const int q  = s1_block_pixel<TC, 1>((BY_TAPS ? 0 : wn * TN) + j) + (lane & 31);
+    const int q  = ((BY_TAPS ? 0 : wn * TN) + j) * 32 + (lane & 31);
     const int ti = q >> (a.log_tr + LOG_TC);
     const int r  = (q >> LOG_TC) & (a.TR - 1);
     const int c  = q & (TC - 1);
@@ -335,7 +336,7 @@ __device__ __forceinline__ void conv_x3_workgroup(const ConvS1Args &a, const int
     }
   }
   x3_redo_exceptional<R, S, TC, TM, TN>(a, acc, wn, lane, img0, y0, x0, m0, kc_lo, kc_hi);
-  s1_epilogue<TC, TM, TN, TC != 64>(a, acc, wn, lane, img0, y0, x0, m0, bz);
+  s1_epilogue<TC, TM, TN, POOL>(a, acc, wn, lane, img0, y0, x0, m0, bz);
   }
 }
 
