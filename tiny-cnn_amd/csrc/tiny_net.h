@@ -70,6 +70,7 @@ struct TinyPlan {
   double flop_per_sample;
   int first_dx_as_job;         // the first layer's input gradient is computed beside the parameter gradients,
   float *first_w;              // ... from this copy of its filters (memory), which the step kernel makes
+  int by_rows;                 // weight gradients of convolutions sample by sample (a window is not 3x3 or 5x5, or strided)
   int skip_first_dx;           // nobody wants the gradient of the net's input: it is not computed
   int lds_job_floats;          // LDS of the parameter-gradient kernel
 };

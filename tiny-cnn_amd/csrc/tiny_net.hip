@@ -1916,7 +1916,8 @@ tiny_net_back_kernel(const TinyPlan *__restrict__ plan, const int m, const float
 // us, a slice per sample and the optimizer's launch / here: LeNet-5, batch 16 8.7 + 4.9 / 8.0 (and 2 in the back kernel), 64
 // 23.6 + 6.2 / 13.8 + 4.6, 128 40.2 + 9.6 / 21.8 + 5.4, 256 70.9 + 15.8 / 38.7 + 7.7.
 constexpr int TP_THREADS = 512, TP_WAVES = TP_THREADS / 64;
-enum { TP_CONV, TP_CONV_WAVES, TP_ROWS, TP_BIAS, TP_OUTER, TP_OUTER4, TP_COLUMNS, TP_POOL, TP_SLICES_W, TP_SLICES_B };   // what a range of workgroups does
+constexpr int TR_THREADS = 256;   // where the convolutions go sample by sample: more and smaller workgroups share the chip more evenly
+enum { TP_CONV, TP_CONV_WAVES, TP_ROWS, TP_OUTER, TP_OUTER4, TP_COLUMNS, TP_POOL, TP_SLICES_W, TP_SLICES_B };   // what a range of workgroups does
 constexpr int TP_RANGES = 2 * TINY_MAX_LAYERS;
 struct TinyRanges {
   int first[TP_RANGES];     // first workgroup; past the last range larger than any
@@ -1989,6 +1990,7 @@ TN_INLINE void tn_finish(const TinyTarget &t, TinyOld o, const int e, const floa
 
 // x_plane values of the layer's input (one of its planes, or some that follow each other) and one plane of its output
 // gradient, of ns samples, into LDS, all of a trip's reads before its first store
+template <int NT>
 TN_INLINE void stage_planes(const TinyLayer *__restrict__ L, float *xl, const float *__restrict__ x, const int x_stride,
                             const int x_plane, const FastDiv d_x, float *dl, const float *__restrict__ d, const int d_stride,
                             const int ns) {
@@ -2004,38 +2006,39 @@ TN_INLINE void stage_planes(const TinyLayer *__restrict__ L, float *xl, const fl
   };
   if (vec) {
     constexpr int AHEAD = 4;
-    for (int base = 4 * threadIdx.x; base < total; base += 4 * AHEAD * TP_THREADS) {
+    for (int base = 4 * threadIdx.x; base < total; base += 4 * AHEAD * NT) {
       float4 v[AHEAD];
 #pragma unroll
-      for (int j = 0; j < AHEAD; ++j) v[j] = *reinterpret_cast<const float4 *>(from(min(base + 4 * j * TP_THREADS, total - 4)));
+      for (int j = 0; j < AHEAD; ++j) v[j] = *reinterpret_cast<const float4 *>(from(min(base + 4 * j * NT, total - 4)));
 #pragma unroll
       for (int j = 0; j < AHEAD; ++j) {
-        const int e = base + 4 * j * TP_THREADS;
+        const int e = base + 4 * j * NT;
         if (e < total) *reinterpret_cast<float4 *>(e < nx ? xl + e : dl + e - nx) = v[j];
       }
     }
   } else {
     constexpr int AHEAD = 12;
-    for (int base = threadIdx.x; base < total; base += AHEAD * TP_THREADS) {
+    for (int base = threadIdx.x; base < total; base += AHEAD * NT) {
       float v[AHEAD];
 #pragma unroll
-      for (int j = 0; j < AHEAD; ++j) v[j] = *from(min(base + j * TP_THREADS, total - 1));
+      for (int j = 0; j < AHEAD; ++j) v[j] = *from(min(base + j * NT, total - 1));
 #pragma unroll
       for (int j = 0; j < AHEAD; ++j) {
-        const int e = base + j * TP_THREADS;
+        const int e = base + j * NT;
         if (e < total) *(e < nx ? xl + e : dl + e - nx) = v[j];
       }
     }
   }
 }
-// sum over the workgroup, in every thread of its first wave; `red`: TP_WAVES floats of LDS that nobody else uses
+// sum over the workgroup, in every thread of its first wave; `red`: NT / 64 floats of LDS that nobody else uses
+template <int NT>
 TN_INLINE float workgroup_sum(float v, float *red) {
   v = wave_sum_63(v);
   if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6] = v;
   lds_barrier();
   v = red[0];
 #pragma unroll
-  for (int k = 1; k < TP_WAVES; ++k) v += red[k];
+  for (int k = 1; k < NT / 64; ++k) v += red[k];
   return v;
 }
 
@@ -2085,7 +2088,7 @@ TN_INLINE void conv_param_pair(const TinyLayer *__restrict__ L, const float *__r
   for (int s0 = s_beg; s0 < s_end; s0 += chunk) {
     const int ns = min(chunk, s_end - s0);
     if (s0 > s_beg) lds_barrier();
-    stage_planes(L, xl, gin + static_cast<size_t>(s0) * in_sz + ci_first * iplane, in_sz, x_plane, d_x, dl,
+    stage_planes<TP_THREADS>(L, xl, gin + static_cast<size_t>(s0) * in_sz + ci_first * iplane, in_sz, x_plane, d_x, dl,
                  gdy + static_cast<size_t>(s0) * out_sz + co * plane, out_sz, ns);
     lds_barrier();
     const int units = here ? ns * quads * OW : 0;
@@ -2164,73 +2167,106 @@ TN_INLINE void conv_param_pair(const TinyLayer *__restrict__ L, const float *__r
 // pixels of its rows whose window element lies inside the input, and the group adds up with butterfly shuffles. Workgroup
 // `block` has as many (weight, lane) units as threads. (A workgroup per channel pair over several samples, as above, is few and long
 // for wide windows, and short of work for small planes. 28x28, 1 -> 8, 7x7, pool, 8 -> 16, 4x4, the launch, us, so / here: 16 samples
-// 26.9 / 7.7, 64 28.5 / 15.7, 256 57 / 43; 28x28, 1 -> 8 -> 16 channels, stride 2, 16 samples 10.6 / 7.1, 256 38 / 22.)
-__host__ __device__ inline int conv_rows_lanes(const TinyLayer &L) {
+// 26.9 / 6.4, 256 53 / 33; 32x32, 1 -> 8, 4x4, pool, 16 samples 84 / 6.7; 8x8, 1 -> 24, 4x4, 24 -> 8, 2x2, 8 -> 16, 3x3, 218 samples 65 / 15.)
+// A few samples may be one group, added up one after the other and updated here (tiny_groups): 12x12, 3 -> 4, 2x2, the step, us, two samples
+// 20.1 where a slice each takes 23, four 24.2 and 23.8; 32x32, 1 -> 8, 4x4, two 67.4 and 65.6.
+__host__ __device__ inline int conv_rows_lanes(const TinyLayer &L, const int batch) {
   int g = 32;
-  while (g > 1 && (32 * g > L.OH * L.OW || g > L.OH)) g >>= 1;   // 32 output pixels or more per lane
+  const int pixels = batch <= 8 ? 8 : 32;   // or more per lane; few samples leave units to spare
+  while (g > 1 && (pixels * g > L.OH * L.OW || g > L.OH)) g >>= 1;
   return g;
 }
-TN_INLINE void conv_param_rows(const TinyLayer *__restrict__ L, const float *__restrict__ gin, const float *__restrict__ gdy,
-                               const int block, float *__restrict__ slice, float *lds) {
-  const int H = L->H, W = L->W, K = L->K, OH = L->OH, OW = L->OW, sh = L->sh, sw = L->sw, plane = OH * OW;
+// Behind the weights' units, in waves of their own, come the biases', conv_rows_bias_lanes a channel.
+__host__ __device__ inline int conv_rows_bias_lanes(const TinyLayer &L) {
+  int g = 64;
+  while (g > 1 && (L.nb * g > TR_THREADS || g > L.OH * L.OW)) g >>= 1;
+  return g;
+}
+__host__ __device__ inline int conv_rows_weight_units(const TinyLayer &L, const int batch) { return (L.nw * conv_rows_lanes(L, batch) + 63) & ~63; }
+template <int KIND>
+TN_INLINE void conv_param_rows(const TinyLayer *__restrict__ L, const float *__restrict__ gin, const int in_sz,
+                               const float *__restrict__ gdy, const int out_sz, const int s_beg, const int s_end, const int block,
+                               const int group, const int batch, const TinyUpdate &u, float *lds) {
+  const int H = L->H, W = L->W, K = L->K, OH = L->OH, OW = L->OW, sh = L->sh, sw = L->sw, plane = OH * OW, nw = L->nw, nb = L->nb;
   const FastDiv d_taps = L->d_taps, d_s = L->d_s, d_c = L->d_c;
   const uint8_t *__restrict__ tbl = L->tbl;
-  const int g = conv_rows_lanes(*L), gs = __ffs(g) - 1, end = L->nw << gs;
-  const int base = block * TP_THREADS, it = base + static_cast<int>(threadIdx.x), idx = min(it, end - 1) >> gs, part = it & (g - 1);
+  const int g = conv_rows_lanes(*L, batch), gs = __ffs(g) - 1, end = nw << gs, biases = conv_rows_weight_units(*L, batch);
+  const int base = block * TR_THREADS, it = base + static_cast<int>(threadIdx.x);
+  const bool of_bias = base + 64 * wave_index() >= biases;
+  const int lanes = of_bias ? conv_rows_bias_lanes(*L) : g, part = it & (lanes - 1);
+  const int idx = of_bias ? (it - biases) >> (__ffs(lanes) - 1) : min(it, end - 1) >> gs;
+  const bool mine = of_bias ? idx < nb : it < end;
+  const TinyTarget target = tn_target<KIND>(u, L, of_bias, group);
+  const TinyOld old = tn_old<KIND>(target, idx, mine && part == 0);
   // (of dY, the planes of the output channels that these units are of)
-  const int co_lo = static_cast<int>(L->d_nk.div(base >> gs));
-  const int co_hi = static_cast<int>(L->d_nk.div((min(base + TP_THREADS, end) - 1) >> gs));
-  float *in = lds, *dy = lds + quad_pitch(L->in_size);
-  fill_lds<TP_THREADS>(in, gin, L->in_size);
-  fill_lds<TP_THREADS>(dy, gdy + co_lo * plane, (co_hi - co_lo + 1) * plane);
-  lds_barrier();
+  const bool has_bias = base + TR_THREADS > biases && nb;
+  const int co_lo = has_bias ? 0 : static_cast<int>(L->d_nk.div(base >> gs));
+  const int co_hi = has_bias ? K - 1 : static_cast<int>(L->d_nk.div((min(base + TR_THREADS, end) - 1) >> gs));
+  float *in = lds, *dy = lds + quad_pitch(in_sz);
   uint32_t pair, tap, co, ci, wy, wx;
-  d_taps.divmod(idx, pair, tap);
+  d_taps.divmod(of_bias ? 0 : idx, pair, tap);
   d_c.divmod(pair, co, ci);
   d_s.divmod(tap, wy, wx);
+  // iy = oy*sh + wy - ph in [0, H), ix = ox*sw + wx - pw in [0, W)
+  const int yoff = static_cast<int>(wy) - L->ph, xoff = static_cast<int>(wx) - L->pw;
+  int oy_lo = max(0, -yoff), oy_hi = min(OH, H - yoff), ox_lo = max(0, -xoff), ox_hi = min(OW, W - xoff);
+  if (sh != 1 || sw != 1) {
+    oy_lo = yoff >= 0 ? 0 : (-yoff + sh - 1) / sh, oy_hi = H - 1 - yoff < 0 ? 0 : min(OH, (H - 1 - yoff) / sh + 1);
+    ox_lo = xoff >= 0 ? 0 : (-xoff + sw - 1) / sw, ox_hi = W - 1 - xoff < 0 ? 0 : min(OW, (W - 1 - xoff) / sw + 1);
+  }
+  const bool connected = mine && (of_bias || !tbl || tbl[ci * K + co]);
   float sum = 0.0f;
-  if (it < end && (!tbl || tbl[ci * K + co])) {
-    // iy = oy*sh + wy - ph in [0, H), ix = ox*sw + wx - pw in [0, W)
-    const int yoff = static_cast<int>(wy) - L->ph, xoff = static_cast<int>(wx) - L->pw;
-    const int oy_lo = yoff >= 0 ? 0 : (-yoff + sh - 1) / sh, oy_hi = H - 1 - yoff < 0 ? 0 : min(OH, (H - 1 - yoff) / sh + 1);
-    const int ox_lo = xoff >= 0 ? 0 : (-xoff + sw - 1) / sw, ox_hi = W - 1 - xoff < 0 ? 0 : min(OW, (W - 1 - xoff) / sw + 1);
+  for (int s = s_beg; s < s_end; ++s) {
+    if (s > s_beg) lds_barrier();
+    if (base < end) fill_lds<TR_THREADS>(in, gin + static_cast<size_t>(s) * in_sz, in_sz);
+    fill_lds<TR_THREADS>(dy, gdy + static_cast<size_t>(s) * out_sz + co_lo * plane, (co_hi - co_lo + 1) * plane);
+    lds_barrier();
+    if (!connected) continue;
+    if (of_bias) {
+      for (int p = part; p < plane; p += lanes) sum += dy[idx * plane + p];
+      continue;
+    }
     const float *ip = in + (static_cast<int>(ci) * H + yoff) * W + xoff, *dp = dy + (static_cast<int>(co) - co_lo) * plane;
-    for (int oy = oy_lo + part; oy < oy_hi; oy += g) {
-      const float *ir = ip + oy * sh * W, *dr = dp + oy * OW;
-      int ox = ox_lo;
-      for (; ox + 4 <= ox_hi; ox += 4)
-        sum += ir[ox * sw] * dr[ox] + ir[(ox + 1) * sw] * dr[ox + 1] + ir[(ox + 2) * sw] * dr[ox + 2] + ir[(ox + 3) * sw] * dr[ox + 3];
-      for (; ox < ox_hi; ++ox) sum += ir[ox * sw] * dr[ox];
+    const auto rows = [&](auto step) {
+      for (int oy = oy_lo + part; oy < oy_hi; oy += g) {
+        const float *ir = ip + oy * sh * W, *dr = dp + oy * OW;
+        int ox = ox_lo;
+        for (; ox + 4 <= ox_hi; ox += 4)
+          sum += ir[ox * step] * dr[ox] + ir[(ox + 1) * step] * dr[ox + 1] + ir[(ox + 2) * step] * dr[ox + 2] + ir[(ox + 3) * step] * dr[ox + 3];
+        for (; ox < ox_hi; ++ox) sum += ir[ox * step] * dr[ox];
+      }
+    };
+    if (g > 4 && (OW & 7) == 0 && ox_lo < ox_hi) {
+      // The lanes of a group read rows that lie a multiple of eight words apart: each begins a pixel further, or they
+      // meet on a few banks (32x32, 1 -> 8, 4x4, one sample, the launch 17.7 us without, 6 so).
+      const int n = ox_hi - ox_lo, first = ox_lo + (part < n ? part : part % n);
+      for (int oy = oy_lo + part; oy < oy_hi; oy += g) {
+        const float *ir = ip + oy * sh * W, *dr = dp + oy * OW;
+        int ox = first;
+        for (int i = 0; i < n; ++i) {
+          sum += ir[ox * sw] * dr[ox];
+          ox = ox + 1 == ox_hi ? ox_lo : ox + 1;
+        }
+      }
+    } else if (sw == 1) {
+      rows(std::integral_constant<int, 1>());   // (words that follow each other: two a read)
+    } else {
+      rows(sw);
     }
   }
-  sum = group_sum(sum, g);
-  if (it < end && part == 0) slice[idx] = sum;
-}
-// the bias gradient of such a convolution, a workgroup of its own: a group of lanes a channel
-TN_INLINE void conv_param_bias(const TinyLayer *__restrict__ L, const float *__restrict__ gdy, float *__restrict__ slice) {
-  const int nb = L->nb, plane = L->OH * L->OW;
-  int g = 64;
-  while (g > 1 && (nb * g > 2 * TP_THREADS || g > plane)) g >>= 1;
-  const int total = nb * g, gs = __ffs(g) - 1;
-  for (int base = 0; base < total; base += TP_THREADS) {
-    const int it = base + static_cast<int>(threadIdx.x), co = it >> gs, part = it & (g - 1);
-    float sum = 0.0f;
-    if (it < total)
-      for (int p = part; p < plane; p += g) sum += gdy[co * plane + p];
-    sum = group_sum(sum, g);
-    if (it < total && part == 0) slice[co] = sum;
-  }
+  sum = group_sum(sum, lanes);
+  if (mine && part == 0) tn_finish<KIND>(target, old, idx, sum);
 }
 // A fully-connected layer, or a convolution that is one: a weight is the sum over the samples of one input times one
 // output gradient. V weights a thread, neighbours along the faster index (V = 4: its rows are whole, aligned words).
-template <int KIND, int V, int AHEAD>
+template <int KIND, int V, int AHEAD, int NT>
 TN_INLINE void outer_param(const TinyLayer *__restrict__ L, const float *__restrict__ gin, const int in_sz,
                            const float *__restrict__ gdy, const int out_sz, const int s_beg, const int s_end,
                            const int block, const int group, const TinyUpdate &u) {
   const bool conv = L->kind == TDH_L_CONV;   // [co][k], or [input][output]
   const float *fast = conv ? gin : gdy, *slow = conv ? gdy : gin;
   const int fast_stride = conv ? in_sz : out_sz, slow_stride = conv ? out_sz : in_sz, nw = L->nw;
-  const int e = (block * TP_THREADS + static_cast<int>(threadIdx.x)) * V;
+  const int e = (block * NT + static_cast<int>(threadIdx.x)) * V;
   if (e >= nw) return;
   uint32_t r, c;
   if (conv) L->d_nk.divmod(e, r, c);
@@ -2271,10 +2307,10 @@ TN_INLINE void outer_param(const TinyLayer *__restrict__ L, const float *__restr
   }
 }
 // element e of n: the sum over the samples of src[sample][stride]
-template <int KIND>
+template <int KIND, int NT>
 TN_INLINE void column_param(const float *__restrict__ src, const size_t stride, const int n, const int s_beg, const int s_end,
                             const int block, const TinyTarget &t) {
-  const int e = block * TP_THREADS + threadIdx.x;
+  const int e = block * NT + threadIdx.x;
   if (e >= n) return;
   const TinyOld old = tn_old<KIND>(t, e, true);
   constexpr int AHEAD = 16;
@@ -2289,7 +2325,7 @@ TN_INLINE void column_param(const float *__restrict__ src, const size_t stride, 
   tn_finish<KIND>(t, old, e, sum);
 }
 // an average pool's channel (average_pooling_layer.h:58-106): dW = scale * sum of (window sum * dY), db = sum of dY
-template <int KIND>
+template <int KIND, int NT>
 TN_INLINE void pool_param(const TinyLayer *__restrict__ L, const float *__restrict__ gin, const int in_sz,
                           const float *__restrict__ gdy, const int out_sz, const int s_beg, const int s_end, const int c,
                           const int group, const TinyUpdate &u, float *lds) {
@@ -2300,10 +2336,10 @@ TN_INLINE void pool_param(const TinyLayer *__restrict__ L, const float *__restri
   for (int s0 = s_beg; s0 < s_end; s0 += chunk) {
     const int ns = min(chunk, s_end - s0);
     lds_barrier();
-    stage_planes(L, xl, gin + static_cast<size_t>(s0) * in_sz + c * iplane, in_sz, iplane, L->d_iplane, dl,
+    stage_planes<NT>(L, xl, gin + static_cast<size_t>(s0) * in_sz + c * iplane, in_sz, iplane, L->d_iplane, dl,
                  gdy + static_cast<size_t>(s0) * out_sz + c * plane, out_sz, ns);
     lds_barrier();
-    for (int i = threadIdx.x; i < ns * plane; i += TP_THREADS) {
+    for (int i = threadIdx.x; i < ns * plane; i += NT) {
       uint32_t s, r, oy, ox;
       d_oplane.divmod(i, s, r);
       d_ow.divmod(r, oy, ox);
@@ -2316,8 +2352,8 @@ TN_INLINE void pool_param(const TinyLayer *__restrict__ L, const float *__restri
     }
   }
   lds_barrier();
-  dw = workgroup_sum(dw, lds);
-  db = workgroup_sum(db, lds + TP_WAVES);
+  dw = workgroup_sum<NT>(dw, lds);
+  db = workgroup_sum<NT>(db, lds + NT / 64);
   if (threadIdx.x == 0) {
     const TinyTarget tw = tn_target<KIND>(u, L, false, group), tb = tn_target<KIND>(u, L, true, group);
     tn_finish<KIND>(tw, tn_old<KIND>(tw, c, true), c, dw * L->scale);
@@ -2338,7 +2374,7 @@ __host__ __device__ inline DxBand dx_band(const TinyLayer &L) {
   b.floats = L.K * (b.rows + L.R - 1) * quad_pitch(L.W + L.S - 1) + 4 + TP_THREADS * 4;
   return b;
 }
-template <int R, int S>
+template <int R, int S, int NT>
 TN_INLINE void conv_dx_band(const TinyLayer *__restrict__ L, const float *__restrict__ w, const float *__restrict__ gdy,
                             float *__restrict__ gdx, const int ci, const int band, float *lds) {
   const int C = L->C, H = L->H, W = L->W, K = L->K, OH = L->OH, OW = L->OW, PW = quad_pitch(W + S - 1), units_w = (W + 3) >> 2;
@@ -2347,20 +2383,20 @@ TN_INLINE void conv_dx_band(const TinyLayer *__restrict__ L, const float *__rest
   const FastDiv d_pw = L->d_pw4;
   const uint8_t *__restrict__ tbl = L->tbl;
   constexpr int AHEAD = 8;
-  for (int base = threadIdx.x; base < cells; base += AHEAD * TP_THREADS) {
+  for (int base = threadIdx.x; base < cells; base += AHEAD * NT) {
     float v[AHEAD];
     bool in[AHEAD];
 #pragma unroll
     for (int j = 0; j < AHEAD; ++j) {
       uint32_t line, px;
-      d_pw.divmod(min(base + j * TP_THREADS, cells - 1), line, px);
+      d_pw.divmod(min(base + j * NT, cells - 1), line, px);
       const int co = static_cast<int>(line) / fr, oy = oy0 + static_cast<int>(line) - co * fr, ox = ox0 + static_cast<int>(px);
       in[j] = static_cast<unsigned>(oy) < static_cast<unsigned>(OH) && static_cast<unsigned>(ox) < static_cast<unsigned>(OW);
       v[j]  = gdy[in[j] ? (co * OH + oy) * OW + ox : 0];
     }
 #pragma unroll
     for (int j = 0; j < AHEAD; ++j)
-      if (base + j * TP_THREADS < cells) lds[base + j * TP_THREADS] = in[j] ? v[j] : 0.0f;
+      if (base + j * NT < cells) lds[base + j * NT] = in[j] ? v[j] : 0.0f;
   }
   lds_barrier();
   constexpr int taps = R * S;
@@ -2369,7 +2405,7 @@ TN_INLINE void conv_dx_band(const TinyLayer *__restrict__ L, const float *__rest
   for (int u0 = 0; u0 < units; u0 += 64) {     // (one trip unless a row has more units than a wave lanes)
     const int unit = min(u0 + lane, units - 1), iy = unit / units_w, ix = (unit - iy * units_w) << 2;
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int co = wave; co < K; co += TP_WAVES) {
+    for (int co = wave; co < K; co += NT / 64) {
       if (tbl && !tbl[ci * K + co]) continue;
       const ScalarFloats wq = (ScalarFloats)(w + static_cast<size_t>(co * C + ci) * taps);
       const float *dp = lds + co * PP + iy * PW + ix;
@@ -2394,7 +2430,7 @@ TN_INLINE void conv_dx_band(const TinyLayer *__restrict__ L, const float *__rest
     if (threadIdx.x < 256 && mine < units && mx < W) {
       float v = scratch[threadIdx.x];
 #pragma unroll
-      for (int k = 1; k < TP_WAVES; ++k) v += scratch[256 * k + threadIdx.x];
+      for (int k = 1; k < NT / 64; ++k) v += scratch[256 * k + threadIdx.x];
       gdx[(y0 + my) * W + mx] = v;
     }
     lds_barrier();
@@ -2402,14 +2438,16 @@ TN_INLINE void conv_dx_band(const TinyLayer *__restrict__ L, const float *__rest
 }
 
 // ROADS: what there is code for. TP_HAS_PAIRS: 3x3 or 5x5 windows of stride 1, and the first layer's dX; TP_HAS_WAVES: a wave a pair;
-// TP_HAS_ROWS: other windows. (All of it in one kernel, LeNet-5's step at 16 samples takes 41.1 us instead of 40.7: more scalars than
-// there are registers for.)
-constexpr int TP_HAS_PAIRS = 1, TP_HAS_WAVES = 2, TP_HAS_ROWS = 4;
+// TP_HAS_ROWS: sample by sample, any window; TP_HAS_DX: the first layer's dX beside it. (All of it in one kernel, LeNet-5's step at 16
+// samples takes 41.1 us instead of 40.7: more scalars than there are registers for.)
+constexpr int TP_HAS_PAIRS = 1, TP_HAS_WAVES = 2, TP_HAS_ROWS = 4, TP_HAS_DX = 8;
+__host__ __device__ constexpr int param_threads(const int roads) { return roads & TP_HAS_ROWS ? TR_THREADS : TP_THREADS; }
 template <int KIND, int ROADS>
-__global__ void __launch_bounds__(TP_THREADS, ROADS & TP_HAS_PAIRS ? 4 : 6)
+__global__ void __launch_bounds__(param_threads(ROADS), ROADS & TP_HAS_PAIRS ? 4 : 7)
 tiny_net_param_kernel(const TinyPlan *__restrict__ plan, const float *__restrict__ x, const TinyRanges ranges,
                       const TinyUpdate u, const int batch, const int param_blocks) {
   extern __shared__ float lds[];
+  constexpr int NT = param_threads(ROADS);
   constexpr int AHEAD = ROADS & TP_HAS_PAIRS ? 16 : 4;   // samples that an outer product has in flight
   if (KIND >= 0 && opt_powers(KIND) > 0 && u.powers_in && blockIdx.x == 0 && threadIdx.x == 0) {   // (as opt_multi_kernel)
     float q1 = u.powers_in[0], q2 = u.powers_in[1];
@@ -2422,14 +2460,14 @@ tiny_net_param_kernel(const TinyPlan *__restrict__ plan, const float *__restrict
   }
   const int n = plan->n;
   int id = blockIdx.x;
-  if ((ROADS & TP_HAS_PAIRS) && id >= param_blocks) {   // workgroups (band, input channel, sample), samples fastest
+  if ((ROADS & (TP_HAS_PAIRS | TP_HAS_DX)) && id >= param_blocks) {   // workgroups (band, input channel, sample), samples fastest
     id -= param_blocks;
     const TinyLayer *__restrict__ L = &plan->l[0];
     const int rest = id / batch, s = id - rest * batch, ci = rest % L->C, band = rest / L->C;
     const float *gdy = plan->l[1].dx + static_cast<size_t>(s) * L->out_size;
     float *gdx = L->dx + static_cast<size_t>(s) * L->in_size + ci * L->H * L->W;
-    if (L->R == 5) conv_dx_band<5, 5>(L, plan->first_w, gdy, gdx, ci, band, lds);
-    else conv_dx_band<3, 3>(L, plan->first_w, gdy, gdx, ci, band, lds);
+    if (L->R == 5) conv_dx_band<5, 5, NT>(L, plan->first_w, gdy, gdx, ci, band, lds);
+    else conv_dx_band<3, 3, NT>(L, plan->first_w, gdy, gdx, ci, band, lds);
     return;
   }
   int first = 0, job = ranges.job[0], per_group = ranges.per_group[0], size = ranges.size[0];
@@ -2441,7 +2479,10 @@ tiny_net_param_kernel(const TinyPlan *__restrict__ plan, const float *__restrict
     per_group = on ? ranges.per_group[k] : per_group;
     size      = on ? ranges.size[k] : size;
   }
-  const int li = job >> 4, what = job & 15, group = (id - first) / per_group, block = id - first - group * per_group;
+  const int li = job >> 4, what = job & 15, part = id - first;
+  // (a sample after the other in dispatch order, where a group is one: the workgroups of a sample then meet on few of the chip's second-level caches)
+  const int groups = (batch + size - 1) / size, group = ROADS & TP_HAS_ROWS ? part % groups : part / per_group;
+  const int block = ROADS & TP_HAS_ROWS ? part / groups : part - group * per_group;
   const TinyLayer *__restrict__ L = &plan->l[li];
   const int in_sz = L->in_size, out_sz = L->out_size;
   const float *gin = li == 0 ? x : plan->l[li - 1].out;
@@ -2466,22 +2507,15 @@ tiny_net_param_kernel(const TinyPlan *__restrict__ plan, const float *__restrict
         else pad ? run(three, std::true_type()) : run(three, std::false_type());
       }
       break;
-    // (groups of one sample, slices only)
     case TP_ROWS:
-      if constexpr (ROADS & TP_HAS_ROWS)
-        conv_param_rows(L, gin + static_cast<size_t>(s_beg) * in_sz, gdy + static_cast<size_t>(s_beg) * out_sz, block,
-                        L->gw + static_cast<size_t>(group) * L->nw, lds);
+      if constexpr (ROADS & TP_HAS_ROWS) conv_param_rows<KIND>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, block, group, batch, u, lds);
       break;
-    case TP_BIAS:
-      if constexpr (ROADS & TP_HAS_ROWS)
-        conv_param_bias(L, gdy + static_cast<size_t>(s_beg) * out_sz, L->gb + static_cast<size_t>(group) * L->nb);
-      break;
-    case TP_OUTER: outer_param<KIND, 1, AHEAD>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, block, group, u); break;
-    case TP_OUTER4: outer_param<KIND, 4, AHEAD>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, block, group, u); break;
-    case TP_COLUMNS: column_param<KIND>(gdy, out_sz, L->nb, s_beg, s_end, block, tn_target<KIND>(u, L, true, group)); break;
-    case TP_POOL: pool_param<KIND>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, block, group, u, lds); break;
-    case TP_SLICES_W: column_param<KIND>(L->pw_part, L->nw, L->nw, s_beg, s_end, block, tn_target<KIND>(u, L, false, group)); break;
-    default: column_param<KIND>(L->pb_part, L->nb, L->nb, s_beg, s_end, block, tn_target<KIND>(u, L, true, group)); break;
+    case TP_OUTER: outer_param<KIND, 1, AHEAD, NT>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, block, group, u); break;
+    case TP_OUTER4: outer_param<KIND, 4, AHEAD, NT>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, block, group, u); break;
+    case TP_COLUMNS: column_param<KIND, NT>(gdy, out_sz, L->nb, s_beg, s_end, block, tn_target<KIND>(u, L, true, group)); break;
+    case TP_POOL: pool_param<KIND, NT>(L, gin, in_sz, gdy, out_sz, s_beg, s_end, block, group, u, lds); break;
+    case TP_SLICES_W: column_param<KIND, NT>(L->pw_part, L->nw, L->nw, s_beg, s_end, block, tn_target<KIND>(u, L, false, group)); break;
+    default: column_param<KIND, NT>(L->pb_part, L->nb, L->nb, s_beg, s_end, block, tn_target<KIND>(u, L, true, group)); break;
   }
 }
 
@@ -2501,19 +2535,23 @@ tiny_net_merge_kernel(const TinyMerge m) {
 }  // namespace
 
 // of an optimizer kind, or -1 for slices, which may be of every road
+template <int KIND>
+static decltype(&tiny_net_param_kernel<-1, 0>) param_kernel_of(const int roads) {
+  if (roads & TP_HAS_ROWS) return roads & TP_HAS_DX ? tiny_net_param_kernel<KIND, TP_HAS_ROWS | TP_HAS_DX> : tiny_net_param_kernel<KIND, TP_HAS_ROWS>;
+  if constexpr (KIND < 0)
+    if (roads & TP_HAS_WAVES) return tiny_net_param_kernel<KIND, TP_HAS_PAIRS | TP_HAS_WAVES>;
+  return tiny_net_param_kernel<KIND, TP_HAS_PAIRS>;
+}
 static decltype(&tiny_net_param_kernel<-1, 0>) param_kernel(const int kind, const int roads) {
   switch (kind) {
-    case -1:
-      return roads == TP_HAS_ROWS                     ? tiny_net_param_kernel<-1, TP_HAS_ROWS>
-             : roads & (TP_HAS_WAVES | TP_HAS_ROWS) ? tiny_net_param_kernel<-1, TP_HAS_PAIRS | TP_HAS_WAVES | TP_HAS_ROWS>
-                                                    : tiny_net_param_kernel<-1, TP_HAS_PAIRS>;
-    case TDH_OPT_SGD: return tiny_net_param_kernel<TDH_OPT_SGD, TP_HAS_PAIRS>;
-    case TDH_OPT_MOMENTUM: return tiny_net_param_kernel<TDH_OPT_MOMENTUM, TP_HAS_PAIRS>;
-    case TDH_OPT_NESTEROV: return tiny_net_param_kernel<TDH_OPT_NESTEROV, TP_HAS_PAIRS>;
-    case TDH_OPT_ADAM: return tiny_net_param_kernel<TDH_OPT_ADAM, TP_HAS_PAIRS>;
-    case TDH_OPT_ADAGRAD: return tiny_net_param_kernel<TDH_OPT_ADAGRAD, TP_HAS_PAIRS>;
-    case TDH_OPT_RMSPROP: return tiny_net_param_kernel<TDH_OPT_RMSPROP, TP_HAS_PAIRS>;
-    case TDH_OPT_ADAMAX: return tiny_net_param_kernel<TDH_OPT_ADAMAX, TP_HAS_PAIRS>;
+    case -1: return param_kernel_of<-1>(roads);
+    case TDH_OPT_SGD: return param_kernel_of<TDH_OPT_SGD>(roads);
+    case TDH_OPT_MOMENTUM: return param_kernel_of<TDH_OPT_MOMENTUM>(roads);
+    case TDH_OPT_NESTEROV: return param_kernel_of<TDH_OPT_NESTEROV>(roads);
+    case TDH_OPT_ADAM: return param_kernel_of<TDH_OPT_ADAM>(roads);
+    case TDH_OPT_ADAGRAD: return param_kernel_of<TDH_OPT_ADAGRAD>(roads);
+    case TDH_OPT_RMSPROP: return param_kernel_of<TDH_OPT_RMSPROP>(roads);
+    case TDH_OPT_ADAMAX: return param_kernel_of<TDH_OPT_ADAMAX>(roads);
     default: return nullptr;
   }
 }
@@ -2524,8 +2562,9 @@ int tiny_prepare() {
     const auto of = [](auto k) { return reinterpret_cast<const void *>(k); };
     std::vector<const void *> kernels = {of(&tiny_net_step_kernel<false>), of(&tiny_net_step_kernel<true>), of(&tiny_net_front_kernel),
                                          of(&tiny_net_back_kernel)};
-    for (int kind = -1; kind <= TDH_OPT_NESTEROV; ++kind) kernels.push_back(of(param_kernel(kind, TP_HAS_PAIRS)));
-    for (int roads : {TP_HAS_ROWS, TP_HAS_PAIRS | TP_HAS_ROWS}) kernels.push_back(of(param_kernel(-1, roads)));
+    for (int kind = -1; kind <= TDH_OPT_NESTEROV; ++kind)
+      for (int roads : {TP_HAS_PAIRS, TP_HAS_ROWS, TP_HAS_ROWS | TP_HAS_DX}) kernels.push_back(of(param_kernel(kind, roads)));
+    kernels.push_back(of(param_kernel(-1, TP_HAS_WAVES)));
     for (const void *k : kernels)
       TDH_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(TINY_LDS_MAX_BYTES)));
     attr_set = true;
@@ -2562,10 +2601,14 @@ static void plan_split(TinyPlan &P) {
   P.split = m;
 }
 
-// convolutions whose weight gradients are added up sample by sample (conv_param_rows)
-static bool conv_by_rows(const TinyLayer &L) {
+// A window without an unrolled form in conv_param_pair
+static bool conv_any_window(const TinyLayer &L) {
   return L.kind == TDH_L_CONV && !conv_is_matvec(L) &&
          !(L.sh == 1 && L.sw == 1 && ((L.R == 5 && L.S == 5) || (L.R == 3 && L.S == 3)));
+}
+// Convolutions whose weight gradients are added up sample by sample (conv_param_rows): all of a net that has any such window
+static bool conv_by_rows(const TinyPlan &plan, const TinyLayer &L) {
+  return plan.by_rows && L.kind == TDH_L_CONV && !conv_is_matvec(L);
 }
 int tiny_layout(TinyPlan &P) {
   size_t framed = 0, lds = 26 * TP_WAVES;   // (conv_param_pair's sums)
@@ -2579,19 +2622,24 @@ int tiny_layout(TinyPlan &P) {
     }
   }
   P.first_dx_as_job = P.l[0].dx_framed && P.n > 1 && !P.skip_first_dx;
+  P.by_rows = std::any_of(P.l, P.l + P.n, conv_any_window);
+  int room = P.by_rows ? 4096 : 12288;
+  for (int i = 0; i < P.n; ++i)
+    if (conv_by_rows(P, P.l[i])) room = std::min(std::max(room, quad_pitch(P.l[i].in_size) + P.l[i].out_size), 12288);
   for (int i = 0; i < P.n; ++i) {
     TinyLayer &L = P.l[i];
     L.dw_chunk = 512;   // (what needs no LDS)
     if (i == 0 && P.first_dx_as_job) lds = std::max(lds, static_cast<size_t>(dx_band(L).floats));
     else if (L.dx_framed) framed = std::max(framed, static_cast<size_t>(conv_framed_floats(L)));
     if (!L.nw || L.kind == TDH_L_FC || conv_is_matvec(L)) continue;
-    if (conv_by_rows(L)) {
+    if (conv_by_rows(P, L)) {
       lds = std::max(lds, static_cast<size_t>(quad_pitch(L.in_size)) + L.out_size);
       continue;
     }
-    // planes of the input and the output gradient: as many samples at a time as fit 48 KB
+    // planes of the input and the output gradient: as many samples at a time as fit 48 KB, or beside single samples' sums
+    // no more than those take, or 16 KB (a workgroup a sample and lot of weights: three or four of them a compute unit)
     const int planes = L.H * L.W + L.OH * L.OW;
-    L.dw_chunk = std::min(std::max(12288 / planes, 1), 32);
+    L.dw_chunk = std::min(std::max(room / planes, 1), 32);
     lds = std::max(lds, static_cast<size_t>(L.dw_chunk) * planes + 4);
     if (L.kind != TDH_L_CONV || L.C == 1) continue;
     const int channels = std::min(L.C, TP_WAVES), more = channels * L.H * L.W + L.OH * L.OW;
@@ -2716,9 +2764,10 @@ TinyGroups tiny_groups(const TinyPlan &plan, const int batch) {
   for (int i = 0; i < plan.n; ++i) {
     const TinyLayer &L = plan.l[i];
     if (!L.nw || i < m) continue;
-    if (conv_by_rows(L)) {
+    if (conv_by_rows(plan, L)) {
       rows  = true;
-      g.one = false;
+      // (a sample after the other: a trip to memory and some 0.1 us a lane's pixel, where the optimizer's launch takes 4.3)
+      g.one = g.one && (batch - 1) * (1.2 + 0.1 * ceil_div(L.OH, conv_rows_lanes(L, batch)) * L.OW) <= 4.3;
     } else if (L.kind == TDH_L_CONV && !conv_is_matvec(L)) {
       pairs   = true;
       if (!g.one) continue;
@@ -2732,17 +2781,17 @@ TinyGroups tiny_groups(const TinyPlan &plan, const int batch) {
   g.one = g.one && one <= several + 5.0 && (batch <= 32 || !(pairs || pools || m));
   for (int i = 0; i < plan.n; ++i) {
     const TinyLayer &L = plan.l[i];
-    g.size[i] = g.one ? batch : std::min(batch, 16);
+    // (beside single samples' sums the kernel has registers for four samples in flight: one trip each, unless that makes many slices)
+    g.size[i] = g.one ? batch : std::min(batch, rows && static_cast<long>(L.nw) * ceil_div(batch, 4) <= 1L << 18 ? 4 : 16);
     if (!L.nw || i < m) continue;
-    if (conv_by_rows(L)) {
-      g.size[i] = 1;
+    if (conv_by_rows(plan, L)) {
+      g.size[i] = g.one ? batch : 1;
     } else if (L.kind == TDH_L_CONV && !conv_is_matvec(L)) {
       const PairSplit p = best_pair_split(L, batch, g.one);
       g.size[i]  = p.size;
       g.waves[i] = p.waves;
     } else if (L.kind == TDH_L_AVEPOOL) {
-      g.size[i] = std::min(g.size[i], L.dw_chunk);
-      if (rows) g.size[i] = std::min(g.size[i], std::max(4, batch * L.C / 256));   // (whose others are of one sample)
+      g.size[i] = std::min({g.size[i], L.dw_chunk, rows ? std::max(4, batch * L.C / 256) : batch});
     }
   }
   return g;
@@ -2782,7 +2831,8 @@ int launch_tiny_params(const TinyPlan &plan, const TinyPlan *dev_plan, const Tin
                        tdh_opt *update, int n_tensors, const float *powers_in, float *powers_out) {
   TinyRanges r;
   int n = 0, blocks = 0;
-  int roads = plan.first_dx_as_job ? TP_HAS_PAIRS : 0;
+  int roads = (plan.first_dx_as_job ? TP_HAS_DX : 0) | (plan.by_rows ? TP_HAS_ROWS : 0);
+  const int threads = param_threads(roads);
   auto add = [&](int layer, int what, int count) {
     r.first[n]     = blocks;
     r.job[n]       = layer * 16 + what;
@@ -2797,15 +2847,13 @@ int launch_tiny_params(const TinyPlan &plan, const TinyPlan *dev_plan, const Tin
       const bool pair = L.kind == TDH_L_CONV && !conv_is_matvec(L);
       if (!L.nw || pair != (pass == 0)) continue;
       if (i < m) {   // left by the back kernel, sample by sample
-        add(i, TP_SLICES_W, ceil_div(L.nw, TP_THREADS));
-        if (L.nb) add(i, TP_SLICES_B, ceil_div(L.nb, TP_THREADS));
-      } else if (conv_by_rows(L)) {
-        add(i, TP_ROWS, ceil_div(L.nw * conv_rows_lanes(L), TP_THREADS));
-        if (L.nb) add(i, TP_BIAS, 1);
-        roads |= TP_HAS_ROWS;
+        add(i, TP_SLICES_W, ceil_div(L.nw, threads));
+        if (L.nb) add(i, TP_SLICES_B, ceil_div(L.nb, threads));
+      } else if (conv_by_rows(plan, L)) {
+        add(i, TP_ROWS, ceil_div(conv_rows_weight_units(L, batch) + L.nb * conv_rows_bias_lanes(L), threads));
       } else if (pair) {
         const bool waves = groups.waves[i];
-        roads |= TP_HAS_PAIRS | (waves ? TP_HAS_WAVES : 0);
+        roads |= waves ? TP_HAS_WAVES : 0;
         add(i, waves ? TP_CONV_WAVES : TP_CONV, L.K * (waves ? ceil_div(L.C, TP_WAVES) : L.C));
       } else if (L.kind == TDH_L_AVEPOOL) {
         add(i, TP_POOL, L.C);
@@ -2813,8 +2861,8 @@ int launch_tiny_params(const TinyPlan &plan, const TinyPlan *dev_plan, const Tin
         const bool conv = L.kind == TDH_L_CONV;
         const int fast = conv ? L.in_size : L.out_size;
         const bool vec = fast % 4 == 0 && (i > 0 || !conv || (reinterpret_cast<uintptr_t>(x) & 15u) == 0);
-        add(i, vec ? TP_OUTER4 : TP_OUTER, ceil_div(L.nw, (vec ? 4 : 1) * TP_THREADS));
-        if (L.nb) add(i, TP_COLUMNS, ceil_div(L.nb, TP_THREADS));
+        add(i, vec ? TP_OUTER4 : TP_OUTER, ceil_div(L.nw, (vec ? 4 : 1) * threads));
+        if (L.nb) add(i, TP_COLUMNS, ceil_div(L.nb, threads));
       }
     }
   for (int k = n; k < TP_RANGES; ++k) {
@@ -2833,7 +2881,7 @@ int launch_tiny_params(const TinyPlan &plan, const TinyPlan *dev_plan, const Tin
     ProfScope prof(roads & TP_HAS_ROWS ? "tiny_net_param_grads_any" : roads & TP_HAS_WAVES ? "tiny_net_param_grads_waves" : "tiny_net_param_grads", plan.flop_per_sample * batch * (1.0 / 3.0), WORK_FLOP);
     const auto kernel = param_kernel(update ? update->kind : -1, roads);
     if (!kernel) return set_error(TDH_ERR_INVALID, "optimizer kind %d is not supported", update->kind);
-    TDH_LAUNCH(kernel, dim3(blocks + dx_blocks), dim3(TP_THREADS), plan.lds_job_floats * sizeof(float),
+    TDH_LAUNCH(kernel, dim3(blocks + dx_blocks), dim3(threads), plan.lds_job_floats * sizeof(float),
                ctx().stream, dev_plan, x, r, u, batch, blocks);
     TDH_LAUNCH_CHECK();
   }
