@@ -994,7 +994,8 @@ constexpr int FDW_DEPTH = 4;              // sample pairs per group of loads
 // In front of the products, shared out evenly over the workgroups: the slices of dX (whose launch was the one before) added
 // up, and the bias gradient's column sums. 4096 x 4096, batch 256, us: launches of their own 8.6 + 4.8, here 7.5 of the kernel's
 // (half of the workgroups behind their products instead, so that the other one on a compute unit has the matrix cores
-// meanwhile: no different); 3000 x 3000, batch 100, the layer's forward, backward and update 154.5 / 150.
+// meanwhile: no different); 3000 x 3000, batch 100, the layer's forward, backward and update 154.5 / 150. SUMS: there are some; dW alone
+// has an instance without the divisions, 0.5 % of 31 drawn layers (4712 x 2566, batch 13 14.1 / 13.6).
 struct FcDwDirect {
   const float *x, *dy;
   float *dw;
@@ -1008,18 +1009,18 @@ typedef float fdw_x16 __attribute__((ext_vector_type(16)));
 
 // CA, CB: consecutive inputs and outputs a lane reads. Measured on 4096 x 4096 x 256: 4 x 2
 // (two waves per SIMD) 80 us, 4 x 4 (one wave per SIMD) 80 us, 2 x 2 (four waves) 93 us.
-template <int CA, int CB>
+template <int CA, int CB, bool SUMS>
 __global__ void __launch_bounds__(64 * FDW_WM * FDW_WN) __attribute__((amdgpu_waves_per_eu(CA * CB > 8 ? 1 : CA * CB > 4 ? 2 : 4, 8)))
 fc_dw_direct_kernel(const FcDwDirect f) {
   constexpr int FDW_TM = 32 * CA, FDW_TN = 32 * CB;
   typedef float avec __attribute__((ext_vector_type(CA)));
   typedef float bvec __attribute__((ext_vector_type(CB)));
   static_assert(64 * FDW_WM * FDW_WN == 256, "the sums are for 256 threads");
-  __shared__ float col_sums[8][32];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = lane & 31, h = lane >> 5;
-  const unsigned self = blockIdx.x + gridDim.x * blockIdx.y, all = gridDim.x * gridDim.y;
-  {
+  if constexpr (SUMS) {
+    __shared__ float col_sums[8][32];
+    const unsigned self = blockIdx.x + gridDim.x * blockIdx.y, all = gridDim.x * gridDim.y;
     auto first = [&](unsigned i, int blocks) { return static_cast<unsigned>(static_cast<unsigned long long>(i) * blocks / all); };
     for (unsigned u = first(self, f.sum_blocks); u < first(self + 1, f.sum_blocks); ++u)
       splitk_reduce_wide(f.sums.partial, f.sums.splits, f.sums.M, f.sums.N, f.sums.epi, u);
@@ -1415,7 +1416,8 @@ int fc_bwd(int in, int out, int has_bias, int batch, const float *x, const float
       ProfScope prof(left.partial ? "fc_dw_direct_sums" : "fc_dw_direct", in, out, batch);
       const FcDwDirect f{x, dy, dw, batch, in, out, accumulate, left, db, left.partial ? ceil_div(batch * in, REDUCE_WIDE_OUTPUTS) : 0,
                          bias_grad ? ceil_div(out, 32) : 0};
-      TDH_LAUNCH((fc_dw_direct_kernel<4, 2>), dim3(ceil_div(out, 64 * FDW_WN), ceil_div(in, 128 * FDW_WM)),
+      const auto kernel = f.sum_blocks + f.db_blocks ? fc_dw_direct_kernel<4, 2, true> : fc_dw_direct_kernel<4, 2, false>;
+      TDH_LAUNCH(kernel, dim3(ceil_div(out, 64 * FDW_WN), ceil_div(in, 128 * FDW_WM)),
                  dim3(64 * FDW_WM * FDW_WN), 0, ctx().stream, f);
       TDH_LAUNCH_CHECK();
     } else
