@@ -339,7 +339,9 @@ float *tdh_net_param(tdh_net *net, int layer, int which);
  * memory: in a train step with TDH_NET_FUSE_ACT_GRAD a convolution kernel that also writes the
  * pointwise activation or computes the 2x2 max-pool behind the convolution keeps the
  * convolution's own output in registers (nothing in the backward pass reads it: the gradients
- * of tanh, relu and sigmoid are functions of their outputs); tdh_net_forward always writes it */
+ * of tanh, relu and sigmoid are functions of their outputs), with a pool directly behind the
+ * convolution only in layers of few input channels or few tiles and in rows of fewer than 24 pixels;
+ * tdh_net_forward always writes it */
 const float *tdh_net_layer_out(const tdh_net *net, int layer);
 /* the gradient with respect to the layer's input as the last step left it, or NULL where
  * that step never wrote it to memory: with TDH_NET_FUSE_ACT_GRAD the gradient of a folded
